@@ -9,6 +9,7 @@
 #include "conv_mfma.hpp"
 #include "conv_f32.hpp"
 #include "conv_patch.hpp"
+#include "conv_stem.hpp"
 #include "conv_thin.hpp"
 #include "halo.hpp"
 #include "loss.hpp"
@@ -210,6 +211,16 @@ bool is_one_channel_cube(const sfh_conv3d_desc& p) {
   return p.cin == 1 && p.kd == p.kh && p.kh == p.kw && (p.kd == 2 || p.kd == 3);
 }
 
+// The network's first convolution on the matrix cores (conv_stem.hip): 1 to 4 input channels, 3x3x3 at unit stride.
+bool uses_stem(const sfh_conv3d_desc& p, int dtype, const int32_t out[3], StemArgs& a) {
+  if (p.kd != 3 || p.kh != 3 || p.kw != 3 || p.sd != 1 || p.sh != 1 || p.sw != 1 || p.dd != 1 || p.dh != 1 || p.dw != 1) return false;
+  a = StemArgs{};
+  a.n = p.n; a.od = out[0]; a.oh = out[1]; a.ow = out[2]; a.cw = p.cout;
+  a.td = p.in_d; a.th = p.in_h; a.tw = p.in_w; a.ct = p.cin;
+  a.pd = p.pd; a.ph = p.ph; a.pw = p.pw;
+  return stem_supported(a, dtype);
+}
+
 ThinArgs thin_base(const sfh_conv3d_desc& p, const int32_t out[3]) {
   ThinArgs a{};
   a.n = p.n; a.od = out[0]; a.oh = out[1]; a.ow = out[2];
@@ -370,14 +381,13 @@ static int conv3d_fwd_any(const sfh_conv3d_desc* p, int dtype, const void* x, co
     return mfma_conv_persist(a, dtype, x, workspace, bias, y, partial, st, gn, in2);
   }
   if (in2 != nullptr) return fail(SFH_ERR_UNSUPPORTED, "conv3d fwd: this problem does not take its input as two tensors");
-  if (gn != nullptr) {  // the one-channel stem is the only other kernel that leaves them
-    ThinArgs t;
-    if ((flags & SFH_FLAG_WEIGHT_PACKED) || thin_fwd_plan(*p, dtype, out, t) != kThinWideOut || thin_wide_out_gn_records(t, dtype, gn->groups) == 0)
-      return fail(SFH_ERR_UNSUPPORTED, "conv3d fwd: GroupNorm partials are not offered for this problem");
-    t.ws_kd = w_stride[2]; t.ws_kh = w_stride[3]; t.ws_kw = w_stride[4];
-    t.ws_wide = w_stride[0]; t.ws_thin = w_stride[1];
-    return thin_wide_out(t, dtype, x, w, bias, y, st, gn);
+  StemArgs stem;
+  if (!(flags & (SFH_FLAG_FORCE_GENERIC | SFH_FLAG_WEIGHT_PACKED)) && uses_stem(*p, dtype, out, stem) && on_16_bytes(y)) {
+    stem.ws_wide = w_stride[0]; stem.ws_thin = w_stride[1];
+    stem.ws_kd = w_stride[2]; stem.ws_kh = w_stride[3]; stem.ws_kw = w_stride[4];
+    return stem_fwd(stem, dtype, x, w, bias, y, st, gn != nullptr ? *gn : GnPartialOut{nullptr, 0, 0, 0});
   }
+  if (gn != nullptr) return fail(SFH_ERR_UNSUPPORTED, "conv3d fwd: GroupNorm partials are not offered for this problem");
   // the fp32 tiles move 16-byte pieces of x, bias and y: a view 4 bytes off that grid runs the direct kernel instead
   if (!(flags & (SFH_FLAG_FORCE_GENERIC | SFH_FLAG_WEIGHT_PACKED)) && fwd_uses_f32_tiles(*p, dtype, out) && on_16_bytes(x) &&
       on_16_bytes(y) && on_16_bytes(bias)) {
@@ -433,9 +443,8 @@ extern "C" int32_t sfh_conv3d_fwd_gn_records(const sfh_conv3d_desc* p, int dtype
   if (check_conv(p, dtype, out) != SFH_OK || groups < 1 || p->n == 0) return 0;
   if (fwd_uses_mfma(*p, dtype, out)) return mfma_conv_gn_records(fwd_mfma_args(*p, out), groups);
   if (fwd_uses_f32_tiles(*p, dtype, out) || fwd_uses_patch(*p, dtype, out)) return 0;
-  ThinArgs t;
-  if (thin_fwd_plan(*p, dtype, out, t) == kThinWideOut) return thin_wide_out_gn_records(t, dtype, groups);
-  return 0;
+  StemArgs stem;
+  return uses_stem(*p, dtype, out, stem) ? stem_gn_records(stem, groups) : 0;
 }
 
 extern "C" int sfh_conv3d_fwd_gn(const sfh_conv3d_desc* p, int dtype, const void* x, const void* w, const int64_t w_stride[5],
@@ -599,6 +608,8 @@ extern "C" int sfh_conv3d_wgrad_splits(const sfh_conv3d_desc* p, int dtype) {
   if (wgrad_uses_mfma(*p, dtype, out)) return mfma_wgrad_splits(wgrad_args(*p, out));
   if (wgrad_uses_f32_tiles(*p, dtype, out)) return f32_wgrad_splits(wgrad_args(*p, out));
   if (wgrad_uses_patch(*p, dtype, out)) return patch_reduce_splits(patch_args(*p, out));
+  StemArgs stem;
+  if (uses_stem(*p, dtype, out, stem)) return stem_wgrad_splits(stem);
   ThinArgs t;
   bool thin_is_x;
   if (thin_wgrad_plan(*p, dtype, out, t, thin_is_x) == kThinReduce) return thin_reduce_splits(t);
@@ -611,10 +622,12 @@ extern "C" size_t sfh_conv3d_wgrad_workspace_bytes(const sfh_conv3d_desc* p, int
   if (wgrad_uses_mfma(*p, dtype, out)) return mfma_wgrad_workspace_bytes(wgrad_args(*p, out));
   if (wgrad_uses_f32_tiles(*p, dtype, out)) return f32_wgrad_workspace_bytes(wgrad_args(*p, out));
   if (wgrad_uses_patch(*p, dtype, out)) return patch_reduce_workspace_bytes(patch_args(*p, out));
+  StemArgs stem;
+  const size_t stem_bytes = uses_stem(*p, dtype, out, stem) ? stem_wgrad_workspace_bytes(stem) : 0;
   ThinArgs t;
   bool thin_is_x;
-  if (thin_wgrad_plan(*p, dtype, out, t, thin_is_x) == kThinReduce) return thin_reduce_workspace_bytes(t);
-  return 0;
+  const size_t thin_bytes = thin_wgrad_plan(*p, dtype, out, t, thin_is_x) == kThinReduce ? thin_reduce_workspace_bytes(t) : 0;
+  return stem_bytes > thin_bytes ? stem_bytes : thin_bytes;  // the alignment of the operands decides between the two
 }
 
 static int conv3d_wgrad_any(const sfh_conv3d_desc* p, int dtype, const void* x, const void* gy, void* gw, void* workspace,
@@ -645,6 +658,13 @@ static int conv3d_wgrad_any(const sfh_conv3d_desc* p, int dtype, const void* x, 
     if (workspace == nullptr || workspace_bytes < need)
       return fail(SFH_ERR_WORKSPACE, "conv3d wgrad: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
     return patch_reduce(a, dtype, gy, x, gw, gw_dtype, workspace, st);
+  }
+  StemArgs stem;
+  if (!(flags & SFH_FLAG_FORCE_GENERIC) && uses_stem(*p, dtype, out, stem) && on_16_bytes(gy)) {
+    const size_t need = stem_wgrad_workspace_bytes(stem);
+    if (workspace == nullptr || workspace_bytes < need)
+      return fail(SFH_ERR_WORKSPACE, "conv3d wgrad: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+    return stem_wgrad(stem, dtype, x, gy, gw, gw_dtype, workspace, st);
   }
   if (!(flags & SFH_FLAG_FORCE_GENERIC)) {
     ThinArgs t;
