@@ -27,6 +27,7 @@ ordinary padded convolution.
 
 from __future__ import annotations
 
+import math
 from typing import Optional
 
 import torch
@@ -135,15 +136,29 @@ _WEIGHT_GRAD_QUEUE: list = []
 _BATCHABLE: dict = {}
 
 
+#: A weight gradient of more operations than this is computed in its own node although the module defers.  What a place
+#: in the batch saves is a launch and a slice sum (20 us), a tenth of such a problem's time; what it costs is that the
+#: operands have left the caches when the pass ends, and in early mode that half of the device works on it while the other
+#: half runs out of work.  Measured on captured steps (ms; everything deferred early / this rule): base width 64 on 128^3
+#: (problems of 464 and 928 GFLOP) 16.02 / 14.62, on 64 x 128 x 128 8.76 / 8.39, two samples of 64 x 70 x 75 6.52 / 6.29;
+#: base width 32 on 128^3 (its largest problem has 232 GFLOP) 4.96 deferred against 4.98 with a limit of 125 and 5.05 of 60.
+_DEFER_MAX_FLOPS = 250e9
+
+
 def _deferrable(param, in_shape, wshape, stride, padding, dilation, dtype) -> int:
-    """Whether a weight gradient can wait for the end of the pass: the parameter is a leaf that takes a ``.grad`` and the
-    library batches the problem.  0, or the launch of the batch that takes it (``conv3d.weight_grad_batch_family``)."""
+    """Whether a weight gradient can wait for the end of the pass: the parameter is a leaf that takes a ``.grad``, the
+    library batches the problem and it is not too large to gain from that.  0, or the launch of the batch that takes it
+    (``conv3d.weight_grad_batch_family``)."""
     if param is None or not param.is_leaf or not param.requires_grad:
         return 0
     key = (in_shape, wshape, stride, padding, dilation, dtype)
     ok = _BATCHABLE.get(key)
     if ok is None:
         ok = _c3.weight_grad_batch_family(in_shape, wshape, stride, padding, dilation, dtype)
+        if ok:
+            n, cout, *out = _c3.output_shape(in_shape, wshape, stride, padding, dilation)
+            if 2.0 * n * math.prod(out) * cout * math.prod(wshape[1:]) > _DEFER_MAX_FLOPS:
+                ok = 0
         if len(_BATCHABLE) > 256:
             _BATCHABLE.clear()
         _BATCHABLE[key] = ok
