@@ -229,6 +229,25 @@ def lib() -> ctypes.CDLL:
         return _lib
 
 
+_native = None
+
+
+def native():
+    """The C++ host path (``csrc/host/native.cpp``): raises :class:`ScaffoldLibraryError` if it is not built."""
+    global _native
+    if _native is None:
+        lib()  # the kernels it launches; a missing library is reported as such
+        try:
+            from . import _native as module
+        except ImportError as exc:
+            raise ScaffoldLibraryError(
+                f"scaffold_amd/_native.so cannot be loaded ({exc}); run `python -c 'import __graft_entry__ as g; g.build()'` "
+                "or `make -C scaffold_amd/csrc/host`. There is no fallback path.") from exc
+        module.set_callbacks(ScaffoldKernelError, _note_device)
+        _native = module
+    return _native
+
+
 def dtype_code(dtype: torch.dtype) -> int:
     try:
         return _DTYPE_CODE[dtype]

@@ -299,6 +299,20 @@ def is_supported_all(x, w, bias=None, stride=1, padding=0, dilation=1, groups: i
 # ---------------------------------------------------------------------------------------------
 # helpers
 # ---------------------------------------------------------------------------------------------
+# Which arguments the C++ host path can take as they are; anything else goes through the checks in Python, which say
+# what is wrong with it.
+def _tensors(a, b) -> bool:
+    return isinstance(a, torch.Tensor) and isinstance(b, torch.Tensor)
+
+
+def _tensors_or_none(*ts) -> bool:
+    return all([t is None or isinstance(t, torch.Tensor) for t in ts])
+
+
+def _sizes(v) -> bool:
+    return isinstance(v, torch.Size) or (isinstance(v, (tuple, list)) and all([type(e) is int for e in v]))
+
+
 def _check_out(y: torch.Tensor, shape: tuple[int, ...], like: torch.Tensor) -> None:
     if tuple(y.shape) != tuple(shape):
         raise ValueError(f"out= must have shape {tuple(shape)}, got {tuple(y.shape)}")
@@ -588,6 +602,15 @@ def conv3d_forward(
     as ``result._sfh_gn_partials`` and spare :func:`scaffold_amd.group_norm` its statistics pass. The result itself is the
     same bits either way, and the records are a function of the result alone (no state from earlier calls).
     """
+    if config is None and weight_rsck is None and out is None and not (weight_flip or force_generic) and groups == 1 \
+            and _tensors(x, w) and _tensors_or_none(bias, packed_weight):
+        done = _lib.native().conv_forward(x, w, bias, stride, padding, dilation, packed_weight, int(gn_groups), _second)
+        if done is not None:
+            y, partials, records = done
+            if partials is not None:
+                # valid for these bits of y only: the version lets the consumer see an in-place change
+                y._sfh_gn_partials = (partials, records, int(gn_groups), y._version)
+            return y
     if not _checked and not is_supported(x, w, bias, stride, padding, dilation, groups):
         raise NotImplementedError(
             f"unsupported: x={tuple(getattr(x, 'shape', ()))}/{getattr(x, 'dtype', None)} "
@@ -684,6 +707,11 @@ def conv3d_backward_data(
     taps mirrored and padding ``dil*(k-1) - p``; the swap and the mirror happen while the library
     repacks the weight, so no transformed copy of the weight is made here.
     """
+    if config is None and weight_rsck is None and out is None and not force_generic and groups == 1 and not _cin_first \
+            and _tensors(grad_output, weight) and _tensors_or_none(packed_weight) and _sizes(input_shape):
+        gx = _lib.native().conv_backward_data(grad_output, weight, input_shape, stride, padding, dilation, packed_weight)
+        if gx is not None:
+            return gx
     if not _checked and not is_supported_bwd_data(grad_output, weight, input_shape, stride, padding, dilation, groups):
         raise NotImplementedError(
             f"unsupported: grad_output={tuple(getattr(grad_output, 'shape', ()))}/{getattr(grad_output, 'dtype', None)} "
@@ -780,6 +808,11 @@ def conv3d_backward_weight(
     the fp32 sum of the slices unrounded (the gradient of an fp32 master weight under autocast, without the
     rounding and the up-cast); shapes only the untiled kernel serves raise ``NotImplementedError`` for it.
     """
+    if config is None and workspace is None and out is None and not force_generic and deterministic and groups == 1 \
+            and grad_dtype is None and _second is None and _tensors(input, grad_output) and _sizes(weight_shape):
+        gw = _lib.native().conv_backward_weight(input, weight_shape, grad_output, stride, padding, dilation)
+        if gw is not None:
+            return gw
     if not _checked and not is_supported_bwd_weight(input, weight_shape, grad_output, stride, padding, dilation, groups):
         raise NotImplementedError(
             f"unsupported: input={tuple(getattr(input, 'shape', ()))}/{getattr(input, 'dtype', None)} "

@@ -1,0 +1,858 @@
+// The host path of the eager ops in C++: gates, allocations, launches through the C ABI, and the autograd nodes.
+//
+// A train step of the U-Net is a few hundred launches of 3 to 60 us.  Issued from Python -- argument checks, ctypes, one
+// torch.autograd.Function per op, whose backward runs in the engine's thread and takes the interpreter lock -- an op cost
+// 25 us of host time in the forward pass and 40 us in the backward pass, which is what a step on a volume of 64^3 or less
+// took.  Here a forward op is one call into this module and a backward node runs without the interpreter.
+//
+// Every function either serves a call or returns None with nothing launched; the Python layer then takes the call apart
+// and raises what the contract says.  Nothing is kept from call to call but sizes derived from a problem's shape.
+#include <torch/extension.h>
+
+#include <ATen/autocast_mode.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+
+#include <atomic>
+#include <cstring>
+#include <string>
+#include <unordered_map>
+
+#include "../../../include/scaffold_hip.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+constexpr auto kCL3D = at::MemoryFormat::ChannelsLast3d;
+using MaybeTensor = std::optional<Tensor>;
+
+// ---- the Python side -----------------------------------------------------------------------------------------------------
+PyObject* g_kernel_error = nullptr;    // scaffold_amd._lib.ScaffoldKernelError
+PyObject* g_note_device = nullptr;     // scaffold_amd._lib._note_device(device)
+PyObject* g_queue_weight = nullptr;    // scaffold_amd.modules._queue_from_node(...)
+
+// A status code as the exception the entry points raise (the interpreter lock is taken if this thread does not hold it).
+void check(int rc, const char* what) {
+  if (rc == SFH_OK) return;
+  const char* said = sfh_last_error();
+  const std::string text = std::string(what) + ": " + (said != nullptr && *said ? said : "unknown error");
+  const bool called_from_python = PyGILState_Check() != 0;
+  py::gil_scoped_acquire gil;
+  PyObject* cls = rc == SFH_ERR_UNSUPPORTED ? PyExc_NotImplementedError
+                  : rc == SFH_ERR_INVALID || rc == SFH_ERR_WORKSPACE ? PyExc_ValueError
+                  : g_kernel_error != nullptr ? g_kernel_error : PyExc_RuntimeError;
+  PyErr_SetString(cls, text.c_str());
+  if (called_from_python) throw py::error_already_set();
+  python_error e;  // in a backward node: the engine carries it to the thread that called backward()
+  e.persist();
+  throw std::move(e);
+}
+
+std::atomic<uint64_t> g_devices_seen{0};
+
+// The stream torch is issuing work to on the tensor's device; the first call per device has Python look the device over.
+void* stream_of(const Tensor& t) {
+  const auto index = t.device().index();
+  const uint64_t bit = 1ull << (index & 63);
+  if (!(g_devices_seen.load(std::memory_order_relaxed) & bit)) {
+    g_devices_seen.fetch_or(bit);
+    if (g_note_device != nullptr) {
+      py::gil_scoped_acquire gil;
+      py::reinterpret_borrow<py::function>(g_note_device)(py::cast(t.device()));
+    }
+  }
+  return (void*)c10::hip::getCurrentHIPStream(index).stream();
+}
+
+int code_of(at::ScalarType t) {
+  return t == at::kBFloat16 ? SFH_BF16 : t == at::kHalf ? SFH_FP16 : t == at::kFloat ? SFH_FP32 : -1;
+}
+
+bool on_gpu(const Tensor& t) { return t.is_cuda() && t.layout() == at::kStrided; }
+const void* ptr(const Tensor& t) { return t.defined() ? t.const_data_ptr() : nullptr; }
+void* out_ptr(const Tensor& t) { return t.defined() ? t.mutable_data_ptr() : nullptr; }
+Tensor dense(const Tensor& t) { return t.is_contiguous(kCL3D) ? t : t.contiguous(kCL3D); }
+Tensor volume(at::IntArrayRef sizes, const Tensor& like, at::ScalarType dtype) {
+  return at::empty(sizes, like.options().dtype(dtype), kCL3D);
+}
+Tensor bytes(size_t n, const Tensor& like) { return n == 0 ? Tensor() : at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
+
+// An int or three ints; false for any other spelling (the Python layer then says what is wrong with it).
+bool three(py::handle h, int32_t v[3]) {
+  auto one = [](PyObject* o, int32_t& to) {
+    if (!PyLong_CheckExact(o)) return false;
+    int overflow = 0;
+    const long x = PyLong_AsLongAndOverflow(o, &overflow);
+    if (overflow || x < INT32_MIN || x > INT32_MAX) return false;
+    to = (int32_t)x;
+    return true;
+  };
+  if (PyLong_CheckExact(h.ptr())) return one(h.ptr(), v[0]) && (v[1] = v[2] = v[0], true);
+  if (!PyTuple_Check(h.ptr()) && !PyList_CheckExact(h.ptr())) return false;
+  if (PySequence_Fast_GET_SIZE(h.ptr()) != 3) return false;
+  for (int i = 0; i < 3; ++i)
+    if (!one(PySequence_Fast_GET_ITEM(h.ptr(), i), v[i])) return false;
+  return true;
+}
+
+// ---- convolution problems ------------------------------------------------------------------------------------------------
+// What the library says about a problem, asked once per shape and thread.
+struct Sizes {
+  size_t packed[2];           // bytes of the packed weight each direction reads
+  size_t work[3];             // workspace bytes: forward, data gradient, weight gradient
+  size_t work_bias;           // weight gradient with the bias gradient in the same pass (0: not offered)
+  int32_t groups = -1, records = 0;  // GroupNorm records for the last group count asked for
+};
+
+struct ProblemKey {
+  sfh_conv3d_desc d;
+  int32_t code;
+  bool operator==(const ProblemKey& o) const { return std::memcmp(this, &o, sizeof(ProblemKey)) == 0; }
+};
+static_assert(sizeof(ProblemKey) == 19 * sizeof(int32_t), "no padding in the key");
+struct ProblemHash {
+  size_t operator()(const ProblemKey& k) const {
+    const auto* p = reinterpret_cast<const uint32_t*>(&k);
+    uint64_t h = 1469598103934665603ull;
+    for (size_t i = 0; i < sizeof(ProblemKey) / 4; ++i) h = (h ^ p[i]) * 1099511628211ull;
+    return (size_t)(h ^ h >> 29);
+  }
+};
+
+struct Problem {
+  ProblemKey key;
+  int32_t out[3];
+  Sizes* sizes;
+  const sfh_conv3d_desc* desc() const { return &key.d; }
+  int32_t records(int groups) const {
+    if (sizes->groups != groups) {
+      sizes->records = sfh_conv3d_fwd_gn_records(&key.d, key.code, groups);
+      sizes->groups = groups;
+    }
+    return sizes->records;
+  }
+};
+
+Sizes* sizes_of(const ProblemKey& k) {
+  thread_local std::unordered_map<ProblemKey, Sizes, ProblemHash> known;
+  auto it = known.find(k);
+  if (it == known.end()) {
+    if (known.size() > 4096) known.clear();
+    Sizes s;
+    for (int dir = 0; dir < 2; ++dir) s.packed[dir] = sfh_conv3d_packed_weight_bytes(&k.d, k.code, dir);
+    s.work[0] = sfh_conv3d_fwd_workspace_bytes(&k.d, k.code);
+    s.work[1] = sfh_conv3d_dgrad_workspace_bytes(&k.d, k.code);
+    s.work[2] = sfh_conv3d_wgrad_workspace_bytes(&k.d, k.code);
+    s.work_bias = sfh_conv3d_wgrad_bias_workspace_bytes(&k.d, k.code);
+    it = known.emplace(k, s).first;
+  }
+  return &it->second;
+}
+
+// Geometry of conv3d(in, w) with (N, C, D, H, W) and (Cout, Cin, kd, kh, kw) sizes. False: not a problem the library has.
+bool make_problem(at::IntArrayRef in, at::IntArrayRef w, const int32_t s[3], const int32_t p[3], const int32_t d[3], int code, Problem& r) {
+  if (in.size() != 5 || w.size() != 5 || code < 0) return false;
+  for (auto v : in) if (v < 1 || v > INT32_MAX) return false;
+  for (auto v : w) if (v < 1 || v > INT32_MAX) return false;
+  for (int i = 0; i < 3; ++i) {
+    if (s[i] < 1 || d[i] < 1 || p[i] < 0) return false;
+    const int64_t span = in[2 + i] + 2 * (int64_t)p[i] - (int64_t)d[i] * (w[2 + i] - 1) - 1;
+    if (span < 0) return false;
+    r.out[i] = (int32_t)(span / s[i] + 1);
+  }
+  r.key.d = sfh_conv3d_desc{(int32_t)in[0], (int32_t)in[1], (int32_t)in[2], (int32_t)in[3], (int32_t)in[4], (int32_t)w[0],
+                            (int32_t)w[2], (int32_t)w[3], (int32_t)w[4], s[0], s[1], s[2], p[0], p[1], p[2], d[0], d[1], d[2]};
+  r.key.code = code;
+  r.sizes = sizes_of(r.key);
+  return true;
+}
+
+bool bias_fits(const MaybeTensor& b, const Tensor& x, int64_t channels) {
+  return !b.has_value() || (b->dim() == 1 && b->size(0) == channels && b->scalar_type() == x.scalar_type() && b->device() == x.device() &&
+                            b->stride(0) == 1);
+}
+
+// The gate of the forward (conv3d.is_supported), and with `all` of both gradients too (is_supported_all).
+bool conv_gate(const Tensor& x, const Tensor& w, const MaybeTensor& bias, const int32_t s[3], const int32_t p[3], const int32_t d[3],
+               bool all, Problem& prob, int64_t more_channels = 0) {
+  if (x.dim() != 5 || w.dim() != 5 || !on_gpu(x) || !on_gpu(w) || x.device() != w.device()) return false;
+  if (x.scalar_type() != w.scalar_type() || x.size(1) + more_channels != w.size(1)) return false;
+  if (!bias_fits(bias, x, w.size(0))) return false;
+  const int64_t in[5] = {x.size(0), w.size(1), x.size(2), x.size(3), x.size(4)};
+  if (!make_problem(in, w.sizes(), s, p, d, code_of(x.scalar_type()), prob)) return false;
+  if (all)
+    for (int i = 0; i < 3; ++i)
+      if (s[i] != 1 || p[i] > d[i] * ((int32_t)w.size(2 + i) - 1)) return false;
+  return true;
+}
+
+bool packed_fits(const Tensor& packed, size_t want, const Tensor& like) {
+  return want != 0 && packed.scalar_type() == at::kByte && packed.dim() == 1 && packed.is_contiguous() && packed.device() == like.device() &&
+         (size_t)packed.numel() == want;
+}
+
+struct ConvResult {
+  Tensor y, partials;
+  int32_t records = 0;
+};
+
+// x (and second: the channels after x's), dense channels-last, gated.
+ConvResult launch_conv(const Problem& prob, const Tensor& x, const Tensor& second, const Tensor& w, const Tensor& bias, const Tensor& packed,
+                       int groups) {
+  c10::OptionalDeviceGuard guard(x.device());
+  ConvResult r;
+  r.y = volume({prob.key.d.n, prob.key.d.cout, prob.out[0], prob.out[1], prob.out[2]}, x, x.scalar_type());
+  const Tensor ws = bytes(prob.sizes->work[0] - (packed.defined() ? prob.sizes->packed[0] : 0), x);
+  const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+  const uint32_t flags = packed.defined() ? SFH_FLAG_WEIGHT_PACKED : 0;
+  const void* wp = packed.defined() ? ptr(packed) : ptr(w);
+  const int64_t* strides = packed.defined() ? nullptr : w.strides().data();
+  void* st = stream_of(x);
+  int rc = SFH_ERR_UNSUPPORTED;
+  r.records = groups > 0 ? prob.records(groups) : 0;
+  if (r.records > 0) {
+    r.partials = at::empty({(int64_t)prob.key.d.n * r.records * groups * 4}, x.options().dtype(at::kFloat));
+    rc = second.defined()
+             ? sfh_conv3d_fwd_pair(prob.desc(), prob.key.code, ptr(x), ptr(second), (int32_t)x.size(1), wp, strides, ptr(bias), out_ptr(r.y),
+                                   out_ptr(ws), ws_bytes, flags, groups, (float*)out_ptr(r.partials), (size_t)r.partials.numel() * 4, st)
+             : sfh_conv3d_fwd_gn(prob.desc(), prob.key.code, ptr(x), wp, strides, ptr(bias), out_ptr(r.y), out_ptr(ws), ws_bytes, flags, groups,
+                                 (float*)out_ptr(r.partials), (size_t)r.partials.numel() * 4, st);
+  }
+  if (rc == SFH_ERR_UNSUPPORTED) {  // no statistics asked for, or not offered: the plain launch
+    r.records = 0;
+    rc = second.defined() ? sfh_conv3d_fwd_pair(prob.desc(), prob.key.code, ptr(x), ptr(second), (int32_t)x.size(1), wp, strides, ptr(bias),
+                                                out_ptr(r.y), out_ptr(ws), ws_bytes, flags, 0, nullptr, 0, st)
+                          : sfh_conv3d_fwd(prob.desc(), prob.key.code, ptr(x), wp, strides, ptr(bias), out_ptr(r.y), out_ptr(ws), ws_bytes, flags, st);
+  }
+  check(rc, "conv3d_forward");
+  return r;
+}
+
+// The data gradient; `first` > 0: as two tensors cut at that channel.
+std::pair<Tensor, Tensor> launch_dgrad(const Problem& prob, const Tensor& gy, const Tensor& w, const Tensor& packed, int64_t first) {
+  c10::OptionalDeviceGuard guard(gy.device());
+  const auto& d = prob.key.d;
+  const int64_t c1 = first > 0 ? first : d.cin;
+  Tensor gx = volume({d.n, c1, d.in_d, d.in_h, d.in_w}, gy, gy.scalar_type()), gx2;
+  if (first > 0) gx2 = volume({d.n, d.cin - first, d.in_d, d.in_h, d.in_w}, gy, gy.scalar_type());
+  const Tensor ws = bytes(prob.sizes->work[1] - (packed.defined() ? prob.sizes->packed[1] : 0), gy);
+  const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+  const uint32_t flags = packed.defined() ? SFH_FLAG_WEIGHT_PACKED : 0;
+  const void* wp = packed.defined() ? ptr(packed) : ptr(w);
+  const int64_t* strides = packed.defined() ? nullptr : w.strides().data();
+  const int rc = first > 0 ? sfh_conv3d_dgrad_pair(prob.desc(), prob.key.code, ptr(gy), wp, strides, out_ptr(gx), out_ptr(gx2), (int32_t)first,
+                                                   out_ptr(ws), ws_bytes, flags, stream_of(gy))
+                           : sfh_conv3d_dgrad(prob.desc(), prob.key.code, ptr(gy), wp, strides, out_ptr(gx), out_ptr(ws), ws_bytes, flags, stream_of(gy));
+  check(rc, "conv3d_backward_data");
+  return {gx, gx2};
+}
+
+// The weight gradient in the operands' dtype or, with `fp32`, unrounded where the kernel that serves the problem has that
+// form (else widened afterwards: what autocast's cast node would have done).
+Tensor launch_wgrad(const Problem& prob, const Tensor& x, const Tensor& second, const Tensor& gy, bool fp32) {
+  c10::OptionalDeviceGuard guard(gy.device());
+  const auto& d = prob.key.d;
+  const bool widen = fp32 && gy.scalar_type() != at::kFloat;
+  const Tensor ws = bytes(prob.sizes->work[2], gy);
+  const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+  for (int attempt = widen ? 0 : 1; attempt < 2; ++attempt) {
+    Tensor gw = volume({d.cout, d.cin, d.kd, d.kh, d.kw}, gy, attempt == 0 ? at::kFloat : gy.scalar_type());
+    const uint32_t flags = attempt == 0 ? SFH_FLAG_GRAD_FP32 : 0;
+    const int rc = second.defined() ? sfh_conv3d_wgrad_pair(prob.desc(), prob.key.code, ptr(x), ptr(second), (int32_t)x.size(1), ptr(gy), out_ptr(gw),
+                                                            out_ptr(ws), ws_bytes, flags, stream_of(gy))
+                                    : sfh_conv3d_wgrad(prob.desc(), prob.key.code, ptr(x), ptr(gy), out_ptr(gw), out_ptr(ws), ws_bytes, flags, stream_of(gy));
+    if (attempt == 0 && rc == SFH_ERR_UNSUPPORTED) continue;
+    check(rc, "conv3d_backward_weight");
+    return widen && attempt == 1 ? gw.to(at::kFloat) : gw;
+  }
+  return Tensor();
+}
+
+// grad_output.sum((0, 2, 3, 4)) in a fixed order
+Tensor launch_bias_grad(const Tensor& gy, at::ScalarType dtype) {
+  c10::OptionalDeviceGuard guard(gy.device());
+  const int64_t c = gy.size(1), rows = gy.numel() / c;
+  Tensor gb = at::empty({c}, gy.options().dtype(dtype));
+  const Tensor ws = bytes(sfh_bias_grad_workspace_bytes(rows, (int32_t)c), gy);
+  check(sfh_bias_grad(code_of(gy.scalar_type()), code_of(dtype), ptr(gy), rows, (int32_t)c, out_ptr(gb), out_ptr(ws),
+                      ws.defined() ? (size_t)ws.numel() : 0, stream_of(gy)), "bias_grad");
+  return gb;
+}
+
+// ---- autograd ------------------------------------------------------------------------------------------------------------
+// A node whose gradients are computed by launches: under create_graph its results refuse to be differentiated again.
+struct LaunchNode : public Node {
+  virtual variable_list backward(variable_list& grads) = 0;
+  variable_list apply(variable_list&& grads) override {
+    bool twice = false;
+    if (at::GradMode::is_enabled())
+      for (const auto& g : grads) twice = twice || (g.defined() && g.requires_grad());
+    variable_list outs;
+    {
+      at::AutoGradMode no_grad(false);
+      outs = backward(grads);
+    }
+    if (!twice) return outs;
+    variable_list marked;
+    for (const auto& o : outs) {
+      if (!o.defined()) {
+        marked.push_back(o);
+        continue;
+      }
+      auto refuse = std::make_shared<torch::autograd::DelayedError>("trying to differentiate twice a function that was marked with @once_differentiable", 1);
+      marked.push_back((*refuse)({o.detach().set_requires_grad(true)})[0]);
+    }
+    return marked;
+  }
+};
+
+template <typename N> std::shared_ptr<N> new_node() { return {new N(), torch::autograd::deleteNode}; }
+
+bool wants_grad(std::initializer_list<const Tensor*> ts) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor* t : ts)
+    if (t != nullptr && t->defined() && t->requires_grad()) return true;
+  return false;
+}
+
+Tensor or_none(const MaybeTensor& t) { return t.has_value() ? *t : Tensor(); }
+
+// The convolution over x, or over the pair (x, second).  Edges: x, weight, bias, second.  In the depth-shard form the
+// tensors that are saved are slabs of which x and second are the depth interiors.
+struct ConvNode : public LaunchNode {
+  SavedVariable x, second, w, packed_dgrad;
+  Tensor param;             // the parameter whose weight gradient waits for the end of the pass (undefined: computed here)
+  int family = 0;
+  bool early = false, pair = false, has_bias = false, master = false;
+  at::ScalarType bias_dtype = at::kFloat;
+  int32_t s[3], p[3], d[3];
+  int64_t halo = 0, depth = 0, first_channels = 0;
+  std::vector<int64_t> in_sizes;
+
+  std::string name() const override { return "ScaffoldConv3dBackward"; }
+  void release_variables() override {
+    x.reset_data(); second.reset_data(); w.reset_data(); packed_dgrad.reset_data();
+    param.reset();
+  }
+  variable_list backward(variable_list& grads) override {
+    variable_list out(4);
+    if (!grads[0].defined()) return out;
+    const Tensor xs = x.unpack(), x2 = second.unpack(), wt = w.unpack(), packed = packed_dgrad.unpack();
+    const Tensor gy = dense(grads[0]);
+    Problem prob;
+    TORCH_INTERNAL_ASSERT(make_problem(in_sizes, wt.sizes(), s, p, d, code_of(gy.scalar_type()), prob));
+    const bool need_x = task_should_compute_output(0), need_w = task_should_compute_output(1), need_b = has_bias && task_should_compute_output(2),
+               need_2 = pair && task_should_compute_output(3);
+    if (need_x || need_2) {
+      auto gx = launch_dgrad(prob, gy, wt, packed, pair ? first_channels : 0);
+      if (halo > 0) {
+        gx.first = gx.first.narrow(2, halo, depth);
+        if (pair) gx.second = gx.second.narrow(2, halo, depth);
+      }
+      if (need_x) out[0] = gx.first;
+      if (need_2) out[3] = gx.second;
+    }
+    if (need_w && need_b && !pair && prob.sizes->work_bias > 0) {
+      // both parameter gradients from one pass over the output gradient (the 1x1x1 head)
+      c10::OptionalDeviceGuard guard(gy.device());
+      const auto& pd = prob.key.d;
+      const auto dtype = master ? at::kFloat : gy.scalar_type();
+      Tensor gw = volume({pd.cout, pd.cin, pd.kd, pd.kh, pd.kw}, gy, dtype), gb = at::empty({pd.cout}, gy.options().dtype(dtype));
+      const Tensor ws = bytes(prob.sizes->work_bias, gy);
+      const int rc = sfh_conv3d_wgrad_bias(prob.desc(), prob.key.code, ptr(xs), ptr(gy), out_ptr(gw), out_ptr(gb), out_ptr(ws), prob.sizes->work_bias,
+                                           dtype != gy.scalar_type() ? SFH_FLAG_GRAD_FP32 : 0, stream_of(gy));
+      if (rc != SFH_ERR_UNSUPPORTED) {
+        check(rc, "conv3d_backward_weight_bias");
+        out[1] = gw;
+        out[2] = gb.scalar_type() == bias_dtype ? gb : gb.to(bias_dtype);
+        return out;
+      }
+    }
+    if (need_w && param.defined()) {
+      py::gil_scoped_acquire gil;
+      py::reinterpret_borrow<py::function>(g_queue_weight)(py::cast(param), py::cast(xs), pair ? py::cast(x2) : py::none(), py::cast(gy),
+                                                           py::make_tuple(p[0], p[1], p[2]), master, family, early);
+    } else if (need_w) {
+      out[1] = launch_wgrad(prob, xs, x2, gy, master);
+    }
+    if (need_b) out[2] = launch_bias_grad(gy, bias_dtype);
+    return out;
+  }
+};
+
+// Records the node of y = conv(x[, second]) that a launch has just produced.  `x_read` / `second_read`: the tensors the
+// kernels read (slabs in the depth-shard form, halo > 0; else x and second themselves).
+void record_conv(Tensor y, const Tensor& x, const Tensor& weight, const MaybeTensor& bias, const MaybeTensor& second, const Tensor& x_read,
+                 const MaybeTensor& second_read, const Tensor& w, const MaybeTensor& packed_dgrad, int64_t halo, py::handle stride,
+                 py::handle padding, py::handle dilation, bool master, int family, bool early) {
+  const Tensor b = or_none(bias), x2 = or_none(second);
+  if (!wants_grad({&x, &weight, &b, &x2})) return;
+  auto node = new_node<ConvNode>();
+  TORCH_CHECK_VALUE(three(stride, node->s) && three(padding, node->p) && three(dilation, node->d), "stride, padding and dilation are ints or three ints");
+  node->set_next_edges(torch::autograd::collect_next_edges(x, weight, b, x2));
+  const Tensor read2 = or_none(second_read);
+  node->x = SavedVariable(x_read, false);
+  node->second = SavedVariable(read2, false);
+  node->w = SavedVariable(w, false);
+  node->packed_dgrad = SavedVariable(or_none(packed_dgrad), false);
+  node->pair = x2.defined();
+  node->has_bias = b.defined();
+  if (b.defined()) node->bias_dtype = b.scalar_type();
+  node->master = master;
+  node->halo = halo;
+  node->depth = x.size(2);
+  node->first_channels = x_read.size(1);
+  node->in_sizes = x_read.sizes().vec();
+  if (read2.defined()) node->in_sizes[1] += read2.size(1);
+  if (family > 0) node->param = weight;
+  node->family = family;
+  node->early = early;
+  torch::autograd::set_history(y, node);
+}
+
+py::object tensor_or_none(const Tensor& t) { return t.defined() ? py::cast(t) : py::none(); }
+
+// conv3d.conv3d_forward / conv3d_forward_pair: (y, partials, records), or None for a call that is not served as it stands.
+py::object conv_forward(const Tensor& x, const Tensor& w, const MaybeTensor& bias, py::handle stride, py::handle padding, py::handle dilation,
+                        const MaybeTensor& packed, int gn_groups, const MaybeTensor& second) {
+  int32_t s[3], p[3], d[3];
+  if (!three(stride, s) || !three(padding, p) || !three(dilation, d)) return py::none();
+  Problem prob;
+  if (!conv_gate(x, w, bias, s, p, d, false, prob, second.has_value() && second->dim() == 5 ? second->size(1) : 0)) return py::none();
+  if (packed.has_value() && !packed_fits(*packed, prob.sizes->packed[0], x)) return py::none();
+  if (second.has_value() && (second->dim() != 5 || !on_gpu(*second) || second->device() != x.device() || second->scalar_type() != x.scalar_type() ||
+                             second->size(0) != x.size(0) || second->size(2) != x.size(2) || second->size(3) != x.size(3) || second->size(4) != x.size(4)))
+    return py::none();
+  const ConvResult r = launch_conv(prob, dense(x), second.has_value() ? dense(*second) : Tensor(), w, or_none(bias), or_none(packed), gn_groups);
+  return py::make_tuple(r.y, tensor_or_none(r.records > 0 ? r.partials : Tensor()), r.records);
+}
+
+// conv3d.is_supported_all for exact argument kinds (False also where the Python gate has to look closer)
+bool conv_supported(const Tensor& x, const Tensor& w, const MaybeTensor& bias, py::handle stride, py::handle padding, py::handle dilation, bool all) {
+  int32_t s[3], p[3], d[3];
+  Problem prob;
+  return three(stride, s) && three(padding, p) && three(dilation, d) && conv_gate(x, w, bias, s, p, d, all, prob);
+}
+
+// conv3d.conv3d_backward_data
+py::object conv_backward_data(const Tensor& grad_output, const Tensor& w, at::IntArrayRef in_sizes, py::handle stride, py::handle padding,
+                              py::handle dilation, const MaybeTensor& packed) {
+  int32_t s[3], p[3], d[3];
+  if (!three(stride, s) || !three(padding, p) || !three(dilation, d)) return py::none();
+  if (grad_output.dim() != 5 || w.dim() != 5 || in_sizes.size() != 5 || !on_gpu(grad_output) || !on_gpu(w)) return py::none();
+  if (grad_output.device() != w.device() || grad_output.scalar_type() != w.scalar_type() || in_sizes[1] != w.size(1)) return py::none();
+  for (int i = 0; i < 3; ++i)
+    if (s[i] != 1 || p[i] > d[i] * ((int32_t)w.size(2 + i) - 1)) return py::none();
+  Problem prob;
+  if (!make_problem(in_sizes, w.sizes(), s, p, d, code_of(w.scalar_type()), prob)) return py::none();
+  if (grad_output.size(0) != prob.key.d.n || grad_output.size(1) != prob.key.d.cout) return py::none();
+  for (int i = 0; i < 3; ++i)
+    if (grad_output.size(2 + i) != prob.out[i]) return py::none();
+  if (packed.has_value() && !packed_fits(*packed, prob.sizes->packed[1], grad_output)) return py::none();
+  return py::cast(launch_dgrad(prob, dense(grad_output), w, or_none(packed), 0).first);
+}
+
+// conv3d.conv3d_backward_weight in the operands' dtype
+py::object conv_backward_weight(const Tensor& x, at::IntArrayRef w_sizes, const Tensor& grad_output, py::handle stride, py::handle padding,
+                                py::handle dilation) {
+  int32_t s[3], p[3], d[3];
+  if (!three(stride, s) || !three(padding, p) || !three(dilation, d)) return py::none();
+  if (x.dim() != 5 || grad_output.dim() != 5 || w_sizes.size() != 5 || !on_gpu(x) || !on_gpu(grad_output)) return py::none();
+  if (x.device() != grad_output.device() || x.scalar_type() != grad_output.scalar_type() || x.size(1) != w_sizes[1]) return py::none();
+  Problem prob;
+  if (!make_problem(x.sizes(), w_sizes, s, p, d, code_of(x.scalar_type()), prob)) return py::none();
+  if (grad_output.size(0) != prob.key.d.n || grad_output.size(1) != prob.key.d.cout) return py::none();
+  for (int i = 0; i < 3; ++i)
+    if (grad_output.size(2 + i) != prob.out[i]) return py::none();
+  return py::cast(launch_wgrad(prob, dense(x), Tensor(), dense(grad_output), false));
+}
+
+// ---- the 2x2x2-like transposed convolution (kernel == stride) ------------------------------------------------------------
+struct ConvTransposeNode : public LaunchNode {  // edges: x, weight, bias
+  SavedVariable x, w, packed_fwd;
+  int32_t k[3];
+  bool has_bias = false, master = false;
+  at::ScalarType bias_dtype = at::kFloat;
+  std::string name() const override { return "ScaffoldConvTranspose3dBackward"; }
+  void release_variables() override { x.reset_data(); w.reset_data(); packed_fwd.reset_data(); }
+  variable_list backward(variable_list& grads) override {
+    variable_list out(3);
+    if (!grads[0].defined()) return out;
+    const Tensor xs = x.unpack(), wt = w.unpack(), packed = packed_fwd.unpack();
+    const Tensor gy = dense(grads[0]);
+    if (gy.numel() == 0) {
+      const auto dtype = master ? at::kFloat : gy.scalar_type();
+      out[0] = volume(xs.sizes(), gy, gy.scalar_type());
+      out[1] = volume(wt.sizes(), gy, dtype).zero_();
+      if (has_bias) out[2] = at::zeros({wt.size(1)}, gy.options().dtype(bias_dtype));
+      return out;
+    }
+    // the stride-k convolution over gy whose forward is the data gradient and whose weight gradient is this one's
+    const int32_t zero[3] = {0, 0, 0}, one[3] = {1, 1, 1};
+    Problem prob;
+    TORCH_INTERNAL_ASSERT(make_problem(gy.sizes(), wt.sizes(), k, zero, one, code_of(gy.scalar_type()), prob));
+    const bool need_w = task_should_compute_output(1), need_b = has_bias && task_should_compute_output(2);
+    if (task_should_compute_output(0)) out[0] = launch_conv(prob, gy, Tensor(), wt, Tensor(), packed, 0).y;
+    if (need_w && need_b) {
+      c10::OptionalDeviceGuard guard(gy.device());
+      const sfh_convT3d_desc td{(int32_t)xs.size(0), (int32_t)xs.size(1), (int32_t)xs.size(2), (int32_t)xs.size(3), (int32_t)xs.size(4),
+                                (int32_t)wt.size(1), k[0], k[1], k[2]};
+      const size_t need = sfh_convT3d_wgrad_bias_workspace_bytes(&td, prob.key.code);
+      if (need > 0) {
+        const auto dtype = master ? at::kFloat : gy.scalar_type();
+        Tensor gw = volume(wt.sizes(), gy, dtype), gb = at::empty({wt.size(1)}, gy.options().dtype(dtype));
+        const Tensor ws = bytes(need, gy);
+        const int rc = sfh_convT3d_wgrad_bias(&td, prob.key.code, ptr(xs), ptr(gy), out_ptr(gw), out_ptr(gb), out_ptr(ws), need,
+                                              dtype != gy.scalar_type() ? SFH_FLAG_GRAD_FP32 : 0, stream_of(gy));
+        if (rc != SFH_ERR_UNSUPPORTED) {
+          check(rc, "conv_transpose3d_backward_weight_bias");
+          out[1] = gw;
+          out[2] = gb.scalar_type() == bias_dtype ? gb : gb.to(bias_dtype);
+          return out;
+        }
+      }
+    }
+    if (need_w) out[1] = launch_wgrad(prob, gy, Tensor(), xs, master);
+    if (need_b) out[2] = launch_bias_grad(gy, bias_dtype);
+    return out;
+  }
+};
+
+// FastConvTranspose3d: y (and the slab it lies in, or None), or None for a call that is not served as it stands.  `weight` /
+// `bias` receive gradients, `w` / `b` are what the kernels read; the packed forms are those of the stride-k convolution.
+py::object conv_transpose(const Tensor& x_in, const Tensor& weight, const MaybeTensor& bias, const Tensor& w, const MaybeTensor& b, py::handle stride,
+                          const MaybeTensor& packed_fwd, const MaybeTensor& packed_dgrad, int64_t halo, bool master) {
+  int32_t k[3];
+  if (!three(stride, k) || x_in.dim() != 5 || w.dim() != 5 || !on_gpu(x_in) || !on_gpu(w) || x_in.device() != w.device()) return py::none();
+  if (x_in.scalar_type() != w.scalar_type() || x_in.size(1) != w.size(0) || !bias_fits(b, x_in, w.size(1))) return py::none();
+  int64_t big[5] = {x_in.size(0), w.size(1), 0, 0, 0};
+  for (int i = 0; i < 3; ++i) {
+    if (k[i] < 1 || w.size(2 + i) != k[i] || x_in.size(2 + i) < 1) return py::none();
+    big[2 + i] = x_in.size(2 + i) * k[i];
+  }
+  const int32_t zero[3] = {0, 0, 0}, one[3] = {1, 1, 1};
+  Problem prob;
+  const bool empty = big[0] == 0;  // a batch of no samples: an empty result, zero parameter gradients
+  if (empty && code_of(x_in.scalar_type()) < 0) return py::none();
+  if (!empty && !make_problem(big, w.sizes(), k, zero, one, code_of(x_in.scalar_type()), prob)) return py::none();
+  if (!empty && packed_dgrad.has_value() && !packed_fits(*packed_dgrad, prob.sizes->packed[1], x_in)) return py::none();
+  if (!empty && packed_fwd.has_value() && !packed_fits(*packed_fwd, prob.sizes->packed[0], x_in)) return py::none();
+  const Tensor weight_b = or_none(bias);
+  const bool graph = wants_grad({&x_in, &weight, &weight_b});
+  Tensor x = x_in, y, slab;
+  if (empty) {
+    y = volume(big, x, x.scalar_type());
+  } else {
+    at::AutoGradMode no_grad(false);
+    x = dense(x_in);
+    c10::OptionalDeviceGuard guard(x.device());
+    const sfh_convT3d_desc td{(int32_t)x.size(0), (int32_t)x.size(1), (int32_t)x.size(2), (int32_t)x.size(3), (int32_t)x.size(4),
+                              (int32_t)w.size(1), k[0], k[1], k[2]};
+    const int code = prob.key.code;
+    const Tensor ws = packed_dgrad.has_value() ? Tensor() : bytes(sfh_convT3d_fwd_workspace_bytes(&td, code), x);
+    const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+    const void* wp = packed_dgrad.has_value() ? ptr(*packed_dgrad) : ptr(w);
+    const int64_t* strides = packed_dgrad.has_value() ? nullptr : w.strides().data();
+    const uint32_t flags = packed_dgrad.has_value() ? SFH_FLAG_WEIGHT_PACKED : 0;
+    int rc = SFH_ERR_UNSUPPORTED;
+    if (halo > 0 && x.size(0) == 1) {
+      slab = volume({1, big[1], big[2] + 2 * halo, big[3], big[4]}, x, x.scalar_type());
+      rc = sfh_convT3d_fwd_slab(&td, code, ptr(x), wp, strides, ptr(or_none(b)), out_ptr(slab), halo * big[3] * big[4] * big[1], out_ptr(ws), ws_bytes,
+                                flags, stream_of(x));
+      if (rc != SFH_ERR_UNSUPPORTED) y = slab.narrow(2, halo, big[2]);
+    }
+    if (rc == SFH_ERR_UNSUPPORTED) {
+      slab = Tensor();
+      y = volume(big, x, x.scalar_type());
+      rc = sfh_convT3d_fwd(&td, code, ptr(x), wp, strides, ptr(or_none(b)), out_ptr(y), out_ptr(ws), ws_bytes, flags, stream_of(x));
+    }
+    check(rc, "conv_transpose3d_forward");
+  }
+  if (graph) {
+    auto node = new_node<ConvTransposeNode>();
+    node->set_next_edges(torch::autograd::collect_next_edges(x_in, weight, weight_b));
+    node->x = SavedVariable(x, false);
+    node->w = SavedVariable(w, false);
+    node->packed_fwd = SavedVariable(or_none(packed_fwd), false);
+    std::memcpy(node->k, k, sizeof(k));
+    node->has_bias = weight_b.defined();
+    if (weight_b.defined()) node->bias_dtype = weight_b.scalar_type();
+    node->master = master;
+    if (slab.defined()) y = y.detach();  // a tensor of its own: a view would keep the slab as its differentiable base
+    torch::autograd::set_history(y, node);
+  }
+  return py::make_tuple(y, tensor_or_none(slab));
+}
+
+// ---- GroupNorm -----------------------------------------------------------------------------------------------------------
+struct GroupNormNode : public LaunchNode {  // edges: input, weight, bias
+  SavedVariable input, weight, bias, stats;
+  int groups = 1;
+  bool relu = false;
+  std::string name() const override { return "ScaffoldGroupNormBackward"; }
+  void release_variables() override { input.reset_data(); weight.reset_data(); bias.reset_data(); stats.reset_data(); }
+  variable_list backward(variable_list& grads) override {
+    variable_list out(3);
+    if (!grads[0].defined()) return out;
+    const Tensor x = dense(input.unpack()), st = stats.unpack();
+    Tensor w = weight.unpack(), b = bias.unpack();
+    Tensor gy = dense(grads[0]);
+    if (gy.scalar_type() != x.scalar_type() && gy.scalar_type() != at::kFloat) gy = gy.to(x.scalar_type());
+    const Tensor w_in = w, b_in = b;
+    if (w.defined()) w = w.contiguous();
+    if (b.defined()) b = b.contiguous();
+    if (w.defined() && b.defined() && w.scalar_type() != b.scalar_type()) b = b.to(w.scalar_type());
+    c10::OptionalDeviceGuard guard(x.device());
+    const int64_t c = x.size(1), n = x.size(0);
+    const sfh_groupnorm_desc d{(int32_t)n, (int32_t)c, groups, relu ? 1 : 0, x.numel() / (n * c), 0.f};
+    const int code = code_of(x.scalar_type());
+    Tensor dx = volume(x.sizes(), x, x.scalar_type()), dw, db;
+    if (w.defined()) dw = at::empty({c}, x.options().dtype(at::kFloat));
+    if (b.defined()) db = at::empty({c}, x.options().dtype(at::kFloat));
+    const Tensor ws = bytes(sfh_groupnorm_bwd_workspace_bytes(&d, code), x);
+    const float* mean = (const float*)ptr(st);
+    check(sfh_groupnorm_bwd(&d, code, code_of(gy.scalar_type()), code_of(w.defined() ? w.scalar_type() : b.defined() ? b.scalar_type() : x.scalar_type()),
+                            ptr(gy), ptr(x), ptr(w), ptr(b), mean, mean + n * groups, out_ptr(dx), (float*)out_ptr(dw), (float*)out_ptr(db), out_ptr(ws),
+                            ws.defined() ? (size_t)ws.numel() : 0, stream_of(x)), "group_norm_backward");
+    if (task_should_compute_output(0)) out[0] = dx;
+    if (dw.defined() && task_should_compute_output(1)) out[1] = dw.scalar_type() == w_in.scalar_type() ? dw : dw.to(w_in.scalar_type());
+    if (db.defined() && task_should_compute_output(2)) out[2] = db.scalar_type() == b_in.scalar_type() ? db : db.to(b_in.scalar_type());
+    return out;
+  }
+};
+
+// groupnorm.group_norm outside torch.compile: (y, slab or None), or None for a call that is not served as it stands.
+// `out_dtype`: None or "stock" (what F.group_norm would return: fp32 inside autocast); `partials`: Welford records the
+// producer of `input` left for these very bits, `records` per sample.
+py::object group_norm(const Tensor& input, int64_t groups, const MaybeTensor& weight, const MaybeTensor& bias, double eps, bool relu,
+                      std::optional<at::ScalarType> out_dtype, bool stock_dtype, int64_t halo, const MaybeTensor& partials, int32_t records) {
+  if (input.dim() != 5 || !on_gpu(input) || input.numel() == 0) return py::none();
+  const int code = code_of(input.scalar_type());
+  const int64_t n = input.size(0), c = input.size(1);
+  if (code < 0 || groups < 1 || c % groups != 0 || !input.is_contiguous(kCL3D)) return py::none();
+  const int64_t spatial = input.numel() / (n * c);
+  if ((c == groups && input.numel() == c) || n > INT32_MAX || c > INT32_MAX) return py::none();
+  const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
+  for (const MaybeTensor* t : {&weight, &bias}) {
+    if (!t->has_value()) continue;
+    if ((*t)->dim() != 1 || (*t)->numel() != c || (*t)->device() != input.device()) return py::none();
+    if ((*t)->scalar_type() != input.scalar_type() && ((*t)->scalar_type() != at::kFloat || !autocast)) return py::none();
+  }
+  at::ScalarType odt = out_dtype.value_or(input.scalar_type());
+  if (stock_dtype) odt = input.scalar_type() != at::kFloat && autocast ? at::kFloat : input.scalar_type();
+  if (code_of(odt) < 0) return py::none();
+  const Tensor w_in = or_none(weight), b_in = or_none(bias);
+  const bool graph = wants_grad({&input, &w_in, &b_in});
+  Tensor y, slab, stats;
+  {
+    at::AutoGradMode no_grad(false);
+    c10::OptionalDeviceGuard guard(input.device());
+    Tensor w = w_in.defined() ? w_in.contiguous() : w_in, b = b_in.defined() ? b_in.contiguous() : b_in;
+    if (w.defined() && b.defined() && w.scalar_type() != b.scalar_type()) b = b.to(w.scalar_type());
+    const int pcode = code_of(w.defined() ? w.scalar_type() : b.defined() ? b.scalar_type() : input.scalar_type());
+    stats = at::empty({2, n, groups}, input.options().dtype(at::kFloat));  // mean, rstd
+    float* mean = (float*)out_ptr(stats);
+    float* rstd = mean + n * groups;
+    const sfh_groupnorm_desc d{(int32_t)n, (int32_t)c, (int32_t)groups, relu ? 1 : 0, spatial, (float)eps};
+    void* st = stream_of(input);
+    int64_t halo_rows = 0;
+    if (halo > 0 && n == 1 && c10::elementSize(odt) == input.element_size()) {
+      slab = volume({1, c, input.size(2) + 2 * halo, input.size(3), input.size(4)}, input, odt);
+      y = slab.narrow(2, halo, input.size(2));
+      halo_rows = halo * input.size(3) * input.size(4);
+    } else {
+      y = volume(input.sizes(), input, odt);
+    }
+    int rc = SFH_ERR_UNSUPPORTED;
+    if (partials.has_value())
+      rc = sfh_groupnorm_fwd_from_partials(&d, code, code_of(odt), pcode, ptr(input), ptr(w), ptr(b), out_ptr(slab.defined() ? slab : y), halo_rows, mean,
+                                           rstd, (const float*)ptr(*partials), (size_t)partials->numel() * 4, records, st);
+    if (rc == SFH_ERR_UNSUPPORTED) {
+      const Tensor ws = bytes(sfh_groupnorm_fwd_workspace_bytes(&d, code), input);
+      const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+      if (slab.defined()) {
+        rc = sfh_groupnorm_fwd_slab(&d, code, code_of(odt), pcode, ptr(input), ptr(w), ptr(b), out_ptr(slab), halo_rows, mean, rstd, out_ptr(ws), ws_bytes, st);
+        if (rc == SFH_ERR_UNSUPPORTED) {  // channel counts off the vector path: the plain form
+          slab = Tensor();
+          y = volume(input.sizes(), input, odt);
+        }
+      }
+      if (rc == SFH_ERR_UNSUPPORTED)
+        rc = sfh_groupnorm_fwd(&d, code, code_of(odt), pcode, ptr(input), ptr(w), ptr(b), out_ptr(y), mean, rstd, out_ptr(ws), ws_bytes, st);
+    }
+    check(rc, "group_norm");
+  }
+  if (graph) {
+    auto node = new_node<GroupNormNode>();
+    node->set_next_edges(torch::autograd::collect_next_edges(input, w_in, b_in));
+    node->input = SavedVariable(input, false);
+    node->weight = SavedVariable(w_in, false);
+    node->bias = SavedVariable(b_in, false);
+    node->stats = SavedVariable(stats, false);
+    node->groups = (int)groups;
+    node->relu = relu;
+    if (slab.defined()) y = y.detach();
+    torch::autograd::set_history(y, node);
+  }
+  return py::make_tuple(y, tensor_or_none(slab));
+}
+
+// ---- MaxPool3d(2) --------------------------------------------------------------------------------------------------------
+struct MaxPoolNode : public LaunchNode {  // edge: x; the second output, where there is one, is an alias of x (the skip connection)
+  SavedVariable idx;
+  std::vector<int64_t> sizes;
+  std::string name() const override { return "ScaffoldMaxPool3dBackward"; }
+  void release_variables() override { idx.reset_data(); }
+  variable_list backward(variable_list& grads) override {
+    variable_list out(1);
+    const Tensor skip = grads.size() > 1 ? grads[1] : Tensor();
+    if (!grads[0].defined()) {
+      out[0] = skip;
+      return out;
+    }
+    const Tensor gy = dense(grads[0]), ix = idx.unpack();
+    c10::OptionalDeviceGuard guard(gy.device());
+    Tensor gx = volume(sizes, gy, gy.scalar_type());
+    const sfh_pool_desc d{(int32_t)sizes[0], (int32_t)sizes[1], (int32_t)sizes[2], (int32_t)sizes[3], (int32_t)sizes[4]};
+    const int code = code_of(gy.scalar_type());
+    if (skip.defined()) {
+      Tensor gs = dense(skip);
+      if (gs.scalar_type() != gy.scalar_type()) gs = gs.to(gy.scalar_type());
+      check(sfh_maxpool2_bwd_add(&d, code, ptr(gy), (const uint8_t*)ptr(ix), ptr(gs), out_ptr(gx), stream_of(gy)), "max_pool3d_2x backward");
+    } else {
+      check(sfh_maxpool2_bwd(&d, code, ptr(gy), (const uint8_t*)ptr(ix), out_ptr(gx), stream_of(gy)), "max_pool3d_2x backward");
+    }
+    out[0] = gx;
+    return out;
+  }
+};
+
+// pooling.max_pool3d_2x: (y, slab or None[, alias of x]), or None for a call that is not served.
+py::object max_pool(const Tensor& x_in, int64_t halo, bool with_skip) {
+  if (x_in.dim() != 5 || !on_gpu(x_in) || code_of(x_in.scalar_type()) < 0 || x_in.size(1) < 1) return py::none();
+  for (int i = 2; i < 5; ++i)
+    if (x_in.size(i) < 1) return py::none();
+  const bool graph = wants_grad({&x_in});
+  Tensor y, slab, idx, skip;
+  const auto z = x_in.sizes();
+  {
+    at::AutoGradMode no_grad(false);
+    const Tensor x = dense(x_in);
+    c10::OptionalDeviceGuard guard(x.device());
+    const int64_t n = z[0], c = z[1], d2 = z[2] / 2, h2 = z[3] / 2, w2 = z[4] / 2;
+    idx = at::empty({n, d2, h2, w2, c}, x.options().dtype(at::kByte));
+    const sfh_pool_desc d{(int32_t)n, (int32_t)c, (int32_t)z[2], (int32_t)z[3], (int32_t)z[4]};
+    const int code = code_of(x.scalar_type());
+    int rc = SFH_ERR_UNSUPPORTED;
+    if (halo > 0 && n == 1 && d2 > 0 && h2 > 0 && w2 > 0) {
+      slab = volume({1, c, d2 + 2 * halo, h2, w2}, x, x.scalar_type());
+      rc = sfh_maxpool2_fwd_slab(&d, code, ptr(x), out_ptr(slab), halo * h2 * w2 * c, (uint8_t*)out_ptr(idx), stream_of(x));
+      if (rc != SFH_ERR_UNSUPPORTED) y = slab.narrow(2, halo, d2);
+    }
+    if (rc == SFH_ERR_UNSUPPORTED) {
+      slab = Tensor();
+      y = volume({n, c, d2, h2, w2}, x, x.scalar_type());
+      rc = sfh_maxpool2_fwd(&d, code, ptr(x), out_ptr(y), (uint8_t*)out_ptr(idx), stream_of(x));
+    }
+    check(rc, "max_pool3d_2x");
+    if (with_skip) skip = x_in.detach();
+    if (graph && slab.defined()) y = y.detach();
+  }
+  if (graph) {
+    auto node = new_node<MaxPoolNode>();
+    node->set_next_edges(torch::autograd::collect_next_edges(x_in));
+    node->idx = SavedVariable(idx, false);
+    node->sizes = z.vec();
+    torch::autograd::set_history(y, node);
+    if (with_skip) torch::autograd::set_history(skip, node);
+  }
+  return with_skip ? py::make_tuple(y, tensor_or_none(slab), skip) : py::make_tuple(y, tensor_or_none(slab));
+}
+
+// ---- loss head -----------------------------------------------------------------------------------------------------------
+struct LossNode : public LaunchNode {  // edge: logits
+  SavedVariable logits, labels, stats, class_weight;
+  sfh_loss_desc d{};
+  std::string name() const override { return "ScaffoldCeDiceBackward"; }
+  void release_variables() override { logits.reset_data(); labels.reset_data(); stats.reset_data(); class_weight.reset_data(); }
+  variable_list backward(variable_list& grads) override {
+    variable_list out(1);
+    if (!grads[0].defined()) return out;
+    const Tensor x = logits.unpack(), lab = labels.unpack(), st = stats.unpack(), cw = class_weight.unpack();
+    c10::OptionalDeviceGuard guard(x.device());
+    const Tensor g = grads[0].to(x.device(), at::kFloat).reshape({1}).contiguous();
+    Tensor dx = volume(x.sizes(), x, x.scalar_type());
+    check(sfh_ce_dice_bwd(&d, code_of(x.scalar_type()), ptr(x), (const int64_t*)ptr(lab), (const float*)ptr(cw), (const float*)ptr(st), (const float*)ptr(g),
+                          out_ptr(dx), stream_of(x)), "ce_dice_loss backward");
+    out[0] = dx;
+    return out;
+  }
+};
+
+// losses.ce_dice_loss: the 0-dim loss, or None for a call that is not served.
+py::object ce_dice_loss(const Tensor& logits, const Tensor& labels, const MaybeTensor& class_weight, double eps) {
+  if (logits.dim() != 5 || labels.dim() != 4 || !on_gpu(logits) || labels.device() != logits.device() || labels.scalar_type() != at::kLong) return py::none();
+  const int code = code_of(logits.scalar_type());
+  const int64_t n = logits.size(0), c = logits.size(1);
+  if (code < 0 || c < 2 || c > 32 || logits.numel() == 0 || labels.size(0) != n) return py::none();
+  for (int i = 0; i < 3; ++i)
+    if (labels.size(1 + i) != logits.size(2 + i)) return py::none();
+  if (class_weight.has_value() && (class_weight->device() != logits.device() || class_weight->dim() != 1 || class_weight->size(0) != c ||
+                                   !at::isFloatingType(class_weight->scalar_type())))
+    return py::none();
+  const bool graph = wants_grad({&logits});
+  Tensor x, lab, cw, loss, stats;
+  const sfh_loss_desc d{(int32_t)n, (int32_t)c, logits.numel() / (n * c), (float)eps};
+  {
+    at::AutoGradMode no_grad(false);
+    c10::OptionalDeviceGuard guard(logits.device());
+    x = dense(logits);
+    lab = labels.contiguous();
+    if (class_weight.has_value()) cw = class_weight->detach().to(at::kFloat).contiguous();
+    loss = at::empty({}, x.options().dtype(at::kFloat));
+    stats = at::empty({n * 3 * c + 2}, x.options().dtype(at::kFloat));
+    const Tensor ws = bytes(sfh_ce_dice_workspace_bytes(&d), x);
+    check(sfh_ce_dice_fwd(&d, code, ptr(x), (const int64_t*)ptr(lab), (const float*)ptr(cw), (float*)out_ptr(loss), (float*)out_ptr(stats), out_ptr(ws),
+                          ws.defined() ? (size_t)ws.numel() : 0, stream_of(x)), "ce_dice_loss");
+  }
+  if (graph) {
+    auto node = new_node<LossNode>();
+    node->set_next_edges(torch::autograd::collect_next_edges(logits));
+    node->logits = SavedVariable(x, false);
+    node->labels = SavedVariable(lab, false);
+    node->stats = SavedVariable(stats, false);
+    node->class_weight = SavedVariable(cw, false);
+    node->d = d;
+    torch::autograd::set_history(loss, node);
+  }
+  return py::cast(loss);
+}
+
+void set_callbacks(py::object kernel_error, py::object note_device) {
+  g_kernel_error = kernel_error.release().ptr();
+  g_note_device = note_device.release().ptr();
+}
+void set_weight_queue(py::object queue) { g_queue_weight = queue.release().ptr(); }
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("set_callbacks", &set_callbacks);
+  m.def("set_weight_queue", &set_weight_queue);
+  m.def("conv_forward", &conv_forward);
+  m.def("conv_supported", &conv_supported);
+  m.def("conv_backward_data", &conv_backward_data);
+  m.def("conv_backward_weight", &conv_backward_weight);
+  m.def("record_conv", &record_conv);
+  m.def("conv_transpose", &conv_transpose);
+  m.def("group_norm", &group_norm);
+  m.def("max_pool", &max_pool);
+  m.def("ce_dice_loss", &ce_dice_loss);
+}

@@ -103,35 +103,8 @@ def _plan(input, num_groups: int, eps: float, activation, backward: bool):
     return plan
 
 
-def _launch_forward(L, desc, xcode, odt, need, input, weight, bias, out, slab, out_halo, mean, rstd):
-    """The statistics pass + normalisation; returns the status, or ``(status, output)`` when the slab form was refused and
-    a plain output took its place."""
-    ws = _lib.workspace(need, input.device)
-    if slab is None:
-        return L.sfh_groupnorm_fwd(
-            ctypes.byref(desc), xcode, _lib.dtype_code(odt), _lib.dtype_code(_param_dtype(weight, bias, input)),
-            _lib.ptr(input), _lib.ptr(weight), _lib.ptr(bias), _lib.ptr(out), _lib.ptr(mean), _lib.ptr(rstd),
-            _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream_ptr(input.device))
-    rc = L.sfh_groupnorm_fwd_slab(
-        ctypes.byref(desc), xcode, _lib.dtype_code(odt), _lib.dtype_code(_param_dtype(weight, bias, input)),
-        _lib.ptr(input), _lib.ptr(weight), _lib.ptr(bias), _lib.ptr(slab), out_halo * int(input.shape[3]) * int(input.shape[4]),
-        _lib.ptr(mean), _lib.ptr(rstd), _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream_ptr(input.device))
-    if rc == _lib.SFH_ERR_UNSUPPORTED:  # channel counts off the vector path: the plain form
-        out = torch.empty_like(input, dtype=odt)
-        rc = L.sfh_groupnorm_fwd(
-            ctypes.byref(desc), xcode, _lib.dtype_code(odt), _lib.dtype_code(_param_dtype(weight, bias, input)),
-            _lib.ptr(input), _lib.ptr(weight), _lib.ptr(bias), _lib.ptr(out), _lib.ptr(mean), _lib.ptr(rstd),
-            _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream_ptr(input.device))
-        return rc, out
-    return rc
-
-
-def _forward_impl(input, num_groups, weight, bias, eps, activation, out_dtype, out_halo: int = 0):
-    """The forward launch: ``(output, mean, rstd)``; shared by the registered operator and the eager autograd node.
-
-    ``out_halo > 0`` (one sample, output of the input's element width): the output is the interior view of a slab with
-    ``out_halo`` zero depth planes on each face, which rides along as ``output._sfh_slab = (slab, out_halo)`` for a
-    consumer that wants the extended tensor (a depth shard's convolution) without copying the interior."""
+def _forward_impl(input, num_groups, weight, bias, eps, activation, out_dtype):
+    """The registered operator's forward launch: ``(output, mean, rstd)``."""
     _validate(input, num_groups, weight, bias, activation)
     weight = None if weight is None else weight.contiguous()
     bias = None if bias is None else bias.contiguous()
@@ -139,14 +112,7 @@ def _forward_impl(input, num_groups, weight, bias, eps, activation, out_dtype, o
         bias = bias.to(weight.dtype)
     odt = out_dtype or input.dtype
     n = int(input.shape[0])
-    slab = None
-    if out_halo > 0 and n == 1 and odt.itemsize == input.dtype.itemsize and input.numel() > 0:
-        c, d, h, w = (int(v) for v in input.shape[1:])
-        slab = torch.empty((1, c, d + 2 * out_halo, h, w), dtype=odt, device=input.device, memory_format=_CL3D)
-        out = slab.narrow(2, out_halo, d)
-        out._sfh_slab = (slab, out_halo)
-    else:
-        out = torch.empty_like(input, dtype=odt)  # keeps the channels_last_3d strides
+    out = torch.empty_like(input, dtype=odt)  # keeps the channels_last_3d strides
     mean = torch.empty((n, num_groups), dtype=torch.float32, device=input.device)
     rstd = torch.empty((n, num_groups), dtype=torch.float32, device=input.device)
     if input.numel() == 0:
@@ -160,14 +126,14 @@ def _forward_impl(input, num_groups, weight, bias, eps, activation, out_dtype, o
             # the producer of `input` left per-group Welford records of these very bits: no statistics pass
             rc = L.sfh_groupnorm_fwd_from_partials(
                 ctypes.byref(desc), xcode, _lib.dtype_code(odt), _lib.dtype_code(_param_dtype(weight, bias, input)),
-                _lib.ptr(input), _lib.ptr(weight), _lib.ptr(bias), _lib.ptr(out if slab is None else slab),
-                0 if slab is None else out_halo * int(input.shape[3]) * int(input.shape[4]),
-                _lib.ptr(mean), _lib.ptr(rstd), _lib.ptr(given[0]), given[0].numel() * 4, given[1],
+                _lib.ptr(input), _lib.ptr(weight), _lib.ptr(bias), _lib.ptr(out), 0, _lib.ptr(mean), _lib.ptr(rstd), _lib.ptr(given[0]), given[0].numel() * 4, given[1],
                 _lib.stream_ptr(input.device))
         if rc == _lib.SFH_ERR_UNSUPPORTED:
-            rc = _launch_forward(L, desc, xcode, odt, need, input, weight, bias, out, slab, out_halo, mean, rstd)
-            if isinstance(rc, tuple):
-                rc, out = rc
+            ws = _lib.workspace(need, input.device)
+            rc = L.sfh_groupnorm_fwd(
+                ctypes.byref(desc), xcode, _lib.dtype_code(odt), _lib.dtype_code(_param_dtype(weight, bias, input)),
+                _lib.ptr(input), _lib.ptr(weight), _lib.ptr(bias), _lib.ptr(out), _lib.ptr(mean), _lib.ptr(rstd),
+                _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream_ptr(input.device))
     _lib.check(rc, "group_norm")
     return out, mean, rstd
 
@@ -286,29 +252,6 @@ def _gradients_through_the_op(ctx, grad_out, _grad_mean, _grad_rstd):
 torch.library.register_autograd("scaffold_gn::group_norm", _gradients_through_the_op, setup_context=_remember_for_backward)
 
 
-class _EagerGroupNormFn(torch.autograd.Function):
-    """The same two launches as the registered operators, as a plain autograd node: outside ``torch.compile`` the
-    operator registry's dispatch costs more host time per call than both launches together."""
-
-    @staticmethod
-    def forward(ctx, input, num_groups, weight, bias, eps, activation, out_dtype, out_halo=0):
-        out, mean, rstd = _forward_impl(input, num_groups, weight, bias, eps, activation, out_dtype, out_halo)
-        ctx.save_for_backward(input, weight, bias, mean, rstd)
-        ctx.num_groups = num_groups
-        ctx.activation = activation
-        return out
-
-    @staticmethod
-    @torch.autograd.function.once_differentiable
-    def backward(ctx, grad_out):
-        input, weight, bias, mean, rstd = ctx.saved_tensors
-        need_x, need_w, need_b = ctx.needs_input_grad[0], ctx.needs_input_grad[2], ctx.needs_input_grad[3]
-        if not (need_x or need_w or need_b):
-            return None, None, None, None, None, None, None, None
-        d_input, d_weight, d_bias = _backward_impl(grad_out, input, weight, bias, mean, rstd, ctx.num_groups, ctx.activation)
-        return (d_input if need_x else None, None, d_weight if need_w else None, d_bias if need_b else None, None, None, None, None)
-
-
 # ---------------------------------------------------------------------------------------------
 # public API
 # ---------------------------------------------------------------------------------------------
@@ -372,6 +315,10 @@ def is_supported(input, num_groups: int, weight=None, bias=None, activation: Opt
         return False
 
 
+def _tensor_or_none(t) -> bool:
+    return t is None or isinstance(t, torch.Tensor)
+
+
 def group_norm(input, num_groups: int, weight=None, bias=None, eps: float = 1e-5, activation: Optional[str] = None, *,
                out_dtype=MATCH_STOCK_DTYPE, out_halo: int = 0):
     """``F.group_norm(input, num_groups, weight, bias, eps)`` (then ``F.relu`` when ``activation="relu"``)
@@ -385,6 +332,20 @@ def group_norm(input, num_groups: int, weight=None, bias=None, eps: float = 1e-5
         raise ValueError(
             f"out_dtype must be MATCH_STOCK_DTYPE, None (the input's dtype) or one of {SUPPORTED_DTYPES}, got {out_dtype!r}"
         )
+    compiling = torch.compiler.is_compiling()
+    if not compiling and isinstance(input, torch.Tensor) and type(num_groups) is int and _tensor_or_none(weight) and _tensor_or_none(bias):
+        given = getattr(input, "_sfh_gn_partials", None)
+        if given is not None and (given[2] != num_groups or given[3] != input._version or given[0].device != input.device):
+            given = None
+        stock = out_dtype is MATCH_STOCK_DTYPE
+        # the producer of `input` may have left per-group Welford records of these very bits: then no statistics pass
+        done = _lib.native().group_norm(input, num_groups, weight, bias, float(eps), activation == "relu", None if stock else out_dtype,
+                                        stock, int(out_halo), None if given is None else given[0], 0 if given is None else given[1])
+        if done is not None:
+            out, slab = done
+            if slab is not None:
+                out._sfh_slab = (slab, int(out_halo))
+            return out
     if not is_supported(input, num_groups, weight, bias, activation):
         if isinstance(input, torch.Tensor) and input.dim() == 5 and input.is_cuda:
             # shapes F.group_norm rejects keep F.group_norm's own exception type
@@ -397,13 +358,10 @@ def group_norm(input, num_groups: int, weight=None, bias=None, eps: float = 1e-5
             f"unsupported group_norm call: input={tuple(getattr(input, 'shape', ()))}/{getattr(input, 'dtype', None)} on "
             f"{getattr(input, 'device', None)}, num_groups={num_groups}; needs a channels_last_3d CUDA tensor"
         )
-    if torch.compiler.is_compiling():
-        out, _mean, _rstd = torch.ops.scaffold_gn.group_norm(
-            input, num_groups, weight, bias, float(eps), activation, _resolve_out_dtype(input, out_dtype)
-        )
-        return out
-    return _EagerGroupNormFn.apply(input, num_groups, weight, bias, float(eps), activation, _resolve_out_dtype(input, out_dtype),
-                                   int(out_halo))
+    out, _mean, _rstd = torch.ops.scaffold_gn.group_norm(
+        input, num_groups, weight, bias, float(eps), activation, _resolve_out_dtype(input, out_dtype)
+    )
+    return out
 
 
 #: the reference's name for :func:`group_norm`

@@ -11,18 +11,13 @@ materialised in fp32.
 
 from __future__ import annotations
 
-import ctypes
 from typing import Optional
 
 import torch
-from torch.autograd.function import once_differentiable
 
 from . import _lib
-from ._lib import LossDesc
 
 __all__ = ["ce_dice_loss", "is_supported_loss"]
-
-_CL3D = torch.channels_last_3d
 
 
 def is_supported_loss(logits, labels, class_weight=None) -> bool:
@@ -46,53 +41,17 @@ def is_supported_loss(logits, labels, class_weight=None) -> bool:
         return False
 
 
-class _CeDiceFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, logits, labels, class_weight, eps):
-        x = logits.contiguous(memory_format=_CL3D)
-        lab = labels.contiguous()
-        cw = None if class_weight is None else class_weight.detach().to(torch.float32).contiguous()
-        n, c, d, h, w = (int(v) for v in x.shape)
-        desc = LossDesc(n, c, d * h * w, float(eps))
-        L = _lib.lib()
-        loss = torch.empty((), dtype=torch.float32, device=x.device)
-        stats = torch.empty((n * 3 * c + 2,), dtype=torch.float32, device=x.device)
-        with _lib.device_guard(x.device):
-            ws = _lib.workspace(int(L.sfh_ce_dice_workspace_bytes(ctypes.byref(desc))), x.device)
-            rc = L.sfh_ce_dice_fwd(ctypes.byref(desc), _lib.dtype_code(x.dtype), _lib.ptr(x), _lib.ptr(lab), _lib.ptr(cw),
-                                   _lib.ptr(loss), _lib.ptr(stats), _lib.ptr(ws), 0 if ws is None else ws.numel(),
-                                   _lib.stream_ptr(x.device))
-        _lib.check(rc, "ce_dice_loss")
-        ctx.save_for_backward(x, lab, stats) if cw is None else ctx.save_for_backward(x, lab, stats, cw)
-        ctx.loss_args = (n, c, d * h * w, float(eps), cw is not None)
-        return loss
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx, grad_loss):
-        n, c, s, eps, weighted = ctx.loss_args
-        saved = ctx.saved_tensors
-        x, lab, stats = saved[:3]
-        cw = saved[3] if weighted else None
-        desc = LossDesc(n, c, s, eps)
-        g = grad_loss.detach().to(device=x.device, dtype=torch.float32).reshape(1).contiguous()
-        dx = torch.empty_like(x, memory_format=_CL3D)
-        L = _lib.lib()
-        with _lib.device_guard(x.device):
-            rc = L.sfh_ce_dice_bwd(ctypes.byref(desc), _lib.dtype_code(x.dtype), _lib.ptr(x), _lib.ptr(lab), _lib.ptr(cw),
-                                   _lib.ptr(stats), _lib.ptr(g), _lib.ptr(dx), _lib.stream_ptr(x.device))
-        _lib.check(rc, "ce_dice_loss backward")
-        return dx, None, None, None
-
-
 def ce_dice_loss(logits: torch.Tensor, labels: torch.Tensor, class_weight: Optional[torch.Tensor] = None,
                  eps: float = 1e-6) -> torch.Tensor:
     """``CE(logits, labels[, class_weight]) + 1 - mean foreground soft Dice`` as a 0-dim fp32 tensor.
 
     ``logits``: ``(N, C, D, H, W)`` bf16 / fp16 / fp32 on the GPU (any memory format; channels-last is read in
     place); ``labels``: ``(N, D, H, W)`` int64 class ids, ids outside ``[0, C)`` contribute nothing."""
-    if not is_supported_loss(logits, labels, class_weight):
+    loss = None
+    if isinstance(logits, torch.Tensor) and isinstance(labels, torch.Tensor) and (class_weight is None or isinstance(class_weight, torch.Tensor)):
+        loss = _lib.native().ce_dice_loss(logits, labels, class_weight, float(eps))
+    if loss is None:
         raise NotImplementedError(
             f"unsupported: logits={tuple(getattr(logits, 'shape', ()))}/{getattr(logits, 'dtype', None)} "
             f"labels={tuple(getattr(labels, 'shape', ()))}/{getattr(labels, 'dtype', None)}")
-    return _CeDiceFn.apply(logits, labels, class_weight, eps)
+    return loss

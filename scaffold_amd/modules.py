@@ -32,13 +32,11 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
-from torch.autograd.function import once_differentiable
 
+from . import _lib
 from . import conv3d as _c3
 from . import groupnorm as _gn
 from . import halo as _halo
-from . import transposed as _ct
 
 __all__ = ["FastConv3d", "FastConvTranspose3d", "FastGroupNorm", "autocast_dtype", "cast_operand", "compute_copy",
            "flush_weight_gradients"]
@@ -104,15 +102,6 @@ def _current_packs(owner: torch.Tensor, source: torch.Tensor, in_shape, stride, 
         e.repack(source)
         e.version = owner._version
     return e
-
-
-def _fp32_weight_grad(fn, *args, **kwargs):
-    """Weight gradient straight in fp32 where the tiled kernels serve the shape, else in the operands' dtype and
-    widened afterwards (what autocast's cast node would have done)."""
-    try:
-        return fn(*args, grad_dtype=torch.float32, **kwargs)
-    except NotImplementedError:
-        return fn(*args, **kwargs).to(torch.float32)
 
 
 # ---- weight gradients of a backward pass in one launch -----------------------------------------------------------------
@@ -234,173 +223,47 @@ def flush_weight_gradients() -> None:
             _add_to_grads(items, grads)
 
 
-# positions in _Conv3dFn.forward's argument list (after ctx): the gradients come back in this order
-_ARG_SECOND, _N_ARGS = 11, 14
+def _queue_from_node(param, x, second, gy, padding, master, family, early) -> None:
+    """A convolution's backward node leaves its weight gradient to the end of the pass (called by the node)."""
+    _queue_weight_grad(_QueuedWeightGrad(param, x if second is None else (x, second), param.shape, gy, padding,
+                                         torch.float32 if master else x.dtype, family, early))
 
 
-class _Conv3dFn(torch.autograd.Function):
-    """The caller (``FastConv3d.forward``) has passed the gate for all three directions with these very operands, and
-    autograd hands ``backward`` a gradient of the output's shape and dtype: the per-call gates are not repeated."""
-
-    @staticmethod
-    def forward(ctx, x, weight, bias, stride, padding, dilation, weight_compute=None, bias_compute=None, packs=None, slab=None,
-                gn_groups=0, second=None, slab2=None, defer_weight_grad=False):
-        # weight / bias are the tensors that receive gradients; when half-precision copies of fp32 masters are
-        # given, the kernels read those and the gradients are produced in the masters' dtype directly
-        wc = weight if weight_compute is None else weight_compute
-        bc = bias if bias_compute is None else bias_compute
-        # `slab` = (tensor, halo): x is the depth interior of that tensor, whose faces already hold the halo; the
-        # kernels read the whole of it and the data gradient of its interior is x's
-        ctx.halo = 0
-        if slab is not None:
-            ctx.halo, ctx.depth = slab[1], x.shape[2]
-            x = slab[0]
-        # `second`: the input is the pair (x, second) whose channels follow each other -- a skip connection and the
-        # upsampled tensor, never concatenated; `slab2` is to `second` what `slab` is to x
-        ctx.pair = second is not None
-        if slab2 is not None:
-            second = slab2[0]
-        in_shape = x.shape if second is None else torch.Size((x.shape[0], x.shape[1] + second.shape[1], *x.shape[2:]))
-        pf = pd = None
-        if packs is not None:
-            # packed forms that are current (kept by the module, refreshed by whoever writes the weight)
-            pf, pd = packs.fwd, packs.dgrad
-        elif ctx.needs_input_grad[0] and (PACK_WEIGHTS_ONCE or torch.cuda.is_current_stream_capturing()):
-            # When the data gradient will be wanted too, the weight can be packed for both directions in one launch.
-            # That saves a launch per convolution on the GPU and costs a little more host time, so it is done where
-            # host time is free (under graph capture) or when asked for (PACK_WEIGHTS_ONCE).
-            pf, pd = _c3.pack_weights(wc, in_shape, stride, padding, dilation)
-        # gn_groups: a GroupNorm of that many groups follows; the launch leaves its statistics on y where it can
-        if second is None:
-            y = _c3.conv3d_forward(x, wc, bc, stride, padding, dilation, 1, packed_weight=pf, gn_groups=gn_groups, _checked=True)
-            ctx.save_for_backward(x, wc) if pd is None else ctx.save_for_backward(x, wc, pd)
-        else:
-            y = _c3.conv3d_forward_pair(x, second, wc, bc, stride, padding, dilation, packed_weight=pf, gn_groups=gn_groups,
-                                        _checked=True)
-            ctx.save_for_backward(x, wc, second) if pd is None else ctx.save_for_backward(x, wc, second, pd)
-        ctx.conv_args = (stride, padding, dilation, bias is not None, None if bias is None else bias.dtype,
-                         weight.dtype is not wc.dtype)
-        # the parameter whose .grad a deferred weight gradient is added to (see flush_weight_gradients)
-        ctx.defer_param = weight if defer_weight_grad else None
-        ctx.defer_early = defer_weight_grad == 2
-        return y
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx, grad_output):
-        if ctx.pair:
-            return _Conv3dFn._backward_pair(ctx, grad_output)
-        x, weight, *packed = ctx.saved_tensors
-        stride, padding, dilation, has_bias, bias_dtype, master = ctx.conv_args
-        needs_x, needs_w, needs_b = ctx.needs_input_grad[:3]
-        grad_output = grad_output.contiguous(memory_format=_CL3D)
-        grad_x = _c3.conv3d_backward_data(grad_output, weight, x.shape, stride, padding, dilation, 1,
-                                          packed_weight=packed[0] if packed else None, _checked=True) if needs_x else None
-        if ctx.halo and grad_x is not None:
-            grad_x = grad_x.narrow(2, ctx.halo, ctx.depth)
-        grad_w = None
-        if needs_w and has_bias and needs_b:
-            # both parameter gradients from one pass over grad_output where the library offers it (the 1x1x1 head)
-            both = _c3.conv3d_backward_weight_bias(x, weight.shape, grad_output, stride, padding, dilation, 1,
-                                                   grad_dtype=torch.float32 if master else None, _checked=True)
-            if both is not None:
-                grad_w, grad_b = both
-                if grad_b.dtype is not bias_dtype:
-                    grad_b = grad_b.to(bias_dtype)
-                return grad_x, grad_w, grad_b, None, None, None, None, None, None, None, None, None, None, None
-        family = _deferrable(ctx.defer_param, x.shape, weight.shape, stride, padding, dilation, x.dtype) if needs_w else 0
-        if family:
-            _queue_weight_grad(_QueuedWeightGrad(ctx.defer_param, x, weight.shape, grad_output, padding,
-                                                 torch.float32 if master else x.dtype, family, ctx.defer_early))
-        elif needs_w:
-            if master:
-                grad_w = _fp32_weight_grad(_c3.conv3d_backward_weight, x, weight.shape, grad_output, stride, padding, dilation, 1,
-                                           _checked=True)
-            else:
-                grad_w = _c3.conv3d_backward_weight(x, weight.shape, grad_output, stride, padding, dilation, 1, _checked=True)
-        grad_b = _c3.bias_grad(grad_output, bias_dtype) if (has_bias and needs_b) else None
-        return grad_x, grad_w, grad_b, None, None, None, None, None, None, None, None, None, None, None
-
-    @staticmethod
-    def _backward_pair(ctx, grad_output):
-        """The three gradients of the convolution over (x, second): the data gradient comes back as the two tensors the
-        concatenation's backward would have cut it into."""
-        x, weight, second, *packed = ctx.saved_tensors
-        stride, padding, dilation, has_bias, bias_dtype, master = ctx.conv_args
-        needs_x, needs_w, needs_b = ctx.needs_input_grad[:3]
-        needs_second = ctx.needs_input_grad[_ARG_SECOND]
-        grad_output = grad_output.contiguous(memory_format=_CL3D)
-        grad_x = grad_second = None
-        if needs_x or needs_second:
-            in_shape = torch.Size((x.shape[0], x.shape[1] + second.shape[1], *x.shape[2:]))
-            grad_x, grad_second = _c3.conv3d_backward_data_pair(grad_output, weight, in_shape, int(x.shape[1]), stride, padding,
-                                                                dilation, packed_weight=packed[0] if packed else None, _checked=True)
-            if ctx.halo:  # both tensors are slabs of the same depth: the interiors are the inputs' gradients
-                grad_x = grad_x.narrow(2, ctx.halo, ctx.depth)
-                grad_second = grad_second.narrow(2, ctx.halo, ctx.depth)
-        grad_w = None
-        family = 0
-        if needs_w:
-            family = _deferrable(ctx.defer_param, torch.Size((x.shape[0], x.shape[1] + second.shape[1], *x.shape[2:])), weight.shape,
-                                 stride, padding, dilation, x.dtype)
-        if family:
-            _queue_weight_grad(_QueuedWeightGrad(ctx.defer_param, (x, second), weight.shape, grad_output, padding,
-                                                 torch.float32 if master else x.dtype, family, ctx.defer_early))
-        elif needs_w:
-            if master:
-                grad_w = _fp32_weight_grad(_c3.conv3d_backward_weight_pair, x, second, weight.shape, grad_output, stride, padding,
-                                           dilation, _checked=True)
-            else:
-                grad_w = _c3.conv3d_backward_weight_pair(x, second, weight.shape, grad_output, stride, padding, dilation, _checked=True)
-        grad_b = _c3.bias_grad(grad_output, bias_dtype) if (has_bias and needs_b) else None
-        grads = [None] * _N_ARGS
-        grads[0], grads[1], grads[2] = (grad_x if needs_x else None), grad_w, grad_b
-        grads[_ARG_SECOND] = grad_second if needs_second else None
-        return tuple(grads)
+_node_queue_set = False
 
 
-class _ConvTranspose3dFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, weight, bias, stride, weight_compute=None, bias_compute=None, packs=None, out_halo=0):
-        wc = weight if weight_compute is None else weight_compute
-        bc = bias if bias_compute is None else bias_compute
-        # `out_halo` (one sample): the result is written into the interior of a depth slab with that many zero planes on
-        # each face, which rides along as y._sfh_slab for a following FastConv3d.shard_halo
-        # `packs`: kept packed forms of the kernel == stride convolution this op transposes; its data-gradient form is
-        # what this forward reads, its forward form what the data gradient below reads
-        y = _ct.conv_transpose3d_forward(x, wc, bc, stride, 0, 0, 1, 1, packed_weight=None if packs is None else packs.dgrad,
-                                         out_halo=out_halo)
-        pf = None if packs is None else packs.fwd
-        ctx.save_for_backward(x, wc) if pf is None else ctx.save_for_backward(x, wc, pf)
-        ctx.conv_args = (stride, bias is not None, None if bias is None else bias.dtype, weight.dtype is not wc.dtype)
-        return y
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx, grad_output):
-        x, weight, *packed = ctx.saved_tensors
-        stride, has_bias, bias_dtype, master = ctx.conv_args
-        needs_x, needs_w, needs_b = ctx.needs_input_grad[:3]
-        grad_output = grad_output.contiguous(memory_format=_CL3D)
-        grad_x = _ct.conv_transpose3d_backward_data(grad_output, weight, x.shape, stride, 0, 0, 1, 1,
-                                                    packed_weight=packed[0] if packed else None) if needs_x else None
-        grad_w = grad_b = None
-        if needs_w and has_bias and needs_b:
-            # both from one pass over grad_output where the library offers it (the 2x2x2 matrix-core problems)
-            both = _ct.conv_transpose3d_backward_weight_bias(x, weight.shape, grad_output, stride, 0, 0, 1, 1,
-                                                             grad_dtype=torch.float32 if master else None)
-            if both is not None:
-                grad_w, grad_b = both
-                if grad_b.dtype is not bias_dtype:
-                    grad_b = grad_b.to(bias_dtype)
-                return grad_x, grad_w, grad_b, None, None, None, None, None
-        if needs_w:
-            if master:
-                grad_w = _fp32_weight_grad(_ct.conv_transpose3d_backward_weight, x, weight.shape, grad_output, stride, 0, 0, 1, 1)
-            else:
-                grad_w = _ct.conv_transpose3d_backward_weight(x, weight.shape, grad_output, stride, 0, 0, 1, 1)
-        grad_b = _c3.bias_grad(grad_output, bias_dtype) if (has_bias and needs_b) else None
-        return grad_x, grad_w, grad_b, None, None, None, None, None
+def _run_conv(x, second, x_read, second_read, weight, bias, w, b, packs, halo, stride, padding, dilation, master, gn_groups, defer):
+    """The forward launch of a convolution and its autograd node.  ``x`` / ``second`` are the tensors that receive gradients,
+    ``x_read`` / ``second_read`` what the kernels read (slabs of which x and second are the depth interiors when ``halo`` > 0,
+    else the same tensors).  ``weight`` / ``bias`` receive gradients, ``w`` / ``b`` are what the kernels read: when half-precision
+    copies of fp32 masters are given (``master``) the gradients are produced in the masters' dtype directly.  The caller has
+    passed the gate (for all three directions when the call will be differentiated)."""
+    global _node_queue_set
+    pf = pd = None
+    in_shape = x_read.shape if second is None else torch.Size((x_read.shape[0], x_read.shape[1] + second_read.shape[1], *x_read.shape[2:]))
+    if packs is not None:
+        # packed forms that are current (kept by the module, refreshed by whoever writes the weight)
+        pf, pd = packs.fwd, packs.dgrad
+    elif torch.is_grad_enabled() and x.requires_grad and (PACK_WEIGHTS_ONCE or torch.cuda.is_current_stream_capturing()):
+        # When the data gradient will be wanted too, the weight can be packed for both directions in one launch.
+        # That saves a launch per convolution on the GPU and costs a little more host time, so it is done where
+        # host time is free (under graph capture) or when asked for (PACK_WEIGHTS_ONCE).
+        pf, pd = _c3.pack_weights(w, in_shape, stride, padding, dilation)
+    # gn_groups: a GroupNorm of that many groups follows; the launch leaves its statistics on y where it can
+    if second is None:
+        y = _c3.conv3d_forward(x_read, w, b, stride, padding, dilation, 1, packed_weight=pf, gn_groups=gn_groups, _checked=True)
+    else:
+        y = _c3.conv3d_forward_pair(x_read, second_read, w, b, stride, padding, dilation, packed_weight=pf, gn_groups=gn_groups,
+                                    _checked=True)
+    if _wants_grad(x, second, weight, bias):
+        native = _lib.native()
+        if not _node_queue_set:
+            native.set_weight_queue(_queue_from_node)
+            _node_queue_set = True
+        family = _deferrable(weight, in_shape, w.shape, stride, padding, dilation, x_read.dtype) if defer else 0
+        native.record_conv(y, x, weight, bias, second, x_read, second_read, w, pd, halo, stride, padding, dilation, master, family,
+                           defer == 2)
+    return y
 
 
 def _wants_grad(*tensors) -> bool:
@@ -499,13 +362,14 @@ class FastConv3d(nn.Conv3d):
                 f"FastConv3d: pair not served: x={tuple(x_read.shape)}/{x_read.dtype} second={tuple(second_read.shape)} on {x.device}, "
                 f"weight={tuple(w.shape)}/{w.dtype}, stride={stride} padding={padding} dilation={dilation}")
         in_shape = torch.Size((x_read.shape[0], x_read.shape[1] + second_read.shape[1], *x_read.shape[2:]))
+        halo = 0 if slab is None else slab[1]
         if master:
-            return _Conv3dFn.apply(x, weight, bias, stride, padding, dilation, w, b,
-                                   _current_packs(weight, w, in_shape, stride, padding, dilation), slab, self.gn_groups,
-                                   second, slab2, self.defer_weight_grad)
+            packs = _current_packs(weight, w, in_shape, stride, padding, dilation)
+            return _run_conv(x, second, x_read, second_read, weight, bias, w, b, packs, halo, stride, padding, dilation, True,
+                             self.gn_groups, self.defer_weight_grad)
         packs = _current_packs(w, w, in_shape, stride, padding, dilation) if w is weight else None
-        return _Conv3dFn.apply(x, w, b, stride, padding, dilation, None, None, packs, slab, self.gn_groups, second,
-                               slab2, self.defer_weight_grad if w is weight else False)
+        return _run_conv(x, second, x_read, second_read, w, b, w, b, packs, halo, stride, padding, dilation, False, self.gn_groups,
+                         self.defer_weight_grad if w is weight else False)
 
     def forward(self, x: torch.Tensor, second: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``second``: the input is ``torch.cat([x, second], 1)``, read from the two tensors themselves (the decoder's skip
@@ -538,24 +402,24 @@ class FastConv3d(nn.Conv3d):
         x = x.contiguous(memory_format=_CL3D)
         # the node below skips its own gates on the strength of this one (a call that will be differentiated is
         # gated for all three directions here)
-        gate = _c3.is_supported_all if _wants_grad(inner, w, b) else _c3.is_supported
-        if not gate(x, w, b, self.stride, padding, self.dilation, self.groups):
+        wants = _wants_grad(inner, w, b)
+        stride, dilation = tuple(self.stride), tuple(self.dilation)
+        if self.groups != 1 or not (_lib.native().conv_supported(x, w, b, stride, padding, dilation, wants) or
+                                    (_c3.is_supported_all if wants else _c3.is_supported)(x, w, b, stride, padding, dilation, 1)):
             raise NotImplementedError(
                 f"FastConv3d: not served: x={tuple(x.shape)}/{x.dtype} on {x.device}, weight={tuple(w.shape)}/{w.dtype}, "
                 f"stride={self.stride} padding={padding} dilation={self.dilation} groups={self.groups}"
             )
-        stride, dilation = tuple(self.stride), tuple(self.dilation)
         if slab is None:
             inner = x
+        halo = 0 if slab is None else slab[1]
         if master:
-            return _Conv3dFn.apply(inner, weight, bias, stride, padding, dilation, w, b,
-                                   _current_packs(weight, w, x.shape, stride, padding, dilation), slab, self.gn_groups,
-                                   None, None, self.defer_weight_grad)
-        if w is weight:
-            return _Conv3dFn.apply(inner, w, b, stride, padding, dilation, None, None,
-                                   _current_packs(w, w, x.shape, stride, padding, dilation), slab, self.gn_groups,
-                                   None, None, self.defer_weight_grad)
-        return _Conv3dFn.apply(inner, w, b, stride, padding, dilation, None, None, None, slab, self.gn_groups)
+            packs = _current_packs(weight, w, x.shape, stride, padding, dilation)
+            return _run_conv(inner, None, x, None, weight, bias, w, b, packs, halo, stride, padding, dilation, True, self.gn_groups,
+                             self.defer_weight_grad)
+        packs = _current_packs(w, w, x.shape, stride, padding, dilation) if w is weight else None
+        return _run_conv(inner, None, x, None, w, b, w, b, packs, halo, stride, padding, dilation, False, self.gn_groups,
+                         self.defer_weight_grad if w is weight else False)
 
 
 class FastConvTranspose3d(nn.ConvTranspose3d):
@@ -575,26 +439,29 @@ class FastConvTranspose3d(nn.ConvTranspose3d):
         master = wc is not None and (bias is None or bc is not None)
         w = wc if master else cast_operand(weight, dt)
         b = bc if master else cast_operand(bias, dt)
-        x = x.contiguous(memory_format=_CL3D)
-        gate = _ct.is_supported_transposed_all if _wants_grad(x, w, b) else _ct.is_supported_transposed
-        if not gate(x, w, b, self.stride, self.padding, self.output_padding, self.dilation, self.groups):
+        stride, done = tuple(self.stride), None
+        if self.groups == 1 and tuple(self.padding) == tuple(self.output_padding) == (0, 0, 0) and tuple(self.dilation) == (1, 1, 1):
+            packs = None
+            if (master or w is weight) and x.dim() == 5:
+                # the problem the packed forms belong to: the stride-k convolution over this op's output
+                n, _, d, h, wd = x.shape
+                big = torch.Size((n, w.shape[1], d * stride[0], h * stride[1], wd * stride[2]))
+                packs = _current_packs(weight, w, big, stride, (0, 0, 0), (1, 1, 1))
+                if packs is not None and (packs.fwd is None or packs.dgrad is None):
+                    packs = None
+            pf, pd = (None, None) if packs is None else (packs.fwd, packs.dgrad)
+            done = _lib.native().conv_transpose(x, weight if master else w, bias if master else b, w, b, stride, pf, pd,
+                                                self.out_halo, master)
+        if done is None:
             raise NotImplementedError(
                 f"FastConvTranspose3d: not served: x={tuple(x.shape)}/{x.dtype} on {x.device}, weight={tuple(w.shape)}, "
                 f"stride={self.stride} padding={self.padding} output_padding={self.output_padding} "
                 f"dilation={self.dilation} groups={self.groups}"
             )
-        stride = tuple(self.stride)
-        if master or w is weight:
-            # the problem the packed forms belong to: the stride-k convolution over this op's output
-            n, _, d, h, wd = x.shape
-            big = torch.Size((n, w.shape[1], d * stride[0], h * stride[1], wd * stride[2]))
-            packs = _current_packs(weight, w, big, stride, (0, 0, 0), (1, 1, 1))
-            if packs is not None and (packs.fwd is None or packs.dgrad is None):
-                packs = None
-            if master:
-                return _ConvTranspose3dFn.apply(x, weight, bias, stride, w, b, packs, self.out_halo)
-            return _ConvTranspose3dFn.apply(x, w, b, stride, None, None, packs, self.out_halo)
-        return _ConvTranspose3dFn.apply(x, w, b, stride, None, None, None, self.out_halo)
+        y, slab = done
+        if slab is not None:
+            y._sfh_slab = (slab, self.out_halo)
+        return y
 
 
 class FastGroupNorm(nn.GroupNorm):

@@ -8,14 +8,10 @@ writes the input gradient in one pass.
 
 from __future__ import annotations
 
-import ctypes
-
 import torch
 import torch.nn as nn
-from torch.autograd.function import once_differentiable
 
 from . import _lib
-from ._lib import PoolDesc
 
 __all__ = ["max_pool3d_2x_with_skip", "max_pool3d_2x", "is_supported_pool", "FastMaxPool3d"]
 
@@ -31,90 +27,28 @@ def is_supported_pool(x) -> bool:
         return False
 
 
-class _MaxPool2Fn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, out_halo=0):
-        x = x.contiguous(memory_format=_CL3D)
-        n, c, d, h, w = (int(v) for v in x.shape)
-        idx = torch.empty((n, d // 2, h // 2, w // 2, c), dtype=torch.uint8, device=x.device)
-        desc = PoolDesc(n, c, d, h, w)
-        y = None
-        if out_halo > 0 and n == 1 and min(d, h, w) >= 2:
-            # the result in the interior of a depth slab with zero faces (the launch zeroes them), for a following
-            # FastConv3d.shard_halo; where the library does not offer it for these extents, the plain launch below
-            slab = torch.empty((1, c, d // 2 + 2 * out_halo, h // 2, w // 2), dtype=x.dtype, device=x.device, memory_format=_CL3D)
-            with _lib.device_guard(x.device):
-                rc = _lib.lib().sfh_maxpool2_fwd_slab(ctypes.byref(desc), _lib.dtype_code(x.dtype), _lib.ptr(x), _lib.ptr(slab),
-                                                      out_halo * (h // 2) * (w // 2) * c, _lib.ptr(idx), _lib.stream_ptr(x.device))
-            if rc != _lib.SFH_ERR_UNSUPPORTED:
-                _lib.check(rc, "max_pool3d_2x")
-                y = slab.narrow(2, out_halo, d // 2)
-                y._sfh_slab = (slab, out_halo)
-        if y is None:
-            y = torch.empty((n, c, d // 2, h // 2, w // 2), dtype=x.dtype, device=x.device, memory_format=_CL3D)
-            with _lib.device_guard(x.device):
-                rc = _lib.lib().sfh_maxpool2_fwd(ctypes.byref(desc), _lib.dtype_code(x.dtype), _lib.ptr(x), _lib.ptr(y), _lib.ptr(idx),
-                                                 _lib.stream_ptr(x.device))
-            _lib.check(rc, "max_pool3d_2x")
-        ctx.save_for_backward(idx)
-        ctx.pool_shape = (n, c, d, h, w)
-        return y
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx, grad_y):
-        (idx,) = ctx.saved_tensors
-        n, c, d, h, w = ctx.pool_shape
-        gy = grad_y.contiguous(memory_format=_CL3D)
-        gx = torch.empty((n, c, d, h, w), dtype=gy.dtype, device=gy.device, memory_format=_CL3D)
-        desc = PoolDesc(n, c, d, h, w)
-        with _lib.device_guard(gy.device):
-            rc = _lib.lib().sfh_maxpool2_bwd(ctypes.byref(desc), _lib.dtype_code(gy.dtype), _lib.ptr(gy), _lib.ptr(idx), _lib.ptr(gx),
-                                             _lib.stream_ptr(gy.device))
-        _lib.check(rc, "max_pool3d_2x backward")
-        return gx, None
+def _refuse(x):
+    raise NotImplementedError(f"unsupported: x={tuple(getattr(x, 'shape', ()))}/{getattr(x, 'dtype', None)}")
 
 
-class _MaxPool2SkipFn(torch.autograd.Function):
-    """Pooling of a tensor that is also carried on as a skip connection: returns ``(pooled, x)``; the two gradients
-    of ``x`` (through the pooling and through the skip) are summed inside the pooling-gradient kernel instead of by a
-    separate addition over the full-size tensor."""
-
-    @staticmethod
-    def forward(ctx, x, out_halo=0):
-        y = _MaxPool2Fn.forward(ctx, x, out_halo)
-        return y, x  # autograd hands out an alias of x with this node as its history
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx, grad_y, grad_skip):
-        if grad_skip is None:
-            return _MaxPool2Fn.backward(ctx, grad_y)
-        if grad_y is None:
-            return grad_skip, None
-        (idx,) = ctx.saved_tensors
-        n, c, d, h, w = ctx.pool_shape
-        gy = grad_y.contiguous(memory_format=_CL3D)
-        gs = grad_skip.contiguous(memory_format=_CL3D)
-        if gs.dtype is not gy.dtype:
-            gs = gs.to(gy.dtype)
-        gx = torch.empty((n, c, d, h, w), dtype=gy.dtype, device=gy.device, memory_format=_CL3D)
-        desc = PoolDesc(n, c, d, h, w)
-        with _lib.device_guard(gy.device):
-            rc = _lib.lib().sfh_maxpool2_bwd_add(ctypes.byref(desc), _lib.dtype_code(gy.dtype), _lib.ptr(gy), _lib.ptr(idx),
-                                                 _lib.ptr(gs), _lib.ptr(gx), _lib.stream_ptr(gy.device))
-        _lib.check(rc, "max_pool3d_2x backward")
-        return gx, None
+def _pool(x, out_halo, with_skip):
+    """The launch and its autograd node: ``(pooled, ...)``; the pooled tensor carries the slab it lies in, if any."""
+    done = _lib.native().max_pool(x, int(out_halo), with_skip) if isinstance(x, torch.Tensor) else None
+    if done is None:
+        _refuse(x)
+    if done[1] is not None:
+        done[0]._sfh_slab = (done[1], int(out_halo))
+    return done
 
 
 def max_pool3d_2x_with_skip(x: torch.Tensor, out_halo: int = 0):
     """``(F.max_pool3d(x, 2), x)``: use the returned ``x`` for the skip connection and the gradients of both uses are
     combined in one kernel (same values as autograd's own addition: one fp32 sum, one rounding)."""
     if not is_supported_pool(x):
-        raise NotImplementedError(f"unsupported: x={tuple(getattr(x, 'shape', ()))}/{getattr(x, 'dtype', None)}")
+        _refuse(x)
     if not x.is_contiguous(memory_format=_CL3D):
-        return _MaxPool2Fn.apply(x, int(out_halo)), x
-    pooled, skip = _MaxPool2SkipFn.apply(x, int(out_halo))
+        return _pool(x, out_halo, False)[0], x
+    pooled, _, skip = _pool(x, out_halo, True)
     slab = getattr(x, "_sfh_slab", None)
     if slab is not None:  # the alias is the same memory: still the interior of the slab its producer wrote it into
         skip._sfh_slab = slab
@@ -124,9 +58,7 @@ def max_pool3d_2x_with_skip(x: torch.Tensor, out_halo: int = 0):
 def max_pool3d_2x(x: torch.Tensor, out_halo: int = 0) -> torch.Tensor:
     """``F.max_pool3d(x, 2)`` for a 5-D GPU tensor; the result is channels-last.  ``out_halo=h`` (one sample): the result is
     the interior view of a slab with ``h`` zero depth planes on each face (``result._sfh_slab``), for ``FastConv3d.shard_halo``."""
-    if not is_supported_pool(x):
-        raise NotImplementedError(f"unsupported: x={tuple(getattr(x, 'shape', ()))}/{getattr(x, 'dtype', None)}")
-    return _MaxPool2Fn.apply(x, int(out_halo))
+    return _pool(x, out_halo, False)[0]
 
 
 def _all_equal(v, want) -> bool:

@@ -1,0 +1,63 @@
+"""The C++ host path (``scaffold_amd/_native``): its autograd nodes where they differ from an ordinary forward and backward."""
+
+import pytest
+import torch
+
+import scaffold_amd as sa
+
+pytestmark = pytest.mark.gpu
+CL = torch.channels_last_3d
+
+
+def _x(device, c=32, n=1, dtype=torch.bfloat16):
+    return torch.randn(n, c, 4, 4, 8, device=device).to(dtype).contiguous(memory_format=CL).requires_grad_()
+
+
+def _ops(device):
+    conv = sa.FastConv3d(32, 32, 3, padding=1, device=device, dtype=torch.bfloat16)
+    up = sa.FastConvTranspose3d(32, 32, 2, stride=2, device=device, dtype=torch.bfloat16)
+    norm = sa.FastGroupNorm(8, 32, activation="relu", device=device, dtype=torch.bfloat16)
+    labels = torch.zeros(1, 4, 4, 8, dtype=torch.long, device=device)
+    return {"conv": conv, "up": up, "norm": norm, "pool": sa.FastMaxPool3d(2), "skip": lambda x: sa.FastMaxPool3d(2).with_skip(x)[0],
+            "loss": lambda x: sa.ce_dice_loss(x, labels)}
+
+
+@pytest.mark.parametrize("name", ["conv", "up", "norm", "pool", "skip", "loss"])
+def test_no_op_is_differentiated_twice_in_silence(device, name):
+    """The gradient under create_graph is the ordinary one, and differentiating it raises instead of returning zeros."""
+    op, x = _ops(device)[name], _x(device)
+    (plain,) = torch.autograd.grad(op(x).float().square().sum(), x)
+    (gx,) = torch.autograd.grad(op(x).float().square().sum(), x, create_graph=True)
+    assert torch.equal(plain, gx) and gx.requires_grad
+    with pytest.raises(RuntimeError, match="once_differentiable"):
+        gx.float().sum().backward()
+
+
+def test_gradients_only_where_they_are_wanted(device):
+    conv, norm = _ops(device)["conv"], _ops(device)["norm"]
+    x = _x(device)
+    for op in (conv, norm):
+        (gw,) = torch.autograd.grad(op(x.detach()).float().square().sum(), op.weight)
+        gx, gw2, gb = torch.autograd.grad(op(x).float().square().sum(), (x, op.weight, op.bias))
+        assert torch.equal(gw, gw2) and gx.shape == x.shape and gb.shape == op.bias.shape
+        with torch.no_grad():
+            assert not op(x).requires_grad
+
+
+def test_empty_batch_through_the_up_convolution(device):
+    up = _ops(device)["up"]
+    x = torch.empty(0, 32, 4, 4, 8, device=device, dtype=torch.bfloat16).requires_grad_()
+    y = up(x)
+    assert y.shape == (0, 32, 8, 8, 16)
+    gx, gw, gb = torch.autograd.grad(y.float().sum(), (x, up.weight, up.bias))
+    assert gx.shape == x.shape and not gw.any() and not gb.any()
+
+
+def test_a_tensor_changed_after_the_forward_is_noticed(device):
+    conv, x = _ops(device)["conv"], _x(device)
+    h = x * 1
+    y = conv(h)
+    with torch.no_grad():
+        h.add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.float().sum().backward()
