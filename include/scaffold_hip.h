@@ -92,7 +92,8 @@ typedef struct sfh_groupnorm_desc {
  * workspace with those functions are unaffected).
  * 104: sfh_conv3d_wgrad_batch, sfh_conv3d_wgrad_batch_supported, sfh_conv3d_wgrad_batch_workspace_bytes added;
  * SFH_KERNEL_SPLIT (6) is a value sfh_conv3d_launch_geometry may report. Nothing removed or changed.
- * 105: SFH_FLAG_SHARE_DEVICE; sfh_conv3d_wgrad_batch_workspace_bytes takes the call's flags (changed: one more argument). */
+ * 105: SFH_FLAG_SHARE_DEVICE; sfh_conv3d_wgrad_batch_workspace_bytes takes the call's flags (changed: one more argument).
+ * 106: sfh_conv3d_pack_master_weights added. */
 int sfh_version(void);
 const char* sfh_last_error(void);
 /* Fills name (<= name_len bytes), compute-unit count, LDS bytes per workgroup. */
@@ -203,6 +204,12 @@ size_t sfh_conv3d_packed_weight_bytes(const sfh_conv3d_desc* p, int dtype, int d
 int sfh_conv3d_pack_weights(const sfh_conv3d_desc* p, int dtype, const void* w,
                             const int64_t w_stride[5], void* packed_fwd, void* packed_dgrad,
                             void* stream);
+
+/* The same from an fp32 master weight, rounded to `dtype` (to nearest even) on the way: what a cast of the weight in
+ * front of sfh_conv3d_pack_weights gives, bit for bit, without the cast. */
+int sfh_conv3d_pack_master_weights(const sfh_conv3d_desc* p, int dtype, const float* w,
+                                   const int64_t w_stride[5], void* packed_fwd, void* packed_dgrad,
+                                   void* stream);
 
 /* The packings of many weights in as few launches as possible (a training loop repacks every
  * convolution weight once per optimizer step). Each item is one sfh_conv3d_pack_weights call;

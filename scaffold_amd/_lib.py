@@ -128,6 +128,7 @@ _SIGNATURES = {
                                  c_size_t, c_uint32, c_void_p]),
     "sfh_conv3d_packed_weight_bytes": (c_size_t, [POINTER(ConvDesc), c_int, c_int]),
     "sfh_conv3d_pack_weights": (c_int, [POINTER(ConvDesc), c_int, c_void_p, POINTER(c_int64), c_void_p, c_void_p, c_void_p]),
+    "sfh_conv3d_pack_master_weights": (c_int, [POINTER(ConvDesc), c_int, c_void_p, POINTER(c_int64), c_void_p, c_void_p, c_void_p]),
     "sfh_conv3d_pack_weights_batch": (c_int, [POINTER(PackItem), c_int32, c_int, c_void_p]),
     "sfh_conv3d_wgrad_splits": (c_int, [POINTER(ConvDesc), c_int]),
     "sfh_conv3d_wgrad_workspace_bytes": (c_size_t, [POINTER(ConvDesc), c_int]),

@@ -291,7 +291,7 @@ __global__ void __launch_bounds__(256) stream_copy_kernel(const uint4* __restric
 
 using namespace sfh;
 
-extern "C" int sfh_version(void) { return 105; }
+extern "C" int sfh_version(void) { return 106; }
 
 extern "C" const char* sfh_last_error(void) { return g_error; }
 
@@ -473,30 +473,40 @@ extern "C" size_t sfh_conv3d_packed_weight_bytes(const sfh_conv3d_desc* p, int d
 // Appends the packings one weight asks for (its forward form and / or its data-gradient form) to jobs[njobs...]; the
 // caller leaves room for two.
 static int collect_pack_jobs(const sfh_conv3d_desc* p, int dtype, const void* w, const int64_t* w_stride, void* packed_fwd,
-                             void* packed_dgrad, MfmaPackItem* jobs, int* njobs) {
+                             void* packed_dgrad, MfmaPackItem* jobs, int* njobs, bool fp32_source = false) {
   int32_t out[3];
   if (int rc = check_conv(p, dtype, out)) return rc;
   if (w == nullptr || w_stride == nullptr) return fail(SFH_ERR_INVALID, "conv3d pack: null weight");
   if (packed_fwd != nullptr) {
     const PackSpec spec = fwd_pack_spec(*p, dtype, out, w_stride);
     if (!spec.any) return fail(SFH_ERR_UNSUPPORTED, "conv3d pack: the forward of this problem does not read a packed weight");
-    jobs[(*njobs)++] = MfmaPackItem{spec.a, w, spec.s_out, spec.s_red, w_stride[2], w_stride[3], w_stride[4], spec.flip, packed_fwd};
+    jobs[(*njobs)++] = MfmaPackItem{spec.a, w, spec.s_out, spec.s_red, w_stride[2], w_stride[3], w_stride[4], spec.flip, packed_fwd, fp32_source};
   }
   if (packed_dgrad != nullptr) {
     const PackSpec spec = dgrad_pack_spec(*p, dtype, out, w_stride);
     if (!spec.any) return fail(SFH_ERR_UNSUPPORTED, "conv3d pack: the data gradient of this problem does not read a packed weight");
-    jobs[(*njobs)++] = MfmaPackItem{spec.a, w, spec.s_out, spec.s_red, w_stride[2], w_stride[3], w_stride[4], spec.flip, packed_dgrad};
+    jobs[(*njobs)++] = MfmaPackItem{spec.a, w, spec.s_out, spec.s_red, w_stride[2], w_stride[3], w_stride[4], spec.flip, packed_dgrad, fp32_source};
   }
   return SFH_OK;
 }
 
-extern "C" int sfh_conv3d_pack_weights(const sfh_conv3d_desc* p, int dtype, const void* w, const int64_t w_stride[5], void* packed_fwd,
-                                       void* packed_dgrad, void* stream) {
+static int pack_weights(const sfh_conv3d_desc* p, int dtype, const void* w, const int64_t w_stride[5], void* packed_fwd,
+                        void* packed_dgrad, bool fp32_source, void* stream) {
   MfmaPackItem jobs[2];
   int njobs = 0;
-  if (int rc = collect_pack_jobs(p, dtype, w, w_stride, packed_fwd, packed_dgrad, jobs, &njobs)) return rc;
+  if (int rc = collect_pack_jobs(p, dtype, w, w_stride, packed_fwd, packed_dgrad, jobs, &njobs, fp32_source)) return rc;
   if (njobs == 0) return SFH_OK;
   return mfma_pack_weight_batch(jobs, njobs, dtype, (hipStream_t)stream);
+}
+
+extern "C" int sfh_conv3d_pack_weights(const sfh_conv3d_desc* p, int dtype, const void* w, const int64_t w_stride[5], void* packed_fwd,
+                                       void* packed_dgrad, void* stream) {
+  return pack_weights(p, dtype, w, w_stride, packed_fwd, packed_dgrad, false, stream);
+}
+
+extern "C" int sfh_conv3d_pack_master_weights(const sfh_conv3d_desc* p, int dtype, const float* w, const int64_t w_stride[5], void* packed_fwd,
+                                              void* packed_dgrad, void* stream) {
+  return pack_weights(p, dtype, w, w_stride, packed_fwd, packed_dgrad, true, stream);
 }
 
 extern "C" int sfh_conv3d_pack_weights_batch(const sfh_pack_item* items, int32_t nitems, int dtype, void* stream) {

@@ -24,6 +24,7 @@
 // padding k-1-p (triton_conv3d/bwd_data.py:344-363).
 #include "conv_mfma.hpp"
 #include "mma.hpp"
+#include "vec_io.hpp"
 #include "gn_stats.hpp"
 #include "reduce.hpp"
 
@@ -296,16 +297,15 @@ struct PackJob {
   const void* w;
   void* packed;
   int cout, cred;
-  int taps;  // kd | kh << 8 | kw << 16 | flip << 24 (one word: 48 jobs fit a 4 KB table of kernel arguments)
+  int taps;  // kd | kh << 8 | kw << 16 | flip << 24 | fp32 source << 25 (one word: 48 jobs fit a 4 KB table of kernel arguments)
   int64_t s_out, s_red, s_kd, s_kh, s_kw;
   int64_t pieces;
 };
 
 template <typename T>
 __device__ __forceinline__ void pack_piece(const PackJob& j, int64_t idx) {
-  const T* w = static_cast<const T*>(j.w);
   T* packed = static_cast<T*>(j.packed);
-  const int kh = (j.taps >> 8) & 0xff, kw = (j.taps >> 16) & 0xff, flip = j.taps >> 24;
+  const int kh = (j.taps >> 8) & 0xff, kw = (j.taps >> 16) & 0xff, flip = (j.taps >> 24) & 1;
   const int taps = (j.taps & 0xff) * kh * kw;
   int64_t r = idx;
   const int lane = (int)(r % 64); r /= 64;
@@ -318,7 +318,20 @@ __device__ __forceinline__ void pack_piece(const PackJob& j, int64_t idx) {
   const int ci = cc * kChunk + ks * 16 + (lane >> 5) * 8;
   if (flip) tap = taps - 1 - tap;
   const int tkw = tap % kw, tkh = (tap / kw) % kh, tkd = tap / (kw * kh);
-  const T* src = w + co * j.s_out + ci * j.s_red + tkd * j.s_kd + tkh * j.s_kh + tkw * j.s_kw;
+  const int64_t at = co * j.s_out + ci * j.s_red + tkd * j.s_kd + tkh * j.s_kh + tkw * j.s_kw;
+  if (j.taps >> 25) {  // an fp32 master weight: rounded here, once, instead of by a cast of its own in front
+    const float* src = static_cast<const float*>(j.w) + at;
+    float f[8];
+    if (j.s_red == 1 && (reinterpret_cast<uintptr_t>(src) & 15) == 0) {
+      Ld<float, 8>::run(src, f);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] = src[e * j.s_red];
+    }
+    St<T, 8>::run(packed + idx * 8, f);
+    return;
+  }
+  const T* src = static_cast<const T*>(j.w) + at;
   uint4 v;
   if (j.s_red == 1 && (reinterpret_cast<uintptr_t>(src) & 15) == 0) {
     v = *reinterpret_cast<const uint4*>(src);
@@ -513,10 +526,10 @@ size_t mfma_conv_packed_weight_bytes(const MfmaConvArgs& a) {
 
 namespace {
 PackJob pack_job(const MfmaConvArgs& a, const void* w, int64_t s_out, int64_t s_red, int64_t s_kd, int64_t s_kh, int64_t s_kw, int flip,
-                 void* packed) {
+                 void* packed, bool fp32_source = false) {
   PackJob j{};
   j.w = w; j.packed = packed;
-  j.cout = a.cout; j.cred = a.cred; j.taps = a.kd | (a.kh << 8) | (a.kw << 16) | ((flip ? 1 : 0) << 24);  // (kernel extents are at most 3)
+  j.cout = a.cout; j.cred = a.cred; j.taps = a.kd | (a.kh << 8) | (a.kw << 16) | ((flip ? 1 : 0) << 24) | ((fp32_source ? 1 : 0) << 25);  // (kernel extents are at most 3)
   j.s_out = s_out; j.s_red = s_red; j.s_kd = s_kd; j.s_kh = s_kh; j.s_kw = s_kw;
   j.pieces = (int64_t)a.cout * a.cred * a.kd * a.kh * a.kw / 8;  // 16-byte pieces
   return j;
@@ -543,7 +556,7 @@ int mfma_pack_weight_batch(const MfmaPackItem* items, int n, int dtype, hipStrea
     int64_t blocks = 0;
     for (int i = i0; i < n && i < i0 + kPackBatch; ++i) {
       const MfmaPackItem& it = items[i];
-      const PackJob job = pack_job(it.a, it.w, it.s_out, it.s_red, it.s_kd, it.s_kh, it.s_kw, it.flip, it.packed);
+      const PackJob job = pack_job(it.a, it.w, it.s_out, it.s_red, it.s_kd, it.s_kh, it.s_kw, it.flip, it.packed, it.fp32_source);
       if (job.pieces <= 0) continue;
       b.job[b.njobs] = job;
       b.first_block[b.njobs] = (int)blocks;

@@ -33,6 +33,7 @@ struct MfmaPackItem {
   int64_t s_out, s_red, s_kd, s_kh, s_kw;
   int flip;
   void* packed;
+  bool fp32_source;  // `w` is fp32: rounded to the packed dtype on the way
 };
 int mfma_pack_weight_batch(const MfmaPackItem* items, int n, int dtype, hipStream_t st);
 // Bytes of fp32 slices the kernel needs when it cuts the reduction channels to fill the chip (0 when it does not).

@@ -181,9 +181,9 @@ bool bias_fits(const MaybeTensor& b, const Tensor& x, int64_t channels) {
 
 // The gate of the forward (conv3d.is_supported), and with `all` of both gradients too (is_supported_all).
 bool conv_gate(const Tensor& x, const Tensor& w, const MaybeTensor& bias, const int32_t s[3], const int32_t p[3], const int32_t d[3],
-               bool all, Problem& prob, int64_t more_channels = 0) {
+               bool all, Problem& prob, int64_t more_channels = 0, bool packed = false) {
   if (x.dim() != 5 || w.dim() != 5 || !on_gpu(x) || !on_gpu(w) || x.device() != w.device()) return false;
-  if (x.scalar_type() != w.scalar_type() || x.size(1) + more_channels != w.size(1)) return false;
+  if ((x.scalar_type() != w.scalar_type() && !packed) || x.size(1) + more_channels != w.size(1)) return false;
   if (!bias_fits(bias, x, w.size(0))) return false;
   const int64_t in[5] = {x.size(0), w.size(1), x.size(2), x.size(3), x.size(4)};
   if (!make_problem(in, w.sizes(), s, p, d, code_of(x.scalar_type()), prob)) return false;
@@ -425,7 +425,7 @@ py::object conv_forward(const Tensor& x, const Tensor& w, const MaybeTensor& bia
   int32_t s[3], p[3], d[3];
   if (!three(stride, s) || !three(padding, p) || !three(dilation, d)) return py::none();
   Problem prob;
-  if (!conv_gate(x, w, bias, s, p, d, false, prob, second.has_value() && second->dim() == 5 ? second->size(1) : 0)) return py::none();
+  if (!conv_gate(x, w, bias, s, p, d, false, prob, second.has_value() && second->dim() == 5 ? second->size(1) : 0, packed.has_value())) return py::none();
   if (packed.has_value() && !packed_fits(*packed, prob.sizes->packed[0], x)) return py::none();
   if (second.has_value() && (second->dim() != 5 || !on_gpu(*second) || second->device() != x.device() || second->scalar_type() != x.scalar_type() ||
                              second->size(0) != x.size(0) || second->size(2) != x.size(2) || second->size(3) != x.size(3) || second->size(4) != x.size(4)))
@@ -435,10 +435,12 @@ py::object conv_forward(const Tensor& x, const Tensor& w, const MaybeTensor& bia
 }
 
 // conv3d.is_supported_all for exact argument kinds (False also where the Python gate has to look closer)
-bool conv_supported(const Tensor& x, const Tensor& w, const MaybeTensor& bias, py::handle stride, py::handle padding, py::handle dilation, bool all) {
+// `packed`: the kernels read packed forms, w may be the fp32 master they were made from
+bool conv_supported(const Tensor& x, const Tensor& w, const MaybeTensor& bias, py::handle stride, py::handle padding, py::handle dilation, bool all,
+                    bool packed) {
   int32_t s[3], p[3], d[3];
   Problem prob;
-  return three(stride, s) && three(padding, p) && three(dilation, d) && conv_gate(x, w, bias, s, p, d, all, prob);
+  return three(stride, s) && three(padding, p) && three(dilation, d) && conv_gate(x, w, bias, s, p, d, all, prob, 0, packed);
 }
 
 // conv3d.conv3d_backward_data
@@ -472,6 +474,24 @@ py::object conv_backward_weight(const Tensor& x, at::IntArrayRef w_sizes, const 
   for (int i = 0; i < 3; ++i)
     if (grad_output.size(2 + i) != prob.out[i]) return py::none();
   return py::cast(launch_wgrad(prob, dense(x), Tensor(), dense(grad_output), false));
+}
+
+// The packed forms of an fp32 master weight for a 16-bit convolution of an input of `in_sizes`, in one launch:
+// (packed_fwd, packed_dgrad, complete).  A form is None when that direction does not read one or (data gradient) was not
+// asked for; `complete`: every direction asked for has its form, so nobody reads the weight itself.
+py::object pack_master(const Tensor& weight, at::ScalarType dtype, at::IntArrayRef in_sizes, py::handle stride, py::handle padding, py::handle dilation,
+                       bool want_dgrad) {
+  int32_t s[3], p[3], d[3];
+  Problem prob;
+  if (!three(stride, s) || !three(padding, p) || !three(dilation, d) || weight.scalar_type() != at::kFloat || !on_gpu(weight) ||
+      !make_problem(in_sizes, weight.sizes(), s, p, d, code_of(dtype), prob))
+    return py::make_tuple(py::none(), py::none(), false);
+  c10::OptionalDeviceGuard guard(weight.device());
+  const Tensor pf = bytes(prob.sizes->packed[0], weight), pd = want_dgrad ? bytes(prob.sizes->packed[1], weight) : Tensor();
+  if (pf.defined() || pd.defined())
+    check(sfh_conv3d_pack_master_weights(prob.desc(), prob.key.code, (const float*)ptr(weight), weight.strides().data(), out_ptr(pf), out_ptr(pd),
+                                         stream_of(weight)), "pack_weights");
+  return py::make_tuple(tensor_or_none(pf), tensor_or_none(pd), pf.defined() && (pd.defined() || !want_dgrad));
 }
 
 // ---- the 2x2x2-like transposed convolution (kernel == stride) ------------------------------------------------------------
@@ -531,7 +551,8 @@ py::object conv_transpose(const Tensor& x_in, const Tensor& weight, const MaybeT
                           const MaybeTensor& packed_fwd, const MaybeTensor& packed_dgrad, int64_t halo, bool master) {
   int32_t k[3];
   if (!three(stride, k) || x_in.dim() != 5 || w.dim() != 5 || !on_gpu(x_in) || !on_gpu(w) || x_in.device() != w.device()) return py::none();
-  if (x_in.scalar_type() != w.scalar_type() || x_in.size(1) != w.size(0) || !bias_fits(b, x_in, w.size(1))) return py::none();
+  const bool all_packed = packed_fwd.has_value() && packed_dgrad.has_value();  // the weight itself is then not read
+  if ((x_in.scalar_type() != w.scalar_type() && !all_packed) || x_in.size(1) != w.size(0) || !bias_fits(b, x_in, w.size(1))) return py::none();
   int64_t big[5] = {x_in.size(0), w.size(1), 0, 0, 0};
   for (int i = 0; i < 3; ++i) {
     if (k[i] < 1 || w.size(2 + i) != k[i] || x_in.size(2 + i) < 1) return py::none();
@@ -848,6 +869,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("set_weight_queue", &set_weight_queue);
   m.def("conv_forward", &conv_forward);
   m.def("conv_supported", &conv_supported);
+  m.def("pack_master", &pack_master);
   m.def("conv_backward_data", &conv_backward_data);
   m.def("conv_backward_weight", &conv_backward_weight);
   m.def("record_conv", &record_conv);

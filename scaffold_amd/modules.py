@@ -232,6 +232,23 @@ def _queue_from_node(param, x, second, gy, padding, master, family, early) -> No
 _node_queue_set = False
 
 
+def _narrowed(weight, bias, dt, x_dtype) -> bool:
+    """Whether autocast narrows these parameters to the 16-bit dtype of the activations."""
+    return dt in (torch.bfloat16, torch.float16) and x_dtype is dt and weight.dtype is torch.float32 and weight.is_cuda \
+        and (bias is None or bias.dtype is torch.float32 or bias.dtype is dt)
+
+
+def _master_operands(weight, bias, dt, in_shape, stride, padding, dilation, want_dgrad):
+    """What the kernels read of fp32 parameters under 16-bit autocast when nobody keeps half-precision copies:
+    ``(w, b, (packed_fwd, packed_dgrad), complete)``.  The packed forms come from the master in one launch, rounded on the
+    way; only a direction that reads the weight where it lies (the stem, the 1x1x1 head) needs a cast of it.  The parameters'
+    gradients are then produced in fp32 directly: no cast nodes either way."""
+    pf, pd, complete = _lib.native().pack_master(weight, dt, in_shape, stride, padding, dilation, want_dgrad)
+    w = weight if complete else weight.detach().to(dt)
+    b = None if bias is None else (bias if bias.dtype is dt else bias.detach().to(dt))
+    return w, b, (pf, pd), complete
+
+
 def _run_conv(x, second, x_read, second_read, weight, bias, w, b, packs, halo, stride, padding, dilation, master, gn_groups, defer):
     """The forward launch of a convolution and its autograd node.  ``x`` / ``second`` are the tensors that receive gradients,
     ``x_read`` / ``second_read`` what the kernels read (slabs of which x and second are the depth interiors when ``halo`` > 0,
@@ -242,8 +259,7 @@ def _run_conv(x, second, x_read, second_read, weight, bias, w, b, packs, halo, s
     pf = pd = None
     in_shape = x_read.shape if second is None else torch.Size((x_read.shape[0], x_read.shape[1] + second_read.shape[1], *x_read.shape[2:]))
     if packs is not None:
-        # packed forms that are current (kept by the module, refreshed by whoever writes the weight)
-        pf, pd = packs.fwd, packs.dgrad
+        pf, pd = packs
     elif torch.is_grad_enabled() and x.requires_grad and (PACK_WEIGHTS_ONCE or torch.cuda.is_current_stream_capturing()):
         # When the data gradient will be wanted too, the weight can be packed for both directions in one launch.
         # That saves a launch per convolution on the GPU and costs a little more host time, so it is done where
@@ -343,6 +359,24 @@ class FastConv3d(nn.Conv3d):
             table[key] = ok
         return ok
 
+    def _kernel_operands(self, weight, bias, dt, x_dtype, in_shape, stride, padding, dilation, want_dgrad):
+        """``(w, b, packs, master, complete)``: what the kernels read of the parameters (``packs``: the packed forms that are
+        current, or None), whether the parameters are fp32 masters whose gradients are produced in fp32 directly, and whether
+        the packed forms are all that is read (``w`` is then the master itself)."""
+        # under autocast, up-to-date half-precision copies kept by the optimizer, with their packed forms
+        wc = compute_copy(weight, dt)
+        if wc is not None:
+            bc = compute_copy(bias, dt)
+            if bias is None or bc is not None:
+                packs = _current_packs(weight, wc, in_shape, stride, padding, dilation)
+                return wc, bc, None if packs is None else (packs.fwd, packs.dgrad), True, False
+        if _narrowed(weight, bias, dt, x_dtype) and self.groups == 1:
+            w, b, packs, complete = _master_operands(weight, bias, dt, in_shape, stride, padding, dilation, want_dgrad)
+            return w, b, packs, True, complete
+        w, b = cast_operand(weight, dt), cast_operand(bias, dt)
+        packs = _current_packs(w, w, in_shape, stride, padding, dilation) if w is weight else None
+        return w, b, None if packs is None else (packs.fwd, packs.dgrad), False, False
+
     def _forward_pair(self, x, second):
         ops = self._pair_operands(x, second)
         if ops is None:
@@ -351,25 +385,17 @@ class FastConv3d(nn.Conv3d):
         x_read, second_read, padding, slab, slab2 = ops
         dt = autocast_dtype(x)
         weight, bias = self.weight, self.bias  # (each lookup of a parameter is a call into Module.__getattr__)
-        wc = compute_copy(weight, dt)
-        bc = compute_copy(bias, dt) if wc is not None else None
-        master = wc is not None and (bias is None or bc is not None)
-        w = wc if master else cast_operand(weight, dt)
-        b = bc if master else cast_operand(bias, dt)
         stride, dilation = tuple(self.stride), tuple(self.dilation)
-        if w.dtype is not x_read.dtype or not self._pair_gate(x_read, second_read, padding):
+        in_shape = torch.Size((x_read.shape[0], x_read.shape[1] + second_read.shape[1], *x_read.shape[2:]))
+        want_dgrad = torch.is_grad_enabled() and (x.requires_grad or second.requires_grad)
+        w, b, packs, master, complete = self._kernel_operands(weight, bias, dt, x_read.dtype, in_shape, stride, padding, dilation, want_dgrad)
+        if not (complete or w.dtype is x_read.dtype) or not self._pair_gate(x_read, second_read, padding):
             raise NotImplementedError(
                 f"FastConv3d: pair not served: x={tuple(x_read.shape)}/{x_read.dtype} second={tuple(second_read.shape)} on {x.device}, "
                 f"weight={tuple(w.shape)}/{w.dtype}, stride={stride} padding={padding} dilation={dilation}")
-        in_shape = torch.Size((x_read.shape[0], x_read.shape[1] + second_read.shape[1], *x_read.shape[2:]))
         halo = 0 if slab is None else slab[1]
-        if master:
-            packs = _current_packs(weight, w, in_shape, stride, padding, dilation)
-            return _run_conv(x, second, x_read, second_read, weight, bias, w, b, packs, halo, stride, padding, dilation, True,
-                             self.gn_groups, self.defer_weight_grad)
-        packs = _current_packs(w, w, in_shape, stride, padding, dilation) if w is weight else None
-        return _run_conv(x, second, x_read, second_read, w, b, w, b, packs, halo, stride, padding, dilation, False, self.gn_groups,
-                         self.defer_weight_grad if w is weight else False)
+        return _run_conv(x, second, x_read, second_read, weight if master else w, bias if master else b, w, b, packs, halo, stride, padding,
+                         dilation, master, self.gn_groups, self.defer_weight_grad if master or w is weight else False)
 
     def forward(self, x: torch.Tensor, second: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``second``: the input is ``torch.cat([x, second], 1)``, read from the two tensors themselves (the decoder's skip
@@ -381,12 +407,6 @@ class FastConv3d(nn.Conv3d):
         dt = autocast_dtype(x)
         x = cast_operand(x, dt)
         weight, bias = self.weight, self.bias  # (each lookup of a parameter is a call into Module.__getattr__)
-        # under autocast, an up-to-date half-precision copy kept by the optimizer replaces the per-call cast
-        wc = compute_copy(weight, dt)
-        bc = compute_copy(bias, dt) if wc is not None else None
-        master = wc is not None and (bias is None or bc is not None)
-        w = wc if master else cast_operand(weight, dt)
-        b = bc if master else cast_operand(bias, dt)
         padding = tuple(self.padding)
         inner, slab = x, None
         if self.shard_halo and padding[0] > 0:
@@ -402,9 +422,11 @@ class FastConv3d(nn.Conv3d):
         x = x.contiguous(memory_format=_CL3D)
         # the node below skips its own gates on the strength of this one (a call that will be differentiated is
         # gated for all three directions here)
-        wants = _wants_grad(inner, w, b)
+        wants = _wants_grad(inner, weight, bias)
         stride, dilation = tuple(self.stride), tuple(self.dilation)
-        if self.groups != 1 or not (_lib.native().conv_supported(x, w, b, stride, padding, dilation, wants) or
+        w, b, packs, master, complete = self._kernel_operands(weight, bias, dt, x.dtype, x.shape, stride, padding, dilation,
+                                                              wants and inner.requires_grad)
+        if self.groups != 1 or not (_lib.native().conv_supported(x, w, b, stride, padding, dilation, wants, complete) or
                                     (_c3.is_supported_all if wants else _c3.is_supported)(x, w, b, stride, padding, dilation, 1)):
             raise NotImplementedError(
                 f"FastConv3d: not served: x={tuple(x.shape)}/{x.dtype} on {x.device}, weight={tuple(w.shape)}/{w.dtype}, "
@@ -413,13 +435,8 @@ class FastConv3d(nn.Conv3d):
         if slab is None:
             inner = x
         halo = 0 if slab is None else slab[1]
-        if master:
-            packs = _current_packs(weight, w, x.shape, stride, padding, dilation)
-            return _run_conv(inner, None, x, None, weight, bias, w, b, packs, halo, stride, padding, dilation, True, self.gn_groups,
-                             self.defer_weight_grad)
-        packs = _current_packs(w, w, x.shape, stride, padding, dilation) if w is weight else None
-        return _run_conv(inner, None, x, None, w, b, w, b, packs, halo, stride, padding, dilation, False, self.gn_groups,
-                         self.defer_weight_grad if w is weight else False)
+        return _run_conv(inner, None, x, None, weight if master else w, bias if master else b, w, b, packs, halo, stride, padding, dilation,
+                         master, self.gn_groups, self.defer_weight_grad if master or w is weight else False)
 
 
 class FastConvTranspose3d(nn.ConvTranspose3d):
@@ -437,19 +454,23 @@ class FastConvTranspose3d(nn.ConvTranspose3d):
         wc = compute_copy(weight, dt)
         bc = compute_copy(bias, dt) if wc is not None else None
         master = wc is not None and (bias is None or bc is not None)
-        w = wc if master else cast_operand(weight, dt)
-        b = bc if master else cast_operand(bias, dt)
-        stride, done = tuple(self.stride), None
-        if self.groups == 1 and tuple(self.padding) == tuple(self.output_padding) == (0, 0, 0) and tuple(self.dilation) == (1, 1, 1):
-            packs = None
-            if (master or w is weight) and x.dim() == 5:
-                # the problem the packed forms belong to: the stride-k convolution over this op's output
-                n, _, d, h, wd = x.shape
-                big = torch.Size((n, w.shape[1], d * stride[0], h * stride[1], wd * stride[2]))
-                packs = _current_packs(weight, w, big, stride, (0, 0, 0), (1, 1, 1))
-                if packs is not None and (packs.fwd is None or packs.dgrad is None):
-                    packs = None
-            pf, pd = (None, None) if packs is None else (packs.fwd, packs.dgrad)
+        stride, done, w, b = tuple(self.stride), None, weight, bias
+        if self.groups == 1 and tuple(self.padding) == tuple(self.output_padding) == (0, 0, 0) and tuple(self.dilation) == (1, 1, 1) \
+                and x.dim() == 5:
+            # the problem the packed forms belong to: the stride-k convolution over this op's output
+            n, _, d, h, wd = x.shape
+            big = torch.Size((n, weight.shape[1], d * stride[0], h * stride[1], wd * stride[2]))
+            pf = pd = None
+            if not master and _narrowed(weight, bias, dt, x.dtype):
+                w, b, (pf, pd), _ = _master_operands(weight, bias, dt, big, stride, (0, 0, 0), (1, 1, 1), True)
+                master = True
+            else:
+                w, b = (wc, bc) if master else (cast_operand(weight, dt), cast_operand(bias, dt))
+                packs = _current_packs(weight, w, big, stride, (0, 0, 0), (1, 1, 1)) if master or w is weight else None
+                if packs is not None:
+                    pf, pd = packs.fwd, packs.dgrad
+            if pf is None or pd is None:
+                pf = pd = None
             done = _lib.native().conv_transpose(x, weight if master else w, bias if master else b, w, b, stride, pf, pd,
                                                 self.out_halo, master)
         if done is None:
