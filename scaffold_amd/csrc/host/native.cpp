@@ -12,13 +12,16 @@
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/engine.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <unordered_map>
 
@@ -36,7 +39,8 @@ using MaybeTensor = std::optional<Tensor>;
 // ---- the Python side -----------------------------------------------------------------------------------------------------
 PyObject* g_kernel_error = nullptr;    // scaffold_amd._lib.ScaffoldKernelError
 PyObject* g_note_device = nullptr;     // scaffold_amd._lib._note_device(device)
-PyObject* g_queue_weight = nullptr;    // scaffold_amd.modules._queue_from_node(...)
+PyObject* g_send_early = nullptr;      // scaffold_amd.modules._send_early_batch(batch)
+PyObject* g_join_early = nullptr;      // scaffold_amd.modules._join_early()
 
 // A status code as the exception the entry points raise (the interpreter lock is taken if this thread does not hold it).
 void check(int rc, const char* what) {
@@ -324,6 +328,153 @@ bool wants_grad(std::initializer_list<const Tensor*> ts) {
 
 Tensor or_none(const MaybeTensor& t) { return t.has_value() ? *t : Tensor(); }
 
+// ---- weight gradients of a backward pass in one launch ---------------------------------------------------------------------
+// See scaffold_amd/modules.py: a convolution whose module defers leaves (parameter, operands) here instead of computing its
+// weight gradient; when the pass ends -- still inside backward() -- all that the pass queued are computed by one batched
+// call and added to the parameters' .grad.  The queue is kept per backward pass (graph task), so passes that run at the
+// same time on other threads or streams never take each other's entries.
+struct QueuedWeight {
+  Tensor param, x, second, gy;
+  int32_t p[3];
+  bool master = false, early = false;
+  int family = 1;  // the launch of the batch that takes it (1: large rows, 2: small volumes)
+};
+
+struct WeightBatch {
+  std::vector<QueuedWeight> items;
+  std::vector<Tensor> grads;
+  size_t size() const { return items.size(); }
+};
+
+struct PassQueue {
+  std::vector<QueuedWeight> items;
+  std::vector<std::shared_ptr<WeightBatch>> sent;  // on their way on a side stream
+};
+
+std::mutex g_pass_lock;
+std::unordered_map<int, PassQueue> g_passes;
+
+// The gradients of `batch` (one device, operand dtype and gradient dtype) on the current stream, in calls of at most
+// SFH_WGRAD_BATCH_MAX problems filled family by family.
+void launch_batch(WeightBatch& batch, bool share_device) {
+  if (batch.items.empty()) return;
+  const Tensor& like = batch.items[0].gy;
+  c10::OptionalDeviceGuard guard(like.device());
+  const int code = code_of(like.scalar_type());
+  const bool fp32 = batch.items[0].master;
+  const uint32_t flags = (fp32 ? SFH_FLAG_GRAD_FP32 : 0) | (share_device ? SFH_FLAG_SHARE_DEVICE : 0);
+  std::vector<sfh_conv3d_wgrad_item> work(batch.items.size());
+  const int32_t one[3] = {1, 1, 1};
+  for (size_t i = 0; i < batch.items.size(); ++i) {
+    const QueuedWeight& q = batch.items[i];
+    int64_t in[5];
+    std::copy(q.x.sizes().begin(), q.x.sizes().end(), in);
+    if (q.second.defined()) in[1] += q.second.size(1);
+    Problem prob;
+    TORCH_INTERNAL_ASSERT(make_problem(in, q.param.sizes(), one, q.p, one, code, prob));
+    batch.grads.push_back(volume(q.param.sizes(), like, fp32 ? at::kFloat : like.scalar_type()));
+    work[i] = sfh_conv3d_wgrad_item{prob.key.d, ptr(q.x), ptr(q.second), q.second.defined() ? (int32_t)q.x.size(1) : 0, ptr(q.gy), out_ptr(batch.grads[i])};
+  }
+  for (int family = 1; family <= 2; ++family) {
+    std::vector<sfh_conv3d_wgrad_item> call;
+    auto send = [&] {
+      if (call.empty()) return;
+      const size_t need = sfh_conv3d_wgrad_batch_workspace_bytes(call.data(), (int32_t)call.size(), code, flags);
+      const Tensor ws = bytes(need, like);
+      check(sfh_conv3d_wgrad_batch(call.data(), (int32_t)call.size(), code, out_ptr(ws), need, flags, stream_of(like)), "conv3d_backward_weight_batch");
+      call.clear();
+    };
+    for (size_t i = 0; i < work.size(); ++i) {
+      if (batch.items[i].family != family) continue;
+      call.push_back(work[i]);
+      if (call.size() == SFH_WGRAD_BATCH_MAX) send();
+    }
+    send();
+  }
+}
+
+void add_to_grads(WeightBatch& batch) {
+  for (size_t i = 0; i < batch.items.size(); ++i) {
+    const Tensor &param = batch.items[i].param, &gw = batch.grads[i];
+    Tensor& grad = param.mutable_grad();
+    if (grad.defined()) grad.add_(gw);
+    else grad = gw.strides() == param.strides() ? gw : at::empty_like(param).copy_(gw);  // the parameter's own layout, as the engine leaves it
+  }
+}
+
+// Computes what a pass has queued and adds it (no entry: nothing to do).
+void finish_pass(int id) {
+  PassQueue pass;
+  {
+    std::lock_guard<std::mutex> hold(g_pass_lock);
+    auto it = g_passes.find(id);
+    if (it == g_passes.end()) return;
+    pass = std::move(it->second);
+    g_passes.erase(it);
+  }
+  at::AutoGradMode no_grad(false);
+  if (!pass.sent.empty()) {
+    py::gil_scoped_acquire gil;
+    py::reinterpret_borrow<py::function>(g_join_early)();
+  }
+  for (auto& batch : pass.sent) add_to_grads(*batch);
+  while (!pass.items.empty()) {
+    WeightBatch batch;
+    std::vector<QueuedWeight> rest;
+    for (auto& q : pass.items) {
+      const bool same = batch.items.empty() || (q.gy.device() == batch.items[0].gy.device() && q.gy.scalar_type() == batch.items[0].gy.scalar_type() &&
+                                                q.master == batch.items[0].master);
+      (same ? batch.items : rest).push_back(std::move(q));
+    }
+    pass.items = std::move(rest);
+    launch_batch(batch, false);
+    add_to_grads(batch);
+  }
+}
+
+void finish_all_passes() {
+  std::vector<int> ids;
+  {
+    std::lock_guard<std::mutex> hold(g_pass_lock);
+    for (const auto& kv : g_passes) ids.push_back(kv.first);
+  }
+  for (int id : ids) finish_pass(id);
+}
+
+void queue_weight(QueuedWeight&& q) {
+  const int id = torch::autograd::get_current_graph_task_id();
+  std::shared_ptr<WeightBatch> leave;
+  {
+    std::lock_guard<std::mutex> hold(g_pass_lock);
+    auto found = g_passes.find(id);
+    if (found == g_passes.end()) {
+      torch::autograd::Engine::get_default_engine().queue_callback([id] { finish_pass(id); });
+      found = g_passes.emplace(id, PassQueue{}).first;
+    }
+    auto& items = found->second.items;
+    if (q.early && q.family == 2) {
+      // The pass has reached a small volume: the deep levels, whose kernels are bound by latency and leave most of the
+      // device idle.  The large-row gradients queued so far (the decoder's upper levels) go out now, on a stream of their
+      // own and on half of the compute units, beside the rest of the pass.
+      auto goes = [&](const QueuedWeight& o) {
+        return o.family == 1 && o.early && o.gy.device() == q.gy.device() && o.gy.scalar_type() == q.gy.scalar_type() && o.master == q.master;
+      };
+      if (std::count_if(items.begin(), items.end(), goes) >= 2) {
+        leave = std::make_shared<WeightBatch>();
+        std::vector<QueuedWeight> rest;
+        for (auto& o : items) (goes(o) ? leave->items : rest).push_back(std::move(o));
+        items = std::move(rest);
+        found->second.sent.push_back(leave);
+      }
+    }
+    items.push_back(std::move(q));
+  }
+  if (leave) {
+    py::gil_scoped_acquire gil;
+    py::reinterpret_borrow<py::function>(g_send_early)(leave);
+  }
+}
+
 // The convolution over x, or over the pair (x, second).  Edges: x, weight, bias, second.  In the depth-shard form the
 // tensors that are saved are slabs of which x and second are the depth interiors.
 struct ConvNode : public LaunchNode {
@@ -376,9 +527,7 @@ struct ConvNode : public LaunchNode {
       }
     }
     if (need_w && param.defined()) {
-      py::gil_scoped_acquire gil;
-      py::reinterpret_borrow<py::function>(g_queue_weight)(py::cast(param), py::cast(xs), pair ? py::cast(x2) : py::none(), py::cast(gy),
-                                                           py::make_tuple(p[0], p[1], p[2]), master, family, early);
+      queue_weight(QueuedWeight{param, xs, x2, gy, {p[0], p[1], p[2]}, master, early, family});
     } else if (need_w) {
       out[1] = launch_wgrad(prob, xs, x2, gy, master);
     }
@@ -860,13 +1009,20 @@ void set_callbacks(py::object kernel_error, py::object note_device) {
   g_kernel_error = kernel_error.release().ptr();
   g_note_device = note_device.release().ptr();
 }
-void set_weight_queue(py::object queue) { g_queue_weight = queue.release().ptr(); }
+void set_early_callbacks(py::object send, py::object join) {
+  g_send_early = send.release().ptr();
+  g_join_early = join.release().ptr();
+}
 
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("set_callbacks", &set_callbacks);
-  m.def("set_weight_queue", &set_weight_queue);
+  m.def("set_early_callbacks", &set_early_callbacks);
+  py::class_<WeightBatch, std::shared_ptr<WeightBatch>>(m, "WeightBatch").def("__len__", &WeightBatch::size);
+  m.def("launch_batch", [](WeightBatch& batch, bool share_device) { launch_batch(batch, share_device); });
+  m.def("batch_device", [](const WeightBatch& batch) { return batch.items.at(0).gy.device(); });
+  m.def("finish_all_passes", &finish_all_passes);
   m.def("conv_forward", &conv_forward);
   m.def("conv_supported", &conv_supported);
   m.def("pack_master", &pack_master);

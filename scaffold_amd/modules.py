@@ -107,23 +107,22 @@ def _current_packs(owner: torch.Tensor, source: torch.Tensor, in_shape, stride, 
 # ---- weight gradients of a backward pass in one launch -----------------------------------------------------------------
 # Nothing reads a weight gradient before the optimizer (``ScaFFold/utils/trainer.py:678-694``), and a launch of the
 # weight-gradient kernel costs 15-20 us whatever the problem.  A convolution whose module has ``defer_weight_grad`` set
-# therefore does not compute its weight gradient in its own backward node: the node leaves (parameter, operands) in a
-# queue and returns no gradient for the weight, and a callback the autograd engine runs when the backward pass has
-# finished -- still inside ``backward()`` -- computes all queued gradients with :func:`conv3d_backward_weight_batch` and
+# therefore does not compute its weight gradient in its own backward node: the node leaves (parameter, operands) in the
+# pass's queue (``csrc/host/native.cpp``) and returns no gradient for the weight, and a callback the autograd engine runs
+# when the backward pass has finished -- still inside ``backward()`` -- computes all queued gradients in one batched call and
 # adds them to the parameters' ``.grad``.  After ``backward()`` returns the gradients are where they always are.  What
 # differs: hooks on the parameter's gradient accumulation do not see these gradients, and the operands stay alive until
 # the end of the pass.
 class _QueuedWeightGrad:
-    __slots__ = ("param", "inp", "wshape", "gy", "padding", "grad_dtype", "family", "early")
+    __slots__ = ("param", "inp", "wshape", "gy", "padding", "grad_dtype")
 
-    def __init__(self, param, inp, wshape, gy, padding, grad_dtype, family=1, early=False):
+    def __init__(self, param, inp, wshape, gy, padding, grad_dtype):
         self.param, self.inp, self.wshape, self.gy, self.padding, self.grad_dtype = param, inp, wshape, gy, padding, grad_dtype
-        self.family, self.early = family, early  # the launch that takes it (1: large rows, 2: small volumes); early mode
 
 
+#: weight gradients queued by hand, for ``flush_weight_gradients()`` (a backward pass keeps its own queue)
 _WEIGHT_GRAD_QUEUE: list = []
 _BATCHABLE: dict = {}
-
 
 #: A weight gradient of more operations than this is computed in its own node although the module defers.  What a place
 #: in the batch saves is a launch and a slice sum (20 us), a tenth of such a problem's time; what it costs is that the
@@ -154,63 +153,34 @@ def _deferrable(param, in_shape, wshape, stride, padding, dilation, dtype) -> in
     return ok
 
 
-def _queue_weight_grad(item: _QueuedWeightGrad) -> None:
-    _WEIGHT_GRAD_QUEUE.append(item)
-    # one callback per queued gradient: the first to run takes the whole queue, the others find it empty (a pass that
-    # raised before its callbacks ran leaves its entries to the next pass's callbacks, or to flush_weight_gradients())
-    torch.autograd.Variable._execution_engine.queue_callback(flush_weight_gradients)
-    if item.early and item.family == 2:
-        # The pass has reached a small volume: the deep levels, whose kernels are bound by latency and leave most of the
-        # device idle. The large-row gradients queued so far (the decoder's upper levels) go out now, on a stream of their own
-        # and on half of the compute units, beside the rest of the pass; flush_weight_gradients() joins them.
-        waiting = [it for it in _WEIGHT_GRAD_QUEUE if it.family == 1 and it.early and it.gy.device == item.gy.device and
-                   it.gy.dtype is item.gy.dtype and it.grad_dtype is item.grad_dtype]
-        if len(waiting) >= 2:
-            for it in waiting:
-                _WEIGHT_GRAD_QUEUE.remove(it)
-            _send_early(waiting)
-
-
 _EARLY_STREAMS: dict = {}
 _EARLY_DONE: list = []
 
 
-def _send_early(items) -> None:
-    dev = items[0].gy.device
+def _send_early(batch) -> None:
+    dev = _lib.native().batch_device(batch)
     side = _EARLY_STREAMS.get(dev)
     if side is None:
         side = _EARLY_STREAMS[dev] = torch.cuda.Stream(device=dev)
-    # Every use of the side stream starts by waiting for the current one and ends (in flush_weight_gradients) with the
+    # Every use of the side stream starts by waiting for the current one and ends (in _join_early) with the
     # current one waiting for it, and the operands stay referenced until then: memory the caching allocator hands to
     # either stream is never in use on the other.
     side.wait_stream(torch.cuda.current_stream(dev))
-    gdt, dt = items[0].grad_dtype, items[0].gy.dtype
     with torch.no_grad(), torch.cuda.stream(side):
-        grads = _c3.conv3d_backward_weight_batch([(it.inp, it.wshape, it.gy, it.padding) for it in items],
-                                                 grad_dtype=None if gdt is dt else gdt, share_device=True)
-    _EARLY_DONE.append((items, grads, side))
+        _lib.native().launch_batch(batch, True)
+    _EARLY_DONE.append((dev, side))
 
 
-def _add_to_grads(items, grads) -> None:
-    for it, gw in zip(items, grads):
-        p = it.param
-        if p.grad is None:
-            # in the parameter's own layout, as the engine's accumulation would leave it
-            p.grad = gw if gw.stride() == p.stride() else torch.empty_like(p).copy_(gw)
-        else:
-            p.grad.add_(gw)
+def _join_early() -> None:
+    while _EARLY_DONE:
+        dev, side = _EARLY_DONE.pop(0)
+        torch.cuda.current_stream(dev).wait_stream(side)
 
 
 def flush_weight_gradients() -> None:
-    """Compute the queued weight gradients and add them to their parameters' ``.grad`` (runs by itself at the end of a
-    backward pass; callable by hand after a pass that raised)."""
-    while _EARLY_DONE:
-        items, grads, side = _EARLY_DONE.pop(0)
-        torch.cuda.current_stream(items[0].gy.device).wait_stream(side)
-        with torch.no_grad():
-            _add_to_grads(items, grads)
-    if not _WEIGHT_GRAD_QUEUE:
-        return
+    """Compute the weight gradients that wait -- left by a pass that raised, or queued by hand -- and add them to their
+    parameters' ``.grad`` (a pass that ends does this by itself)."""
+    _lib.native().finish_all_passes()
     queue = list(_WEIGHT_GRAD_QUEUE)
     _WEIGHT_GRAD_QUEUE.clear()
     groups: dict = {}
@@ -220,16 +190,33 @@ def flush_weight_gradients() -> None:
         for (_, dt, gdt), items in groups.items():
             grads = _c3.conv3d_backward_weight_batch([(it.inp, it.wshape, it.gy, it.padding) for it in items],
                                                      grad_dtype=None if gdt is dt else gdt)
-            _add_to_grads(items, grads)
+            for it, gw in zip(items, grads):
+                p = it.param
+                if p.grad is None:
+                    # in the parameter's own layout, as the engine's accumulation would leave it
+                    p.grad = gw if gw.stride() == p.stride() else torch.empty_like(p).copy_(gw)
+                else:
+                    p.grad.add_(gw)
 
 
-def _queue_from_node(param, x, second, gy, padding, master, family, early) -> None:
-    """A convolution's backward node leaves its weight gradient to the end of the pass (called by the node)."""
-    _queue_weight_grad(_QueuedWeightGrad(param, x if second is None else (x, second), param.shape, gy, padding,
-                                         torch.float32 if master else x.dtype, family, early))
+_early_callbacks_set = False
 
 
-_node_queue_set = False
+def _narrowed(weight, bias, dt, x_dtype) -> bool:
+    """Whether autocast narrows these parameters to the 16-bit dtype of the activations."""
+    return dt in (torch.bfloat16, torch.float16) and x_dtype is dt and weight.dtype is torch.float32 and weight.is_cuda \
+        and (bias is None or bias.dtype is torch.float32 or bias.dtype is dt)
+
+
+def _master_operands(weight, bias, dt, in_shape, stride, padding, dilation, want_dgrad):
+    """What the kernels read of fp32 parameters under 16-bit autocast when nobody keeps half-precision copies:
+    ``(w, b, (packed_fwd, packed_dgrad), complete)``.  The packed forms come from the master in one launch, rounded on the
+    way; only a direction that reads the weight where it lies (the stem, the 1x1x1 head) needs a cast of it.  The parameters'
+    gradients are then produced in fp32 directly: no cast nodes either way."""
+    pf, pd, complete = _lib.native().pack_master(weight, dt, in_shape, stride, padding, dilation, want_dgrad)
+    w = weight if complete else weight.detach().to(dt)
+    b = None if bias is None else (bias if bias.dtype is dt else bias.detach().to(dt))
+    return w, b, (pf, pd), complete
 
 
 def _narrowed(weight, bias, dt, x_dtype) -> bool:
@@ -255,7 +242,7 @@ def _run_conv(x, second, x_read, second_read, weight, bias, w, b, packs, halo, s
     else the same tensors).  ``weight`` / ``bias`` receive gradients, ``w`` / ``b`` are what the kernels read: when half-precision
     copies of fp32 masters are given (``master``) the gradients are produced in the masters' dtype directly.  The caller has
     passed the gate (for all three directions when the call will be differentiated)."""
-    global _node_queue_set
+    global _early_callbacks_set
     pf = pd = None
     in_shape = x_read.shape if second is None else torch.Size((x_read.shape[0], x_read.shape[1] + second_read.shape[1], *x_read.shape[2:]))
     if packs is not None:
@@ -273,9 +260,10 @@ def _run_conv(x, second, x_read, second_read, weight, bias, w, b, packs, halo, s
                                     _checked=True)
     if _wants_grad(x, second, weight, bias):
         native = _lib.native()
-        if not _node_queue_set:
-            native.set_weight_queue(_queue_from_node)
-            _node_queue_set = True
+        if not _early_callbacks_set:
+            # (looked up in the module at the time of the call)
+            native.set_early_callbacks(lambda batch: _send_early(batch), lambda: _join_early())
+            _early_callbacks_set = True
         family = _deferrable(weight, in_shape, w.shape, stride, padding, dilation, x_read.dtype) if defer else 0
         native.record_conv(y, x, weight, bias, second, x_read, second_read, w, pd, halo, stride, padding, dilation, master, family,
                            defer == 2)

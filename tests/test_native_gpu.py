@@ -61,3 +61,39 @@ def test_a_tensor_changed_after_the_forward_is_noticed(device):
         h.add_(1)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         y.float().sum().backward()
+
+
+def test_passes_that_overlap_keep_their_weight_gradients_apart(device):
+    """Two threads run backward passes with deferred weight gradients at the same time, each on a stream of its own: every
+    gradient is the one its pass alone would give."""
+    import threading
+
+    def make(seed):
+        torch.manual_seed(seed)
+        net = sa.UNet(1, 3, layers=2, base_width=32).to(device).to(torch.bfloat16).to(memory_format=CL).defer_weight_gradients()
+        x = torch.randn(1, 1, 8, 16, 32, device=device).to(torch.bfloat16).contiguous(memory_format=CL)
+        return net, x, torch.randint(0, 3, (1, 8, 16, 32), device=device)
+
+    def grads(net, x, labels):
+        net.zero_grad(set_to_none=True)
+        sa.ce_dice_loss(net(x), labels).backward()
+        return [p.grad.clone() for p in net.parameters()]
+
+    jobs = [make(1), make(2)]
+    want = [grads(*job) for job in jobs]
+    got = [None, None]
+
+    def run(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(3):
+                got[i] = grads(*jobs[i])
+            torch.cuda.current_stream().synchronize()
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for w, g in zip(want, got):
+        assert all(torch.equal(a, b) for a, b in zip(w, g))
