@@ -10,6 +10,7 @@
 #include <torch/extension.h>
 
 #include <ATen/autocast_mode.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/engine.h>
@@ -83,10 +84,14 @@ bool on_gpu(const Tensor& t) { return t.is_cuda() && t.layout() == at::kStrided;
 const void* ptr(const Tensor& t) { return t.defined() ? t.const_data_ptr() : nullptr; }
 void* out_ptr(const Tensor& t) { return t.defined() ? t.mutable_data_ptr() : nullptr; }
 Tensor dense(const Tensor& t) { return t.is_contiguous(kCL3D) ? t : t.contiguous(kCL3D); }
-Tensor volume(at::IntArrayRef sizes, const Tensor& like, at::ScalarType dtype) {
-  return at::empty(sizes, like.options().dtype(dtype), kCL3D);
+// (the backend's own factory: a pass allocates a few hundred tensors, and the dispatcher is a third of what that costs)
+Tensor plain(at::IntArrayRef sizes, const Tensor& like, at::ScalarType dtype) {
+  return Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), std::nullopt));
 }
-Tensor bytes(size_t n, const Tensor& like) { return n == 0 ? Tensor() : at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
+Tensor volume(at::IntArrayRef sizes, const Tensor& like, at::ScalarType dtype) {
+  return Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), kCL3D));
+}
+Tensor bytes(size_t n, const Tensor& like) { return n == 0 ? Tensor() : plain({(int64_t)n}, like, at::kByte); }
 
 // An int or three ints; false for any other spelling (the Python layer then says what is wrong with it).
 bool three(py::handle h, int32_t v[3]) {
@@ -222,7 +227,7 @@ ConvResult launch_conv(const Problem& prob, const Tensor& x, const Tensor& secon
   int rc = SFH_ERR_UNSUPPORTED;
   r.records = groups > 0 ? prob.records(groups) : 0;
   if (r.records > 0) {
-    r.partials = at::empty({(int64_t)prob.key.d.n * r.records * groups * 4}, x.options().dtype(at::kFloat));
+    r.partials = plain({(int64_t)prob.key.d.n * r.records * groups * 4}, x, at::kFloat);
     rc = second.defined()
              ? sfh_conv3d_fwd_pair(prob.desc(), prob.key.code, ptr(x), ptr(second), (int32_t)x.size(1), wp, strides, ptr(bias), out_ptr(r.y),
                                    out_ptr(ws), ws_bytes, flags, groups, (float*)out_ptr(r.partials), (size_t)r.partials.numel() * 4, st)
@@ -283,7 +288,7 @@ Tensor launch_wgrad(const Problem& prob, const Tensor& x, const Tensor& second, 
 Tensor launch_bias_grad(const Tensor& gy, at::ScalarType dtype) {
   c10::OptionalDeviceGuard guard(gy.device());
   const int64_t c = gy.size(1), rows = gy.numel() / c;
-  Tensor gb = at::empty({c}, gy.options().dtype(dtype));
+  Tensor gb = plain({c}, gy, dtype);
   const Tensor ws = bytes(sfh_bias_grad_workspace_bytes(rows, (int32_t)c), gy);
   check(sfh_bias_grad(code_of(gy.scalar_type()), code_of(dtype), ptr(gy), rows, (int32_t)c, out_ptr(gb), out_ptr(ws),
                       ws.defined() ? (size_t)ws.numel() : 0, stream_of(gy)), "bias_grad");
@@ -475,9 +480,9 @@ void queue_weight(QueuedWeight&& q) {
   }
 }
 
-// The convolution over x, or over the pair (x, second).  Edges: x, weight, bias, second.  In the depth-shard form the
-// tensors that are saved are slabs of which x and second are the depth interiors.
-struct ConvNode : public LaunchNode {
+// What the backward of a convolution over x, or over the pair (x, second), needs.  In the depth-shard form the tensors that
+// are saved are slabs of which x and second are the depth interiors.
+struct ConvSaved {
   SavedVariable x, second, w, packed_dgrad;
   Tensor param;             // the parameter whose weight gradient waits for the end of the pass (undefined: computed here)
   int family = 0;
@@ -487,20 +492,15 @@ struct ConvNode : public LaunchNode {
   int64_t halo = 0, depth = 0, first_channels = 0;
   std::vector<int64_t> in_sizes;
 
-  std::string name() const override { return "ScaffoldConv3dBackward"; }
-  void release_variables() override {
+  void release() {
     x.reset_data(); second.reset_data(); w.reset_data(); packed_dgrad.reset_data();
     param.reset();
   }
-  variable_list backward(variable_list& grads) override {
-    variable_list out(4);
-    if (!grads[0].defined()) return out;
+  // out: the gradients of x, weight, bias and second that are wanted (gy dense)
+  void backward(const Tensor& gy, bool need_x, bool need_w, bool need_b, bool need_2, Tensor out[4]) {
     const Tensor xs = x.unpack(), x2 = second.unpack(), wt = w.unpack(), packed = packed_dgrad.unpack();
-    const Tensor gy = dense(grads[0]);
     Problem prob;
     TORCH_INTERNAL_ASSERT(make_problem(in_sizes, wt.sizes(), s, p, d, code_of(gy.scalar_type()), prob));
-    const bool need_x = task_should_compute_output(0), need_w = task_should_compute_output(1), need_b = has_bias && task_should_compute_output(2),
-               need_2 = pair && task_should_compute_output(3);
     if (need_x || need_2) {
       auto gx = launch_dgrad(prob, gy, wt, packed, pair ? first_channels : 0);
       if (halo > 0) {
@@ -515,7 +515,7 @@ struct ConvNode : public LaunchNode {
       c10::OptionalDeviceGuard guard(gy.device());
       const auto& pd = prob.key.d;
       const auto dtype = master ? at::kFloat : gy.scalar_type();
-      Tensor gw = volume({pd.cout, pd.cin, pd.kd, pd.kh, pd.kw}, gy, dtype), gb = at::empty({pd.cout}, gy.options().dtype(dtype));
+      Tensor gw = volume({pd.cout, pd.cin, pd.kd, pd.kh, pd.kw}, gy, dtype), gb = plain({pd.cout}, gy, dtype);
       const Tensor ws = bytes(prob.sizes->work_bias, gy);
       const int rc = sfh_conv3d_wgrad_bias(prob.desc(), prob.key.code, ptr(xs), ptr(gy), out_ptr(gw), out_ptr(gb), out_ptr(ws), prob.sizes->work_bias,
                                            dtype != gy.scalar_type() ? SFH_FLAG_GRAD_FP32 : 0, stream_of(gy));
@@ -523,7 +523,7 @@ struct ConvNode : public LaunchNode {
         check(rc, "conv3d_backward_weight_bias");
         out[1] = gw;
         out[2] = gb.scalar_type() == bias_dtype ? gb : gb.to(bias_dtype);
-        return out;
+        return;
       }
     }
     if (need_w && param.defined()) {
@@ -532,9 +532,36 @@ struct ConvNode : public LaunchNode {
       out[1] = launch_wgrad(prob, xs, x2, gy, master);
     }
     if (need_b) out[2] = launch_bias_grad(gy, bias_dtype);
+  }
+};
+
+struct ConvNode : public LaunchNode {  // edges: x, weight, bias, second
+  ConvSaved saved;
+  std::string name() const override { return "ScaffoldConv3dBackward"; }
+  void release_variables() override { saved.release(); }
+  variable_list backward(variable_list& grads) override {
+    variable_list out(4);
+    if (grads[0].defined())
+      saved.backward(dense(grads[0]), task_should_compute_output(0), task_should_compute_output(1), saved.has_bias && task_should_compute_output(2),
+                     saved.pair && task_should_compute_output(3), out.data());
     return out;
   }
 };
+
+void save_conv(ConvSaved& c, const Tensor& x, const Tensor& x_read, const Tensor& w, const Tensor& packed_dgrad, int64_t halo, bool master,
+               const Tensor& param, int family, bool early) {
+  c.x = SavedVariable(x_read, false);
+  c.w = SavedVariable(w, false);
+  c.packed_dgrad = SavedVariable(packed_dgrad, false);
+  c.halo = halo;
+  c.depth = x.size(2);
+  c.first_channels = x_read.size(1);
+  c.in_sizes = x_read.sizes().vec();
+  c.master = master;
+  c.param = param;
+  c.family = family;
+  c.early = early;
+}
 
 // Records the node of y = conv(x[, second]) that a launch has just produced.  `x_read` / `second_read`: the tensors the
 // kernels read (slabs in the depth-shard form, halo > 0; else x and second themselves).
@@ -544,25 +571,16 @@ void record_conv(Tensor y, const Tensor& x, const Tensor& weight, const MaybeTen
   const Tensor b = or_none(bias), x2 = or_none(second);
   if (!wants_grad({&x, &weight, &b, &x2})) return;
   auto node = new_node<ConvNode>();
-  TORCH_CHECK_VALUE(three(stride, node->s) && three(padding, node->p) && three(dilation, node->d), "stride, padding and dilation are ints or three ints");
+  ConvSaved& c = node->saved;
+  TORCH_CHECK_VALUE(three(stride, c.s) && three(padding, c.p) && three(dilation, c.d), "stride, padding and dilation are ints or three ints");
   node->set_next_edges(torch::autograd::collect_next_edges(x, weight, b, x2));
   const Tensor read2 = or_none(second_read);
-  node->x = SavedVariable(x_read, false);
-  node->second = SavedVariable(read2, false);
-  node->w = SavedVariable(w, false);
-  node->packed_dgrad = SavedVariable(or_none(packed_dgrad), false);
-  node->pair = x2.defined();
-  node->has_bias = b.defined();
-  if (b.defined()) node->bias_dtype = b.scalar_type();
-  node->master = master;
-  node->halo = halo;
-  node->depth = x.size(2);
-  node->first_channels = x_read.size(1);
-  node->in_sizes = x_read.sizes().vec();
-  if (read2.defined()) node->in_sizes[1] += read2.size(1);
-  if (family > 0) node->param = weight;
-  node->family = family;
-  node->early = early;
+  save_conv(c, x, x_read, w, or_none(packed_dgrad), halo, master, family > 0 ? weight : Tensor(), family, early);
+  c.second = SavedVariable(read2, false);
+  c.pair = x2.defined();
+  if (read2.defined()) c.in_sizes[1] += read2.size(1);
+  c.has_bias = b.defined();
+  if (b.defined()) c.bias_dtype = b.scalar_type();
   torch::autograd::set_history(y, node);
 }
 
@@ -676,7 +694,7 @@ struct ConvTransposeNode : public LaunchNode {  // edges: x, weight, bias
       const size_t need = sfh_convT3d_wgrad_bias_workspace_bytes(&td, prob.key.code);
       if (need > 0) {
         const auto dtype = master ? at::kFloat : gy.scalar_type();
-        Tensor gw = volume(wt.sizes(), gy, dtype), gb = at::empty({wt.size(1)}, gy.options().dtype(dtype));
+        Tensor gw = volume(wt.sizes(), gy, dtype), gb = plain({wt.size(1)}, gy, dtype);
         const Tensor ws = bytes(need, gy);
         const int rc = sfh_convT3d_wgrad_bias(&td, prob.key.code, ptr(xs), ptr(gy), out_ptr(gw), out_ptr(gb), out_ptr(ws), need,
                                               dtype != gy.scalar_type() ? SFH_FLAG_GRAD_FP32 : 0, stream_of(gy));
@@ -762,18 +780,16 @@ py::object conv_transpose(const Tensor& x_in, const Tensor& weight, const MaybeT
 }
 
 // ---- GroupNorm -----------------------------------------------------------------------------------------------------------
-struct GroupNormNode : public LaunchNode {  // edges: input, weight, bias
+// What the backward of GroupNorm (+ ReLU) needs.
+struct NormSaved {
   SavedVariable input, weight, bias, stats;
   int groups = 1;
   bool relu = false;
-  std::string name() const override { return "ScaffoldGroupNormBackward"; }
-  void release_variables() override { input.reset_data(); weight.reset_data(); bias.reset_data(); stats.reset_data(); }
-  variable_list backward(variable_list& grads) override {
-    variable_list out(3);
-    if (!grads[0].defined()) return out;
+  void release() { input.reset_data(); weight.reset_data(); bias.reset_data(); stats.reset_data(); }
+  void backward(const Tensor& grad, Tensor& dx, Tensor& dw, Tensor& db) {
     const Tensor x = dense(input.unpack()), st = stats.unpack();
     Tensor w = weight.unpack(), b = bias.unpack();
-    Tensor gy = dense(grads[0]);
+    Tensor gy = dense(grad);
     if (gy.scalar_type() != x.scalar_type() && gy.scalar_type() != at::kFloat) gy = gy.to(x.scalar_type());
     const Tensor w_in = w, b_in = b;
     if (w.defined()) w = w.contiguous();
@@ -783,17 +799,94 @@ struct GroupNormNode : public LaunchNode {  // edges: input, weight, bias
     const int64_t c = x.size(1), n = x.size(0);
     const sfh_groupnorm_desc d{(int32_t)n, (int32_t)c, groups, relu ? 1 : 0, x.numel() / (n * c), 0.f};
     const int code = code_of(x.scalar_type());
-    Tensor dx = volume(x.sizes(), x, x.scalar_type()), dw, db;
-    if (w.defined()) dw = at::empty({c}, x.options().dtype(at::kFloat));
-    if (b.defined()) db = at::empty({c}, x.options().dtype(at::kFloat));
+    dx = volume(x.sizes(), x, x.scalar_type());
+    if (w.defined()) dw = plain({c}, x, at::kFloat);
+    if (b.defined()) db = plain({c}, x, at::kFloat);
     const Tensor ws = bytes(sfh_groupnorm_bwd_workspace_bytes(&d, code), x);
     const float* mean = (const float*)ptr(st);
     check(sfh_groupnorm_bwd(&d, code, code_of(gy.scalar_type()), code_of(w.defined() ? w.scalar_type() : b.defined() ? b.scalar_type() : x.scalar_type()),
                             ptr(gy), ptr(x), ptr(w), ptr(b), mean, mean + n * groups, out_ptr(dx), (float*)out_ptr(dw), (float*)out_ptr(db), out_ptr(ws),
                             ws.defined() ? (size_t)ws.numel() : 0, stream_of(x)), "group_norm_backward");
-    if (task_should_compute_output(0)) out[0] = dx;
-    if (dw.defined() && task_should_compute_output(1)) out[1] = dw.scalar_type() == w_in.scalar_type() ? dw : dw.to(w_in.scalar_type());
-    if (db.defined() && task_should_compute_output(2)) out[2] = db.scalar_type() == b_in.scalar_type() ? db : db.to(b_in.scalar_type());
+    if (dw.defined() && dw.scalar_type() != w_in.scalar_type()) dw = dw.to(w_in.scalar_type());
+    if (db.defined() && db.scalar_type() != b_in.scalar_type()) db = db.to(b_in.scalar_type());
+  }
+};
+
+struct NormResult {
+  Tensor y, slab, stats;  // stats: mean and rstd
+};
+
+// The gate of the forward (groupnorm.is_supported) for an input of this description.
+bool norm_gate(const Tensor& like, int64_t n, int64_t c, int64_t spatial, int64_t groups, const MaybeTensor& weight, const MaybeTensor& bias) {
+  if (code_of(like.scalar_type()) < 0 || groups < 1 || c % groups != 0 || n * c * spatial == 0) return false;
+  if ((c == groups && n * spatial == 1) || n > INT32_MAX || c > INT32_MAX) return false;
+  for (const MaybeTensor* t : {&weight, &bias}) {
+    if (!t->has_value()) continue;
+    if ((*t)->dim() != 1 || (*t)->numel() != c || (*t)->device() != like.device()) return false;
+    if ((*t)->scalar_type() != like.scalar_type() && ((*t)->scalar_type() != at::kFloat || !at::autocast::is_autocast_enabled(at::kCUDA))) return false;
+  }
+  return true;
+}
+
+NormResult launch_norm(const Tensor& input, int64_t groups, const Tensor& weight, const Tensor& bias, double eps, bool relu, at::ScalarType odt, int64_t halo,
+                       const Tensor& partials, int32_t records) {
+  c10::OptionalDeviceGuard guard(input.device());
+  const int64_t n = input.size(0), c = input.size(1);
+  const int code = code_of(input.scalar_type());
+  NormResult r;
+  Tensor w = weight.defined() ? weight.contiguous() : weight, b = bias.defined() ? bias.contiguous() : bias;
+  if (w.defined() && b.defined() && w.scalar_type() != b.scalar_type()) b = b.to(w.scalar_type());
+  const int pcode = code_of(w.defined() ? w.scalar_type() : b.defined() ? b.scalar_type() : input.scalar_type());
+  r.stats = plain({2, n, groups}, input, at::kFloat);
+  float* mean = (float*)out_ptr(r.stats);
+  float* rstd = mean + n * groups;
+  const sfh_groupnorm_desc d{(int32_t)n, (int32_t)c, (int32_t)groups, relu ? 1 : 0, input.numel() / (n * c), (float)eps};
+  void* st = stream_of(input);
+  int64_t halo_rows = 0;
+  if (halo > 0 && n == 1 && c10::elementSize(odt) == input.element_size()) {
+    r.slab = volume({1, c, input.size(2) + 2 * halo, input.size(3), input.size(4)}, input, odt);
+    r.y = r.slab.narrow(2, halo, input.size(2));
+    halo_rows = halo * input.size(3) * input.size(4);
+  } else {
+    r.y = volume(input.sizes(), input, odt);
+  }
+  int rc = SFH_ERR_UNSUPPORTED;
+  if (partials.defined())
+    rc = sfh_groupnorm_fwd_from_partials(&d, code, code_of(odt), pcode, ptr(input), ptr(w), ptr(b), out_ptr(r.slab.defined() ? r.slab : r.y), halo_rows, mean,
+                                         rstd, (const float*)ptr(partials), (size_t)partials.numel() * 4, records, st);
+  if (rc == SFH_ERR_UNSUPPORTED) {
+    const Tensor ws = bytes(sfh_groupnorm_fwd_workspace_bytes(&d, code), input);
+    const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+    if (r.slab.defined()) {
+      rc = sfh_groupnorm_fwd_slab(&d, code, code_of(odt), pcode, ptr(input), ptr(w), ptr(b), out_ptr(r.slab), halo_rows, mean, rstd, out_ptr(ws), ws_bytes, st);
+      if (rc == SFH_ERR_UNSUPPORTED) {  // channel counts off the vector path: the plain form
+        r.slab = Tensor();
+        r.y = volume(input.sizes(), input, odt);
+      }
+    }
+    if (rc == SFH_ERR_UNSUPPORTED)
+      rc = sfh_groupnorm_fwd(&d, code, code_of(odt), pcode, ptr(input), ptr(w), ptr(b), out_ptr(r.y), mean, rstd, out_ptr(ws), ws_bytes, st);
+  }
+  check(rc, "group_norm");
+  return r;
+}
+
+void save_norm(NormSaved& s, const Tensor& input, const Tensor& weight, const Tensor& bias, const Tensor& stats, int64_t groups, bool relu) {
+  s.input = SavedVariable(input, false);
+  s.weight = SavedVariable(weight, false);
+  s.bias = SavedVariable(bias, false);
+  s.stats = SavedVariable(stats, false);
+  s.groups = (int)groups;
+  s.relu = relu;
+}
+
+struct GroupNormNode : public LaunchNode {  // edges: input, weight, bias
+  NormSaved saved;
+  std::string name() const override { return "ScaffoldGroupNormBackward"; }
+  void release_variables() override { saved.release(); }
+  variable_list backward(variable_list& grads) override {
+    variable_list out(3);
+    if (grads[0].defined()) saved.backward(grads[0], out[0], out[1], out[2]);
     return out;
   }
 };
@@ -803,75 +896,80 @@ struct GroupNormNode : public LaunchNode {  // edges: input, weight, bias
 // producer of `input` left for these very bits, `records` per sample.
 py::object group_norm(const Tensor& input, int64_t groups, const MaybeTensor& weight, const MaybeTensor& bias, double eps, bool relu,
                       std::optional<at::ScalarType> out_dtype, bool stock_dtype, int64_t halo, const MaybeTensor& partials, int32_t records) {
-  if (input.dim() != 5 || !on_gpu(input) || input.numel() == 0) return py::none();
-  const int code = code_of(input.scalar_type());
-  const int64_t n = input.size(0), c = input.size(1);
-  if (code < 0 || groups < 1 || c % groups != 0 || !input.is_contiguous(kCL3D)) return py::none();
-  const int64_t spatial = input.numel() / (n * c);
-  if ((c == groups && input.numel() == c) || n > INT32_MAX || c > INT32_MAX) return py::none();
-  const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
-  for (const MaybeTensor* t : {&weight, &bias}) {
-    if (!t->has_value()) continue;
-    if ((*t)->dim() != 1 || (*t)->numel() != c || (*t)->device() != input.device()) return py::none();
-    if ((*t)->scalar_type() != input.scalar_type() && ((*t)->scalar_type() != at::kFloat || !autocast)) return py::none();
-  }
+  if (input.dim() != 5 || !on_gpu(input) || input.numel() == 0 || !input.is_contiguous(kCL3D)) return py::none();
+  if (!norm_gate(input, input.size(0), input.size(1), input.numel() / (input.size(0) * input.size(1)), groups, weight, bias)) return py::none();
   at::ScalarType odt = out_dtype.value_or(input.scalar_type());
-  if (stock_dtype) odt = input.scalar_type() != at::kFloat && autocast ? at::kFloat : input.scalar_type();
+  if (stock_dtype) odt = input.scalar_type() != at::kFloat && at::autocast::is_autocast_enabled(at::kCUDA) ? at::kFloat : input.scalar_type();
   if (code_of(odt) < 0) return py::none();
-  const Tensor w_in = or_none(weight), b_in = or_none(bias);
-  const bool graph = wants_grad({&input, &w_in, &b_in});
-  Tensor y, slab, stats;
+  const Tensor w = or_none(weight), b = or_none(bias);
+  const bool graph = wants_grad({&input, &w, &b});
+  NormResult r;
   {
     at::AutoGradMode no_grad(false);
-    c10::OptionalDeviceGuard guard(input.device());
-    Tensor w = w_in.defined() ? w_in.contiguous() : w_in, b = b_in.defined() ? b_in.contiguous() : b_in;
-    if (w.defined() && b.defined() && w.scalar_type() != b.scalar_type()) b = b.to(w.scalar_type());
-    const int pcode = code_of(w.defined() ? w.scalar_type() : b.defined() ? b.scalar_type() : input.scalar_type());
-    stats = at::empty({2, n, groups}, input.options().dtype(at::kFloat));  // mean, rstd
-    float* mean = (float*)out_ptr(stats);
-    float* rstd = mean + n * groups;
-    const sfh_groupnorm_desc d{(int32_t)n, (int32_t)c, (int32_t)groups, relu ? 1 : 0, spatial, (float)eps};
-    void* st = stream_of(input);
-    int64_t halo_rows = 0;
-    if (halo > 0 && n == 1 && c10::elementSize(odt) == input.element_size()) {
-      slab = volume({1, c, input.size(2) + 2 * halo, input.size(3), input.size(4)}, input, odt);
-      y = slab.narrow(2, halo, input.size(2));
-      halo_rows = halo * input.size(3) * input.size(4);
-    } else {
-      y = volume(input.sizes(), input, odt);
-    }
-    int rc = SFH_ERR_UNSUPPORTED;
-    if (partials.has_value())
-      rc = sfh_groupnorm_fwd_from_partials(&d, code, code_of(odt), pcode, ptr(input), ptr(w), ptr(b), out_ptr(slab.defined() ? slab : y), halo_rows, mean,
-                                           rstd, (const float*)ptr(*partials), (size_t)partials->numel() * 4, records, st);
-    if (rc == SFH_ERR_UNSUPPORTED) {
-      const Tensor ws = bytes(sfh_groupnorm_fwd_workspace_bytes(&d, code), input);
-      const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
-      if (slab.defined()) {
-        rc = sfh_groupnorm_fwd_slab(&d, code, code_of(odt), pcode, ptr(input), ptr(w), ptr(b), out_ptr(slab), halo_rows, mean, rstd, out_ptr(ws), ws_bytes, st);
-        if (rc == SFH_ERR_UNSUPPORTED) {  // channel counts off the vector path: the plain form
-          slab = Tensor();
-          y = volume(input.sizes(), input, odt);
-        }
-      }
-      if (rc == SFH_ERR_UNSUPPORTED)
-        rc = sfh_groupnorm_fwd(&d, code, code_of(odt), pcode, ptr(input), ptr(w), ptr(b), out_ptr(y), mean, rstd, out_ptr(ws), ws_bytes, st);
-    }
-    check(rc, "group_norm");
+    r = launch_norm(input, groups, w, b, eps, relu, odt, halo, or_none(partials), records);
+    if (graph && r.slab.defined()) r.y = r.y.detach();  // a tensor of its own: a view would keep the slab as its differentiable base
   }
   if (graph) {
     auto node = new_node<GroupNormNode>();
-    node->set_next_edges(torch::autograd::collect_next_edges(input, w_in, b_in));
-    node->input = SavedVariable(input, false);
-    node->weight = SavedVariable(w_in, false);
-    node->bias = SavedVariable(b_in, false);
-    node->stats = SavedVariable(stats, false);
-    node->groups = (int)groups;
-    node->relu = relu;
-    if (slab.defined()) y = y.detach();
-    torch::autograd::set_history(y, node);
+    node->set_next_edges(torch::autograd::collect_next_edges(input, w, b));
+    save_norm(node->saved, input, w, b, r.stats, groups, relu);
+    torch::autograd::set_history(r.y, node);
   }
-  return py::make_tuple(y, tensor_or_none(slab));
+  return py::make_tuple(r.y, tensor_or_none(r.slab));
+}
+
+// ---- a convolution and the GroupNorm that reads it -----------------------------------------------------------------------
+// One call and one node for the pair every block of the U-Net is made of (bias-free convolution): half of the module calls
+// and of the nodes of a pass.
+struct ConvNormNode : public LaunchNode {  // edges: x, convolution weight, norm weight, norm bias
+  ConvSaved conv;
+  NormSaved norm;
+  std::string name() const override { return "ScaffoldConvGroupNormBackward"; }
+  void release_variables() override { conv.release(); norm.release(); }
+  variable_list backward(variable_list& grads) override {
+    variable_list out(4);
+    if (!grads[0].defined()) return out;
+    Tensor gy, c[4];
+    norm.backward(grads[0], gy, out[2], out[3]);
+    conv.backward(gy, task_should_compute_output(0), task_should_compute_output(1), false, false, c);
+    out[0] = c[0];
+    out[1] = c[1];
+    return out;
+  }
+};
+
+// modules.conv_then_norm: (y, slab or None), or None (nothing launched) for a call that is not served as it stands.
+// x / x_read, weight / w, packed forms, halo, master, family and early as in record_conv.
+py::object conv_norm(const Tensor& x, const Tensor& x_read, const Tensor& weight, const Tensor& w, const MaybeTensor& packed_fwd, const MaybeTensor& packed_dgrad,
+                     int64_t halo, py::handle stride, py::handle padding, py::handle dilation, bool master, int family, bool early, int64_t groups,
+                     const Tensor& norm_weight, const Tensor& norm_bias, double eps, bool relu, int64_t out_halo) {
+  int32_t s[3], p[3], d[3];
+  if (!three(stride, s) || !three(padding, p) || !three(dilation, d) || !x_read.is_contiguous(kCL3D)) return py::none();
+  const bool graph = wants_grad({&x, &weight, &norm_weight, &norm_bias});
+  Problem prob;
+  if (!conv_gate(x_read, w, std::nullopt, s, p, d, graph, prob, 0, packed_fwd.has_value())) return py::none();
+  if (packed_fwd.has_value() && !packed_fits(*packed_fwd, prob.sizes->packed[0], x_read)) return py::none();
+  if (packed_dgrad.has_value() && !packed_fits(*packed_dgrad, prob.sizes->packed[1], x_read)) return py::none();
+  if (!norm_gate(x_read, prob.key.d.n, prob.key.d.cout, (int64_t)prob.out[0] * prob.out[1] * prob.out[2], groups, norm_weight, norm_bias)) return py::none();
+  ConvResult c;
+  NormResult r;
+  {
+    at::AutoGradMode no_grad(false);
+    c = launch_conv(prob, x_read, Tensor(), w, Tensor(), or_none(packed_fwd), (int)groups);
+    r = launch_norm(c.y, groups, norm_weight, norm_bias, eps, relu, c.y.scalar_type(), out_halo, c.records > 0 ? c.partials : Tensor(), c.records);
+    if (graph && r.slab.defined()) r.y = r.y.detach();
+  }
+  if (graph) {
+    auto node = new_node<ConvNormNode>();
+    node->set_next_edges(torch::autograd::collect_next_edges(x, weight, norm_weight, norm_bias));
+    std::memcpy(node->conv.s, s, sizeof(s));
+    std::memcpy(node->conv.p, p, sizeof(p));
+    std::memcpy(node->conv.d, d, sizeof(d));
+    save_conv(node->conv, x, x_read, w, or_none(packed_dgrad), halo, master, family > 0 ? weight : Tensor(), family, early);
+    save_norm(node->norm, c.y, norm_weight, norm_bias, r.stats, groups, relu);
+    torch::autograd::set_history(r.y, node);
+  }
+  return py::make_tuple(r.y, tensor_or_none(r.slab));
 }
 
 // ---- MaxPool3d(2) --------------------------------------------------------------------------------------------------------
@@ -917,7 +1015,7 @@ py::object max_pool(const Tensor& x_in, int64_t halo, bool with_skip) {
     const Tensor x = dense(x_in);
     c10::OptionalDeviceGuard guard(x.device());
     const int64_t n = z[0], c = z[1], d2 = z[2] / 2, h2 = z[3] / 2, w2 = z[4] / 2;
-    idx = at::empty({n, d2, h2, w2, c}, x.options().dtype(at::kByte));
+    idx = plain({n, d2, h2, w2, c}, x, at::kByte);
     const sfh_pool_desc d{(int32_t)n, (int32_t)c, (int32_t)z[2], (int32_t)z[3], (int32_t)z[4]};
     const int code = code_of(x.scalar_type());
     int rc = SFH_ERR_UNSUPPORTED;
@@ -986,8 +1084,8 @@ py::object ce_dice_loss(const Tensor& logits, const Tensor& labels, const MaybeT
     x = dense(logits);
     lab = labels.contiguous();
     if (class_weight.has_value()) cw = class_weight->detach().to(at::kFloat).contiguous();
-    loss = at::empty({}, x.options().dtype(at::kFloat));
-    stats = at::empty({n * 3 * c + 2}, x.options().dtype(at::kFloat));
+    loss = plain({}, x, at::kFloat);
+    stats = plain({n * 3 * c + 2}, x, at::kFloat);
     const Tensor ws = bytes(sfh_ce_dice_workspace_bytes(&d), x);
     check(sfh_ce_dice_fwd(&d, code, ptr(x), (const int64_t*)ptr(lab), (const float*)ptr(cw), (float*)out_ptr(loss), (float*)out_ptr(stats), out_ptr(ws),
                           ws.defined() ? (size_t)ws.numel() : 0, stream_of(x)), "ce_dice_loss");
@@ -1031,6 +1129,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("record_conv", &record_conv);
   m.def("conv_transpose", &conv_transpose);
   m.def("group_norm", &group_norm);
+  m.def("conv_norm", &conv_norm);
   m.def("max_pool", &max_pool);
   m.def("ce_dice_loss", &ce_dice_loss);
 }

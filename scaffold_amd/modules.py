@@ -202,6 +202,14 @@ def flush_weight_gradients() -> None:
 _early_callbacks_set = False
 
 
+def _set_early_callbacks() -> None:
+    global _early_callbacks_set
+    if not _early_callbacks_set:
+        # (looked up in the module at the time of the call)
+        _lib.native().set_early_callbacks(lambda batch: _send_early(batch), lambda: _join_early())
+        _early_callbacks_set = True
+
+
 def _narrowed(weight, bias, dt, x_dtype) -> bool:
     """Whether autocast narrows these parameters to the 16-bit dtype of the activations."""
     return dt in (torch.bfloat16, torch.float16) and x_dtype is dt and weight.dtype is torch.float32 and weight.is_cuda \
@@ -242,7 +250,6 @@ def _run_conv(x, second, x_read, second_read, weight, bias, w, b, packs, halo, s
     else the same tensors).  ``weight`` / ``bias`` receive gradients, ``w`` / ``b`` are what the kernels read: when half-precision
     copies of fp32 masters are given (``master``) the gradients are produced in the masters' dtype directly.  The caller has
     passed the gate (for all three directions when the call will be differentiated)."""
-    global _early_callbacks_set
     pf = pd = None
     in_shape = x_read.shape if second is None else torch.Size((x_read.shape[0], x_read.shape[1] + second_read.shape[1], *x_read.shape[2:]))
     if packs is not None:
@@ -259,13 +266,11 @@ def _run_conv(x, second, x_read, second_read, weight, bias, w, b, packs, halo, s
         y = _c3.conv3d_forward_pair(x_read, second_read, w, b, stride, padding, dilation, packed_weight=pf, gn_groups=gn_groups,
                                     _checked=True)
     if _wants_grad(x, second, weight, bias):
-        native = _lib.native()
-        if not _early_callbacks_set:
-            # (looked up in the module at the time of the call)
-            native.set_early_callbacks(lambda batch: _send_early(batch), lambda: _join_early())
-            _early_callbacks_set = True
-        family = _deferrable(weight, in_shape, w.shape, stride, padding, dilation, x_read.dtype) if defer else 0
-        native.record_conv(y, x, weight, bias, second, x_read, second_read, w, pd, halo, stride, padding, dilation, master, family,
+        family = 0
+        if defer:
+            _set_early_callbacks()
+            family = _deferrable(weight, in_shape, w.shape, stride, padding, dilation, x_read.dtype)
+        _lib.native().record_conv(y, x, weight, bias, second, x_read, second_read, w, pd, halo, stride, padding, dilation, master, family,
                            defer == 2)
     return y
 
@@ -425,6 +430,53 @@ class FastConv3d(nn.Conv3d):
         halo = 0 if slab is None else slab[1]
         return _run_conv(inner, None, x, None, weight if master else w, bias if master else b, w, b, packs, halo, stride, padding, dilation,
                          master, self.gn_groups, self.defer_weight_grad if master or w is weight else False)
+
+
+def _unhooked(module) -> bool:
+    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+
+
+def conv_then_norm(conv, norm, x):
+    """``norm(conv(x))`` as one call into the host path and one autograd node, or ``None`` where the two modules have to run
+    by themselves (a bias, hooks on either, a subclass, an input that is not channels-last, ...)."""
+    if type(conv) is not FastConv3d or type(norm) is not FastGroupNorm or conv.groups != 1 or torch.compiler.is_compiling() \
+            or conv.padding_mode != "zeros" or isinstance(conv.padding, str) or not _unhooked(conv) or not _unhooked(norm) \
+            or torch.nn.modules.module._has_any_global_hook() or not isinstance(x, torch.Tensor) or x.dim() != 5:
+        return None
+    weight, gamma, beta = conv.weight, norm.weight, norm.bias
+    if conv.bias is not None or gamma is None or beta is None:
+        return None
+    dt = autocast_dtype(x)
+    x = cast_operand(x, dt)
+    padding, stride, dilation = tuple(conv.padding), tuple(conv.stride), tuple(conv.dilation)
+    x_read, halo = x, 0
+    if conv.shard_halo and padding[0] > 0:
+        slab = getattr(x, "_sfh_slab", None)
+        if slab is None or slab[1] != padding[0] or slab[0].dtype is not x.dtype:
+            return None
+        x_read, halo = slab
+        padding = (0, padding[1], padding[2])
+    if not x_read.is_contiguous(memory_format=_CL3D):
+        return None
+    in_shape = x_read.shape
+    grad = torch.is_grad_enabled()
+    w, _, packs, master, _ = conv._kernel_operands(weight, None, dt, x.dtype, in_shape, stride, padding, dilation, grad and x.requires_grad)
+    if packs is None and torch.cuda.is_current_stream_capturing():
+        return None  # the module packs for both directions at once under capture
+    receives = weight if master else w
+    family, defer = 0, conv.defer_weight_grad
+    if defer and grad and receives is weight:
+        family = _deferrable(weight, in_shape, weight.shape, stride, padding, dilation, x_read.dtype)
+        _set_early_callbacks()
+    pf, pd = (None, None) if packs is None else packs
+    done = _lib.native().conv_norm(x, x_read, receives, w, pf, pd, halo, stride, padding, dilation, master, family, defer == 2, norm.num_groups,
+                                   gamma, beta, norm.eps, norm.activation == "relu", norm.out_halo)
+    if done is None:
+        return None
+    y, slab = done
+    if slab is not None:
+        y._sfh_slab = (slab, norm.out_halo)
+    return y
 
 
 class FastConvTranspose3d(nn.ConvTranspose3d):

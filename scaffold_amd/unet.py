@@ -21,7 +21,7 @@ import torch.nn.functional as F
 import torch.utils.checkpoint
 
 from . import concat as _cat
-from .modules import FastConv3d, FastConvTranspose3d, FastGroupNorm, autocast_dtype
+from .modules import FastConv3d, FastConvTranspose3d, FastGroupNorm, autocast_dtype, conv_then_norm
 from .pooling import FastMaxPool3d
 
 __all__ = ["UNet", "DoubleConv", "Down", "Up", "OutConv", "skip_concat"]
@@ -108,7 +108,8 @@ class DoubleConv(nn.Module):
             return self.double_conv(x if second is None else torch.cat([x, second], dim=1))
         for c, g in self._pairs:  # the Identity modules between the pairs only keep the reference's state-dict indices
             conv, norm = self.double_conv[c], self.double_conv[g]
-            x = norm(conv(x) if second is None else conv(x, second))
+            y = conv_then_norm(conv, norm, x) if second is None else None
+            x = y if y is not None else norm(conv(x) if second is None else conv(x, second))
             second = None
         return x
 

@@ -97,3 +97,37 @@ def test_passes_that_overlap_keep_their_weight_gradients_apart(device):
         t.join()
     for w, g in zip(want, got):
         assert all(torch.equal(a, b) for a, b in zip(w, g))
+
+
+def test_convolution_and_norm_in_one_call_are_the_two_modules(device):
+    """``conv_then_norm`` gives the bits of ``norm(conv(x))`` in the forward and in every gradient, plain and into a slab, and
+    leaves hooked or biased modules alone."""
+    from scaffold_amd.modules import conv_then_norm
+
+    def pair(bias=False):
+        torch.manual_seed(3)
+        conv = sa.FastConv3d(32, 64, 3, padding=1, bias=bias).to(device).to(memory_format=CL)
+        norm = sa.FastGroupNorm(8, 64, activation="relu").to(device)
+        conv.gn_groups = 8
+        return conv, norm
+
+    for halo in (0, 1):
+        conv, norm = pair()
+        norm.out_halo = halo
+        x = _x(device).detach()
+        runs = []
+        for fused in (True, False):
+            xi = x.clone().requires_grad_()
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                y = conv_then_norm(conv, norm, xi) if fused else norm(conv(xi))
+            assert hasattr(y, "_sfh_slab") == bool(halo)
+            grads = torch.autograd.grad(y, (xi, conv.weight, norm.weight, norm.bias), torch.ones_like(y) / 8)
+            runs.append((y, *grads))
+        assert all(torch.equal(a, b) for a, b in zip(*runs))
+    conv, norm = pair()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        handle = conv.register_forward_hook(lambda *a: None)
+        assert conv_then_norm(conv, norm, x) is None
+        handle.remove()
+        assert conv_then_norm(conv, norm, x) is not None
+        assert conv_then_norm(pair(bias=True)[0], norm, x) is None
