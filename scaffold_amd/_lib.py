@@ -249,6 +249,50 @@ def native():
     return _native
 
 
+def under_transform() -> bool:
+    """Whether a tracer records this thread, a forward-mode level is open or a functorch transform is active: the nodes of
+    the host path are not seen by these, so a differentiable op then goes through :func:`one_node`."""
+    return torch._C._get_tracing_state() is not None or torch.autograd.forward_ad._current_level >= 0 \
+        or torch._C._are_functorch_transforms_active()
+
+
+class _OneNode(torch.autograd.Function):
+    """``fn(*tensors)`` as one ``autograd.Function``, which a tracer records and replays and which refuses forward-mode and
+    functorch transforms: the host path's own nodes run inside it."""
+
+    @staticmethod
+    def forward(ctx, fn, *tensors):
+        tracing = torch._C._get_tracing_state()
+        torch._C._set_tracing_state(None)  # the node is what is recorded, not its parts
+        try:
+            with torch.enable_grad():
+                ctx.leaves = [None if t is None else t.detach().requires_grad_(need) for t, need in zip(tensors, ctx.needs_input_grad[1:])]
+                ctx.results = fn(*ctx.leaves)
+            result = ctx.results.detach()
+        finally:
+            torch._C._set_tracing_state(tracing)
+        ctx.save_for_backward(*tensors)
+        if tracing is None:
+            return result
+        out = torch.empty_strided(result.shape, result.stride(), dtype=result.dtype, device=result.device)  # a tensor the tracer has seen made
+        out.set_(result)
+        return out
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad):
+        ctx.saved_tensors  # raises where the pass before has freed the graph
+        wanted = [t for t, need in zip(ctx.leaves, ctx.needs_input_grad[1:]) if need]
+        with torch.enable_grad():
+            grads = iter(torch.autograd.grad(ctx.results, wanted, grad, retain_graph=True, allow_unused=True))
+        return (None, *(next(grads) if need else None for need in ctx.needs_input_grad[1:]))
+
+
+def one_node(fn, *tensors):
+    """``fn(*tensors)`` (tensors or ``None`` in, one tensor out) as a single node that tracers and transforms see."""
+    return _OneNode.apply(fn, *tensors)
+
+
 def dtype_code(dtype: torch.dtype) -> int:
     try:
         return _DTYPE_CODE[dtype]

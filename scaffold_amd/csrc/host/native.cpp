@@ -41,7 +41,7 @@ using MaybeTensor = std::optional<Tensor>;
 PyObject* g_kernel_error = nullptr;    // scaffold_amd._lib.ScaffoldKernelError
 PyObject* g_note_device = nullptr;     // scaffold_amd._lib._note_device(device)
 PyObject* g_send_early = nullptr;      // scaffold_amd.modules._send_early_batch(batch)
-PyObject* g_join_early = nullptr;      // scaffold_amd.modules._join_early()
+PyObject* g_join_early = nullptr;      // scaffold_amd.modules._join_early(batch)
 
 // A status code as the exception the entry points raise (the interpreter lock is taken if this thread does not hold it).
 void check(int rc, const char* what) {
@@ -420,7 +420,7 @@ void finish_pass(int id) {
   at::AutoGradMode no_grad(false);
   if (!pass.sent.empty()) {
     py::gil_scoped_acquire gil;
-    py::reinterpret_borrow<py::function>(g_join_early)();
+    for (auto& batch : pass.sent) py::reinterpret_borrow<py::function>(g_join_early)(batch);
   }
   for (auto& batch : pass.sent) add_to_grads(*batch);
   while (!pass.items.empty()) {
@@ -469,14 +469,17 @@ void queue_weight(QueuedWeight&& q) {
         std::vector<QueuedWeight> rest;
         for (auto& o : items) (goes(o) ? leave->items : rest).push_back(std::move(o));
         items = std::move(rest);
-        found->second.sent.push_back(leave);
       }
     }
     items.push_back(std::move(q));
   }
   if (leave) {
-    py::gil_scoped_acquire gil;
-    py::reinterpret_borrow<py::function>(g_send_early)(leave);
+    {
+      py::gil_scoped_acquire gil;
+      py::reinterpret_borrow<py::function>(g_send_early)(leave);
+    }
+    std::lock_guard<std::mutex> hold(g_pass_lock);
+    g_passes[id].sent.push_back(leave);
   }
 }
 

@@ -333,6 +333,10 @@ def group_norm(input, num_groups: int, weight=None, bias=None, eps: float = 1e-5
             f"out_dtype must be MATCH_STOCK_DTYPE, None (the input's dtype) or one of {SUPPORTED_DTYPES}, got {out_dtype!r}"
         )
     compiling = torch.compiler.is_compiling()
+    if not compiling and _lib.under_transform() and is_supported(input, num_groups, weight, bias, activation) and input.numel() > 0:
+        odt = _resolve_out_dtype(input, out_dtype)
+        return _lib.one_node(lambda *ts: _lib.native().group_norm(ts[0], num_groups, ts[1], ts[2], float(eps), activation == "relu", odt, False,
+                                                                  0, None, 0)[0], input, weight, bias)
     if not compiling and isinstance(input, torch.Tensor) and type(num_groups) is int and _tensor_or_none(weight) and _tensor_or_none(bias):
         given = getattr(input, "_sfh_gn_partials", None)
         if given is not None and (given[2] != num_groups or given[3] != input._version or given[0].device != input.device):

@@ -49,6 +49,9 @@ def ce_dice_loss(logits: torch.Tensor, labels: torch.Tensor, class_weight: Optio
     place); ``labels``: ``(N, D, H, W)`` int64 class ids, ids outside ``[0, C)`` contribute nothing."""
     loss = None
     if isinstance(logits, torch.Tensor) and isinstance(labels, torch.Tensor) and (class_weight is None or isinstance(class_weight, torch.Tensor)):
+        if _lib.under_transform() and is_supported_loss(logits, labels, class_weight):
+            return _lib.one_node(lambda *ts: _lib.native().ce_dice_loss(*ts, float(eps)), logits, labels,
+                                 None if class_weight is None else class_weight.detach())
         loss = _lib.native().ce_dice_loss(logits, labels, class_weight, float(eps))
     if loss is None:
         raise NotImplementedError(

@@ -154,7 +154,7 @@ def _deferrable(param, in_shape, wshape, stride, padding, dilation, dtype) -> in
 
 
 _EARLY_STREAMS: dict = {}
-_EARLY_DONE: list = []
+_EARLY_DONE: list = []  # batches sent and not joined yet
 
 
 def _send_early(batch) -> None:
@@ -168,13 +168,14 @@ def _send_early(batch) -> None:
     side.wait_stream(torch.cuda.current_stream(dev))
     with torch.no_grad(), torch.cuda.stream(side):
         _lib.native().launch_batch(batch, True)
-    _EARLY_DONE.append((dev, side))
+    _EARLY_DONE.append(batch)
 
 
-def _join_early() -> None:
-    while _EARLY_DONE:
-        dev, side = _EARLY_DONE.pop(0)
-        torch.cuda.current_stream(dev).wait_stream(side)
+def _join_early(batch) -> None:
+    # (each pass joins its own batches: another thread's pass may run at the same time, on a stream of its own)
+    dev = _lib.native().batch_device(batch)
+    _EARLY_DONE.remove(batch)
+    torch.cuda.current_stream(dev).wait_stream(_EARLY_STREAMS[dev])
 
 
 def flush_weight_gradients() -> None:
@@ -206,31 +207,14 @@ def _set_early_callbacks() -> None:
     global _early_callbacks_set
     if not _early_callbacks_set:
         # (looked up in the module at the time of the call)
-        _lib.native().set_early_callbacks(lambda batch: _send_early(batch), lambda: _join_early())
+        _lib.native().set_early_callbacks(lambda batch: _send_early(batch), lambda batch: _join_early(batch))
         _early_callbacks_set = True
 
 
 def _narrowed(weight, bias, dt, x_dtype) -> bool:
     """Whether autocast narrows these parameters to the 16-bit dtype of the activations."""
     return dt in (torch.bfloat16, torch.float16) and x_dtype is dt and weight.dtype is torch.float32 and weight.is_cuda \
-        and (bias is None or bias.dtype is torch.float32 or bias.dtype is dt)
-
-
-def _master_operands(weight, bias, dt, in_shape, stride, padding, dilation, want_dgrad):
-    """What the kernels read of fp32 parameters under 16-bit autocast when nobody keeps half-precision copies:
-    ``(w, b, (packed_fwd, packed_dgrad), complete)``.  The packed forms come from the master in one launch, rounded on the
-    way; only a direction that reads the weight where it lies (the stem, the 1x1x1 head) needs a cast of it.  The parameters'
-    gradients are then produced in fp32 directly: no cast nodes either way."""
-    pf, pd, complete = _lib.native().pack_master(weight, dt, in_shape, stride, padding, dilation, want_dgrad)
-    w = weight if complete else weight.detach().to(dt)
-    b = None if bias is None else (bias if bias.dtype is dt else bias.detach().to(dt))
-    return w, b, (pf, pd), complete
-
-
-def _narrowed(weight, bias, dt, x_dtype) -> bool:
-    """Whether autocast narrows these parameters to the 16-bit dtype of the activations."""
-    return dt in (torch.bfloat16, torch.float16) and x_dtype is dt and weight.dtype is torch.float32 and weight.is_cuda \
-        and (bias is None or bias.dtype is torch.float32 or bias.dtype is dt)
+        and not _lib.under_transform() and (bias is None or bias.dtype is torch.float32 or bias.dtype is dt)
 
 
 def _master_operands(weight, bias, dt, in_shape, stride, padding, dilation, want_dgrad):
@@ -250,6 +234,17 @@ def _run_conv(x, second, x_read, second_read, weight, bias, w, b, packs, halo, s
     else the same tensors).  ``weight`` / ``bias`` receive gradients, ``w`` / ``b`` are what the kernels read: when half-precision
     copies of fp32 masters are given (``master``) the gradients are produced in the masters' dtype directly.  The caller has
     passed the gate (for all three directions when the call will be differentiated)."""
+    if _lib.under_transform():
+        # (the packed forms and half-precision copies belong to the parameters, not to what a replay is given)
+        return _lib.one_node(
+            lambda x_, w_, b_, x2_, r_, r2_: _run_conv_here(x_, x2_, x_ if x_read is x else r_, x2_ if second_read is second else r2_, w_, b_,
+                                                            w_ if w is weight else w, b_ if b is bias else b, None, halo, stride, padding,
+                                                            dilation, master, 0, False),
+            x, weight, bias, second, None if x_read is x else x_read.detach(), None if second_read is second else second_read.detach())
+    return _run_conv_here(x, second, x_read, second_read, weight, bias, w, b, packs, halo, stride, padding, dilation, master, gn_groups, defer)
+
+
+def _run_conv_here(x, second, x_read, second_read, weight, bias, w, b, packs, halo, stride, padding, dilation, master, gn_groups, defer):
     pf = pd = None
     in_shape = x_read.shape if second is None else torch.Size((x_read.shape[0], x_read.shape[1] + second_read.shape[1], *x_read.shape[2:]))
     if packs is not None:
@@ -441,7 +436,7 @@ def conv_then_norm(conv, norm, x):
     by themselves (a bias, hooks on either, a subclass, an input that is not channels-last, ...)."""
     if type(conv) is not FastConv3d or type(norm) is not FastGroupNorm or conv.groups != 1 or torch.compiler.is_compiling() \
             or conv.padding_mode != "zeros" or isinstance(conv.padding, str) or not _unhooked(conv) or not _unhooked(norm) \
-            or torch.nn.modules.module._has_any_global_hook() or not isinstance(x, torch.Tensor) or x.dim() != 5:
+            or torch.nn.modules.module._has_any_global_hook() or _lib.under_transform() or not isinstance(x, torch.Tensor) or x.dim() != 5:
         return None
     weight, gamma, beta = conv.weight, norm.weight, norm.bias
     if conv.bias is not None or gamma is None or beta is None:
@@ -485,6 +480,15 @@ class FastConvTranspose3d(nn.ConvTranspose3d):
     #: depth planes of zero halo to leave around the output for a following ``FastConv3d.shard_halo`` (0: none)
     out_halo = 0
 
+    def _served(self, done, x, w):
+        if done is None:
+            raise NotImplementedError(
+                f"FastConvTranspose3d: not served: x={tuple(x.shape)}/{x.dtype} on {x.device}, weight={tuple(w.shape)}, "
+                f"stride={self.stride} padding={self.padding} output_padding={self.output_padding} "
+                f"dilation={self.dilation} groups={self.groups}"
+            )
+        return done
+
     def forward(self, x: torch.Tensor, output_size=None) -> torch.Tensor:
         if output_size is not None:
             raise NotImplementedError("FastConvTranspose3d: output_size is not supported")
@@ -511,15 +515,13 @@ class FastConvTranspose3d(nn.ConvTranspose3d):
                     pf, pd = packs.fwd, packs.dgrad
             if pf is None or pd is None:
                 pf = pd = None
-            done = _lib.native().conv_transpose(x, weight if master else w, bias if master else b, w, b, stride, pf, pd,
-                                                self.out_halo, master)
-        if done is None:
-            raise NotImplementedError(
-                f"FastConvTranspose3d: not served: x={tuple(x.shape)}/{x.dtype} on {x.device}, weight={tuple(w.shape)}, "
-                f"stride={self.stride} padding={self.padding} output_padding={self.output_padding} "
-                f"dilation={self.dilation} groups={self.groups}"
-            )
-        y, slab = done
+            takes_w, takes_b = weight if master else w, bias if master else b
+            if _lib.under_transform():
+                return _lib.one_node(
+                    lambda x_, w_, b_: self._served(_lib.native().conv_transpose(x_, w_, b_, w_ if takes_w is w else w, b_ if takes_b is b else b,
+                                                                                 stride, None, None, 0, master), x, w)[0], x, takes_w, takes_b)
+            done = _lib.native().conv_transpose(x, takes_w, takes_b, w, b, stride, pf, pd, self.out_halo, master)
+        y, slab = self._served(done, x, w)
         if slab is not None:
             y._sfh_slab = (slab, self.out_halo)
         return y

@@ -46,8 +46,8 @@ def max_pool3d_2x_with_skip(x: torch.Tensor, out_halo: int = 0):
     combined in one kernel (same values as autograd's own addition: one fp32 sum, one rounding)."""
     if not is_supported_pool(x):
         _refuse(x)
-    if not x.is_contiguous(memory_format=_CL3D):
-        return _pool(x, out_halo, False)[0], x
+    if not x.is_contiguous(memory_format=_CL3D) or _lib.under_transform():
+        return max_pool3d_2x(x, out_halo), x
     pooled, _, skip = _pool(x, out_halo, True)
     slab = getattr(x, "_sfh_slab", None)
     if slab is not None:  # the alias is the same memory: still the interior of the slab its producer wrote it into
@@ -58,6 +58,8 @@ def max_pool3d_2x_with_skip(x: torch.Tensor, out_halo: int = 0):
 def max_pool3d_2x(x: torch.Tensor, out_halo: int = 0) -> torch.Tensor:
     """``F.max_pool3d(x, 2)`` for a 5-D GPU tensor; the result is channels-last.  ``out_halo=h`` (one sample): the result is
     the interior view of a slab with ``h`` zero depth planes on each face (``result._sfh_slab``), for ``FastConv3d.shard_halo``."""
+    if _lib.under_transform() and is_supported_pool(x):
+        return _lib.one_node(lambda t: _pool(t, 0, False)[0], x)
     return _pool(x, out_halo, False)[0]
 
 
