@@ -966,6 +966,204 @@ __global__ void __launch_bounds__(kBlock) gn_dx(const T* __restrict__ x, const T
   }
 }
 
+// ---- small groups: a whole (sample, group) in one workgroup's registers ---------------------------------------------------
+// A group of at most kSmallPieces 16-byte pieces (64 KiB) is read once and kept packed in the registers of one workgroup:
+// statistics and result (forward), or per-channel sums and result (backward), are one launch instead of two.  What bounds
+// it is the launch and one trip to memory; a launch costs 4.5 to 6 us on these sizes whatever it computes, and its issue
+// 4 us of host time.  G workgroups leave most of the chip idle, which is why the size is limited (small_groups()).
+// The statistics are those of two passes over registers (mean, then sums about it), summed in a fixed order.
+constexpr int kSmallThreads = 1024, kSmallPerThread = 4, kSmallPieces = kSmallThreads * kSmallPerThread;
+constexpr int kSmallRow = 16;  // pieces of one voxel's group at most (a power of two: a thread's channels are the same in all its pieces)
+
+// Sums over the workgroup in a fixed order, the same in every thread.
+__device__ __forceinline__ void small_sum2(float& a, float& b, float (*red)[2]) {
+  a = wave_sum(a);
+  b = wave_sum(b);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6][0] = a; red[threadIdx.x >> 6][1] = b; }
+  __syncthreads();
+  a = b = 0.f;
+  for (int w = 0; w < (int)blockDim.x >> 6; ++w) { a += red[w][0]; b += red[w][1]; }
+}
+
+template <typename T, typename TO, int NP>
+__global__ void __launch_bounds__(kSmallThreads) gn_small_fwd(const T* __restrict__ x, TO* __restrict__ y, float* __restrict__ mean,
+                                                              float* __restrict__ rstd, const void* __restrict__ gamma,
+                                                              const void* __restrict__ beta, int param_dtype, int S, int C, int G,
+                                                              int row_log2, float m, float eps, int relu, int64_t y_halo) {
+  constexpr int V = VecOf<T>::N;
+  __shared__ float red[kSmallThreads / 64][2];
+  const int tid = threadIdx.x, g = blockIdx.x, n = blockIdx.y;
+  const int c0 = (g << row_log2) * V + (tid & ((1 << row_log2) - 1)) * V;
+  const T* xs = x + (int64_t)n * S * C + c0;
+  Piece<T, V> cur[NP];
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    const int row = (tid + u * (int)blockDim.x) >> row_log2;
+    cur[u].load(xs + (int64_t)(row < S ? row : 0) * C);
+  }
+  float ga[V], be[V];
+  load_params<V>(gamma, param_dtype, c0, 1.f, ga);
+  load_params<V>(beta, param_dtype, c0, 0.f, be);
+  float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    float f[V];
+    cur[u].unpack(f);
+    if ((tid + u * (int)blockDim.x) >> row_log2 < S) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) s1 += f[e];
+    }
+  }
+  small_sum2(s1, s2, red);
+  const float about = s1 / m;
+  s1 = s2 = 0.f;
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    float f[V];
+    cur[u].unpack(f);
+    if ((tid + u * (int)blockDim.x) >> row_log2 < S) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const float d = f[e] - about;
+        s1 += d;
+        s2 = fmaf(d, d, s2);
+      }
+    }
+  }
+  small_sum2(s1, s2, red);
+  const float d = s1 / m;
+  float var = fmaf(-d, d, s2 / m);
+  var = var < 0.f ? 0.f : var;
+  const float mu = about + d, rs = 1.f / sqrtf(var + eps);
+  if (tid == 0) {  // for the backward pass
+    mean[n * G + g] = mu;
+    rstd[n * G + g] = rs;
+  }
+  const int64_t y_sample = (int64_t)n * (S + 2 * y_halo) * C;
+  if (y_halo > 0) {  // the sample's workgroups zero the slab's two faces between them
+    const int64_t face_pieces = y_halo * C * (int64_t)sizeof(TO) / 16;
+    uint4* lo = reinterpret_cast<uint4*>(y + y_sample);
+    uint4* hi = reinterpret_cast<uint4*>(y + y_sample + (y_halo + S) * C);
+    for (int64_t u = (int64_t)g * blockDim.x + tid; u < face_pieces; u += (int64_t)G * blockDim.x) {
+      lo[u] = make_uint4(0, 0, 0, 0);
+      hi[u] = make_uint4(0, 0, 0, 0);
+    }
+  }
+  TO* ys = y + y_sample + y_halo * C + c0;
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    const int row = (tid + u * (int)blockDim.x) >> row_log2;
+    if (row < S) {
+      float f[V], o[V];
+      cur[u].unpack(f);
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const float v = fmaf((f[e] - mu) * rs, ga[e], be[e]);
+        o[e] = relu ? relu_keep_nan(v) : v;
+      }
+      St<TO, V>::run(ys + (int64_t)row * C, o);
+    }
+  }
+}
+
+// One sample: the group's channels get their parameter gradients from the same workgroup.
+template <typename T, typename TG, int NP>
+__global__ void __launch_bounds__(kSmallThreads) gn_small_bwd(const T* __restrict__ x, const TG* __restrict__ dy, T* __restrict__ dx,
+                                                              const float* __restrict__ mean, const float* __restrict__ rstd,
+                                                              const void* __restrict__ gamma, const void* __restrict__ beta, int param_dtype,
+                                                              float* __restrict__ dgamma, float* __restrict__ dbeta, int S, int C, int row_log2,
+                                                              float m, int relu) {
+  constexpr int V = VecOf<T>::N;
+  __shared__ float part[kSmallThreads / 64][kSmallRow * V][2];
+  __shared__ float tot[kSmallRow * V][2];  // sum dy' xhat, sum dy'
+  __shared__ float gam[kSmallRow * V];
+  const int tid = threadIdx.x, g = blockIdx.x, lane = tid & 63, waves = (int)blockDim.x >> 6;
+  const int row_pieces = 1 << row_log2, cg = row_pieces * V, own = (tid & (row_pieces - 1)) * V, c0 = g * cg + own;
+  Piece<T, V> cx[NP];
+  Piece<TG, V> cd[NP];
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    const int row = (tid + u * (int)blockDim.x) >> row_log2;
+    const int64_t at = (int64_t)(row < S ? row : 0) * C + c0;
+    cx[u].load(x + at);
+    cd[u].load(dy + at);
+  }
+  const float mu = mean[g], rs = rstd[g];
+  float ga[V], be[V];
+  load_params<V>(gamma, param_dtype, c0, 1.f, ga);
+  load_params<V>(beta, param_dtype, c0, 0.f, be);
+  float a1[V], a2[V];
+#pragma unroll
+  for (int e = 0; e < V; ++e) a1[e] = a2[e] = 0.f;
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    float f[V], d[V];
+    cx[u].unpack(f);
+    cd[u].unpack(d);
+    if ((tid + u * (int)blockDim.x) >> row_log2 < S) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const float xh = (f[e] - mu) * rs;
+        if (relu) d[e] = fmaf(xh, ga[e], be[e]) <= 0.f ? 0.f : d[e];
+        a1[e] = fmaf(d[e], xh, a1[e]);
+        a2[e] += d[e];
+      }
+    }
+  }
+  // lanes that hold the same channels meet in a butterfly, the wavefronts in order through LDS
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+    for (int off = 32; off >= row_pieces; off >>= 1) {
+      a1[e] += __shfl_xor(a1[e], off, 64);
+      a2[e] += __shfl_xor(a2[e], off, 64);
+    }
+  }
+  if (tid < row_pieces) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) gam[own + e] = ga[e];
+  }
+  if (lane < row_pieces) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      part[tid >> 6][own + e][0] = a1[e];
+      part[tid >> 6][own + e][1] = a2[e];
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < 2 * cg; i += (int)blockDim.x) {
+    float t = 0.f;
+    for (int w = 0; w < waves; ++w) t += part[w][i >> 1][i & 1];
+    tot[i >> 1][i & 1] = t;
+    float* dst = (i & 1) ? dbeta : dgamma;
+    if (dst != nullptr) dst[g * cg + (i >> 1)] = t;
+  }
+  __syncthreads();
+  float ca = 0.f, cb = 0.f;  // every wavefront folds the group by itself, all in the same order
+  for (int c = lane; c < cg; c += 64) {
+    cb = fmaf(gam[c], tot[c][0], cb);
+    ca = fmaf(gam[c], tot[c][1], ca);
+  }
+  ca = __shfl(wave_sum(ca), 0, 64) / m;
+  cb = __shfl(wave_sum(cb), 0, 64) / m;
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    const int row = (tid + u * (int)blockDim.x) >> row_log2;
+    if (row < S) {
+      float f[V], d[V], o[V];
+      cx[u].unpack(f);
+      cd[u].unpack(d);
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const float xh = (f[e] - mu) * rs;
+        if (relu) d[e] = fmaf(xh, ga[e], be[e]) <= 0.f ? 0.f : d[e];
+        o[e] = rs * ((d[e] * ga[e] - ca) - xh * cb);
+      }
+      St<T, V>::run(dx + (int64_t)row * C + c0, o);
+    }
+  }
+}
+
 // ---- scalar path: one workgroup per (group, sample) ---------------------------------------
 __device__ __forceinline__ float block_sum(float v, float* red) {
   __syncthreads();
@@ -1120,6 +1318,31 @@ size_t bwd_ws_floats(const sfh_groupnorm_desc& p, const GnPlan& pl) {
          (size_t)p.n * pl.nsplit * 2 * p.groups;
 }
 
+// The launch of the small-group kernels: threads (0: not taken), pieces per thread, log2 of a row's pieces.
+struct SmallGroups {
+  int threads = 0, per_thread = 0, row_log2 = 0;
+};
+
+// Taken by groups whose voxel row is 1, 2, 4, 8 or 16 pieces, up to the size at which one workgroup per group loses to two
+// launches over the whole chip; narrow rows get there earlier, since every workgroup then fetches cache lines of which it
+// uses a part.  Measured in captured chains (us, two launches / one; 8 groups): forward 512 channels x 256 voxels (2048 pieces)
+// 9.3 / 5.3, 256 x 1024 (4096) 9.2 / 6.3, 128 x 2048 (4096) 8.8 / 6.8, but rows of one piece 64 x 4096 (4096) 8.7 / 8.6.
+// Backward with two casts of the parameter gradients, 512 x 256 13.3 / 10.1, 128 x 512 (1024) 12.8 / 10.9, 64 x 2048 (2048)
+// 13.3 / 12.9, 512 x 512 (4096) 14.2 / 13.0, but 128 x 2048 (4096) 12.7 / 15.5; two samples one after the other 13.0 / 14.8.
+SmallGroups small_groups(const sfh_groupnorm_desc& p, const GnPlan& pl, bool backward) {
+  SmallGroups r;
+  const int cg = p.c / p.groups;
+  if (!pl.vector || cg % pl.vec != 0 || (backward && p.n > 1)) return r;
+  const int row = cg / pl.vec;
+  const int limit = row >= (backward ? 8 : 2) ? kSmallPieces : kSmallPieces / 2;
+  if (p.spatial > limit || row > kSmallRow || (row & (row - 1)) != 0 || p.spatial * row > limit) return r;
+  const int pieces = (int)p.spatial * row;
+  while ((1 << r.row_log2) < row) ++r.row_log2;
+  r.per_thread = pieces <= kSmallThreads ? 1 : pieces <= 2 * kSmallThreads ? 2 : 4;
+  r.threads = (int)align_up((size_t)cdiv(pieces, r.per_thread), 64);
+  return r;
+}
+
 template <typename T, typename TO>
 int fwd_typed(const sfh_groupnorm_desc& p, const GnPlan& pl, int param_dtype, const void* x, const void* gamma, const void* beta,
               void* y, int64_t y_halo, float* mean, float* rstd, float* ws, hipStream_t st, const float* given_records = nullptr,
@@ -1137,6 +1360,19 @@ int fwd_typed(const sfh_groupnorm_desc& p, const GnPlan& pl, int param_dtype, co
     hipLaunchKernelGGL((gn_scalar_normalize<T, TO>), dim3((unsigned)cdiv(total, kBlock)), dim3(kBlock), 0, st, (const T*)x,
                        (TO*)y, mean, rstd, gamma, beta, param_dtype, S, C, G, total, p.relu);
     return check_launch("gn_scalar_normalize");
+  }
+  if (given_records == nullptr) {
+    const SmallGroups sg = small_groups(p, pl, false);
+    if (sg.threads > 0) {
+#define SFH_GN_SMALL(NP)                                                                                                            \
+  hipLaunchKernelGGL((gn_small_fwd<T, TO, NP>), dim3(G, p.n), dim3(sg.threads), 0, st, (const T*)x, (TO*)y, mean, rstd, gamma, beta, \
+                     param_dtype, (int)S, C, G, sg.row_log2, (float)S * (float)(C / G), p.eps, p.relu, y_halo)
+      if (sg.per_thread == 1) SFH_GN_SMALL(1);
+      else if (sg.per_thread == 2) SFH_GN_SMALL(2);
+      else SFH_GN_SMALL(4);
+#undef SFH_GN_SMALL
+      return check_launch("gn_small_fwd");
+    }
   }
   const dim3 grid(pl.nsplit, p.n);
   const float* shift = nullptr;
@@ -1198,6 +1434,17 @@ int bwd_typed(const sfh_groupnorm_desc& p, const GnPlan& pl, int param_dtype, co
     hipLaunchKernelGGL((gn_scalar_dx<T, TG>), dim3((unsigned)cdiv(total, kBlock)), dim3(kBlock), 0, st, (const T*)x,
                        (const TG*)dy, (T*)dx, mean, rstd, gamma, beta, param_dtype, coef, S, C, G, total, p.relu);
     return check_launch("gn_scalar_dx");
+  }
+  const SmallGroups sg = small_groups(p, pl, true);
+  if (sg.threads > 0) {
+#define SFH_GN_SMALL(NP)                                                                                                          \
+  hipLaunchKernelGGL((gn_small_bwd<T, TG, NP>), dim3(G), dim3(sg.threads), 0, st, (const T*)x, (const TG*)dy, (T*)dx, mean, rstd, \
+                     gamma, beta, param_dtype, dgamma, dbeta, (int)S, C, sg.row_log2, (float)S * (float)(C / G), p.relu)
+    if (sg.per_thread == 1) SFH_GN_SMALL(1);
+    else if (sg.per_thread == 2) SFH_GN_SMALL(2);
+    else SFH_GN_SMALL(4);
+#undef SFH_GN_SMALL
+    return check_launch("gn_small_bwd");
   }
   constexpr int V = VecOf<T>::N;
   const dim3 grid(pl.nsplit, p.n);
