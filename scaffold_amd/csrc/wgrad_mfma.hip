@@ -37,10 +37,13 @@ constexpr int odd16(int bytes) {  // smallest odd multiple of 16 that is >= byte
   return (u % 2 == 0 ? u + 1 : u) * 16;
 }
 
-template <int TD_, int TH_, int TW_>
+// PLANES: the workgroup computes the nine taps of one kd only, so the brick has no halo in depth.
+template <int TD_, int TH_, int TW_, bool PLANES_ = false>
 struct WTile {
   static constexpr int TD = TD_, TH = TH_, TW = TW_;
-  static constexpr int BD = TD + 2, BH = TH + 2;
+  static constexpr bool PLANES = PLANES_;
+  static constexpr int UNITS = PLANES ? 3 : 1;        // workgroups that share a block's 27 taps
+  static constexpr int BD = PLANES ? TD : TD + 2, BH = TH + 2;
   static constexpr int NBR = BD * BH;                 // brick rows
   static constexpr int XR = (TW + 2 + 7) / 8 * 8;     // elements per stored brick row
   static constexpr int NQX = (TW + 2 + 3) / 4;        // 4-voxel groups staged per brick row
@@ -161,20 +164,76 @@ __device__ __forceinline__ void wave_compute(const char* lds, int lane, int wave
   }
 }
 
-template <typename C>
-__device__ __forceinline__ void wave_store(const f32x16_t (&acc)[7], float* __restrict__ dst, int cin, int lane, int wave) {
-  const int j = lane & 31, kg = lane >> 5;
+// The same for one kd: wavefronts 0 .. 2 take the three kw taps of brick row offset kh = wavefront, the fourth only meets the
+// barriers.  Three MFMAs a k-step do not cover a trip to LDS, so fragments are requested two k-steps ahead.
+template <typename T, typename C>
+__device__ __forceinline__ void wave_compute_plane(const char* lds, int lane, int kh, f32x16_t (&acc)[3]) {
+  const int i = lane & 31, kg = lane >> 5;
+  const char* gsrc = lds + C::GOFF + i * C::GC + kg * 16;
+  const char* row = lds + i * C::XC + (C::TW == 8 ? kg * C::XR * 2 : kg * 16) + kh * C::XR * 2;
+  constexpr int LEAD = 2;
+  uint4 af[LEAD + 1], lo[LEAD + 1];
+  uint32_t nx[LEAD + 1];
+  auto load = [&](int ks) {
+    const int b = ks % (LEAD + 1), koff = x_window_off<C>(ks, 0, 0);
+    af[b] = *reinterpret_cast<const uint4*>(gsrc + ks * 32);
+    lo[b] = *reinterpret_cast<const uint4*>(row + koff);
+    nx[b] = *reinterpret_cast<const uint32_t*>(row + koff + 16);
+  };
 #pragma unroll
-  for (int t = 0; t < 7; ++t) {
-    if (t == 6 && wave == 3) break;
-    const int tap = t < 3 ? 6 * wave + t : (t < 6 ? 6 * wave + t : 24 + wave);
+  for (int ks = 0; ks < LEAD; ++ks) load(ks);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int co = 8 * (r / 4) + 4 * kg + (r % 4);
-      dst[((int64_t)co * 27 + tap) * cin + j] = acc[t][r];
+  for (int ks = 0; ks < C::NKS; ++ks) {
+    const int b = ks % (LEAD + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    acc[0] = Mma32<T>::run(af[b], lo[b], acc[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (ks + LEAD < C::NKS) load(ks + LEAD);
+    __builtin_amdgcn_sched_barrier(0);
+    acc[1] = Mma32<T>::run(af[b], shift_one(lo[b], nx[b]), acc[1]);
+    acc[2] = Mma32<T>::run(af[b], make_uint4(lo[b].y, lo[b].z, lo[b].w, nx[b]), acc[2]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// What a compute wavefront accumulates: the 32 x 32 blocks of its taps.
+template <typename T, typename C>
+struct WaveTaps {
+  static constexpr int N = C::PLANES ? 3 : 7;
+  f32x16_t acc[N];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int t = 0; t < N; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+  }
+  __device__ __forceinline__ void add(const char* lds, int lane, int wave) {
+    if constexpr (C::PLANES) {
+      if (wave < 3) wave_compute_plane<T, C>(lds, lane, wave, acc);
+    } else {
+      wave_compute<T, C>(lds, lane, wave, acc);
     }
   }
-}
+  template <typename TOut>
+  __device__ __forceinline__ void store(TOut* __restrict__ dst, int cin, int lane, int wave, int kd) const {
+    if (C::PLANES && wave == 3) return;
+    const int j = lane & 31;
+    int kg = lane >> 5;
+    // (opaque to the optimiser: in a loop over units it would otherwise compute all the store offsets ahead of the loop
+    // and keep them in scratch memory)
+    asm volatile("" : "+v"(kg));
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
+      if (t == 6 && wave == 3) break;
+      const int tap = C::PLANES ? 9 * kd + 3 * wave + t : t < 6 ? 6 * wave + t : 24 + wave;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int co = 8 * (r / 4) + 4 * kg + (r % 4);
+        dst[((int64_t)co * 27 + tap) * cin + j] = elem<TOut>::from_float(acc[t][r]);
+      }
+    }
+  }
+};
 
 // A staging item is (8-channel piece, 4-voxel slot). Within a wavefront the 16 lanes of a quarter share the
 // piece and take 16 consecutive slots: their transposed 8-byte LDS writes to one channel row are then
@@ -314,9 +373,9 @@ struct SlotLoop {
 // staging arithmetic out of the MFMA wavefront's instruction stream (and the two streams on different
 // wavefronts, which issue to different ports concurrently) is what lets the MFMA pipe stay busy.
 // One barrier per tile joins all eight wavefronts.
-template <typename T, typename C>
+template <typename T, typename C, typename TOut>
 __global__ void __launch_bounds__(512)
-wgrad_mfma_kernel(WgradArgs a, const T* __restrict__ x, const T* __restrict__ gy, float* __restrict__ ws, int tiles_d,
+wgrad_mfma_kernel(WgradArgs a, const T* __restrict__ x, const T* __restrict__ gy, TOut* __restrict__ ws, int tiles_d,
                   int tiles_h, int tiles_w, int ntiles, int tiles_per_split, int nblk_ci, int nblk, uint32_t total,
                   const T* __restrict__ x1, int c_first) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -326,6 +385,8 @@ wgrad_mfma_kernel(WgradArgs a, const T* __restrict__ x, const T* __restrict__ gy
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   uint32_t wg = xcd_remap(blockIdx.x, total);
+  const int kd = C::PLANES ? (int)(wg % 3) : 0;  // (neighbours read the same tiles)
+  wg /= C::UNITS;
   const int blk = wg % nblk;
   const int split = wg / nblk;
   const int cib = blk % nblk_ci, cob = blk / nblk_ci;
@@ -341,6 +402,7 @@ wgrad_mfma_kernel(WgradArgs a, const T* __restrict__ x, const T* __restrict__ gy
     // the workgroup's 32 input channels lie in one of them, and from here on that tensor IS the input -- its channel
     // count in `as`, the block's index inside it in `cis`. Only the gradient's own indexing keeps a.cin and cib.
     WgradArgs as = a;
+    as.pd -= kd;
     const T* xs = x;
     int cis = cib;
     if (x1 != nullptr) {
@@ -372,22 +434,18 @@ wgrad_mfma_kernel(WgradArgs a, const T* __restrict__ x, const T* __restrict__ gy
   }
 
   // ---- compute wavefronts ----
-  f32x16_t acc[7];
-#pragma unroll
-  for (int t = 0; t < 7; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+  WaveTaps<T, C> taps;
+  taps.clear();
   if (t_begin < t_end) {
     __builtin_amdgcn_s_barrier();  // the first tile is staged
     for (int tile = t_begin; tile < t_end; ++tile) {
       const char* cur = ((tile - t_begin) & 1) ? buf1 : buf0;
       asm volatile("" ::: "memory");  // LDS changes behind this wavefront's back: reload every tile
-      wave_compute<T, C>(cur, lane, wave, acc);
+      taps.add(cur, lane, wave);
       __builtin_amdgcn_s_barrier();
     }
   }
-  float* dst = ws + ((int64_t)split * a.cout + cob * 32) * 27 * a.cin + cib * 32;
-  wave_store<C>(acc, dst, a.cin, lane, wave);
+  taps.store(ws + ((int64_t)split * a.cout + cob * 32) * 27 * a.cin + cib * 32, a.cin, lane, wave, kd);
 #endif
 }
 
@@ -417,37 +475,20 @@ struct WTileBatchEntry {
 
 struct WTileBatch {
   int count, wgs, total;
+  bool planes;                         // units are (problem, block, kd)
   WTileBatchEntry e[kWgradBatchMax];
 };
-
-template <typename C, typename TOut>
-__device__ __forceinline__ void wave_store_block(const f32x16_t (&acc)[7], TOut* __restrict__ dst, int cin, int lane, int wave) {
-  const int j = lane & 31;
-  int kg = lane >> 5;
-  // (opaque to the optimiser: in the loop over units it would otherwise compute all 112 store offsets ahead of the loop
-  // and keep them in scratch memory)
-  asm volatile("" : "+v"(kg));
-#pragma unroll
-  for (int t = 0; t < 7; ++t) {
-    if (t == 6 && wave == 3) break;
-    const int tap = t < 3 ? 6 * wave + t : (t < 6 ? 6 * wave + t : 24 + wave);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int co = 8 * (r / 4) + 4 * kg + (r % 4);
-      dst[((int64_t)co * 27 + tap) * cin + j] = elem<TOut>::from_float(acc[t][r]);
-    }
-  }
-}
 
 // One unit: all tiles of block (cob, cib) of a problem, the finished block stored at gw. The staging wavefronts and
 // the compute wavefronts meet at 1 + ntiles barriers, as in the kernel above.
 template <typename T, typename C, typename TOut>
 __device__ __forceinline__ void wtile_unit(const WgradArgs& a, const T* __restrict__ x, const T* __restrict__ x1, int c_first,
                                            const T* __restrict__ gy, TOut* __restrict__ gw, int tiles_d, int tiles_h, int tiles_w,
-                                           int ntiles, int cib, int cob, char* buf0, char* buf1, int tid) {
+                                           int ntiles, int cib, int cob, int kd, char* buf0, char* buf1, int tid) {
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (wave >= 4) {
     WgradArgs as = a;
+    as.pd -= kd;
     const T* xs = x;
     int cis = cib;
     if (x1 != nullptr) {
@@ -471,31 +512,28 @@ __device__ __forceinline__ void wtile_unit(const WgradArgs& a, const T* __restri
       __builtin_amdgcn_s_barrier();
     }
   } else {
-    f32x16_t acc[7];
-#pragma unroll
-    for (int t = 0; t < 7; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+    WaveTaps<T, C> taps;
+    taps.clear();
     __builtin_amdgcn_s_barrier();  // the first tile is staged
     for (int tile = 0; tile < ntiles; ++tile) {
       const char* cur = (tile & 1) ? buf1 : buf0;
       asm volatile("" ::: "memory");  // LDS changes behind this wavefront's back: reload every tile
-      wave_compute<T, C>(cur, lane, wave, acc);
+      taps.add(cur, lane, wave);
       __builtin_amdgcn_s_barrier();
     }
-    wave_store_block<C, TOut>(acc, gw + ((int64_t)cob * 32 * 27) * a.cin + cib * 32, a.cin, lane, wave);
+    taps.store(gw + ((int64_t)cob * 32 * 27) * a.cin + cib * 32, a.cin, lane, wave, kd);
   }
 }
 
-typedef WTile<2, 8, 16> WTile16;
-typedef WTile<4, 8, 8> WTile8;
-constexpr int kBatchLds = WTile16::LDS > WTile8::LDS ? WTile16::LDS : WTile8::LDS;
 
 __host__ __device__ __forceinline__ int tile_batch_cut(int w, int total, int wgs) { return (int)((uint32_t)w * (uint32_t)total / (uint32_t)wgs); }
 
-template <typename T, typename TOut>
+template <typename T, typename TOut, bool PLANES>
 __global__ void __launch_bounds__(512) wgrad_mfma_batch_kernel(WTileBatch b) {
 #if defined(__HIP_DEVICE_COMPILE__)
+  typedef WTile<2, 8, 16, PLANES> Tile16;
+  typedef WTile<4, 8, 8, PLANES> Tile8;
+  constexpr int kUnits = Tile16::UNITS, kBatchLds = Tile16::LDS > Tile8::LDS ? Tile16::LDS : Tile8::LDS;
   __shared__ __attribute__((aligned(16))) char buf0[kBatchLds];
   __shared__ __attribute__((aligned(16))) char buf1[kBatchLds];
   const int tid = threadIdx.x;
@@ -508,7 +546,7 @@ __global__ void __launch_bounds__(512) wgrad_mfma_batch_kernel(WTileBatch b) {
       if (pos >= b.e[k].pos_begin) p = k;
     const int ntiles = b.e[p].ntiles, cost = ntiles + kUnitCost;
     const int unit = (pos - b.e[p].pos_begin + cost - 1) / cost;  // the first unit that starts at or behind pos
-    if (unit >= b.e[p].nblk) {  // none left in this problem: on to the next one's first unit
+    if (unit >= b.e[p].nblk * kUnits) {  // none left in this problem: on to the next one's first unit
       pos = p + 1 < b.count ? b.e[p + 1].pos_begin : hi;
       continue;
     }
@@ -516,13 +554,14 @@ __global__ void __launch_bounds__(512) wgrad_mfma_batch_kernel(WTileBatch b) {
     if (start >= hi) break;
     const WgradArgs a = b.e[p].a;
     const int nblk_ci = b.e[p].nblk_ci;
-    const int cib = unit % nblk_ci, cob = unit / nblk_ci;
+    const int kd = PLANES ? unit % 3 : 0, blk = unit / kUnits;
+    const int cib = blk % nblk_ci, cob = blk / nblk_ci;
     if (b.e[p].tw == 16)
-      wtile_unit<T, WTile16, TOut>(a, (const T*)b.e[p].x, (const T*)b.e[p].x1, b.e[p].c_first, (const T*)b.e[p].gy, (TOut*)b.e[p].gw,
-                                   b.e[p].tiles_d, b.e[p].tiles_h, b.e[p].tiles_w, ntiles, cib, cob, buf0, buf1, tid);
+      wtile_unit<T, Tile16, TOut>(a, (const T*)b.e[p].x, (const T*)b.e[p].x1, b.e[p].c_first, (const T*)b.e[p].gy, (TOut*)b.e[p].gw,
+                                   b.e[p].tiles_d, b.e[p].tiles_h, b.e[p].tiles_w, ntiles, cib, cob, kd, buf0, buf1, tid);
     else
-      wtile_unit<T, WTile8, TOut>(a, (const T*)b.e[p].x, (const T*)b.e[p].x1, b.e[p].c_first, (const T*)b.e[p].gy, (TOut*)b.e[p].gw,
-                                  b.e[p].tiles_d, b.e[p].tiles_h, b.e[p].tiles_w, ntiles, cib, cob, buf0, buf1, tid);
+      wtile_unit<T, Tile8, TOut>(a, (const T*)b.e[p].x, (const T*)b.e[p].x1, b.e[p].c_first, (const T*)b.e[p].gy, (TOut*)b.e[p].gw,
+                                  b.e[p].tiles_d, b.e[p].tiles_h, b.e[p].tiles_w, ntiles, cib, cob, kd, buf0, buf1, tid);
     pos = start + cost;
   }
 #endif
@@ -533,6 +572,7 @@ struct Plan {
   int tiles_d, tiles_h, tiles_w, ntiles;
   int nblk_ci, nblk;
   int splits, tiles_per_split;
+  bool planes;  // three workgroups to a block, one per kd
 };
 
 // Rows of more than 16 voxels take the column-walking kernel.
@@ -560,48 +600,86 @@ Plan make_plan(const WgradArgs& a) {
   // block is 108 KiB of fp32 that is written and, when there is more than one slice, read again by the ordered sum
   // (a launch of its own). Units of 0.01 us, constants fitted to timings of the U-Net's levels: the small-volume
   // levels (8 tiles for 64-128 blocks) are cheaper with 1-4 slices than with one per CU.
-  int target = kTargetWorkgroups;
-  int want = target / p.nblk;
-  if (want < 1) want = 1;
-  if (want > p.ntiles) want = p.ntiles;
+  // Three workgroups to a block, nine taps each, stage less per tile and compute for half the time (130 instead of 240), at
+  // the price of staging the gradient three times: worth it while the chip has room for them.  Measured (us, gradient in 16
+  // bits, one workgroup to a block and a sum pass / three, stored in place where one slice is left): 256 -> 256 channels on
+  // 8 x 16 x 16 32.9 / 19.6, on 8 x 8 x 8 18.3 / 9.0, 128 -> 128 on 16 x 16 x 16 21.8 / 17.7 (four slices).
   int64_t best = -1;
-  for (int s = want; s >= 1; s /= 2) {
-    const int tps = (int)cdiv(p.ntiles, s), eff = (int)cdiv(p.ntiles, tps);
-    const int64_t cost = eff > 1 ? 240LL * tps + 1000 + 64LL * eff * p.nblk / 10 : 240LL * tps + 600 + 32LL * p.nblk / 10;
-    if (best < 0 || cost < best) {
-      best = cost;
-      p.tiles_per_split = tps;
-      p.splits = eff;
+  for (int units = 1; units <= 3; units += 2) {
+    if (units == 3 && (p.tw == 32 || units * p.nblk > kTargetWorkgroups)) break;
+    const int64_t tile = units == 3 ? 130 : 240;
+    int want = kTargetWorkgroups / (p.nblk * units);
+    if (want < 1) want = 1;
+    if (want > p.ntiles) want = p.ntiles;
+    for (int s = want; s >= 1; s /= 2) {
+      const int tps = (int)cdiv(p.ntiles, s), eff = (int)cdiv(p.ntiles, tps);
+      const int64_t cost = eff > 1 ? tile * tps + 1000 + 64LL * eff * p.nblk / 10 : tile * tps + 600 + 32LL * p.nblk / 10;
+      if (best < 0 || cost < best) {
+        best = cost;
+        p.tiles_per_split = tps;
+        p.splits = eff;
+        p.planes = units == 3;
+      }
     }
   }
   return p;
 }
 
 template <typename T, typename C>
-int launch_tile(const WgradArgs& a, const Plan& p, const void* x, const void* gy, float* ws, hipStream_t st, const ChannelPair& x2) {
-  const int64_t total = (int64_t)p.splits * p.nblk;
-  hipLaunchKernelGGL((wgrad_mfma_kernel<T, C>), dim3((unsigned)total), dim3(512), 0, st, a, (const T*)x, (const T*)gy, ws,
-                     p.tiles_d, p.tiles_h, p.tiles_w, p.ntiles, p.tiles_per_split, p.nblk_ci, p.nblk, (uint32_t)total,
-                     (const T*)x2.second, x2.first);
+int launch_tile(const WgradArgs& a, const Plan& p, const void* x, const void* gy, void* out, bool own_dtype, hipStream_t st, const ChannelPair& x2) {
+  const int64_t total = (int64_t)p.splits * p.nblk * C::UNITS;
+#define SFH_WGRAD_TILE(TOUT)                                                                                                        \
+  hipLaunchKernelGGL((wgrad_mfma_kernel<T, C, TOUT>), dim3((unsigned)total), dim3(512), 0, st, a, (const T*)x, (const T*)gy, (TOUT*)out, \
+                     p.tiles_d, p.tiles_h, p.tiles_w, p.ntiles, p.tiles_per_split, p.nblk_ci, p.nblk, (uint32_t)total,               \
+                     (const T*)x2.second, x2.first)
+  if (own_dtype) SFH_WGRAD_TILE(T);
+  else SFH_WGRAD_TILE(float);
+#undef SFH_WGRAD_TILE
   return check_launch("wgrad_mfma_kernel");
 }
 
 template <typename T>
 int launch_typed(const WgradArgs& a, const void* x, const void* gy, void* gw, int gw_dtype, void* workspace, hipStream_t st,
                  const ChannelPair& x2) {
+  constexpr int kOwn = std::is_same<T, bf16_t>::value ? SFH_BF16 : SFH_FP16;
   const Plan p = make_plan(a);
-  // One slice and an fp32 gradient (the deepest levels under fp32 master weights): the kernel's slice IS the
-  // gradient, so it is written in place and no sum pass follows.
-  const bool direct = p.splits == 1 && gw_dtype == SFH_FP32;
-  float* ws = direct ? (float*)gw : (float*)workspace;
+  const bool ring = ring_serves(a);
+  // One slice: what the kernel stores IS the gradient (rounded on the way if it is a 16-bit one), so it is written in place
+  // and no sum pass follows.
+  const bool direct = p.splits == 1 && (gw_dtype == SFH_FP32 || (gw_dtype == kOwn && !ring));
+  const bool own = direct && gw_dtype == kOwn;
+  void* out = direct ? gw : workspace;
   int rc;
-  if (ring_serves(a)) rc = mfma_wgrad_ring(a, std::is_same<T, bf16_t>::value ? SFH_BF16 : SFH_FP16, x, gy, ws, st, x2);
-  else if (p.tw == 32) rc = launch_tile<T, WTile<2, 4, 32>>(a, p, x, gy, ws, st, x2);
-  else if (p.tw == 16) rc = launch_tile<T, WTile<2, 8, 16>>(a, p, x, gy, ws, st, x2);
-  else rc = launch_tile<T, WTile<4, 8, 8>>(a, p, x, gy, ws, st, x2);
+  if (ring) rc = mfma_wgrad_ring(a, kOwn, x, gy, (float*)out, st, x2);
+  else if (p.tw == 32) rc = launch_tile<T, WTile<2, 4, 32>>(a, p, x, gy, out, own, st, x2);
+  else if (p.tw == 16 && p.planes) rc = launch_tile<T, WTile<2, 8, 16, true>>(a, p, x, gy, out, own, st, x2);
+  else if (p.tw == 16) rc = launch_tile<T, WTile<2, 8, 16>>(a, p, x, gy, out, own, st, x2);
+  else if (p.planes) rc = launch_tile<T, WTile<4, 8, 8, true>>(a, p, x, gy, out, own, st, x2);
+  else rc = launch_tile<T, WTile<4, 8, 8>>(a, p, x, gy, out, own, st, x2);
   if (rc != SFH_OK || direct) return rc;
   const int64_t nelem = (int64_t)a.cout * 27 * a.cin;
-  return sum_slices(gw_dtype, ws, gw, nelem, p.splits, st);
+  return sum_slices(gw_dtype, (const float*)workspace, gw, nelem, p.splits, st);
+}
+
+// The largest load of a workgroup, in cost, when every block is `units` units (a line of cost `units` times as long).
+int64_t busiest(const WTileBatch& b, int units) {
+  const int total = b.total * units, wgs = total < kTargetWorkgroups ? total : kTargetWorkgroups;
+  int64_t most = 0;
+  int p = 0;
+  for (int w = 0; w < wgs; ++w) {
+    const int hi = tile_batch_cut(w + 1, total, wgs);
+    int64_t load = 0;
+    for (int pos = tile_batch_cut(w, total, wgs); pos < hi;) {
+      while (p + 1 < b.count && pos >= b.e[p + 1].pos_begin * units) ++p;
+      const int begin = b.e[p].pos_begin * units, cost = b.e[p].ntiles + kUnitCost;
+      const int end = p + 1 < b.count ? b.e[p + 1].pos_begin * units : total;
+      const int upto = end < hi ? end : hi;
+      load += (int64_t)((upto - begin + cost - 1) / cost - (pos - begin + cost - 1) / cost) * cost;  // units that start in [pos, upto)
+      pos = upto;
+    }
+    if (load > most) most = load;
+  }
+  return most;
 }
 
 bool tile_batch_plan(const WgradBatchItem* items, int count, WTileBatch& b) {
@@ -626,14 +704,33 @@ bool tile_batch_plan(const WgradBatchItem* items, int count, WTileBatch& b) {
   }
   b.total = (int)pos;
   b.wgs = b.total < kTargetWorkgroups ? b.total : kTargetWorkgroups;
+  // Blocks shared by three workgroups: where the busiest one's load, in tiles of 1.7 us instead of 2.4, is then smaller.
+  // (With at least one block per compute unit the chip is busy as it is.)
+  if (pos * 3 <= 0x7fffff) {
+    int64_t blocks = 0;
+    for (int i = 0; i < count; ++i) blocks += b.e[i].nblk;
+    if (3 * blocks <= kTargetWorkgroups || (blocks <= kTargetWorkgroups && 17 * busiest(b, 3) < 24 * busiest(b, 1))) {
+      b.planes = true;
+      b.total *= 3;
+      for (int i = 0; i < count; ++i) b.e[i].pos_begin *= 3;
+      b.wgs = b.total < kTargetWorkgroups ? b.total : kTargetWorkgroups;
+    }
+  }
   return true;
 }
 
 template <typename T>
 int launch_tile_batch(const WTileBatch& b, int gw_dtype, hipStream_t st) {
   if (b.total == 0) return SFH_OK;
-  if (gw_dtype == SFH_FP32) hipLaunchKernelGGL((wgrad_mfma_batch_kernel<T, float>), dim3((unsigned)b.wgs), dim3(512), 0, st, b);
-  else hipLaunchKernelGGL((wgrad_mfma_batch_kernel<T, T>), dim3((unsigned)b.wgs), dim3(512), 0, st, b);
+#define SFH_WGRAD_BATCH(TOUT, PLANES) hipLaunchKernelGGL((wgrad_mfma_batch_kernel<T, TOUT, PLANES>), dim3((unsigned)b.wgs), dim3(512), 0, st, b)
+  if (b.planes) {
+    if (gw_dtype == SFH_FP32) SFH_WGRAD_BATCH(float, true);
+    else SFH_WGRAD_BATCH(T, true);
+  } else {
+    if (gw_dtype == SFH_FP32) SFH_WGRAD_BATCH(float, false);
+    else SFH_WGRAD_BATCH(T, false);
+  }
+#undef SFH_WGRAD_BATCH
   return check_launch("wgrad_mfma_batch_kernel");
 }
 

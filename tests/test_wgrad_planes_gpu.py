@@ -1,0 +1,52 @@
+"""Small-volume weight gradients whose blocks are shared by three workgroups (nine taps each), alone and in a list: ragged tiles
+on every axis, paddings, batches, both tile shapes, one and several slices, results in the operands' type and in fp32."""
+import pytest
+import torch
+
+import scaffold_amd as sa
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+# (n, cin, cout, spatial, padding, dtype)
+CASES = [
+    (1, 32, 32, (1, 1, 1), 1, torch.bfloat16), (1, 64, 32, (5, 7, 9), 1, torch.bfloat16), (2, 32, 64, (3, 9, 16), 1, torch.float16),
+    (1, 64, 64, (4, 8, 8), 1, torch.bfloat16), (1, 32, 32, (12, 10, 8), (0, 1, 2), torch.bfloat16), (2, 96, 64, (9, 17, 11), (2, 0, 1), torch.bfloat16),
+    (1, 256, 256, (8, 16, 16), 1, torch.float16),  # 64 blocks: one slice, stored in place
+    (1, 288, 256, (3, 5, 8), 1, torch.bfloat16),   # 72 blocks
+    (1, 320, 288, (3, 5, 8), 1, torch.bfloat16),   # 90 blocks: more than the chip has room for three times
+]
+
+
+def _problem(n, cin, cout, spatial, padding, dtype, seed):
+    prob = orc.ConvProblem(n=n, cin=cin, cout=cout, spatial=spatial, dtype=dtype,
+                           padding=(padding,) * 3 if isinstance(padding, int) else padding)
+    return prob, orc.make_inputs(prob, seed=seed)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_alone(case):
+    prob, ops = _problem(*case, seed=3)
+    x, gy = ops["input"].cuda(), ops["grad_output"].cuda()
+    want = orc.conv_reference(prob, ops, "bwd-weight")
+    got = sa.conv3d_backward_weight(x, prob.weight_shape, gy, 1, case[4])
+    orc.assert_close(got, want, prob, "bwd-weight")
+    wide = sa.conv3d_backward_weight(x, prob.weight_shape, gy, 1, case[4], grad_dtype=torch.float32)
+    assert torch.equal(wide.to(got.dtype), got)
+
+
+@pytest.mark.parametrize("grad_dtype", [None, torch.float32])
+@pytest.mark.parametrize("extra", [0, 1])
+def test_in_a_list(grad_dtype, extra):
+    # extra: a problem of 64 blocks more, which takes the list past one round of shared blocks; the bits do not change
+    cases = [(1, 32, 32, (12, 10, 8), (0, 1, 2), torch.bfloat16), (1, 64, 64, (4, 8, 8), 1, torch.bfloat16), (1, 64, 32, (5, 7, 9), 1, torch.bfloat16),
+             (1, 64, 64, (16, 16, 16), 1, torch.bfloat16)]
+    problems = [_problem(*c, seed=5 + i) for i, c in enumerate(cases + [(1, 256, 256, (4, 8, 8), 1, torch.bfloat16)] * extra)]
+    items = [(o["input"].cuda(), p.weight_shape, o["grad_output"].cuda(), c) for (p, o), c in
+             zip(problems, [(0, 1, 2), (1, 1, 1), (1, 1, 1), (1, 1, 1), (1, 1, 1)])]
+    got = sa.conv3d_backward_weight_batch(items, grad_dtype=grad_dtype)
+    for (prob, ops), g in zip(problems, got):
+        orc.assert_close(g.to(torch.bfloat16), orc.conv_reference(prob, ops, "bwd-weight"), prob, "bwd-weight")
+    if extra:
+        short = sa.conv3d_backward_weight_batch(items[:4], grad_dtype=grad_dtype)
+        assert all(torch.equal(a, b) for a, b in zip(short, got))
