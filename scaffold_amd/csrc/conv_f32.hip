@@ -41,6 +41,10 @@ struct FTile {
   static constexpr int PLANE = plane_bytes(BV);
   static constexpr int LDS = 4 * PLANE;
   static constexpr int MS = TD * TH * TW / 128;  // 32-voxel sub-tiles per wavefront
+  // One sub-tile to a wavefront is what a volume gets that does not fill the chip: nothing else on the SIMD hides a trip to
+  // memory or LDS, and there are registers for requesting the next chunk's brick and the next tap's activations ahead.
+  // 32 -> 32 channels on 32^3: 27.4 -> 20.5 us a launch (its MFMAs alone 11.5).
+  static constexpr bool AHEAD = MS == 1;
   static_assert(TD * TH * TW % 128 == 0, "tile must split into 4 wavefronts of 32-voxel sub-tiles");
   static_assert(2 * LDS <= 160 * 1024, "two workgroups in the 160 KB LDS of a CU");
   static_assert(PLANE + (2 * BH * BW + 2 * BW + 2) * 16 < 65536, "ds_read immediate range");
@@ -87,59 +91,84 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
   const int ncc = a.cred / kChunk;
   constexpr int PIECES = C::BV * 4;
   constexpr int ITERS = (PIECES + 255) / 256;
-  constexpr int BATCH = 8;  // staging loads in flight before the first LDS write
+  constexpr int BATCH = C::AHEAD ? ITERS : 8;  // staging loads in flight before the first LDS write
   const float* xn = x + (int64_t)n * a.id * a.ih * a.iw * a.cred;
-  for (int cc = 0; cc < ncc; ++cc) {
-    __syncthreads();  // every wave is done reading the previous chunk
+  auto request = [&](int cc, int it0, float4 (&v)[BATCH]) {
 #pragma unroll
-    for (int it0 = 0; it0 < ITERS; it0 += BATCH) {
-      float4 v[BATCH];
-#pragma unroll
-      for (int u = 0; u < BATCH; ++u) {
-        if (it0 + u < ITERS) {
-          // unconditional load from a clamped address, masked afterwards (a load under a branch waits for the one before)
-          const int p = (it0 + u) * 256 + tid;
-          const int vox = p >> 2, piece = p & 3;
-          const int bw = vox % C::BW, bh = (vox / C::BW) % C::BH, bd = vox / (C::BW * C::BH);
-          const int id = id0 + bd, ih = ih0 + bh, iw = iw0 + bw;
-          const bool in = p < PIECES && (unsigned)id < (unsigned)a.id && (unsigned)ih < (unsigned)a.ih && (unsigned)iw < (unsigned)a.iw;
-          const int64_t at = in ? (((int64_t)id * a.ih + ih) * a.iw + iw) * a.cred + cc * kChunk + piece * 4 : 0;
-          const float4 got = *reinterpret_cast<const float4*>(xn + at);
-          v[u] = in ? got : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
+    for (int u = 0; u < BATCH; ++u) {
+      if (it0 + u < ITERS) {
+        // unconditional load from a clamped address, masked afterwards (a load under a branch waits for the one before)
+        const int p = (it0 + u) * 256 + tid;
+        const int vox = p >> 2, piece = p & 3;
+        const int bw = vox % C::BW, bh = (vox / C::BW) % C::BH, bd = vox / (C::BW * C::BH);
+        const int id = id0 + bd, ih = ih0 + bh, iw = iw0 + bw;
+        const bool in = p < PIECES && (unsigned)id < (unsigned)a.id && (unsigned)ih < (unsigned)a.ih && (unsigned)iw < (unsigned)a.iw;
+        const int64_t at = in ? (((int64_t)id * a.ih + ih) * a.iw + iw) * a.cred + cc * kChunk + piece * 4 : 0;
+        const float4 got = *reinterpret_cast<const float4*>(xn + at);
+        v[u] = in ? got : make_float4(0.f, 0.f, 0.f, 0.f);
       }
+    }
+  };
+  auto stage = [&](int it0, const float4 (&v)[BATCH]) {
 #pragma unroll
-      for (int u = 0; u < BATCH; ++u) {
-        if (it0 + u < ITERS) {
-          const int p = (it0 + u) * 256 + tid;
-          if (p < PIECES) *reinterpret_cast<float4*>(lds + (p & 3) * C::PLANE + (p >> 2) * 16) = v[u];
-        }
+    for (int u = 0; u < BATCH; ++u) {
+      if (it0 + u < ITERS) {
+        const int p = (it0 + u) * 256 + tid;
+        if (p < PIECES) *reinterpret_cast<float4*>(lds + (p & 3) * C::PLANE + (p >> 2) * 16) = v[u];
+      }
+    }
+  };
+  // weight fragments of tap t: packed + (((nb * ncc + cc) * 27 + t) * 2 + q) * 256 floats + lane * 4; the taps of a chunk
+  // are followed by the next chunk's, so the requests ahead run on over the end of a chunk
+  const float* wcc = wp + ((int64_t)(nb * ncc) * kTaps * 2) * 256 + lane * 4;
+  constexpr int WDEPTH = 3;  // taps requested ahead
+  static_assert(kTaps % WDEPTH == 0, "a chunk ends where the ring of requests began");
+  float4 wq[WDEPTH][2];
+#pragma unroll
+  for (int d = 0; d < WDEPTH; ++d)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) wq[d][q] = *reinterpret_cast<const float4*>(wcc + (d * 2 + q) * 256);
+  float4 v[BATCH];
+  if (C::AHEAD) request(0, 0, v);
+  for (int cc = 0; cc < ncc; ++cc, wcc += kTaps * 2 * 256) {
+    const bool more = cc + 1 < ncc;
+    __syncthreads();  // every wave is done reading the previous chunk
+    if constexpr (C::AHEAD) {
+      stage(0, v);
+    } else {
+#pragma unroll
+      for (int it0 = 0; it0 < ITERS; it0 += BATCH) {
+        request(cc, it0, v);
+        stage(it0, v);
       }
     }
     __syncthreads();
+    if (C::AHEAD && more) request(cc + 1, 0, v);
 
-    // weight fragments of tap t: packed + (((nb * ncc + cc) * 27 + t) * 2 + q) * 256 floats + lane * 4
-    const float* wcc = wp + ((int64_t)(nb * ncc + cc) * kTaps * 2) * 256 + lane * 4;
-    constexpr int WDEPTH = 3;  // taps requested ahead
-    float4 wq[WDEPTH][2];
+    constexpr int ADEPTH = C::AHEAD ? 2 : 1;  // taps whose activations are held
+    float4 af[ADEPTH][C::MS][2];
+    auto activations = [&](int tap) {
 #pragma unroll
-    for (int d = 0; d < WDEPTH; ++d)
-#pragma unroll
-      for (int q = 0; q < 2; ++q) wq[d][q] = *reinterpret_cast<const float4*>(wcc + (d * 2 + q) * 256);
+      for (int ms = 0; ms < C::MS; ++ms) {
+        af[tap % ADEPTH][ms][0] = *reinterpret_cast<const float4*>(lds + lbase[ms] + tap_off<C>(tap));
+        af[tap % ADEPTH][ms][1] = *reinterpret_cast<const float4*>(lds + lbase[ms] + C::PLANE + tap_off<C>(tap));
+      }
+    };
+    if (C::AHEAD) activations(0);
 #pragma unroll
     for (int tap = 0; tap < kTaps; ++tap) {
       float4 wf[2] = {wq[tap % WDEPTH][0], wq[tap % WDEPTH][1]};
-      if (tap + WDEPTH < kTaps) {
+      if (tap + WDEPTH < kTaps || more) {
 #pragma unroll
         for (int q = 0; q < 2; ++q) wq[tap % WDEPTH][q] = *reinterpret_cast<const float4*>(wcc + ((tap + WDEPTH) * 2 + q) * 256);
       }
-      // the sub-tiles take turns, so consecutive MFMAs do not wait for one another's result
-      float4 af[C::MS][2];
-#pragma unroll
-      for (int ms = 0; ms < C::MS; ++ms) {
-        af[ms][0] = *reinterpret_cast<const float4*>(lds + lbase[ms] + tap_off<C>(tap));
-        af[ms][1] = *reinterpret_cast<const float4*>(lds + lbase[ms] + C::PLANE + tap_off<C>(tap));
+      if constexpr (C::AHEAD) {
+        if (tap + 1 < kTaps) activations(tap + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+        activations(tap);
       }
+      // the sub-tiles take turns, so consecutive MFMAs do not wait for one another's result
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         const float wv[4] = {wf[q].x, wf[q].y, wf[q].z, wf[q].w};
@@ -147,11 +176,13 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
         for (int e = 0; e < 4; ++e) {
 #pragma unroll
           for (int ms = 0; ms < C::MS; ++ms) {
-            const float av[4] = {af[ms][q].x, af[ms][q].y, af[ms][q].z, af[ms][q].w};
+            const float4 act = af[tap % ADEPTH][ms][q];
+            const float av[4] = {act.x, act.y, act.z, act.w};
             acc[ms] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[e], av[e], acc[ms], 0, 0, 0);
           }
         }
       }
+      if constexpr (C::AHEAD) __builtin_amdgcn_sched_barrier(0);
     }
   }
 
@@ -213,21 +244,37 @@ int launch(const MfmaConvArgs& a, const void* x, const void* packed, const void*
 // TWO voxels and a lane supplies ONE value per operand: row operand gy[voxel 2s + kg][co = lane % 32], column operand
 // x[that voxel + tap][ci = lane % 32] -- both are 32 consecutive floats of a channels-last row, so unlike the 16-bit
 // kernel nothing has to be transposed and the operands come straight from global memory (L1 / L2 serve the 27-fold
-// reuse of x). A workgroup owns one (32 co, 32 ci) block and a contiguous range of output rows; its four wavefronts
-// split the 27 taps 7 / 7 / 7 / 6. Split-K over the rows: fp32 partial slices [Cout][27][Cin] at fixed workspace slots,
+// reuse of x). A workgroup owns one (32 co, 32 ci) block and a contiguous range of passes (8 voxels of an output row); its
+// wavefronts split the 27 taps 7 / 7 / 7 / 6. Split-K over the passes: fp32 partial slices [Cout][27][Cin] at fixed workspace slots,
 // summed in fixed order afterwards (reduce_gemm.py:396-435) -- no float atomics, split count a pure function of shape.
-constexpr int kPairsPerPass = 4;  // voxel pairs whose loads are issued before the first MFMA of a pass
+//
+// What bounds it at 32^3 and below is not the matrix pipe but the slices (110 KB each, written and read again) and the trip
+// to memory in front of every pass. So a workgroup is eight wavefronts, two to a tap range: they take the passes of the
+// range in turn and meet in LDS (114 KB) before the slice is written, which gives the same wavefronts per CU from half of
+// the slices; a pass's operands are requested while the pass before it computes.
+// 32 -> 32 channels on 32^3: kernel 42.1 -> 35.4 us (its MFMAs alone 11.5), slice sum 9.8 -> 5.9.  One set of eight wavefronts
+// without the requests ahead: 45.6.
+constexpr int kPairsPerPass = 4;  // voxel pairs of a pass
+constexpr int kPassVoxels = 2 * kPairsPerPass;
+constexpr uint32_t kOutside = 0x7ffffff0;  // an offset behind every row (f32_wgrad_supported)
 
-__global__ void __launch_bounds__(256, 2)
+struct PassOperands {
+  float gy[kPairsPerPass], x[kPairsPerPass][7];
+};
+
+__global__ void __launch_bounds__(512, 2)
 wgrad_f32_kernel(WgradArgs a, const float* __restrict__ x, const float* __restrict__ gy, float* __restrict__ partial, int nsplit, int cibs) {
+  __shared__ float meet[4][7 * 16][64];
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wave8 & 3, half = wave8 >> 2;
   const int i = lane & 31, kg = lane >> 5;
   int b = blockIdx.x;
   const int split = b % nsplit; b /= nsplit;
   const int cib = b % cibs, cob = b / cibs;
-  const int64_t rows = (int64_t)a.n * a.od * a.oh;
-  const int64_t r_begin = split * rows / nsplit, r_end = (split + 1) * rows / nsplit;
+  const int row_passes = (a.ow + kPassVoxels - 1) / kPassVoxels;
+  const int64_t passes = (int64_t)a.n * a.od * a.oh * row_passes;  // below 2^31 (f32_wgrad_supported)
+  const int p_begin = (int)(split * passes / nsplit), p_end = (int)((split + 1) * passes / nsplit);
   const int ntaps = wave < 3 ? 7 : 6;
   const int tap0 = wave * 7;
 
@@ -237,44 +284,63 @@ wgrad_f32_kernel(WgradArgs a, const float* __restrict__ x, const float* __restri
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
 
-  const float* gyb = gy + cob * 32 + i;
-  const float* xb = x + cib * 32 + i;
-  for (int64_t row = r_begin; row < r_end; ++row) {
-    const int oh = (int)(row % a.oh);
-    const int od = (int)((row / a.oh) % a.od);
-    const int n = (int)(row / ((int64_t)a.oh * a.od));
-    const float* gyr = gyb + row * a.ow * a.cout;
-    // per tap of this wavefront: pointer to x at (n, od + kd - pd, oh + kh - ph, kw - pw) or null when that input row is padding
-    const float* xr[7];
+  const float* gyb = gy + cob * 32;
+  const float* xb = x + cib * 32;
+  // One buffer per operand row: a voxel outside of it -- padding, the end of a row, a row of padding (no records) -- reads
+  // as zero, with no mask on the loaded value (which would wait for it). A negative offset is as far out as a large one.
+  auto request = [&](int pass, PassOperands& o) {
+    const int row = pass / row_passes, w0 = (pass - row * row_passes) * kPassVoxels;
+    const int plane = row / a.oh, oh = row - plane * a.oh, n = plane / a.od, od = plane - n * a.od;
+    const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(gyb + (int64_t)row * a.ow * a.cout), 0, a.ow * a.cout * 4 - cob * 128, 0x00020000);
+    const int gat = (w0 + kg) * a.cout * 4 + i * 4, xat = (w0 + kg - a.pw) * a.cin * 4 + i * 4;
+#pragma unroll
+    for (int u = 0; u < kPairsPerPass; ++u)
+      o.gy[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(gr, gat + 2 * u * a.cout * 4, 0, 0));
 #pragma unroll
     for (int t = 0; t < 7; ++t) {
       const int tap = tap0 + t;
       const int kd = tap / 9, kh = (tap / 3) % 3, kw = tap % 3;
       const int id = od + kd - a.pd, ih = oh + kh - a.ph;
-      const bool ok = t < ntaps && (unsigned)id < (unsigned)a.id && (unsigned)ih < (unsigned)a.ih;
-      xr[t] = ok ? xb + ((((int64_t)n * a.id + id) * a.ih + ih) * a.iw + (kw - a.pw)) * a.cin : nullptr;
-    }
-    for (int w0 = 0; w0 < a.ow; w0 += 2 * kPairsPerPass) {
-      float av[kPairsPerPass], bv[kPairsPerPass][7];
+      const int64_t xrow = ((int64_t)n * a.id + id) * a.ih + ih;
+      // (voxels that belong to no output of the row end the records too: 0 x infinity is not 0)
+      const int w_end = a.iw < a.ow + kw - a.pw ? a.iw : a.ow + kw - a.pw;
+      const bool row_ok = (t < ntaps) & (w_end > 0) & ((unsigned)id < (unsigned)a.id) & ((unsigned)ih < (unsigned)a.ih);
+      const int records = w_end * a.cin * 4 - cib * 128;
+      const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xb + xrow * a.iw * a.cin), 0,
+                                                                          row_ok ? records : 0, 0x00020000);
 #pragma unroll
       for (int u = 0; u < kPairsPerPass; ++u) {
-        const int w = w0 + 2 * u + kg;  // this lane's voxel of pair u
-        const bool wok = w < a.ow;
-        av[u] = wok ? gyr[(int64_t)w * a.cout] : 0.f;
-#pragma unroll
-        for (int t = 0; t < 7; ++t) {
-          const int kw = (tap0 + t) % 3;
-          const int iw = w + kw - a.pw;
-          const bool ok = wok && xr[t] != nullptr && (unsigned)iw < (unsigned)a.iw;
-          bv[u][t] = ok ? xr[t][(int64_t)w * a.cin] : 0.f;
-        }
+        const uint32_t at = (uint32_t)(xat + (2 * u + kw) * a.cin * 4);
+        o.x[u][t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, at < kOutside ? at : kOutside, 0, 0));
       }
-#pragma unroll
-      for (int u = 0; u < kPairsPerPass; ++u)
-#pragma unroll
-        for (int t = 0; t < 7; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[u], bv[u][t], acc[t], 0, 0, 0);
     }
+  };
+  auto compute = [&](const PassOperands& o) {
+#pragma unroll
+    for (int u = 0; u < kPairsPerPass; ++u)
+#pragma unroll
+      for (int t = 0; t < 7; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(o.gy[u], o.x[u][t], acc[t], 0, 0, 0);
+  };
+  PassOperands now, next;
+  int pass = p_begin + half;
+  if (pass < p_end) request(pass, now);
+  for (; pass < p_end; pass += 2) {
+    request(pass + 2 < p_end ? pass + 2 : pass, next);  // (behind the end the last pass once more, not used)
+    __builtin_amdgcn_sched_barrier(0);
+    compute(now);
+    __builtin_amdgcn_sched_barrier(0);
+    now = next;
   }
+
+  if (half == 1) {
+#pragma unroll
+    for (int t = 0; t < 7; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) meet[wave][t * 16 + r][lane] = acc[t][r];
+  }
+  __syncthreads();
+  if (half == 1) return;
   // result register r of a lane: column ci = lane % 32, row co = 8 * (r / 4) + 4 * kg + r % 4
   float* dst = partial + (int64_t)split * a.cout * kTaps * a.cin + ((int64_t)cob * 32 * kTaps) * a.cin + cib * 32 + i;
 #pragma unroll
@@ -283,7 +349,7 @@ wgrad_f32_kernel(WgradArgs a, const float* __restrict__ x, const float* __restri
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int co = 8 * (r / 4) + 4 * kg + (r % 4);
-      dst[((int64_t)co * kTaps + tap0 + t) * a.cin] = acc[t][r];
+      dst[((int64_t)co * kTaps + tap0 + t) * a.cin] = acc[t][r] + meet[wave][t * 16 + r][lane];
     }
   }
 }
@@ -321,13 +387,17 @@ int f32_conv(const MfmaConvArgs& a, const void* x, const void* packed, const voi
 namespace sfh {
 
 bool f32_wgrad_supported(const WgradArgs& a) {
+  // offsets inside a row and the count of passes are 32-bit
+  const int64_t reach = 4LL * (a.iw > a.ow ? a.iw : a.ow) + 64 + 4LL * a.pw;
+  if (reach * (a.cin > a.cout ? a.cin : a.cout) >= 0x7ffffff0LL) return false;
+  if ((int64_t)a.n * a.od * a.oh * ((a.ow + kPassVoxels - 1) / kPassVoxels) >= 0x7fffffffLL - 4) return false;
   return a.cin % 32 == 0 && a.cout % 32 == 0 && a.n >= 1 && a.od >= 1 && a.oh >= 1 && a.ow >= 1 && a.pd >= 0 && a.ph >= 0 && a.pw >= 0;
 }
 
 int f32_wgrad_splits(const WgradArgs& a) {
   const int64_t rows = (int64_t)a.n * a.od * a.oh;
   const int64_t blocks = (int64_t)(a.cout / 32) * (a.cin / 32);
-  int64_t s = 2 * kComputeUnits / blocks;  // two workgroups per CU
+  int64_t s = kComputeUnits / blocks;  // one workgroup of eight wavefronts per CU
   if (s < 1) s = 1;
   if (s > rows) s = rows;
   return (int)s;
@@ -342,9 +412,11 @@ int f32_wgrad(const WgradArgs& a, const void* x, const void* gy, void* gw, void*
   const int cibs = a.cin / 32, cobs = a.cout / 32;
   const int64_t total = (int64_t)nsplit * cibs * cobs;
   if (total > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv fp32 wgrad: too many workgroups");
-  hipLaunchKernelGGL(wgrad_f32_kernel, dim3((unsigned)total), dim3(256), 0, st, a, (const float*)x, (const float*)gy, (float*)workspace,
-                     nsplit, cibs);
+  // one slice is the gradient itself
+  hipLaunchKernelGGL(wgrad_f32_kernel, dim3((unsigned)total), dim3(512), 0, st, a, (const float*)x, (const float*)gy,
+                     (float*)(nsplit == 1 ? gw : workspace), nsplit, cibs);
   if (int rc = check_launch("wgrad_f32_kernel")) return rc;
+  if (nsplit == 1) return SFH_OK;
   return sum_slices(SFH_FP32, (const float*)workspace, gw, (int64_t)a.cout * kTaps * a.cin, nsplit, st);
 }
 
