@@ -324,6 +324,33 @@ struct LaunchNode : public Node {
 
 template <typename N> std::shared_ptr<N> new_node() { return {new N(), torch::autograd::deleteNode}; }
 
+// A tensor kept for the backward pass.  Saved-tensor hooks decide what comes back: save_on_cpu returns the values in the
+// default layout, whatever the layout was.  The kernels read plain pointers, so the layout they take is restored here, and
+// anything that is not the tensor that was kept (a hook that left it on the host, say) is refused.
+struct Kept {
+  SavedVariable saved;
+  c10::DimVector sizes;
+  at::ScalarType dtype = at::kFloat;
+  c10::Device device{c10::DeviceType::CPU};
+  void keep(const Tensor& t) {
+    saved = SavedVariable(t, false);
+    if (!t.defined()) return;
+    sizes.assign(t.sizes().begin(), t.sizes().end());
+    dtype = t.scalar_type();
+    device = t.device();
+  }
+  void reset() { saved.reset_data(); }
+  Tensor get() const {  // in any layout
+    const Tensor t = saved.unpack();
+    TORCH_CHECK(!t.defined() || (t.sizes() == c10::IntArrayRef(sizes) && t.scalar_type() == dtype && t.device() == device && t.layout() == at::kStrided),
+                "a saved tensor came back as ", t.sizes(), " ", t.scalar_type(), " on ", t.device(), "; it was ", c10::IntArrayRef(sizes), " ", dtype,
+                " on ", device);
+    return t;
+  }
+  Tensor volume() const { const Tensor t = get(); return t.defined() ? dense(t) : t; }
+  Tensor flat() const { const Tensor t = get(); return t.defined() ? t.contiguous() : t; }
+};
+
 bool wants_grad(std::initializer_list<const Tensor*> ts) {
   if (!at::GradMode::is_enabled()) return false;
   for (const Tensor* t : ts)
@@ -486,7 +513,7 @@ void queue_weight(QueuedWeight&& q) {
 // What the backward of a convolution over x, or over the pair (x, second), needs.  In the depth-shard form the tensors that
 // are saved are slabs of which x and second are the depth interiors.
 struct ConvSaved {
-  SavedVariable x, second, w, packed_dgrad;
+  Kept x, second, w, packed_dgrad;
   Tensor param;             // the parameter whose weight gradient waits for the end of the pass (undefined: computed here)
   int family = 0;
   bool early = false, pair = false, has_bias = false, master = false;
@@ -496,12 +523,12 @@ struct ConvSaved {
   std::vector<int64_t> in_sizes;
 
   void release() {
-    x.reset_data(); second.reset_data(); w.reset_data(); packed_dgrad.reset_data();
+    x.reset(); second.reset(); w.reset(); packed_dgrad.reset();
     param.reset();
   }
   // out: the gradients of x, weight, bias and second that are wanted (gy dense)
   void backward(const Tensor& gy, bool need_x, bool need_w, bool need_b, bool need_2, Tensor out[4]) {
-    const Tensor xs = x.unpack(), x2 = second.unpack(), wt = w.unpack(), packed = packed_dgrad.unpack();
+    const Tensor xs = x.volume(), x2 = second.volume(), wt = w.get(), packed = packed_dgrad.flat();
     Problem prob;
     TORCH_INTERNAL_ASSERT(make_problem(in_sizes, wt.sizes(), s, p, d, code_of(gy.scalar_type()), prob));
     if (need_x || need_2) {
@@ -553,9 +580,9 @@ struct ConvNode : public LaunchNode {  // edges: x, weight, bias, second
 
 void save_conv(ConvSaved& c, const Tensor& x, const Tensor& x_read, const Tensor& w, const Tensor& packed_dgrad, int64_t halo, bool master,
                const Tensor& param, int family, bool early) {
-  c.x = SavedVariable(x_read, false);
-  c.w = SavedVariable(w, false);
-  c.packed_dgrad = SavedVariable(packed_dgrad, false);
+  c.x.keep(x_read);
+  c.w.keep(w);
+  c.packed_dgrad.keep(packed_dgrad);
   c.halo = halo;
   c.depth = x.size(2);
   c.first_channels = x_read.size(1);
@@ -579,7 +606,7 @@ void record_conv(Tensor y, const Tensor& x, const Tensor& weight, const MaybeTen
   node->set_next_edges(torch::autograd::collect_next_edges(x, weight, b, x2));
   const Tensor read2 = or_none(second_read);
   save_conv(c, x, x_read, w, or_none(packed_dgrad), halo, master, family > 0 ? weight : Tensor(), family, early);
-  c.second = SavedVariable(read2, false);
+  c.second.keep(read2);
   c.pair = x2.defined();
   if (read2.defined()) c.in_sizes[1] += read2.size(1);
   c.has_bias = b.defined();
@@ -666,16 +693,16 @@ py::object pack_master(const Tensor& weight, at::ScalarType dtype, at::IntArrayR
 
 // ---- the 2x2x2-like transposed convolution (kernel == stride) ------------------------------------------------------------
 struct ConvTransposeNode : public LaunchNode {  // edges: x, weight, bias
-  SavedVariable x, w, packed_fwd;
+  Kept x, w, packed_fwd;
   int32_t k[3];
   bool has_bias = false, master = false;
   at::ScalarType bias_dtype = at::kFloat;
   std::string name() const override { return "ScaffoldConvTranspose3dBackward"; }
-  void release_variables() override { x.reset_data(); w.reset_data(); packed_fwd.reset_data(); }
+  void release_variables() override { x.reset(); w.reset(); packed_fwd.reset(); }
   variable_list backward(variable_list& grads) override {
     variable_list out(3);
     if (!grads[0].defined()) return out;
-    const Tensor xs = x.unpack(), wt = w.unpack(), packed = packed_fwd.unpack();
+    const Tensor xs = x.volume(), wt = w.get(), packed = packed_fwd.flat();
     const Tensor gy = dense(grads[0]);
     if (gy.numel() == 0) {
       const auto dtype = master ? at::kFloat : gy.scalar_type();
@@ -769,9 +796,9 @@ py::object conv_transpose(const Tensor& x_in, const Tensor& weight, const MaybeT
   if (graph) {
     auto node = new_node<ConvTransposeNode>();
     node->set_next_edges(torch::autograd::collect_next_edges(x_in, weight, weight_b));
-    node->x = SavedVariable(x, false);
-    node->w = SavedVariable(w, false);
-    node->packed_fwd = SavedVariable(or_none(packed_fwd), false);
+    node->x.keep(x);
+    node->w.keep(w);
+    node->packed_fwd.keep(or_none(packed_fwd));
     std::memcpy(node->k, k, sizeof(k));
     node->has_bias = weight_b.defined();
     if (weight_b.defined()) node->bias_dtype = weight_b.scalar_type();
@@ -785,18 +812,16 @@ py::object conv_transpose(const Tensor& x_in, const Tensor& weight, const MaybeT
 // ---- GroupNorm -----------------------------------------------------------------------------------------------------------
 // What the backward of GroupNorm (+ ReLU) needs.
 struct NormSaved {
-  SavedVariable input, weight, bias, stats;
+  Kept input, weight, bias, stats;
   int groups = 1;
   bool relu = false;
-  void release() { input.reset_data(); weight.reset_data(); bias.reset_data(); stats.reset_data(); }
+  void release() { input.reset(); weight.reset(); bias.reset(); stats.reset(); }
   void backward(const Tensor& grad, Tensor& dx, Tensor& dw, Tensor& db) {
-    const Tensor x = dense(input.unpack()), st = stats.unpack();
-    Tensor w = weight.unpack(), b = bias.unpack();
+    const Tensor x = input.volume(), st = stats.flat();
+    Tensor w = weight.flat(), b = bias.flat();
     Tensor gy = dense(grad);
     if (gy.scalar_type() != x.scalar_type() && gy.scalar_type() != at::kFloat) gy = gy.to(x.scalar_type());
     const Tensor w_in = w, b_in = b;
-    if (w.defined()) w = w.contiguous();
-    if (b.defined()) b = b.contiguous();
     if (w.defined() && b.defined() && w.scalar_type() != b.scalar_type()) b = b.to(w.scalar_type());
     c10::OptionalDeviceGuard guard(x.device());
     const int64_t c = x.size(1), n = x.size(0);
@@ -846,7 +871,7 @@ NormResult launch_norm(const Tensor& input, int64_t groups, const Tensor& weight
   const sfh_groupnorm_desc d{(int32_t)n, (int32_t)c, (int32_t)groups, relu ? 1 : 0, input.numel() / (n * c), (float)eps};
   void* st = stream_of(input);
   int64_t halo_rows = 0;
-  if (halo > 0 && n == 1 && c10::elementSize(odt) == input.element_size()) {
+  if (halo > 0 && n == 1 && (int64_t)c10::elementSize(odt) == (int64_t)input.element_size()) {
     r.slab = volume({1, c, input.size(2) + 2 * halo, input.size(3), input.size(4)}, input, odt);
     r.y = r.slab.narrow(2, halo, input.size(2));
     halo_rows = halo * input.size(3) * input.size(4);
@@ -875,10 +900,10 @@ NormResult launch_norm(const Tensor& input, int64_t groups, const Tensor& weight
 }
 
 void save_norm(NormSaved& s, const Tensor& input, const Tensor& weight, const Tensor& bias, const Tensor& stats, int64_t groups, bool relu) {
-  s.input = SavedVariable(input, false);
-  s.weight = SavedVariable(weight, false);
-  s.bias = SavedVariable(bias, false);
-  s.stats = SavedVariable(stats, false);
+  s.input.keep(input);
+  s.weight.keep(weight);
+  s.bias.keep(bias);
+  s.stats.keep(stats);
   s.groups = (int)groups;
   s.relu = relu;
 }
@@ -977,10 +1002,10 @@ py::object conv_norm(const Tensor& x, const Tensor& x_read, const Tensor& weight
 
 // ---- MaxPool3d(2) --------------------------------------------------------------------------------------------------------
 struct MaxPoolNode : public LaunchNode {  // edge: x; the second output, where there is one, is an alias of x (the skip connection)
-  SavedVariable idx;
+  Kept idx;
   std::vector<int64_t> sizes;
   std::string name() const override { return "ScaffoldMaxPool3dBackward"; }
-  void release_variables() override { idx.reset_data(); }
+  void release_variables() override { idx.reset(); }
   variable_list backward(variable_list& grads) override {
     variable_list out(1);
     const Tensor skip = grads.size() > 1 ? grads[1] : Tensor();
@@ -988,7 +1013,7 @@ struct MaxPoolNode : public LaunchNode {  // edge: x; the second output, where t
       out[0] = skip;
       return out;
     }
-    const Tensor gy = dense(grads[0]), ix = idx.unpack();
+    const Tensor gy = dense(grads[0]), ix = idx.flat();
     c10::OptionalDeviceGuard guard(gy.device());
     Tensor gx = volume(sizes, gy, gy.scalar_type());
     const sfh_pool_desc d{(int32_t)sizes[0], (int32_t)sizes[1], (int32_t)sizes[2], (int32_t)sizes[3], (int32_t)sizes[4]};
@@ -1039,7 +1064,7 @@ py::object max_pool(const Tensor& x_in, int64_t halo, bool with_skip) {
   if (graph) {
     auto node = new_node<MaxPoolNode>();
     node->set_next_edges(torch::autograd::collect_next_edges(x_in));
-    node->idx = SavedVariable(idx, false);
+    node->idx.keep(idx);
     node->sizes = z.vec();
     torch::autograd::set_history(y, node);
     if (with_skip) torch::autograd::set_history(skip, node);
@@ -1049,14 +1074,14 @@ py::object max_pool(const Tensor& x_in, int64_t halo, bool with_skip) {
 
 // ---- loss head -----------------------------------------------------------------------------------------------------------
 struct LossNode : public LaunchNode {  // edge: logits
-  SavedVariable logits, labels, stats, class_weight;
+  Kept logits, labels, stats, class_weight;
   sfh_loss_desc d{};
   std::string name() const override { return "ScaffoldCeDiceBackward"; }
-  void release_variables() override { logits.reset_data(); labels.reset_data(); stats.reset_data(); class_weight.reset_data(); }
+  void release_variables() override { logits.reset(); labels.reset(); stats.reset(); class_weight.reset(); }
   variable_list backward(variable_list& grads) override {
     variable_list out(1);
     if (!grads[0].defined()) return out;
-    const Tensor x = logits.unpack(), lab = labels.unpack(), st = stats.unpack(), cw = class_weight.unpack();
+    const Tensor x = logits.volume(), lab = labels.flat(), st = stats.flat(), cw = class_weight.flat();
     c10::OptionalDeviceGuard guard(x.device());
     const Tensor g = grads[0].to(x.device(), at::kFloat).reshape({1}).contiguous();
     Tensor dx = volume(x.sizes(), x, x.scalar_type());
@@ -1096,10 +1121,10 @@ py::object ce_dice_loss(const Tensor& logits, const Tensor& labels, const MaybeT
   if (graph) {
     auto node = new_node<LossNode>();
     node->set_next_edges(torch::autograd::collect_next_edges(logits));
-    node->logits = SavedVariable(x, false);
-    node->labels = SavedVariable(lab, false);
-    node->stats = SavedVariable(stats, false);
-    node->class_weight = SavedVariable(cw, false);
+    node->logits.keep(x);
+    node->labels.keep(lab);
+    node->stats.keep(stats);
+    node->class_weight.keep(cw);
     node->d = d;
     torch::autograd::set_history(loss, node);
   }
