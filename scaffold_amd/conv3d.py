@@ -457,6 +457,8 @@ def _pack_plan(w, in_shape, stride, padding, dilation):
     if plan is None:
         s, p, d = _triple(stride, "stride"), _triple(padding, "padding"), _triple(dilation, "dilation")
         nbf, nbd = packed_weight_bytes(in_shape, w.shape, s, p, d, w.dtype)
+        if (nbf or nbd) and int(in_shape[1]) != int(w.shape[1]):  # packing walks the input's channels
+            raise ValueError(f"pack_weights: a weight of shape {tuple(w.shape)} does not belong to an input of shape {tuple(in_shape)}")
         n, cin, *in_sp = (int(v) for v in in_shape)
         k = tuple(int(v) for v in w.shape[2:])
         plan = (nbf, nbd, _desc(n, cin, in_sp, int(w.shape[0]), k, s, p, d), _lib.dtype_code(w.dtype) if (nbf or nbd) else -1)

@@ -675,13 +675,14 @@ py::object conv_backward_weight(const Tensor& x, at::IntArrayRef w_sizes, const 
 
 // The packed forms of an fp32 master weight for a 16-bit convolution of an input of `in_sizes`, in one launch:
 // (packed_fwd, packed_dgrad, complete).  A form is None when that direction does not read one or (data gradient) was not
-// asked for; `complete`: every direction asked for has its form, so nobody reads the weight itself.
+// asked for; `complete`: every direction asked for has its form, so nobody reads the weight itself.  Nothing is packed for
+// an input whose channels are not the weight's.
 py::object pack_master(const Tensor& weight, at::ScalarType dtype, at::IntArrayRef in_sizes, py::handle stride, py::handle padding, py::handle dilation,
                        bool want_dgrad) {
   int32_t s[3], p[3], d[3];
   Problem prob;
   if (!three(stride, s) || !three(padding, p) || !three(dilation, d) || weight.scalar_type() != at::kFloat || !on_gpu(weight) ||
-      !make_problem(in_sizes, weight.sizes(), s, p, d, code_of(dtype), prob))
+      weight.dim() != 5 || in_sizes.size() != 5 || in_sizes[1] != weight.size(1) || !make_problem(in_sizes, weight.sizes(), s, p, d, code_of(dtype), prob))
     return py::make_tuple(py::none(), py::none(), false);
   c10::OptionalDeviceGuard guard(weight.device());
   const Tensor pf = bytes(prob.sizes->packed[0], weight), pd = want_dgrad ? bytes(prob.sizes->packed[1], weight) : Tensor();

@@ -350,7 +350,10 @@ class FastConv3d(nn.Conv3d):
     def _kernel_operands(self, weight, bias, dt, x_dtype, in_shape, stride, padding, dilation, want_dgrad):
         """``(w, b, packs, master, complete)``: what the kernels read of the parameters (``packs``: the packed forms that are
         current, or None), whether the parameters are fp32 masters whose gradients are produced in fp32 directly, and whether
-        the packed forms are all that is read (``w`` is then the master itself)."""
+        the packed forms are all that is read (``w`` is then the master itself).  The caller has not passed its gate yet: a
+        weight that does not belong to an input of this shape is not packed (packing walks the input's channels)."""
+        if len(in_shape) != 5 or in_shape[1] != weight.shape[1] or self.groups != 1:
+            return cast_operand(weight, dt), cast_operand(bias, dt), None, False, False
         # under autocast, up-to-date half-precision copies kept by the optimizer, with their packed forms
         wc = compute_copy(weight, dt)
         if wc is not None:
@@ -358,7 +361,7 @@ class FastConv3d(nn.Conv3d):
             if bias is None or bc is not None:
                 packs = _current_packs(weight, wc, in_shape, stride, padding, dilation)
                 return wc, bc, None if packs is None else (packs.fwd, packs.dgrad), True, False
-        if _narrowed(weight, bias, dt, x_dtype) and self.groups == 1:
+        if _narrowed(weight, bias, dt, x_dtype):
             w, b, packs, complete = _master_operands(weight, bias, dt, in_shape, stride, padding, dilation, want_dgrad)
             return w, b, packs, True, complete
         w, b = cast_operand(weight, dt), cast_operand(bias, dt)
