@@ -606,7 +606,7 @@ def conv3d_forward(
     """
     if config is None and weight_rsck is None and out is None and not (weight_flip or force_generic) and groups == 1 \
             and _tensors(x, w) and _tensors_or_none(bias, packed_weight):
-        done = _lib.native().conv_forward(x, w, bias, stride, padding, dilation, packed_weight, int(gn_groups), _second)
+        done = _lib.native().conv_forward(x, w, bias, stride, padding, dilation, packed_weight, int(gn_groups), _second, _checked)
         if done is not None:
             y, partials, records = done
             if partials is not None:

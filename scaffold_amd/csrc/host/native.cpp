@@ -188,11 +188,13 @@ bool bias_fits(const MaybeTensor& b, const Tensor& x, int64_t channels) {
                             b->stride(0) == 1);
 }
 
-// The gate of the forward (conv3d.is_supported), and with `all` of both gradients too (is_supported_all).
+// The gate of the forward (conv3d.is_supported), and with `all` of both gradients too (is_supported_all).  `packed`: the
+// caller has made packed forms of x's dtype from w, so an fp32 master may stand in w's place (nothing else may: packed forms
+// of bf16 and fp16 weights have the same size).
 bool conv_gate(const Tensor& x, const Tensor& w, const MaybeTensor& bias, const int32_t s[3], const int32_t p[3], const int32_t d[3],
                bool all, Problem& prob, int64_t more_channels = 0, bool packed = false) {
   if (x.dim() != 5 || w.dim() != 5 || !on_gpu(x) || !on_gpu(w) || x.device() != w.device()) return false;
-  if ((x.scalar_type() != w.scalar_type() && !packed) || x.size(1) + more_channels != w.size(1)) return false;
+  if ((x.scalar_type() != w.scalar_type() && !(packed && w.scalar_type() == at::kFloat)) || x.size(1) + more_channels != w.size(1)) return false;
   if (!bias_fits(bias, x, w.size(0))) return false;
   const int64_t in[5] = {x.size(0), w.size(1), x.size(2), x.size(3), x.size(4)};
   if (!make_problem(in, w.sizes(), s, p, d, code_of(x.scalar_type()), prob)) return false;
@@ -617,12 +619,13 @@ void record_conv(Tensor y, const Tensor& x, const Tensor& weight, const MaybeTen
 py::object tensor_or_none(const Tensor& t) { return t.defined() ? py::cast(t) : py::none(); }
 
 // conv3d.conv3d_forward / conv3d_forward_pair: (y, partials, records), or None for a call that is not served as it stands.
+// `master`: w may be the fp32 master that `packed` was made from.
 py::object conv_forward(const Tensor& x, const Tensor& w, const MaybeTensor& bias, py::handle stride, py::handle padding, py::handle dilation,
-                        const MaybeTensor& packed, int gn_groups, const MaybeTensor& second) {
+                        const MaybeTensor& packed, int gn_groups, const MaybeTensor& second, bool master) {
   int32_t s[3], p[3], d[3];
   if (!three(stride, s) || !three(padding, p) || !three(dilation, d)) return py::none();
   Problem prob;
-  if (!conv_gate(x, w, bias, s, p, d, false, prob, second.has_value() && second->dim() == 5 ? second->size(1) : 0, packed.has_value())) return py::none();
+  if (!conv_gate(x, w, bias, s, p, d, false, prob, second.has_value() && second->dim() == 5 ? second->size(1) : 0, master && packed.has_value())) return py::none();
   if (packed.has_value() && !packed_fits(*packed, prob.sizes->packed[0], x)) return py::none();
   if (second.has_value() && (second->dim() != 5 || !on_gpu(*second) || second->device() != x.device() || second->scalar_type() != x.scalar_type() ||
                              second->size(0) != x.size(0) || second->size(2) != x.size(2) || second->size(3) != x.size(3) || second->size(4) != x.size(4)))
@@ -749,7 +752,8 @@ py::object conv_transpose(const Tensor& x_in, const Tensor& weight, const MaybeT
                           const MaybeTensor& packed_fwd, const MaybeTensor& packed_dgrad, int64_t halo, bool master) {
   int32_t k[3];
   if (!three(stride, k) || x_in.dim() != 5 || w.dim() != 5 || !on_gpu(x_in) || !on_gpu(w) || x_in.device() != w.device()) return py::none();
-  const bool all_packed = packed_fwd.has_value() && packed_dgrad.has_value();  // the weight itself is then not read
+  // an fp32 master that nobody reads: both packed forms were made from it in x's dtype
+  const bool all_packed = master && w.scalar_type() == at::kFloat && packed_fwd.has_value() && packed_dgrad.has_value();
   if ((x_in.scalar_type() != w.scalar_type() && !all_packed) || x_in.size(1) != w.size(0) || !bias_fits(b, x_in, w.size(1))) return py::none();
   int64_t big[5] = {x_in.size(0), w.size(1), 0, 0, 0};
   for (int i = 0; i < 3; ++i) {
@@ -976,7 +980,7 @@ py::object conv_norm(const Tensor& x, const Tensor& x_read, const Tensor& weight
   if (!three(stride, s) || !three(padding, p) || !three(dilation, d) || !x_read.is_contiguous(kCL3D)) return py::none();
   const bool graph = wants_grad({&x, &weight, &norm_weight, &norm_bias});
   Problem prob;
-  if (!conv_gate(x_read, w, std::nullopt, s, p, d, graph, prob, 0, packed_fwd.has_value())) return py::none();
+  if (!conv_gate(x_read, w, std::nullopt, s, p, d, graph, prob, 0, master && packed_fwd.has_value())) return py::none();
   if (packed_fwd.has_value() && !packed_fits(*packed_fwd, prob.sizes->packed[0], x_read)) return py::none();
   if (packed_dgrad.has_value() && !packed_fits(*packed_dgrad, prob.sizes->packed[1], x_read)) return py::none();
   if (!norm_gate(x_read, prob.key.d.n, prob.key.d.cout, (int64_t)prob.out[0] * prob.out[1] * prob.out[2], groups, norm_weight, norm_bias)) return py::none();

@@ -54,3 +54,27 @@ def test_packing_refuses_a_weight_of_another_input(device):
     assert _lib.native().pack_master(w, torch.bfloat16, (1, 64, 4, 8, 32), 1, 1, 1, True) == (None, None, False)
     with pytest.raises(ValueError, match="does not belong"):
         sa.pack_weights(w.to(torch.bfloat16), (1, 64, 4, 8, 32), 1, 1, 1)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "shadows"])
+def test_two_16_bit_types_do_not_meet_over_a_packed_weight(device, kind):
+    """Packed forms of a bf16 and of an fp16 weight have the same size: the weight's own dtype decides."""
+    x = _x(device, 32, torch.float16)
+    stages = [sa.FastConv3d(32, 32, 3, padding=1, bias=False), DoubleConv(32, 32, 8), sa.FastConvTranspose3d(32, 32, 2, stride=2, bias=False)]
+    for module in stages:
+        module = _weights(module, device, kind)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=kind != "bf16"):
+            module(x.to(torch.bfloat16))            # the packed forms exist
+            for grad in (True, False):
+                with torch.set_grad_enabled(grad), pytest.raises(NotImplementedError):
+                    module(x)
+
+
+def test_an_operators_packed_weight_does_not_lift_the_dtype_rule(device):
+    w = torch.randn(32, 32, 3, 3, 3, device=device).to(torch.bfloat16)
+    x = _x(device, 32)
+    pf, pd = sa.pack_weights(w, x.shape, 1, 1, 1)
+    assert torch.equal(sa.conv3d_forward(x, w, None, 1, 1, packed_weight=pf), sa.conv3d_forward(x, w, None, 1, 1))
+    for a, b in ((x.to(torch.float16), w), (x, w.to(torch.float16)), (x, w.float())):
+        with pytest.raises(NotImplementedError):
+            sa.conv3d_forward(a, b, None, 1, 1, packed_weight=pf)
