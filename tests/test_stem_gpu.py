@@ -76,3 +76,30 @@ def test_stem_weight_gradient_in_fp32_rounds_to_the_16_bit_one(device):
     g16 = sa.conv3d_backward_weight(x, (64, 3, 3, 3, 3), gy, 1, 1)
     g32 = sa.conv3d_backward_weight(x, (64, 3, 3, 3, 3), gy, 1, 1, grad_dtype=torch.float32)
     assert g32.dtype is torch.float32 and torch.equal(g32.to(torch.bfloat16), g16)
+
+
+@pytest.mark.parametrize("cin", [1, 3])
+@pytest.mark.parametrize("spatial,padding", [((3, 6, 40), (1, 1, 1)), ((2, 4, 33), (1, 1, 1)), ((5, 7, 17), (0, 1, 1)), ((3, 5, 66), (2, 0, 0)),
+                                             ((4, 4, 47), (1, 2, 2))])
+def test_stem_weight_gradient_keeps_nan_and_inf_to_their_taps(device, cin, spatial, padding):
+    """A tile reaches past the output: a voxel there has no gradient, and an infinity that only its taps would meet (0 x
+    infinity) stays out.  One infinity or NaN at a corner or edge of the input: exactly the taps that some output reads it
+    through are not finite, the others are the sums without it."""
+    shape = (32, cin, 3, 3, 3)
+    g = torch.Generator().manual_seed(13)
+    x = torch.randint(-2, 3, (1, cin, *spatial), generator=g).to(torch.bfloat16)
+    out = [s + 2 * p - 2 for s, p in zip(spatial, padding)]
+    gy = torch.randint(-1, 2, (1, 32, *out), generator=g).to(torch.bfloat16)
+    gy[gy == 0] = 2
+    d, h, w = (s - 1 for s in spatial)
+    for at, value in (((d, h, w), "inf"), ((0, 0, w), "nan"), ((d, 0, 0), "inf"), ((d // 2, h, w), "inf"), ((0, h, w // 2), "nan")):
+        clean, dirty = x.clone(), x.clone()
+        clean[(0, cin - 1, *at)], dirty[(0, cin - 1, *at)] = 0, float(value)
+        want = torch.nn.grad.conv3d_weight(clean.double(), shape, gy.double(), 1, padding)
+        met = torch.zeros(cin, 3, 3, 3, dtype=torch.bool)
+        for tap in torch.cartesian_prod(*[torch.arange(3)] * 3).tolist():
+            met[(cin - 1, *tap)] = all(0 <= a + p - t < o for a, p, t, o in zip(at, padding, tap, out))
+        got = sa.conv3d_backward_weight(dirty.to(device).contiguous(memory_format=CL), shape, gy.to(device).contiguous(memory_format=CL), 1,
+                                        padding, grad_dtype=torch.float32).cpu()
+        assert torch.equal(~torch.isfinite(got), met.expand(32, -1, -1, -1, -1)), (at, value)
+        assert torch.equal(got[:, ~met].double(), want[:, ~met])
