@@ -515,7 +515,8 @@ void queue_weight(QueuedWeight&& q) {
 // What the backward of a convolution over x, or over the pair (x, second), needs.  In the depth-shard form the tensors that
 // are saved are slabs of which x and second are the depth interiors.
 struct ConvSaved {
-  Kept x, second, w, packed_dgrad;
+  Kept x, second, w, packed_dgrad;  // w undefined: an fp32 master of which only the packed forms are read
+  c10::DimVector w_sizes;
   Tensor param;             // the parameter whose weight gradient waits for the end of the pass (undefined: computed here)
   int family = 0;
   bool early = false, pair = false, has_bias = false, master = false;
@@ -532,7 +533,7 @@ struct ConvSaved {
   void backward(const Tensor& gy, bool need_x, bool need_w, bool need_b, bool need_2, Tensor out[4]) {
     const Tensor xs = x.volume(), x2 = second.volume(), wt = w.get(), packed = packed_dgrad.flat();
     Problem prob;
-    TORCH_INTERNAL_ASSERT(make_problem(in_sizes, wt.sizes(), s, p, d, code_of(gy.scalar_type()), prob));
+    TORCH_INTERNAL_ASSERT(make_problem(in_sizes, w_sizes, s, p, d, code_of(gy.scalar_type()), prob));
     if (need_x || need_2) {
       auto gx = launch_dgrad(prob, gy, wt, packed, pair ? first_channels : 0);
       if (halo > 0) {
@@ -580,10 +581,15 @@ struct ConvNode : public LaunchNode {  // edges: x, weight, bias, second
   }
 };
 
+// The weight a node keeps: one that was packed from an fp32 master is not read again, and a program may step the master
+// between forward and backward, as it may where autocast has cast it.
+Tensor unless_packed_master(const Tensor& w, const Tensor& x) { return w.scalar_type() == x.scalar_type() ? w : Tensor(); }
+
 void save_conv(ConvSaved& c, const Tensor& x, const Tensor& x_read, const Tensor& w, const Tensor& packed_dgrad, int64_t halo, bool master,
                const Tensor& param, int family, bool early) {
   c.x.keep(x_read);
-  c.w.keep(w);
+  c.w.keep(unless_packed_master(w, x_read));
+  c.w_sizes.assign(w.sizes().begin(), w.sizes().end());
   c.packed_dgrad.keep(packed_dgrad);
   c.halo = halo;
   c.depth = x.size(2);
@@ -697,7 +703,8 @@ py::object pack_master(const Tensor& weight, at::ScalarType dtype, at::IntArrayR
 
 // ---- the 2x2x2-like transposed convolution (kernel == stride) ------------------------------------------------------------
 struct ConvTransposeNode : public LaunchNode {  // edges: x, weight, bias
-  Kept x, w, packed_fwd;
+  Kept x, w, packed_fwd;  // w as in ConvSaved
+  c10::DimVector w_sizes;
   int32_t k[3];
   bool has_bias = false, master = false;
   at::ScalarType bias_dtype = at::kFloat;
@@ -711,24 +718,24 @@ struct ConvTransposeNode : public LaunchNode {  // edges: x, weight, bias
     if (gy.numel() == 0) {
       const auto dtype = master ? at::kFloat : gy.scalar_type();
       out[0] = volume(xs.sizes(), gy, gy.scalar_type());
-      out[1] = volume(wt.sizes(), gy, dtype).zero_();
-      if (has_bias) out[2] = at::zeros({wt.size(1)}, gy.options().dtype(bias_dtype));
+      out[1] = volume(w_sizes, gy, dtype).zero_();
+      if (has_bias) out[2] = at::zeros({w_sizes[1]}, gy.options().dtype(bias_dtype));
       return out;
     }
     // the stride-k convolution over gy whose forward is the data gradient and whose weight gradient is this one's
     const int32_t zero[3] = {0, 0, 0}, one[3] = {1, 1, 1};
     Problem prob;
-    TORCH_INTERNAL_ASSERT(make_problem(gy.sizes(), wt.sizes(), k, zero, one, code_of(gy.scalar_type()), prob));
+    TORCH_INTERNAL_ASSERT(make_problem(gy.sizes(), w_sizes, k, zero, one, code_of(gy.scalar_type()), prob));
     const bool need_w = task_should_compute_output(1), need_b = has_bias && task_should_compute_output(2);
     if (task_should_compute_output(0)) out[0] = launch_conv(prob, gy, Tensor(), wt, Tensor(), packed, 0).y;
     if (need_w && need_b) {
       c10::OptionalDeviceGuard guard(gy.device());
       const sfh_convT3d_desc td{(int32_t)xs.size(0), (int32_t)xs.size(1), (int32_t)xs.size(2), (int32_t)xs.size(3), (int32_t)xs.size(4),
-                                (int32_t)wt.size(1), k[0], k[1], k[2]};
+                                (int32_t)w_sizes[1], k[0], k[1], k[2]};
       const size_t need = sfh_convT3d_wgrad_bias_workspace_bytes(&td, prob.key.code);
       if (need > 0) {
         const auto dtype = master ? at::kFloat : gy.scalar_type();
-        Tensor gw = volume(wt.sizes(), gy, dtype), gb = plain({wt.size(1)}, gy, dtype);
+        Tensor gw = volume(w_sizes, gy, dtype), gb = plain({w_sizes[1]}, gy, dtype);
         const Tensor ws = bytes(need, gy);
         const int rc = sfh_convT3d_wgrad_bias(&td, prob.key.code, ptr(xs), ptr(gy), out_ptr(gw), out_ptr(gb), out_ptr(ws), need,
                                               dtype != gy.scalar_type() ? SFH_FLAG_GRAD_FP32 : 0, stream_of(gy));
@@ -802,7 +809,8 @@ py::object conv_transpose(const Tensor& x_in, const Tensor& weight, const MaybeT
     auto node = new_node<ConvTransposeNode>();
     node->set_next_edges(torch::autograd::collect_next_edges(x_in, weight, weight_b));
     node->x.keep(x);
-    node->w.keep(w);
+    node->w.keep(unless_packed_master(w, x));
+    node->w_sizes.assign(w.sizes().begin(), w.sizes().end());
     node->packed_fwd.keep(or_none(packed_fwd));
     std::memcpy(node->k, k, sizeof(k));
     node->has_bias = weight_b.defined();

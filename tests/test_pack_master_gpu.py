@@ -55,3 +55,28 @@ def test_autocast_modules_without_an_optimizers_copies(device):
             assert p.grad.dtype is torch.float32 and torch.equal(p.grad.to(torch.bfloat16), q.grad)
         with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
             assert torch.equal(m(x), y.detach())
+
+
+def test_a_master_may_step_between_forward_and_backward(device):
+    """As where autocast has cast the weight: the gradients are those of the weight the forward read."""
+    from scaffold_amd.modules import conv_then_norm
+
+    torch.manual_seed(6)
+    norm = sa.FastGroupNorm(8, 32, activation="relu").to(device)
+    conv = sa.FastConv3d(32, 32, 3, padding=1, bias=False)
+    pair = sa.FastConv3d(64, 32, 3, padding=1, bias=False)
+    x = torch.randn(1, 32, 4, 8, 32, device=device).to(torch.bfloat16).contiguous(memory_format=CL)
+    for module, call in ((conv, conv), (conv, lambda t: conv_then_norm(conv, norm, t)), (pair, lambda t: pair(t, x)),
+                         (sa.FastConv3d(32, 6, 1), None), (sa.FastConvTranspose3d(32, 32, 2, stride=2), None)):
+        module.to(device).to(memory_format=CL)
+        runs = []
+        for step in (False, True):
+            a = x.clone().requires_grad_()
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                y = (call or module)(a)
+            if step:
+                with torch.no_grad():
+                    for p in module.parameters():
+                        p.mul_(2)
+            runs.append(torch.autograd.grad(y, (a, *module.parameters()), torch.ones_like(y)))
+        assert all(torch.equal(p, q) for p, q in zip(*runs))
