@@ -40,7 +40,7 @@ using MaybeTensor = std::optional<Tensor>;
 // ---- the Python side -----------------------------------------------------------------------------------------------------
 PyObject* g_kernel_error = nullptr;    // scaffold_amd._lib.ScaffoldKernelError
 PyObject* g_note_device = nullptr;     // scaffold_amd._lib._note_device(device)
-PyObject* g_send_early = nullptr;      // scaffold_amd.modules._send_early_batch(batch)
+PyObject* g_send_early = nullptr;      // scaffold_amd.modules._send_early(batch)
 PyObject* g_join_early = nullptr;      // scaffold_amd.modules._join_early(batch)
 
 // A status code as the exception the entry points raise (the interpreter lock is taken if this thread does not hold it).
@@ -366,7 +366,8 @@ Tensor or_none(const MaybeTensor& t) { return t.has_value() ? *t : Tensor(); }
 // See scaffold_amd/modules.py: a convolution whose module defers leaves (parameter, operands) here instead of computing its
 // weight gradient; when the pass ends -- still inside backward() -- all that the pass queued are computed by one batched
 // call and added to the parameters' .grad.  The queue is kept per backward pass (graph task), so passes that run at the
-// same time on other threads or streams never take each other's entries.
+// same time on other threads or streams never take each other's entries, and it ends with its pass: what a pass that
+// raised has queued is dropped with it.
 struct QueuedWeight {
   Tensor param, x, second, gy;
   int32_t p[3];
@@ -436,21 +437,28 @@ void add_to_grads(WeightBatch& batch) {
   }
 }
 
-// Computes what a pass has queued and adds it (no entry: nothing to do).
-void finish_pass(int id) {
+PassQueue take_pass(int id) {
+  std::lock_guard<std::mutex> hold(g_pass_lock);
   PassQueue pass;
-  {
-    std::lock_guard<std::mutex> hold(g_pass_lock);
-    auto it = g_passes.find(id);
-    if (it == g_passes.end()) return;
+  auto it = g_passes.find(id);
+  if (it != g_passes.end()) {
     pass = std::move(it->second);
     g_passes.erase(it);
   }
+  return pass;
+}
+
+void join_sent(const PassQueue& pass) {
+  if (pass.sent.empty()) return;
+  py::gil_scoped_acquire gil;
+  for (const auto& batch : pass.sent) py::reinterpret_borrow<py::function>(g_join_early)(batch);
+}
+
+// Computes what a pass has queued and adds it (no entry: nothing to do).
+void finish_pass(int id) {
+  PassQueue pass = take_pass(id);
   at::AutoGradMode no_grad(false);
-  if (!pass.sent.empty()) {
-    py::gil_scoped_acquire gil;
-    for (auto& batch : pass.sent) py::reinterpret_borrow<py::function>(g_join_early)(batch);
-  }
+  join_sent(pass);
   for (auto& batch : pass.sent) add_to_grads(*batch);
   while (!pass.items.empty()) {
     WeightBatch batch;
@@ -466,13 +474,32 @@ void finish_pass(int id) {
   }
 }
 
-void finish_all_passes() {
-  std::vector<int> ids;
-  {
-    std::lock_guard<std::mutex> hold(g_pass_lock);
-    for (const auto& kv : g_passes) ids.push_back(kv.first);
+// Lives as long as the pass whose final callback holds it.  A pass that raises runs no callback: its entry is dropped here,
+// after the launches already sent to a side stream have been joined (they read the operands that are let go).
+struct PassEnd {
+  const int id;
+  explicit PassEnd(int pass) : id(pass) {}
+  PassEnd(const PassEnd&) = delete;
+  ~PassEnd() {
+    try {
+      join_sent(take_pass(id));
+    } catch (const std::exception& e) {
+      TORCH_WARN("weight gradients of a backward pass that raised: ", e.what());
+    }
   }
-  for (int id : ids) finish_pass(id);
+};
+
+// What the pass this thread is in has queued so far (outside of a pass nothing waits).
+void finish_current_pass() { finish_pass(torch::autograd::get_current_graph_task_id()); }
+
+size_t waiting_weight_gradients() {
+  std::lock_guard<std::mutex> hold(g_pass_lock);
+  size_t n = 0;
+  for (const auto& kv : g_passes) {
+    n += kv.second.items.size();
+    for (const auto& batch : kv.second.sent) n += batch->size();
+  }
+  return n;
 }
 
 void queue_weight(QueuedWeight&& q) {
@@ -482,7 +509,7 @@ void queue_weight(QueuedWeight&& q) {
     std::lock_guard<std::mutex> hold(g_pass_lock);
     auto found = g_passes.find(id);
     if (found == g_passes.end()) {
-      torch::autograd::Engine::get_default_engine().queue_callback([id] { finish_pass(id); });
+      torch::autograd::Engine::get_default_engine().queue_callback([end = std::make_shared<PassEnd>(id)] { finish_pass(end->id); });
       found = g_passes.emplace(id, PassQueue{}).first;
     }
     auto& items = found->second.items;
@@ -1161,7 +1188,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   py::class_<WeightBatch, std::shared_ptr<WeightBatch>>(m, "WeightBatch").def("__len__", &WeightBatch::size);
   m.def("launch_batch", [](WeightBatch& batch, bool share_device) { launch_batch(batch, share_device); });
   m.def("batch_device", [](const WeightBatch& batch) { return batch.items.at(0).gy.device(); });
-  m.def("finish_all_passes", &finish_all_passes);
+  m.def("finish_current_pass", &finish_current_pass);
+  m.def("waiting_weight_gradients", &waiting_weight_gradients);
   m.def("conv_forward", &conv_forward);
   m.def("conv_supported", &conv_supported);
   m.def("pack_master", &pack_master);

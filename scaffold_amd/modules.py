@@ -112,16 +112,7 @@ def _current_packs(owner: torch.Tensor, source: torch.Tensor, in_shape, stride, 
 # when the backward pass has finished -- still inside ``backward()`` -- computes all queued gradients in one batched call and
 # adds them to the parameters' ``.grad``.  After ``backward()`` returns the gradients are where they always are.  What
 # differs: hooks on the parameter's gradient accumulation do not see these gradients, and the operands stay alive until
-# the end of the pass.
-class _QueuedWeightGrad:
-    __slots__ = ("param", "inp", "wshape", "gy", "padding", "grad_dtype")
-
-    def __init__(self, param, inp, wshape, gy, padding, grad_dtype):
-        self.param, self.inp, self.wshape, self.gy, self.padding, self.grad_dtype = param, inp, wshape, gy, padding, grad_dtype
-
-
-#: weight gradients queued by hand, for ``flush_weight_gradients()`` (a backward pass keeps its own queue)
-_WEIGHT_GRAD_QUEUE: list = []
+# the end of the pass.  A pass that raises drops what it has queued.
 _BATCHABLE: dict = {}
 
 #: A weight gradient of more operations than this is computed in its own node although the module defers.  What a place
@@ -179,25 +170,10 @@ def _join_early(batch) -> None:
 
 
 def flush_weight_gradients() -> None:
-    """Compute the weight gradients that wait -- left by a pass that raised, or queued by hand -- and add them to their
-    parameters' ``.grad`` (a pass that ends does this by itself)."""
-    _lib.native().finish_all_passes()
-    queue = list(_WEIGHT_GRAD_QUEUE)
-    _WEIGHT_GRAD_QUEUE.clear()
-    groups: dict = {}
-    for it in queue:
-        groups.setdefault((it.gy.device, it.gy.dtype, it.grad_dtype), []).append(it)
-    with torch.no_grad():
-        for (_, dt, gdt), items in groups.items():
-            grads = _c3.conv3d_backward_weight_batch([(it.inp, it.wshape, it.gy, it.padding) for it in items],
-                                                     grad_dtype=None if gdt is dt else gdt)
-            for it, gw in zip(items, grads):
-                p = it.param
-                if p.grad is None:
-                    # in the parameter's own layout, as the engine's accumulation would leave it
-                    p.grad = gw if gw.stride() == p.stride() else torch.empty_like(p).copy_(gw)
-                else:
-                    p.grad.add_(gw)
+    """Compute the weight gradients that the backward pass this is called from (by a hook, say) has queued so far and add them
+    to their parameters' ``.grad``.  A pass that ends does this by itself, and one that raises drops what it has queued:
+    outside of a pass nothing waits."""
+    _lib.native().finish_current_pass()
 
 
 _early_callbacks_set = False

@@ -11,6 +11,8 @@ summation-order rounding, the same bits on every run and for every list with the
 launch -- of a list with a problem the batch does not serve.
 """
 
+import gc
+
 import pytest
 import torch
 
@@ -148,6 +150,10 @@ def test_what_is_refused(device):
     assert L.sfh_conv3d_wgrad_batch(items, 2, code, _lib.ptr(ws), need, 0, stream) == _lib.SFH_ERR_UNSUPPORTED
 
 
+def _waiting() -> int:
+    return _lib.native().waiting_weight_gradients()
+
+
 def _tiny_net(device, defer, layers=2):
     torch.manual_seed(7)
     net = sa.UNet(1, 3, layers=layers, base_width=32).to(device).to(memory_format=CL).set_shard_halo(True)
@@ -179,7 +185,7 @@ def test_backward_pass_with_deferred_weight_gradients(device, master):
             else:
                 logits = net(x.to(torch.bfloat16))
             sa.ce_dice_loss(logits, target).backward()
-            assert not modules._WEIGHT_GRAD_QUEUE
+            assert not _waiting()
             if rep == 0:
                 grads[defer, 0] = {n: p.grad.detach().clone() for n, p in net.named_parameters()}
         grads[defer, 1] = {n: p.grad.detach().clone() for n, p in net.named_parameters()}
@@ -202,25 +208,86 @@ def test_backward_pass_with_deferred_weight_gradients(device, master):
         assert (g.float() - 2 * first).abs().max().item() <= 2.0 ** -6 * max(first.abs().max().item(), 1e-30), n
 
 
-def test_flush_by_hand_and_unbatchable_weights_are_computed_in_place(device):
+def test_unbatchable_weights_are_computed_in_place(device):
     """A convolution the batch does not serve (rows of 16 voxels, 160 tiles) computes its gradient in its own node although
-    the flag is set; a queue left by a pass that raised is emptied by ``flush_weight_gradients()``."""
+    the flag is set."""
     torch.manual_seed(1)
     conv = sa.FastConv3d(32, 32, 3, padding=1, bias=False).to(device).to(torch.bfloat16).to(memory_format=CL)
     conv.defer_weight_grad = True
     x = torch.randn(1, 32, 40, 64, 16, device=device, dtype=torch.bfloat16).contiguous(memory_format=CL).requires_grad_()
     conv(x).sum().backward()
-    assert conv.weight.grad is not None and not modules._WEIGHT_GRAD_QUEUE
+    assert conv.weight.grad is not None and not _waiting()
     ref = sa.conv3d_backward_weight(x.detach(), conv.weight.shape, torch.ones(1, 32, 40, 64, 16, device=device, dtype=torch.bfloat16), 1, 1, 1)
     assert torch.equal(conv.weight.grad, ref)
-    # a queued entry that no callback took: flush by hand
-    conv.weight.grad = None
-    x2 = torch.randn(1, 32, 4, 8, 32, device=device, dtype=torch.bfloat16).contiguous(memory_format=CL)
+
+
+def test_flush_by_hand_inside_a_pass(device):
+    """A hook that runs after a deferring convolution's node finds its gradient waiting; ``flush_weight_gradients()`` computes it
+    there and then, and the end of the pass adds nothing to it."""
+    torch.manual_seed(1)
+    conv = sa.FastConv3d(32, 32, 3, padding=1, bias=False).to(device).to(torch.bfloat16).to(memory_format=CL)
+    conv.defer_weight_grad = True
+    x = torch.randn(1, 32, 4, 8, 32, device=device, dtype=torch.bfloat16).contiguous(memory_format=CL).requires_grad_()
     gy = torch.randn(1, 32, 4, 8, 32, device=device, dtype=torch.bfloat16).contiguous(memory_format=CL)
-    modules._WEIGHT_GRAD_QUEUE.append(modules._QueuedWeightGrad(conv.weight, x2, conv.weight.shape, gy, (1, 1, 1), torch.bfloat16))
+    seen = []
+
+    def hook(_):
+        seen.append((_waiting(), conv.weight.grad))
+        modules.flush_weight_gradients()
+        seen.append((_waiting(), conv.weight.grad))
+
+    x.register_hook(hook)
+    modules.flush_weight_gradients()  # outside of a pass nothing waits
+    conv(x).backward(gy)
+    assert seen[0] == (1, None) and seen[1][0] == 0 and seen[1][1] is conv.weight.grad
+    assert torch.equal(conv.weight.grad, sa.conv3d_backward_weight_batch([(x.detach(), conv.weight.shape, gy, (1, 1, 1))])[0])
+
+
+@pytest.mark.parametrize("defer", [True, "early"])
+def test_a_pass_that_raises_drops_what_it_has_queued(device, defer):
+    """An exception in the middle of a backward pass (out of memory, a hook): the operands it kept for its weight gradients are
+    let go with it, its half of the gradients reaches no ``.grad``, and the next pass is an ordinary one."""
+    net = _tiny_net(device, defer, layers=3)
+    opt = sa.FusedClipAdam(net.parameters(), lr=1e-3, max_norm=1.0, shadow_dtype=torch.bfloat16)
+    target = torch.randint(0, 3, (1, 8, 32, 64), device=device)
+    deferred = [m.weight for m in net.modules() if isinstance(m, sa.FastConv3d) and m.kernel_size == (3, 3, 3) and m.in_channels > 1]
+
+    def run(fail):
+        opt.zero_grad(set_to_none=True)
+        x = torch.randn(1, 1, 8, 32, 64, device=device, generator=torch.Generator(device).manual_seed(3)).contiguous(memory_format=CL)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            feats = net.down_list[0](x)
+            if fail:  # the pass has been through everything but the first block when this runs
+                def hook(_):
+                    held.append(_waiting())
+                    raise RuntimeError("stop here")
+                feats.register_hook(hook)
+            net.down_list[0].forward = lambda _: feats
+            logits = net(x)
+            del net.down_list[0].forward
+        loss = sa.ce_dice_loss(logits, target)
+        if not fail:
+            loss.backward()
+            return [p.grad.clone() for p in net.parameters()]
+        with pytest.raises(RuntimeError, match="stop here"):
+            loss.backward()
+
+    held = []
+    want = run(False)
+    opt.zero_grad(set_to_none=True)
+    gc.collect()
+    torch.cuda.synchronize()
+    allocated = torch.cuda.memory_allocated()
+    run(True)
+    assert held and held[0] > 4 and not _waiting() and not modules._EARLY_DONE
+    assert all(w.grad is None for w in deferred)
     modules.flush_weight_gradients()
-    assert not modules._WEIGHT_GRAD_QUEUE
-    assert torch.equal(conv.weight.grad, sa.conv3d_backward_weight_batch([(x2, conv.weight.shape, gy, (1, 1, 1))])[0])
+    assert all(w.grad is None for w in deferred)
+    opt.zero_grad(set_to_none=True)
+    gc.collect()  # what the traceback holds
+    torch.cuda.synchronize()
+    assert torch.cuda.memory_allocated() == allocated
+    assert all(torch.equal(a, b) for a, b in zip(want, run(False)))
 
 
 def test_deferred_step_as_a_hip_graph_and_under_checkpointing(device):
@@ -263,7 +330,7 @@ def test_deferred_step_as_a_hip_graph_and_under_checkpointing(device):
         got.append(static_loss.item())
         torch.randn(1 << 16, device=device).sum().item()
     assert got == want[1:]
-    assert not modules._WEIGHT_GRAD_QUEUE
+    assert not _waiting()
 
     grads = {}
     for ckpt in (False, True):
@@ -274,7 +341,7 @@ def test_deferred_step_as_a_hip_graph_and_under_checkpointing(device):
         with torch.autocast("cuda", dtype=torch.bfloat16):
             logits = net(x.clone().requires_grad_(True) if ckpt else x)
         sa.ce_dice_loss(logits, target).backward()
-        assert not modules._WEIGHT_GRAD_QUEUE
+        assert not _waiting()
         grads[ckpt] = {n: p.grad.detach().clone() for n, p in net.named_parameters()}
     for n, g in grads[False].items():
         d = grads[True][n].float()
@@ -299,7 +366,7 @@ def test_early_weight_gradients_on_a_stream_of_their_own(device, monkeypatch):
             with torch.autocast("cuda", dtype=torch.bfloat16):
                 logits = net(x)
             sa.ce_dice_loss(logits, target).backward()
-            assert not modules._WEIGHT_GRAD_QUEUE and not modules._EARLY_DONE
+            assert not _waiting() and not modules._EARLY_DONE
         grads[defer] = {n: p.grad.detach().clone() for n, p in net.named_parameters()}
     assert sent and all(n >= 2 for n in sent)                 # the side stream was used, once per pass
     for n, g in grads[False].items():
@@ -340,4 +407,4 @@ def test_early_weight_gradients_on_a_stream_of_their_own(device, monkeypatch):
         got.append(static_loss.item())
         torch.randn(1 << 16, device=device).sum().item()
     assert got == want[1:]
-    assert not modules._WEIGHT_GRAD_QUEUE and not modules._EARLY_DONE
+    assert not _waiting() and not modules._EARLY_DONE
