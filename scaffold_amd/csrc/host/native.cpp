@@ -389,26 +389,34 @@ struct PassQueue {
 std::mutex g_pass_lock;
 std::unordered_map<int, PassQueue> g_passes;
 
-// The gradients of `batch` (one device, operand dtype and gradient dtype) on the current stream, in calls of at most
-// SFH_WGRAD_BATCH_MAX problems filled family by family.
+Problem problem_of(const QueuedWeight& q, int code) {
+  int64_t in[5];
+  std::copy(q.x.sizes().begin(), q.x.sizes().end(), in);
+  if (q.second.defined()) in[1] += q.second.size(1);
+  const int32_t one[3] = {1, 1, 1};
+  Problem prob;
+  TORCH_INTERNAL_ASSERT(make_problem(in, q.param.sizes(), one, q.p, one, code, prob));
+  return prob;
+}
+
+// Where the gradients of `batch` (one device, operand dtype and gradient dtype) go: memory of the current stream.
+void allocate_grads(WeightBatch& batch) {
+  for (const QueuedWeight& q : batch.items) batch.grads.push_back(volume(q.param.sizes(), q.gy, q.master ? at::kFloat : q.gy.scalar_type()));
+}
+
+// Computes them on the current stream, in calls of at most SFH_WGRAD_BATCH_MAX problems filled family by family.
 void launch_batch(WeightBatch& batch, bool share_device) {
   if (batch.items.empty()) return;
   const Tensor& like = batch.items[0].gy;
   c10::OptionalDeviceGuard guard(like.device());
   const int code = code_of(like.scalar_type());
-  const bool fp32 = batch.items[0].master;
-  const uint32_t flags = (fp32 ? SFH_FLAG_GRAD_FP32 : 0) | (share_device ? SFH_FLAG_SHARE_DEVICE : 0);
+  const uint32_t flags = (batch.items[0].master ? SFH_FLAG_GRAD_FP32 : 0) | (share_device ? SFH_FLAG_SHARE_DEVICE : 0);
+  if (batch.grads.empty()) allocate_grads(batch);
   std::vector<sfh_conv3d_wgrad_item> work(batch.items.size());
-  const int32_t one[3] = {1, 1, 1};
   for (size_t i = 0; i < batch.items.size(); ++i) {
     const QueuedWeight& q = batch.items[i];
-    int64_t in[5];
-    std::copy(q.x.sizes().begin(), q.x.sizes().end(), in);
-    if (q.second.defined()) in[1] += q.second.size(1);
-    Problem prob;
-    TORCH_INTERNAL_ASSERT(make_problem(in, q.param.sizes(), one, q.p, one, code, prob));
-    batch.grads.push_back(volume(q.param.sizes(), like, fp32 ? at::kFloat : like.scalar_type()));
-    work[i] = sfh_conv3d_wgrad_item{prob.key.d, ptr(q.x), ptr(q.second), q.second.defined() ? (int32_t)q.x.size(1) : 0, ptr(q.gy), out_ptr(batch.grads[i])};
+    work[i] = sfh_conv3d_wgrad_item{problem_of(q, code).key.d, ptr(q.x), ptr(q.second), q.second.defined() ? (int32_t)q.x.size(1) : 0, ptr(q.gy),
+                                    out_ptr(batch.grads[i])};
   }
   for (int family = 1; family <= 2; ++family) {
     std::vector<sfh_conv3d_wgrad_item> call;
@@ -530,6 +538,7 @@ void queue_weight(QueuedWeight&& q) {
     items.push_back(std::move(q));
   }
   if (leave) {
+    allocate_grads(*leave);  // here and not on the side stream: the pass and the optimizer read them on this one
     {
       py::gil_scoped_acquire gil;
       py::reinterpret_borrow<py::function>(g_send_early)(leave);

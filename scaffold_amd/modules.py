@@ -28,6 +28,7 @@ ordinary padded convolution.
 from __future__ import annotations
 
 import math
+import threading
 from typing import Optional
 
 import torch
@@ -144,29 +145,49 @@ def _deferrable(param, in_shape, wshape, stride, padding, dilation, dtype) -> in
     return ok
 
 
-_EARLY_STREAMS: dict = {}
-_EARLY_DONE: list = []  # batches sent and not joined yet
+_EARLY_LOCK = threading.Lock()
+_EARLY_STREAMS: dict = {}  # (device, a pass's stream) -> the side stream beside it
+_EARLY_DONE: dict = {}  # batch sent and not joined yet -> (the pass's stream, event behind the batch's launches)
+
+
+def _early_stream(main):
+    """The side stream of passes on ``main``.  Each has its own: a pass that is being captured takes its side stream into the
+    capture, and what a pass on another stream sent there meanwhile would become part of that graph."""
+    with _EARLY_LOCK:
+        key = (main.device, main.cuda_stream)
+        side = _EARLY_STREAMS.get(key)
+        if side is None:
+            if len(_EARLY_STREAMS) >= 16:  # half of the streams torch hands out in turn
+                _EARLY_STREAMS.clear()
+            taken = [main, *_EARLY_STREAMS.values()]
+            while side is None or side in taken:
+                side = torch.cuda.Stream(device=main.device)
+            _EARLY_STREAMS[key] = side
+        return side
 
 
 def _send_early(batch) -> None:
-    dev = _lib.native().batch_device(batch)
-    side = _EARLY_STREAMS.get(dev)
-    if side is None:
-        side = _EARLY_STREAMS[dev] = torch.cuda.Stream(device=dev)
-    # Every use of the side stream starts by waiting for the current one and ends (in _join_early) with the
-    # current one waiting for it, and the operands stay referenced until then: memory the caching allocator hands to
-    # either stream is never in use on the other.
-    side.wait_stream(torch.cuda.current_stream(dev))
-    with torch.no_grad(), torch.cuda.stream(side):
-        _lib.native().launch_batch(batch, True)
-    _EARLY_DONE.append(batch)
+    # Operands and gradients are memory of the pass's stream: the side stream starts behind that stream, and they stay
+    # referenced until that stream has been made to wait for the batch (in _join_early, or here if a launch is refused), so
+    # the caching allocator hands none of it out while the batch runs.
+    main = torch.cuda.current_stream(_lib.native().batch_device(batch))
+    side = _early_stream(main)
+    side.wait_stream(main)
+    try:
+        with torch.no_grad(), torch.cuda.stream(side):
+            _lib.native().launch_batch(batch, True)
+    except BaseException:
+        main.wait_stream(side)
+        raise
+    _EARLY_DONE[batch] = main, side.record_event()
 
 
 def _join_early(batch) -> None:
-    # (each pass joins its own batches: another thread's pass may run at the same time, on a stream of its own)
-    dev = _lib.native().batch_device(batch)
-    _EARLY_DONE.remove(batch)
-    torch.cuda.current_stream(dev).wait_stream(_EARLY_STREAMS[dev])
+    main, done = _EARLY_DONE.pop(batch)
+    main.wait_event(done)
+    current = torch.cuda.current_stream(main.device)
+    if current != main:
+        current.wait_event(done)
 
 
 def flush_weight_gradients() -> None:

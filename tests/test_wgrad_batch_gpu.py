@@ -12,6 +12,7 @@ launch -- of a list with a problem the batch does not serve.
 """
 
 import gc
+import threading
 
 import pytest
 import torch
@@ -408,3 +409,66 @@ def test_early_weight_gradients_on_a_stream_of_their_own(device, monkeypatch):
         torch.randn(1 << 16, device=device).sum().item()
     assert got == want[1:]
     assert not _waiting() and not modules._EARLY_DONE
+
+
+def test_early_batches_of_passes_on_different_streams(device):
+    """Two threads run early-mode passes at the same time, each on a stream of its own, accumulating over two passes and letting
+    the gradients go in between: every gradient is the one its passes alone give, and no side stream serves both."""
+    target = torch.randint(0, 3, (1, 8, 32, 64), device=device)
+
+    def make(seed):
+        net = _tiny_net(device, "early", layers=3)
+        g = torch.Generator(device).manual_seed(seed)
+        return net, torch.randn(1, 1, 8, 32, 64, device=device, generator=g).contiguous(memory_format=CL)
+
+    def grads(net, x):
+        net.zero_grad(set_to_none=True)
+        for _ in range(2):
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                logits = net(x)
+            sa.ce_dice_loss(logits, target).backward()
+        return [p.grad.clone() for p in net.parameters()]
+
+    jobs = [make(1), make(2)]
+    want = [grads(*job) for job in jobs]
+    streams = [torch.cuda.Stream() for _ in jobs]
+    sides = [modules._early_stream(s) for s in (torch.cuda.current_stream(), *streams)]
+    assert len({s.cuda_stream for s in (*sides, *streams)}) == 5 and modules._early_stream(streams[0]) is sides[1]
+    got = [[], []]
+
+    def run(i):
+        with torch.cuda.stream(streams[i]):
+            for _ in range(4):
+                got[i].append(grads(*jobs[i]))
+            torch.cuda.current_stream().synchronize()
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for w, runs in zip(want, got):
+        assert len(runs) == 4 and all(torch.equal(a, b) for g in runs for a, b in zip(w, g))
+    assert not _waiting() and not modules._EARLY_DONE
+
+
+def test_gradients_of_an_early_batch_are_memory_of_the_passs_stream(device, monkeypatch):
+    """What a pass lets go returns to its own stream's pool, which the next pass on that stream is served from."""
+    net = _tiny_net(device, "early", layers=3)
+    x = torch.randn(1, 1, 8, 32, 64, device=device).contiguous(memory_format=CL)
+    target = torch.randint(0, 3, (1, 8, 32, 64), device=device)
+    sent = []
+    real = modules._send_early
+    monkeypatch.setattr(modules, "_send_early", lambda batch: (sent.append(torch.cuda.current_stream().cuda_stream), real(batch)))
+    with torch.cuda.stream(torch.cuda.Stream()) as _, torch.autocast("cuda", dtype=torch.bfloat16):
+        sa.ce_dice_loss(net(x), target).backward()
+        stream = torch.cuda.current_stream().cuda_stream
+        torch.cuda.synchronize()
+    assert sent == [stream]
+    blocks = {}
+    for segment in torch.cuda.memory_snapshot():
+        for b in segment["blocks"]:
+            blocks[b["address"]] = segment["stream"]
+    deferred = [m.weight for m in net.modules() if isinstance(m, sa.FastConv3d) and m.kernel_size == (3, 3, 3) and m.in_channels > 1]
+    assert deferred and all(blocks[w.grad.data_ptr()] == stream for w in deferred)
