@@ -12,6 +12,8 @@
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/Event.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/engine.h>
 #include <torch/csrc/autograd/function.h>
@@ -75,6 +77,8 @@ void* stream_of(const Tensor& t) {
   }
   return (void*)c10::hip::getCurrentHIPStream(index).stream();
 }
+
+c10::Stream stream_on(c10::Device device) { return c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getStream(device); }
 
 int code_of(at::ScalarType t) {
   return t == at::kBFloat16 ? SFH_BF16 : t == at::kHalf ? SFH_FP16 : t == at::kFloat ? SFH_FP32 : -1;
@@ -370,6 +374,7 @@ Tensor or_none(const MaybeTensor& t) { return t.has_value() ? *t : Tensor(); }
 // raised has queued is dropped with it.
 struct QueuedWeight {
   Tensor param, x, second, gy;
+  c10::Stream stream;  // the one they are ready on
   int32_t p[3];
   bool master = false, early = false;
   int family = 1;  // the launch of the batch that takes it (1: large rows, 2: small volumes)
@@ -436,6 +441,26 @@ void launch_batch(WeightBatch& batch, bool share_device) {
   }
 }
 
+// A pass computes on the stream of whoever called backward(), and its nodes ran on the streams of their forward ops: what
+// came from another stream is waited for, and its memory is not handed out before this stream has read it.
+void take_over(WeightBatch& batch) {
+  if (batch.items.empty()) return;
+  const c10::Stream here = stream_on(batch.items[0].gy.device());
+  std::vector<c10::Stream> met;
+  for (size_t i = 0; i < batch.items.size(); ++i) {
+    const QueuedWeight& q = batch.items[i];
+    if (q.stream == here) continue;
+    if (std::find(met.begin(), met.end(), q.stream) == met.end()) {
+      met.push_back(q.stream);
+      c10::Event ready(c10::DeviceType::CUDA);
+      ready.record(q.stream);
+      ready.block(here);
+    }
+    for (const Tensor& t : {q.x, q.second, q.gy, batch.grads.empty() ? Tensor() : batch.grads[i]})
+      if (t.defined()) t.record_stream(here);
+  }
+}
+
 void add_to_grads(WeightBatch& batch) {
   for (size_t i = 0; i < batch.items.size(); ++i) {
     const Tensor &param = batch.items[i].param, &gw = batch.grads[i];
@@ -467,7 +492,10 @@ void finish_pass(int id) {
   PassQueue pass = take_pass(id);
   at::AutoGradMode no_grad(false);
   join_sent(pass);
-  for (auto& batch : pass.sent) add_to_grads(*batch);
+  for (auto& batch : pass.sent) {
+    take_over(*batch);
+    add_to_grads(*batch);
+  }
   while (!pass.items.empty()) {
     WeightBatch batch;
     std::vector<QueuedWeight> rest;
@@ -477,6 +505,7 @@ void finish_pass(int id) {
       (same ? batch.items : rest).push_back(std::move(q));
     }
     pass.items = std::move(rest);
+    take_over(batch);
     launch_batch(batch, false);
     add_to_grads(batch);
   }
@@ -526,7 +555,7 @@ void queue_weight(QueuedWeight&& q) {
       // device idle.  The large-row gradients queued so far (the decoder's upper levels) go out now, on a stream of their
       // own and on half of the compute units, beside the rest of the pass.
       auto goes = [&](const QueuedWeight& o) {
-        return o.family == 1 && o.early && o.gy.device() == q.gy.device() && o.gy.scalar_type() == q.gy.scalar_type() && o.master == q.master;
+        return o.family == 1 && o.early && o.stream == q.stream && o.gy.scalar_type() == q.gy.scalar_type() && o.master == q.master;
       };
       if (std::count_if(items.begin(), items.end(), goes) >= 2) {
         leave = std::make_shared<WeightBatch>();
@@ -596,7 +625,7 @@ struct ConvSaved {
       }
     }
     if (need_w && param.defined()) {
-      queue_weight(QueuedWeight{param, xs, x2, gy, {p[0], p[1], p[2]}, master, early, family});
+      queue_weight(QueuedWeight{param, xs, x2, gy, stream_on(gy.device()), {p[0], p[1], p[2]}, master, early, family});
     } else if (need_w) {
       out[1] = launch_wgrad(prob, xs, x2, gy, master);
     }

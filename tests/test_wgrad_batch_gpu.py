@@ -472,3 +472,43 @@ def test_gradients_of_an_early_batch_are_memory_of_the_passs_stream(device, monk
             blocks[b["address"]] = segment["stream"]
     deferred = [m.weight for m in net.modules() if isinstance(m, sa.FastConv3d) and m.kernel_size == (3, 3, 3) and m.in_channels > 1]
     assert deferred and all(blocks[w.grad.data_ptr()] == stream for w in deferred)
+
+
+@pytest.mark.parametrize("defer", [False, True, "early"])
+def test_a_pass_started_from_another_stream_than_its_forward(device, defer):
+    """The nodes run on the forward's stream, the end of the pass on the caller's: what waits for the end is not read before it
+    is there (the output gradients come late here), nor let go before it has been read."""
+    torch.manual_seed(5)
+    convs = torch.nn.ModuleList([sa.FastConv3d(32, 32, 3, padding=1, bias=False) for _ in range(4)]).to(device).to(torch.bfloat16).to(memory_format=CL)
+    for c in convs:
+        c.defer_weight_grad = {"early": 2}.get(defer, defer)
+    pool = sa.FastMaxPool3d(2)
+    x = torch.randn(1, 32, 8, 32, 64, device=device, dtype=torch.bfloat16).contiguous(memory_format=CL)
+    gy = torch.randn(1, 32, 2, 8, 16, device=device, dtype=torch.bfloat16).contiguous(memory_format=CL)
+
+    def late(g):
+        for _ in range(100):
+            g = g * 1
+        return g
+
+    def grads(stream):
+        convs.zero_grad(set_to_none=True)
+        with torch.cuda.stream(stream):
+            h = convs[0](x)
+            for c in convs[1:3]:
+                h = c(h)
+                h.register_hook(late)
+            y = convs[3](pool(pool(h)))
+            y.register_hook(late)
+        y.backward(gy)
+        out = [c.weight.grad.clone() for c in convs]
+        del y, h
+        torch.cuda.synchronize()
+        return out
+
+    want = grads(torch.cuda.current_stream())
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    for _ in range(3):
+        assert all(torch.equal(a, b) for a, b in zip(want, grads(side)))
+    assert not _waiting() and not modules._EARLY_DONE
