@@ -14,6 +14,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/Event.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/engine.h>
 #include <torch/csrc/autograd/function.h>
@@ -461,12 +462,33 @@ void take_over(WeightBatch& batch) {
   }
 }
 
+// Passes of several threads may meet in one parameter: its .grad is written by one at a time, on the device as well (the
+// additions of a pass on another stream come first).  Inside a capture the recorded order is all there is.
+std::mutex g_add_lock;
+struct LastAddition {
+  c10::Stream stream;
+  c10::Event done{c10::DeviceType::CUDA};
+};
+std::unordered_map<int, LastAddition> g_last_addition;  // by device
+
 void add_to_grads(WeightBatch& batch) {
+  if (batch.items.empty()) return;
+  const c10::Device device = batch.items[0].gy.device();
+  c10::OptionalDeviceGuard guard(device);
+  const c10::Stream here = stream_on(device);
+  const bool eager = c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
+  std::lock_guard<std::mutex> hold(g_add_lock);
+  auto last = g_last_addition.try_emplace(device.index(), LastAddition{here}).first;
+  if (eager && last->second.stream != here) last->second.done.block(here);
   for (size_t i = 0; i < batch.items.size(); ++i) {
     const Tensor &param = batch.items[i].param, &gw = batch.grads[i];
     Tensor& grad = param.mutable_grad();
     if (grad.defined()) grad.add_(gw);
     else grad = gw.strides() == param.strides() ? gw : at::empty_like(param).copy_(gw);  // the parameter's own layout, as the engine leaves it
+  }
+  if (eager) {
+    last->second.stream = here;
+    last->second.done.record(here);
   }
 }
 
@@ -1226,7 +1248,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   py::class_<WeightBatch, std::shared_ptr<WeightBatch>>(m, "WeightBatch").def("__len__", &WeightBatch::size);
   m.def("launch_batch", [](WeightBatch& batch, bool share_device) { launch_batch(batch, share_device); });
   m.def("batch_device", [](const WeightBatch& batch) { return batch.items.at(0).gy.device(); });
-  m.def("finish_current_pass", &finish_current_pass);
+  m.def("finish_current_pass", &finish_current_pass, py::call_guard<py::gil_scoped_release>());
   m.def("waiting_weight_gradients", &waiting_weight_gradients);
   m.def("conv_forward", &conv_forward);
   m.def("conv_supported", &conv_supported);

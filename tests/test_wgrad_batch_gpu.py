@@ -512,3 +512,42 @@ def test_a_pass_started_from_another_stream_than_its_forward(device, defer):
     for _ in range(3):
         assert all(torch.equal(a, b) for a, b in zip(want, grads(side)))
     assert not _waiting() and not modules._EARLY_DONE
+
+
+@pytest.mark.parametrize("defer", [True, "early"])
+def test_passes_that_meet_in_the_same_parameters(device, defer):
+    """Two threads run a pass each over one network at the same time, on streams of their own: both end up in ``.grad``, whichever
+    comes first (a sum of two does not depend on the order)."""
+    net = _tiny_net(device, defer, layers=3)
+    target = torch.randint(0, 3, (1, 8, 32, 64), device=device)
+    inputs = [torch.randn(1, 1, 8, 32, 64, device=device).contiguous(memory_format=CL) for _ in range(2)]
+
+    def run(x):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            logits = net(x)
+        sa.ce_dice_loss(logits, target).backward()
+
+    alone = []
+    for x in inputs:
+        net.zero_grad(set_to_none=True)
+        run(x)
+        alone.append([p.grad.clone() for p in net.parameters()])
+    streams = [torch.cuda.Stream() for _ in inputs]
+
+    def work(i):
+        with torch.cuda.stream(streams[i]):
+            run(inputs[i])
+
+    for _ in range(4):
+        net.zero_grad(set_to_none=True)
+        torch.cuda.synchronize()
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+        for (n, p), a, b in zip(net.named_parameters(), *alone):
+            if n.endswith("weight") and p.dim() == 5 and p.shape[1] > 1 and p.shape[2] == 3:
+                assert torch.equal(p.grad, a + b), n
+    assert not _waiting() and not modules._EARLY_DONE
