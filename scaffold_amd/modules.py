@@ -427,15 +427,17 @@ class FastConv3d(nn.Conv3d):
                          master, self.gn_groups, self.defer_weight_grad if master or w is weight else False)
 
 
-def _unhooked(module) -> bool:
-    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+def _plain_call(module) -> bool:
+    """Whether calling the module is its class's ``forward`` and nothing else: no hooks, no ``forward`` or compiled call of its own."""
+    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                or "forward" in module.__dict__ or module._compiled_call_impl is not None)
 
 
 def conv_then_norm(conv, norm, x):
     """``norm(conv(x))`` as one call into the host path and one autograd node, or ``None`` where the two modules have to run
-    by themselves (a bias, hooks on either, a subclass, an input that is not channels-last, ...)."""
+    by themselves (a bias, hooks on either or a ``forward`` of its own, a subclass, an input that is not channels-last, ...)."""
     if type(conv) is not FastConv3d or type(norm) is not FastGroupNorm or conv.groups != 1 or torch.compiler.is_compiling() \
-            or conv.padding_mode != "zeros" or isinstance(conv.padding, str) or not _unhooked(conv) or not _unhooked(norm) \
+            or conv.padding_mode != "zeros" or isinstance(conv.padding, str) or not _plain_call(conv) or not _plain_call(norm) \
             or torch.nn.modules.module._has_any_global_hook() or _lib.under_transform() or not isinstance(x, torch.Tensor) or x.dim() != 5:
         return None
     weight, gamma, beta = conv.weight, norm.weight, norm.bias

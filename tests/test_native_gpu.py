@@ -131,3 +131,22 @@ def test_convolution_and_norm_in_one_call_are_the_two_modules(device):
         handle.remove()
         assert conv_then_norm(conv, norm, x) is not None
         assert conv_then_norm(pair(bias=True)[0], norm, x) is None
+
+
+@pytest.mark.parametrize("attribute", ["forward", "_compiled_call_impl"])
+def test_a_block_calls_what_an_instance_has_put_in_place_of_its_forward(device, attribute):
+    """A wrapper set on one convolution or norm (an offloading hook, a probe, ``module.compile()``) runs inside a block too."""
+    from scaffold_amd.unet import DoubleConv
+
+    block = DoubleConv(32, 32, 8).to(device).to(memory_format=CL)
+    x = _x(device).detach()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        want = block(x)
+        for i in (0, 1, 3, 4):
+            module, calls = block.double_conv[i], []
+            setattr(module, attribute, lambda *a, _f=module.forward, **k: (calls.append(1), _f(*a, **k))[1])
+            assert torch.equal(block(x), want) and len(calls) == 1
+            if attribute == "forward":
+                del module.forward
+            else:
+                module._compiled_call_impl = None
