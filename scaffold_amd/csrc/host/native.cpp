@@ -98,17 +98,18 @@ Tensor volume(at::IntArrayRef sizes, const Tensor& like, at::ScalarType dtype) {
 }
 Tensor bytes(size_t n, const Tensor& like) { return n == 0 ? Tensor() : plain({(int64_t)n}, like, at::kByte); }
 
-// An int or three ints; false for any other spelling (the Python layer then says what is wrong with it).
+// An int or three ints, as the Python layer has it (subclasses of int, no bool); false for any other spelling (the Python
+// layer then says what is wrong with it).
 bool three(py::handle h, int32_t v[3]) {
   auto one = [](PyObject* o, int32_t& to) {
-    if (!PyLong_CheckExact(o)) return false;
+    if (!PyLong_Check(o) || PyBool_Check(o)) return false;
     int overflow = 0;
     const long x = PyLong_AsLongAndOverflow(o, &overflow);
     if (overflow || x < INT32_MIN || x > INT32_MAX) return false;
     to = (int32_t)x;
     return true;
   };
-  if (PyLong_CheckExact(h.ptr())) return one(h.ptr(), v[0]) && (v[1] = v[2] = v[0], true);
+  if (PyLong_Check(h.ptr())) return one(h.ptr(), v[0]) && (v[1] = v[2] = v[0], true);
   if (!PyTuple_Check(h.ptr()) && !PyList_CheckExact(h.ptr())) return false;
   if (PySequence_Fast_GET_SIZE(h.ptr()) != 3) return false;
   for (int i = 0; i < 3; ++i)

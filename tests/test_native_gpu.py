@@ -150,3 +150,23 @@ def test_a_block_calls_what_an_instance_has_put_in_place_of_its_forward(device, 
                 del module.forward
             else:
                 module._compiled_call_impl = None
+
+
+def test_geometry_in_a_subclass_of_int(device):
+    """Sizes may be any ``int`` (a configuration's enum, say), through the modules and their gradients too."""
+    import enum
+
+    n = enum.IntEnum("n", {"one": 1, "two": 2})
+    for dtype in (torch.bfloat16, torch.float32):
+        for plain, other in ((sa.FastConv3d(32, 32, 3, padding=1), sa.FastConv3d(32, 32, 3, n.one, n.one, n.one)),
+                             (sa.FastConvTranspose3d(32, 32, 2, 2), sa.FastConvTranspose3d(32, 32, n.two, n.two))):
+            other.load_state_dict(plain.state_dict())
+            runs = []
+            for module in (plain, other):
+                module.to(device, dtype).to(memory_format=CL)
+                x = torch.linspace(-1, 1, 32 * 128, device=device).view(1, 32, 4, 4, 8).to(dtype).contiguous(memory_format=CL).requires_grad_()
+                y = module(x)
+                runs.append((y, *torch.autograd.grad(y, (x, *module.parameters()), torch.ones_like(y))))
+            assert all(torch.equal(a, b) for a, b in zip(*runs))
+    with pytest.raises(NotImplementedError):  # a bool is none
+        sa.conv3d_forward(x.detach(), plain.weight.detach(), None, True, 1)
