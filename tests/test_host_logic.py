@@ -1,6 +1,11 @@
 """Host-side mirror of the reference interface, without a GPU: gates are total, unsupported calls raise the
 reference's exception types, modules keep stock state dicts, the U-Net has the reference's census."""
 
+import os
+import shutil
+import subprocess
+import sys
+
 import pytest
 import torch
 import torch.nn as nn
@@ -217,3 +222,16 @@ def test_a_callers_packed_weight_is_validated_not_trusted(monkeypatch):
     prob.packed = (0, 0)                            # a problem whose kernels read the weight where it lies
     with pytest.raises(ValueError, match="does not read a packed weight"):
         prob.check_packed(torch.empty(0, dtype=torch.uint8), False, like)
+
+
+@pytest.mark.parametrize("header", ["torch/extension.h", "c10/core/Event.h"])
+def test_the_host_path_is_compiled_again_for_another_torch(header):
+    """``native.cpp`` is built against torch's headers, internals among them: a torch that changes makes the object stale."""
+    if shutil.which("make") is None:
+        pytest.skip("no make here")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    path = os.path.join(os.path.dirname(torch.__file__), "include", header)
+    assert os.path.exists(path)
+    plan = subprocess.run(["make", "-C", os.path.join(root, "scaffold_amd", "csrc", "host"), "-n", "-W", path, f"PY={sys.executable}"],
+                          check=True, stdout=subprocess.PIPE, text=True).stdout
+    assert "-c native.cpp" in plan
