@@ -78,13 +78,14 @@ def compute_copy(param: Optional[torch.Tensor], dtype: Optional[torch.dtype]):
 
 
 def _current_packs(owner: torch.Tensor, source: torch.Tensor, in_shape, stride, padding, dilation):
-    """The packed forms of a parameter's weight for this problem, or ``None`` when the problem reads no packed weight.
+    """The packed forms of a parameter's weight for this problem, or ``None`` when the problem reads no packed weight (or the
+    weight is not on a GPU: the caller's gate comes after this and refuses).
 
     They are kept on the parameter (``owner._sfh_packs``) and trusted without a launch only under the rule that also
     guards the optimizer's half-precision copies: the optimizer that writes the parameter refreshes them inside its
     step (``maintained``) and nothing else has written the parameter since (torch's version counter).  Otherwise they
     are packed again here, in one launch for both directions."""
-    if source.dtype is torch.float32:
+    if source.dtype is torch.float32 or not source.is_cuda:
         return None
     table = owner.__dict__.get("_sfh_packs")
     if table is None:

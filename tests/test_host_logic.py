@@ -15,7 +15,7 @@ from scaffold_amd import conv3d as c3
 from scaffold_amd import groupnorm as gnm
 from scaffold_amd import transposed as ct
 from scaffold_amd.modules import FastConv3d, FastConvTranspose3d, FastGroupNorm, cast_operand
-from scaffold_amd.unet import UNet, skip_concat
+from scaffold_amd.unet import DoubleConv, UNet, skip_concat
 
 
 def test_gates_are_total():
@@ -235,3 +235,23 @@ def test_the_host_path_is_compiled_again_for_another_torch(header):
     plan = subprocess.run(["make", "-C", os.path.join(root, "scaffold_amd", "csrc", "host"), "-n", "-W", path, f"PY={sys.executable}"],
                           check=True, stdout=subprocess.PIPE, text=True).stdout
     assert "-c native.cpp" in plan
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_a_model_on_the_host_is_refused_before_anything_is_packed(dtype, monkeypatch):
+    """The packing of a weight comes before the module's gate and is a kernel that reads the weight where it lies: a model that
+    was never moved to the GPU packs nothing and is refused like any other call that is not served."""
+    def packed(*a, **k):
+        raise AssertionError("a weight on the host was handed to the packing kernel")
+
+    monkeypatch.setattr(c3, "PackedWeights", packed)
+    x = torch.randn(1, 32, 4, 8, 32).to(dtype)
+    block = DoubleConv(32, 32, 8).to(dtype)
+    conv, pair = FastConv3d(32, 32, 3, padding=1, bias=False).to(dtype), FastConv3d(64, 32, 3, padding=1).to(dtype)
+    up = FastConvTranspose3d(32, 32, 2, stride=2).to(dtype)
+    for call in (lambda: conv(x), lambda: pair(x, x), lambda: up(x), lambda: block(x)):
+        for grad in (True, False):
+            with torch.set_grad_enabled(grad), pytest.raises(NotImplementedError):
+                call()
+    with pytest.raises(NotImplementedError):
+        c3.pack_weights(conv.weight.detach(), x.shape, 1, 1, 1)

@@ -78,3 +78,20 @@ def test_an_operators_packed_weight_does_not_lift_the_dtype_rule(device):
     for a, b in ((x.to(torch.float16), w), (x, w.to(torch.float16)), (x, w.float())):
         with pytest.raises(NotImplementedError):
             sa.conv3d_forward(a, b, None, 1, 1, packed_weight=pf)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "masters", "shadows"])
+def test_a_weight_on_the_host_meets_no_kernel(device, kind, monkeypatch):
+    """A module that was never moved to the GPU, given an input that was: refused before anything reads its weight."""
+    packed = []
+    for name in ("pack_weights", "PackedWeights"):
+        monkeypatch.setattr(c3, name, lambda *a, **k: packed.append(a))
+    host = torch.device("cpu")
+    modules_ = [_weights(m, host, kind) for m in (sa.FastConv3d(32, 32, 3, padding=1, bias=False), DoubleConv(32, 32, 8),
+                                                  sa.FastConvTranspose3d(32, 32, 2, stride=2, bias=False))]
+    x = _x(device, 32)
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=kind != "bf16"):
+        for module in modules_:
+            with pytest.raises(NotImplementedError):
+                module(x)
+    assert not packed
