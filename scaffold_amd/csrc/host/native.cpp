@@ -1159,7 +1159,8 @@ py::object max_pool(const Tensor& x_in, int64_t halo, bool with_skip) {
       rc = sfh_maxpool2_fwd(&d, code, ptr(x), out_ptr(y), (uint8_t*)out_ptr(idx), stream_of(x));
     }
     check(rc, "max_pool3d_2x");
-    if (with_skip) skip = x_in.detach();
+    // (a view made without a graph: what is written into it would also change x_in, whose other uses autograd could not tell)
+    if (with_skip) skip = graph ? x_in.view_as(x_in) : x_in.detach();
     if (graph && slab.defined()) y = y.detach();
   }
   if (graph) {

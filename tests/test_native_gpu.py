@@ -170,3 +170,18 @@ def test_geometry_in_a_subclass_of_int(device):
             assert all(torch.equal(a, b) for a, b in zip(*runs))
     with pytest.raises(NotImplementedError):  # a bool is none
         sa.conv3d_forward(x.detach(), plain.weight.detach(), None, True, 1)
+
+
+def test_the_skip_connection_is_not_written_in_place(device):
+    """It is the pooled tensor's own memory: a write into it would change that tensor under its other uses, so autograd refuses
+    it, as for any output of a function that returns views; out of place the gradients are those of x used three times."""
+    pool = sa.FastMaxPool3d(2)
+    x = _x(device)
+    h = x * 1
+    y, skip = pool.with_skip(h)
+    assert skip.data_ptr() == h.data_ptr()
+    with pytest.raises(RuntimeError, match="modified inplace"):
+        skip.mul_(2)
+    (got,) = torch.autograd.grad(y.float().sum() + (skip * 2).float().sum() + h.float().sum(), x)
+    want = 3 + torch.autograd.grad(torch.nn.functional.max_pool3d(x.float(), 2).sum(), x)[0]
+    assert torch.equal(got, want)
