@@ -394,7 +394,7 @@ struct PassQueue {
 };
 
 std::mutex g_pass_lock;
-std::unordered_map<int, PassQueue> g_passes;
+auto& g_passes = *new std::unordered_map<int, PassQueue>;  // never destroyed: a thread may still be in a pass at exit
 
 Problem problem_of(const QueuedWeight& q, int code) {
   int64_t in[5];
@@ -470,7 +470,7 @@ struct LastAddition {
   c10::Stream stream;
   c10::Event done{c10::DeviceType::CUDA};
 };
-std::unordered_map<int, LastAddition> g_last_addition;  // by device
+auto& g_last_addition = *new std::unordered_map<int, LastAddition>;  // by device (never destroyed: the runtime may be gone before)
 
 void add_to_grads(WeightBatch& batch) {
   if (batch.items.empty()) return;
