@@ -159,6 +159,13 @@ MfmaConvArgs patch_pack_args(int produced, int reduced) {
   return a;
 }
 
+// A 2x2x2 weight (csmall, cbig, 2, 2, 2) in channels-last memory order, [csmall][tap][cbig], on 16 bytes: the kernels of the
+// family that keep their weights in registers fetch it as it lies.
+bool dense_patch_weight(const void* w, const int64_t ws[5], int cbig) {
+  return on_16_bytes(w) && ws[0] == 8 * (int64_t)cbig && ws[1] == 1 && ws[2] == 4 * (int64_t)cbig && ws[3] == 2 * (int64_t)cbig &&
+         ws[4] == cbig;
+}
+
 PatchArgs convT_patch_args(const sfh_convT3d_desc& p) {
   PatchArgs a{};
   a.n = p.n;
@@ -922,7 +929,7 @@ static int convT3d_fwd_any(const sfh_convT3d_desc* p, int dtype, const void* x, 
     // w is the packed form: the data-gradient packing of the kernel == stride convolution this one transposes
     if ((flags & SFH_FLAG_FORCE_GENERIC) || !convT_uses_patch(*p, dtype))
       return fail(SFH_ERR_INVALID, "convT3d fwd: this problem does not read a packed weight");
-    return patch_scatter(convT_patch_args(*p), dtype, x, w, bias, y, (hipStream_t)stream, halo_elems);
+    return patch_scatter(convT_patch_args(*p), dtype, x, w, false, bias, y, (hipStream_t)stream, halo_elems);
   }
   if (!(flags & SFH_FLAG_FORCE_GENERIC) && convT_uses_patch(*p, dtype)) {
     // produced channel = Cout (w_stride[1]), reduced channel = Cin (w_stride[0])
@@ -931,9 +938,12 @@ static int convT3d_fwd_any(const sfh_convT3d_desc* p, int dtype, const void* x, 
     if (workspace == nullptr || workspace_bytes < need)
       return fail(SFH_ERR_WORKSPACE, "convT3d fwd: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
     hipStream_t st = (hipStream_t)stream;
+    const PatchArgs a = convT_patch_args(*p);
+    if (patch_scatter_reads_dense(a) && dense_patch_weight(w, w_stride, a.cbig))
+      return patch_scatter(a, dtype, x, w, true, bias, y, st, halo_elems);
     if (int rc = mfma_pack_weight(pk, dtype, w, w_stride[1], w_stride[0], w_stride[2], w_stride[3], w_stride[4], 0, workspace, st))
       return rc;
-    return patch_scatter(convT_patch_args(*p), dtype, x, workspace, bias, y, st, halo_elems);
+    return patch_scatter(a, dtype, x, workspace, false, bias, y, st, halo_elems);
   }
   if (halo_elems > 0) return fail(SFH_ERR_UNSUPPORTED, "convT3d fwd: only the 2x2x2 matrix-core kernel writes into a slab");
   return direct_convT(*p, dtype, w_stride, x, w, bias, y, (hipStream_t)stream);

@@ -3,8 +3,9 @@
 // convolution, transposed.py:1073) and its weight gradient (transposed.py:1113).
 //
 // Windows do not overlap, so there is no halo and nothing to reuse between neighbouring voxels: the
-// three kernels are HBM-bound GEMMs with M = small voxels. The gather and the scatter take both MFMA
-// operands straight from global memory (a lane's fragment is 8 consecutive channels of one voxel, one
+// three kernels are HBM-bound GEMMs with M = small voxels. The scatter keeps its weights in registers and
+// turns voxel tiles through LDS; the gather and the scatter's general form take both MFMA operands
+// straight from global memory (a lane's fragment is 8 consecutive channels of one voxel, one
 // 16-byte load; the weight is pre-packed in fragment order and stays in L1/L2). The weight gradient
 // contracts over voxels, so both operands must be transposed: tiles are staged in LDS in their natural
 // [voxel][channel] layout and read with ds_read_b64_tr_b16, which hands each lane four consecutive
@@ -44,6 +45,27 @@ __device__ __forceinline__ int64_t big_index(const PatchArgs& a, const Voxel& v,
   return (((int64_t)v.nn * a.bd + 2 * v.d + (tap >> 2)) * a.bh + 2 * v.h + ((tap >> 1) & 1)) * a.bw + 2 * v.w + (tap & 1);
 }
 
+// Operand fragment (32 channels x 16 voxels) from a natural-layout LDS tile: `tile` points at the first
+// of the 16 voxel rows, channel 0 of the block. Within each group of 16 lanes the transposing read takes
+// lane m's address as (voxel m / 4, channels 4 * (m % 4) .. + 3) and returns to lane m channel m of the
+// four voxels, so two reads give a lane its 8 voxels of the k-step.
+template <typename T>
+__device__ __forceinline__ uint4 tr_fragment(const T* tile, int row_stride, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef short v4s __attribute__((__vector_size__(4 * sizeof(short))));
+  const int g = lane >> 4, m = lane & 15;
+  const T* p0 = tile + ((g >> 1) * 8 + (m >> 2)) * row_stride + (g & 1) * 16 + 4 * (m & 3);
+  const T* p1 = p0 + 4 * row_stride;
+  const v4s r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(p0));
+  const v4s r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(p1));
+  uint4 out;
+  out.x = __builtin_bit_cast(uint2, r0).x; out.y = __builtin_bit_cast(uint2, r0).y;
+  out.z = __builtin_bit_cast(uint2, r1).x; out.w = __builtin_bit_cast(uint2, r1).y;
+  return out;
+#else
+  return make_uint4(0, 0, 0, 0);
+#endif
+}
 
 // ---- gather: stride-2 convolution --------------------------------------------------------------
 // A wavefront owns 32 small voxels x NB blocks of 32 produced channels. grid = (voxel tiles of 128, groups of NB blocks).
@@ -142,6 +164,145 @@ __global__ void __launch_bounds__(256) patch_gather_deep_kernel(PatchArgs a, con
 }
 
 // ---- scatter: transposed convolution -----------------------------------------------------------
+// Zeroes the two faces of `face_pieces` 16-byte pieces around a depth slab's interior `big` of `big_elems` elements,
+// spread over the `nthreads` threads of the launch.
+template <typename T>
+__device__ __forceinline__ void zero_faces(T* big, int64_t face_pieces, int64_t big_elems, int64_t me, int64_t nthreads) {
+  uint4* lo = reinterpret_cast<uint4*>(big) - face_pieces;
+  uint4* hi = reinterpret_cast<uint4*>(big + big_elems);
+  for (int64_t p = me; p < face_pieces; p += nthreads) {
+    lo[p] = make_uint4(0, 0, 0, 0);
+    hi[p] = make_uint4(0, 0, 0, 0);
+  }
+}
+
+// Columns (tap, block of 32 big channels) of the 2 x 2 x 2 patch are numbered as they lie in memory: blocks, then the taps.
+// A workgroup owns 4 * C neighbouring columns, a wavefront C of them, whose weights it KEEPS in registers (csmall = 16 * KS
+// channels: 4 * C * KS registers a lane) while the workgroup walks tiles of 32 voxels: a tile is fetched in whole lines one
+// tile ahead, laid into LDS as [8-channel piece][voxel] and read from there by all four wavefronts; the results leave in
+// runs of 64 * C bytes per voxel (whole lines for C = 2).
+// What bounds the general form is the CU's address path: a fragment straight from memory is 32 lines of 32 bytes each,
+// and a wavefront of it fetched its weights and its tile for two taps only.
+// grid = groups of tiles (in eights, one per XCD) x (cbig / 16 / C) groups of columns, those of a tile on one XCD.
+// PACKED: `w` is in fragment order; else dense [csmall][tap][cbig], turned through LDS once per wavefront.
+template <typename T, int KS, int C, bool PACKED>
+__global__ void __launch_bounds__(256, 2) patch_scatter_kernel(PatchArgs a, const T* __restrict__ small, const T* __restrict__ w,
+                                                               const T* __restrict__ bias, T* __restrict__ big, int64_t total,
+                                                               int groups, int64_t face_pieces, int64_t big_elems) {
+  constexpr int PIECES = 2 * KS;                        // 16-byte pieces of a voxel
+  constexpr int PLANE = 512 + (PIECES >= 16 ? 16 : 32);  // bytes; writes of a voxel's pieces fall into different banks
+  constexpr int PER = PIECES * 32 / 256;                // pieces a thread moves per tile
+  constexpr int kTurn = 4;                              // k-steps of a weight column turned at a time
+  constexpr int kLds = 2 * PIECES * PLANE > 4 * kTurn * 1024 || PACKED ? 2 * PIECES * PLANE : 4 * kTurn * 1024;
+  constexpr int kOutRow = 64 * C + 16;                  // LDS bytes of a voxel's run of 64 * C bytes
+  constexpr int kLanes = 4 * C;                         // lanes that store one such run
+  __shared__ __attribute__((aligned(16))) char lds[kLds];
+  __shared__ __attribute__((aligned(16))) char s_out[4][32 * kOutRow];
+  if (face_pieces > 0)
+    zero_faces(big, face_pieces, big_elems, (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int kg = lane >> 5;
+  const int nblk = a.cbig / 32;
+  const int ncol = 2 * nblk / C;
+  const int slot = blockIdx.x / kXcds;
+  const int group = slot / ncol * kXcds + blockIdx.x % kXcds;
+  if (group >= groups) return;
+  const int c0 = slot % ncol * 4 * C + C * wave;  // this wavefront's first column
+  const int64_t tiles = (total + 31) / 32, pieces = total * PIECES;
+  char* out = s_out[wave];
+  uint4 next[PER];
+  auto fetch = [&](int64_t tile) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      int64_t q = tile * (32 * PIECES) + i * 256 + tid;
+      next[i] = load16(small + (q < pieces ? q : pieces - 1) * 8);
+    }
+  };
+  fetch(group);
+  int blk[C];
+  uint4 wf[C][KS];
+  float add[C][16];
+#pragma unroll
+  for (int j = 0; j < C; ++j) {
+    const int tap = (c0 + j) / nblk;
+    blk[j] = (c0 + j) % nblk;
+    if constexpr (PACKED) {
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        wf[j][k] = load16(w + (((((int64_t)blk[j] * (KS / 2) + (k >> 1)) * kTaps + tap) * 2 + (k & 1)) * 64 + lane) * 8);
+    } else {
+      T* mine = reinterpret_cast<T*>(lds) + wave * (kTurn * 512);
+      const T* src = w + ((int64_t)(lane >> 2) * kTaps + tap) * a.cbig + blk[j] * 32 + (lane & 3) * 8;
+#pragma unroll
+      for (int k0 = 0; k0 < KS; k0 += kTurn) {
+        uint4 raw[kTurn];
+#pragma unroll
+        for (int k = 0; k < kTurn; ++k) raw[k] = load16(src + (int64_t)(k0 + k) * 16 * kTaps * a.cbig);
+        __syncthreads();  // the previous k-steps have been read
+#pragma unroll
+        for (int k = 0; k < kTurn; ++k) *reinterpret_cast<uint4*>(mine + k * 512 + lane * 8) = raw[k];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kTurn; ++k) wf[j][k0 + k] = tr_fragment<T>(mine + k * 512, 32, lane);
+      }
+    }
+    load_block_bias<T>(bias, blk[j] * 32, kg, add[j]);
+  }
+  if constexpr (!PACKED) __syncthreads();
+  const int run0 = c0 % (2 * nblk) * 32;  // from the first of the two big voxels along W
+  int phase = 0;
+  for (int64_t t = group; t < tiles; t += groups, phase ^= 1) {
+    char* tile = lds + phase * (PIECES * PLANE);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int q = i * 256 + tid;
+      *reinterpret_cast<uint4*>(tile + (q % PIECES) * PLANE + (q / PIECES) * 16) = next[i];
+    }
+    __syncthreads();  // the other half was read before the barrier of the tile behind it
+    fetch(t + groups < tiles ? t + groups : t);
+    f32x16_t acc[C];
+#pragma unroll
+    for (int j = 0; j < C; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      const uint4 f = *reinterpret_cast<const uint4*>(tile + (2 * k + kg) * PLANE + (lane & 31) * 16);
+#pragma unroll
+      for (int j = 0; j < C; ++j) acc[j] = Mma32<T>::run(wf[j][k], f, acc[j]);
+    }
+    // the columns of a voxel are contiguous: turned through LDS so that neighbouring lanes store one run
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      uint32_t run[4][2];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        run[g][0] = Mma32<T>::pack2(acc[j][4 * g] + add[j][4 * g], acc[j][4 * g + 1] + add[j][4 * g + 1]);
+        run[g][1] = Mma32<T>::pack2(acc[j][4 * g + 2] + add[j][4 * g + 2], acc[j][4 * g + 3] + add[j][4 * g + 3]);
+      }
+      uint4 piece[2];
+      trade_channel_runs(run, piece);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        *reinterpret_cast<uint4*>(out + (lane & 31) * kOutRow + j * 64 + h * 32 + kg * 16) = piece[h];
+    }
+    const int64_t v = t * 32 + (lane & 31);
+    const Voxel vx = decode_small(a, v < total ? v : total - 1);
+    const int at = (int)big_index(a, vx, c0 / nblk & 6);
+    const int left = (int)(total - t * 32 < 32 ? total - t * 32 : 32);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < kLanes / 2; ++i) {
+      const int row = (i * 64 + lane) / kLanes;
+      const uint4 piece = *reinterpret_cast<const uint4*>(out + row * kOutRow + (lane % kLanes) * 16);
+      const int64_t vox = __shfl(at, row);
+      if (row < left) *reinterpret_cast<uint4*>(big + vox * a.cbig + run0 + (lane % kLanes) * 8) = piece;
+    }
+  }
+}
+
+// The general form, for reduction widths whose weights do not fit in registers.
 // A wavefront owns 32 small voxels x one block of 32 big channels x TS of the 8 taps.
 // grid = (voxel tiles of 128, cbig / 32, 8 / TS). TS = 8 reads the small tensor once; TS = 1 and 2 are for launches that
 // would otherwise leave most of the chip idle or give a CU a single long chain of dependent loads (the deeper levels):
@@ -149,18 +310,13 @@ __global__ void __launch_bounds__(256) patch_gather_deep_kernel(PatchArgs a, con
 // `face_pieces` > 0: `big` is the interior of a depth slab whose two faces of that many 16-byte pieces (in front of it and
 // behind its `big_elems` elements) the launch zeroes as well, spread over all its threads.
 template <typename T, int TS>
-__global__ void __launch_bounds__(256) patch_scatter_kernel(PatchArgs a, const T* __restrict__ small, const T* __restrict__ packed,
+__global__ void __launch_bounds__(256) patch_scatter_any_kernel(PatchArgs a, const T* __restrict__ small, const T* __restrict__ packed,
                                                             const T* __restrict__ bias, T* __restrict__ big, int64_t total,
                                                             int64_t face_pieces, int64_t big_elems) {
   if (face_pieces > 0) {
     const int64_t nthreads = (int64_t)gridDim.x * gridDim.y * gridDim.z * 256;
-    const int64_t me = (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
-    uint4* lo = reinterpret_cast<uint4*>(big) - face_pieces;
-    uint4* hi = reinterpret_cast<uint4*>(big + big_elems);
-    for (int64_t p = me; p < face_pieces; p += nthreads) {
-      lo[p] = make_uint4(0, 0, 0, 0);
-      hi[p] = make_uint4(0, 0, 0, 0);
-    }
+    zero_faces(big, face_pieces, big_elems, (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * 256 + threadIdx.x,
+               nthreads);
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int kg = lane >> 5;
@@ -212,24 +368,6 @@ constexpr int kVx = 32;             // voxels staged per round (two k-steps of 1
 constexpr int kSmallTile = 64;      // small channels per workgroup (two row blocks)
 constexpr int kSRow = kSmallTile + 8;  // LDS row strides in elements: 16-byte aligned, off the 128-byte period
 constexpr int kBRow = 32 + 8;
-
-// Operand fragment (32 channels x 16 voxels) from a natural-layout LDS tile: `tile` points at the first
-// of the 16 voxel rows, channel 0 of the block. Within each group of 16 lanes the transposing read takes
-// lane m's address as (voxel m / 4, channels 4 * (m % 4) .. + 3) and returns to lane m channel m of the
-// four voxels, so two reads give a lane its 8 voxels of the k-step.
-template <typename T>
-__device__ __forceinline__ uint4 tr_fragment(const T* tile, int row_stride, int lane) {
-  typedef short v4s __attribute__((__vector_size__(4 * sizeof(short))));
-  const int g = lane >> 4, m = lane & 15;
-  const T* p0 = tile + ((g >> 1) * 8 + (m >> 2)) * row_stride + (g & 1) * 16 + 4 * (m & 3);
-  const T* p1 = p0 + 4 * row_stride;
-  const v4s r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(p0));
-  const v4s r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(p1));
-  uint4 out;
-  out.x = __builtin_bit_cast(uint2, r0).x; out.y = __builtin_bit_cast(uint2, r0).y;
-  out.z = __builtin_bit_cast(uint2, r1).x; out.w = __builtin_bit_cast(uint2, r1).y;
-  return out;
-}
 
 // grid = (splits, csmall / 64, cbig / 32). Wavefront w accumulates taps 2w and 2w + 1 for both row blocks.
 // BIAS: the workgroups of the first small-channel tile also add up the big tensor itself over the voxels -- the bias
@@ -352,8 +490,26 @@ int launch_gather(const PatchArgs& a, const void* big, const void* packed, const
   return check_launch("patch_gather_kernel");
 }
 
+template <typename T, int KS, int C>
+int launch_scatter_kept(const PatchArgs& a, const void* small, const void* w, bool dense, const void* bias, void* big, hipStream_t st,
+                        int64_t face_pieces, int64_t big_elems) {
+  const int64_t total = small_voxels(a), tiles = cdiv(total, 32);
+  const int ncol = 2 * (a.cbig / 32) / C;
+  // two workgroups per CU are what the registers allow (three and four: 5 to 20 % slower, the weights are fetched more often)
+  int64_t groups = cdiv(2 * kComputeUnits, ncol);
+  if (groups > tiles) groups = tiles;
+  const dim3 grid((unsigned)(cdiv(groups, kXcds) * kXcds * ncol));
+  if (dense)
+    hipLaunchKernelGGL((patch_scatter_kernel<T, KS, C, false>), grid, dim3(256), 0, st, a, (const T*)small, (const T*)w, (const T*)bias,
+                       (T*)big, total, (int)groups, face_pieces, big_elems);
+  else
+    hipLaunchKernelGGL((patch_scatter_kernel<T, KS, C, true>), grid, dim3(256), 0, st, a, (const T*)small, (const T*)w, (const T*)bias,
+                       (T*)big, total, (int)groups, face_pieces, big_elems);
+  return check_launch("patch_scatter_kernel");
+}
+
 template <typename T>
-int launch_scatter(const PatchArgs& a, const void* small, const void* packed, const void* bias, void* big, hipStream_t st,
+int launch_scatter(const PatchArgs& a, const void* small, const void* w, bool dense, const void* bias, void* big, hipStream_t st,
                    int64_t halo_elems) {
   const int64_t total = small_voxels(a);
   const int64_t big_elems = (int64_t)a.n * a.bd * a.bh * a.bw * a.cbig;
@@ -361,25 +517,35 @@ int launch_scatter(const PatchArgs& a, const void* small, const void* packed, co
                          (halo_elems * (int64_t)sizeof(T)) % 16 != 0))
     return fail(SFH_ERR_UNSUPPORTED, "convT3d fwd: a slab output needs one sample and 16-byte aligned faces");
   const int64_t face_pieces = halo_elems > 0 ? halo_elems * (int64_t)sizeof(T) / 16 : 0;
+  // Weights of one (512 channels) or two columns fit in a wavefront's registers: the kept form, at every volume. General form ->
+  // kept form, packed weight, us: 128 -> 64 at 64^3 120 -> 74, at 32^3 20.7 -> 12.3, at 16x32x32 12 -> 8.5; 64 -> 32 at 64^3 47 -> 28,
+  // at 32x64x64 25 -> 17; 256 -> 128 at 32^3 48 -> 26, at 8x16x16 7.8 -> 5.9; 512 -> 256 at 16^3 29 -> 15, at 4x8x8 7.2 -> 4.8.
+  if (patch_scatter_reads_dense(a)) {
+    if (a.csmall == 64) return launch_scatter_kept<T, 4, 2>(a, small, w, dense, bias, big, st, face_pieces, big_elems);
+    if (a.csmall == 128) return launch_scatter_kept<T, 8, 2>(a, small, w, dense, bias, big, st, face_pieces, big_elems);
+    if (a.csmall == 256) return launch_scatter_kept<T, 16, 2>(a, small, w, dense, bias, big, st, face_pieces, big_elems);
+    return launch_scatter_kept<T, 32, 1>(a, small, w, dense, bias, big, st, face_pieces, big_elems);
+  }
+  if (dense) return fail(SFH_ERR_INVALID, "convT3d fwd: this problem reads a packed weight");
   dim3 grid((unsigned)cdiv(total, 128), (unsigned)(a.cbig / 32));
   const int64_t wgs = (int64_t)grid.x * grid.y;
   if (wgs < kComputeUnits) {  // under one workgroup per CU: one tap per workgroup
     grid.z = kTaps;
-    hipLaunchKernelGGL((patch_scatter_kernel<T, 1>), grid, dim3(256), 0, st, a, (const T*)small, (const T*)packed, (const T*)bias,
+    hipLaunchKernelGGL((patch_scatter_any_kernel<T, 1>), grid, dim3(256), 0, st, a, (const T*)small, (const T*)w, (const T*)bias,
                        (T*)big, total, face_pieces, big_elems);
   } else if (wgs < 4 * kComputeUnits) {  // under four per CU: two taps (the big voxels next to each other along W)
     grid.z = kTaps / 2;
-    hipLaunchKernelGGL((patch_scatter_kernel<T, 2>), grid, dim3(256), 0, st, a, (const T*)small, (const T*)packed, (const T*)bias,
+    hipLaunchKernelGGL((patch_scatter_any_kernel<T, 2>), grid, dim3(256), 0, st, a, (const T*)small, (const T*)w, (const T*)bias,
                        (T*)big, total, face_pieces, big_elems);
   } else {
     // four taps (one big depth plane of the 2 x 2 x 2 patch) per workgroup: eight taps need 295 registers a lane, i.e. one
     // wavefront per SIMD walking four dependent trips to memory each (31 us at 64 -> 32 on 32 x 64 x 64); with half the
     // accumulators three wavefronts share a SIMD, and the small tensor read twice costs less than that gains
     grid.z = 2;
-    hipLaunchKernelGGL((patch_scatter_kernel<T, 4>), grid, dim3(256), 0, st, a, (const T*)small, (const T*)packed, (const T*)bias,
+    hipLaunchKernelGGL((patch_scatter_any_kernel<T, 4>), grid, dim3(256), 0, st, a, (const T*)small, (const T*)w, (const T*)bias,
                        (T*)big, total, face_pieces, big_elems);
   }
-  return check_launch("patch_scatter_kernel");
+  return check_launch("patch_scatter_any_kernel");
 }
 
 struct ReducePlan { int splits; int64_t per_split; };
@@ -440,10 +606,16 @@ int patch_gather(const PatchArgs& a, int dtype, const void* big, const void* pac
   return launch_gather<fp16_t>(a, big, packed, bias, small, st);
 }
 
-int patch_scatter(const PatchArgs& a, int dtype, const void* small, const void* packed, const void* bias, void* big, hipStream_t st,
-                  int64_t halo_elems) {
-  if (dtype == SFH_BF16) return launch_scatter<bf16_t>(a, small, packed, bias, big, st, halo_elems);
-  return launch_scatter<fp16_t>(a, small, packed, bias, big, st, halo_elems);
+// (the kept form numbers big voxels in 32 bits)
+bool patch_scatter_reads_dense(const PatchArgs& a) {
+  return (a.csmall == 64 || a.csmall == 128 || a.csmall == 256 || a.csmall == 512) &&
+         (int64_t)a.n * a.bd * a.bh * a.bw <= 0x7fffffffLL;
+}
+
+int patch_scatter(const PatchArgs& a, int dtype, const void* small, const void* w, bool dense, const void* bias, void* big,
+                  hipStream_t st, int64_t halo_elems) {
+  if (dtype == SFH_BF16) return launch_scatter<bf16_t>(a, small, w, dense, bias, big, st, halo_elems);
+  return launch_scatter<fp16_t>(a, small, w, dense, bias, big, st, halo_elems);
 }
 
 int patch_reduce_splits(const PatchArgs& a) { return reduce_plan(a).splits; }

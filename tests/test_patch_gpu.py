@@ -1,0 +1,61 @@
+"""The 2x2x2 stride-2 kernels where their launch forms change: every register-kept width, several tiles per workgroup with a cut
+last tile, fewer tiles than workgroups, and the three ways a weight can lie (packed, channels-last, anything else)."""
+
+import pytest
+import torch
+
+import scaffold_amd as sa
+from scaffold_amd import conv3d as c3
+
+CL = torch.channels_last_3d
+pytestmark = pytest.mark.gpu
+
+#        n, cin, cout, small extents
+SHAPES = [
+    (1, 64, 32, (33, 36, 36)),      # 1337 tiles on 512 groups, the last one cut
+    (1, 64, 96, (5, 6, 7)),         # three blocks: column pairs that reach over two taps
+    (2, 128, 64, (17, 31, 33)),     # 1088 tiles, two samples in one tile
+    (1, 128, 32, (1, 1, 1)),
+    (1, 256, 128, (7, 9, 11)),
+    (1, 256, 64, (16, 16, 17)),
+    (1, 512, 256, (3, 5, 7)),
+    (1, 512, 32, (12, 13, 14)),
+    (1, 96, 32, (9, 10, 11)),       # no kept form: general kernels
+    (1, 1024, 64, (2, 3, 3)),
+]
+
+
+def _operands(n, cin, cout, extents, dtype):
+    g = torch.Generator("cuda").manual_seed(11)
+    d, h, w = extents
+    x = torch.randn((n, cin, d, h, w), generator=g, device="cuda").to(dtype).contiguous(memory_format=CL)
+    gy = torch.randn((n, cout, 2 * d, 2 * h, 2 * w), generator=g, device="cuda").to(dtype).contiguous(memory_format=CL)
+    wt = (torch.randn((cin, cout, 2, 2, 2), generator=g, device="cuda") / cin ** 0.5).to(dtype).contiguous(memory_format=CL)
+    b = torch.randn(cout, generator=g, device="cuda").to(dtype)
+    return x, gy, wt, b
+
+
+def _close(got, want, dtype):
+    # one rounding of the result (2^-9 bf16, 2^-12 fp16, relative to each element) on top of an fp32 sum of a few thousand terms
+    ulp = 2.0 ** -8 if dtype is torch.bfloat16 else 2.0 ** -11
+    scale = want.abs().max()
+    assert torch.all((got.double() - want).abs() <= ulp * want.abs() + 1e-5 * scale)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,cin,cout,extents", SHAPES)
+def test_forward(n, cin, cout, extents, dtype):
+    x, gy, wt, b = _operands(n, cin, cout, extents, dtype)
+    y = sa.conv_transpose3d_forward(x, wt, b, 2)
+    rows = x.permute(0, 2, 3, 4, 1).reshape(-1, cin).double() @ wt.double().permute(0, 2, 3, 4, 1).reshape(cin, -1)
+    d, h, w = extents
+    want = rows.view(n, d, h, w, 2, 2, 2, cout).permute(0, 7, 1, 4, 2, 5, 3, 6).reshape(n, cout, 2 * d, 2 * h, 2 * w)
+    _close(y, want + b.double()[None, :, None, None, None], dtype)
+    # the same bits whatever the weight's layout: packed, another memory order, off the 16-byte grid
+    _, pd = c3.pack_weights(wt, gy.shape, stride=2, padding=0)
+    assert torch.equal(sa.conv_transpose3d_forward(x, wt, b, 2, packed_weight=pd), y)
+    assert torch.equal(sa.conv_transpose3d_forward(x, wt.contiguous(), b, 2), y)
+    flat = torch.empty(wt.numel() + 1, dtype=dtype, device="cuda")[1:]
+    off = flat.as_strided(wt.shape, wt.stride())
+    off.copy_(wt)
+    assert torch.equal(sa.conv_transpose3d_forward(x, off, b, 2), y)
