@@ -406,16 +406,18 @@ static int conv3d_fwd_any(const sfh_conv3d_desc* p, int dtype, const void* x, co
     return f32_conv(a, x, workspace, bias, y, st);
   }
   if (!(flags & SFH_FLAG_FORCE_GENERIC) && (flags & SFH_FLAG_WEIGHT_PACKED) && fwd_uses_patch(*p, dtype, out))
-    return patch_gather(patch_args(*p, out), dtype, x, w, bias, y, st);
+    return patch_gather(patch_args(*p, out), dtype, x, w, false, bias, y, st);
   if (flags & SFH_FLAG_WEIGHT_PACKED) return fail(SFH_ERR_INVALID, "conv3d fwd: this problem does not read a packed weight");
   if (!(flags & SFH_FLAG_FORCE_GENERIC) && fwd_uses_patch(*p, dtype, out)) {
     const MfmaConvArgs pk = patch_pack_args(p->cout, p->cin);
     const size_t need = mfma_conv_packed_weight_bytes(pk);
     if (workspace == nullptr || workspace_bytes < need)
       return fail(SFH_ERR_WORKSPACE, "conv3d fwd: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+    const PatchArgs a = patch_args(*p, out);
+    if (patch_gather_reads_dense(a) && dense_patch_weight(w, w_stride, a.cbig)) return patch_gather(a, dtype, x, w, true, bias, y, st);
     if (int rc = mfma_pack_weight(pk, dtype, w, w_stride[0], w_stride[1], w_stride[2], w_stride[3], w_stride[4], 0, workspace, st))
       return rc;
-    return patch_gather(patch_args(*p, out), dtype, x, workspace, bias, y, st);
+    return patch_gather(a, dtype, x, workspace, false, bias, y, st);
   }
   if (!(flags & SFH_FLAG_FORCE_GENERIC)) {
     ThinArgs t;

@@ -3,10 +3,10 @@
 // convolution, transposed.py:1073) and its weight gradient (transposed.py:1113).
 //
 // Windows do not overlap, so there is no halo and nothing to reuse between neighbouring voxels: the
-// three kernels are HBM-bound GEMMs with M = small voxels. The scatter keeps its weights in registers and
-// turns voxel tiles through LDS; the gather and the scatter's general form take both MFMA operands
-// straight from global memory (a lane's fragment is 8 consecutive channels of one voxel, one
-// 16-byte load; the weight is pre-packed in fragment order and stays in L1/L2). The weight gradient
+// three kernels are HBM-bound GEMMs with M = small voxels. The gather and the scatter keep their weights
+// in registers and turn voxel tiles through LDS; their general forms take both MFMA operands straight from
+// global memory (a lane's fragment is 8 consecutive channels of one voxel, one 16-byte load; the weight is
+// pre-packed in fragment order and stays in L1/L2). The weight gradient
 // contracts over voxels, so both operands must be transposed: tiles are staged in LDS in their natural
 // [voxel][channel] layout and read with ds_read_b64_tr_b16, which hands each lane four consecutive
 // voxels of one channel.
@@ -68,7 +68,131 @@ __device__ __forceinline__ uint4 tr_fragment(const T* tile, int row_stride, int 
 }
 
 // ---- gather: stride-2 convolution --------------------------------------------------------------
-// A wavefront owns 32 small voxels x NB blocks of 32 produced channels. grid = (voxel tiles of 128, groups of NB blocks).
+// The kept form. A wavefront owns one block of 32 small channels and KEEPS its weights in registers -- all eight taps of cbig
+// channels, those of a depth tap (KH = 2) or of a row of the patch (KH = 4) -- while its workgroup walks tiles of 32 * VS
+// voxels: the tile's patches are fetched in whole rows (2 * cbig contiguous channels) one tile ahead, laid into LDS as
+// [8-channel piece][voxel] and read from there by the wavefronts of every block, so the big tensor is read once per NBW blocks.
+// The KH parts of a block meet in LDS in their order. Like the scatter's general form, this one's was bound by the address path.
+// grid = groups of tiles (in eights, one per XCD) x groups of NBW blocks.
+// PACKED: `w` is in fragment order; else dense [csmall][tap][cbig], laid out block by block like a tile.
+template <int CB>
+struct GatherKept {
+  static constexpr int KH = CB <= 64 ? 1 : CB / 64;  // parts of the reduction
+  static constexpr int NBW = CB == 32 || CB == 256 ? 2 : 4;  // blocks of 32 small channels per workgroup
+  static constexpr int VS = CB == 32 ? 2 : 1;        // 32-voxel parts of a tile
+  static constexpr int UNITS = NBW * VS, THREADS = 64 * KH * UNITS;
+  static constexpr int V = 32 * VS;
+  static constexpr int ROW = CB / 4;                 // 16-byte pieces of the two big voxels along W
+  static constexpr int PIECES = 4 * ROW;
+  static constexpr int KSW = CB / 2 / KH;            // k-steps of a wavefront
+  static constexpr int PLANE = V * 16 + (ROW >= 16 ? 16 : 32);  // writes of a voxel's pieces fall into different banks
+  static constexpr int VOX = ROW * V / THREADS;      // voxels a thread fetches for, four rows each
+  static constexpr int WPER = PIECES * 32 / THREADS; // pieces of a weight block a thread moves
+  static constexpr int BUFS = KH == 4 ? 1 : 2;       // tiles in LDS (the barrier in front of the parts' sum also frees the one)
+};
+
+template <typename T, int CB, bool PACKED>
+__global__ void __launch_bounds__(GatherKept<CB>::THREADS, 2)
+patch_gather_kept_kernel(PatchArgs a, const T* __restrict__ big, const T* __restrict__ w, const T* __restrict__ bias,
+                         T* __restrict__ small, int64_t total, int groups) {
+  using C = GatherKept<CB>;
+  __shared__ __attribute__((aligned(16))) char lds[C::BUFS][C::PIECES * C::PLANE];
+  __shared__ float s_part[C::KH == 1 ? 1 : (C::KH - 1) * C::UNITS * 16 * 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int kg = lane >> 5;
+  const int ncol = a.csmall / (32 * C::NBW);
+  const int slot = blockIdx.x / kXcds;
+  const int group = slot / ncol * kXcds + blockIdx.x % kXcds;
+  if (group >= groups) return;
+  const int kpart = wave / C::UNITS, unit = wave % C::UNITS;  // unit: (voxel part, block)
+  const int part = unit / C::NBW;
+  const int blk0 = slot % ncol * C::NBW, blk = blk0 + unit % C::NBW;
+  const int64_t tiles = (total + C::V - 1) / C::V;
+  uint4 next[C::VOX][4];
+  auto fetch = [&](int64_t tile) {
+#pragma unroll
+    for (int i = 0; i < C::VOX; ++i) {
+      const int64_t v = tile * C::V + (i * C::THREADS + tid) / C::ROW;
+      const T* src = big + big_index(a, decode_small(a, v < total ? v : total - 1), 0) * CB + tid % C::ROW * 8;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) next[i][r] = load16(src + ((int64_t)(r >> 1) * a.bh + (r & 1)) * a.bw * CB);
+    }
+  };
+  fetch(group);
+  uint4 wf[C::KSW];
+  if constexpr (PACKED) {
+#pragma unroll
+    for (int i = 0; i < C::KSW; ++i) {
+      const int k = kpart * C::KSW + i, tap = k / (CB / 16), c16 = k % (CB / 16);
+      wf[i] = load16(w + (((((int64_t)blk * (CB / 32) + (c16 >> 1)) * kTaps + tap) * 2 + (c16 & 1)) * 64 + lane) * 8);
+    }
+  } else {
+    uint4 raw[C::WPER];
+    auto fetch_block = [&](int b) {
+#pragma unroll
+      for (int i = 0; i < C::WPER; ++i) raw[i] = load16(w + ((int64_t)(blk0 + b) * 32 * C::PIECES + i * C::THREADS + tid) * 8);
+    };
+    fetch_block(0);
+#pragma unroll
+    for (int b = 0; b < C::NBW; ++b) {
+      char* buf = lds[b % C::BUFS];
+#pragma unroll
+      for (int i = 0; i < C::WPER; ++i) {
+        const int q = i * C::THREADS + tid;
+        *reinterpret_cast<uint4*>(buf + q % C::PIECES * C::PLANE + q / C::PIECES * 16) = raw[i];
+      }
+      if (b + 1 < C::NBW) fetch_block(b + 1);
+      __syncthreads();
+      if (unit % C::NBW == b) {
+#pragma unroll
+        for (int i = 0; i < C::KSW; ++i)
+          wf[i] = *reinterpret_cast<const uint4*>(buf + (2 * (kpart * C::KSW + i) + kg) * C::PLANE + (lane & 31) * 16);
+      }
+      if constexpr (C::BUFS == 1) __syncthreads();
+    }
+  }
+  float add[16];
+  load_block_bias<T>(bias, blk * 32, kg, add);
+  int phase = 0;
+  for (int64_t t = group; t < tiles; t += groups, phase ^= C::BUFS - 1) {
+    char* tile = lds[phase];
+#pragma unroll
+    for (int i = 0; i < C::VOX; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<uint4*>(tile + (r * C::ROW + tid % C::ROW) * C::PLANE + (i * C::THREADS + tid) / C::ROW * 16) = next[i][r];
+    __syncthreads();  // with two buffers the other one was read before the barrier of the tile behind it
+    fetch(t + groups < tiles ? t + groups : t);
+    f32x16_t acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int i = 0; i < C::KSW; ++i) {
+      const int k = kpart * C::KSW + i;
+      acc = Mma32<T>::run(wf[i], *reinterpret_cast<const uint4*>(tile + (2 * k + kg) * C::PLANE + (part * 32 + (lane & 31)) * 16), acc);
+    }
+    if constexpr (C::KH > 1) {
+      if (kpart > 0) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s_part[(((kpart - 1) * C::UNITS + unit) * 16 + r) * 64 + lane] = acc[r];
+      }
+      __syncthreads();
+      if (kpart == 0) {
+#pragma unroll
+        for (int p = 0; p < C::KH - 1; ++p)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[r] += s_part[((p * C::UNITS + unit) * 16 + r) * 64 + lane];
+      }
+    }
+    if (kpart == 0) {
+      const int64_t v = t * C::V + part * 32 + (lane & 31);
+      const bool valid = v < total;
+      store_block_plus<T>(acc, small + (valid ? v : total - 1) * a.csmall + blk * 32, add, kg, valid);
+    }
+  }
+}
+
+// The general form. A wavefront owns 32 small voxels x NB blocks of 32 produced channels. grid = (voxel tiles of 128, groups of NB blocks).
 template <typename T, int NB>
 __global__ void __launch_bounds__(256) patch_gather_kernel(PatchArgs a, const T* __restrict__ big, const T* __restrict__ packed,
                                                            const T* __restrict__ bias, T* __restrict__ small, int64_t total) {
@@ -469,18 +593,54 @@ int gather_blocks(const PatchArgs& a) {
   return nb;
 }
 
+// The kept form takes the channel counts it has tiles for once there are a few dozen tiles; below that the chain of one
+// workgroup's tile is longer than the deep kernel's. Before -> kept, packed weight, us: 64 -> 32 at 64^3 34 -> 26, at 32x64x64
+// 19 -> 15, at 16^3 3.3 -> 4.2; 128 -> 64 at 64^3 108 -> 65, at 32^3 15.1 -> 11.2, at 16x32x32 11.8 -> 7.3, at 8^3 3.7 -> 4.8;
+// 256 -> 128 at 32^3 38 -> 25, at 8x16x16 6.9 -> 6.7, at 5x7x9 (two samples) 4.8 -> 6.7; 512 -> 256 at 16^3 38 -> 23.
+bool gather_kept(const PatchArgs& a) {
+  if (small_voxels(a) * a.cbig < (1 << 18)) return false;
+  return a.cbig == 32 || a.cbig == 256 ? a.csmall % 64 == 0 : (a.cbig == 64 || a.cbig == 128) && a.csmall % 128 == 0;
+}
+
+template <typename T, int CB>
+int launch_gather_kept(const PatchArgs& a, const void* big, const void* w, bool dense, const void* bias, void* small, hipStream_t st) {
+  using C = GatherKept<CB>;
+  const int64_t total = small_voxels(a), tiles = cdiv(total, C::V);
+  const int ncol = a.csmall / (32 * C::NBW);
+  int64_t groups = cdiv((C::KH == 1 ? 2 : 1) * kComputeUnits, ncol);  // what LDS lets be resident
+  if (groups > tiles) groups = tiles;
+  const dim3 grid((unsigned)(cdiv(groups, kXcds) * kXcds * ncol));
+  if constexpr (CB != 256) {
+    if (dense) {
+      hipLaunchKernelGGL((patch_gather_kept_kernel<T, CB, false>), grid, dim3(C::THREADS), 0, st, a, (const T*)big, (const T*)w,
+                         (const T*)bias, (T*)small, total, (int)groups);
+      return check_launch("patch_gather_kept_kernel");
+    }
+  }
+  hipLaunchKernelGGL((patch_gather_kept_kernel<T, CB, true>), grid, dim3(C::THREADS), 0, st, a, (const T*)big, (const T*)w,
+                     (const T*)bias, (T*)small, total, (int)groups);
+  return check_launch("patch_gather_kept_kernel");
+}
+
 template <typename T>
-int launch_gather(const PatchArgs& a, const void* big, const void* packed, const void* bias, void* small, hipStream_t st) {
+int launch_gather(const PatchArgs& a, const void* big, const void* w, bool dense, const void* bias, void* small, hipStream_t st) {
+  if (dense && !patch_gather_reads_dense(a)) return fail(SFH_ERR_INVALID, "conv3d fwd: this problem reads a packed weight");
+  if (gather_kept(a)) {
+    if (a.cbig == 32) return launch_gather_kept<T, 32>(a, big, w, dense, bias, small, st);
+    if (a.cbig == 64) return launch_gather_kept<T, 64>(a, big, w, dense, bias, small, st);
+    if (a.cbig == 128) return launch_gather_kept<T, 128>(a, big, w, dense, bias, small, st);
+    return launch_gather_kept<T, 256>(a, big, w, dense, bias, small, st);
+  }
   const int64_t total = small_voxels(a);
   const int nb = gather_blocks(a);
   const dim3 grid((unsigned)cdiv(total, 128), (unsigned)(a.csmall / 32 / nb));
   if (nb == 1 && (int64_t)grid.x * grid.y < kComputeUnits) {  // under one workgroup per CU (no gain measured above that)
     hipLaunchKernelGGL((patch_gather_deep_kernel<T>), dim3((unsigned)cdiv(total, 32), (unsigned)(a.csmall / 32)), dim3(256), 0, st, a,
-                       (const T*)big, (const T*)packed, (const T*)bias, (T*)small, total);
+                       (const T*)big, (const T*)w, (const T*)bias, (T*)small, total);
     return check_launch("patch_gather_deep_kernel");
   }
 #define SFH_PATCH_GATHER(NB)                                                                                              \
-  hipLaunchKernelGGL((patch_gather_kernel<T, NB>), grid, dim3(256), 0, st, a, (const T*)big, (const T*)packed, (const T*)bias, \
+  hipLaunchKernelGGL((patch_gather_kernel<T, NB>), grid, dim3(256), 0, st, a, (const T*)big, (const T*)w, (const T*)bias, \
                      (T*)small, total)
   if (nb == 8) SFH_PATCH_GATHER(8);
   else if (nb == 4) SFH_PATCH_GATHER(4);
@@ -601,11 +761,14 @@ bool patch_reduce_supported(const PatchArgs& a, int dtype) {
          a.csmall / kSmallTile <= 65535;
 }
 
-int patch_gather(const PatchArgs& a, int dtype, const void* big, const void* packed, const void* bias, void* small, hipStream_t st) {
-  if (dtype == SFH_BF16) return launch_gather<bf16_t>(a, big, packed, bias, small, st);
-  return launch_gather<fp16_t>(a, big, packed, bias, small, st);
+int patch_gather(const PatchArgs& a, int dtype, const void* big, const void* w, bool dense, const void* bias, void* small,
+                 hipStream_t st) {
+  if (dtype == SFH_BF16) return launch_gather<bf16_t>(a, big, w, dense, bias, small, st);
+  return launch_gather<fp16_t>(a, big, w, dense, bias, small, st);
 }
 
+// (256 channels: the registers of the weights and of the layout pass together spill, 33 us against 23 + a packing at 16^3)
+bool patch_gather_reads_dense(const PatchArgs& a) { return gather_kept(a) && a.cbig != 256; }
 // (the kept form numbers big voxels in 32 bits)
 bool patch_scatter_reads_dense(const PatchArgs& a) {
   return (a.csmall == 64 || a.csmall == 128 || a.csmall == 256 || a.csmall == 512) &&

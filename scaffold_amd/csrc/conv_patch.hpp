@@ -20,10 +20,13 @@ bool patch_supported(const PatchArgs& a, int dtype);         // gather and scatt
 bool patch_reduce_supported(const PatchArgs& a, int dtype);
 // `packed` holds the weight in MFMA fragment order [produced/32][reduced/32][tap][kstep][lane][8]
 // (mfma_pack_weight): produced = csmall for gather, cbig for scatter.
-int patch_gather(const PatchArgs& a, int dtype, const void* big, const void* packed, const void* bias, void* small, hipStream_t st);
+// `dense`: w is no packed form but the weight as it lies in a channels-last tensor, [csmall][tap][cbig] on 16 bytes; offered
+// where patch_gather_reads_dense / patch_scatter_reads_dense.
+bool patch_gather_reads_dense(const PatchArgs& a);
+int patch_gather(const PatchArgs& a, int dtype, const void* big, const void* w, bool dense, const void* bias, void* small,
+                 hipStream_t st);
 // `halo_elems` > 0 (one sample): big is the interior of a depth slab with that many elements of face on either side,
-// which the launch zeroes too. `dense`: w is no packed form but the weight as it lies in a channels-last tensor,
-// [csmall][tap][cbig] on 16 bytes; offered where patch_scatter_reads_dense.
+// which the launch zeroes too.
 bool patch_scatter_reads_dense(const PatchArgs& a);
 int patch_scatter(const PatchArgs& a, int dtype, const void* small, const void* w, bool dense, const void* bias, void* big,
                   hipStream_t st, int64_t halo_elems = 0);

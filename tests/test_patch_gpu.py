@@ -59,3 +59,34 @@ def test_forward(n, cin, cout, extents, dtype):
     off = flat.as_strided(wt.shape, wt.stride())
     off.copy_(wt)
     assert torch.equal(sa.conv_transpose3d_forward(x, off, b, 2), y)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,cin,cout,extents,odd", [
+    (1, 64, 32, (33, 36, 36), 0),     # tiles of 64 voxels, several per workgroup, the last one cut
+    (1, 64, 32, (20, 20, 20), 1),     # 8000 voxels, under the rule's line; a big volume with a plane no window covers
+    (1, 64, 32, (8, 32, 32), 1),      # 8192, on it
+    (2, 128, 64, (17, 31, 33), 1),
+    (1, 128, 64, (8, 17, 31), 0),
+    (1, 256, 128, (13, 13, 13), 0),   # the reduction in two parts
+    (1, 256, 128, (2, 32, 32), 1),
+    (1, 512, 256, (9, 11, 13), 1),    # in four
+    (1, 192, 32, (20, 21, 22), 0),    # three groups of two blocks
+    (1, 64, 64, (16, 17, 18), 0),     # no kept form for this pair
+])
+def test_backward_data(n, cin, cout, extents, odd, dtype):
+    _, _, wt, _ = _operands(n, cin, cout, (1, 1, 1), dtype)
+    g = torch.Generator("cuda").manual_seed(5)
+    d, h, w = extents
+    big = torch.randn((n, cout, 2 * d + odd, 2 * h + odd, 2 * w + odd), generator=g, device="cuda").to(dtype).contiguous(memory_format=CL)
+    b = torch.randn(cin, generator=g, device="cuda").to(dtype)
+    y = sa.conv3d_forward(big, wt, b, 2, 0)
+    rows = big[:, :, :2 * d, :2 * h, :2 * w].double().reshape(n, cout, d, 2, h, 2, w, 2).permute(0, 2, 4, 6, 3, 5, 7, 1).reshape(n * d * h * w, -1)
+    want = rows @ wt.double().permute(2, 3, 4, 1, 0).reshape(-1, cin) + b.double()
+    _close(y.permute(0, 2, 3, 4, 1).reshape(-1, cin), want, dtype)
+    pf, _ = c3.pack_weights(wt, big.shape, stride=2, padding=0)
+    assert torch.equal(sa.conv3d_forward(big, wt, b, 2, 0, packed_weight=pf), y)
+    assert torch.equal(sa.conv3d_forward(big, wt.contiguous(), b, 2, 0), y)
+    if not odd:
+        gx = sa.conv_transpose3d_backward_data(big, wt, (n, cin, d, h, w), 2)
+        _close(gx.permute(0, 2, 3, 4, 1).reshape(-1, cin), want - b.double(), dtype)
