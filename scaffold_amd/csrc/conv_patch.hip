@@ -45,6 +45,36 @@ __device__ __forceinline__ int64_t big_index(const PatchArgs& a, const Voxel& v,
   return (((int64_t)v.nn * a.bd + 2 * v.d + (tap >> 2)) * a.bh + 2 * v.h + ((tap >> 1) & 1)) * a.bw + 2 * v.w + (tap & 1);
 }
 
+// A voxel that moves on by the same number of voxels every time (decoding it anew costs three divisions: at two wavefronts a
+// SIMD some 1200 cycles a round, which bounded the weight gradient). `at`: its patch's first big voxel.
+struct VoxelStep { int w, h, d; int64_t at, carry_w, carry_h, carry_d; };
+__device__ __forceinline__ VoxelStep voxel_step(const PatchArgs& a, int64_t voxels) {
+  const Voxel s = decode_small(a, voxels);
+  VoxelStep r;
+  r.w = s.w; r.h = s.h; r.d = s.d;
+  r.at = big_index(a, s, 0);
+  r.carry_w = 2 * ((int64_t)a.bw - a.sw);
+  r.carry_h = 2 * ((int64_t)a.bh - a.sh) * a.bw;
+  r.carry_d = ((int64_t)a.bd - 2 * a.sd) * a.bh * a.bw;
+  return r;
+}
+struct VoxelWalk {
+  int w, h, d;
+  int64_t at;
+  __device__ __forceinline__ void start(const PatchArgs& a, int64_t v) {
+    const Voxel s = decode_small(a, v);
+    w = s.w; h = s.h; d = s.d;
+    at = big_index(a, s, 0);
+  }
+  __device__ __forceinline__ void advance(const PatchArgs& a, const VoxelStep& s) {
+    at += s.at;
+    w += s.w; h += s.h; d += s.d;
+    if (w >= a.sw) { w -= a.sw; ++h; at += s.carry_w; }
+    if (h >= a.sh) { h -= a.sh; ++d; at += s.carry_h; }
+    if (d >= a.sd) { d -= a.sd; at += s.carry_d; }
+  }
+};
+
 // Operand fragment (32 channels x 16 voxels) from a natural-layout LDS tile: `tile` points at the first
 // of the 16 voxel rows, channel 0 of the block. Within each group of 16 lanes the transposing read takes
 // lane m's address as (voxel m / 4, channels 4 * (m % 4) .. + 3) and returns to lane m channel m of the
@@ -490,23 +520,34 @@ __global__ void __launch_bounds__(256) patch_scatter_any_kernel(PatchArgs a, con
 // ---- reduce: weight gradient -------------------------------------------------------------------
 constexpr int kVx = 32;             // voxels staged per round (two k-steps of 16)
 constexpr int kSmallTile = 64;      // small channels per workgroup (two row blocks)
-constexpr int kSRow = kSmallTile + 8;  // LDS row strides in elements: 16-byte aligned, off the 128-byte period
-constexpr int kBRow = 32 + 8;
 
-// grid = (splits, csmall / 64, cbig / 32). Wavefront w accumulates taps 2w and 2w + 1 for both row blocks.
+// A workgroup accumulates 64 small channels x 8 taps x 32 big channels over a range of voxels; its two halves of four wavefronts
+// take the rounds of 32 voxels in turn (wavefront w of a half: taps 2w and 2w + 1 for both row blocks) and meet in LDS at the
+// end, half 0 plus half 1, so that twice the wavefronts load without a second fp32 slice in memory. A round's operands are
+// requested two rounds ahead and laid into the two phases of LDS in turn; a channel block's rows of 64 bytes
+// lie dense, which neither the 16-byte writes nor the transposing reads meet a bank conflict on.
+// grid: `by_xcd` ? eight-fold splits x tiles, the tiles of a range of voxels on one XCD (its lines come from HBM once; spread
+// over the XCDs 128 -> 64 at 48x40x56 took 84 us instead of 41) : tiles x splits.
 // BIAS: the workgroups of the first small-channel tile also add up the big tensor itself over the voxels -- the bias
 // gradient of the transposed convolution whose weight gradient this is (every big voxel is a tap of exactly one small
-// voxel there) -- as one more MFMA row block of ones: bias_part[split][tap][cb], the same fixed order as the weights'.
+// voxel there) -- as one more MFMA row block of ones: bias_part[split][cb], in a fixed order.
 template <typename T, bool BIAS>
-__global__ void __launch_bounds__(256) patch_reduce_kernel(PatchArgs a, const T* __restrict__ small, const T* __restrict__ big,
-                                                           float* __restrict__ part, int64_t total, int64_t per_split,
-                                                           float* __restrict__ bias_part) {
+__global__ void __launch_bounds__(512, 2) patch_reduce_kernel(PatchArgs a, const T* __restrict__ small, const T* __restrict__ big,
+                                                              float* __restrict__ part, int64_t total, int64_t per_split, int splits,
+                                                              int by_xcd, float* __restrict__ bias_part) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __shared__ __attribute__((aligned(16))) T s_tile[kVx * kSRow];
-  __shared__ __attribute__((aligned(16))) T b_tile[kTaps * kVx * kBRow];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int cs0 = blockIdx.y * kSmallTile, cb0 = blockIdx.z * 32;
-  const int64_t begin = (int64_t)blockIdx.x * per_split;
+  constexpr int D = 2;                           // rounds requested ahead
+  constexpr int kBlock = kVx * 32;               // elements of one [voxel][32 channels] block
+  constexpr int kRound = (2 + kTaps) * kBlock;   // two blocks of the small tensor, one per tap of the big
+  __shared__ __attribute__((aligned(16))) T lds[2][2][kRound];
+  const int nz = a.cbig / 32, tiles = a.csmall / kSmallTile * nz;
+  const int slot = blockIdx.x / kXcds;
+  const int split = by_xcd ? slot / tiles * kXcds + (int)(blockIdx.x % kXcds) : (int)blockIdx.x / tiles;
+  const int tile = (by_xcd ? slot : (int)blockIdx.x) % tiles;
+  if (split >= splits) return;
+  const int half = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+  const int cs0 = tile / nz * kSmallTile, cb0 = tile % nz * 32;
+  const int64_t begin = (int64_t)split * per_split;
   int64_t end = begin + per_split;
   if (end > total) end = total;
   f32x16_t acc[2][2];
@@ -521,62 +562,108 @@ __global__ void __launch_bounds__(256) patch_reduce_kernel(PatchArgs a, const T*
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int r = 0; r < 16; ++r) bacc[j][r] = 0.f;
-  const bool sums_big = BIAS && blockIdx.y == 0;
+  const bool sums_big = BIAS && cs0 == 0;
   const uint32_t one2 = sizeof(T) == 2 && std::is_same<T, bf16_t>::value ? 0x3f803f80u : 0x3c003c00u;  // two ones of T
   const uint4 ones = make_uint4(one2, one2, one2, one2);
   const int s_vox = tid >> 3, s_piece = tid & 7;          // small tile: 32 voxels x 8 pieces of 16 bytes
   const int b_vox = (tid >> 2) & 31, b_piece = tid & 3;   // big tiles: 4 taps (tid/128, +2, +4, +6) of one voxel
   const int b_tap0 = tid >> 7;
   const uint4 zero = make_uint4(0, 0, 0, 0);
-  for (int64_t v0 = begin; v0 < end; v0 += kVx) {
-    uint4 sv = zero, bv[4] = {zero, zero, zero, zero};
-    if (v0 + s_vox < end) sv = load16(small + (v0 + s_vox) * a.csmall + cs0 + s_piece * 8);
+  VoxelWalk walk;
+  walk.start(a, begin + half * kVx + b_vox);
+  const VoxelStep step = voxel_step(a, 2 * kVx);
+  int64_t tap_at[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) tap_at[i] = big_index(a, Voxel{0, 0, 0, 0}, b_tap0 + 2 * i);
+  struct Round { uint4 s, b[4]; } ahead[D];
+  auto fetch = [&](Round& o, int64_t v0) {
+    o.s = zero;
+    if (v0 + s_vox < end) o.s = load16(small + (v0 + s_vox) * a.csmall + cs0 + s_piece * 8);
     if (v0 + b_vox < end) {
-      const Voxel vx = decode_small(a, v0 + b_vox);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) bv[i] = load16(big + big_index(a, vx, b_tap0 + 2 * i) * a.cbig + cb0 + b_piece * 8);
+      for (int i = 0; i < 4; ++i) o.b[i] = load16(big + (walk.at + tap_at[i]) * a.cbig + cb0 + b_piece * 8);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o.b[i] = zero;
     }
-    __syncthreads();  // the previous round's reads are done
-    *reinterpret_cast<uint4*>(s_tile + s_vox * kSRow + s_piece * 8) = sv;
+    walk.advance(a, step);
+  };
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      *reinterpret_cast<uint4*>(b_tile + ((b_tap0 + 2 * i) * kVx + b_vox) * kBRow + b_piece * 8) = bv[i];
-    __syncthreads();
+  for (int u = 0; u < D; ++u) fetch(ahead[u], begin + (2 * u + half) * kVx);
+  for (int64_t v0 = begin; v0 < end; v0 += 2 * D * kVx) {
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      uint4 af[2], bf[2];
+    for (int u = 0; u < D; ++u) {
+      const int64_t v = v0 + 2 * u * kVx;
+      if (u > 0 && v >= end) break;
+      T* s_tile = lds[u & 1][half];
+      T* b_tile = s_tile + 2 * kBlock;
+      *reinterpret_cast<uint4*>(s_tile + (s_piece >> 2) * kBlock + s_vox * 32 + (s_piece & 3) * 8) = ahead[u].s;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) af[i] = tr_fragment<T>(s_tile + ks * 16 * kSRow + i * 32, kSRow, lane);
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<uint4*>(b_tile + (b_tap0 + 2 * i) * kBlock + b_vox * 32 + b_piece * 8) = ahead[u].b[i];
+      __syncthreads();  // the other phase was read before the barrier of the round behind it
+      fetch(ahead[u], v + (2 * D + half) * kVx);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) bf[j] = tr_fragment<T>(b_tile + ((2 * wave + j) * kVx + ks * 16) * kBRow, kBRow, lane);
+      for (int ks = 0; ks < 2; ++ks) {
+        uint4 af[2], bf[2];
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 2; ++i) af[i] = tr_fragment<T>(s_tile + i * kBlock + ks * 16 * 32, 32, lane);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = Mma32<T>::run(af[i], bf[j], acc[i][j]);
-      if constexpr (BIAS) {
-        if (sums_big) {  // every row of the block is the column sum
+        for (int j = 0; j < 2; ++j) bf[j] = tr_fragment<T>(b_tile + (2 * wave + j) * kBlock + ks * 16 * 32, 32, lane);
 #pragma unroll
-          for (int j = 0; j < 2; ++j) bacc[j] = Mma32<T>::run(ones, bf[j], bacc[j]);
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = Mma32<T>::run(af[i], bf[j], acc[i][j]);
+        if constexpr (BIAS) {
+          if (sums_big) {  // every row of the block is the column sum
+#pragma unroll
+            for (int j = 0; j < 2; ++j) bacc[j] = Mma32<T>::run(ones, bf[j], bacc[j]);
+          }
         }
       }
     }
   }
-  // part[split][cs][tap][cb]: a lane holds column cb = lane % 32 and 16 rows of each block
-  float* dst = part + (int64_t)blockIdx.x * a.csmall * kTaps * a.cbig;
+  // half h keeps row block h and hands the other one over
+  __syncthreads();
+  float* hand = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float v0 = acc[0][j][r], v1 = acc[1][j][r];
+      hand[((half * 2 + j) * 16 + r) * 256 + tid] = half ? v0 : v1;
+    }
+  if constexpr (BIAS) {
+    if (half) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) hand[(64 + j) * 256 + tid] = bacc[j][0];
+    }
+  }
+  __syncthreads();
+  // part[split][cs][tap][cb]: a lane holds column cb = lane % 32 and 16 rows of its block
+  float* dst = part + (int64_t)split * a.csmall * kTaps * a.cbig;
   const int col = lane & 31, kg = lane >> 5;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int cs = cs0 + i * 32 + 8 * (r >> 2) + 4 * kg + (r & 3);
-        dst[((int64_t)cs * kTaps + 2 * wave + j) * a.cbig + cb0 + col] = acc[i][j][r];
-      }
+    for (int r = 0; r < 16; ++r) {
+      const float v0 = acc[0][j][r], v1 = acc[1][j][r];
+      const float other = hand[(((half ^ 1) * 2 + j) * 16 + r) * 256 + tid];
+      const int cs = cs0 + half * 32 + 8 * (r >> 2) + 4 * kg + (r & 3);
+      dst[((int64_t)cs * kTaps + 2 * wave + j) * a.cbig + cb0 + col] = half ? other + v1 : v0 + other;
+    }
   if constexpr (BIAS) {
-    if (sums_big && kg == 0) {
+    float* sums = hand + 66 * 256;  // [tap][channel], then their sum in tap order: one row of channels per split
+    if (half == 0 && kg == 0) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) bias_part[((int64_t)blockIdx.x * kTaps + 2 * wave + j) * a.cbig + cb0 + col] = bacc[j][0];
+      for (int j = 0; j < 2; ++j) sums[(2 * wave + j) * 32 + col] = bacc[j][0] + hand[(64 + j) * 256 + tid];
+    }
+    __syncthreads();
+    if (sums_big && threadIdx.x < 32) {
+      float sum = 0.f;
+#pragma unroll
+      for (int t = 0; t < kTaps; ++t) sum += sums[t * 32 + threadIdx.x];
+      bias_part[(int64_t)split * a.cbig + cb0 + threadIdx.x] = sum;
     }
   }
 #endif
@@ -710,15 +797,24 @@ int launch_scatter(const PatchArgs& a, const void* small, const void* w, bool de
 
 struct ReducePlan { int splits; int64_t per_split; };
 
+// Splits of the voxels: up to one workgroup per CU, and fewer where the slices (written, then read by the sum) cost more than
+// the shorter ranges gain. 0.7 us is a round of both halves, 0.6 us a megabyte of slices, fitted to sweeps of 1 to 256 splits over
+// 17 problems (best plan within 5 % on each). Two workgroups of four wavefronts per CU, a slice each -> this, us with the sum: 128 -> 64
+// at 64^3 119 -> 106, at 32^3 24.4 -> 20.5, at 48x40x56 84 -> 38; 64 -> 32 at 64^3 36 -> 33; 256 -> 128 at 32^3 49 -> 41, at 8x16x16 23 -> 15;
+// 512 -> 256 at 4x8x8 24 -> 13. Eight at a time: a range of voxels per XCD.
 ReducePlan reduce_plan(const PatchArgs& a) {
   const int64_t total = small_voxels(a);
   const int64_t tiles = (int64_t)(a.csmall / kSmallTile) * (a.cbig / 32);
   const int64_t rounds = cdiv(total, kVx);
-  int64_t splits = cdiv(2 * kComputeUnits, tiles);  // every split writes a whole fp32 slice: more would be write-bound
-  if (splits > rounds) splits = rounds;
-  if (splits < 1) splits = 1;
+  const double slice_us = 0.6e-6 * 4 * kTaps * a.csmall * a.cbig;
+  int64_t best = 1;
+  double best_us = 1e30;
+  for (int64_t s = 1; s <= rounds && (s == 1 || s * tiles <= kComputeUnits); s = s < 8 ? 2 * s : s + 8) {
+    const double us = 0.7 * (double)(cdiv(s * tiles, kComputeUnits) * cdiv(cdiv(rounds, s), 2)) + slice_us * (double)s;
+    if (us < best_us) { best_us = us; best = s; }
+  }
   ReducePlan p;
-  p.per_split = cdiv(rounds, splits) * kVx;
+  p.per_split = cdiv(rounds, best) * kVx;
   p.splits = (int)cdiv(total, p.per_split);
   return p;
 }
@@ -727,19 +823,21 @@ template <typename T>
 int launch_reduce(const PatchArgs& a, const void* small, const void* big, void* g, int g_dtype, void* ws, hipStream_t st, void* gb) {
   const ReducePlan p = reduce_plan(a);
   const int64_t total = small_voxels(a);
-  const dim3 grid((unsigned)p.splits, (unsigned)(a.csmall / kSmallTile), (unsigned)(a.cbig / 32));
+  const int64_t tiles = (int64_t)(a.csmall / kSmallTile) * (a.cbig / 32);
+  const int by_xcd = p.splits > 4;
+  const dim3 grid((unsigned)((by_xcd ? cdiv(p.splits, kXcds) * kXcds : p.splits) * tiles));
   const int64_t nelem = (int64_t)a.csmall * kTaps * a.cbig;
   float* bias_part = (float*)ws + (int64_t)p.splits * nelem;  // behind the weight slices
   if (gb != nullptr)
-    hipLaunchKernelGGL((patch_reduce_kernel<T, true>), grid, dim3(256), 0, st, a, (const T*)small, (const T*)big, (float*)ws, total,
-                       p.per_split, bias_part);
+    hipLaunchKernelGGL((patch_reduce_kernel<T, true>), grid, dim3(512), 0, st, a, (const T*)small, (const T*)big, (float*)ws, total,
+                       p.per_split, p.splits, by_xcd, bias_part);
   else
-    hipLaunchKernelGGL((patch_reduce_kernel<T, false>), grid, dim3(256), 0, st, a, (const T*)small, (const T*)big, (float*)ws, total,
-                       p.per_split, (float*)nullptr);
+    hipLaunchKernelGGL((patch_reduce_kernel<T, false>), grid, dim3(512), 0, st, a, (const T*)small, (const T*)big, (float*)ws, total,
+                       p.per_split, p.splits, by_xcd, (float*)nullptr);
   if (int rc = check_launch("patch_reduce_kernel")) return rc;
   if (gb == nullptr) return sum_slices(g_dtype, (const float*)ws, g, nelem, p.splits, st);
-  // both sums in one launch; the bias partials are [split][tap][channel]: slices of cbig elements
-  return sum_slices_two(g_dtype, (const float*)ws, g, nelem, p.splits, bias_part, gb, a.cbig, p.splits * kTaps, st);
+  // both sums in one launch
+  return sum_slices_two(g_dtype, (const float*)ws, g, nelem, p.splits, bias_part, gb, a.cbig, p.splits, st);
 }
 
 bool geometry_ok(const PatchArgs& a, int dtype) {
@@ -785,7 +883,7 @@ int patch_reduce_splits(const PatchArgs& a) { return reduce_plan(a).splits; }
 
 size_t patch_reduce_workspace_bytes(const PatchArgs& a, bool with_bias) {
   const size_t splits = (size_t)reduce_plan(a).splits;
-  return splits * a.csmall * kTaps * a.cbig * sizeof(float) + (with_bias ? splits * kTaps * a.cbig * sizeof(float) : 0);
+  return splits * a.csmall * kTaps * a.cbig * sizeof(float) + (with_bias ? splits * a.cbig * sizeof(float) : 0);
 }
 
 int patch_reduce(const PatchArgs& a, int dtype, const void* small, const void* big, void* g, int g_dtype, void* ws, hipStream_t st,

@@ -90,3 +90,32 @@ def test_backward_data(n, cin, cout, extents, odd, dtype):
     if not odd:
         gx = sa.conv_transpose3d_backward_data(big, wt, (n, cin, d, h, w), 2)
         _close(gx.permute(0, 2, 3, 4, 1).reshape(-1, cin), want - b.double(), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,cin,cout,extents", [
+    (1, 64, 32, (1, 1, 1)),           # one voxel: one split, one half idle
+    (1, 64, 32, (3, 3, 5)),           # 45: a cut round in the second half
+    (1, 128, 96, (9, 10, 11)),        # six tiles
+    (2, 128, 64, (11, 15, 18)),       # a range of voxels per XCD, the last one short
+    (1, 512, 256, (4, 8, 8)),         # 64 tiles, one split
+    (1, 512, 256, (5, 9, 9)),         # two splits
+    (1, 64, 32, (33, 36, 36)),
+    (1, 1024, 1056, (2, 2, 2)),       # more tiles than compute units
+])
+def test_backward_weight(n, cin, cout, extents, dtype):
+    from scaffold_amd import transposed as ct
+
+    x, gy, wt, _ = _operands(n, cin, cout, extents, dtype)
+    d, h, w = extents
+    big = gy.double().reshape(n, cout, d, 2, h, 2, w, 2).permute(0, 2, 4, 6, 3, 5, 7, 1).reshape(n * d * h * w, -1)
+    want = (x.permute(0, 2, 3, 4, 1).reshape(-1, cin).double().t() @ big).view(cin, 2, 2, 2, cout).permute(0, 4, 1, 2, 3)
+    gw = sa.conv_transpose3d_backward_weight(x, wt.shape, gy, 2)
+    _close(gw, want, dtype)
+    fw, fb = ct.conv_transpose3d_backward_weight_bias(x, wt.shape, gy, 2, grad_dtype=torch.float32)
+    # fp32 sums of unit-variance products: 1e-6 of the largest entry covers their round-off at these counts
+    assert (fw.double() - want).abs().max() <= 1e-6 * want.abs().max()
+    bias = gy.double().sum((0, 2, 3, 4))
+    assert (fb.double() - bias).abs().max() <= 1e-6 * gy.double().abs().sum((0, 2, 3, 4)).max()
+    bw, _ = ct.conv_transpose3d_backward_weight_bias(x, wt.shape, gy, 2)
+    assert torch.equal(bw, gw)
