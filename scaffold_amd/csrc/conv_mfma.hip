@@ -345,14 +345,6 @@ __device__ __forceinline__ void pack_piece(const PackJob& j, int64_t idx) {
   *reinterpret_cast<uint4*>(packed + idx * 8) = v;
 }
 
-// Up to two packings of one weight (the forward's and the data gradient's) in one launch.
-template <typename T>
-__global__ void __launch_bounds__(256) pack_weight_kernel(PackJob first, PackJob second) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx < first.pieces) pack_piece<T>(first, idx);
-  else if (idx - first.pieces < second.pieces) pack_piece<T>(second, idx - first.pieces);
-}
-
 // Many packings in one launch: a workgroup finds its job from the table of first workgroups.
 constexpr int kPackBatch = 48;  // (the table stays under 4 KB of kernel arguments)
 struct PackBatch {
@@ -368,6 +360,74 @@ __global__ void __launch_bounds__(256) pack_weight_batch_kernel(PackBatch b) {
   while (j + 1 < b.njobs && (int)blockIdx.x >= b.first_block[j + 1]) ++j;
   const int64_t idx = (int64_t)((int)blockIdx.x - b.first_block[j]) * 256 + threadIdx.x;
   if (idx < b.job[j].pieces) pack_piece<T>(b.job[j], idx);
+}
+
+// Dense channels-last weights [c0][taps][c1] of whole 32-channel blocks, in one read for both forms. A wavefront turns one tile of
+// 32 x 32 channels of one tap through 2 KiB of LDS: the form whose rows are c0 (forward) reads it along c1, the form whose rows are c1
+// (data gradient) with the transposing read. pack_piece above spends some 500 instructions of 64-bit divisions on 16 bytes and
+// gathers the second form two bytes at a time: it is left for every other layout. In us, pack_piece -> tiles,
+// both forms, caches warm: 256 x 256 x 27 5.1 -> 3.6, 512 x 512 x 27 12.8 -> 7.7, 1024 x 512 x 27 22.9 -> 13.8; 32 x 32 x 27 2.75 -> 2.4 (the launch).
+struct TileJob {
+  const void* w;
+  void* rows;  // [c0 / 32][c1 / 32][tap][kstep][lane][8], or null
+  void* cols;  // [c1 / 32][c0 / 32][tap][kstep][lane][8], taps reversed with `flip`, or null
+  int nb0, nb1, taps;
+  uint16_t flip, fp32;
+};
+constexpr int kTileBatch = 72;  // (the table stays under 4 KB of kernel arguments)
+template <int N>
+struct TileBatch {
+  TileJob job[N];
+  int first_block[N + 1];
+  int njobs;
+};
+static_assert(sizeof(TileBatch<kTileBatch>) <= 4096, "kernel arguments");
+
+template <typename T, int N>
+__global__ void __launch_bounds__(256) pack_tiles_kernel(TileBatch<N> b) {
+  __shared__ __attribute__((aligned(16))) T lds[4][32 * 32];
+  int n = 0;
+  while (n + 1 < b.njobs && (int)blockIdx.x >= b.first_block[n + 1]) ++n;
+  const TileJob& j = b.job[n];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t t = (blockIdx.x - (uint32_t)b.first_block[n]) * 4 + wave;
+  const uint32_t b1 = t % (uint32_t)j.nb1, r = t / (uint32_t)j.nb1;
+  const uint32_t tap = r % (uint32_t)j.taps, b0 = r / (uint32_t)j.taps;
+  if (b0 >= (uint32_t)j.nb0) return;  // (wavefronts share nothing)
+  T* tile = lds[wave];
+  const int64_t row_step = (int64_t)j.taps * j.nb1 * 32;
+  const int64_t at = (int64_t)b0 * 32 * row_step + ((int64_t)tap * j.nb1 + b1) * 32;
+  if (j.fp32) {  // an fp32 master weight: rounded here, once
+    const float* src = static_cast<const float*>(j.w) + at + (lane >> 3) * row_step + (lane & 7) * 4;
+    float4 raw[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) raw[i] = *reinterpret_cast<const float4*>(src + 8 * i * row_step);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<uint2*>(tile + (8 * i + (lane >> 3)) * 32 + (lane & 7) * 4) =
+          make_uint2(Mma32<T>::pack2(raw[i].x, raw[i].y), Mma32<T>::pack2(raw[i].z, raw[i].w));
+  } else {
+    const T* src = static_cast<const T*>(j.w) + at + (lane >> 2) * row_step + (lane & 3) * 8;
+    uint4 raw[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) raw[i] = load16(src + 16 * i * row_step);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) *reinterpret_cast<uint4*>(tile + (16 * i + (lane >> 2)) * 32 + (lane & 3) * 8) = raw[i];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (j.rows != nullptr) {
+    T* dst = static_cast<T*>(j.rows) + ((((int64_t)b0 * j.nb1 + b1) * j.taps + tap) * 2 * 64 + lane) * 8;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      *reinterpret_cast<uint4*>(dst + ks * 512) = *reinterpret_cast<const uint4*>(tile + (lane & 31) * 32 + ks * 16 + (lane >> 5) * 8);
+  }
+  if (j.cols != nullptr) {
+    const uint32_t to = j.flip ? j.taps - 1 - tap : tap;
+    T* dst = static_cast<T*>(j.cols) + ((((int64_t)b1 * j.nb0 + b0) * j.taps + to) * 2 * 64 + lane) * 8;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) *reinterpret_cast<uint4*>(dst + ks * 512) = tr_fragment<T>(tile + ks * 16 * 32, 32, lane);
+  }
 }
 
 struct GatherPlan { int shape; int nsub; int ksplit; int64_t tiles; };
@@ -534,43 +594,90 @@ PackJob pack_job(const MfmaConvArgs& a, const void* w, int64_t s_out, int64_t s_
   j.pieces = (int64_t)a.cout * a.cred * a.kd * a.kh * a.kw / 8;  // 16-byte pieces
   return j;
 }
-int launch_pack(int dtype, const PackJob& first, const PackJob& second, hipStream_t st) {
-  const int64_t total = first.pieces + second.pieces;
-  if (total <= 0) return SFH_OK;
-  const unsigned blocks = (unsigned)cdiv(total, 256);
-  if (dtype == SFH_BF16) hipLaunchKernelGGL(pack_weight_kernel<bf16_t>, dim3(blocks), dim3(256), 0, st, first, second);
-  else hipLaunchKernelGGL(pack_weight_kernel<fp16_t>, dim3(blocks), dim3(256), 0, st, first, second);
-  return check_launch("pack_weight_kernel");
+
+// The packing as a tile job; false where the weight's layout is not the dense channels-last one.
+bool tile_job(const MfmaPackItem& it, TileJob& out) {
+  const int64_t taps = (int64_t)it.a.kd * it.a.kh * it.a.kw;
+  const bool rows = it.s_red == 1 && it.flip == 0;
+  const int c0 = rows ? it.a.cout : it.a.cred, c1 = rows ? it.a.cred : it.a.cout;
+  if (c0 % 32 != 0 || c1 % 32 != 0 || (reinterpret_cast<uintptr_t>(it.w) & 15) != 0) return false;
+  if ((rows ? it.s_red : it.s_out) != 1 || (rows ? it.s_out : it.s_red) != taps * c1) return false;
+  if (it.s_kw != c1 || it.s_kh != (int64_t)it.a.kw * c1 || it.s_kd != (int64_t)it.a.kh * it.a.kw * c1) return false;
+  out = TileJob{it.w, rows ? it.packed : nullptr, rows ? nullptr : it.packed, c0 / 32, c1 / 32, (int)taps,
+                (uint16_t)(it.flip ? 1 : 0), (uint16_t)(it.fp32_source ? 1 : 0)};
+  return true;
+}
+
+int launch_tiles(int dtype, TileBatch<kTileBatch>& b, int64_t blocks, hipStream_t st) {
+  if (b.njobs == 0) return SFH_OK;
+  if (blocks > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv3d pack: batch too large");
+  b.first_block[b.njobs] = (int)blocks;
+  if (b.njobs == 1) {  // one weight: no table to copy
+    const TileBatch<1> one{{b.job[0]}, {0, (int)blocks}, 1};
+    if (dtype == SFH_BF16) hipLaunchKernelGGL((pack_tiles_kernel<bf16_t, 1>), dim3((unsigned)blocks), dim3(256), 0, st, one);
+    else hipLaunchKernelGGL((pack_tiles_kernel<fp16_t, 1>), dim3((unsigned)blocks), dim3(256), 0, st, one);
+  } else {
+    if (dtype == SFH_BF16) hipLaunchKernelGGL((pack_tiles_kernel<bf16_t, kTileBatch>), dim3((unsigned)blocks), dim3(256), 0, st, b);
+    else hipLaunchKernelGGL((pack_tiles_kernel<fp16_t, kTileBatch>), dim3((unsigned)blocks), dim3(256), 0, st, b);
+  }
+  return check_launch("pack_tiles_kernel");
+}
+
+int launch_pieces(int dtype, PackBatch& b, int64_t blocks, hipStream_t st) {
+  if (b.njobs == 0) return SFH_OK;
+  if (blocks > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv3d pack: batch too large");
+  b.first_block[b.njobs] = (int)blocks;
+  if (dtype == SFH_BF16) hipLaunchKernelGGL(pack_weight_batch_kernel<bf16_t>, dim3((unsigned)blocks), dim3(256), 0, st, b);
+  else hipLaunchKernelGGL(pack_weight_batch_kernel<fp16_t>, dim3((unsigned)blocks), dim3(256), 0, st, b);
+  return check_launch("pack_weight_batch_kernel");
 }
 }  // namespace
 
 int mfma_pack_weight(const MfmaConvArgs& a, int dtype, const void* w, int64_t s_out, int64_t s_red, int64_t s_kd, int64_t s_kh,
                      int64_t s_kw, int flip, void* packed, hipStream_t st) {
-  PackJob none{};
-  return launch_pack(dtype, pack_job(a, w, s_out, s_red, s_kd, s_kh, s_kw, flip, packed), none, st);
+  const MfmaPackItem item{a, w, s_out, s_red, s_kd, s_kh, s_kw, flip, packed, false};
+  return mfma_pack_weight_batch(&item, 1, dtype, st);
 }
 
 int mfma_pack_weight_batch(const MfmaPackItem* items, int n, int dtype, hipStream_t st) {
-  for (int i0 = 0; i0 < n; i0 += kPackBatch) {
-    PackBatch b{};
-    int64_t blocks = 0;
-    for (int i = i0; i < n && i < i0 + kPackBatch; ++i) {
-      const MfmaPackItem& it = items[i];
-      const PackJob job = pack_job(it.a, it.w, it.s_out, it.s_red, it.s_kd, it.s_kh, it.s_kw, it.flip, it.packed, it.fp32_source);
-      if (job.pieces <= 0) continue;
-      b.job[b.njobs] = job;
-      b.first_block[b.njobs] = (int)blocks;
-      blocks += cdiv(job.pieces, 256);
-      ++b.njobs;
-      if (blocks > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv3d pack: batch too large");
+  TileBatch<kTileBatch> tiles{};
+  PackBatch pieces{};
+  int64_t tile_blocks = 0, piece_blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    const MfmaPackItem& it = items[i];
+    const PackJob job = pack_job(it.a, it.w, it.s_out, it.s_red, it.s_kd, it.s_kh, it.s_kw, it.flip, it.packed, it.fp32_source);
+    if (job.pieces <= 0) continue;
+    TileJob tile;
+    if (tile_job(it, tile)) {
+      TileJob* last = tiles.njobs > 0 ? &tiles.job[tiles.njobs - 1] : nullptr;
+      if (last != nullptr && last->w == tile.w && last->nb0 == tile.nb0 && last->nb1 == tile.nb1 && last->taps == tile.taps &&
+          last->fp32 == tile.fp32 && last->cols == nullptr && tile.rows == nullptr) {  // the weight's other form
+        last->cols = tile.cols;
+        last->flip = tile.flip;
+        continue;
+      }
+      if (tiles.njobs == kTileBatch) {
+        if (int rc = launch_tiles(dtype, tiles, tile_blocks, st)) return rc;
+        tiles = TileBatch<kTileBatch>{};
+        tile_blocks = 0;
+      }
+      tiles.job[tiles.njobs] = tile;
+      tiles.first_block[tiles.njobs++] = (int)tile_blocks;
+      tile_blocks += cdiv((int64_t)tile.nb0 * tile.nb1 * tile.taps, 4);
+    } else {
+      if (pieces.njobs == kPackBatch) {
+        if (int rc = launch_pieces(dtype, pieces, piece_blocks, st)) return rc;
+        pieces = PackBatch{};
+        piece_blocks = 0;
+      }
+      pieces.job[pieces.njobs] = job;
+      pieces.first_block[pieces.njobs++] = (int)piece_blocks;
+      piece_blocks += cdiv(job.pieces, 256);
     }
-    b.first_block[b.njobs] = (int)blocks;
-    if (b.njobs == 0) continue;
-    if (dtype == SFH_BF16) hipLaunchKernelGGL(pack_weight_batch_kernel<bf16_t>, dim3((unsigned)blocks), dim3(256), 0, st, b);
-    else hipLaunchKernelGGL(pack_weight_batch_kernel<fp16_t>, dim3((unsigned)blocks), dim3(256), 0, st, b);
-    if (int rc = check_launch("pack_weight_batch_kernel")) return rc;
+    if (tile_blocks > 0x7fffffffLL || piece_blocks > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv3d pack: batch too large");
   }
-  return SFH_OK;
+  if (int rc = launch_tiles(dtype, tiles, tile_blocks, st)) return rc;
+  return launch_pieces(dtype, pieces, piece_blocks, st);
 }
 
 size_t mfma_conv_partial_bytes(const MfmaConvArgs& a) {

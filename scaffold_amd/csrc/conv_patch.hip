@@ -75,28 +75,6 @@ struct VoxelWalk {
   }
 };
 
-// Operand fragment (32 channels x 16 voxels) from a natural-layout LDS tile: `tile` points at the first
-// of the 16 voxel rows, channel 0 of the block. Within each group of 16 lanes the transposing read takes
-// lane m's address as (voxel m / 4, channels 4 * (m % 4) .. + 3) and returns to lane m channel m of the
-// four voxels, so two reads give a lane its 8 voxels of the k-step.
-template <typename T>
-__device__ __forceinline__ uint4 tr_fragment(const T* tile, int row_stride, int lane) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef short v4s __attribute__((__vector_size__(4 * sizeof(short))));
-  const int g = lane >> 4, m = lane & 15;
-  const T* p0 = tile + ((g >> 1) * 8 + (m >> 2)) * row_stride + (g & 1) * 16 + 4 * (m & 3);
-  const T* p1 = p0 + 4 * row_stride;
-  const v4s r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(p0));
-  const v4s r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(p1));
-  uint4 out;
-  out.x = __builtin_bit_cast(uint2, r0).x; out.y = __builtin_bit_cast(uint2, r0).y;
-  out.z = __builtin_bit_cast(uint2, r1).x; out.w = __builtin_bit_cast(uint2, r1).y;
-  return out;
-#else
-  return make_uint4(0, 0, 0, 0);
-#endif
-}
-
 // ---- gather: stride-2 convolution --------------------------------------------------------------
 // The kept form. A wavefront owns one block of 32 small channels and KEEPS its weights in registers -- all eight taps of cbig
 // channels, those of a depth tap (KH = 2) or of a row of the patch (KH = 4) -- while its workgroup walks tiles of 32 * VS
