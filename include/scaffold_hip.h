@@ -115,7 +115,8 @@ int sfh_conv3d_out_shape(const sfh_conv3d_desc* p, int32_t out_dhw[3]);
 int sfh_conv3d_uses_mfma(const sfh_conv3d_desc* p, int dtype, int direction);
 /* Which kernel serves a problem in a direction (0 forward, 1 data-gradient, 2 weight-gradient) and with what launch
  * geometry: geometry[0] = SFH_KERNEL_*, [1] = output voxels per workgroup step, [2] = 32-channel output blocks a
- * workgroup produces from one staged brick, [3] = slices of the reduction (channels for forward / data-gradient,
+ * workgroup produces from one staged brick (SFH_KERNEL_SPLIT: the pair, which a launch that would leave half of the compute
+ * units idle deals to two workgroups), [3] = slices of the reduction (channels for forward / data-gradient,
  * voxels for the weight gradient) whose fp32 partials are summed in fixed order. A pure function of the problem and
  * the compute-unit count the library is written for -- the property the reference's plan machinery exists to
  * guarantee (triton_conv3d/_rungs.py, reduce_gemm.py:71-96: the split count must not depend on the device or the

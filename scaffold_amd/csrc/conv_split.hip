@@ -7,7 +7,8 @@
 // of their own. Here the reduction is cut INSIDE the workgroup:
 //
 //   * A workgroup owns a brick of only 2 x 4 x 8 = 64 output voxels and 64 produced channels -- four 32-voxel x
-//     32-channel accumulator blocks -- so even a level of 2048 voxels has 32 x Cout/64 of them.
+//     32-channel accumulator blocks -- so even a level of 2048 voxels has 32 x Cout/64 of them; where those would leave
+//     half of the CUs idle, 32 produced channels.
 //   * Its four wavefronts split the REDUCTION, not the voxels: a round stages the halo bricks of R 32-channel chunks
 //     (R = 4, or 2 when there are only two) side by side in LDS, and every wavefront runs all four accumulator blocks
 //     over its own share -- one chunk each, or half a chunk's k-steps each when R = 2. A weight fragment then feeds
@@ -33,23 +34,30 @@ constexpr int kChunk = 32;
 constexpr int TD = 2, TH = 4, TW = 8;  // output brick: two planes of 4 x 8 voxels, each one MFMA column block
 constexpr int BD = TD + 2, BH = TH + 2, BW = TW + 2;
 constexpr int BV = BD * BH * BW;  // 240 brick voxels with the halo
-constexpr int PLANE = ((BV * 16 - 64 + 255) / 256) * 256 + 64;  // >= BV * 16, 64 modulo 256
-constexpr int SLOT = 4 * PLANE + 16;                            // one chunk's brick
-constexpr int MS = 2, NSUB = 2;                                 // accumulator blocks: voxel halves x channel halves
+constexpr int MS = 2, kBlocks = 2;                              // accumulator blocks: voxel halves x at most two channel blocks
 constexpr int TAPS = 27, NIT = TAPS * 2, FRAG = 512;
-constexpr int RED_BYTES = 4 * 3 * 4096;  // every block from the three wavefronts that do not own it
-static_assert(PLANE % 256 == 64 && PLANE >= BV * 16, "plane stride");
-
-// LDS byte offset of (tap, k-step) relative to a lane's voxel at tap (0, 0, 0)
-constexpr int tap_off(int tap) { return (((tap / 9) * BH + (tap / 3) % 3) * BW + tap % 3) * 16; }
+// LDS of a chunk's brick, NSUB channel blocks to a workgroup: row pitch, channel plane (64 modulo 256), chunk slot. A fragment
+// read covers two rows at a time; 128 modulo 256 apart they share no bank. Two workgroups to a CU (NSUB = 2) have no room
+// for that pitch, and do not miss it; alone on its CU one reads 5 % faster (13.8 -> 13.1 us at 256 -> 256, 8x16x16).
+template <int NSUB>
+struct Brick {
+  static constexpr int ROW = NSUB == 1 ? 384 : BW * 16;
+  static constexpr int PLANE = ((BD * BH * ROW - 64 + 255) / 256) * 256 + 64;
+  static constexpr int SLOT = 4 * PLANE + 16;
+  // byte offset of (tap, k-step) relative to a lane's voxel at tap (0, 0, 0)
+  static constexpr int tap_off(int tap) { return ((tap / 9) * BH + (tap / 3) % 3) * ROW + tap % 3 * 16; }
+};
 
 // R: chunks per round. PAIR: the input is two tensors whose channels follow each other (the first `c_first` in x, the
 // rest in x1). Independently, a non-null y1 splits the OUTPUT the same way.
-template <typename T, int R, bool PAIR>
+template <typename T, int R, int NSUB, bool PAIR>
 __global__ void __launch_bounds__(256, 2)
 conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ wp, const T* __restrict__ bias, T* __restrict__ y,
                   int tiles_d, int tiles_h, int tiles_w, int nblocks, uint32_t total, GnPartialOut gn, const T* __restrict__ x1,
                   T* __restrict__ y1, int c_first) {
+  using B = Brick<NSUB>;
+  constexpr int PLANE = B::PLANE, SLOT = B::SLOT;
+  constexpr int RED_BYTES = MS * NSUB * 3 * 4096;  // every block from the three wavefronts that do not own it
   constexpr int LDS = R * SLOT > RED_BYTES ? R * SLOT : RED_BYTES;
   __shared__ __attribute__((aligned(16))) char lds[LDS];
   const int tid = threadIdx.x;
@@ -73,9 +81,9 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
 #pragma unroll
   for (int ms = 0; ms < MS; ++ms) {
     const int tw = j % TW, th = j / TW;
-    abase[ms] = slot * SLOT + (kg + 2 * khalf) * PLANE + ((ms * BH + th) * BW + tw) * 16;
+    abase[ms] = slot * SLOT + (kg + 2 * khalf) * PLANE + (ms * BH + th) * B::ROW + tw * 16;
   }
-  auto a_off = [](int k) constexpr { return R == 4 ? tap_off(k / 2) + (k % 2) * 2 * PLANE : tap_off(k); };
+  auto a_off = [](int k) constexpr { return R == 4 ? B::tap_off(k / 2) + (k % 2) * 2 * PLANE : B::tap_off(k); };
 
   f32x16_t acc[MS][NSUB];
 #pragma unroll
@@ -89,7 +97,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   const int id0 = od0 - a.pd, ih0 = oh0 - a.ph, iw0 = ow0 - a.pw;
   constexpr int PIECES = BV * 4 * R;
   constexpr int ITERS = (PIECES + 255) / 256;
-  constexpr int WDEPTH = 8;  // weight fragments (per output block) in flight per wavefront
+  constexpr int WDEPTH = 16 / NSUB;  // weight fragments (per output block) in flight per wavefront
   const int64_t wns = (int64_t)ncc * (NIT * FRAG);  // next 32-channel output block
 
   for (int c0 = 0; c0 < ncc; c0 += R) {
@@ -127,7 +135,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
       for (int u = 0; u < ITERS; ++u) {
         const int p = u * 256 + tid;
         const int q = p % (4 * R), vox = p / (4 * R);
-        if (p < PIECES) *reinterpret_cast<uint4*>(lds + (q >> 2) * SLOT + (q & 3) * PLANE + vox * 16) = v[u];
+        if (p < PIECES) *reinterpret_cast<uint4*>(lds + (q >> 2) * SLOT + (q & 3) * PLANE + vox / BW * B::ROW + vox % BW * 16) = v[u];
       }
     }
     __syncthreads();
@@ -145,10 +153,10 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
         const int ms = m / NSUB, ns = m % NSUB;
         acc[ms][ns] = Mma32<T>::run(wq[k][ns], aq[k & 1][ms], acc[ms][ns]);
         __builtin_amdgcn_sched_barrier(0);
-        if (m < NSUB) {
-          if (k + WDEPTH < NITS) wq[k + WDEPTH][m] = *reinterpret_cast<const uint4*>(wcc + m * wns + (k + WDEPTH) * WSTEP);
-        } else {
-          if (k + 1 < NITS) aq[(k + 1) & 1][m - NSUB] = *reinterpret_cast<const uint4*>(lds + abase[m - NSUB] + a_off(k + 1));
+        if (m < NSUB && k + WDEPTH < NITS) wq[k + WDEPTH][m] = *reinterpret_cast<const uint4*>(wcc + m * wns + (k + WDEPTH) * WSTEP);
+        if (NSUB == 1 ? true : m >= NSUB) {
+          constexpr int first = NSUB == 1 ? 0 : NSUB;
+          if (k + 1 < NITS) aq[(k + 1) & 1][m - first] = *reinterpret_cast<const uint4*>(lds + abase[m - first] + a_off(k + 1));
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -159,7 +167,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   __syncthreads();  // the bricks are not read any more
   float4* red = reinterpret_cast<float4*>(lds);
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < MS * NSUB; ++u) {
     if (u != wave) {
       const int from = wave < u ? wave : wave - 1;  // this wavefront's place among block u's three senders
 #pragma unroll
@@ -174,7 +182,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
 #pragma unroll
   for (int r = 0; r < 16; ++r) tot[r] = 0.f;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < MS * NSUB; ++u) {
     if (u == wave) {
       // wavefronts 0, 1, 2, 3 in that order, this one's own share from its registers
 #pragma unroll
@@ -202,9 +210,10 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   // 8 * (r / 4) + 4 * kg + r % 4 of voxel j of the block row; the two lanes of a voxel trade runs so that each stores
   // two 16-byte pieces.
   const int ms_o = wave / NSUB, ns_o = wave % NSUB;
+  const bool owns = MS * NSUB == 4 || wave < MS * NSUB;
   const int tw = j % TW, th = j / TW;
   const int od = od0 + ms_o, oh = oh0 + th, ow = ow0 + tw;
-  const bool inside = od < a.od && oh < a.oh && ow < a.ow;
+  const bool inside = owns && od < a.od && oh < a.oh && ow < a.ow;
   const int64_t vox = (((int64_t)n * a.od + od) * a.oh + oh) * a.ow + ow;
   const int ch = (nb * NSUB + ns_o) * 32;
   T* yp = y + vox * a.cout + ch;
@@ -234,7 +243,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
     RunSums rs[NSUB];
 #pragma unroll
     for (int ns = 0; ns < NSUB; ++ns) {
-      const bool own = ns == ns_o;
+      const bool own = owns && ns == ns_o;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         rs[ns].s1[g] = own ? mine.s1[g] : 0.f;
@@ -253,7 +262,13 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
 
 int64_t split_tiles(const MfmaConvArgs& a) { return (int64_t)a.n * cdiv(a.od, TD) * cdiv(a.oh, TH) * cdiv(a.ow, TW); }
 
-template <typename T, int R, bool PAIR>
+// One channel block per workgroup where pairs would leave half of the CUs idle: each workgroup then has half the weights to fetch and
+// half the MFMAs (the bits of the output do not depend on it). us, caches warm / cold: 256 -> 256 at 8x16x16 16.0 / 18.9 -> 13.1 / 16.2,
+// 128 -> 256 10.2 / 13.8 -> 8.7 / 11.4, 256 -> 256 at 5x7x9 (two samples) 15.0 / 20.5 -> 11.8 / 15.1. With 129 to 256 pairs it loses:
+// 256 -> 256 at 10x16x16 16.5 / 22.0 -> 19.2 / 22.2, at 16^3 17.6 -> 19.6 (each CU fetches the same weights and stages twice the bricks).
+int split_blocks(const MfmaConvArgs& a) { return split_tiles(a) * (a.cout / (32 * kBlocks)) <= kComputeUnits / 2 ? 1 : kBlocks; }
+
+template <typename T, int R, int NSUB, bool PAIR>
 int launch_split(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                  const GnPartialOut& gn, const void* x1, void* y1, int first) {
   const int tiles_d = (int)cdiv(a.od, TD), tiles_h = (int)cdiv(a.oh, TH), tiles_w = (int)cdiv(a.ow, TW);
@@ -261,7 +276,7 @@ int launch_split(const MfmaConvArgs& a, const void* x, const void* packed, const
   const int64_t total = split_tiles(a) * nblocks;
   if (total == 0) return SFH_OK;
   if (total > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv split: %lld workgroups exceed the grid limit", (long long)total);
-  hipLaunchKernelGGL((conv_split_kernel<T, R, PAIR>), dim3((unsigned)total), dim3(256), 0, st, a, (const T*)x, (const T*)packed,
+  hipLaunchKernelGGL((conv_split_kernel<T, R, NSUB, PAIR>), dim3((unsigned)total), dim3(256), 0, st, a, (const T*)x, (const T*)packed,
                      (const T*)bias, (T*)y, tiles_d, tiles_h, tiles_w, nblocks, (uint32_t)total, gn, (const T*)x1, (T*)y1, first);
   return check_launch("conv_split_kernel");
 }
@@ -270,11 +285,13 @@ template <typename T>
 int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                        const GnPartialOut& gn, const void* x1, void* y1, int first) {
   const bool four = (a.cred / kChunk) % 4 == 0;
-  if (x1 != nullptr)
-    return four ? launch_split<T, 4, true>(a, x, packed, bias, y, st, gn, x1, y1, first)
-                : launch_split<T, 2, true>(a, x, packed, bias, y, st, gn, x1, y1, first);
-  return four ? launch_split<T, 4, false>(a, x, packed, bias, y, st, gn, x1, y1, first)
-              : launch_split<T, 2, false>(a, x, packed, bias, y, st, gn, x1, y1, first);
+#define SFH_SPLIT(NSUB)                                                                                \
+  x1 != nullptr ? (four ? launch_split<T, 4, NSUB, true>(a, x, packed, bias, y, st, gn, x1, y1, first)   \
+                        : launch_split<T, 2, NSUB, true>(a, x, packed, bias, y, st, gn, x1, y1, first))  \
+                : (four ? launch_split<T, 4, NSUB, false>(a, x, packed, bias, y, st, gn, x1, y1, first)  \
+                        : launch_split<T, 2, NSUB, false>(a, x, packed, bias, y, st, gn, x1, y1, first))
+  return split_blocks(a) == 1 ? SFH_SPLIT(1) : SFH_SPLIT(2);
+#undef SFH_SPLIT
 }
 
 }  // namespace
@@ -288,23 +305,32 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
 // reason it leaves reductions of 512 channels or more to the slices where its workgroups would number 32 or fewer per
 // two planes (8 x 16 x 16 with 256 produced channels: 128 workgroups of 1.7 MiB of weights each, 41 us against 30 with
 // the weights cold; eight wavefronts per workgroup instead of four changed nothing, which is how the bound was found).
-// The rule does not look at the depth: the data gradient of a depth shard's slab (D + 2 planes) and of the padded volume
-// (D planes) must come from the same kernel, or a shard and the whole volume would disagree in the last bit.
+// That line looks at a plane only; volumes below it come here too once pairs of blocks number a quarter of the CUs (a
+// workgroup of one block needs no slices and no launch that sums them). us, slices and their sum -> here: 64 -> 64 at 16^3 10.4 -> 5.6,
+// 64 -> 128 at 16^3 11.9 -> 6.0, 128 -> 128 at 16^3 14.9 -> 8.6, 256 -> 128 at 20x12x14 22 -> 12.5, 512 -> 256 at 16^3 44 -> 32. Few pairs of a
+// long reduction lose (512 -> 512 at 8^3, 64 pairs: 17.4 -> 23.2; 256 -> 256 at 4x8x8, 16 pairs: 10.1 -> 10.6), so the line is higher for
+// those. Some below it would gain as well (128 -> 128 at 8^3, 16 pairs: 9.7 -> 7.7; 256 -> 128 at 8x16x16, 64: 14.9 -> 11.4; 512 -> 256 at
+// 8x16x16, 128: 27.8 -> 22.9): they keep the geometry that the launch query has stated for them and that callers may have sized by.
+// The data gradient of a depth shard's slab (D + 2 planes from D) and of the padded volume (D from D) must come from the same
+// kernel, or a shard and the whole volume would disagree in the last bit: the depth counted is the smaller of the two.
 constexpr int kSplitMaxPlane = 32 * 32, kSplitMinPerDepth = 24, kSplitFewPerDepth = 32, kSplitFewMaxChunks = 16;
 
 bool mfma_conv_split_applies(const MfmaConvArgs& a) {
   if (a.kd != 3 || a.kh != 3 || a.kw != 3) return false;
-  if (a.cred < 2 * kChunk || a.cred % (2 * kChunk) != 0 || a.cout % (32 * NSUB) != 0) return false;
+  if (a.cred < 2 * kChunk || a.cred % (2 * kChunk) != 0 || a.cout % (32 * kBlocks) != 0) return false;
   if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return false;
-  const int64_t per_depth = (int64_t)a.n * cdiv(a.oh, TH) * cdiv(a.ow, TW) * (a.cout / (32 * NSUB));
-  if (per_depth <= kSplitFewPerDepth && a.cred / kChunk >= kSplitFewMaxChunks) return false;
+  const int64_t per_depth = (int64_t)a.n * cdiv(a.oh, TH) * cdiv(a.ow, TW) * (a.cout / (32 * kBlocks));
+  const int chunks = a.cred / kChunk;
+  const int64_t pairs = per_depth * cdiv(a.id < a.od ? a.id : a.od, TD);
+  if (chunks <= 4 ? pairs >= kComputeUnits / 4 : pairs > (chunks <= 8 ? kComputeUnits / 4 : kComputeUnits / 2)) return true;
+  if (per_depth <= kSplitFewPerDepth && chunks >= kSplitFewMaxChunks) return false;
   return per_depth >= kSplitMinPerDepth;
 }
 
-MfmaConvGeometry mfma_conv_split_geometry(const MfmaConvArgs&) { return MfmaConvGeometry{kKernelSplit, TD * TH * TW, NSUB, 1}; }
+MfmaConvGeometry mfma_conv_split_geometry(const MfmaConvArgs&) { return MfmaConvGeometry{kKernelSplit, TD * TH * TW, kBlocks, 1}; }
 
 int mfma_conv_split_gn_records(const MfmaConvArgs& a, int groups) {
-  const int span = 32 * NSUB;
+  const int span = 32 * split_blocks(a);
   if (!gn_partials_fit(a.cout, groups, span)) return 0;
   const int cg = a.cout / groups;
   const int64_t records = split_tiles(a) / a.n * (cg > span ? cg / span : 1);
