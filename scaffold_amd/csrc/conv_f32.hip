@@ -211,13 +211,20 @@ pack_f32_kernel(const float* __restrict__ w, float* __restrict__ packed, int cre
                 int64_t s_red, int64_t s_kd, int64_t s_kh, int64_t s_kw, int64_t pieces) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= pieces) return;
-  int64_t r = idx;
-  const int lane = (int)(r % 64); r /= 64;
-  const int q = (int)(r % 2); r /= 2;
-  int tap = (int)(r % kTaps); r /= kTaps;
+  const int lane = (int)(idx % 64), q = (int)(idx / 64 % 2);
   const int ncc = cred / kChunk;
-  const int cc = (int)(r % ncc);
-  const int nblk = (int)(r / ncc);
+  int tap, cc, nblk;
+  if (pieces <= 0x7fffffff) {  // (64-bit divisions by numbers that are not constants would be most of the kernel)
+    uint32_t r = (uint32_t)idx / 128u;
+    tap = (int)(r % kTaps); r /= kTaps;
+    cc = (int)(r % (uint32_t)ncc);
+    nblk = (int)(r / (uint32_t)ncc);
+  } else {
+    int64_t r = idx / 128;
+    tap = (int)(r % kTaps); r /= kTaps;
+    cc = (int)(r % ncc);
+    nblk = (int)(r / ncc);
+  }
   const int co = nblk * 32 + (lane & 31);
   const int ci = cc * kChunk + (lane >> 5) * 8 + q * 4;
   if (flip) tap = kTaps - 1 - tap;
@@ -243,115 +250,146 @@ int launch(const MfmaConvArgs& a, const void* x, const void* packed, const void*
 // GEMM view (triton_conv3d/reduce_gemm.py:137-393): M = Cout, N = 27 x Cin, K = output voxels. One fp32 MFMA contracts
 // TWO voxels and a lane supplies ONE value per operand: row operand gy[voxel 2s + kg][co = lane % 32], column operand
 // x[that voxel + tap][ci = lane % 32] -- both are 32 consecutive floats of a channels-last row, so unlike the 16-bit
-// kernel nothing has to be transposed and the operands come straight from global memory (L1 / L2 serve the 27-fold
-// reuse of x). A workgroup owns one (32 co, 32 ci) block and a contiguous range of passes (8 voxels of an output row); its
-// wavefronts split the 27 taps 7 / 7 / 7 / 6. Split-K over the passes: fp32 partial slices [Cout][27][Cin] at fixed workspace slots,
-// summed in fixed order afterwards (reduce_gemm.py:396-435) -- no float atomics, split count a pure function of shape.
+// kernel nothing has to be transposed. A workgroup owns the nine taps of one kd of a (32 co, 32 ci) block and a range of steps; a
+// step is 64 voxels of the output, four rows of 16, whose gy and whose x rows with their halo lie in LDS as they lie in memory. Its twelve
+// wavefronts are three kh x the rows; along W the taps share operands (a pair of kw = 2 is the next pair of kw = 0), so three
+// MFMAs take three LDS reads. The rows meet in LDS before the slice is written. Split-K over the steps: fp32 partial slices
+// [Cout][27][Cin] at fixed workspace slots, summed in fixed order afterwards (reduce_gemm.py:396-435) -- no float atomics,
+// split count a pure function of shape.
 //
-// What bounds it at 32^3 and below is not the matrix pipe but the slices (110 KB each, written and read again) and the trip
-// to memory in front of every pass. So a workgroup is eight wavefronts, two to a tap range: they take the passes of the
-// range in turn and meet in LDS (114 KB) before the slice is written, which gives the same wavefronts per CU from half of
-// the slices; a pass's operands are requested while the pass before it computes.
-// 32 -> 32 channels on 32^3: kernel 42.1 -> 35.4 us (its MFMAs alone 11.5), slice sum 9.8 -> 5.9.  One set of eight wavefronts
-// without the requests ahead: 45.6.
-constexpr int kPairsPerPass = 4;  // voxel pairs of a pass
-constexpr int kPassVoxels = 2 * kPairsPerPass;
-constexpr uint32_t kOutside = 0x7ffffff0;  // an offset behind every row (f32_wgrad_supported)
+// What bounds it is the matrix pipe, below 64^3 with the launch, the first step's trip to memory and the slices (36 KB a
+// workgroup). Before, a lane's value per operand was a load of its own, 1.14 per MFMA: the CU's address path needs as long for one as
+// its matrix pipes for an MFMA, and a workgroup owned all taps, three times the slices. us with the slice sum, before -> now:
+// 32 -> 32 channels at 32^3 45.6 -> 34.0, at 16x24x20 29.4 -> 17.7, at 64^3 (two samples) 384 -> 293 (its MFMAs alone 188); 64 -> 64 at 64^3
+// 752 -> 578; 128 -> 128 at 16^3 67 -> 49; 256 -> 256 at 8x16x16 114 -> 97; 512 -> 512 at 4x8x8 56.6 -> 52.
+constexpr int kRowWaves = 4;                  // wavefronts that share the rows of a step
+constexpr int kWgradThreads = 64 * 3 * kRowWaves;
+typedef float Quad __attribute__((ext_vector_type(4), aligned(4)));  // the operands may be views 4 bytes off the 16-byte grid
 
-struct PassOperands {
-  float gy[kPairsPerPass], x[kPairsPerPass][7];
-};
-
-__global__ void __launch_bounds__(512, 2)
-wgrad_f32_kernel(WgradArgs a, const float* __restrict__ x, const float* __restrict__ gy, float* __restrict__ partial, int nsplit, int cibs) {
-  __shared__ float meet[4][7 * 16][64];
+// SEG: voxels of a step's rows, 16, or 8 with twice the rows where a row has no more.
+template <int SEG>
+__global__ void __launch_bounds__(kWgradThreads, 3)
+wgrad_f32_kernel(WgradArgs a, const float* __restrict__ x, const float* __restrict__ gy, float* __restrict__ partial, int nsplit, int per,
+                 int steps, int cibs) {
+  constexpr int kRows = kRowWaves * (16 / SEG), kSeg = SEG;
+  constexpr int kXSeg = kSeg + 2, kXPieces = (kRows + 2) * kXSeg * 8, kGyPieces = kRows * kSeg * 8;  // 16-byte pieces of 32 channels
+  constexpr int kPiecesPer = (kXPieces + kGyPieces + kWgradThreads - 1) / kWgradThreads;
+  constexpr int kStep = (kXPieces + kGyPieces) * 16, kMeet = (kRowWaves - 1) * 3 * 3 * 16 * 64 * 4;
+  __shared__ __attribute__((aligned(16))) char lds[2 * kStep > kMeet ? 2 * kStep : kMeet];
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave = wave8 & 3, half = wave8 >> 2;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kh = wave % 3, row = wave / 3;
   const int i = lane & 31, kg = lane >> 5;
   int b = blockIdx.x;
   const int split = b % nsplit; b /= nsplit;
+  const int kd = b % 3; b /= 3;
   const int cib = b % cibs, cob = b / cibs;
-  const int row_passes = (a.ow + kPassVoxels - 1) / kPassVoxels;
-  const int64_t passes = (int64_t)a.n * a.od * a.oh * row_passes;  // below 2^31 (f32_wgrad_supported)
-  const int p_begin = (int)(split * passes / nsplit), p_end = (int)((split + 1) * passes / nsplit);
-  const int ntaps = wave < 3 ? 7 : 6;
-  const int tap0 = wave * 7;
-
-  f32x16_t acc[7];
+  const int segs = (a.ow + kSeg - 1) / kSeg, row_tiles = (a.oh + kRows - 1) / kRows;
+  const int begin = split * per, end = begin + per < steps ? begin + per : steps;
+  // The range's steps in turn, segments first: positions are kept and moved on (all of it scalar), a thread's places in a step and
+  // its offsets from the step's first voxel are constants.
+  const int next_plane = begin / segs / row_tiles;
+  int next_seg = begin % segs, next_tile = begin / segs % row_tiles;
+  int next_od = next_plane % a.od, next_n = next_plane / a.od;
+  int rr[kPiecesPer], vv[kPiecesPer], off[kPiecesPer];
+  bool of_x[kPiecesPer], used[kPiecesPer];
 #pragma unroll
-  for (int t = 0; t < 7; ++t)
+  for (int k = 0; k < kPiecesPer; ++k) {
+    const int p = k * kWgradThreads + tid, q = p - kXPieces;
+    of_x[k] = p < kXPieces;
+    used[k] = q < kGyPieces;
+    rr[k] = of_x[k] ? p / (kXSeg * 8) - a.ph : q / (kSeg * 8);
+    vv[k] = of_x[k] ? p / 8 % kXSeg - a.pw : q / 8 % kSeg;
+    off[k] = of_x[k] ? (rr[k] * a.iw + vv[k]) * a.cin + cib * 32 + (p & 7) * 4 : (rr[k] * a.ow + vv[k]) * a.cout + cob * 32 + (p & 7) * 4;
+  }
+  struct Ahead { float4 piece[kPiecesPer]; int oh, ow; } ahead[2];
+  auto request = [&](Ahead& o) {
+    const int oh = next_tile * kRows, ow = next_seg * kSeg, id = next_od + kd - a.pd;
+    const bool plane_in = (unsigned)id < (unsigned)a.id;
+    const float* xs = x + ((((int64_t)next_n * a.id + id) * a.ih + oh) * a.iw + ow) * a.cin;
+    const float* gs = gy + ((((int64_t)next_n * a.od + next_od) * a.oh + oh) * a.ow + ow) * a.cout;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
-
-  const float* gyb = gy + cob * 32;
-  const float* xb = x + cib * 32;
-  // One buffer per operand row: a voxel outside of it -- padding, the end of a row, a row of padding (no records) -- reads
-  // as zero, with no mask on the loaded value (which would wait for it). A negative offset is as far out as a large one.
-  auto request = [&](int pass, PassOperands& o) {
-    const int row = pass / row_passes, w0 = (pass - row * row_passes) * kPassVoxels;
-    const int plane = row / a.oh, oh = row - plane * a.oh, n = plane / a.od, od = plane - n * a.od;
-    const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(gyb + (int64_t)row * a.ow * a.cout), 0, a.ow * a.cout * 4 - cob * 128, 0x00020000);
-    const int gat = (w0 + kg) * a.cout * 4 + i * 4, xat = (w0 + kg - a.pw) * a.cin * 4 + i * 4;
-#pragma unroll
-    for (int u = 0; u < kPairsPerPass; ++u)
-      o.gy[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(gr, gat + 2 * u * a.cout * 4, 0, 0));
-#pragma unroll
-    for (int t = 0; t < 7; ++t) {
-      const int tap = tap0 + t;
-      const int kd = tap / 9, kh = (tap / 3) % 3, kw = tap % 3;
-      const int id = od + kd - a.pd, ih = oh + kh - a.ph;
-      const int64_t xrow = ((int64_t)n * a.id + id) * a.ih + ih;
-      // (voxels that belong to no output of the row end the records too: 0 x infinity is not 0)
-      const int w_end = a.iw < a.ow + kw - a.pw ? a.iw : a.ow + kw - a.pw;
-      const bool row_ok = (t < ntaps) & (w_end > 0) & ((unsigned)id < (unsigned)a.id) & ((unsigned)ih < (unsigned)a.ih);
-      const int records = w_end * a.cin * 4 - cib * 128;
-      const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xb + xrow * a.iw * a.cin), 0,
-                                                                          row_ok ? records : 0, 0x00020000);
-#pragma unroll
-      for (int u = 0; u < kPairsPerPass; ++u) {
-        const uint32_t at = (uint32_t)(xat + (2 * u + kw) * a.cin * 4);
-        o.x[u][t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, at < kOutside ? at : kOutside, 0, 0));
+    for (int k = 0; k < kPiecesPer; ++k) {
+      const unsigned h = (unsigned)(rr[k] + oh), w = (unsigned)(vv[k] + ow);
+      const bool in = used[k] && (of_x[k] ? plane_in && h < (unsigned)a.ih && w < (unsigned)a.iw : h < (unsigned)a.oh && w < (unsigned)a.ow);
+      const float* src = (of_x[k] ? xs : gs) + off[k];
+      const Quad got = *reinterpret_cast<const Quad*>(in ? src : x);  // (unconditional, masked afterwards: nothing waits for it here)
+      o.piece[k] = in ? make_float4(got.x, got.y, got.z, got.w) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    o.oh = oh; o.ow = ow;
+    if (++next_seg == segs) {
+      next_seg = 0;
+      if (++next_tile == row_tiles) {
+        next_tile = 0;
+        if (++next_od == a.od) { next_od = 0; ++next_n; }
       }
     }
   };
-  auto compute = [&](const PassOperands& o) {
+
+  f32x16_t acc[3];
 #pragma unroll
-    for (int u = 0; u < kPairsPerPass; ++u)
+  for (int t = 0; t < 3; ++t)
 #pragma unroll
-      for (int t = 0; t < 7; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(o.gy[u], o.x[u][t], acc[t], 0, 0, 0);
+    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+  // Two steps ahead: a wavefront requests behind its MFMAs, where the addresses cost the matrix pipe nothing.
+  auto run = [&](Ahead& o, char* tile, bool more) {
+#pragma unroll
+    for (int k = 0; k < kPiecesPer; ++k) {
+      const int p = k * kWgradThreads + tid;
+      if (p < kXPieces + kGyPieces) *reinterpret_cast<float4*>(tile + p * 16) = o.piece[k];
+    }
+    __syncthreads();  // the other phase was read before the barrier of the step behind it
+#pragma unroll
+    for (int rw = row; rw < row + kRows; rw += kRowWaves) {
+      if (o.oh + rw >= a.oh) break;
+      const int left = a.ow - o.ow;  // voxels of the row from the step's first on
+      const float* xr = reinterpret_cast<const float*>(tile) + ((rw + kh) * kXSeg + kg) * 32 + i;
+      const float* gr = reinterpret_cast<const float*>(tile + kXPieces * 16) + (rw * kSeg + kg) * 32 + i;
+      float even = xr[0];
+#pragma unroll
+      for (int u = 0; u < kSeg / 2; ++u) {
+        if (2 * u >= left) break;
+        const float g = gr[u * 64], odd = xr[u * 64 + 32], after = xr[u * 64 + 64];
+        // a voxel that belongs to no output of the row meets a zero of gy: it must be zero itself, 0 x infinity is not
+        const bool in = 2 * u + kg < left;
+        acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(g, in ? even : 0.f, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(g, in ? odd : 0.f, acc[1], 0, 0, 0);
+        acc[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(g, in ? after : 0.f, acc[2], 0, 0, 0);
+        even = after;
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (more) request(o);
   };
-  PassOperands now, next;
-  int pass = p_begin + half;
-  if (pass < p_end) request(pass, now);
-  for (; pass < p_end; pass += 2) {
-    request(pass + 2 < p_end ? pass + 2 : pass, next);  // (behind the end the last pass once more, not used)
-    __builtin_amdgcn_sched_barrier(0);
-    compute(now);
-    __builtin_amdgcn_sched_barrier(0);
-    now = next;
+  if (begin < end) request(ahead[0]);
+  if (begin + 1 < end) request(ahead[1]);
+  for (int step = begin; step < end; step += 2) {
+    run(ahead[0], lds, step + 2 < end);
+    if (step + 1 < end) run(ahead[1], lds + kStep, step + 3 < end);
   }
 
-  if (half == 1) {
+  __syncthreads();  // the tiles are not read any more
+  float* meet = reinterpret_cast<float*>(lds);
+  if (row > 0) {
 #pragma unroll
-    for (int t = 0; t < 7; ++t)
+    for (int t = 0; t < 3; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) meet[wave][t * 16 + r][lane] = acc[t][r];
+      for (int r = 0; r < 16; ++r) meet[((((row - 1) * 3 + kh) * 3 + t) * 16 + r) * 64 + lane] = acc[t][r];
   }
   __syncthreads();
-  if (half == 1) return;
+  if (row > 0) return;
   // result register r of a lane: column ci = lane % 32, row co = 8 * (r / 4) + 4 * kg + r % 4
-  float* dst = partial + (int64_t)split * a.cout * kTaps * a.cin + ((int64_t)cob * 32 * kTaps) * a.cin + cib * 32 + i;
+  float* dst = partial + (int64_t)split * a.cout * kTaps * a.cin + ((int64_t)cob * 32 * kTaps + kd * 9 + kh * 3) * a.cin + cib * 32 + i;
 #pragma unroll
-  for (int t = 0; t < 7; ++t) {
-    if (t >= ntaps) break;
+  for (int t = 0; t < 3; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int co = 8 * (r / 4) + 4 * kg + (r % 4);
-      dst[((int64_t)co * kTaps + tap0 + t) * a.cin] = acc[t][r] + meet[wave][t * 16 + r][lane];
+      float sum = acc[t][r];
+#pragma unroll
+      for (int q = 0; q < kRowWaves - 1; ++q) sum += meet[(((q * 3 + kh) * 3 + t) * 16 + r) * 64 + lane];
+      dst[((int64_t)co * kTaps + t) * a.cin] = sum;
     }
-  }
 }
 
 }  // namespace
@@ -386,22 +424,29 @@ int f32_conv(const MfmaConvArgs& a, const void* x, const void* packed, const voi
 
 namespace sfh {
 
+// Steps of a weight gradient, and how many a workgroup takes: about one workgroup per CU over the blocks and kd, and no more slices
+// than the longest range asks for.
+static int wgrad_segment(const WgradArgs& a) { return a.ow <= 8 ? 8 : 16; }
+static int64_t wgrad_steps(const WgradArgs& a) {
+  const int seg = wgrad_segment(a);
+  return (int64_t)a.n * a.od * cdiv(a.oh, kRowWaves * (16 / seg)) * cdiv(a.ow, seg);
+}
+
+static int64_t wgrad_per(const WgradArgs& a) {
+  const int64_t units = 3 * (int64_t)(a.cout / 32) * (a.cin / 32), steps = wgrad_steps(a);
+  const int64_t s = kComputeUnits / units;
+  return s > 1 ? cdiv(steps, s) : steps;
+}
+
 bool f32_wgrad_supported(const WgradArgs& a) {
-  // offsets inside a row and the count of passes are 32-bit
+  // offsets inside a row and the count of passes of 8 voxels are 32-bit
   const int64_t reach = 4LL * (a.iw > a.ow ? a.iw : a.ow) + 64 + 4LL * a.pw;
   if (reach * (a.cin > a.cout ? a.cin : a.cout) >= 0x7ffffff0LL) return false;
-  if ((int64_t)a.n * a.od * a.oh * ((a.ow + kPassVoxels - 1) / kPassVoxels) >= 0x7fffffffLL - 4) return false;
+  if ((int64_t)a.n * a.od * a.oh * ((a.ow + 7) / 8) >= 0x7fffffffLL - 4) return false;
   return a.cin % 32 == 0 && a.cout % 32 == 0 && a.n >= 1 && a.od >= 1 && a.oh >= 1 && a.ow >= 1 && a.pd >= 0 && a.ph >= 0 && a.pw >= 0;
 }
 
-int f32_wgrad_splits(const WgradArgs& a) {
-  const int64_t rows = (int64_t)a.n * a.od * a.oh;
-  const int64_t blocks = (int64_t)(a.cout / 32) * (a.cin / 32);
-  int64_t s = kComputeUnits / blocks;  // one workgroup of eight wavefronts per CU
-  if (s < 1) s = 1;
-  if (s > rows) s = rows;
-  return (int)s;
-}
+int f32_wgrad_splits(const WgradArgs& a) { return (int)cdiv(wgrad_steps(a), wgrad_per(a)); }
 
 size_t f32_wgrad_workspace_bytes(const WgradArgs& a) {
   return align_up((size_t)f32_wgrad_splits(a) * a.cout * kTaps * a.cin * sizeof(float), 256);
@@ -410,11 +455,16 @@ size_t f32_wgrad_workspace_bytes(const WgradArgs& a) {
 int f32_wgrad(const WgradArgs& a, const void* x, const void* gy, void* gw, void* workspace, hipStream_t st) {
   const int nsplit = f32_wgrad_splits(a);
   const int cibs = a.cin / 32, cobs = a.cout / 32;
-  const int64_t total = (int64_t)nsplit * cibs * cobs;
+  const int64_t total = (int64_t)nsplit * 3 * cibs * cobs;
   if (total > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv fp32 wgrad: too many workgroups");
-  // one slice is the gradient itself
-  hipLaunchKernelGGL(wgrad_f32_kernel, dim3((unsigned)total), dim3(512), 0, st, a, (const float*)x, (const float*)gy,
-                     (float*)(nsplit == 1 ? gw : workspace), nsplit, cibs);
+  float* slices = (float*)(nsplit == 1 ? gw : workspace);  // one slice is the gradient itself
+  const int per = (int)wgrad_per(a), steps = (int)wgrad_steps(a);
+  if (wgrad_segment(a) == 8)
+    hipLaunchKernelGGL(wgrad_f32_kernel<8>, dim3((unsigned)total), dim3(kWgradThreads), 0, st, a, (const float*)x, (const float*)gy, slices,
+                       nsplit, per, steps, cibs);
+  else
+    hipLaunchKernelGGL(wgrad_f32_kernel<16>, dim3((unsigned)total), dim3(kWgradThreads), 0, st, a, (const float*)x, (const float*)gy, slices,
+                       nsplit, per, steps, cibs);
   if (int rc = check_launch("wgrad_f32_kernel")) return rc;
   if (nsplit == 1) return SFH_OK;
   return sum_slices(SFH_FP32, (const float*)workspace, gw, (int64_t)a.cout * kTaps * a.cin, nsplit, st);
