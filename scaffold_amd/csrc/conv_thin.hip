@@ -286,7 +286,9 @@ __global__ void __launch_bounds__(kBlock) head_wide_out_kernel(ThinArgs a, const
 }
 
 // reduce: G[j][c] = sum_v thin[v][j] * wide[v][c]. The contraction runs over voxels, so both operands are read from
-// LDS against their storage order (8 voxels of one channel per lane). A workgroup owns a contiguous voxel range in
+// LDS against their storage order (8 voxels of one channel per lane; the wide rows by the transposing read). Bound by HBM: a round
+// that waited for its operands, and eight 2-byte LDS reads per fragment of the wide side, took 105 us for 64 -> 6 channels at 128^3,
+// 24.1 for 32 -> 6 at 64^3 and 17.5 for 32 -> 11 at 32^3 (16 workgroups of 16 rounds); now 48, 8.0 and 6.7, with the slice sum. A workgroup owns a contiguous voxel range in
 // rounds of 128, its four wavefronts a quarter of each round; their tiles are folded in wave order into one fp32
 // partial slice, already in the layout of the weight gradient. Tile rows at and beyond J carry garbage that is
 // never written out; voxels beyond the range are zero on both sides.
@@ -316,21 +318,46 @@ __global__ void __launch_bounds__(kBlock) head_reduce_kernel(ThinArgs a, const T
   const int64_t begin = (int64_t)blockIdx.x * per_split;
   int64_t end = begin + per_split;
   if (end > total) end = total;
+  // A whole round's pieces are requested while the round before is multiplied; the cut last one of the tensor is fetched in place
+  // (its voxel count is taken in that branch: clamped in front of it the compiler lost the clamp).
+  constexpr int WPER = kHeadVoxels * CW / 8 / kBlock, TPER = kHeadVoxels * kHeadThinMax / 8 / kBlock;
+  const int tpieces = kHeadVoxels * J / 8;
+  uint4 wahead[WPER], tahead[TPER];
+#pragma unroll
+  for (int i = 0; i < WPER; ++i) wahead[i] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < TPER; ++i) tahead[i] = make_uint4(0, 0, 0, 0);
+  auto request = [&](int64_t base) {
+    const uint4* tsrc = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(thin) + base * J);
+    const uint4* wsrc = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(wide) + base * CW);
+    const bool whole = base + kHeadVoxels <= end;
+#pragma unroll
+    for (int i = 0; i < WPER; ++i)
+      if (whole) wahead[i] = wsrc[i * kBlock + tid];
+#pragma unroll
+    for (int i = 0; i < TPER; ++i)
+      if (whole && i * kBlock + tid < tpieces) tahead[i] = tsrc[i * kBlock + tid];
+  };
+  request(begin);
   for (int64_t base = begin; base < end; base += kHeadVoxels) {
-    const int64_t left = end - base;
-    const int nv = left < kHeadVoxels ? (int)left : kHeadVoxels;
-    {
-      const int nelem = nv * J, npiece = nelem / 8;
+    if (base + kHeadVoxels <= end) {
+#pragma unroll
+      for (int i = 0; i < WPER; ++i) reinterpret_cast<uint4*>(wrows)[i * kBlock + tid] = wahead[i];
+#pragma unroll
+      for (int i = 0; i < TPER; ++i)
+        if (i * kBlock + tid < tpieces) reinterpret_cast<uint4*>(trows)[i * kBlock + tid] = tahead[i];
+    } else {
+      const int nv = (int)(end - base), nelem = nv * J, npiece = nelem / 8;
       const uint16_t* src = reinterpret_cast<const uint16_t*>(thin) + base * J;
       for (int i = tid; i < npiece; i += kBlock) reinterpret_cast<uint4*>(trows)[i] = reinterpret_cast<const uint4*>(src)[i];
       for (int i = npiece * 8 + tid; i < nelem; i += kBlock) trows[i] = src[i];
-      if (nv < kHeadVoxels)
-        for (int i = nelem + tid; i < kHeadVoxels * J; i += kBlock) trows[i] = 0;
+      for (int i = nelem + tid; i < kHeadVoxels * J; i += kBlock) trows[i] = 0;
       const uint4* wsrc = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(wide) + base * CW);
       for (int i = tid; i < kHeadVoxels * CW / 8; i += kBlock)
         reinterpret_cast<uint4*>(wrows)[i] = i < nv * CW / 8 ? wsrc[i] : make_uint4(0, 0, 0, 0);
     }
     __syncthreads();
+    request(base + kHeadVoxels);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       const int v0 = wave * 32 + ks * 16 + kg * 8;
@@ -340,12 +367,8 @@ __global__ void __launch_bounds__(kBlock) head_reduce_kernel(ThinArgs a, const T
       const uint4 tf = make_uint4(h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16);
       if (bias_part != nullptr) bacc = Mma32<T>::run(tf, ones, bacc);  // every column is the row sum
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) h[e] = wrows[(v0 + e) * CW + cc * 32 + col];
-        const uint4 xf = make_uint4(h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16);
-        acc[cc] = Mma32<T>::run(tf, xf, acc[cc]);
-      }
+      for (int cc = 0; cc < NC; ++cc)
+        acc[cc] = Mma32<T>::run(tf, tr_fragment(wrows + (wave * 32 + ks * 16) * CW + cc * 32, CW, lane), acc[cc]);
     }
     __syncthreads();
   }
@@ -728,8 +751,9 @@ bool thin_supported(const ThinArgs& a, int dtype) {
 
 int thin_reduce_splits(const ThinArgs& a) {
   const int64_t total = (int64_t)a.n * a.od * a.oh * a.ow;
-  // at least 2048 voxels per workgroup so that the fold at the end stays a small share
-  int64_t n = cdiv(total, 2048);
+  // at least 2048 voxels per workgroup so that the fold at the end stays a small share; the head's kernel, whose rounds of 128
+  // voxels run one after the other, 512 (2048: 24 us instead of 8 at 64^3)
+  int64_t n = cdiv(total, head_reduce_applies(a) ? 512 : 2048);
   if (n > kComputeUnits * 2) n = kComputeUnits * 2;
   return (int)(n < 1 ? 1 : n);
 }
