@@ -470,6 +470,28 @@ GatherPlan gather_plan(const MfmaConvArgs& a) {
       }
     }
   }
+  // Launches that fill the chip may take the bricks of shorter rows: what a row of 32 leaves over at its end is often more than
+  // the halo of a stubbier brick, and that of 8 x 8 x 8 with two blocks is the smallest of all. Weights per output voxel and
+  // block against 4 x 4 x 32 with one, from 64 -> 64 channels at 128^3 where nothing is left over (us 4x4x32 / 4x8x16 / 8x8x8, one block
+  // 422 / 420 / 465, two 420 / 421 / 406; halves of them 505 / 501 / 482, 459 / 456 / 443). us, rows of 32 -> the choice: 64 -> 64 at
+  // 96x80x112 197 -> 173, at 100^3 229 -> 212, at 60x72x48 64 -> 49, at 22x30x37 (two samples) 24.5 -> 18; 128 -> 128 at 48x40x56 101 -> 93,
+  // at 64^3 191 -> 187; 64 -> 32 at 44x60x75 (two samples) 59 -> 55. The sums of a voxel do not depend on its brick.
+  constexpr int kStubby[2][2][2] = {{{100, 97}, {115, 111}}, {{111, 94}, {112, 108}}};  // [class - 1][size][nsub - 1]
+  if (best_wgs >= kComputeUnits) {
+    best *= 100;  // (the native costs count two factors of a hundred, these one)
+    for (int c = cls + 1; c < 3; ++c)
+      for (int size = 0; size < 2; ++size)
+        for (int nsub = 1; nsub <= (a.cout % 64 == 0 ? 2 : 1); ++nsub) {
+          const int* t = kTileDims[c][size];
+          const int64_t tiles = tiles_of(a, c, size), wgs = tiles * (a.cout / (32 * nsub));
+          const int64_t cost = cdiv(wgs, kComputeUnits) * (t[0] * t[1] * t[2]) * nsub * kStubby[c - 1][size][nsub - 1] * 10000;
+          if (cost < best && wgs > kComputeUnits / 2) {
+            best = cost; best_wgs = wgs;
+            p.shape = c * 3 + size; p.tiles = tiles; p.nsub = nsub;
+          }
+        }
+    return GatherPlan{p.shape, p.nsub, 1, p.tiles};
+  }
   p.ksplit = 1;
   if (best_wgs > 0 && best_wgs < kComputeUnits) {
     const int64_t room = kComputeUnits / best_wgs;
