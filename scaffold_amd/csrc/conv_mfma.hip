@@ -430,7 +430,7 @@ __global__ void __launch_bounds__(256) pack_tiles_kernel(TileBatch<N> b) {
   }
 }
 
-struct GatherPlan { int shape; int nsub; int ksplit; int64_t tiles; };
+struct GatherPlan { int shape; int nsub; int ksplit; int64_t tiles; int64_t cost; };  // cost: the busiest CU's voxels x blocks, in hundredths
 
 // Brick shapes: the row-length class (32-, 16- or 8-voxel rows) times the tile size (512, 256 or 128 output voxels).
 constexpr int kTileDims[3][3][3] = {
@@ -490,9 +490,10 @@ GatherPlan gather_plan(const MfmaConvArgs& a) {
             p.shape = c * 3 + size; p.tiles = tiles; p.nsub = nsub;
           }
         }
-    return GatherPlan{p.shape, p.nsub, 1, p.tiles};
+    return GatherPlan{p.shape, p.nsub, 1, p.tiles, best / 10000};
   }
   p.ksplit = 1;
+  p.cost = best / 100;
   if (best_wgs > 0 && best_wgs < kComputeUnits) {
     const int64_t room = kComputeUnits / best_wgs;
     while (p.ksplit * 2 <= room && p.ksplit * 2 <= ncc && p.ksplit < 8) p.ksplit *= 2;
@@ -709,6 +710,8 @@ size_t mfma_conv_partial_bytes(const MfmaConvArgs& a) {
   return align_up((size_t)p.ksplit * a.n * a.od * a.oh * a.ow * a.cout * sizeof(float), 256);
 }
 
+int64_t mfma_conv_brick_cost(const MfmaConvArgs& a) { return gather_plan(a).cost; }
+
 MfmaConvGeometry mfma_conv_gather_geometry(const MfmaConvArgs& a) {
   if (mfma_conv_wide_applies(a)) return mfma_conv_wide_geometry(a);
   if (mfma_conv_split_applies(a)) return mfma_conv_split_geometry(a);
@@ -735,7 +738,7 @@ int mfma_conv_gather(const MfmaConvArgs& a, int dtype, const void* x, const void
 }
 
 bool mfma_conv_gather_pair_ok(const MfmaConvArgs& a, int first, bool as_output) {
-  if (mfma_conv_wide_applies(a)) return !as_output && mfma_conv_wide_pair_ok(a, first);
+  if (mfma_conv_wide_fits(a)) return !as_output && mfma_conv_wide_pair_ok(a, first);
   if (mfma_conv_split_applies(a)) return mfma_conv_split_pair_ok(a, first, as_output);
   return gather_pair_ok(a, first, as_output);
 }

@@ -47,6 +47,7 @@ int mfma_conv_gather(const MfmaConvArgs& a, int dtype, const void* x, const void
 // Same contract, wide-tile kernel (64 or more reduction channels, rows of more than 16 voxels): `applies` is a pure
 // function of the shape; mfma_conv_gather routes to it (it needs no partial workspace).
 bool mfma_conv_wide_applies(const MfmaConvArgs& a);
+bool mfma_conv_wide_fits(const MfmaConvArgs& a);  // also where the brick kernel serves it: what pairs of tensors it takes follows this
 int mfma_conv_wide(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                    const GnPartialOut* gn = nullptr, const ChannelPair* in2 = nullptr);
 // Same contract, the kernel for the small volumes of the deep levels: 64-voxel bricks, the reduction cut over the four
@@ -83,6 +84,8 @@ struct MfmaConvGeometry { int kernel, voxels, blocks, slices; };
 MfmaConvGeometry mfma_conv_geometry(const MfmaConvArgs& a);
 bool mfma_conv_persist_applies(const MfmaConvArgs& a);
 MfmaConvGeometry mfma_conv_gather_geometry(const MfmaConvArgs& a);
+// What the brick kernel's launch rule reckons for a problem: output voxels x 32-channel blocks of the busiest CU, in hundredths.
+int64_t mfma_conv_brick_cost(const MfmaConvArgs& a);
 MfmaConvGeometry mfma_conv_wide_geometry(const MfmaConvArgs& a);
 MfmaConvGeometry mfma_conv_split_geometry(const MfmaConvArgs& a);
 

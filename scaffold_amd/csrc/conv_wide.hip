@@ -381,6 +381,7 @@ conv_wide_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ 
 
 struct WidePlan {
   bool use;
+  bool fits;   // the problem is this kernel's, also where the brick kernel takes its place
   int shape;   // 0: 4x4x32 tile with 4 channel blocks, 1: 8x4x32 with 2, 2: 8x4x32 with 1, 3: 4x4x32 with 2, 4: 4x4x32 with 1
 };
 
@@ -394,7 +395,7 @@ int64_t wide_workgroups(const MfmaConvArgs& a, int shape) {
 
 // Launch geometry, a pure function of the problem. Rows of more than 16 voxels only (32-voxel sub-tiles are one row).
 WidePlan wide_plan(const MfmaConvArgs& a) {
-  WidePlan p{false, 0};
+  WidePlan p{false, false, 0};
   if (a.kd != 3 || a.kh != 3 || a.kw != 3 || a.cred < 64 || a.cred % 32 != 0 || a.cout % 32 != 0 || a.ow <= 16) return p;
   // a brick (at most 10 input planes and 6 rows) must span less than kRange bytes of the input
   if (((int64_t)10 * a.ih + 6) * a.iw * a.cred * 2 + 64 >= kRange) return p;
@@ -408,6 +409,16 @@ WidePlan wide_plan(const MfmaConvArgs& a) {
     else if (wide_workgroups(a, 3) >= kComputeUnits) shape = 3;
   }
   if (shape < 0) return p;
+  p.fits = true;
+  // Past two rounds of workgroups the brick kernel takes its place where 8 x 4 x 32 leaves more over than that kernel's choice of
+  // brick, by the busiest CU's share (at equal shares it is the faster one by some 3 % for 128 channels, the slower by 5 for 256).
+  // us, here -> there: 128 -> 64 at 96x80x112 353 -> 315, at 100^3 485 -> 387, at 90^3 331 -> 309, at 128^3 761 -> 739; 256 -> 64 at
+  // 64^3 171 -> 180. As for the small volumes the depth counted is that of a shard's planes in both forms of its gradients.
+  MfmaConvArgs core = a;
+  core.od = a.id < a.od ? a.id : a.od;
+  const int64_t wgs = wide_workgroups(core, 1);
+  if (a.cred % 64 == 0 && wgs > 2 * kComputeUnits &&  // (half of the channels in whole chunks: both kernels take the same pairs)
+      mfma_conv_brick_cost(core) * 100 < cdiv(wgs, kComputeUnits) * 1024 * 2 * 100 * (a.cred < 256 ? 97 : 92)) return p;
   p.use = true;
   p.shape = shape;
   return p;
@@ -467,7 +478,8 @@ int mfma_conv_wide_gn_records(const MfmaConvArgs& a, int groups) {
 }
 
 // The staging offsets of a lane are those of one tensor: a pair must be two tensors of the same channel count.
-bool mfma_conv_wide_pair_ok(const MfmaConvArgs& a, int first) { return wide_plan(a).use && first * 2 == a.cred && first % 16 == 0; }
+bool mfma_conv_wide_fits(const MfmaConvArgs& a) { return wide_plan(a).fits; }
+bool mfma_conv_wide_pair_ok(const MfmaConvArgs& a, int first) { return wide_plan(a).fits && first * 2 == a.cred && first % 16 == 0; }
 
 int mfma_conv_wide(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                    const GnPartialOut* gn, const ChannelPair* in2) {
