@@ -178,11 +178,17 @@ __device__ __forceinline__ uint4 head_weight_thin_run(const ThinArgs& a, const T
   return make_uint4(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16, h[4] | (uint32_t)h[5] << 16, h[6] | (uint32_t)h[7] << 16);
 }
 
-// thin-out: out[v][j] = bias[j] + sum_c wide[v][c] * W[j][c]. Result tile: rows = thin channels, columns = voxels.
+// thin-out: out[v][j] = bias[j] + sum_c wide[v][c] * W[j][c]. Result tile: rows = thin channels, columns = voxels. With 64 wide
+// channels (TURN) a wavefront's 32 voxels are fetched in whole lines a round ahead and turned in LDS, [8-channel piece][voxel];
+// fragments straight from memory are 32 lines of 32 bytes an instruction: 64 -> 6 at 128^3 66 -> 55 us, at 96x80x112 32 -> 30. A row of 32
+// channels is half a line and gains nothing (32 -> 6 at 64^3 10.5 -> 11.2).
 template <typename T, int NC>
 __global__ void __launch_bounds__(kBlock) head_thin_out_kernel(ThinArgs a, const T* __restrict__ wide, const T* __restrict__ wt,
                                                                const T* __restrict__ bias, T* __restrict__ out, int64_t total) {
+  constexpr bool TURN = NC == 2;
+  constexpr int PIECES = NC * 4, PLANE = 512 + 256 / PIECES, PER = PIECES / 2;  // (a voxel's pieces fall into different banks)
   __shared__ __align__(16) T rows[kHeadVoxels * kHeadThinMax];
+  __shared__ __align__(16) char turn[TURN ? 4 : 1][TURN ? PIECES * PLANE : 16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 31, kg = lane >> 5;
   const int J = a.J;
@@ -198,14 +204,41 @@ __global__ void __launch_bounds__(kBlock) head_thin_out_kernel(ThinArgs a, const
     const float b = bias != nullptr ? to_float(bias[j < J ? j : 0]) : 0.f;
     bv[r] = j < J ? b : 0.f;
   }
-  for (int64_t base = (int64_t)blockIdx.x * kHeadVoxels; base < total; base += (int64_t)gridDim.x * kHeadVoxels) {
-    const int64_t v = base + wave * 32 + col;
-    const T* src = wide + (v < total ? v : total - 1) * a.cw + kg * 8;
+  char* tile = turn[TURN ? wave : 0];
+  const int64_t step = (int64_t)gridDim.x * kHeadVoxels, last = total * PIECES - 1;
+  uint4 ahead[PER];
+  auto request = [&](int64_t base) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int64_t q = (base + wave * 32) * PIECES + i * 64 + lane;
+      ahead[i] = load16(wide + (q < last ? q : last) * 8);
+    }
+  };
+  if (TURN) request((int64_t)blockIdx.x * kHeadVoxels);
+  for (int64_t base = (int64_t)blockIdx.x * kHeadVoxels; base < total; base += step) {
     uint4 xf[NC][2];
+    if constexpr (TURN) {
 #pragma unroll
-    for (int cc = 0; cc < NC; ++cc)
+      for (int i = 0; i < PER; ++i) {
+        const int q = i * 64 + lane;
+        *reinterpret_cast<uint4*>(tile + q % PIECES * PLANE + q / PIECES * 16) = ahead[i];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      request(base + step);
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) xf[cc][ks] = load16(src + cc * 32 + ks * 16);
+      for (int cc = 0; cc < NC; ++cc)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+          xf[cc][ks] = *reinterpret_cast<const uint4*>(tile + (cc * 4 + ks * 2 + kg) * PLANE + col * 16);
+    } else {
+      const int64_t v = base + wave * 32 + col;
+      const T* src = wide + (v < total ? v : total - 1) * a.cw + kg * 8;
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) xf[cc][ks] = load16(src + cc * 32 + ks * 16);
+    }
     f32x16_t acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
@@ -231,12 +264,16 @@ __global__ void __launch_bounds__(kBlock) head_thin_out_kernel(ThinArgs a, const
 }
 
 // wide-out: out[v][c] = bias[c] + sum_j thin[v][j] * W[j][c]. Result tile: rows = wide channels, columns = voxels.
-// NK = MFMA steps of 16 thin channels.
+// NK = MFMA steps of 16 thin channels. The 128 bytes of a voxel with 64 channels leave as one line through LDS (LINES): pieces of
+// 32 bytes cost the memory half its rate once the tensor outgrows its caches, 64 -> 6 at 128^3 95 -> 67 us, at 96x80x112 23.6 -> 21.3.
 template <typename T, int NC, int NK>
 __global__ void __launch_bounds__(kBlock) head_wide_out_kernel(ThinArgs a, const T* __restrict__ thin, const T* __restrict__ wt,
                                                                const T* __restrict__ bias, T* __restrict__ out, int64_t total) {
   // one row of slack: the operand read of the last voxel runs up to 16 * NK channels
   __shared__ __align__(16) uint16_t rows[(kHeadVoxels + 1) * kHeadThinMax];
+  constexpr bool LINES = NC == 2;
+  constexpr int ROW = 144;  // LDS bytes of a voxel's line
+  __shared__ __align__(16) char lines[LINES ? 4 : 1][LINES ? 32 * ROW : 16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 31, kg = lane >> 5;
   const int J = a.J;
@@ -279,7 +316,31 @@ __global__ void __launch_bounds__(kBlock) head_wide_out_kernel(ThinArgs a, const
       for (int r = 0; r < 16; ++r) acc[r] = 0.f;
 #pragma unroll
       for (int ks = 0; ks < NK; ++ks) acc = Mma32<T>::run(wf[cc][ks], xf[ks], acc);
-      store_block_plus<T>(acc, dst + cc * 32, bv[cc], kg, valid);
+      if constexpr (LINES) {
+        uint32_t run[4][2];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          run[g][0] = Mma32<T>::pack2(acc[4 * g] + bv[cc][4 * g], acc[4 * g + 1] + bv[cc][4 * g + 1]);
+          run[g][1] = Mma32<T>::pack2(acc[4 * g + 2] + bv[cc][4 * g + 2], acc[4 * g + 3] + bv[cc][4 * g + 3]);
+        }
+        uint4 piece[2];
+        trade_channel_runs(run, piece);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) *reinterpret_cast<uint4*>(lines[wave] + col * ROW + cc * 64 + h * 32 + kg * 16) = piece[h];
+      } else {
+        store_block_plus<T>(acc, dst + cc * 32, bv[cc], kg, valid);
+      }
+    }
+    if constexpr (LINES) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int vox = i * 8 + (lane >> 3);
+        if (wave * 32 + vox < nv)
+          *reinterpret_cast<uint4*>(out + (base + wave * 32 + vox) * a.cw + (lane & 7) * 8) =
+              *reinterpret_cast<const uint4*>(lines[wave] + vox * ROW + (lane & 7) * 16);
+      }
     }
     __syncthreads();
   }
