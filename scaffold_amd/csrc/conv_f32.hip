@@ -291,7 +291,8 @@ wgrad_f32_kernel(WgradArgs a, const float* __restrict__ x, const float* __restri
   const int next_plane = begin / segs / row_tiles;
   int next_seg = begin % segs, next_tile = begin / segs % row_tiles;
   int next_od = next_plane % a.od, next_n = next_plane / a.od;
-  int rr[kPiecesPer], vv[kPiecesPer], off[kPiecesPer];
+  int rr[kPiecesPer], vv[kPiecesPer];
+  int64_t off[kPiecesPer];
   bool of_x[kPiecesPer], used[kPiecesPer];
 #pragma unroll
   for (int k = 0; k < kPiecesPer; ++k) {
@@ -300,7 +301,8 @@ wgrad_f32_kernel(WgradArgs a, const float* __restrict__ x, const float* __restri
     used[k] = q < kGyPieces;
     rr[k] = of_x[k] ? p / (kXSeg * 8) - a.ph : q / (kSeg * 8);
     vv[k] = of_x[k] ? p / 8 % kXSeg - a.pw : q / 8 % kSeg;
-    off[k] = of_x[k] ? (rr[k] * a.iw + vv[k]) * a.cin + cib * 32 + (p & 7) * 4 : (rr[k] * a.ow + vv[k]) * a.cout + cob * 32 + (p & 7) * 4;
+    off[k] = of_x[k] ? ((int64_t)rr[k] * a.iw + vv[k]) * a.cin + cib * 32 + (p & 7) * 4
+                     : ((int64_t)rr[k] * a.ow + vv[k]) * a.cout + cob * 32 + (p & 7) * 4;
   }
   struct Ahead { float4 piece[kPiecesPer]; int oh, ow; } ahead[2];
   auto request = [&](Ahead& o) {
