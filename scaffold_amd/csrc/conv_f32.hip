@@ -328,13 +328,15 @@ wgrad_f32_kernel(WgradArgs a, const float* __restrict__ x, const float* __restri
     }
   };
 
-  f32x16_t acc[3];
+  f32x16_t sums[2][3];  // of the even and the odd steps: against 64 bits 1.7e-7 at 32^3 instead of 2.1e-7 in one chain
 #pragma unroll
-  for (int t = 0; t < 3; ++t)
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sums[h][t][r] = 0.f;
   // Two steps ahead: a wavefront requests behind its MFMAs, where the addresses cost the matrix pipe nothing.
-  auto run = [&](Ahead& o, char* tile, bool more) {
+  auto run = [&](Ahead& o, f32x16_t (&acc)[3], char* tile, bool more) {
 #pragma unroll
     for (int k = 0; k < kPiecesPer; ++k) {
       const int p = k * kWgradThreads + tid;
@@ -366,10 +368,15 @@ wgrad_f32_kernel(WgradArgs a, const float* __restrict__ x, const float* __restri
   if (begin < end) request(ahead[0]);
   if (begin + 1 < end) request(ahead[1]);
   for (int step = begin; step < end; step += 2) {
-    run(ahead[0], lds, step + 2 < end);
-    if (step + 1 < end) run(ahead[1], lds + kStep, step + 3 < end);
+    run(ahead[0], sums[0], lds, step + 2 < end);
+    if (step + 1 < end) run(ahead[1], sums[1], lds + kStep, step + 3 < end);
   }
 
+  f32x16_t(&acc)[3] = sums[0];
+#pragma unroll
+  for (int t = 0; t < 3; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[t][r] += sums[1][t][r];
   __syncthreads();  // the tiles are not read any more
   float* meet = reinterpret_cast<float*>(lds);
   if (row > 0) {
