@@ -501,7 +501,10 @@ constexpr int kSmallTile = 64;      // small channels per workgroup (two row blo
 
 // A workgroup accumulates 64 small channels x 8 taps x 32 big channels over a range of voxels; its two halves of four wavefronts
 // take the rounds of 32 voxels in turn (wavefront w of a half: taps 2w and 2w + 1 for both row blocks) and meet in LDS at the
-// end, half 0 plus half 1, so that twice the wavefronts load without a second fp32 slice in memory. A round's operands are
+// end, half 0 plus half 1, so that twice the wavefronts load without a second fp32 slice in memory. Even and odd k-steps keep sums
+// of their own, which halves the chain of roundings at no cost in time (relative error of the fp32 gradient against 64 bits, one sum ->
+// two, e-7: 128 -> 64 at 32^3 1.36 -> 1.17, 64 -> 32 at 32x64x64 1.44 -> 1.30, 256 -> 128 at 5x7x9 (two samples) 0.67 -> 0.64,
+// 512 -> 256 at 4x8x8, one range, 0.66 -> 0.57). A round's operands are
 // requested two rounds ahead and laid into the two phases of LDS in turn; a channel block's rows of 64 bytes
 // lie dense, which neither the 16-byte writes nor the transposing reads meet a bank conflict on.
 // grid: `by_xcd` ? eight-fold splits x tiles, the tiles of a range of voxels on one XCD (its lines come from HBM once; spread
@@ -528,13 +531,13 @@ __global__ void __launch_bounds__(512, 2) patch_reduce_kernel(PatchArgs a, const
   const int64_t begin = (int64_t)split * per_split;
   int64_t end = begin + per_split;
   if (end > total) end = total;
-  f32x16_t acc[2][2];
+  f32x16_t acc[2][2], odd[2][2];  // the even and the odd k-steps
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = odd[i][j][r] = 0.f;
   f32x16_t bacc[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j)
@@ -591,7 +594,10 @@ __global__ void __launch_bounds__(512, 2) patch_reduce_kernel(PatchArgs a, const
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = Mma32<T>::run(af[i], bf[j], acc[i][j]);
+          for (int j = 0; j < 2; ++j) {
+            f32x16_t& sum = ks ? odd[i][j] : acc[i][j];
+            sum = Mma32<T>::run(af[i], bf[j], sum);
+          }
         if constexpr (BIAS) {
           if (sums_big) {  // every row of the block is the column sum
 #pragma unroll
@@ -601,6 +607,12 @@ __global__ void __launch_bounds__(512, 2) patch_reduce_kernel(PatchArgs a, const
       }
     }
   }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] += odd[i][j][r];
   // half h keeps row block h and hands the other one over
   __syncthreads();
   float* hand = reinterpret_cast<float*>(lds);
