@@ -703,8 +703,13 @@ int mfma_pack_weight_batch(const MfmaPackItem* items, int n, int dtype, hipStrea
   return launch_pieces(dtype, pieces, piece_blocks, st);
 }
 
+// Where the wide kernel steps aside it does so for the brick kernel, whose share it reckoned: not for the small-volume one, which
+// otherwise goes in front of the bricks (us, small-volume / brick / wide: 128 -> 64 on 32 samples of 32^3 455 / 377 / 371, on 8 of
+// 128x32x32 449 / 367 / 370, on 10 of 64x28x28 234 / 218 / 241; 256 -> 64 on 16 of 48x28x20 404 / 387 / 450).
+static bool served_by_split(const MfmaConvArgs& a) { return !mfma_conv_wide_fits(a) && mfma_conv_split_applies(a); }
+
 size_t mfma_conv_partial_bytes(const MfmaConvArgs& a) {
-  if (mfma_conv_wide_applies(a) || mfma_conv_split_applies(a)) return 0;
+  if (mfma_conv_wide_applies(a) || served_by_split(a)) return 0;
   const GatherPlan p = gather_plan(a);
   if (a.cred == kChunk || p.ksplit == 1) return 0;
   return align_up((size_t)p.ksplit * a.n * a.od * a.oh * a.ow * a.cout * sizeof(float), 256);
@@ -714,7 +719,7 @@ int64_t mfma_conv_brick_cost(const MfmaConvArgs& a) { return gather_plan(a).cost
 
 MfmaConvGeometry mfma_conv_gather_geometry(const MfmaConvArgs& a) {
   if (mfma_conv_wide_applies(a)) return mfma_conv_wide_geometry(a);
-  if (mfma_conv_split_applies(a)) return mfma_conv_split_geometry(a);
+  if (served_by_split(a)) return mfma_conv_split_geometry(a);
   const GatherPlan p = gather_plan(a);
   const int* t = kTileDims[p.shape / 3][p.shape % 3];
   return MfmaConvGeometry{kKernelBrick, t[0] * t[1] * t[2], p.nsub, p.ksplit};
@@ -722,7 +727,7 @@ MfmaConvGeometry mfma_conv_gather_geometry(const MfmaConvArgs& a) {
 
 int mfma_conv_gather_gn_records(const MfmaConvArgs& a, int groups) {
   if (mfma_conv_wide_applies(a)) return mfma_conv_wide_gn_records(a, groups);
-  if (mfma_conv_split_applies(a)) return mfma_conv_split_gn_records(a, groups);
+  if (served_by_split(a)) return mfma_conv_split_gn_records(a, groups);
   return gather_gn_records(a, gather_plan(a), groups);
 }
 
@@ -732,14 +737,14 @@ int mfma_conv_gather(const MfmaConvArgs& a, int dtype, const void* x, const void
     if (out2 != nullptr) return fail(SFH_ERR_UNSUPPORTED, "conv wide: the output cannot be a pair of tensors");
     return mfma_conv_wide(a, dtype, x, packed, bias, y, st, gn, in2);
   }
-  if (mfma_conv_split_applies(a)) return mfma_conv_split(a, dtype, x, packed, bias, y, st, gn, in2, out2);
+  if (served_by_split(a)) return mfma_conv_split(a, dtype, x, packed, bias, y, st, gn, in2, out2);
   if (dtype == SFH_BF16) return launch_typed<bf16_t>(a, dtype, x, packed, bias, y, partial, st, gn, in2, out2);
   return launch_typed<fp16_t>(a, dtype, x, packed, bias, y, partial, st, gn, in2, out2);
 }
 
 bool mfma_conv_gather_pair_ok(const MfmaConvArgs& a, int first, bool as_output) {
   if (mfma_conv_wide_fits(a)) return !as_output && mfma_conv_wide_pair_ok(a, first);
-  if (mfma_conv_split_applies(a)) return mfma_conv_split_pair_ok(a, first, as_output);
+  if (served_by_split(a)) return mfma_conv_split_pair_ok(a, first, as_output);
   return gather_pair_ok(a, first, as_output);
 }
 

@@ -37,6 +37,7 @@ def _planes(x, w, planes):
     (1, 96, 96, (33, 41, 50), "brick"),     # three blocks of one
     (1, 128, 64, (65, 77, 90), "brick"),    # in the wide kernel's place: 9 x 20 x 3 of its bricks
     (1, 128, 64, (48, 64, 60), "wide"),     # two rounds of them or fewer stay
+    (10, 128, 64, (64, 28, 28), "brick"),   # planes that the small-volume kernel would take
 ])
 def test_planes_match_float64(n, cin, cout, spatial, kernel, dtype):
     x, w = _tensor((n, cin, *spatial), 1, dtype), _tensor((cout, cin, 3, 3, 3), 2, dtype, (27 * cin) ** -0.5)

@@ -1,0 +1,24 @@
+"""Which kernel a convolution's volume goes to, where two rules meet: the launch query is a pure function of the problem."""
+
+import pytest
+import torch
+
+from scaffold_amd import conv3d as c3
+
+
+def _kernel(n, cin, cout, spatial, direction="fwd", padding=1):
+    return c3.launch_geometry((n, cin, *spatial), (cout, cin, 3, 3, 3), 1, padding, 1, torch.bfloat16, direction)["kernel"]
+
+
+@pytest.mark.parametrize("n,cin,spatial", [
+    (32, 128, (32, 32, 32)),
+    (16, 128, (64, 32, 32)),
+    (8, 128, (128, 32, 32)),
+    (10, 128, (64, 28, 28)),
+    (16, 256, (48, 28, 20)),
+])
+def test_wide_kernel_steps_aside_for_bricks_only(n, cin, spatial):
+    """Many small planes of a 64-channel output: the wide kernel's or, where its rule reckons the bricks cheaper, the brick kernel's.
+    The small-volume kernel takes the same planes by its own rule and stages 3.75 voxels per output voxel."""
+    assert _kernel(n, cin, 64, spatial) in ("wide", "brick")
+    assert _kernel(n, 64, cin, spatial, "bwd-data") in ("wide", "brick")
