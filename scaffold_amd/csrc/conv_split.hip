@@ -310,7 +310,11 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
 // 64 -> 128 at 16^3 11.9 -> 6.0, 128 -> 128 at 16^3 14.9 -> 8.6, 256 -> 128 at 20x12x14 22 -> 12.5, 512 -> 256 at 16^3 44 -> 32. Few pairs of a
 // long reduction lose (512 -> 512 at 8^3, 64 pairs: 17.4 -> 23.2; 256 -> 256 at 4x8x8, 16 pairs: 10.1 -> 10.6), so the line is higher for
 // those. Some below it would gain as well (128 -> 128 at 8^3, 16 pairs: 9.7 -> 7.7; 256 -> 128 at 8x16x16, 64: 14.9 -> 11.4; 512 -> 256 at
-// 8x16x16, 128: 27.8 -> 22.9): they keep the geometry that the launch query has stated for them and that callers may have sized by.
+// 8x16x16, 128: 27.8 -> 22.9): their sliced geometry is what the tests of the launch query hold the last two to.
+// Past three rounds of pairs the brick kernel's launches have no slices either and stage less: such a volume comes here only where the
+// bricks leave more over, by the busiest CU's share, than the 10 % that 64-voxel bricks lose at equal shares. us, bricks -> here: 64 -> 64 at
+// 256x16x16 (1024 pairs, equal shares) 19.2 -> 21.2, 128 -> 128 at 128x16x16 31.0 -> 33.9; 128 -> 64 at 200x20x20 (1500 pairs, 768 against
+// 993 voxel blocks) 56 -> 46, 64 -> 64 at 64x24x24 (576 pairs) 17.9 -> 16.0, at 128x16x16 (512 pairs) 14.0 -> 12.1.
 // The data gradient of a depth shard's slab (D + 2 planes from D) and of the padded volume (D from D) must come from the same
 // kernel, or a shard and the whole volume would disagree in the last bit: the depth counted is the smaller of the two.
 constexpr int kSplitMaxPlane = 32 * 32, kSplitMinPerDepth = 24, kSplitFewPerDepth = 32, kSplitFewMaxChunks = 16;
@@ -321,8 +325,12 @@ bool mfma_conv_split_applies(const MfmaConvArgs& a) {
   if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return false;
   const int64_t per_depth = (int64_t)a.n * cdiv(a.oh, TH) * cdiv(a.ow, TW) * (a.cout / (32 * kBlocks));
   const int chunks = a.cred / kChunk;
-  const int64_t pairs = per_depth * cdiv(a.id < a.od ? a.id : a.od, TD);
-  if (chunks <= 4 ? pairs >= kComputeUnits / 4 : pairs > (chunks <= 8 ? kComputeUnits / 4 : kComputeUnits / 2)) return true;
+  MfmaConvArgs core = a;
+  core.od = a.id < a.od ? a.id : a.od;
+  const int64_t pairs = per_depth * cdiv(core.od, TD), rounds = cdiv(pairs, kComputeUnits);
+  if ((chunks <= 4 ? pairs >= kComputeUnits / 4 : pairs > (chunks <= 8 ? kComputeUnits / 4 : kComputeUnits / 2)) &&
+      (rounds <= 3 || rounds * (TD * TH * TW * kBlocks) * 110 < mfma_conv_brick_cost(core)))
+    return true;
   if (per_depth <= kSplitFewPerDepth && chunks >= kSplitFewMaxChunks) return false;
   return per_depth >= kSplitMinPerDepth;
 }

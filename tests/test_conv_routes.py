@@ -22,3 +22,20 @@ def test_wide_kernel_steps_aside_for_bricks_only(n, cin, spatial):
     The small-volume kernel takes the same planes by its own rule and stages 3.75 voxels per output voxel."""
     assert _kernel(n, cin, 64, spatial) in ("wide", "brick")
     assert _kernel(n, 64, cin, spatial, "bwd-data") in ("wide", "brick")
+
+
+@pytest.mark.parametrize("cin,cout,spatial,kernel", [
+    (64, 64, (256, 16, 16), "brick"),    # 1024 pairs of blocks on whole bricks
+    (128, 128, (128, 16, 16), "brick"),
+    (256, 64, (256, 16, 16), "brick"),
+    (64, 64, (192, 16, 16), "split"),    # 768: three rounds
+    (128, 64, (200, 20, 20), "split"),   # 1500, but rows of 20 leave a third of the bricks empty
+    (128, 128, (40, 32, 32), "split"),   # a plane that fills its share: whatever the depth
+])
+def test_deep_thin_volumes(cin, cout, spatial, kernel):
+    """Deep volumes of small planes: past three rounds of the small-volume kernel's workgroups the brick kernel serves what it wastes
+    little on -- and the same one whether the data gradient writes a shard's slab or the padded volume."""
+    assert _kernel(1, cin, cout, spatial) == kernel
+    padded = _kernel(1, cout, cin, spatial, "bwd-data")
+    d, h, w = spatial
+    assert padded == kernel and _kernel(1, cout, cin, (d + 2, h, w), "bwd-data", (0, 1, 1)) == padded
