@@ -97,7 +97,9 @@ __device__ __forceinline__ void sum_slices_grouped4_body(unsigned block, const f
 // A handful of elements under thousands of slices (the bias gradient an up-convolution's weight-gradient kernel leaves:
 // 32 channels x 32 Ki slices): one workgroup per element, thread t sums slices t, t + 256, ... with eight loads in
 // flight, then a fixed tree over the 256 thread totals. (With 16 slice lanes per element a lane walked 2048 slices:
-// 12.7 us for 4 MB.)
+// 12.7 us for 4 MB.) Bias sums that ride along with a weight gradient's come here from 32 slices on, for their precision: a chain of
+// 16 or 32 slices a lane rounds more often than the tree (error over the sum of magnitudes, e-9, chain -> tree: 6 channels at
+// 32^3 0.66 -> 0.41, at 44x60x75 (two samples) 0.25 -> 0.16, beside 64 channels at 64^3 0.29 -> 0.20; no difference in time).
 template <typename T>
 __device__ __forceinline__ void sum_slices_tall_body(unsigned block, const float* __restrict__ part, T* __restrict__ out, int64_t nelem, int splits) {
   __shared__ float buf[kBlock];
@@ -472,7 +474,9 @@ int launch_sum_two(const SumJob& a, const SumJob& b, hipStream_t st) {
 
 int sum_slices_two(int dtype, const float* part_a, void* out_a, int64_t nelem_a, int splits_a, const float* part_b, void* out_b,
                    int64_t nelem_b, int splits_b, hipStream_t st) {
-  const SumJob a = sum_job(part_a, out_a, nelem_a, splits_a), b = sum_job(part_b, out_b, nelem_b, splits_b);
+  const SumJob a = sum_job(part_a, out_a, nelem_a, splits_a);
+  SumJob b = sum_job(part_b, out_b, nelem_b, splits_b);
+  if (b.kind == kSumGrouped && nelem_b <= 512) { b.kind = kSumTall; b.blocks = (unsigned)nelem_b; }
   if (a.kind == kSumNone || b.kind == kSumNone || (uint64_t)a.blocks + b.blocks > 0x7fffffffu) {
     if (int rc = sum_slices(dtype, part_a, out_a, nelem_a, splits_a, st)) return rc;
     return sum_slices(dtype, part_b, out_b, nelem_b, splits_b, st);
