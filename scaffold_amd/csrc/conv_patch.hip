@@ -501,48 +501,42 @@ constexpr int kSmallTile = 64;      // small channels per workgroup (two row blo
 
 // A workgroup accumulates 64 small channels x 8 taps x 32 big channels over a range of voxels; its two halves of four wavefronts
 // take the rounds of 32 voxels in turn (wavefront w of a half: taps 2w and 2w + 1 for both row blocks) and meet in LDS at the
-// end, half 0 plus half 1, so that twice the wavefronts load without a second fp32 slice in memory. Even and odd k-steps keep sums
-// of their own, which halves the chain of roundings at no cost in time (relative error of the fp32 gradient against 64 bits, one sum ->
-// two, e-7: 128 -> 64 at 32^3 1.36 -> 1.17, 64 -> 32 at 32x64x64 1.44 -> 1.30, 256 -> 128 at 5x7x9 (two samples) 0.67 -> 0.64,
-// 512 -> 256 at 4x8x8, one range, 0.66 -> 0.57). A round's operands are
+// end, half 0 plus half 1, so that twice the wavefronts load without a second fp32 slice in memory. A round's products are summed by
+// the matrix unit from zero and added to the running sums by the vector unit: half of the roundings of a chain through the matrix
+// unit, and no second set of sums to hold -- one per parity of k-step spilled 6 registers in the form with BIAS. Relative error of the
+// fp32 gradient against 64 bits, e-7, sums of the even and odd k-steps -> rounds: 64 -> 32 at 32x64x64 1.31 -> 1.29, 128 -> 64 at 32^3 1.17 ->
+// 1.14, at 48x40x56 1.48 -> 1.37, 512 -> 256 at 12x10x14 0.90 -> 0.86. A round's operands are
 // requested two rounds ahead and laid into the two phases of LDS in turn; a channel block's rows of 64 bytes
 // lie dense, which neither the 16-byte writes nor the transposing reads meet a bank conflict on.
 // grid: `by_xcd` ? eight-fold splits x tiles, the tiles of a range of voxels on one XCD (its lines come from HBM once; spread
-// over the XCDs 128 -> 64 at 48x40x56 took 84 us instead of 41) : tiles x splits.
+// over the XCDs 128 -> 64 at 48x40x56 took 84 us instead of 38) : tiles x splits.
 // BIAS: the workgroups of the first small-channel tile also add up the big tensor itself over the voxels -- the bias
 // gradient of the transposed convolution whose weight gradient this is (every big voxel is a tap of exactly one small
 // voxel there) -- as one more MFMA row block of ones: bias_part[split][cb], in a fixed order.
 template <typename T, bool BIAS>
-__global__ void __launch_bounds__(512, 2) patch_reduce_kernel(PatchArgs a, const T* __restrict__ small, const T* __restrict__ big,
-                                                              float* __restrict__ part, int64_t total, int64_t per_split, int splits,
-                                                              int by_xcd, float* __restrict__ bias_part) {
+__global__ void __launch_bounds__(512, 2)
+patch_reduce_kernel(PatchArgs a, const T* __restrict__ small, const T* __restrict__ big, float* __restrict__ part, int64_t total,
+                    int64_t per_split, int splits, int by_xcd, float* __restrict__ bias_part) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int D = 2;                           // rounds requested ahead
   constexpr int kBlock = kVx * 32;               // elements of one [voxel][32 channels] block
   constexpr int kRound = (2 + kTaps) * kBlock;   // two blocks of the small tensor, one per tap of the big
+  constexpr int kTurn = 2 * kVx;                 // voxels of a round of both halves
   __shared__ __attribute__((aligned(16))) T lds[2][2][kRound];
   const int nz = a.cbig / 32, tiles = a.csmall / kSmallTile * nz;
   const int slot = blockIdx.x / kXcds;
   const int split = by_xcd ? slot / tiles * kXcds + (int)(blockIdx.x % kXcds) : (int)blockIdx.x / tiles;
   const int tile = (by_xcd ? slot : (int)blockIdx.x) % tiles;
   if (split >= splits) return;
-  const int half = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+  const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int cs0 = tile / nz * kSmallTile, cb0 = tile % nz * 32;
   const int64_t begin = (int64_t)split * per_split;
   int64_t end = begin + per_split;
   if (end > total) end = total;
-  f32x16_t acc[2][2], odd[2][2];  // the even and the odd k-steps
+  f32x16_t acc[2][2], none;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = odd[i][j][r] = 0.f;
-  f32x16_t bacc[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) bacc[j][r] = 0.f;
+  for (int r = 0; r < 16; ++r) none[r] = acc[0][0][r] = acc[0][1][r] = acc[1][0][r] = acc[1][1][r] = 0.f;
+  float bsum = 0.f;
   const bool sums_big = BIAS && cs0 == 0;
   const uint32_t one2 = sizeof(T) == 2 && std::is_same<T, bf16_t>::value ? 0x3f803f80u : 0x3c003c00u;  // two ones of T
   const uint4 ones = make_uint4(one2, one2, one2, one2);
@@ -570,11 +564,11 @@ __global__ void __launch_bounds__(512, 2) patch_reduce_kernel(PatchArgs a, const
     walk.advance(a, step);
   };
 #pragma unroll
-  for (int u = 0; u < D; ++u) fetch(ahead[u], begin + (2 * u + half) * kVx);
-  for (int64_t v0 = begin; v0 < end; v0 += 2 * D * kVx) {
+  for (int u = 0; u < D; ++u) fetch(ahead[u], begin + u * kTurn + half * kVx);
+  for (int64_t v0 = begin; v0 < end; v0 += D * kTurn) {
 #pragma unroll
     for (int u = 0; u < D; ++u) {
-      const int64_t v = v0 + 2 * u * kVx;
+      const int64_t v = v0 + u * kTurn;
       if (u > 0 && v >= end) break;
       T* s_tile = lds[u & 1][half];
       T* b_tile = s_tile + 2 * kBlock;
@@ -583,76 +577,76 @@ __global__ void __launch_bounds__(512, 2) patch_reduce_kernel(PatchArgs a, const
       for (int i = 0; i < 4; ++i)
         *reinterpret_cast<uint4*>(b_tile + (b_tap0 + 2 * i) * kBlock + b_vox * 32 + b_piece * 8) = ahead[u].b[i];
       __syncthreads();  // the other phase was read before the barrier of the round behind it
-      fetch(ahead[u], v + (2 * D + half) * kVx);
+      fetch(ahead[u], v + D * kTurn + half * kVx);
+      uint4 af[2][2], bf[2][2];  // [block or tap][k-step]
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        uint4 af[2], bf[2];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) af[i] = tr_fragment<T>(s_tile + i * kBlock + ks * 16 * 32, 32, lane);
+        for (int i = 0; i < 2; ++i) af[i][ks] = tr_fragment<T>(s_tile + i * kBlock + ks * 16 * 32, 32, lane);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) bf[j] = tr_fragment<T>(b_tile + (2 * wave + j) * kBlock + ks * 16 * 32, 32, lane);
+        for (int j = 0; j < 2; ++j) bf[j][ks] = tr_fragment<T>(b_tile + (2 * wave + j) * kBlock + ks * 16 * 32, 32, lane);
+      }
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            f32x16_t& sum = ks ? odd[i][j] : acc[i][j];
-            sum = Mma32<T>::run(af[i], bf[j], sum);
-          }
-        if constexpr (BIAS) {
-          if (sums_big) {  // every row of the block is the column sum
+        for (int j = 0; j < 2; ++j) {
+          const f32x16_t sum = Mma32<T>::run(af[i][1], bf[j][1], Mma32<T>::run(af[i][0], bf[j][0], none));
 #pragma unroll
-            for (int j = 0; j < 2; ++j) bacc[j] = Mma32<T>::run(ones, bf[j], bacc[j]);
-          }
+          for (int r = 0; r < 16; ++r) acc[i][j][r] += sum[r];
+        }
+      if constexpr (BIAS) {
+        if (sums_big) {  // every row of the block is the column sum, of both taps
+          f32x16_t sum = none;
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) sum = Mma32<T>::run(ones, bf[j][ks], sum);
+          bsum += sum[0];
         }
       }
     }
   }
+  // part[split][cs][tap][cb]: a lane holds column cb = lane % 32 and 16 rows of its block
+  float* dst = part + (int64_t)split * a.csmall * kTaps * a.cbig + ((int64_t)cs0 * kTaps + 2 * wave) * a.cbig + cb0 + (lane & 31);
+  const int kg = lane >> 5;
+  auto store = [&](const f32x16_t& sum, int i, int j) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int r = 0; r < 16; ++r) dst[((int64_t)(i * 32 + 8 * (r >> 2) + 4 * kg + (r & 3)) * kTaps + j) * a.cbig] = sum[r];
+  };
+  // half h keeps row block h and hands the other one over
+  float4* hand = reinterpret_cast<float4*>(lds);
+  float* sums = reinterpret_cast<float*>(lds) + 64 * 256;  // [half][tap pair][channel]
+  auto give = [&](const f32x16_t (&sum)[2]) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] += odd[i][j][r];
-  // half h keeps row block h and hands the other one over
+      for (int g = 0; g < 4; ++g)
+        hand[((half * 2 + j) * 4 + g) * 256 + tid] = make_float4(sum[j][4 * g], sum[j][4 * g + 1], sum[j][4 * g + 2], sum[j][4 * g + 3]);
+  };
+  auto take = [&](f32x16_t (&sum)[2], int i) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 o = hand[(((i ^ 1) * 2 + j) * 4 + g) * 256 + tid];
+        sum[j][4 * g] += o.x; sum[j][4 * g + 1] += o.y; sum[j][4 * g + 2] += o.z; sum[j][4 * g + 3] += o.w;
+      }
+      store(sum[j], i, j);
+    }
+  };
   __syncthreads();
-  float* hand = reinterpret_cast<float*>(lds);
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float v0 = acc[0][j][r], v1 = acc[1][j][r];
-      hand[((half * 2 + j) * 16 + r) * 256 + tid] = half ? v0 : v1;
-    }
-  if constexpr (BIAS) {
-    if (half) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) hand[(64 + j) * 256 + tid] = bacc[j][0];
-    }
-  }
+  if (half == 0) give(acc[1]);
+  else give(acc[0]);
   __syncthreads();
-  // part[split][cs][tap][cb]: a lane holds column cb = lane % 32 and 16 rows of its block
-  float* dst = part + (int64_t)split * a.csmall * kTaps * a.cbig;
-  const int col = lane & 31, kg = lane >> 5;
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float v0 = acc[0][j][r], v1 = acc[1][j][r];
-      const float other = hand[(((half ^ 1) * 2 + j) * 16 + r) * 256 + tid];
-      const int cs = cs0 + half * 32 + 8 * (r >> 2) + 4 * kg + (r & 3);
-      dst[((int64_t)cs * kTaps + 2 * wave + j) * a.cbig + cb0 + col] = half ? other + v1 : v0 + other;
-    }
-  if constexpr (BIAS) {
-    float* sums = hand + 66 * 256;  // [tap][channel], then their sum in tap order: one row of channels per split
-    if (half == 0 && kg == 0) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) sums[(2 * wave + j) * 32 + col] = bacc[j][0] + hand[(64 + j) * 256 + tid];
-    }
+  if (half == 0) take(acc[0], 0);
+  else take(acc[1], 1);
+  if constexpr (BIAS) {  // the sums of the wavefronts (tap pairs, halves) in that order: one row of channels per split
+    sums[(half * 4 + wave) * 32 + (lane & 31)] = bsum;
     __syncthreads();
     if (sums_big && threadIdx.x < 32) {
       float sum = 0.f;
 #pragma unroll
-      for (int t = 0; t < kTaps; ++t) sum += sums[t * 32 + threadIdx.x];
+      for (int t = 0; t < 8; ++t) sum += sums[t * 32 + threadIdx.x];
       bias_part[(int64_t)split * a.cbig + cb0 + threadIdx.x] = sum;
     }
   }
@@ -799,7 +793,10 @@ ReducePlan reduce_plan(const PatchArgs& a) {
   const double slice_us = 0.6e-6 * 4 * kTaps * a.csmall * a.cbig;
   int64_t best = 1;
   double best_us = 1e30;
-  for (int64_t s = 1; s <= rounds && (s == 1 || s * tiles <= kComputeUnits); s = s < 8 ? 2 * s : s + 8) {
+  // two ranges at least past four rounds: one of eight rounds rounds a sum more often than eight slices of one do (512 -> 256 at
+  // 4x8x8 0.56e-7 in one range, 0.55 in two; 13.0 -> 13.9 us)
+  const int64_t least = rounds > 4 && 2 * tiles <= kComputeUnits ? 2 : 1;
+  for (int64_t s = least; s <= rounds && (s <= least || s * tiles <= kComputeUnits); s = s < 8 ? 2 * s : s + 8) {
     const double us = 0.7 * (double)(cdiv(s * tiles, kComputeUnits) * cdiv(cdiv(rounds, s), 2)) + slice_us * (double)s;
     if (us < best_us) { best_us = us; best = s; }
   }
