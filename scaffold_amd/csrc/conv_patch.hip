@@ -22,7 +22,7 @@ constexpr int kTaps = 8;
 
 struct Voxel { int nn, d, h, w; };
 
-__device__ __forceinline__ Voxel decode_small(const PatchArgs& a, int64_t v) {
+__host__ __device__ __forceinline__ Voxel decode_small(const PatchArgs& a, int64_t v) {
   Voxel r;
   if (v <= 0x7fffffffLL) {  // 32-bit arithmetic when it fits
     uint32_t t = (uint32_t)v;
@@ -41,14 +41,14 @@ __device__ __forceinline__ Voxel decode_small(const PatchArgs& a, int64_t v) {
   return r;
 }
 
-__device__ __forceinline__ int64_t big_index(const PatchArgs& a, const Voxel& v, int tap) {
+__host__ __device__ __forceinline__ int64_t big_index(const PatchArgs& a, const Voxel& v, int tap) {
   return (((int64_t)v.nn * a.bd + 2 * v.d + (tap >> 2)) * a.bh + 2 * v.h + ((tap >> 1) & 1)) * a.bw + 2 * v.w + (tap & 1);
 }
 
 // A voxel that moves on by the same number of voxels every time (decoding it anew costs three divisions: at two wavefronts a
 // SIMD some 1200 cycles a round, which bounded the weight gradient). `at`: its patch's first big voxel.
 struct VoxelStep { int w, h, d; int64_t at, carry_w, carry_h, carry_d; };
-__device__ __forceinline__ VoxelStep voxel_step(const PatchArgs& a, int64_t voxels) {
+VoxelStep voxel_step(const PatchArgs& a, int64_t voxels) {
   const Voxel s = decode_small(a, voxels);
   VoxelStep r;
   r.w = s.w; r.h = s.h; r.d = s.d;
@@ -515,16 +515,16 @@ constexpr int kSmallTile = 64;      // small channels per workgroup (two row blo
 // voxel there) -- as one more MFMA row block of ones, sixteen voxels at a time from zero and on in 64 bits (four additions a round;
 // error over the sum of magnitudes with a chain of matrix steps and of slices -> with this and the slices' tree, e-9: 64 -> 32 at 64^3
 // 0.10 -> 0.07, at 32x64x64 0.14 -> 0.10, 512 -> 256 at 12x10x14 0.66 -> 0.42): bias_part[split][cb], in a fixed order.
-template <typename T, bool BIAS>
-__global__ void __launch_bounds__(512, 2)
+template <typename T, bool BIAS, int HALVES>
+__global__ void __launch_bounds__(256 * HALVES, 2)
 patch_reduce_kernel(PatchArgs a, const T* __restrict__ small, const T* __restrict__ big, float* __restrict__ part, int64_t total,
-                    int64_t per_split, int splits, int by_xcd, float* __restrict__ bias_part) {
+                    int64_t per_split, int splits, int by_xcd, VoxelStep step, float* __restrict__ bias_part) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int D = 2;                           // rounds requested ahead
   constexpr int kBlock = kVx * 32;               // elements of one [voxel][32 channels] block
   constexpr int kRound = (2 + kTaps) * kBlock;   // two blocks of the small tensor, one per tap of the big
-  constexpr int kTurn = 2 * kVx;                 // voxels of a round of both halves
-  __shared__ __attribute__((aligned(16))) T lds[2][2][kRound];
+  constexpr int kTurn = HALVES * kVx;            // voxels of a round of every half
+  __shared__ __attribute__((aligned(16))) T lds[2][HALVES][kRound];
   const int nz = a.cbig / 32, tiles = a.csmall / kSmallTile * nz;
   const int slot = blockIdx.x / kXcds;
   const int split = by_xcd ? slot / tiles * kXcds + (int)(blockIdx.x % kXcds) : (int)blockIdx.x / tiles;
@@ -548,7 +548,6 @@ patch_reduce_kernel(PatchArgs a, const T* __restrict__ small, const T* __restric
   const uint4 zero = make_uint4(0, 0, 0, 0);
   VoxelWalk walk;
   walk.start(a, begin + half * kVx + b_vox);
-  const VoxelStep step = voxel_step(a, 2 * kVx);
   int64_t tap_at[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) tap_at[i] = big_index(a, Voxel{0, 0, 0, 0}, b_tap0 + 2 * i);
@@ -613,40 +612,49 @@ patch_reduce_kernel(PatchArgs a, const T* __restrict__ small, const T* __restric
 #pragma unroll
     for (int r = 0; r < 16; ++r) dst[((int64_t)(i * 32 + 8 * (r >> 2) + 4 * kg + (r & 3)) * kTaps + j) * a.cbig] = sum[r];
   };
-  // half h keeps row block h and hands the other one over
-  float4* hand = reinterpret_cast<float4*>(lds);
-  double* sums = reinterpret_cast<double*>(lds) + 32 * 256;  // [half][tap pair][channel]
-  auto give = [&](const f32x16_t (&sum)[2]) {
+  double* sums = reinterpret_cast<double*>(lds);  // [half][tap pair][channel]
+  if constexpr (HALVES == 1) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        hand[((half * 2 + j) * 4 + g) * 256 + tid] = make_float4(sum[j][4 * g], sum[j][4 * g + 1], sum[j][4 * g + 2], sum[j][4 * g + 3]);
-  };
-  auto take = [&](f32x16_t (&sum)[2], int i) {
+      for (int j = 0; j < 2; ++j) store(acc[i][j], i, j);
+    if constexpr (BIAS) __syncthreads();
+  } else {
+    // half h keeps row block h and hands the other one over
+    float4* hand = reinterpret_cast<float4*>(lds);
+    sums += 32 * 256;
+    auto give = [&](const f32x16_t (&sum)[2]) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const float4 o = hand[(((i ^ 1) * 2 + j) * 4 + g) * 256 + tid];
-        sum[j][4 * g] += o.x; sum[j][4 * g + 1] += o.y; sum[j][4 * g + 2] += o.z; sum[j][4 * g + 3] += o.w;
+        for (int g = 0; g < 4; ++g)
+          hand[((half * 2 + j) * 4 + g) * 256 + tid] = make_float4(sum[j][4 * g], sum[j][4 * g + 1], sum[j][4 * g + 2], sum[j][4 * g + 3]);
+    };
+    auto take = [&](f32x16_t (&sum)[2], int i) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 o = hand[(((i ^ 1) * 2 + j) * 4 + g) * 256 + tid];
+          sum[j][4 * g] += o.x; sum[j][4 * g + 1] += o.y; sum[j][4 * g + 2] += o.z; sum[j][4 * g + 3] += o.w;
+        }
+        store(sum[j], i, j);
       }
-      store(sum[j], i, j);
-    }
-  };
-  __syncthreads();
-  if (half == 0) give(acc[1]);
-  else give(acc[0]);
-  __syncthreads();
-  if (half == 0) take(acc[0], 0);
-  else take(acc[1], 1);
+    };
+    __syncthreads();
+    if (half == 0) give(acc[1]);
+    else give(acc[0]);
+    __syncthreads();
+    if (half == 0) take(acc[0], 0);
+    else take(acc[1], 1);
+  }
   if constexpr (BIAS) {  // the sums of the wavefronts (tap pairs, halves) in that order: one row of channels per split
     sums[(half * 4 + wave) * 32 + (lane & 31)] = bsum;
     __syncthreads();
     if (sums_big && threadIdx.x < 32) {
       double sum = 0.;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) sum += sums[t * 32 + threadIdx.x];
+      for (int t = 0; t < 4 * HALVES; ++t) sum += sums[t * 32 + threadIdx.x];
       bias_part[(int64_t)split * a.cbig + cb0 + threadIdx.x] = (float)sum;
     }
   }
@@ -779,28 +787,41 @@ int launch_scatter(const PatchArgs& a, const void* small, const void* w, bool de
   return check_launch("patch_scatter_any_kernel");
 }
 
-struct ReducePlan { int splits; int64_t per_split; };
+struct ReducePlan { int halves; int splits; int64_t per_split; };
 
 // Splits of the voxels: up to one workgroup per CU, and fewer where the slices (written, then read by the sum) cost more than
 // the shorter ranges gain. 0.7 us is a round of both halves, 0.6 us a megabyte of slices, fitted to sweeps of 1 to 256 splits over
 // 17 problems (best plan within 5 % on each). Two workgroups of four wavefronts per CU, a slice each -> this, us with the sum: 128 -> 64
-// at 64^3 119 -> 106, at 32^3 24.4 -> 20.5, at 48x40x56 84 -> 38; 64 -> 32 at 64^3 36 -> 33; 256 -> 128 at 32^3 49 -> 41, at 8x16x16 23 -> 15;
-// 512 -> 256 at 4x8x8 24 -> 13. Eight at a time: a range of voxels per XCD.
+// at 64^3 120 -> 113, at 32^3 25 -> 21.5, at 48x40x56 84 -> 39; 64 -> 32 at 64^3 36 -> 34.6; 256 -> 128 at 32^3 49 -> 41, at 8x16x16 23 -> 15;
+// 512 -> 256 at 4x8x8 24 -> 14. Eight at a time: a range of voxels per XCD.
+// Where the rounds of all tiles do not give every CU one, a workgroup has one half: its start, and the two halves' meeting in LDS, cost
+// more than the longer range. 0.65 us is a round then, 0.3 a megabyte of slices, 0.07 each of a few slices or 1.2 the grouped sum of many.
+// us, such slices of a round at most in workgroups of two halves -> one: 64 -> 32 at 4^3 7.7 -> 6.8, at 12^3 10.8 -> 8.9, at 10x8x39 10.9 -> 9.4,
+// 128 -> 64 at 8^3 8.9 -> 8.3, 256 -> 128 at 5x8x4 9.6 -> 9.1; from the line on two are better: 64 -> 32 at 24^3 (432 rounds) 13.2 one, 12.6 two,
+// 256 -> 128 at 8x16x16 (1024) 15.8 and 14.6.
 ReducePlan reduce_plan(const PatchArgs& a) {
   const int64_t total = small_voxels(a);
   const int64_t tiles = (int64_t)(a.csmall / kSmallTile) * (a.cbig / 32);
   const int64_t rounds = cdiv(total, kVx);
-  const double slice_us = 0.6e-6 * 4 * kTaps * a.csmall * a.cbig;
+  const double slice_mb = 4e-6 * kTaps * a.csmall * a.cbig;
   int64_t best = 1;
   double best_us = 1e30;
-  // two ranges at least past four rounds: one of eight rounds rounds a sum more often than eight slices of one do (512 -> 256 at
-  // 4x8x8 0.56e-7 in one range, 0.55 in two; 13.0 -> 13.9 us)
-  const int64_t least = rounds > 4 && 2 * tiles <= kComputeUnits ? 2 : 1;
-  for (int64_t s = least; s <= rounds && (s <= least || s * tiles <= kComputeUnits); s = s < 8 ? 2 * s : s + 8) {
-    const double us = 0.7 * (double)(cdiv(s * tiles, kComputeUnits) * cdiv(cdiv(rounds, s), 2)) + slice_us * (double)s;
-    if (us < best_us) { best_us = us; best = s; }
-  }
   ReducePlan p;
+  p.halves = rounds * tiles < kComputeUnits ? 1 : 2;
+  if (p.halves == 1) {
+    for (int64_t s = 1; s <= rounds; ++s) {
+      const double us = 0.65 * (double)cdiv(rounds, s) + 0.3 * slice_mb * (double)s + (s < 32 ? 0.07 * (double)s : 1.2);
+      if (us < best_us) { best_us = us; best = s; }
+    }
+  } else {
+    // two ranges at least past four rounds: one of eight rounds rounds a sum more often than eight slices of one do (512 -> 256 at
+    // 4x8x8 0.56e-7 in one range, 0.55 in two; 13.0 -> 13.9 us)
+    const int64_t least = rounds > 4 && 2 * tiles <= kComputeUnits ? 2 : 1;
+    for (int64_t s = least; s <= rounds && (s <= least || s * tiles <= kComputeUnits); s = s < 8 ? 2 * s : s + 8) {
+      const double us = 0.7 * (double)(cdiv(s * tiles, kComputeUnits) * cdiv(cdiv(rounds, s), 2)) + 0.6 * slice_mb * (double)s;
+      if (us < best_us) { best_us = us; best = s; }
+    }
+  }
   p.per_split = cdiv(rounds, best) * kVx;
   p.splits = (int)cdiv(total, p.per_split);
   return p;
@@ -814,13 +835,19 @@ int launch_reduce(const PatchArgs& a, const void* small, const void* big, void* 
   const int by_xcd = p.splits > 4;
   const dim3 grid((unsigned)((by_xcd ? cdiv(p.splits, kXcds) * kXcds : p.splits) * tiles));
   const int64_t nelem = (int64_t)a.csmall * kTaps * a.cbig;
+  const VoxelStep step = voxel_step(a, p.halves * kVx);
   float* bias_part = (float*)ws + (int64_t)p.splits * nelem;  // behind the weight slices
-  if (gb != nullptr)
-    hipLaunchKernelGGL((patch_reduce_kernel<T, true>), grid, dim3(512), 0, st, a, (const T*)small, (const T*)big, (float*)ws, total,
-                       p.per_split, p.splits, by_xcd, bias_part);
-  else
-    hipLaunchKernelGGL((patch_reduce_kernel<T, false>), grid, dim3(512), 0, st, a, (const T*)small, (const T*)big, (float*)ws, total,
-                       p.per_split, p.splits, by_xcd, (float*)nullptr);
+#define SFH_PATCH_REDUCE(BIAS, HALVES)                                                                                           \
+  hipLaunchKernelGGL((patch_reduce_kernel<T, BIAS, HALVES>), grid, dim3(256 * HALVES), 0, st, a, (const T*)small, (const T*)big, \
+                     (float*)ws, total, p.per_split, p.splits, by_xcd, step, bias_part)
+  if (gb != nullptr) {
+    if (p.halves == 2) SFH_PATCH_REDUCE(true, 2);
+    else SFH_PATCH_REDUCE(true, 1);
+  } else {
+    if (p.halves == 2) SFH_PATCH_REDUCE(false, 2);
+    else SFH_PATCH_REDUCE(false, 1);
+  }
+#undef SFH_PATCH_REDUCE
   if (int rc = check_launch("patch_reduce_kernel")) return rc;
   if (gb == nullptr) return sum_slices(g_dtype, (const float*)ws, g, nelem, p.splits, st);
   // both sums in one launch

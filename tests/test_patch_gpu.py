@@ -119,3 +119,29 @@ def test_backward_weight(n, cin, cout, extents, dtype):
     assert (fb.double() - bias).abs().max() <= 1e-6 * gy.double().abs().sum((0, 2, 3, 4)).max()
     bw, _ = ct.conv_transpose3d_backward_weight_bias(x, wt.shape, gy, 2)
     assert torch.equal(bw, gw)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("odd", [0, 1])
+@pytest.mark.parametrize("n,cin,cout,extents", [
+    (1, 64, 32, (2, 3, 5)),           # a round that is cut
+    (2, 64, 32, (3, 5, 7)),           # the step of a walk is longer than a row, than a plane, and reaches over samples
+    (1, 64, 32, (12, 12, 12)),        # a range per round
+    (1, 64, 32, (16, 17, 30)),        # 255 rounds: the last of one half
+    (1, 64, 32, (17, 17, 29)),        # 262: two
+    (2, 128, 64, (9, 10, 11)),        # 62 rounds of four tiles
+    (1, 512, 256, (3, 5, 6)),         # three rounds of 64
+    (1, 512, 256, (5, 5, 5)),         # four: two halves
+    (2, 128, 64, (11, 15, 18)),
+])
+def test_weight_gradient_of_small_and_odd_volumes(n, cin, cout, extents, odd, dtype):
+    """The stride-2 convolution's weight gradient is the same kernel with the roles turned; with an odd big extent a walk over the small
+    voxels skips the plane, row or voxel that no window covers."""
+    g = torch.Generator("cuda").manual_seed(3)
+    d, h, w = extents
+    small = torch.randint(-2, 3, (n, cin, d, h, w), generator=g, device="cuda").to(dtype).contiguous(memory_format=CL)
+    big = torch.randint(-2, 3, (n, cout, 2 * d + odd, 2 * h + odd, 2 * w + odd), generator=g, device="cuda").to(dtype).contiguous(memory_format=CL)
+    got = sa.conv3d_backward_weight(big, (cin, cout, 2, 2, 2), small, 2, 0, grad_dtype=torch.float32)
+    rows = big[:, :, :2 * d, :2 * h, :2 * w].double().reshape(n, cout, d, 2, h, 2, w, 2).permute(0, 2, 4, 6, 3, 5, 7, 1).reshape(n * d * h * w, -1)
+    want = (small.permute(0, 2, 3, 4, 1).reshape(-1, cin).double().t() @ rows).view(cin, 2, 2, 2, cout).permute(0, 4, 1, 2, 3)
+    assert torch.equal(got.double(), want)  # whole numbers whose sums stay far below 2^24
