@@ -434,7 +434,7 @@ __global__ void __launch_bounds__(256, 2) patch_scatter_kernel(PatchArgs a, cons
   }
 }
 
-// The general form, for reduction widths whose weights do not fit in registers.
+// The general form, for reduction widths whose weights do not fit in registers and for the smallest volumes.
 // A wavefront owns 32 small voxels x one block of 32 big channels x TS of the 8 taps.
 // grid = (voxel tiles of 128, cbig / 32, 8 / TS). TS = 8 reads the small tensor once; TS = 1 and 2 are for launches that
 // would otherwise leave most of the chip idle or give a CU a single long chain of dependent loads (the deeper levels):
@@ -756,10 +756,14 @@ int launch_scatter(const PatchArgs& a, const void* small, const void* w, bool de
                          (halo_elems * (int64_t)sizeof(T)) % 16 != 0))
     return fail(SFH_ERR_UNSUPPORTED, "convT3d fwd: a slab output needs one sample and 16-byte aligned faces");
   const int64_t face_pieces = halo_elems > 0 ? halo_elems * (int64_t)sizeof(T) / 16 : 0;
-  // Weights of one (512 channels) or two columns fit in a wavefront's registers: the kept form, at every volume. General form ->
+  // Weights of one (512 channels) or two columns fit in a wavefront's registers: the kept form. General form ->
   // kept form, packed weight, us: 128 -> 64 at 64^3 120 -> 74, at 32^3 20.7 -> 12.3, at 16x32x32 12 -> 8.5; 64 -> 32 at 64^3 47 -> 28,
   // at 32x64x64 25 -> 17; 256 -> 128 at 32^3 48 -> 26, at 8x16x16 7.8 -> 5.9; 512 -> 256 at 16^3 29 -> 15, at 4x8x8 7.2 -> 4.8.
-  if (patch_scatter_reads_dense(a)) {
+  // With the weight packed, a launch of few short reductions stays with the general one, whose wavefronts have one tap each and no turn
+  // through LDS: 64 -> 32 at 10^3 4.2 kept, 3.9 general, at 16^3 4.4 and 4.3, 128 -> 64 at 4^3 4.3 and 4.0, 256 -> 128 at 4^3 5.3 and 4.8; from the
+  // line on the kept one is as fast or faster (128 -> 64 at 10^3 4.5 both, 64 -> 32 at 16x41x7 4.4 and 4.9).
+  const int64_t reductions = cdiv(total, 32) * (a.cbig / 32) * a.csmall;
+  if (patch_scatter_reads_dense(a) && (dense || reductions > 64 * 128)) {
     if (a.csmall == 64) return launch_scatter_kept<T, 4, 2>(a, small, w, dense, bias, big, st, face_pieces, big_elems);
     if (a.csmall == 128) return launch_scatter_kept<T, 8, 2>(a, small, w, dense, bias, big, st, face_pieces, big_elems);
     if (a.csmall == 256) return launch_scatter_kept<T, 16, 2>(a, small, w, dense, bias, big, st, face_pieces, big_elems);
