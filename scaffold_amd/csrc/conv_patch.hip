@@ -159,8 +159,15 @@ patch_gather_kept_kernel(PatchArgs a, const T* __restrict__ big, const T* __rest
       if constexpr (C::BUFS == 1) __syncthreads();
     }
   }
+  // with 32 fragments of weights a lane has no registers left for its bias values: they wait in LDS (held, they spilled 8)
+  constexpr bool kBiasInLds = C::KH == 4;
+  __shared__ float s_bias[kBiasInLds ? 32 * C::NBW : 1];
   float add[16];
-  load_block_bias<T>(bias, blk * 32, kg, add);
+  if constexpr (kBiasInLds) {
+    if (tid < 32 * C::NBW) s_bias[tid] = bias != nullptr ? to_float(bias[blk0 * 32 + tid]) : 0.f;
+  } else {
+    load_block_bias<T>(bias, blk * 32, kg, add);
+  }
   int phase = 0;
   for (int64_t t = group; t < tiles; t += groups, phase ^= C::BUFS - 1) {
     char* tile = lds[phase];
@@ -195,6 +202,10 @@ patch_gather_kept_kernel(PatchArgs a, const T* __restrict__ big, const T* __rest
     if (kpart == 0) {
       const int64_t v = t * C::V + part * 32 + (lane & 31);
       const bool valid = v < total;
+      if constexpr (kBiasInLds) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) add[r] = s_bias[unit % C::NBW * 32 + 8 * (r / 4) + 4 * kg + r % 4];
+      }
       store_block_plus<T>(acc, small + (valid ? v : total - 1) * a.csmall + blk * 32, add, kg, valid);
     }
   }
@@ -675,7 +686,7 @@ int gather_blocks(const PatchArgs& a) {
 // The kept form takes the channel counts it has tiles for once there are a few dozen tiles; below that the chain of one
 // workgroup's tile is longer than the deep kernel's. Before -> kept, packed weight, us: 64 -> 32 at 64^3 34 -> 26, at 32x64x64
 // 19 -> 15, at 16^3 3.3 -> 4.2; 128 -> 64 at 64^3 108 -> 65, at 32^3 15.1 -> 11.2, at 16x32x32 11.8 -> 7.3, at 8^3 3.7 -> 4.8;
-// 256 -> 128 at 32^3 38 -> 25, at 8x16x16 6.9 -> 6.7, at 5x7x9 (two samples) 4.8 -> 6.7; 512 -> 256 at 16^3 38 -> 23.
+// 256 -> 128 at 32^3 38 -> 25, at 8x16x16 6.9 -> 6.7, at 5x7x9 (two samples) 4.8 -> 6.7; 512 -> 256 at 16^3 38 -> 22.
 bool gather_kept(const PatchArgs& a) {
   if (small_voxels(a) * a.cbig < (1 << 18)) return false;
   return a.cbig == 32 || a.cbig == 256 ? a.csmall % 64 == 0 : (a.cbig == 64 || a.cbig == 128) && a.csmall % 128 == 0;
@@ -883,7 +894,7 @@ int patch_gather(const PatchArgs& a, int dtype, const void* big, const void* w, 
   return launch_gather<fp16_t>(a, big, w, dense, bias, small, st);
 }
 
-// (256 channels: the registers of the weights and of the layout pass together spill, 33 us against 23 + a packing at 16^3)
+// (256 channels: the registers of the weights and of the layout pass together spill, 33 us against 22 + a packing at 16^3)
 bool patch_gather_reads_dense(const PatchArgs& a) { return gather_kept(a) && a.cbig != 256; }
 // (the kept form numbers big voxels in 32 bits)
 bool patch_scatter_reads_dense(const PatchArgs& a) {

@@ -44,7 +44,7 @@ def _kernels():
                     yield k[".name"], k
 
 
-@pytest.mark.parametrize("kernel", ["patch_reduce_kernel"])
+@pytest.mark.parametrize("kernel", ["patch_reduce_kernel", "patch_gather_kept_kernel"])
 def test_no_scratch(kernel):
     found = [(n, k) for n, k in _kernels() if kernel in n]
     assert found
