@@ -531,12 +531,12 @@ extern "C" int sfh_conv3d_pack_weights_batch(const sfh_pack_item* items, int32_t
         return rc;
     }
   }
-  constexpr int kGroup = 46;  // (an item adds up to two jobs; 48 jobs are one launch)
-  MfmaPackItem jobs[kGroup + 2];
+  constexpr int kGroup = 2 * kPackTable;  // (an item adds up to two jobs: the forms of a full table)
+  MfmaPackItem jobs[kGroup];
   int njobs = 0;
   for (int i = 0; i < nitems; ++i) {
     collect_pack_jobs(&items[i].desc, dtype, items[i].w, items[i].w_stride, items[i].packed_fwd, items[i].packed_dgrad, jobs, &njobs);
-    if (njobs >= kGroup || i + 1 == nitems) {
+    if (njobs + 2 > kGroup || i + 1 == nitems) {
       if (njobs > 0)
         if (int rc = mfma_pack_weight_batch(jobs, njobs, dtype, (hipStream_t)stream)) return rc;
       njobs = 0;

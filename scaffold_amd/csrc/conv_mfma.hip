@@ -374,7 +374,7 @@ struct TileJob {
   int nb0, nb1, taps;
   uint16_t flip, fp32;
 };
-constexpr int kTileBatch = 72;  // (the table stays under 4 KB of kernel arguments)
+constexpr int kTileBatch = kPackTable;
 template <int N>
 struct TileBatch {
   TileJob job[N];

@@ -35,6 +35,7 @@ struct MfmaPackItem {
   void* packed;
   bool fp32_source;  // `w` is fp32: rounded to the packed dtype on the way
 };
+constexpr int kPackTable = 72;  // dense weights, both forms each, that one launch takes (the table stays under 4 KB of kernel arguments)
 int mfma_pack_weight_batch(const MfmaPackItem* items, int n, int dtype, hipStream_t st);
 // Bytes of fp32 slices the kernel needs when it cuts the reduction channels to fill the chip (0 when it does not).
 size_t mfma_conv_partial_bytes(const MfmaConvArgs& a);
