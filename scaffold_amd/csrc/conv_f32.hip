@@ -285,7 +285,7 @@ wgrad_f32_kernel(WgradArgs a, const float* __restrict__ x, const float* __restri
   const int kd = b % 3; b /= 3;
   const int cib = b % cibs, cob = b / cibs;
   const int segs = (a.ow + kSeg - 1) / kSeg, row_tiles = (a.oh + kRows - 1) / kRows;
-  const int begin = split * per, end = begin + per < steps ? begin + per : steps;
+  const int begin = split * per, end = steps - begin < per ? steps : begin + per;
   // The range's steps in turn, segments first: positions are kept and moved on (all of it scalar), a thread's places in a step and
   // its offsets from the step's first voxel are constants.
   const int next_plane = begin / segs / row_tiles;
@@ -448,10 +448,9 @@ static int64_t wgrad_per(const WgradArgs& a) {
 }
 
 bool f32_wgrad_supported(const WgradArgs& a) {
-  // offsets inside a row and the count of passes of 8 voxels are 32-bit
-  const int64_t reach = 4LL * (a.iw > a.ow ? a.iw : a.ow) + 64 + 4LL * a.pw;
-  if (reach * (a.cin > a.cout ? a.cin : a.cout) >= 0x7ffffff0LL) return false;
-  if ((int64_t)a.n * a.od * a.oh * ((a.ow + 7) / 8) >= 0x7fffffffLL - 4) return false;
+  // places along a row and a column and the count of steps are 32-bit, the offsets they make 64-bit
+  constexpr int64_t kLast = 0x7fffffffLL - 64;
+  if (a.n < 1 || a.od < 1 || a.oh > kLast || a.ow > kLast || a.ih > kLast || a.iw > kLast || wgrad_steps(a) > 0x7fffffffLL) return false;
   return a.cin % 32 == 0 && a.cout % 32 == 0 && a.n >= 1 && a.od >= 1 && a.oh >= 1 && a.ow >= 1 && a.pd >= 0 && a.ph >= 0 && a.pw >= 0;
 }
 

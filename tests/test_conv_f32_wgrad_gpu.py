@@ -55,3 +55,20 @@ def test_infinities_that_no_output_meets(width):
     gy = torch.randn((1, 32, 2, 3, width - 2), generator=g, device="cuda").contiguous(memory_format=CL)
     got = sa.conv3d_backward_weight(x, (32, 32, 3, 3, 3), gy, 1, 0)
     assert torch.isfinite(got[..., :2]).all() and not torch.isfinite(got[..., 2]).any()
+
+
+def test_a_row_of_two_gibibytes():
+    """Offsets past 2^31 bytes inside a row, in the first, a middle and the last step: whole numbers, so the sums are exact."""
+    width = 16_800_000
+    g = torch.Generator("cuda").manual_seed(6)
+    x = torch.randint(-1, 2, (width, 32), generator=g, device="cuda", dtype=torch.int8).float()
+    gy = torch.randint(-1, 2, (width, 32), generator=g, device="cuda", dtype=torch.int8).float()
+    as_volume = lambda t: t.view(1, 1, 1, width, 32).permute(0, 4, 1, 2, 3)
+    got = sa.conv3d_backward_weight(as_volume(x), (32, 32, 3, 3, 3), as_volume(gy), 1, 1)
+    want = torch.zeros_like(got, dtype=torch.float64)
+    for kw in range(3):
+        lo, hi = max(0, 1 - kw), min(width, width + 1 - kw)  # outputs whose voxel at this tap exists
+        for part in range(lo, hi, 1 << 21):
+            end = min(hi, part + (1 << 21))
+            want[:, :, 1, 1, kw] += gy[part:end].double().t() @ x[part + kw - 1:end + kw - 1].double()
+    assert torch.equal(got.double(), want)

@@ -39,3 +39,8 @@ def test_deep_thin_volumes(cin, cout, spatial, kernel):
     padded = _kernel(1, cout, cin, spatial, "bwd-data")
     d, h, w = spatial
     assert padded == kernel and _kernel(1, cout, cin, (d + 2, h, w), "bwd-data", (0, 1, 1)) == padded
+
+
+def test_fp32_weight_gradient_of_long_rows():
+    """A row of 2 GiB and more: its offsets are 64-bit, the tiled kernel takes it (the untiled one makes no slices)."""
+    assert c3.split_count((1, 32, 1, 1, 16_800_000), (32, 32, 3, 3, 3), 1, 1, 1, torch.float32) > 1
