@@ -44,6 +44,8 @@ struct Brick {
   static constexpr int ROW = NSUB == 1 ? 384 : BW * 16;
   static constexpr int PLANE = ((BD * BH * ROW - 64 + 255) / 256) * 256 + 64;
   static constexpr int SLOT = 4 * PLANE + 16;
+  // byte offset of a brick voxel in its plane (dense rows: not by row and column, which is 130 instructions a round of four chunks and 1 % of the time)
+  static __device__ __forceinline__ int at(int vox) { return ROW == BW * 16 ? vox * 16 : vox / BW * ROW + vox % BW * 16; }
   // byte offset of (tap, k-step) relative to a lane's voxel at tap (0, 0, 0)
   static constexpr int tap_off(int tap) { return ((tap / 9) * BH + (tap / 3) % 3) * ROW + tap % 3 * 16; }
 };
@@ -135,7 +137,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
       for (int u = 0; u < ITERS; ++u) {
         const int p = u * 256 + tid;
         const int q = p % (4 * R), vox = p / (4 * R);
-        if (p < PIECES) *reinterpret_cast<uint4*>(lds + (q >> 2) * SLOT + (q & 3) * PLANE + vox / BW * B::ROW + vox % BW * 16) = v[u];
+        if (p < PIECES) *reinterpret_cast<uint4*>(lds + (q >> 2) * SLOT + (q & 3) * PLANE + B::at(vox)) = v[u];
       }
     }
     __syncthreads();
