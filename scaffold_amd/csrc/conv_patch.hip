@@ -811,7 +811,7 @@ struct ReducePlan { int halves; int splits; int64_t per_split; };
 // 512 -> 256 at 4x8x8 24 -> 14. Eight at a time: a range of voxels per XCD.
 // Where the rounds of all tiles do not give every CU one, a workgroup has one half: its start, and the two halves' meeting in LDS, cost
 // more than the longer range. 0.65 us is a round then, 0.3 a megabyte of slices, 0.07 each of a few slices or 1.2 the grouped sum of many.
-// us, such slices of a round at most in workgroups of two halves -> one: 64 -> 32 at 4^3 7.7 -> 6.8, at 12^3 10.8 -> 8.9, at 10x8x39 10.9 -> 9.4,
+// us, workgroups of two halves under their own plan -> of one: 64 -> 32 at 4^3 7.7 -> 6.8, at 12^3 10.8 -> 8.9, at 10x8x39 10.9 -> 9.4,
 // 128 -> 64 at 8^3 8.9 -> 8.3, 256 -> 128 at 5x8x4 9.6 -> 9.1; from the line on two are better: 64 -> 32 at 24^3 (432 rounds) 13.2 one, 12.6 two,
 // 256 -> 128 at 8x16x16 (1024) 15.8 and 14.6.
 ReducePlan reduce_plan(const PatchArgs& a) {
