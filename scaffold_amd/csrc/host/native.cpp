@@ -623,10 +623,27 @@ struct ConvSaved {
     Problem prob;
     TORCH_INTERNAL_ASSERT(make_problem(in_sizes, w_sizes, s, p, d, code_of(gy.scalar_type()), prob));
     if (need_x || need_2) {
-      auto gx = launch_dgrad(prob, gy, wt, packed, pair ? first_channels : 0);
-      if (halo > 0) {
-        gx.first = gx.first.narrow(2, halo, depth);
-        if (pair) gx.second = gx.second.narrow(2, halo, depth);
+      // The faces of a slab are zeros that the module put there: nobody receives their gradients.  The planes between them
+      // are the data gradient of the padded problem, whose launch has no planes to drop (on 8 planes a fifth of the work) and
+      // no workgroups past a round for them; a voxel's sum is the same.  Where the padded problem is not one the gradient
+      // serves (a halo wider than the kernel reaches) the slab's is cut.
+      Problem inner = prob;
+      int64_t cut = halo;
+      if (halo > 0 && p[0] + halo <= (int64_t)d[0] * (w_sizes[2] - 1)) {
+        std::vector<int64_t> in = in_sizes;
+        in[2] = depth;
+        const int32_t padding[3] = {p[0] + (int32_t)halo, p[1], p[2]};
+        Problem padded;
+        if (make_problem(in, w_sizes, s, padding, d, prob.key.code, padded) && padded.sizes->packed[1] == prob.sizes->packed[1] &&
+            (!pair || sfh_conv3d_pair_supported(padded.desc(), prob.key.code, (int32_t)first_channels, 1))) {
+          inner = padded;
+          cut = 0;
+        }
+      }
+      auto gx = launch_dgrad(inner, gy, wt, packed, pair ? first_channels : 0);
+      if (cut > 0) {
+        gx.first = gx.first.narrow(2, cut, depth);
+        if (pair) gx.second = gx.second.narrow(2, cut, depth);
       }
       if (need_x) out[0] = gx.first;
       if (need_2) out[3] = gx.second;
