@@ -42,6 +42,13 @@ constexpr int kShiftRows = 32;   // voxels that define the shift K
 constexpr int kMaxSplit = 2048;  // workgroups per sample
 constexpr int kFillWorkgroups = 256;   // workgroups a launch aims for when the sample is small: one per compute unit
 
+// A tensor of more bytes than this is read past the caches' retention (the kernels' STREAM): with its gradient it is more than the
+// 256 MiB memory-side cache holds, so what a pass leaves there is gone before the next pass comes to it, and putting it there
+// pushes out lines that have still to be written. us at 64 channels of 128^3 in bf16 (268 MB): statistics 67 -> 45, gn_normalize
+// 86 -> 82, gn_bwd_partial 132 -> 91, gn_dx 147 -> 150, the four 449 -> 385; in a training step gn_dx 147 -> 132, gn_bwd_partial 108 -> 92,
+// gn_normalize 99 -> 88. Forward and backward alone over the size: 48 MiB 78 -> 80, 64 MiB 95 -> 103, 128 MiB 200 -> 199, 192 MiB 339 -> 314.
+constexpr int64_t kStreamBytes = 128ll << 20;
+
 struct GnPlan {
   bool vector;
   int vec;    // elements per thread and row
@@ -50,6 +57,7 @@ struct GnPlan {
   int slots;  // group slots per thread: max(1, vec / (C/G))
   int nsplit; // workgroups per sample (reduction and elementwise passes alike)
   int64_t rows_per_split;
+  bool stream;  // operands are read past the caches' retention
 };
 
 GnPlan make_plan(const sfh_groupnorm_desc& p, int x_dtype, bool aligned) {
@@ -79,6 +87,7 @@ GnPlan make_plan(const sfh_groupnorm_desc& p, int x_dtype, bool aligned) {
   if (cdiv(p.spatial, rows) > kMaxSplit) rows = cdiv(cdiv(p.spatial, kMaxSplit), pl.rpp) * pl.rpp;
   pl.rows_per_split = rows;
   pl.nsplit = (int)cdiv(p.spatial, rows);
+  pl.stream = (int64_t)p.n * p.spatial * p.c * (x_dtype == SFH_FP32 ? 4 : 2) > kStreamBytes;
   return pl;
 }
 
@@ -217,7 +226,7 @@ __device__ __forceinline__ void fold_groups(const float* buf, float* out, int G,
 
 // ---- forward: partial statistics (vector path) --------------------------------------------
 // scratch (floats): shift[N][G] | part[N][nsplit][2][G]
-template <typename T, int SLOTS>
+template <typename T, int SLOTS, bool STREAM>
 __global__ void __launch_bounds__(kBlock) gn_stats_partial(const T* __restrict__ x, float* __restrict__ shift,
                                                            float* __restrict__ part, int64_t S, int C, int G, int tpr, int rpp,
                                                            int nsplit, int64_t rows_per_split) {
@@ -254,7 +263,7 @@ __global__ void __launch_bounds__(kBlock) gn_stats_partial(const T* __restrict__
   }
   // the workgroup's first rows are requested before the shift is known: the reductions below wait for nothing of theirs
   Piece<T, V> cur[U];
-  fetch_rows<T, V, U>(cur, xs, row, step, end, begin, C, active);
+  fetch_rows<STREAM>(cur, xs, row, step, end, begin, C, active);
   block_row_reduce<SLOTS>(kv, buf, tpr, rpp, active);
   fold_groups<SLOTS, 1>(buf, out, G, cg, V);
   const float kinv = 1.f / ((float)krows * (float)cg);
@@ -274,7 +283,7 @@ __global__ void __launch_bounds__(kBlock) gn_stats_partial(const T* __restrict__
     while (row < end) {
       const int64_t next = row + U * step;
       Piece<T, V> nxt[U];
-      if (next < end) fetch_rows<T, V, U>(nxt, xs, next, step, end, begin, C, true);
+      if (next < end) fetch_rows<STREAM>(nxt, xs, next, step, end, begin, C, true);
       if (row + (U - 1) * step < end) {  // a whole batch
         float f0[V], f1[V], f2[V], f3[V];
         cur[0].unpack(f0);
@@ -501,7 +510,7 @@ __device__ __forceinline__ void fold_welford_records(const float* __restrict__ r
 // When the sample's split partials are few (fold_in_consumer), every workgroup derives mean and rstd from them itself
 // (mean = K + S1/m, var = S2/m - (S1/m)^2, rstd = 1/sqrt(var + eps)): 32 KiB from L2 cost less than a launch of their
 // own, and the first workgroup of a sample writes them out for the backward pass. Otherwise gn_stats_finalize has run.
-template <typename T, typename TO>
+template <typename T, typename TO, bool STREAM>
 __global__ void __launch_bounds__(kBlock) gn_normalize(const T* __restrict__ x, TO* __restrict__ y, const float* __restrict__ shift,
                                                        const float* __restrict__ part, float* __restrict__ mean,
                                                        float* __restrict__ rstd, const void* __restrict__ gamma,
@@ -525,7 +534,7 @@ __global__ void __launch_bounds__(kBlock) gn_normalize(const T* __restrict__ x, 
   const int64_t step = rpp;
   int64_t row = begin + r;
   Piece<T, V> cur[U];
-  fetch_rows<T, V, U>(cur, xs, row, step, end, begin, C, r < rpp);
+  fetch_rows<STREAM>(cur, xs, row, step, end, begin, C, r < rpp);
   // `npart` partial records per sample: the statistics pass's own (one per workgroup of this grid, sums about the
   // common shift), or (`welford`) the records the producer of x left
   if (welford && fold_in_consumer(G, npart, kGnRecordFloats)) {
@@ -588,7 +597,7 @@ __global__ void __launch_bounds__(kBlock) gn_normalize(const T* __restrict__ x, 
   while (row < end) {
     const int64_t next = row + U * step;
     Piece<T, V> nxt[U];
-    if (next < end) fetch_rows<T, V, U>(nxt, xs, next, step, end, begin, C, true);
+    if (next < end) fetch_rows<STREAM>(nxt, xs, next, step, end, begin, C, true);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (row + u * step < end) {
@@ -613,7 +622,7 @@ __global__ void __launch_bounds__(kBlock) gn_normalize(const T* __restrict__ x, 
 
 // ---- backward: per-channel partial sums (vector path) --------------------------------------
 // part (floats): [N][nsplit][2][C]  with q = 0: sum dy'*xhat, q = 1: sum dy'
-template <typename T, typename TG>
+template <typename T, typename TG, bool STREAM>
 __global__ void __launch_bounds__(kBlock) gn_bwd_partial(const T* __restrict__ x, const TG* __restrict__ dy,
                                                          const float* __restrict__ mean, const float* __restrict__ rstd,
                                                          const void* __restrict__ gamma, const void* __restrict__ beta,
@@ -640,8 +649,8 @@ __global__ void __launch_bounds__(kBlock) gn_bwd_partial(const T* __restrict__ x
   int64_t row = begin + r;
   Piece<T, V> cx[U];
   Piece<TG, V> cg_[U];
-  fetch_rows<T, V, U>(cx, xs, row, step, end, begin, C, active);
-  fetch_rows<TG, V, U>(cg_, gs, row, step, end, begin, C, active);
+  fetch_rows<STREAM>(cx, xs, row, step, end, begin, C, active);
+  fetch_rows<STREAM>(cg_, gs, row, step, end, begin, C, active);
   float mu[V], rs[V], ga[V], be[V];
   load_params<V>(gamma, param_dtype, active ? cv * V : 0, 1.f, ga);
   load_params<V>(beta, param_dtype, active ? cv * V : 0, 0.f, be);
@@ -660,8 +669,8 @@ __global__ void __launch_bounds__(kBlock) gn_bwd_partial(const T* __restrict__ x
       Piece<T, V> nx[U];
       Piece<TG, V> ng[U];
       if (next < end) {
-        fetch_rows<T, V, U>(nx, xs, next, step, end, begin, C, true);
-        fetch_rows<TG, V, U>(ng, gs, next, step, end, begin, C, true);
+        fetch_rows<STREAM>(nx, xs, next, step, end, begin, C, true);
+        fetch_rows<STREAM>(ng, gs, next, step, end, begin, C, true);
       }
       if (row + step < end) {  // a whole batch
         float f0[V], g0[V], f1[V], g1[V];
@@ -730,16 +739,7 @@ __global__ void __launch_bounds__(kBlock) gn_bwd_partial(const T* __restrict__ x
   }
 }
 
-// Fixed-order sum over a 256-thread workgroup (wavefront trees, then the four wave totals in order).
-__device__ __forceinline__ float block_sum256(float v, float* red4) {
-  v = wave_sum(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red4[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return (red4[0] + red4[1]) + (red4[2] + red4[3]);
-}
-
-// Two sums at once (the same trees, one pair of barriers).
+// Two sums over a 256-thread workgroup in a fixed order (wavefront trees, then the four wavefronts' totals in order).
 __device__ __forceinline__ void block_sum256_pair(float& a, float& b, float* red8) {
   a = wave_sum(a);
   b = wave_sum(b);
@@ -753,14 +753,32 @@ __device__ __forceinline__ void block_sum256_pair(float& a, float& b, float* red
   b = (red8[4] + red8[5]) + (red8[6] + red8[7]);
 }
 
-// Workgroups [0, N*G): coef[n][g] = (A, B) with A = mean(dy'*gamma), B = mean(dy'*gamma*xhat)
-// over the group. Workgroups [N*G, N*G + C): dgamma[c], dbeta[c] summed over samples and splits.
-__global__ void __launch_bounds__(kBlock) gn_bwd_finalize(const float* __restrict__ part, const void* __restrict__ gamma,
-                                                          int param_dtype, float* __restrict__ coef, float* __restrict__ dgamma,
-                                                          float* __restrict__ dbeta, int N, int C, int G, int nsplit, float m) {
-  __shared__ float red4[4];
+// Two sums at once over a workgroup of kFinalize threads, in a fixed order; thread 0 gets them.
+constexpr int kFinalize = 1024;
+__device__ __forceinline__ void finalize_sum_pair(float& a, float& b, float (*red)[2]) {
+  a = wave_sum(a);
+  b = wave_sum(b);
+  if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6][0] = a; red[threadIdx.x >> 6][1] = b; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    a = b = 0.f;
+#pragma unroll
+    for (int w = 0; w < kFinalize / 64; ++w) { a += red[w][0]; b += red[w][1]; }
+  }
+}
+
+// Workgroups [0, N*G): coef[n][g] = (A, B) with A = mean(dy'*gamma), B = mean(dy'*gamma*xhat) over the group. The others:
+// dgamma[c], dbeta[c] of kFinalizeChannels channels each, summed over samples and splits.
+// A few megabytes out of the caches by a few dozen workgroups: what bounds it is the chain of trips a thread makes. With 256
+// threads, and a workgroup per channel that used 4 bytes of every line it met, 2048 splits of 64 channels took 16 us, now 8.9.
+constexpr int kFinalizeChannels = 16;
+__global__ void __launch_bounds__(kFinalize) gn_bwd_finalize(const float* __restrict__ part, const void* __restrict__ gamma,
+                                                             int param_dtype, float* __restrict__ coef, float* __restrict__ dgamma,
+                                                             float* __restrict__ dbeta, int N, int C, int G, int nsplit, float m) {
+  __shared__ float red[kFinalize / 64][2 * kFinalizeChannels];
   const int b = blockIdx.x;
   const int cg = C / G;
+  constexpr int U = 8;  // loads of either quantity in flight per thread
   if (b < N * G) {
     const int n = b / G, g = b - n * G;
     // One flat index over (split, channel of the group): neighbouring threads read neighbouring channels and every
@@ -768,12 +786,11 @@ __global__ void __launch_bounds__(kBlock) gn_bwd_finalize(const float* __restric
     float s1 = 0.f, s2 = 0.f;
     const float* base = part + (int64_t)n * nsplit * 2 * C + g * cg;
     const int total = nsplit * cg;
-    constexpr int U = 8;  // loads in flight per thread
-    for (int i0 = threadIdx.x; i0 < total; i0 += U * kBlock) {
+    for (int i0 = threadIdx.x; i0 < total; i0 += U * kFinalize) {
       float a1[U], a2[U], w[U];
 #pragma unroll
       for (int k = 0; k < U; ++k) {
-        const int i = i0 + k * kBlock;
+        const int i = i0 + k * kFinalize;
         const int ic = i < total ? i : total - 1;
         const int sp = ic / cg, cc = ic - sp * cg;
         const float* p = base + (int64_t)sp * 2 * C + cc;
@@ -783,30 +800,52 @@ __global__ void __launch_bounds__(kBlock) gn_bwd_finalize(const float* __restric
       }
 #pragma unroll
       for (int k = 0; k < U; ++k) {
-        s1 = fmaf(w[k], a1[k], s1);
-        s2 = fmaf(w[k], a2[k], s2);
+        s1 = fmaf(w[k], i0 + k * kFinalize < total ? a1[k] : 0.f, s1);
+        s2 = fmaf(w[k], i0 + k * kFinalize < total ? a2[k] : 0.f, s2);
       }
     }
-    s1 = block_sum256(s1, red4);
-    s2 = block_sum256(s2, red4);
+    finalize_sum_pair(s1, s2, reinterpret_cast<float(*)[2]>(red));
     if (threadIdx.x == 0) {
       coef[(n * G + g) * 2] = s2 / m;
       coef[(n * G + g) * 2 + 1] = s1 / m;
     }
   } else {
-    const int c = b - N * G;
+    constexpr int ROWS = kFinalize / kFinalizeChannels;
+    const int own = threadIdx.x % kFinalizeChannels, c = (b - N * G) * kFinalizeChannels + own;
     float s1 = 0.f, s2 = 0.f;
-    const int total = N * nsplit;
-    for (int i = threadIdx.x; i < total; i += kBlock) {
-      const float* p = part + (int64_t)i * 2 * C;
-      s1 += p[c];
-      s2 += p[C + c];
+    const int total = c < C ? N * nsplit : 0;
+    for (int i0 = threadIdx.x / kFinalizeChannels; i0 < total; i0 += U * ROWS) {
+      float a1[U], a2[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const int i = i0 + k * ROWS;
+        const float* p = part + (int64_t)(i < total ? i : total - 1) * 2 * C + c;
+        a1[k] = p[0];
+        a2[k] = p[C];
+      }
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        s1 += i0 + k * ROWS < total ? a1[k] : 0.f;
+        s2 += i0 + k * ROWS < total ? a2[k] : 0.f;
+      }
     }
-    s1 = block_sum256(s1, red4);
-    s2 = block_sum256(s2, red4);
-    if (threadIdx.x == 0) {
-      if (dgamma != nullptr) dgamma[c] = s1;
-      if (dbeta != nullptr) dbeta[c] = s2;
+    // the rows of a wavefront meet in a butterfly, the wavefronts in order through LDS
+#pragma unroll
+    for (int off = kFinalizeChannels; off < 64; off <<= 1) {
+      s1 += __shfl_xor(s1, off, 64);
+      s2 += __shfl_xor(s2, off, 64);
+    }
+    if ((threadIdx.x & 63) < kFinalizeChannels) {
+      red[threadIdx.x >> 6][own] = s1;
+      red[threadIdx.x >> 6][kFinalizeChannels + own] = s2;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 * kFinalizeChannels && c < C) {
+      float t = 0.f;
+#pragma unroll
+      for (int w = 0; w < kFinalize / 64; ++w) t += red[w][threadIdx.x];
+      float* dst = threadIdx.x < kFinalizeChannels ? dgamma : dbeta;
+      if (dst != nullptr) dst[c] = t;
     }
   }
 }
@@ -816,7 +855,7 @@ __global__ void __launch_bounds__(kBlock) gn_bwd_finalize(const float* __restric
 // A = mean(dy'*gamma), B = mean(dy'*gamma*xhat) from them itself, and workgroups of sample 0 finish by summing the
 // per-channel partials of one channel each into dgamma / dbeta (samples and splits in index order): no finalize
 // launch. Otherwise gn_bwd_finalize has filled `coef` and the parameter gradients.
-template <typename T, typename TG>
+template <typename T, typename TG, bool STREAM>
 __global__ void __launch_bounds__(kBlock) gn_dx(const T* __restrict__ x, const TG* __restrict__ dy, T* __restrict__ dx,
                                                 const float* __restrict__ mean, const float* __restrict__ rstd,
                                                 const void* __restrict__ gamma, const void* __restrict__ beta, int param_dtype,
@@ -843,8 +882,8 @@ __global__ void __launch_bounds__(kBlock) gn_dx(const T* __restrict__ x, const T
   int64_t row = begin + r;
   Piece<T, V> cx[U];
   Piece<TG, V> cg_[U];
-  fetch_rows<T, V, U>(cx, xs, row, step, end, begin, C, r < rpp);
-  fetch_rows<TG, V, U>(cg_, gs, row, step, end, begin, C, r < rpp);
+  fetch_rows<STREAM>(cx, xs, row, step, end, begin, C, r < rpp);
+  fetch_rows<STREAM>(cg_, gs, row, step, end, begin, C, r < rpp);
   const bool fused = fold_in_consumer(G, nsplit);
   // The workgroup's share of the parameter gradients (the tail of this kernel) reads the per-channel partials of the
   // launch before: its first loads go out now, so that the tail does not start with a trip to memory of its own.
@@ -891,8 +930,8 @@ __global__ void __launch_bounds__(kBlock) gn_dx(const T* __restrict__ x, const T
     Piece<T, V> nx[U];
     Piece<TG, V> ng[U];
     if (next < end) {
-      fetch_rows<T, V, U>(nx, xs, next, step, end, begin, C, true);
-      fetch_rows<TG, V, U>(ng, gs, next, step, end, begin, C, true);
+      fetch_rows<STREAM>(nx, xs, next, step, end, begin, C, true);
+      fetch_rows<STREAM>(ng, gs, next, step, end, begin, C, true);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -1384,7 +1423,7 @@ int fwd_typed(const sfh_groupnorm_desc& p, const GnPlan& pl, int param_dtype, co
     float* my_part = ws + align_up((size_t)p.n * G, 4);
     const size_t lds = (size_t)(2 * pl.slots * kBlock + 2 * G) * sizeof(float);
 #define SFH_GN_STATS(SL)                                                                                                      \
-  hipLaunchKernelGGL((gn_stats_partial<T, SL>), grid, dim3(kBlock), lds, st, (const T*)x, my_shift, my_part, S, C, G, pl.tpr, \
+  hipLaunchKernelGGL((pl.stream ? gn_stats_partial<T, SL, true> : gn_stats_partial<T, SL, false>), grid, dim3(kBlock), lds, st, (const T*)x, my_shift, my_part, S, C, G, pl.tpr, \
                      pl.rpp, pl.nsplit, pl.rows_per_split)
     switch (pl.slots) {
       case 1: SFH_GN_STATS(1); break;
@@ -1406,7 +1445,7 @@ int fwd_typed(const sfh_groupnorm_desc& p, const GnPlan& pl, int param_dtype, co
     hipLaunchKernelGGL(gn_stats_finalize, dim3(G, p.n), dim3(kBlock), 0, st, shift, part, mean, rstd, G, npart, m, p.eps);
     if (int rc = check_launch("gn_stats_finalize")) return rc;
   }
-  hipLaunchKernelGGL((gn_normalize<T, TO>), grid, dim3(kBlock), (size_t)(4 * G + 4 * kBlock) * sizeof(float), st, (const T*)x, (TO*)y, shift, part,
+  hipLaunchKernelGGL((pl.stream ? gn_normalize<T, TO, true> : gn_normalize<T, TO, false>), grid, dim3(kBlock), (size_t)(4 * G + 4 * kBlock) * sizeof(float), st, (const T*)x, (TO*)y, shift, part,
                      mean, rstd, gamma, beta, param_dtype, S, C, G, pl.tpr, pl.rpp, pl.nsplit, pl.rows_per_split, m, p.eps, p.relu, y_halo,
                      npart, welford);
   return check_launch("gn_normalize");
@@ -1448,17 +1487,17 @@ int bwd_typed(const sfh_groupnorm_desc& p, const GnPlan& pl, int param_dtype, co
   }
   constexpr int V = VecOf<T>::N;
   const dim3 grid(pl.nsplit, p.n);
-  hipLaunchKernelGGL((gn_bwd_partial<T, TG>), grid, dim3(kBlock), ((size_t)2 * V * kBlock + C) * sizeof(float), st, (const T*)x,
+  hipLaunchKernelGGL((pl.stream ? gn_bwd_partial<T, TG, true> : gn_bwd_partial<T, TG, false>), grid, dim3(kBlock), ((size_t)2 * V * kBlock + C) * sizeof(float), st, (const T*)x,
                      (const TG*)dy, mean, rstd, gamma, beta, param_dtype, part, gpart, S, C, G, pl.tpr, pl.rpp, pl.nsplit,
                      pl.rows_per_split, p.relu);
   if (int rc = check_launch("gn_bwd_partial")) return rc;
   const float m = (float)S * (float)(C / G);
   if (!fold_in_consumer_host(G, pl.nsplit)) {
-    hipLaunchKernelGGL(gn_bwd_finalize, dim3(p.n * G + C), dim3(kBlock), 0, st, part, gamma, param_dtype, coef, dgamma, dbeta, p.n,
+    hipLaunchKernelGGL(gn_bwd_finalize, dim3(p.n * G + (unsigned)cdiv(C, kFinalizeChannels)), dim3(kFinalize), 0, st, part, gamma, param_dtype, coef, dgamma, dbeta, p.n,
                        C, G, pl.nsplit, m);
     if (int rc = check_launch("gn_bwd_finalize")) return rc;
   }
-  hipLaunchKernelGGL((gn_dx<T, TG>), grid, dim3(kBlock), (size_t)(2 * G + 4 * kBlock) * sizeof(float), st, (const T*)x,
+  hipLaunchKernelGGL((pl.stream ? gn_dx<T, TG, true> : gn_dx<T, TG, false>), grid, dim3(kBlock), (size_t)(2 * G + 4 * kBlock) * sizeof(float), st, (const T*)x,
                      (const TG*)dy, (T*)dx, mean, rstd, gamma, beta, param_dtype, coef, part, gpart, dgamma, dbeta, p.n, S, C, G,
                      pl.tpr, pl.rpp, pl.nsplit, pl.rows_per_split, m, p.relu);
   return check_launch("gn_dx");

@@ -4,6 +4,17 @@
 
 namespace sfh {
 
+// 16 bytes that this pass alone has a use for: a load or store past the caches' retention (the `nt` hint).
+typedef uint32_t stream_vec __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint4 stream_load16(const void* p) {
+  const stream_vec v = __builtin_nontemporal_load(reinterpret_cast<const stream_vec*>(p));
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ void stream_store16(void* p, const uint4 v) {
+  const stream_vec w = {v.x, v.y, v.z, v.w};
+  __builtin_nontemporal_store(w, reinterpret_cast<stream_vec*>(p));
+}
+
 template <typename T, int V> struct Ld;
 template <int V> struct Ld<bf16_t, V> {
   static __device__ __forceinline__ void run(const bf16_t* p, float (&f)[V]) {
@@ -75,7 +86,8 @@ template <> struct VecOf<float> { static constexpr int N = 4; };
 template <typename T, int V> struct Piece;
 template <> struct Piece<bf16_t, 8> {
   uint4 q;
-  __device__ __forceinline__ void load(const bf16_t* p) { q = *reinterpret_cast<const uint4*>(p); }
+  template <bool STREAM = false>
+  __device__ __forceinline__ void load(const bf16_t* p) { q = STREAM ? stream_load16(p) : *reinterpret_cast<const uint4*>(p); }
   __device__ __forceinline__ void unpack(float (&f)[8]) const {
     f[0] = bf16_lo(q.x); f[1] = bf16_hi(q.x); f[2] = bf16_lo(q.y); f[3] = bf16_hi(q.y);
     f[4] = bf16_lo(q.z); f[5] = bf16_hi(q.z); f[6] = bf16_lo(q.w); f[7] = bf16_hi(q.w);
@@ -83,7 +95,8 @@ template <> struct Piece<bf16_t, 8> {
 };
 template <> struct Piece<fp16_t, 8> {
   uint4 q;
-  __device__ __forceinline__ void load(const fp16_t* p) { q = *reinterpret_cast<const uint4*>(p); }
+  template <bool STREAM = false>
+  __device__ __forceinline__ void load(const fp16_t* p) { q = STREAM ? stream_load16(p) : *reinterpret_cast<const uint4*>(p); }
   __device__ __forceinline__ void unpack(float (&f)[8]) const {
     f[0] = fp16_lo(q.x); f[1] = fp16_hi(q.x); f[2] = fp16_lo(q.y); f[3] = fp16_hi(q.y);
     f[4] = fp16_lo(q.z); f[5] = fp16_hi(q.z); f[6] = fp16_lo(q.w); f[7] = fp16_hi(q.w);
@@ -91,9 +104,17 @@ template <> struct Piece<fp16_t, 8> {
 };
 template <int V> struct Piece<float, V> {
   float4 q[V / 4];
+  template <bool STREAM = false>
   __device__ __forceinline__ void load(const float* p) {
 #pragma unroll
-    for (int i = 0; i < V / 4; ++i) q[i] = *reinterpret_cast<const float4*>(p + 4 * i);
+    for (int i = 0; i < V / 4; ++i) {
+      if constexpr (STREAM) {
+        const uint4 v = stream_load16(p + 4 * i);
+        q[i] = make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
+      } else {
+        q[i] = *reinterpret_cast<const float4*>(p + 4 * i);
+      }
+    }
   }
   __device__ __forceinline__ void unpack(float (&f)[V]) const {
 #pragma unroll
@@ -103,13 +124,13 @@ template <int V> struct Piece<float, V> {
 
 // U rows of one thread (row0, row0 + step, ...): rows at or past `end`, and every row of an idle thread, are read from
 // `safe` (a row that exists) and not used.
-template <typename T, int V, int U>
+template <bool STREAM, typename T, int V, int U>
 __device__ __forceinline__ void fetch_rows(Piece<T, V> (&b)[U], const T* xs, int64_t row0, int64_t step, int64_t end, int64_t safe,
                                            int C, bool active) {
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t rr = row0 + u * step;
-    b[u].load(xs + ((active && rr < end) ? rr : safe) * C);
+    b[u].template load<STREAM>(xs + ((active && rr < end) ? rr : safe) * C);
   }
 }
 
