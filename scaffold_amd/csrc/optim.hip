@@ -56,6 +56,21 @@ __device__ __forceinline__ int find_tensor(const Table& t, int chunk) {
   return i;
 }
 
+// A float4 read or written once in a step; STREAM: past the caches' retention.
+template <bool STREAM>
+__device__ __forceinline__ float4 load4(const float4* p) {
+  if constexpr (!STREAM) return *p;
+  const uint4 v = stream_load16(p);
+  return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
+}
+template <bool STREAM>
+__device__ __forceinline__ void store4(float4* p, const float4 v) {
+  if constexpr (!STREAM) *p = v;
+  else stream_store16(p, make_uint4(__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)));
+}
+
+// Bound by memory. Gradients of more than 256 MiB in all are not in the memory-side cache when Adam comes back to them.
+template <bool STREAM>
 __global__ void __launch_bounds__(kBlock) grad_sumsq_kernel(SumsqTable t, float* __restrict__ slots, float* step, int bump_step) {
   __shared__ float red4[4];
   const int chunk = blockIdx.x;
@@ -65,11 +80,17 @@ __global__ void __launch_bounds__(kBlock) grad_sumsq_kernel(SumsqTable t, float*
   const float* g = t.g[ti] + begin;
   float s = 0.f;
   if ((reinterpret_cast<uintptr_t>(g) & 15) == 0) {
-    const int64_t nvec = len / 4;
-    for (int64_t i = threadIdx.x; i < nvec; i += kBlock) {
-      const float4 q = reinterpret_cast<const float4*>(g)[i];
-      s += (q.x * q.x + q.y * q.y) + (q.z * q.z + q.w * q.w);
+    const int nvec = (int)(len / 4);
+    const float4* gv = reinterpret_cast<const float4*>(g);
+    constexpr int U = kOptimChunk / 4 / kBlock;  // a thread's pieces of a chunk, all on their way before the first is squared
+    float4 q[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = threadIdx.x + u * kBlock;
+      q[u] = i < nvec ? load4<STREAM>(gv + i) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
+#pragma unroll
+    for (int u = 0; u < U; ++u) s += (q[u].x * q[u].x + q[u].y * q[u].y) + (q[u].z * q[u].z + q[u].w * q[u].w);
     for (int64_t i = nvec * 4 + threadIdx.x; i < len; i += kBlock) s += g[i] * g[i];
   } else {
     for (int64_t i = threadIdx.x; i < len; i += kBlock) s += g[i] * g[i];
@@ -88,7 +109,9 @@ struct AdamCoef {
 template <typename TS>
 __device__ __forceinline__ void write_shadow(TS* s, int64_t i, float p) { s[i] = elem<TS>::from_float(p); }
 
-template <int SHADOW>  // 0 none, 1 bf16, 2 fp16
+// A workgroup folds the slots once and takes the chunks b, b + gridDim.x, ...: one workgroup per chunk folded as many slots as
+// there are chunks, 11065 times 44 KB out of L2 in front of 128 KB of work.
+template <int SHADOW, bool STREAM>  // SHADOW: 0 none, 1 bf16, 2 fp16
 __global__ void __launch_bounds__(kBlock) clip_adam_kernel(AdamTable t, AdamCoef c, const float* __restrict__ slots, int nslots,
                                                            int slot_base, const float* __restrict__ step_ptr, float* grad_norm) {
   __shared__ float red4[4];
@@ -112,16 +135,6 @@ __global__ void __launch_bounds__(kBlock) clip_adam_kernel(AdamTable t, AdamCoef
   const float bc2_sqrt = sqrtf(1.f - powf(c.beta2, step));
   const float step_size = c.lr / bc1;
 
-  const int chunk = blockIdx.x;
-  const int ti = find_tensor(t, chunk);
-  const int64_t begin = (int64_t)(chunk - t.chunk_start[ti]) * kOptimChunk;
-  const int64_t len = min((int64_t)kOptimChunk, t.numel[ti] - begin);
-  float* p = t.p[ti] + begin;
-  const float* g = t.g[ti] + begin;
-  float* m = t.m[ti] + begin;
-  float* v = t.v[ti] + begin;
-  void* sh = t.shadow[ti];
-
   auto update = [&](float& pe, float ge, float& me, float& ve) {
     float grad = ge * scale;
     if (c.weight_decay != 0.f) grad = fmaf(c.weight_decay, pe, grad);
@@ -131,58 +144,76 @@ __global__ void __launch_bounds__(kBlock) clip_adam_kernel(AdamTable t, AdamCoef
     pe = pe - step_size * (me / denom);
   };
 
-  const bool aligned = ((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(m) |
-                         reinterpret_cast<uintptr_t>(v)) & 15) == 0 &&
-                       (SHADOW == 0 || sh == nullptr || ((reinterpret_cast<uintptr_t>(sh) + 2 * begin) & 7) == 0);
-  int64_t done = 0;
-  if (aligned) {
-    const int64_t nvec = len / 4;
-    // Four of a thread's pieces at a time, all sixteen loads in flight before the first update: a launch of a few dozen
-    // chunks (the tail of the parameter list) has nothing else on its CUs to cover a trip to memory, and one piece
-    // per trip made its chunk of 8192 elements a chain of eight (15.8 us for half a megabyte of parameters).
-    constexpr int U = 4;
-    for (int64_t i0 = threadIdx.x; i0 < nvec; i0 += U * kBlock) {
-      float4 pq[U], gq[U], mq[U], vq[U];
+  const int chunks = t.chunk_start[t.n];
+  for (int chunk = blockIdx.x; chunk < chunks; chunk += gridDim.x) {
+    const int ti = find_tensor(t, chunk);
+    const int64_t begin = (int64_t)(chunk - t.chunk_start[ti]) * kOptimChunk;
+    const int64_t len = min((int64_t)kOptimChunk, t.numel[ti] - begin);
+    float* p = t.p[ti] + begin;
+    const float* g = t.g[ti] + begin;
+    float* m = t.m[ti] + begin;
+    float* v = t.v[ti] + begin;
+    void* sh = t.shadow[ti];
+
+    const bool aligned = ((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(m) |
+                           reinterpret_cast<uintptr_t>(v)) & 15) == 0 &&
+                         (SHADOW == 0 || sh == nullptr || ((reinterpret_cast<uintptr_t>(sh) + 2 * begin) & 7) == 0);
+    int64_t done = 0;
+    if (aligned) {
+      const int64_t nvec = len / 4;
+      // Four of a thread's pieces at a time, all sixteen loads in flight before the first update: a launch of a few dozen
+      // chunks (the tail of the parameter list) has nothing else on its CUs to cover a trip to memory, and one piece
+      // per trip made its chunk of 8192 elements a chain of eight (15.8 us for half a megabyte of parameters).
+      constexpr int U = 4;
+      for (int64_t i0 = threadIdx.x; i0 < nvec; i0 += U * kBlock) {
+        float4 pq[U], gq[U], mq[U], vq[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t i = i0 + u * kBlock;
-        if (i < nvec) {
-          pq[u] = reinterpret_cast<float4*>(p)[i];
-          gq[u] = reinterpret_cast<const float4*>(g)[i];
-          mq[u] = reinterpret_cast<float4*>(m)[i];
-          vq[u] = reinterpret_cast<float4*>(v)[i];
+        for (int u = 0; u < U; ++u) {
+          const int64_t i = i0 + u * kBlock;
+          if (i < nvec) {
+            pq[u] = load4<STREAM>(reinterpret_cast<float4*>(p) + i);
+            gq[u] = load4<STREAM>(reinterpret_cast<const float4*>(g) + i);
+            mq[u] = load4<STREAM>(reinterpret_cast<float4*>(m) + i);
+            vq[u] = load4<STREAM>(reinterpret_cast<float4*>(v) + i);
+          }
         }
-      }
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t i = i0 + u * kBlock;
-        if (i < nvec) {
-          update(pq[u].x, gq[u].x, mq[u].x, vq[u].x);
-          update(pq[u].y, gq[u].y, mq[u].y, vq[u].y);
-          update(pq[u].z, gq[u].z, mq[u].z, vq[u].z);
-          update(pq[u].w, gq[u].w, mq[u].w, vq[u].w);
-          reinterpret_cast<float4*>(p)[i] = pq[u];
-          reinterpret_cast<float4*>(m)[i] = mq[u];
-          reinterpret_cast<float4*>(v)[i] = vq[u];
-          if (SHADOW != 0 && sh != nullptr) {
-            uint2 pk;
-            if (SHADOW == 1) { pk.x = pack_bf16x2(pq[u].x, pq[u].y); pk.y = pack_bf16x2(pq[u].z, pq[u].w); }
-            else { pk.x = pack_fp16x2(pq[u].x, pq[u].y); pk.y = pack_fp16x2(pq[u].z, pq[u].w); }
-            reinterpret_cast<uint2*>(static_cast<char*>(sh) + 2 * begin)[i] = pk;
+        for (int u = 0; u < U; ++u) {
+          const int64_t i = i0 + u * kBlock;
+          if (i < nvec) {
+            update(pq[u].x, gq[u].x, mq[u].x, vq[u].x);
+            update(pq[u].y, gq[u].y, mq[u].y, vq[u].y);
+            update(pq[u].z, gq[u].z, mq[u].z, vq[u].z);
+            update(pq[u].w, gq[u].w, mq[u].w, vq[u].w);
+            store4<STREAM>(reinterpret_cast<float4*>(p) + i, pq[u]);
+            store4<STREAM>(reinterpret_cast<float4*>(m) + i, mq[u]);
+            store4<STREAM>(reinterpret_cast<float4*>(v) + i, vq[u]);
+            if (SHADOW != 0 && sh != nullptr) {
+              uint2 pk;
+              if (SHADOW == 1) { pk.x = pack_bf16x2(pq[u].x, pq[u].y); pk.y = pack_bf16x2(pq[u].z, pq[u].w); }
+              else { pk.x = pack_fp16x2(pq[u].x, pq[u].y); pk.y = pack_fp16x2(pq[u].z, pq[u].w); }
+              reinterpret_cast<uint2*>(static_cast<char*>(sh) + 2 * begin)[i] = pk;
+            }
           }
         }
       }
+      done = nvec * 4;
     }
-    done = nvec * 4;
-  }
-  for (int64_t i = done + threadIdx.x; i < len; i += kBlock) {
-    float pe = p[i], me = m[i], ve = v[i];
-    update(pe, g[i], me, ve);
-    p[i] = pe; m[i] = me; v[i] = ve;
-    if (SHADOW == 1 && sh != nullptr) write_shadow(static_cast<bf16_t*>(sh) + begin, i, pe);
-    if (SHADOW == 2 && sh != nullptr) write_shadow(static_cast<fp16_t*>(sh) + begin, i, pe);
+    for (int64_t i = done + threadIdx.x; i < len; i += kBlock) {
+      float pe = p[i], me = m[i], ve = v[i];
+      update(pe, g[i], me, ve);
+      p[i] = pe; m[i] = me; v[i] = ve;
+      if (SHADOW == 1 && sh != nullptr) write_shadow(static_cast<bf16_t*>(sh) + begin, i, pe);
+      if (SHADOW == 2 && sh != nullptr) write_shadow(static_cast<fp16_t*>(sh) + begin, i, pe);
+    }
   }
 }
+
+constexpr int kAdamWorkgroups = 2048;  // 1024 and 1280 measure the same
+// Bytes of one pass (parameters, moments and gradients, or gradients alone) beyond which it goes past the caches' retention: 256 MiB is
+// the memory-side cache. us of the update of 90 M parameters 500 -> 440 (with the fold once a workgroup), of 22.6 M 111 -> 111 and the
+// packing behind it, which then finds the 16-bit copies in the caches, 28 -> 22.
+constexpr int64_t kStreamBytes = 256ll << 20;
 
 int64_t chunks_of(int64_t numel) { return cdiv(numel, kOptimChunk); }
 
@@ -195,8 +226,10 @@ int64_t optim_chunks(int ntensors, const int64_t* numel) {
 }
 
 int optim_grad_sumsq(int ntensors, const float* const* grads, const int64_t* numel, float* slots, float* step, hipStream_t st) {
-  int64_t slot_base = 0;
+  int64_t slot_base = 0, elements = 0;
   bool first = true;
+  for (int i = 0; i < ntensors; ++i) elements += numel[i];
+  const bool stream = 4 * elements > kStreamBytes;
   for (int base = 0; base < ntensors; base += kMaxTensors) {
     SumsqTable t{};
     t.n = ntensors - base < kMaxTensors ? ntensors - base : kMaxTensors;
@@ -209,7 +242,7 @@ int optim_grad_sumsq(int ntensors, const float* const* grads, const int64_t* num
     }
     t.chunk_start[t.n] = (int)chunks;
     if (chunks > 0x7fffffff) return fail(SFH_ERR_UNSUPPORTED, "adam: too many chunks in one launch");
-    hipLaunchKernelGGL(grad_sumsq_kernel, dim3((unsigned)chunks), dim3(kBlock), 0, st, t, slots + slot_base, step, first ? 1 : 0);
+    hipLaunchKernelGGL((stream ? grad_sumsq_kernel<true> : grad_sumsq_kernel<false>), dim3((unsigned)chunks), dim3(kBlock), 0, st, t, slots + slot_base, step, first ? 1 : 0);
     if (int rc = check_launch("grad_sumsq_kernel")) return rc;
     first = false;
     slot_base += chunks;
@@ -221,6 +254,9 @@ int optim_clip_adam(const sfh_adam_desc& d, int ntensors, float* const* params, 
                     float* const* exp_avg_sq, void* const* shadow, const int64_t* numel, const float* slots, int nslots,
                     const float* step, float* grad_norm, hipStream_t st) {
   const AdamCoef c{d.lr, d.beta1, d.beta2, d.eps, d.weight_decay, d.max_norm};
+  int64_t elements = 0;
+  for (int i = 0; i < ntensors; ++i) elements += numel[i];
+  const bool stream = 16 * elements > kStreamBytes;
   int64_t slot_base = 0;
   for (int base = 0; base < ntensors; base += kMaxTensors) {
     AdamTable t{};
@@ -238,13 +274,14 @@ int optim_clip_adam(const sfh_adam_desc& d, int ntensors, float* const* params, 
     }
     t.chunk_start[t.n] = (int)chunks;
     if (chunks > 0) {
-      const dim3 grid((unsigned)chunks), block(kBlock);
-      if (shadow == nullptr || d.shadow_dtype < 0)
-        hipLaunchKernelGGL(clip_adam_kernel<0>, grid, block, 0, st, t, c, slots, nslots, (int)slot_base, step, grad_norm);
-      else if (d.shadow_dtype == SFH_BF16)
-        hipLaunchKernelGGL(clip_adam_kernel<1>, grid, block, 0, st, t, c, slots, nslots, (int)slot_base, step, grad_norm);
-      else
-        hipLaunchKernelGGL(clip_adam_kernel<2>, grid, block, 0, st, t, c, slots, nslots, (int)slot_base, step, grad_norm);
+      const dim3 grid((unsigned)(chunks < kAdamWorkgroups ? chunks : kAdamWorkgroups)), block(kBlock);
+#define SFH_ADAM(SHADOW)                                                                                                          \
+  hipLaunchKernelGGL((stream ? clip_adam_kernel<SHADOW, true> : clip_adam_kernel<SHADOW, false>), grid, block, 0, st, t, c, slots, \
+                     nslots, (int)slot_base, step, grad_norm)
+      if (shadow == nullptr || d.shadow_dtype < 0) SFH_ADAM(0);
+      else if (d.shadow_dtype == SFH_BF16) SFH_ADAM(1);
+      else SFH_ADAM(2);
+#undef SFH_ADAM
       if (int rc = check_launch("clip_adam_kernel")) return rc;
     }
     slot_base += chunks;
