@@ -23,15 +23,57 @@ __device__ __forceinline__ float wave_sum_all(float v) {
   return v;  // lane 0 holds the sum
 }
 
+// The same total in lane 63, on the vector pipe alone: rows of 16 lanes by shifts of 1, 2, 4 and 8, then rows 0 and 2 into
+// rows 1 and 3 and row 1 into rows 2 and 3. The 3 C + 2 totals of a workgroup made 228 trips through the LDS pipe as shuffles.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, ROWS, 0xf, true));
+}
+__device__ __forceinline__ float wave_sum_last(float v) {
+  v = dpp_add<0x111, 0xf>(v);
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);
+  return dpp_add<0x143, 0xc>(v);
+}
+
+// Voxels a thread works on between two barriers: as many as keep a tile's logits within 32 KiB of LDS, so that four
+// workgroups fit a CU and a workgroup's trips to memory are one or two, not one per 256 voxels. bf16, before and now: partial
+// sums of 11 classes of 64x128x128 27.3 -> 15.8 us (54 MB; the totals' trips through the LDS pipe were 6 us of it), of
+// 6 classes of 128-cube 35.6 -> 15.8, of 11 classes of 32-cube 12.9 -> 5.3; backward 23.4 -> 17.3, 36.7 -> 19.0, 6.9 -> 4.6.
+template <typename T, int CMAX> constexpr int kVoxels = 32768 / (kBlock * CMAX * (int)sizeof(T)) >= 4   ? 4
+                                                        : 32768 / (kBlock * CMAX * (int)sizeof(T)) >= 2 ? 2
+                                                                                                        : 1;
+
+// The kernels are built for up to CMAX classes; a class below the smallest count that CMAX is taken for needs no question.
+template <int CMAX>
+__device__ __forceinline__ bool has_class(int c, int C) {
+  constexpr int kFewest = CMAX == 32 ? 17 : CMAX == 16 ? 13 : CMAX == 4 ? 2 : CMAX - 1;
+  return c < kFewest || c < C;
+}
+
 // A tile's logits are one contiguous byte range whatever the class count (11 classes: 22-byte rows): it moves between
 // global memory and LDS in 16-byte pieces when the range starts on a 16-byte boundary (`vec`), element by element else.
 template <typename T>
 __device__ __forceinline__ void tile_in(T* tile, const T* __restrict__ src, int nelem, bool vec) {
   const int tid = threadIdx.x;
   if (vec) {
-    constexpr int E = 16 / (int)sizeof(T);
+    constexpr int E = 16 / (int)sizeof(T), U = 8;  // pieces of a thread in flight
     const int npiece = nelem / E;
-    for (int i = tid; i < npiece; i += kBlock) reinterpret_cast<uint4*>(tile)[i] = reinterpret_cast<const uint4*>(src)[i];
+    for (int i0 = tid; i0 < npiece; i0 += U * kBlock) {
+      uint4 piece[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const int i = i0 + k * kBlock;
+        piece[k] = reinterpret_cast<const uint4*>(src)[i < npiece ? i : npiece - 1];
+      }
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const int i = i0 + k * kBlock;
+        if (i < npiece) reinterpret_cast<uint4*>(tile)[i] = piece[k];
+      }
+    }
     for (int i = npiece * E + tid; i < nelem; i += kBlock) tile[i] = src[i];
   } else {
     for (int i = tid; i < nelem; i += kBlock) tile[i] = src[i];
@@ -50,57 +92,83 @@ __device__ __forceinline__ void tile_out(T* __restrict__ dst, const T* tile, int
   }
 }
 
+// The labels of a thread's voxels of one tile, asked for before the tile's logits are waited for.  A label outside
+// [0, C) (an ignored voxel) becomes -1.
+template <int VOX>
+__device__ __forceinline__ void labels_in(int (&y)[VOX], const int64_t* __restrict__ lab, int nv, int C) {
+  int64_t raw[VOX];
+#pragma unroll
+  for (int u = 0; u < VOX; ++u) {
+    const int i = (int)threadIdx.x + u * kBlock;
+    raw[u] = lab[i < nv ? i : nv - 1];
+  }
+#pragma unroll
+  for (int u = 0; u < VOX; ++u) y[u] = raw[u] >= 0 && raw[u] < C ? (int)raw[u] : -1;
+}
+
 // Quantities per sample: inter[c], psum[c], tsum[c] (3 * C), then the two launch-wide ones: ce_sum, normaliser.
 template <typename T, int CMAX>
 __global__ void __launch_bounds__(kBlock) ce_dice_partial(const T* __restrict__ logits, const int64_t* __restrict__ labels,
                                                           const float* __restrict__ cw, float* __restrict__ part, int64_t S, int C,
                                                           int nsplit, int64_t per_split, int vec) {
   extern __shared__ __align__(16) char smem_raw[];
-  T* tile = reinterpret_cast<T*>(smem_raw);  // kBlock voxels x C logits
+  T* tile = reinterpret_cast<T*>(smem_raw);  // kVoxels * kBlock voxels x C logits
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = blockIdx.y, split = blockIdx.x;
   const T* src = logits + (int64_t)n * S * C;
   const int64_t* lab = labels + (int64_t)n * S;
-  float inter[CMAX], psum[CMAX], tsum[CMAX], ce = 0.f, norm = 0.f;
+  constexpr int VOX = kVoxels<T, CMAX>;
+  float inter[CMAX], psum[CMAX], ce = 0.f, norm = 0.f;
+  int tsum[CMAX];  // voxels of a class: whole numbers
 #pragma unroll
-  for (int c = 0; c < CMAX; ++c) inter[c] = psum[c] = tsum[c] = 0.f;
+  for (int c = 0; c < CMAX; ++c) {
+    inter[c] = psum[c] = 0.f;
+    tsum[c] = 0;
+  }
   const int64_t begin = (int64_t)split * per_split;
   int64_t end = begin + per_split;
   if (end > S) end = S;
-  for (int64_t v0 = begin; v0 < end; v0 += kBlock) {
-    const int nv = (int)((end - v0) < kBlock ? (end - v0) : kBlock);
+  for (int64_t v0 = begin; v0 < end; v0 += VOX * kBlock) {
+    const int nv = (int)((end - v0) < VOX * kBlock ? (end - v0) : VOX * kBlock);
+    int label[VOX];
+    labels_in<VOX>(label, lab + v0, nv, C);
     __syncthreads();
     tile_in<T>(tile, src + v0 * C, nv * C, vec != 0);
     __syncthreads();
-    if (tid < nv) {
+#pragma unroll 1
+    for (int u = 0; u < VOX; ++u) {
+      const int at = tid + u * kBlock;
+      if (at >= nv) break;
+      const T* row = tile + at * C;
       float x[CMAX];
       float m = -INFINITY;
 #pragma unroll
       for (int c = 0; c < CMAX; ++c) {
-        x[c] = c < C ? to_float(tile[tid * C + c]) : -INFINITY;
+        x[c] = has_class<CMAX>(c, C) ? to_float(row[c]) : -INFINITY;
         m = fmaxf(m, x[c]);
       }
       float s = 0.f;
 #pragma unroll
       for (int c = 0; c < CMAX; ++c) {
-        x[c] = c < C ? expf(x[c] - m) : 0.f;  // x now holds exp(logit - max)
+        x[c] = has_class<CMAX>(c, C) ? expf(x[c] - m) : 0.f;  // x now holds exp(logit - max)
         s += x[c];
       }
       const float inv = 1.f / s, logs = logf(s);
-      const int64_t y = lab[v0 + tid];
-      const bool valid = y >= 0 && y < C;
+      int y = label[0];
+#pragma unroll
+      for (int k = 1; k < VOX; ++k) y = u == k ? label[k] : y;
 #pragma unroll
       for (int c = 0; c < CMAX; ++c) {
         const float p = x[c] * inv;
-        const bool hit = valid && c == (int)y;
+        const bool hit = c == y;
         psum[c] += p;
         inter[c] += hit ? p : 0.f;
-        tsum[c] += hit ? 1.f : 0.f;
+        tsum[c] += hit ? 1 : 0;
       }
-      if (valid) {
+      if (y >= 0) {
         const float w = cw != nullptr ? cw[y] : 1.f;
         // -log p_y = log(sum) - (logit_y - max)
-        ce += w * (logs - (to_float(tile[tid * C + (int)y]) - m));
+        ce += w * (logs - (to_float(row[y]) - m));
         norm += w;
       }
     }
@@ -112,14 +180,14 @@ __global__ void __launch_bounds__(kBlock) ce_dice_partial(const T* __restrict__ 
   float* wave_tot = reinterpret_cast<float*>(smem_raw);  // [4][3 * CMAX + 2]
   constexpr int Q = 3 * CMAX + 2;
   auto park = [&](float v, int slot) {
-    v = wave_sum_all(v);
-    if (lane == 0) wave_tot[wave * Q + slot] = v;
+    v = wave_sum_last(v);
+    if (lane == 63) wave_tot[wave * Q + slot] = v;
   };
 #pragma unroll
   for (int c = 0; c < CMAX; ++c) {
     park(inter[c], c);
     park(psum[c], CMAX + c);
-    park(tsum[c], 2 * CMAX + c);
+    park((float)tsum[c], 2 * CMAX + c);
   }
   park(ce, 3 * CMAX);
   park(norm, 3 * CMAX + 1);
@@ -173,8 +241,8 @@ __global__ void __launch_bounds__(64) ce_dice_sum(const float* __restrict__ part
   }
 }
 
-__global__ void __launch_bounds__(64) ce_dice_scalar(const float* __restrict__ stats, float* __restrict__ loss, int N, int C, float eps) {
-  // one lane per (sample, foreground class) pass; the Dice terms meet in the fixed wavefront tree
+// The loss from the totals, by one wavefront: one lane per (sample, foreground class) pass; the Dice terms meet in the fixed tree.
+__device__ __forceinline__ void loss_from_totals(const float* stats, float* __restrict__ loss, int N, int C, float eps) {
   const float* inter = stats;
   const float* psum = stats + N * C;
   const float* tsum = stats + 2 * N * C;
@@ -196,6 +264,71 @@ __global__ void __launch_bounds__(64) ce_dice_scalar(const float* __restrict__ s
     const float ce = ce_sum / fmaxf(normaliser, 1.1920929e-07f);
     loss[0] = ce + (1.f - dice);
   }
+}
+
+__global__ void __launch_bounds__(64) ce_dice_scalar(const float* __restrict__ stats, float* __restrict__ loss, int N, int C, float eps) {
+  loss_from_totals(stats, loss, N, C, eps);
+}
+
+// Both of the above as one workgroup, for up to kTotalSamples samples and kTotalSlotsMax slots. A wavefront reads a slot's
+// quantities side by side and takes every sixteenth slot, sixteen of them in flight; sums of sixteen by a tree, the
+// wavefronts' by a tree. What bounds it is a launch and the trips of one CU: 128 slots of 35 quantities 5.3 us (the two launches
+// 9.3), 512 slots of 53 10.5 (level), 1024 of 35 17.8.
+constexpr int kTotal = 1024, kTotalWaves = kTotal / 64, kTotalSamples = 4, kTotalQ = 3 * 32 + 2, kTotalSlots = 16, kTotalSlotsMax = 256;
+__global__ void __launch_bounds__(kTotal) ce_dice_total(const float* __restrict__ part, float* __restrict__ stats, float* __restrict__ loss,
+                                                        int N, int C, int nsplit, int unweighted, float count, float eps) {
+  __shared__ float wave_tot[kTotalWaves][kTotalQ];
+  __shared__ float tot[kTotalSamples * 3 * 32 + 2];
+  const int Q = 3 * C + 2;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  float launch_wide = 0.f;  // the last two quantities run over all samples
+  for (int n = 0; n < N; ++n) {
+    const float* src = part + (int64_t)n * nsplit * Q;
+    for (int q = lane; q < Q; q += 64) {
+      float s = 0.f;
+      for (int sp = wave; sp < nsplit; sp += kTotalSlots * kTotalWaves) {
+        float v[kTotalSlots];
+#pragma unroll
+        for (int k = 0; k < kTotalSlots; ++k) {
+          const int at = sp + k * kTotalWaves;
+          v[k] = src[(int64_t)(at < nsplit ? at : sp) * Q + q];
+        }
+#pragma unroll
+        for (int k = 0; k < kTotalSlots; ++k) v[k] = sp + k * kTotalWaves < nsplit ? v[k] : 0.f;
+#pragma unroll
+        for (int h = kTotalSlots / 2; h > 0; h >>= 1)
+#pragma unroll
+          for (int k = 0; k < h; ++k) v[k] += v[k + h];
+        s += v[0];
+      }
+      wave_tot[wave][q] = s;
+    }
+    __syncthreads();
+    if (tid < Q) {
+      float v[kTotalWaves];
+#pragma unroll
+      for (int w = 0; w < kTotalWaves; ++w) v[w] = wave_tot[w][tid];
+#pragma unroll
+      for (int h = kTotalWaves / 2; h > 0; h >>= 1)
+#pragma unroll
+        for (int w = 0; w < h; ++w) v[w] += v[w + h];
+      if (tid < 3 * C) {
+        const int dst = (tid / C) * N * C + n * C + tid % C;
+        tot[dst] = v[0];
+        stats[dst] = v[0];
+      } else {
+        launch_wide += v[0];
+        if (n == N - 1) {
+          // the normaliser of the unweighted mean is the voxel count
+          const float t = tid == 3 * C + 1 && unweighted ? count : launch_wide;
+          tot[N * 3 * C + tid - 3 * C] = t;
+          stats[N * 3 * C + tid - 3 * C] = t;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (wave == 0) loss_from_totals(tot, loss, N, C, eps);
 }
 
 // dlogits[v][j] = gl * ( w_y / normaliser * (p_j - [j == y])  +  p_j * (g_j - sum_c g_c p_c) ),
@@ -231,33 +364,41 @@ __global__ void __launch_bounds__(kBlock) ce_dice_backward(const T* __restrict__
   const int64_t begin = (int64_t)split * per_split;
   int64_t end = begin + per_split;
   if (end > S) end = S;
-  for (int64_t v0 = begin; v0 < end; v0 += kBlock) {
-    const int nv = (int)((end - v0) < kBlock ? (end - v0) : kBlock);
+  constexpr int VOX = kVoxels<T, CMAX>;
+  for (int64_t v0 = begin; v0 < end; v0 += VOX * kBlock) {
+    const int nv = (int)((end - v0) < VOX * kBlock ? (end - v0) : VOX * kBlock);
+    int label[VOX];
+    labels_in<VOX>(label, lab + v0, nv, C);
     __syncthreads();
     tile_in<T>(tile, src + v0 * C, nv * C, vec != 0);
     __syncthreads();
-    if (tid < nv) {
+#pragma unroll 1
+    for (int u = 0; u < VOX; ++u) {
+      const int at = tid + u * kBlock;
+      if (at >= nv) break;
+      T* row = tile + at * C;
       float p[CMAX];
       float m = -INFINITY;
 #pragma unroll
       for (int c = 0; c < CMAX; ++c) {
-        p[c] = c < C ? to_float(tile[tid * C + c]) : -INFINITY;
+        p[c] = has_class<CMAX>(c, C) ? to_float(row[c]) : -INFINITY;
         m = fmaxf(m, p[c]);
       }
       float s = 0.f;
 #pragma unroll
       for (int c = 0; c < CMAX; ++c) {
-        p[c] = c < C ? expf(p[c] - m) : 0.f;
+        p[c] = has_class<CMAX>(c, C) ? expf(p[c] - m) : 0.f;
         s += p[c];
       }
       const float inv = 1.f / s;
-      const int64_t y = lab[v0 + tid];
-      const bool valid = y >= 0 && y < C;
+      int y = label[0];
+#pragma unroll
+      for (int k = 1; k < VOX; ++k) y = u == k ? label[k] : y;
       float g[CMAX], dot = 0.f, wy = 0.f;
 #pragma unroll
       for (int c = 0; c < CMAX; ++c) {
         p[c] *= inv;
-        const bool hit = valid && c == (int)y;
+        const bool hit = c == y;
         g[c] = (hit ? ca[c] : 0.f) - cb[c];
         dot = fmaf(g[c], p[c], dot);
         if (hit) wy = cw != nullptr ? cw[c] : 1.f;
@@ -265,10 +406,10 @@ __global__ void __launch_bounds__(kBlock) ce_dice_backward(const T* __restrict__
       const float cs = ce_scale * wy;
 #pragma unroll
       for (int c = 0; c < CMAX; ++c) {
-        if (c < C) {
-          const bool hit = valid && c == (int)y;
+        if (has_class<CMAX>(c, C)) {
+          const bool hit = c == y;
           const float d = fmaf(p[c], g[c] - dot, cs * (p[c] - (hit ? 1.f : 0.f)));
-          tile[tid * C + c] = elem<T>::from_float(d);
+          row[c] = elem<T>::from_float(d);
         }
       }
     }
@@ -303,11 +444,16 @@ template <typename T, int CMAX>
 int fwd_typed(const sfh_loss_desc& p, const void* logits, const int64_t* labels, const float* cw, float* loss, float* stats,
               float* ws, hipStream_t st) {
   const LossPlan pl = loss_plan(p);
-  size_t lds = (size_t)kBlock * p.classes * sizeof(T);
+  size_t lds = (size_t)kVoxels<T, CMAX> * kBlock * p.classes * sizeof(T);
   if (lds < 4 * (3 * CMAX + 2) * sizeof(float)) lds = 4 * (3 * CMAX + 2) * sizeof(float);  // the fold at the end reuses the tile
   hipLaunchKernelGGL((ce_dice_partial<T, CMAX>), dim3(pl.nsplit, p.n), dim3(kBlock), lds, st, (const T*)logits, labels, cw, ws,
                      p.spatial, p.classes, pl.nsplit, pl.per_split, tiles_on_16_bytes<T>(p, logits, nullptr));
   if (int rc = check_launch("ce_dice_partial")) return rc;
+  if (p.n <= kTotalSamples && (int64_t)p.n * pl.nsplit <= kTotalSlotsMax) {
+    hipLaunchKernelGGL(ce_dice_total, dim3(1), dim3(kTotal), 0, st, ws, stats, loss, p.n, p.classes, pl.nsplit, cw == nullptr ? 1 : 0,
+                       (float)p.n * (float)p.spatial, p.eps);
+    return check_launch("ce_dice_total");
+  }
   hipLaunchKernelGGL(ce_dice_sum, dim3(p.n * 3 * p.classes + 2), dim3(64), 0, st, ws, stats, p.n, p.classes, pl.nsplit,
                      cw == nullptr ? 1 : 0, (float)p.n * (float)p.spatial);
   if (int rc = check_launch("ce_dice_sum")) return rc;
@@ -319,7 +465,7 @@ template <typename T, int CMAX>
 int bwd_typed(const sfh_loss_desc& p, const void* logits, const int64_t* labels, const float* cw, const float* stats,
               const float* grad_loss, void* dlogits, hipStream_t st) {
   const LossPlan pl = loss_plan(p);
-  const size_t lds = (size_t)kBlock * p.classes * sizeof(T);
+  const size_t lds = (size_t)kVoxels<T, CMAX> * kBlock * p.classes * sizeof(T);
   hipLaunchKernelGGL((ce_dice_backward<T, CMAX>), dim3(pl.nsplit, p.n), dim3(kBlock), lds, st, (const T*)logits, labels, cw, stats,
                      grad_loss, (T*)dlogits, p.spatial, p.n, p.classes, p.eps, pl.per_split, tiles_on_16_bytes<T>(p, logits, dlogits));
   return check_launch("ce_dice_backward");
@@ -335,20 +481,22 @@ size_t loss_workspace_bytes(const sfh_loss_desc& p) {
   return (size_t)p.n * loss_plan(p).nsplit * (3 * p.classes + 2) * sizeof(float);
 }
 
-#define SFH_LOSS_DISPATCH(fn, ...)                                               \
-  if (p.classes <= 12) {                                                         \
-    if (dtype == SFH_BF16) return fn<bf16_t, 12>(__VA_ARGS__);                   \
-    if (dtype == SFH_FP16) return fn<fp16_t, 12>(__VA_ARGS__);                   \
-    return fn<float, 12>(__VA_ARGS__);                                           \
-  }                                                                              \
-  if (p.classes <= 16) {                                                         \
-    if (dtype == SFH_BF16) return fn<bf16_t, 16>(__VA_ARGS__);                   \
-    if (dtype == SFH_FP16) return fn<fp16_t, 16>(__VA_ARGS__);                   \
-    return fn<float, 16>(__VA_ARGS__);                                           \
-  }                                                                              \
-  if (dtype == SFH_BF16) return fn<bf16_t, 32>(__VA_ARGS__);                     \
-  if (dtype == SFH_FP16) return fn<fp16_t, 32>(__VA_ARGS__);                     \
-  return fn<float, 32>(__VA_ARGS__);
+// Class counts in steps of two up to 12: a voxel's arithmetic is per class slot, so 6 classes in 12 slots cost as much as 12.
+#define SFH_LOSS_CLASSES(cmax, fn, ...)                         \
+  if (p.classes <= cmax) {                                      \
+    if (dtype == SFH_BF16) return fn<bf16_t, cmax>(__VA_ARGS__); \
+    if (dtype == SFH_FP16) return fn<fp16_t, cmax>(__VA_ARGS__); \
+    return fn<float, cmax>(__VA_ARGS__);                        \
+  }
+#define SFH_LOSS_DISPATCH(fn, ...)        \
+  SFH_LOSS_CLASSES(4, fn, __VA_ARGS__)    \
+  SFH_LOSS_CLASSES(6, fn, __VA_ARGS__)    \
+  SFH_LOSS_CLASSES(8, fn, __VA_ARGS__)    \
+  SFH_LOSS_CLASSES(10, fn, __VA_ARGS__)   \
+  SFH_LOSS_CLASSES(12, fn, __VA_ARGS__)   \
+  SFH_LOSS_CLASSES(16, fn, __VA_ARGS__)   \
+  SFH_LOSS_CLASSES(32, fn, __VA_ARGS__)   \
+  return fail(SFH_ERR_UNSUPPORTED, "ce_dice: %d classes", p.classes);
 
 int loss_forward(const sfh_loss_desc& p, int dtype, const void* logits, const int64_t* labels, const float* cw, float* loss,
                  float* stats, void* ws, hipStream_t st) {

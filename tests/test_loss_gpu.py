@@ -102,3 +102,15 @@ def test_gate_and_determinism(device):
         loss = sa.ce_dice_loss(x, labels)
         (g1,) = torch.autograd.grad(loss, x, create_graph=True)
         g1.sum().backward()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(1, 4, 5, 7, 9), (1, 5, 5, 7, 9), (1, 8, 3, 8, 11), (2, 10, 3, 8, 11), (1, 12, 4, 4, 17), (1, 13, 4, 4, 17),
+                                   (1, 16, 4, 4, 17),       # either end of the kernels' class ranges
+                                   (5, 3, 2, 3, 4),         # more samples than one workgroup totals
+                                   (2, 6, 16, 32, 33),      # more slots than one workgroup totals
+                                   (1, 2, 65, 128, 130)])   # several tiles per workgroup, the last of each cut
+def test_loss_class_ranges_and_totals(device, dtype, shape):
+    """The class ranges, the two ways the totals are taken and the several tiles of a large volume. Tolerances as above: the loss is a
+    quotient of fp32 sums, the gradient is rounded once."""
+    test_loss_and_gradient_match_oracle(device, dtype, shape, False)
