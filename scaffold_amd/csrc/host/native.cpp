@@ -385,6 +385,8 @@ struct QueuedWeight {
 struct WeightBatch {
   std::vector<QueuedWeight> items;
   std::vector<Tensor> grads;
+  std::optional<c10::Stream> beside;  // the pass's stream, while the launches run on a side stream of it
+  c10::Event done{c10::DeviceType::CUDA};  // behind those launches
   size_t size() const { return items.size(); }
 };
 
@@ -491,6 +493,34 @@ void add_to_grads(WeightBatch& batch) {
     last->second.stream = here;
     last->second.done.record(here);
   }
+}
+
+// Sends the batch to `side`, behind what the current stream has been given so far (modules._send_early).
+void launch_beside(WeightBatch& batch, const c10::Stream& side) {
+  const c10::Stream main = stream_on(side.device());
+  const auto behind = [](const c10::Stream& waits, const c10::Stream& for_) {
+    c10::Event reached(c10::DeviceType::CUDA);
+    reached.record(for_);
+    reached.block(waits);
+  };
+  behind(side, main);
+  try {
+    c10::StreamGuard on_side(side);
+    at::AutoGradMode no_grad(false);
+    launch_batch(batch, true);
+  } catch (...) {
+    behind(main, side);
+    throw;
+  }
+  batch.beside = main;
+  batch.done.record(side);
+}
+
+// Makes the pass's stream, and the current one, wait for a batch sent to a side stream.
+void join_beside(WeightBatch& batch) {
+  const c10::Stream here = stream_on(batch.beside.value().device());
+  batch.done.block(*batch.beside);
+  if (here != *batch.beside) batch.done.block(here);
 }
 
 PassQueue take_pass(int id) {
@@ -1265,7 +1295,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("set_callbacks", &set_callbacks);
   m.def("set_early_callbacks", &set_early_callbacks);
   py::class_<WeightBatch, std::shared_ptr<WeightBatch>>(m, "WeightBatch").def("__len__", &WeightBatch::size);
-  m.def("launch_batch", [](WeightBatch& batch, bool share_device) { launch_batch(batch, share_device); });
+  m.def("launch_beside", [](WeightBatch& batch, int64_t stream_id, int64_t device_index) {
+    launch_beside(batch, c10::Stream::unpack3(stream_id, (c10::DeviceIndex)device_index, c10::DeviceType::CUDA));
+  });
+  m.def("join_beside", &join_beside);
   m.def("batch_device", [](const WeightBatch& batch) { return batch.items.at(0).gy.device(); });
   m.def("finish_current_pass", &finish_current_pass, py::call_guard<py::gil_scoped_release>());
   m.def("waiting_weight_gradients", &waiting_weight_gradients);

@@ -148,7 +148,7 @@ def _deferrable(param, in_shape, wshape, stride, padding, dilation, dtype) -> in
 
 _EARLY_LOCK = threading.Lock()
 _EARLY_STREAMS: dict = {}  # (device, a pass's stream) -> the side stream beside it
-_EARLY_DONE: dict = {}  # batch sent and not joined yet -> (the pass's stream, event behind the batch's launches)
+_EARLY_DONE: dict = {}  # batch sent and not joined yet -> the pass's stream
 
 
 def _early_stream(main):
@@ -173,22 +173,13 @@ def _send_early(batch) -> None:
     # the caching allocator hands none of it out while the batch runs.
     main = torch.cuda.current_stream(_lib.native().batch_device(batch))
     side = _early_stream(main)
-    side.wait_stream(main)
-    try:
-        with torch.no_grad(), torch.cuda.stream(side):
-            _lib.native().launch_batch(batch, True)
-    except BaseException:
-        main.wait_stream(side)
-        raise
-    _EARLY_DONE[batch] = main, side.record_event()
+    _lib.native().launch_beside(batch, side.stream_id, side.device_index)
+    _EARLY_DONE[batch] = main
 
 
 def _join_early(batch) -> None:
-    main, done = _EARLY_DONE.pop(batch)
-    main.wait_event(done)
-    current = torch.cuda.current_stream(main.device)
-    if current != main:
-        current.wait_event(done)
+    del _EARLY_DONE[batch]
+    _lib.native().join_beside(batch)
 
 
 def flush_weight_gradients() -> None:
