@@ -6,10 +6,10 @@
 // 1e-5 bar of the fp32 configuration holds; dense fp32 MFMA peak is 157.3 TFLOP/s.
 //
 // GEMM view (gather_gemm.py:112-341): M = output voxels, N = produced channels, K = taps x reduction channels.
-//   * A workgroup owns a TD x TH x 32 brick of output voxels and one block of 32 produced channels; the input brick
+//   * A workgroup owns a TD x TH x TW brick of output voxels and one block of 32 produced channels; the input brick
 //     with its halo is staged in LDS per chunk of 16 reduction channels as four 16-byte channel planes (plane p =
-//     channels 4p .. 4p+3 of every brick voxel; planes 64 bytes apart modulo 256, so a wavefront's ds_read_b128 of 32
-//     consecutive voxels is conflict free and every tap is an immediate offset).
+//     channels 4p .. 4p+3 of every brick voxel; planes 64 bytes apart modulo 256, so a wavefront's ds_read_b128 of rows
+//     of 8 or more voxels is conflict free and every tap is an immediate offset).
 //   * One MFMA contracts 2 reduction channels: k-slot kg (= lane / 32) at step kk of a chunk is channel 8 kg + kk, so a
 //     lane's operands of the 8 steps of a tap are 8 consecutive channels: two 16-byte LDS reads of activations and two
 //     16-byte global loads of the weight, which is repacked once per call into that order
@@ -33,22 +33,34 @@ constexpr int plane_bytes(int voxels) {  // smallest size >= voxels*16 that is 6
   return ((voxels * 16 - 64 + 255) / 256) * 256 + 64;
 }
 
-template <int TD_, int TH_>
+// KS: wavefronts that share a sub-tile's reduction, each a chunk of channels of its own; they meet in LDS in that order. WM: groups of
+// such wavefronts, each with its sub-tiles.
+template <int TD_, int TH_, int TW_, int WM_ = 4, int KS_ = 1>
 struct FTile {
-  static constexpr int TD = TD_, TH = TH_, TW = 32;
+  static constexpr int TD = TD_, TH = TH_, TW = TW_, WM = WM_, KS = KS_;
   static constexpr int BD = TD + 2, BH = TH + 2, BW = TW + 2;
   static constexpr int BV = BD * BH * BW;
   static constexpr int PLANE = plane_bytes(BV);
-  static constexpr int LDS = 4 * PLANE;
-  static constexpr int MS = TD * TH * TW / 128;  // 32-voxel sub-tiles per wavefront
+  static constexpr int CHUNK = 4 * PLANE;
+  static constexpr int MEET = (KS - 1) * WM * 16 * 64 * 4;
+  static constexpr int LDS = KS * CHUNK > MEET ? KS * CHUNK : MEET;
+  static constexpr int THREADS = 64 * WM * KS;
+  static constexpr int MS = TD * TH * TW / (32 * WM);  // 32-voxel sub-tiles per wavefront
   // One sub-tile to a wavefront is what a volume gets that does not fill the chip: nothing else on the SIMD hides a trip to
   // memory or LDS, and there are registers for requesting the next chunk's brick and the next tap's activations ahead.
-  // 32 -> 32 channels on 32^3: 27.4 -> 20.5 us a launch (its MFMAs alone 11.5).
+  // 32 -> 32 channels on 32^3: 27.4 -> 20.5 us a launch (its MFMAs alone 11.5; now 19).
   static constexpr bool AHEAD = MS == 1;
-  static_assert(TD * TH * TW % 128 == 0, "tile must split into 4 wavefronts of 32-voxel sub-tiles");
-  static_assert(2 * LDS <= 160 * 1024, "two workgroups in the 160 KB LDS of a CU");
+  static_assert(TD * TH * TW % (32 * WM) == 0, "tile must split into WM wavefronts of 32-voxel sub-tiles");
+  static_assert(KS == 1 || MS == 1, "the parts of a reduction meet in one sub-tile a wavefront");
+  static_assert((THREADS > 256 ? 1 : 2) * LDS <= 160 * 1024, "eight wavefronts in the 160 KB LDS of a CU");
   static_assert(PLANE + (2 * BH * BW + 2 * BW + 2) * 16 < 65536, "ds_read immediate range");
 };
+
+// The bricks. Rows of 8 or 16 voxels: 32-voxel rows spend three quarters of the matrix pipe on nothing where a volume is 8 wide.
+using WholeTile = FTile<8, 8, 8>;                                                       // 512 voxels, four sub-tiles a wavefront
+template <int TW> using FlatTile = FTile<TW == 8 ? 4 : 2, 4, TW>;                       // 128 voxels
+template <int TW> using HalvedTile = FTile<2, TW == 8 ? 4 : 2, TW, 2, 2>;               // 64 voxels, the reduction in two parts
+using QuarteredTile = FTile<2, 2, 8, 1, 4>;                                             // 32 voxels, in four
 
 template <typename C>
 __device__ __forceinline__ constexpr int tap_off(int tap) {
@@ -57,12 +69,13 @@ __device__ __forceinline__ constexpr int tap_off(int tap) {
 }
 
 template <typename C>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(C::THREADS, 2)
 conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __restrict__ wp, const float* __restrict__ bias,
                 float* __restrict__ y, int tiles_d, int tiles_h, int tiles_w, int nblocks, uint32_t total) {
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = (tid >> 6) % C::WM;
+  const int part = C::KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((tid >> 6) / C::WM);
   const int j = lane & 31, kg = lane >> 5;
 
   uint32_t t = xcd_remap(blockIdx.x, total);
@@ -80,7 +93,7 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
   for (int ms = 0; ms < C::MS; ++ms) {
     const int v = (wave * C::MS + ms) * 32 + j;
     const int tw = v % C::TW, th = (v / C::TW) % C::TH, td = v / (C::TW * C::TH);
-    lbase[ms] = 2 * kg * C::PLANE + ((td * C::BH + th) * C::BW + tw) * 16;
+    lbase[ms] = part * C::CHUNK + 2 * kg * C::PLANE + ((td * C::BH + th) * C::BW + tw) * 16;
   }
   f32x16_t acc[C::MS];
 #pragma unroll
@@ -89,8 +102,8 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
     for (int r = 0; r < 16; ++r) acc[ms][r] = 0.f;
 
   const int ncc = a.cred / kChunk;
-  constexpr int PIECES = C::BV * 4;
-  constexpr int ITERS = (PIECES + 255) / 256;
+  constexpr int PIECES = C::KS * C::BV * 4;  // voxel by voxel the pieces of KS chunks, which lie side by side
+  constexpr int ITERS = (PIECES + C::THREADS - 1) / C::THREADS;
   constexpr int BATCH = C::AHEAD ? ITERS : 8;  // staging loads in flight before the first LDS write
   const float* xn = x + (int64_t)n * a.id * a.ih * a.iw * a.cred;
   auto request = [&](int cc, int it0, float4 (&v)[BATCH]) {
@@ -98,11 +111,11 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
     for (int u = 0; u < BATCH; ++u) {
       if (it0 + u < ITERS) {
         // unconditional load from a clamped address, masked afterwards (a load under a branch waits for the one before)
-        const int p = (it0 + u) * 256 + tid;
-        const int vox = p >> 2, piece = p & 3;
+        const int p = (it0 + u) * C::THREADS + tid;
+        const int vox = p / (4 * C::KS), piece = p % (4 * C::KS);
         const int bw = vox % C::BW, bh = (vox / C::BW) % C::BH, bd = vox / (C::BW * C::BH);
         const int id = id0 + bd, ih = ih0 + bh, iw = iw0 + bw;
-        const bool in = p < PIECES && (unsigned)id < (unsigned)a.id && (unsigned)ih < (unsigned)a.ih && (unsigned)iw < (unsigned)a.iw;
+        const bool in = p < PIECES && (C::KS == 1 || cc * kChunk + piece * 4 < a.cred) && (unsigned)id < (unsigned)a.id && (unsigned)ih < (unsigned)a.ih && (unsigned)iw < (unsigned)a.iw;
         const int64_t at = in ? (((int64_t)id * a.ih + ih) * a.iw + iw) * a.cred + cc * kChunk + piece * 4 : 0;
         const float4 got = *reinterpret_cast<const float4*>(xn + at);
         v[u] = in ? got : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -113,14 +126,15 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
 #pragma unroll
     for (int u = 0; u < BATCH; ++u) {
       if (it0 + u < ITERS) {
-        const int p = (it0 + u) * 256 + tid;
-        if (p < PIECES) *reinterpret_cast<float4*>(lds + (p & 3) * C::PLANE + (p >> 2) * 16) = v[u];
+        const int p = (it0 + u) * C::THREADS + tid;
+        if (p < PIECES) *reinterpret_cast<float4*>(lds + p % (4 * C::KS) / 4 * C::CHUNK + (p & 3) * C::PLANE + p / (4 * C::KS) * 16) = v[u];
       }
     }
   };
   // weight fragments of tap t: packed + (((nb * ncc + cc) * 27 + t) * 2 + q) * 256 floats + lane * 4; the taps of a chunk
   // are followed by the next chunk's, so the requests ahead run on over the end of a chunk
-  const float* wcc = wp + ((int64_t)(nb * ncc) * kTaps * 2) * 256 + lane * 4;
+  const int last = part < ncc ? part + (ncc - 1 - part) / C::KS * C::KS : -1;  // the wavefront's last chunk
+  const float* wcc = wp + ((int64_t)(nb * ncc + (part < ncc ? part : 0)) * kTaps * 2) * 256 + lane * 4;
   constexpr int WDEPTH = 3;  // taps requested ahead
   static_assert(kTaps % WDEPTH == 0, "a chunk ends where the ring of requests began");
   float4 wq[WDEPTH][2];
@@ -130,8 +144,9 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
     for (int q = 0; q < 2; ++q) wq[d][q] = *reinterpret_cast<const float4*>(wcc + (d * 2 + q) * 256);
   float4 v[BATCH];
   if (C::AHEAD) request(0, 0, v);
-  for (int cc = 0; cc < ncc; ++cc, wcc += kTaps * 2 * 256) {
-    const bool more = cc + 1 < ncc;
+  for (int cc = 0; cc < ncc; cc += C::KS) {
+    const bool more = cc + C::KS < ncc;  // of the workgroup; `ahead`: of this wavefront
+    const bool ahead = cc + part < last;
     __syncthreads();  // every wave is done reading the previous chunk
     if constexpr (C::AHEAD) {
       stage(0, v);
@@ -143,7 +158,8 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
       }
     }
     __syncthreads();
-    if (C::AHEAD && more) request(cc + 1, 0, v);
+    if (C::AHEAD && more) request(cc + C::KS, 0, v);
+    if (cc + part > last) continue;
 
     constexpr int ADEPTH = C::AHEAD ? 2 : 1;  // taps whose activations are held
     float4 af[ADEPTH][C::MS][2];
@@ -158,9 +174,10 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
 #pragma unroll
     for (int tap = 0; tap < kTaps; ++tap) {
       float4 wf[2] = {wq[tap % WDEPTH][0], wq[tap % WDEPTH][1]};
-      if (tap + WDEPTH < kTaps || more) {
+      if (tap + WDEPTH < kTaps || ahead) {
+        const int at = tap + WDEPTH < kTaps ? tap + WDEPTH : tap + WDEPTH + (C::KS - 1) * kTaps;
 #pragma unroll
-        for (int q = 0; q < 2; ++q) wq[tap % WDEPTH][q] = *reinterpret_cast<const float4*>(wcc + ((tap + WDEPTH) * 2 + q) * 256);
+        for (int q = 0; q < 2; ++q) wq[tap % WDEPTH][q] = *reinterpret_cast<const float4*>(wcc + (at * 2 + q) * 256);
       }
       if constexpr (C::AHEAD) {
         if (tap + 1 < kTaps) activations(tap + 1);
@@ -184,8 +201,28 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
       }
       if constexpr (C::AHEAD) __builtin_amdgcn_sched_barrier(0);
     }
+    wcc += C::KS * kTaps * 2 * 256;
   }
 
+  if constexpr (C::KS > 1) {
+    float4* meet = reinterpret_cast<float4*>(lds);
+    __syncthreads();  // the last chunks have been read
+    if (part > 0) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        meet[(((part - 1) * C::WM + wave) * 4 + g) * 64 + lane] =
+            make_float4(acc[0][4 * g], acc[0][4 * g + 1], acc[0][4 * g + 2], acc[0][4 * g + 3]);
+    }
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int p = 1; p < C::KS; ++p)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 o = meet[(((p - 1) * C::WM + wave) * 4 + g) * 64 + lane];
+        acc[0][4 * g] += o.x; acc[0][4 * g + 1] += o.y; acc[0][4 * g + 2] += o.z; acc[0][4 * g + 3] += o.w;
+      }
+  }
   // Accumulator register r of a lane is output channel 8 * (r / 4) + 4 * kg + r % 4 of the sub-tile's voxel j.
 #pragma unroll
   for (int ms = 0; ms < C::MS; ++ms) {
@@ -240,9 +277,35 @@ int launch(const MfmaConvArgs& a, const void* x, const void* packed, const void*
   const int64_t total = (int64_t)a.n * tiles_d * tiles_h * tiles_w * nblocks;
   if (total == 0) return SFH_OK;
   if (total > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv fp32: %lld workgroups exceed the grid limit", (long long)total);
-  hipLaunchKernelGGL((conv_f32_kernel<C>), dim3((unsigned)total), dim3(256), 0, st, a, (const float*)x, (const float*)packed,
+  hipLaunchKernelGGL((conv_f32_kernel<C>), dim3((unsigned)total), dim3(C::THREADS), 0, st, a, (const float*)x, (const float*)packed,
                      (const float*)bias, (float*)y, tiles_d, tiles_h, tiles_w, nblocks, (uint32_t)total);
   return check_launch("conv_f32_kernel");
+}
+
+// What a brick costs, us: the matrix pipe's time on the CU with the most workgroups (a wavefront's 216 MFMAs of a chunk take 5.76 us;
+// workgroups that share a CU share its pipes), stretched by what a wavefront waits for, and the launches around it. The slopes and
+// constants are fitted to sweeps of every brick over 16 problems of 32 to 512 channels on 4x8x8 to 64^3, within 15 % on each; the
+// choice is the fastest brick or within 4 % of it. One brick of 32-voxel rows (512 voxels, or 128 below a workgroup per CU) -> this, us
+// with the packing: 256 -> 256 channels at 8^3 124 -> 43, 512 -> 512 at 4x8x8 244 -> 82, 512 -> 256 at 8x16x16 240 -> 133, 128 -> 128 at 16^3 65 -> 38,
+// 64 -> 32 at 16x32x32 35 -> 22 (parts of the reduction on CUs that had no workgroup), two samples of 64 -> 32 at 20x33x41 93 -> 66,
+// 128 -> 64 at 30x17x40 180 -> 95, 256 -> 128 at 20x32x9 355 -> 159 (rows that were padding), 32 -> 32 at 8^3 20 -> 14, at 32^3 22.5 -> 21, 64 -> 64
+// at 64^3 466 -> 454 (no register spilled). A reduction in eight parts was nowhere faster than in four. Relative error against 64 bits, e-7:
+// 256 -> 256 at 8^3 13.6 -> 6.8, 128 -> 128 at 8x10x12 9.8 -> 4.9, 32 -> 32 at 16x16x24 5.1 -> 3.6. A pure function of the shape.
+template <typename C>
+double tile_us(const MfmaConvArgs& a, double slope, double fixed) {
+  const int64_t wgs = (int64_t)a.n * cdiv(a.od, C::TD) * cdiv(a.oh, C::TH) * cdiv(a.ow, C::TW) * (a.cout / 32);
+  const double waves = C::WM * C::KS / 4.0;
+  return slope * 5.76 * (double)cdiv(wgs, kComputeUnits) * waves * C::MS * (double)cdiv(a.cred / kChunk, C::KS) + fixed;
+}
+double tile_us(const MfmaConvArgs& a, int c) {
+  switch (c) {
+    case 0: return tile_us<WholeTile>(a, 1.16, 20.);
+    case 1: return tile_us<FlatTile<8>>(a, 1.245, 10.);
+    case 2: return tile_us<FlatTile<16>>(a, 1.255, 10.);
+    case 3: return tile_us<HalvedTile<8>>(a, 1.25, 10.);
+    case 4: return tile_us<HalvedTile<16>>(a, 1.27, 10.);
+    default: return tile_us<QuarteredTile>(a, 1.3, 9.5);
+  }
 }
 
 // ---- weight gradient ---------------------------------------------------------------------------------------------
@@ -423,10 +486,17 @@ int f32_pack_weight(const MfmaConvArgs& a, const void* w, int64_t s_out, int64_t
 }
 
 int f32_conv(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st) {
-  // Launch geometry, a pure function of the shape: 4 x 4 x 32 bricks when they fill the chip, else 2 x 2 x 32.
-  const int64_t big = (int64_t)a.n * cdiv(a.od, 4) * cdiv(a.oh, 4) * cdiv(a.ow, 32) * (a.cout / 32);
-  if (big >= kComputeUnits) return launch<FTile<4, 4>>(a, x, packed, bias, y, st);
-  return launch<FTile<2, 2>>(a, x, packed, bias, y, st);
+  int best = 0;
+  for (int c = 1; c < 6; ++c)
+    if (tile_us(a, c) < tile_us(a, best)) best = c;
+  switch (best) {
+    case 0: return launch<WholeTile>(a, x, packed, bias, y, st);
+    case 1: return launch<FlatTile<8>>(a, x, packed, bias, y, st);
+    case 2: return launch<FlatTile<16>>(a, x, packed, bias, y, st);
+    case 3: return launch<HalvedTile<8>>(a, x, packed, bias, y, st);
+    case 4: return launch<HalvedTile<16>>(a, x, packed, bias, y, st);
+    default: return launch<QuarteredTile>(a, x, packed, bias, y, st);
+  }
 }
 
 }  // namespace sfh
