@@ -93,7 +93,7 @@ typedef struct sfh_groupnorm_desc {
  * 104: sfh_conv3d_wgrad_batch, sfh_conv3d_wgrad_batch_supported, sfh_conv3d_wgrad_batch_workspace_bytes added;
  * SFH_KERNEL_SPLIT (6) is a value sfh_conv3d_launch_geometry may report. Nothing removed or changed.
  * 105: SFH_FLAG_SHARE_DEVICE; sfh_conv3d_wgrad_batch_workspace_bytes takes the call's flags (changed: one more argument).
- * 106: sfh_conv3d_pack_master_weights added. */
+ * 106: sfh_conv3d_pack_master_weights added. 107: sfh_convT3d_fwd_padded, sfh_convT3d_wgrad_bias_padded added. */
 int sfh_version(void);
 const char* sfh_last_error(void);
 /* Fills name (<= name_len bytes), compute-unit count, LDS bytes per workgroup. */
@@ -351,6 +351,16 @@ int sfh_convT3d_fwd_slab(const sfh_convT3d_desc* p, int dtype, const void* x, co
 size_t sfh_convT3d_wgrad_bias_workspace_bytes(const sfh_convT3d_desc* p, int dtype);
 int sfh_convT3d_wgrad_bias(const sfh_convT3d_desc* p, int dtype, const void* x, const void* gy, void* gw, void* gb,
                            void* workspace, size_t workspace_bytes, uint32_t flags, void* stream);
+
+/* The two with the result padded at the end of its extents, as the U-Net pads an upsampled tensor to an odd level's extents
+ * (ScaFFold/unet/unet_parts.py:212-223): y, and gy, have extents[i] >= 2 * in_i voxels per axis. What is past 2 * in_i is zero in
+ * y, written by the same launch, and is left out of both gradients. 2x2x2 matrix-core problems only; SFH_ERR_UNSUPPORTED otherwise
+ * and where the voxels past the end have 2^31 pieces of 16 bytes or more. Workspaces as above. */
+int sfh_convT3d_fwd_padded(const sfh_convT3d_desc* p, const int32_t extents[3], int dtype, const void* x, const void* w,
+                           const int64_t w_stride[5], const void* bias, void* y, void* workspace, size_t workspace_bytes,
+                           uint32_t flags, void* stream);
+int sfh_convT3d_wgrad_bias_padded(const sfh_convT3d_desc* p, const int32_t extents[3], int dtype, const void* x, const void* gy,
+                                  void* gw, void* gb, void* workspace, size_t workspace_bytes, uint32_t flags, void* stream);
 
 /* ---- GroupNorm forward ---------------------------------------------------------------
  * Stands in for torch.ops.scaffold_gn.group_norm (ScaFFold/unet/triton_group_norm.py:1339)

@@ -153,6 +153,10 @@ _SIGNATURES = {
     "sfh_convT3d_wgrad_bias_workspace_bytes": (c_size_t, [POINTER(ConvTDesc), c_int]),
     "sfh_convT3d_wgrad_bias": (c_int, [POINTER(ConvTDesc), c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_uint32,
                                        c_void_p]),
+    "sfh_convT3d_fwd_padded": (c_int, [POINTER(ConvTDesc), POINTER(c_int32), c_int, c_void_p, c_void_p, POINTER(c_int64), c_void_p, c_void_p,
+                                       c_void_p, c_size_t, c_uint32, c_void_p]),
+    "sfh_convT3d_wgrad_bias_padded": (c_int, [POINTER(ConvTDesc), POINTER(c_int32), c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                              c_size_t, c_uint32, c_void_p]),
     "sfh_convT3d_fwd_slab": (c_int, [POINTER(ConvTDesc), c_int, c_void_p, c_void_p, POINTER(c_int64), c_void_p, c_void_p, c_int64,
                                      c_void_p, c_size_t, c_uint32, c_void_p]),
     "sfh_groupnorm_fwd_workspace_bytes": (c_size_t, [POINTER(GroupNormDesc), c_int]),

@@ -166,10 +166,12 @@ bool dense_patch_weight(const void* w, const int64_t ws[5], int cbig) {
          ws[4] == cbig;
 }
 
-PatchArgs convT_patch_args(const sfh_convT3d_desc& p) {
+// `extents`: of a result padded at the end of its extents (null: twice the input's).
+PatchArgs convT_patch_args(const sfh_convT3d_desc& p, const int32_t* extents = nullptr) {
   PatchArgs a{};
   a.n = p.n;
   a.cbig = p.cout; a.bd = 2 * p.in_d; a.bh = 2 * p.in_h; a.bw = 2 * p.in_w;
+  if (extents != nullptr) { a.bd = extents[0]; a.bh = extents[1]; a.bw = extents[2]; }
   a.csmall = p.cin; a.sd = p.in_d; a.sh = p.in_h; a.sw = p.in_w;
   return a;
 }
@@ -298,7 +300,7 @@ __global__ void __launch_bounds__(256) stream_copy_kernel(const uint4* __restric
 
 using namespace sfh;
 
-extern "C" int sfh_version(void) { return 106; }
+extern "C" int sfh_version(void) { return 107; }
 
 extern "C" const char* sfh_last_error(void) { return g_error; }
 
@@ -922,7 +924,7 @@ extern "C" size_t sfh_convT3d_fwd_workspace_bytes(const sfh_convT3d_desc* p, int
 
 static int convT3d_fwd_any(const sfh_convT3d_desc* p, int dtype, const void* x, const void* w, const int64_t w_stride[5],
                            const void* bias, void* y, void* workspace, size_t workspace_bytes, uint32_t flags, void* stream,
-                           int64_t halo_elems) {
+                           int64_t halo_elems, const int32_t* extents = nullptr) {
   if (int rc = check_convT(p, dtype)) return rc;
   if (x == nullptr || w == nullptr || y == nullptr || (w_stride == nullptr && !(flags & SFH_FLAG_WEIGHT_PACKED)))
     return fail(SFH_ERR_INVALID, "convT3d fwd: null tensor");
@@ -931,7 +933,7 @@ static int convT3d_fwd_any(const sfh_convT3d_desc* p, int dtype, const void* x, 
     // w is the packed form: the data-gradient packing of the kernel == stride convolution this one transposes
     if ((flags & SFH_FLAG_FORCE_GENERIC) || !convT_uses_patch(*p, dtype))
       return fail(SFH_ERR_INVALID, "convT3d fwd: this problem does not read a packed weight");
-    return patch_scatter(convT_patch_args(*p), dtype, x, w, false, bias, y, (hipStream_t)stream, halo_elems);
+    return patch_scatter(convT_patch_args(*p, extents), dtype, x, w, false, bias, y, (hipStream_t)stream, halo_elems);
   }
   if (!(flags & SFH_FLAG_FORCE_GENERIC) && convT_uses_patch(*p, dtype)) {
     // produced channel = Cout (w_stride[1]), reduced channel = Cin (w_stride[0])
@@ -940,14 +942,15 @@ static int convT3d_fwd_any(const sfh_convT3d_desc* p, int dtype, const void* x, 
     if (workspace == nullptr || workspace_bytes < need)
       return fail(SFH_ERR_WORKSPACE, "convT3d fwd: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
     hipStream_t st = (hipStream_t)stream;
-    const PatchArgs a = convT_patch_args(*p);
+    const PatchArgs a = convT_patch_args(*p, extents);
     if (patch_scatter_reads_dense(a) && dense_patch_weight(w, w_stride, a.cbig))
       return patch_scatter(a, dtype, x, w, true, bias, y, st, halo_elems);
     if (int rc = mfma_pack_weight(pk, dtype, w, w_stride[1], w_stride[0], w_stride[2], w_stride[3], w_stride[4], 0, workspace, st))
       return rc;
     return patch_scatter(a, dtype, x, workspace, false, bias, y, st, halo_elems);
   }
-  if (halo_elems > 0) return fail(SFH_ERR_UNSUPPORTED, "convT3d fwd: only the 2x2x2 matrix-core kernel writes into a slab");
+  if (halo_elems > 0 || extents != nullptr)
+    return fail(SFH_ERR_UNSUPPORTED, "convT3d fwd: only the 2x2x2 matrix-core kernel writes into a slab or pads its result");
   return direct_convT(*p, dtype, w_stride, x, w, bias, y, (hipStream_t)stream);
 }
 
@@ -979,19 +982,47 @@ extern "C" size_t sfh_convT3d_wgrad_bias_workspace_bytes(const sfh_convT3d_desc*
   return patch_reduce_workspace_bytes(convT_patch_args(*p), true);
 }
 
-extern "C" int sfh_convT3d_wgrad_bias(const sfh_convT3d_desc* p, int dtype, const void* x, const void* gy, void* gw, void* gb,
-                                      void* workspace, size_t workspace_bytes, uint32_t flags, void* stream) {
+static int convT_wgrad_bias_any(const sfh_convT3d_desc* p, const int32_t* extents, int dtype, const void* x, const void* gy, void* gw,
+                                void* gb, void* workspace, size_t workspace_bytes, uint32_t flags, void* stream) {
   if (int rc = check_convT(p, dtype)) return rc;
   if (x == nullptr || gy == nullptr || gw == nullptr || gb == nullptr) return fail(SFH_ERR_INVALID, "convT3d wgrad: null tensor");
   if ((flags & SFH_FLAG_FORCE_GENERIC) || !convT_wgrad_bias_ok(*p, dtype))
     return fail(SFH_ERR_UNSUPPORTED, "convT3d wgrad with bias gradient: 2x2x2 matrix-core problems only");
-  const PatchArgs a = convT_patch_args(*p);
+  const PatchArgs a = convT_patch_args(*p, extents);
   const size_t need = patch_reduce_workspace_bytes(a, true);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(SFH_ERR_WORKSPACE, "convT3d wgrad: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
   const int g_dtype = (flags & SFH_FLAG_GRAD_FP32) ? SFH_FP32 : dtype;
   // small = the transposed convolution's input, big = its output gradient
   return patch_reduce(a, dtype, x, gy, gw, g_dtype, workspace, (hipStream_t)stream, gb);
+}
+
+extern "C" int sfh_convT3d_wgrad_bias(const sfh_convT3d_desc* p, int dtype, const void* x, const void* gy, void* gw, void* gb,
+                                      void* workspace, size_t workspace_bytes, uint32_t flags, void* stream) {
+  return convT_wgrad_bias_any(p, nullptr, dtype, x, gy, gw, gb, workspace, workspace_bytes, flags, stream);
+}
+
+static int check_padded(const sfh_convT3d_desc* p, const int32_t extents[3], int dtype) {
+  if (int rc = check_convT(p, dtype)) return rc;
+  if (p->n < 1) return fail(SFH_ERR_UNSUPPORTED, "convT3d: no padding around an empty result");
+  const int64_t in[3] = {p->in_d, p->in_h, p->in_w};
+  if (extents == nullptr) return fail(SFH_ERR_INVALID, "convT3d: null extents");
+  for (int i = 0; i < 3; ++i)
+    if (extents[i] < 2 * in[i]) return fail(SFH_ERR_INVALID, "convT3d: a padded extent of %d below 2 x %lld", extents[i], (long long)in[i]);
+  return SFH_OK;
+}
+
+extern "C" int sfh_convT3d_fwd_padded(const sfh_convT3d_desc* p, const int32_t extents[3], int dtype, const void* x, const void* w,
+                                      const int64_t w_stride[5], const void* bias, void* y, void* workspace, size_t workspace_bytes,
+                                      uint32_t flags, void* stream) {
+  if (int rc = check_padded(p, extents, dtype)) return rc;
+  return convT3d_fwd_any(p, dtype, x, w, w_stride, bias, y, workspace, workspace_bytes, flags, stream, 0, extents);
+}
+
+extern "C" int sfh_convT3d_wgrad_bias_padded(const sfh_convT3d_desc* p, const int32_t extents[3], int dtype, const void* x, const void* gy,
+                                             void* gw, void* gb, void* workspace, size_t workspace_bytes, uint32_t flags, void* stream) {
+  if (int rc = check_padded(p, extents, dtype)) return rc;
+  return convT_wgrad_bias_any(p, extents, dtype, x, gy, gw, gb, workspace, workspace_bytes, flags, stream);
 }
 
 // ---- loss head -------------------------------------------------------------------------

@@ -863,6 +863,13 @@ struct ConvTransposeNode : public LaunchNode {  // edges: x, weight, bias
     TORCH_INTERNAL_ASSERT(make_problem(gy.sizes(), w_sizes, k, zero, one, code_of(gy.scalar_type()), prob));
     const bool need_w = task_should_compute_output(1), need_b = has_bias && task_should_compute_output(2);
     if (task_should_compute_output(0)) out[0] = launch_conv(prob, gy, Tensor(), wt, Tensor(), packed, 0).y;
+    // a result padded at the end: what is past the input's patches belongs to nobody
+    int32_t extents[3];
+    bool padded = false;
+    for (int i = 0; i < 3; ++i) {
+      extents[i] = (int32_t)gy.size(2 + i);
+      padded = padded || gy.size(2 + i) != xs.size(2 + i) * k[i];
+    }
     if (need_w && need_b) {
       c10::OptionalDeviceGuard guard(gy.device());
       const sfh_convT3d_desc td{(int32_t)xs.size(0), (int32_t)xs.size(1), (int32_t)xs.size(2), (int32_t)xs.size(3), (int32_t)xs.size(4),
@@ -872,8 +879,8 @@ struct ConvTransposeNode : public LaunchNode {  // edges: x, weight, bias
         const auto dtype = master ? at::kFloat : gy.scalar_type();
         Tensor gw = volume(w_sizes, gy, dtype), gb = plain({w_sizes[1]}, gy, dtype);
         const Tensor ws = bytes(need, gy);
-        const int rc = sfh_convT3d_wgrad_bias(&td, prob.key.code, ptr(xs), ptr(gy), out_ptr(gw), out_ptr(gb), out_ptr(ws), need,
-                                              dtype != gy.scalar_type() ? SFH_FLAG_GRAD_FP32 : 0, stream_of(gy));
+        const int rc = sfh_convT3d_wgrad_bias_padded(&td, extents, prob.key.code, ptr(xs), ptr(gy), out_ptr(gw), out_ptr(gb), out_ptr(ws), need,
+                                                     dtype != gy.scalar_type() ? SFH_FLAG_GRAD_FP32 : 0, stream_of(gy));
         if (rc != SFH_ERR_UNSUPPORTED) {
           check(rc, "conv_transpose3d_backward_weight_bias");
           out[1] = gw;
@@ -883,15 +890,21 @@ struct ConvTransposeNode : public LaunchNode {  // edges: x, weight, bias
       }
     }
     if (need_w) out[1] = launch_wgrad(prob, gy, Tensor(), xs, master);
-    if (need_b) out[2] = launch_bias_grad(gy, bias_dtype);
+    if (need_b) {
+      Tensor under = gy;
+      for (int i = 0; i < 3 && padded; ++i) under = under.narrow(2 + i, 0, xs.size(2 + i) * k[i]);
+      out[2] = launch_bias_grad(dense(under), bias_dtype);
+    }
     return out;
   }
 };
 
 // FastConvTranspose3d: y (and the slab it lies in, or None), or None for a call that is not served as it stands.  `weight` /
-// `bias` receive gradients, `w` / `b` are what the kernels read; the packed forms are those of the stride-k convolution.
+// `bias` receive gradients, `w` / `b` are what the kernels read; the packed forms are those of the stride-k convolution.  `extents`:
+// y is padded with zeros at the end to these (and lies in no slab); the problems that do that themselves only.
 py::object conv_transpose(const Tensor& x_in, const Tensor& weight, const MaybeTensor& bias, const Tensor& w, const MaybeTensor& b, py::handle stride,
-                          const MaybeTensor& packed_fwd, const MaybeTensor& packed_dgrad, int64_t halo, bool master) {
+                          const MaybeTensor& packed_fwd, const MaybeTensor& packed_dgrad, int64_t halo, bool master,
+                          const std::optional<std::vector<int64_t>>& extents) {
   int32_t k[3];
   if (!three(stride, k) || x_in.dim() != 5 || w.dim() != 5 || !on_gpu(x_in) || !on_gpu(w) || x_in.device() != w.device()) return py::none();
   // an fp32 master that nobody reads: both packed forms were made from it in x's dtype
@@ -909,6 +922,22 @@ py::object conv_transpose(const Tensor& x_in, const Tensor& weight, const MaybeT
   if (!empty && !make_problem(big, w.sizes(), k, zero, one, code_of(x_in.scalar_type()), prob)) return py::none();
   if (!empty && packed_dgrad.has_value() && !packed_fits(*packed_dgrad, prob.sizes->packed[1], x_in)) return py::none();
   if (!empty && packed_fwd.has_value() && !packed_fits(*packed_fwd, prob.sizes->packed[0], x_in)) return py::none();
+  int32_t padded[3] = {0, 0, 0};
+  if (extents.has_value()) {
+    if (empty || extents->size() != 3 || k[0] != 2 || k[1] != 2 || k[2] != 2) return py::none();
+    std::vector<int64_t> sizes{big[0], big[1]};
+    for (int i = 0; i < 3; ++i) {
+      if ((*extents)[i] < big[2 + i] || (*extents)[i] > INT32_MAX) return py::none();
+      sizes.push_back(padded[i] = (int32_t)(*extents)[i]);
+    }
+    // both gradients of the padded problem are served, from the same packed forms
+    const sfh_convT3d_desc td{(int32_t)x_in.size(0), (int32_t)x_in.size(1), (int32_t)x_in.size(2), (int32_t)x_in.size(3), (int32_t)x_in.size(4),
+                              (int32_t)w.size(1), k[0], k[1], k[2]};
+    Problem around;
+    if (sfh_convT3d_wgrad_bias_workspace_bytes(&td, prob.key.code) == 0 || !make_problem(sizes, w.sizes(), k, zero, one, prob.key.code, around) ||
+        around.sizes->packed[0] != prob.sizes->packed[0])
+      return py::none();
+  }
   const Tensor weight_b = or_none(bias);
   const bool graph = wants_grad({&x_in, &weight, &weight_b});
   Tensor x = x_in, y, slab;
@@ -927,7 +956,11 @@ py::object conv_transpose(const Tensor& x_in, const Tensor& weight, const MaybeT
     const int64_t* strides = packed_dgrad.has_value() ? nullptr : w.strides().data();
     const uint32_t flags = packed_dgrad.has_value() ? SFH_FLAG_WEIGHT_PACKED : 0;
     int rc = SFH_ERR_UNSUPPORTED;
-    if (halo > 0 && x.size(0) == 1) {
+    if (extents.has_value()) {
+      y = volume({big[0], big[1], padded[0], padded[1], padded[2]}, x, x.scalar_type());
+      rc = sfh_convT3d_fwd_padded(&td, padded, code, ptr(x), wp, strides, ptr(or_none(b)), out_ptr(y), out_ptr(ws), ws_bytes, flags, stream_of(x));
+      if (rc == SFH_ERR_UNSUPPORTED) return py::none();
+    } else if (halo > 0 && x.size(0) == 1) {
       slab = volume({1, big[1], big[2] + 2 * halo, big[3], big[4]}, x, x.scalar_type());
       rc = sfh_convT3d_fwd_slab(&td, code, ptr(x), wp, strides, ptr(or_none(b)), out_ptr(slab), halo * big[3] * big[4] * big[1], out_ptr(ws), ws_bytes,
                                 flags, stream_of(x));

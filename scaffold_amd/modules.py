@@ -486,6 +486,26 @@ class FastConvTranspose3d(nn.ConvTranspose3d):
     def forward(self, x: torch.Tensor, output_size=None) -> torch.Tensor:
         if output_size is not None:
             raise NotImplementedError("FastConvTranspose3d: output_size is not supported")
+        return self._upsample(x, None)
+
+    def padded_to(self, x: torch.Tensor, extents):
+        """``F.pad(self(x), ...)`` with zeros at the end of the axes that are a voxel short of ``extents``, written by the same launch
+        (and left out of the gradients by theirs), or ``None`` where that is not what ``extents`` asks for or the module has to
+        run by itself (hooks or a ``forward`` of its own, a subclass, a transform, a problem off the matrix cores)."""
+        if type(self) is not FastConvTranspose3d or torch.compiler.is_compiling() or not _plain_call(self) \
+                or torch.nn.modules.module._has_any_global_hook() or _lib.under_transform() or not isinstance(x, torch.Tensor) or x.dim() != 5 \
+                or self.groups != 1 or tuple(self.stride) != (2, 2, 2) or tuple(self.padding) != (0, 0, 0) \
+                or tuple(self.output_padding) != (0, 0, 0) or tuple(self.dilation) != (1, 1, 1):
+            return None
+        if (autocast_dtype(x) or x.dtype) not in (torch.bfloat16, torch.float16) or self.in_channels % 64 or self.out_channels % 32 or x.shape[0] == 0:
+            return None  # (said before anything is packed for the call)
+        extents = [int(e) for e in extents]
+        short = [e - 2 * x.shape[2 + i] for i, e in enumerate(extents)]
+        if min(short) < 0 or max(short) != 1:
+            return None
+        return self._upsample(x, extents)
+
+    def _upsample(self, x, extents):
         dt = autocast_dtype(x)
         x = cast_operand(x, dt)
         weight, bias = self.weight, self.bias
@@ -513,8 +533,10 @@ class FastConvTranspose3d(nn.ConvTranspose3d):
             if _lib.under_transform():
                 return _lib.one_node(
                     lambda x_, w_, b_: self._served(_lib.native().conv_transpose(x_, w_, b_, w_ if takes_w is w else w, b_ if takes_b is b else b,
-                                                                                 stride, None, None, 0, master), x, w)[0], x, takes_w, takes_b)
-            done = _lib.native().conv_transpose(x, takes_w, takes_b, w, b, stride, pf, pd, self.out_halo, master)
+                                                                                 stride, None, None, 0, master, None), x, w)[0], x, takes_w, takes_b)
+            done = _lib.native().conv_transpose(x, takes_w, takes_b, w, b, stride, pf, pd, self.out_halo, master, extents)
+        if extents is not None:
+            return None if done is None else done[0]
         y, slab = self._served(done, x, w)
         if slab is not None:
             y._sfh_slab = (slab, self.out_halo)

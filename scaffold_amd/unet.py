@@ -133,7 +133,9 @@ class Up(nn.Module):
         self.conv = DoubleConv(in_channels, out_channels, group_norm_groups, stock=stock)
 
     def forward(self, x1, x2):
-        x1 = self.up(x1)
+        # an odd level: the upsampled tensor is written with its padding where the module does that by itself
+        padded = self.up.padded_to(x1, x2.shape[2:]) if isinstance(self.up, FastConvTranspose3d) else None
+        x1 = self.up(x1) if padded is None else padded
         dz, dy, dx = (x2.size(i) - x1.size(i) for i in (2, 3, 4))
         if dx or dy or dz:
             x1 = F.pad(x1, [dx // 2, dx - dx // 2, dy // 2, dy - dy // 2, dz // 2, dz - dz // 2])
