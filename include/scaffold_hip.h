@@ -278,7 +278,7 @@ int sfh_conv3d_wgrad_pair(const sfh_conv3d_desc* p, int dtype, const void* x_fir
  * work of all of them is laid on one line and cut evenly over the workgroups; a workgroup that covers parts of several
  * 32 x 32 channel blocks writes a slice for each. Small-volume problems (rows of 16 or 8 voxels, at most 32 tiles of
  * 256 voxels) share a second launch in which every 32 x 32 block is walked from its first tile to its last by one
- * workgroup and stored straight into the gradient: no slices, no sum pass. Each item is one sfh_conv3d_wgrad
+ * workgroup, or by a few where they are many under few blocks (then slices and a sum pass). Each item is one sfh_conv3d_wgrad
  * (x_second NULL) or sfh_conv3d_wgrad_pair call; all share `dtype` and the gradient dtype (SFH_FLAG_GRAD_FP32).
  * Results: every gradient is the sum of fp32 partials in a fixed order that is a pure function of the LIST of problems
  * (their shapes, in order) -- the same bits on every run, and within fp32 summation-order rounding of

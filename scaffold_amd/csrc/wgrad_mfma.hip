@@ -455,8 +455,8 @@ wgrad_mfma_kernel(WgradArgs a, const T* __restrict__ x, const T* __restrict__ gy
 // follows -- 23-44 us for 4-29 GFLOP. In a batch the UNITS -- (problem, block) with all its tiles -- of all problems lie
 // on one line of cost (tiles + kUnitCost each), workgroup w of W takes the units that start in
 // [w total / W, (w + 1) total / W), walks each from its first tile to its last and stores the finished block straight
-// into the gradient: no slices, no sum pass, and the order of additions of a block is that of its tiles, whatever else
-// is in the list. The two tile shapes (rows of 16 and of 8 voxels) share a launch.
+// into the gradient, the order of additions of a block being that of its tiles. The units of a problem with few output channels and many tiles
+// are cut into parts (unit_parts): then a slice per part and one sum pass for all. The two tile shapes (rows of 16 and of 8 voxels) share a launch.
 constexpr int kUnitCost = 2;          // what starting and storing a unit costs, in tiles (1 .. 5 measure alike)
 constexpr int kBatchMaxTiles = 32;    // longer units would not balance: such problems are launched alone
 
@@ -469,22 +469,25 @@ struct WTileBatchEntry {
   int c_first;
   int tw;                              // 16 or 8
   int tiles_d, tiles_h, tiles_w, ntiles;
+  int parts, tps;                      // of a unit's tiles, and the tiles of a part
   int nblk_ci, nblk;
   int pos_begin;
+  int quad_begin;                      // parts > 1: of the sum pass, in workgroups of 256
+  float* ws;                           // parts > 1: the slices, [parts][Cout][27][Cin]
 };
 
 struct WTileBatch {
-  int count, wgs, total;
+  int count, wgs, total, sum_wgs;
   bool planes;                         // units are (problem, block, kd)
   WTileBatchEntry e[kWgradBatchMax];
 };
 
-// One unit: all tiles of block (cob, cib) of a problem, the finished block stored at gw. The staging wavefronts and
-// the compute wavefronts meet at 1 + ntiles barriers, as in the kernel above.
+// One unit: tiles t0 .. t1 - 1 of block (cob, cib) of a problem, the block stored at gw or, as a slice, at ws. The staging
+// wavefronts and the compute wavefronts meet at 1 + t1 - t0 barriers, as in the kernel above.
 template <typename T, typename C, typename TOut>
 __device__ __forceinline__ void wtile_unit(const WgradArgs& a, const T* __restrict__ x, const T* __restrict__ x1, int c_first,
-                                           const T* __restrict__ gy, TOut* __restrict__ gw, int tiles_d, int tiles_h, int tiles_w,
-                                           int ntiles, int cib, int cob, int kd, char* buf0, char* buf1, int tid) {
+                                           const T* __restrict__ gy, TOut* __restrict__ gw, float* __restrict__ ws, int tiles_d, int tiles_h,
+                                           int tiles_w, int t0, int t1, int cib, int cob, int kd, char* buf0, char* buf1, int tid) {
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (wave >= 4) {
     WgradArgs as = a;
@@ -499,14 +502,14 @@ __device__ __forceinline__ void wtile_unit(const WgradArgs& a, const T* __restri
     }
     Slots<C> sl;
     init_slots<C>(as, tid - 256, sl);
-    auto origin = [&](int tile) { return decode_tile(tile < ntiles ? tile : ntiles - 1, tiles_d, tiles_h, tiles_w, C::TD, C::TH, C::TW); };
-    SlotLoop<T, C, 0>::fetch_all(as, xs, gy, origin(0), cis, cob, sl);
+    auto origin = [&](int tile) { return decode_tile(tile < t1 ? tile : t1 - 1, tiles_d, tiles_h, tiles_w, C::TD, C::TH, C::TW); };
+    SlotLoop<T, C, 0>::fetch_all(as, xs, gy, origin(t0), cis, cob, sl);
     SlotLoop<T, C, 0>::stage_all(buf0, sl);
-    SlotLoop<T, C, 0>::fetch_all(as, xs, gy, origin(1), cis, cob, sl);
+    SlotLoop<T, C, 0>::fetch_all(as, xs, gy, origin(t0 + 1), cis, cob, sl);
     __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
     __builtin_amdgcn_s_barrier();
-    for (int tile = 0; tile < ntiles; ++tile) {
-      char* idle = (tile & 1) ? buf0 : buf1;
+    for (int tile = t0; tile < t1; ++tile) {
+      char* idle = ((tile - t0) & 1) ? buf0 : buf1;
       SlotLoop<T, C, 0>::stage_and_refill(idle, as, xs, gy, origin(tile + 2), cis, cob, sl);
       __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
       __builtin_amdgcn_s_barrier();
@@ -515,13 +518,15 @@ __device__ __forceinline__ void wtile_unit(const WgradArgs& a, const T* __restri
     WaveTaps<T, C> taps;
     taps.clear();
     __builtin_amdgcn_s_barrier();  // the first tile is staged
-    for (int tile = 0; tile < ntiles; ++tile) {
-      const char* cur = (tile & 1) ? buf1 : buf0;
+    for (int tile = t0; tile < t1; ++tile) {
+      const char* cur = ((tile - t0) & 1) ? buf1 : buf0;
       asm volatile("" ::: "memory");  // LDS changes behind this wavefront's back: reload every tile
       taps.add(cur, lane, wave);
       __builtin_amdgcn_s_barrier();
     }
-    taps.store(gw + ((int64_t)cob * 32 * 27) * a.cin + cib * 32, a.cin, lane, wave, kd);
+    const int64_t at = ((int64_t)cob * 32 * 27) * a.cin + cib * 32;
+    if (ws != nullptr) taps.store(ws + at, a.cin, lane, wave, kd);
+    else taps.store(gw + at, a.cin, lane, wave, kd);
   }
 }
 
@@ -544,27 +549,57 @@ __global__ void __launch_bounds__(512) wgrad_mfma_batch_kernel(WTileBatch b) {
     int p = 0;
     for (int k = 1; k < b.count; ++k)
       if (pos >= b.e[k].pos_begin) p = k;
-    const int ntiles = b.e[p].ntiles, cost = ntiles + kUnitCost;
+    const int tps = b.e[p].tps, cost = tps + kUnitCost, parts = b.e[p].parts;
     const int unit = (pos - b.e[p].pos_begin + cost - 1) / cost;  // the first unit that starts at or behind pos
-    if (unit >= b.e[p].nblk * kUnits) {  // none left in this problem: on to the next one's first unit
+    if (unit >= b.e[p].nblk * kUnits * parts) {  // none left in this problem: on to the next one's first unit
       pos = p + 1 < b.count ? b.e[p + 1].pos_begin : hi;
       continue;
     }
     const int start = b.e[p].pos_begin + unit * cost;
     if (start >= hi) break;
     const WgradArgs a = b.e[p].a;
-    const int nblk_ci = b.e[p].nblk_ci;
-    const int kd = PLANES ? unit % 3 : 0, blk = unit / kUnits;
+    const int nblk_ci = b.e[p].nblk_ci, nblk = b.e[p].nblk;
+    const int kd = PLANES ? unit % 3 : 0, part = unit / kUnits / nblk, blk = unit / kUnits % nblk;
     const int cib = blk % nblk_ci, cob = blk / nblk_ci;
+    const int t0 = part * tps, t1 = t0 + tps < b.e[p].ntiles ? t0 + tps : b.e[p].ntiles;
+    float* ws = parts > 1 ? b.e[p].ws + (int64_t)part * a.cout * 27 * a.cin : nullptr;
     if (b.e[p].tw == 16)
-      wtile_unit<T, Tile16, TOut>(a, (const T*)b.e[p].x, (const T*)b.e[p].x1, b.e[p].c_first, (const T*)b.e[p].gy, (TOut*)b.e[p].gw,
-                                   b.e[p].tiles_d, b.e[p].tiles_h, b.e[p].tiles_w, ntiles, cib, cob, kd, buf0, buf1, tid);
+      wtile_unit<T, Tile16, TOut>(a, (const T*)b.e[p].x, (const T*)b.e[p].x1, b.e[p].c_first, (const T*)b.e[p].gy, (TOut*)b.e[p].gw, ws,
+                                   b.e[p].tiles_d, b.e[p].tiles_h, b.e[p].tiles_w, t0, t1, cib, cob, kd, buf0, buf1, tid);
     else
-      wtile_unit<T, Tile8, TOut>(a, (const T*)b.e[p].x, (const T*)b.e[p].x1, b.e[p].c_first, (const T*)b.e[p].gy, (TOut*)b.e[p].gw,
-                                  b.e[p].tiles_d, b.e[p].tiles_h, b.e[p].tiles_w, ntiles, cib, cob, kd, buf0, buf1, tid);
+      wtile_unit<T, Tile8, TOut>(a, (const T*)b.e[p].x, (const T*)b.e[p].x1, b.e[p].c_first, (const T*)b.e[p].gy, (TOut*)b.e[p].gw, ws,
+                                  b.e[p].tiles_d, b.e[p].tiles_h, b.e[p].tiles_w, t0, t1, cib, cob, kd, buf0, buf1, tid);
     pos = start + cost;
   }
 #endif
+}
+
+// The slices of the problems whose units are cut into parts, added up in their order, one rounding to the gradient's dtype.
+template <typename TOut>
+__global__ void __launch_bounds__(256) wgrad_mfma_batch_sum(WTileBatch b) {
+  int p = 0;
+  for (int k = 0; k < b.count; ++k)
+    if (b.e[k].parts > 1 && (int)blockIdx.x >= b.e[k].quad_begin) p = k;
+  const int64_t nelem = (int64_t)b.e[p].a.cout * 27 * b.e[p].a.cin;
+  const int64_t el = ((int64_t)((int)blockIdx.x - b.e[p].quad_begin) * 256 + threadIdx.x) * 4;
+  if (el >= nelem) return;
+  const float* src = b.e[p].ws + el;
+  const int parts = b.e[p].parts;
+  float4 s = *reinterpret_cast<const float4*>(src);
+  constexpr int U = 8;  // slices in flight
+  for (int k0 = 1; k0 < parts; k0 += U) {
+    float4 v[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) v[k] = *reinterpret_cast<const float4*>(src + (k0 + k < parts ? k0 + k : 0) * nelem);
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+      if (k0 + k < parts) { s.x += v[k].x; s.y += v[k].y; s.z += v[k].z; s.w += v[k].w; }
+  }
+  TOut* out = (TOut*)b.e[p].gw + el;
+  out[0] = elem<TOut>::from_float(s.x);
+  out[1] = elem<TOut>::from_float(s.y);
+  out[2] = elem<TOut>::from_float(s.z);
+  out[3] = elem<TOut>::from_float(s.w);
 }
 
 struct Plan {
@@ -671,7 +706,7 @@ int64_t busiest(const WTileBatch& b, int units) {
     int64_t load = 0;
     for (int pos = tile_batch_cut(w, total, wgs); pos < hi;) {
       while (p + 1 < b.count && pos >= b.e[p + 1].pos_begin * units) ++p;
-      const int begin = b.e[p].pos_begin * units, cost = b.e[p].ntiles + kUnitCost;
+      const int begin = b.e[p].pos_begin * units, cost = b.e[p].tps + kUnitCost;
       const int end = p + 1 < b.count ? b.e[p + 1].pos_begin * units : total;
       const int upto = end < hi ? end : hi;
       load += (int64_t)((upto - begin + cost - 1) / cost - (pos - begin + cost - 1) / cost) * cost;  // units that start in [pos, upto)
@@ -682,11 +717,37 @@ int64_t busiest(const WTileBatch& b, int units) {
   return most;
 }
 
+// Into how many parts the tiles of a block are cut. A volume of 28x13x13 has 28 tiles under a block and the level of 64 channels that
+// it is in a U-Net has 18 blocks: 54 units of 30 tiles' cost each kept 202 workgroups waiting. Where a gradient has up to 64 output
+// channels and more than eight tiles under a block, parts of about six tiles: slices (108 KB a block and part) and a sum pass (5 us) in
+// exchange. Levels of 128 channels and more have blocks enough: cut as well, the lists of 48^3 (width 64) and 125x34x37 (width 32) went
+// from 75 and 45 us to 89 and 53. A function of the problem alone: its bits do not depend on what else is in a list. Lists of the deep
+// levels of a step, us: 56x27x27 47.7 -> 30.4, 32^3 30.2 -> 22.1; 43x124x47, all of 128 channels and more, 54.
+int unit_parts(int ntiles, int cout) { return ntiles <= 8 || cout > 64 ? 1 : (int)cdiv(ntiles, 6); }
+
+// Lays the units out on the line of cost, `units` to a part of a block.
+bool lay_out(WTileBatch& b, int units) {
+  int64_t pos = 0;
+  int quads = 0;
+  for (int i = 0; i < b.count; ++i) {
+    WTileBatchEntry& e = b.e[i];
+    e.pos_begin = (int)pos;
+    pos += (int64_t)units * e.nblk * e.parts * (e.tps + kUnitCost);
+    if (pos > 0x7fffff) return false;  // 32-bit cuts
+    e.quad_begin = quads;
+    if (e.parts > 1) quads += (int)cdiv((int64_t)e.a.cout * 27 * e.a.cin, 1024);
+  }
+  b.total = (int)pos;
+  b.wgs = b.total < kTargetWorkgroups ? b.total : kTargetWorkgroups;
+  b.sum_wgs = quads;
+  b.planes = units == 3;
+  return true;
+}
+
 bool tile_batch_plan(const WgradBatchItem* items, int count, WTileBatch& b) {
   if (count < 1 || count > kWgradBatchMax) return false;
   b = WTileBatch{};
   b.count = count;
-  int64_t pos = 0;
   for (int i = 0; i < count; ++i) {
     const WgradArgs& a = items[i].a;
     if (ring_serves(a)) return false;
@@ -697,26 +758,30 @@ bool tile_batch_plan(const WgradBatchItem* items, int count, WTileBatch& b) {
     e.x = items[i].x; e.x1 = items[i].x1; e.c_first = items[i].c_first; e.gy = items[i].gy; e.gw = items[i].gw;
     e.tw = p.tw;
     e.tiles_d = p.tiles_d; e.tiles_h = p.tiles_h; e.tiles_w = p.tiles_w; e.ntiles = p.ntiles;
+    e.tps = (int)cdiv(p.ntiles, unit_parts(p.ntiles, a.cout));
+    e.parts = (int)cdiv(p.ntiles, e.tps);
     e.nblk_ci = p.nblk_ci; e.nblk = p.nblk;
-    e.pos_begin = (int)pos;
-    pos += (int64_t)p.nblk * (p.ntiles + kUnitCost);
-    if (pos > 0x7fffff) return false;  // 32-bit cuts
   }
-  b.total = (int)pos;
-  b.wgs = b.total < kTargetWorkgroups ? b.total : kTargetWorkgroups;
+  if (!lay_out(b, 1)) return false;
   // Blocks shared by three workgroups: where the busiest one's load, in tiles of 1.7 us instead of 2.4, is then smaller.
   // (With at least one block per compute unit the chip is busy as it is.)
-  if (pos * 3 <= 0x7fffff) {
-    int64_t blocks = 0;
-    for (int i = 0; i < count; ++i) blocks += b.e[i].nblk;
-    if (3 * blocks <= kTargetWorkgroups || (blocks <= kTargetWorkgroups && 17 * busiest(b, 3) < 24 * busiest(b, 1))) {
-      b.planes = true;
-      b.total *= 3;
-      for (int i = 0; i < count; ++i) b.e[i].pos_begin *= 3;
-      b.wgs = b.total < kTargetWorkgroups ? b.total : kTargetWorkgroups;
-    }
-  }
+  int64_t blocks = 0;
+  for (int i = 0; i < count; ++i) blocks += (int64_t)b.e[i].nblk * b.e[i].parts;
+  if ((int64_t)b.total * 3 <= 0x7fffff &&
+      (3 * blocks <= kTargetWorkgroups || (blocks <= kTargetWorkgroups && 17 * busiest(b, 3) < 24 * busiest(b, 1))))
+    lay_out(b, 3);
   return true;
+}
+
+// Bytes of the slices of the problems cut into parts, and where each lies from `ws` on (null: only asked).
+size_t place_slices(WTileBatch& b, char* ws) {
+  size_t bytes = 0;
+  for (int i = 0; i < b.count; ++i) {
+    if (b.e[i].parts == 1) continue;
+    if (ws != nullptr) b.e[i].ws = (float*)(ws + bytes);
+    bytes += align_up((size_t)b.e[i].parts * b.e[i].a.cout * 27 * b.e[i].a.cin * sizeof(float), 256);
+  }
+  return bytes;
 }
 
 template <typename T>
@@ -731,7 +796,11 @@ int launch_tile_batch(const WTileBatch& b, int gw_dtype, hipStream_t st) {
     else SFH_WGRAD_BATCH(T, false);
   }
 #undef SFH_WGRAD_BATCH
-  return check_launch("wgrad_mfma_batch_kernel");
+  if (int rc = check_launch("wgrad_mfma_batch_kernel")) return rc;
+  if (b.sum_wgs == 0) return SFH_OK;
+  if (gw_dtype == SFH_FP32) hipLaunchKernelGGL((wgrad_mfma_batch_sum<float>), dim3((unsigned)b.sum_wgs), dim3(256), 0, st, b);
+  else hipLaunchKernelGGL((wgrad_mfma_batch_sum<T>), dim3((unsigned)b.sum_wgs), dim3(256), 0, st, b);
+  return check_launch("wgrad_mfma_batch_sum");
 }
 
 }  // namespace
@@ -797,9 +866,10 @@ size_t mfma_wgrad_batch_workspace_bytes(const WgradBatchItem* items, int count, 
   if (split_list(items, count, ring, nring, tile, ntile) != SFH_OK) return 0;
   WTileBatch tb;
   if (ntile > 0 && !tile_batch_plan(tile, ntile, tb)) return 0;
-  if (nring == 0) return 256;  // (nothing is needed; a non-zero answer says the list is taken)
+  const size_t slices = ntile > 0 ? place_slices(tb, nullptr) : 0;
+  if (nring == 0) return slices > 0 ? slices : 256;  // (where nothing is needed a non-zero answer says the list is taken)
   const size_t bytes = mfma_wgrad_ring_batch_workspace_bytes(ring, nring, max_wgs);
-  return bytes;
+  return bytes > 0 ? slices + bytes : 0;
 }
 
 int mfma_wgrad_batch(const WgradBatchItem* items, int count, int dtype, int gw_dtype, void* workspace, size_t workspace_bytes,
@@ -811,8 +881,14 @@ int mfma_wgrad_batch(const WgradBatchItem* items, int count, int dtype, int gw_d
     return fail(SFH_ERR_UNSUPPORTED, "conv3d wgrad batch: a problem of the list is served only by a launch of its own");
   WTileBatch tb;
   if (ntile > 0 && !tile_batch_plan(tile, ntile, tb)) return fail(SFH_ERR_UNSUPPORTED, "conv3d wgrad batch: the small-volume problems cannot share a launch");
+  const size_t slices = ntile > 0 ? place_slices(tb, nullptr) : 0;
+  if (slices > 0) {
+    if (workspace == nullptr || workspace_bytes < slices)
+      return fail(SFH_ERR_WORKSPACE, "conv3d wgrad batch: workspace of %zu bytes needed for the small-volume problems, got %zu", slices, workspace_bytes);
+    place_slices(tb, (char*)workspace);
+  }
   if (nring > 0)
-    if (int rc = mfma_wgrad_ring_batch(ring, nring, dtype, gw_dtype, workspace, workspace_bytes, st, max_wgs)) return rc;
+    if (int rc = mfma_wgrad_ring_batch(ring, nring, dtype, gw_dtype, (char*)workspace + slices, workspace_bytes - slices, st, max_wgs)) return rc;
   if (ntile > 0) return dtype == SFH_BF16 ? launch_tile_batch<bf16_t>(tb, gw_dtype, st) : launch_tile_batch<fp16_t>(tb, gw_dtype, st);
   return SFH_OK;
 }

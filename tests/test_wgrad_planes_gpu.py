@@ -50,3 +50,23 @@ def test_in_a_list(grad_dtype, extra):
     if extra:
         short = sa.conv3d_backward_weight_batch(items[:4], grad_dtype=grad_dtype)
         assert all(torch.equal(a, b) for a, b in zip(short, got))
+
+
+@pytest.mark.parametrize("grad_dtype", [None, torch.float32])
+@pytest.mark.parametrize("n,cin,cout,spatial,padding", [
+    (1, 32, 64, (18, 8, 16), 1),       # nine tiles: two parts, the last one short
+    (2, 64, 64, (13, 13, 13), 1),      # 28 tiles in five parts, over two samples
+    (1, 128, 64, (28, 9, 9), (0, 1, 2)),
+    (3, 32, 32, (12, 9, 7), 1),        # rows of eight
+    (1, 64, 128, (28, 13, 13), 1),     # too many output channels: whole
+])
+def test_blocks_cut_into_parts(n, cin, cout, spatial, padding, grad_dtype):
+    """The slices of a list's problems lie beside those of its large rows; alone or not, the bits of a problem are the same."""
+    cases = [(n, cin, cout, spatial, padding, torch.bfloat16), (1, 32, 32, (4, 5, 33), 1, torch.bfloat16), (1, 32, 64, (11, 16, 16), 1, torch.bfloat16)]
+    problems = [_problem(*c, seed=9 + i) for i, c in enumerate(cases)]
+    items = [(o["input"].cuda(), p.weight_shape, o["grad_output"].cuda(), p.padding) for p, o in problems]
+    got = sa.conv3d_backward_weight_batch(items, grad_dtype=grad_dtype)
+    for (prob, ops), g in zip(problems, got):
+        orc.assert_close(g.to(torch.bfloat16), orc.conv_reference(prob, ops, "bwd-weight"), prob, "bwd-weight")
+    alone = sa.conv3d_backward_weight_batch(items[:1], grad_dtype=grad_dtype)
+    assert torch.equal(alone[0], got[0])
