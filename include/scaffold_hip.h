@@ -93,7 +93,8 @@ typedef struct sfh_groupnorm_desc {
  * 104: sfh_conv3d_wgrad_batch, sfh_conv3d_wgrad_batch_supported, sfh_conv3d_wgrad_batch_workspace_bytes added;
  * SFH_KERNEL_SPLIT (6) is a value sfh_conv3d_launch_geometry may report. Nothing removed or changed.
  * 105: SFH_FLAG_SHARE_DEVICE; sfh_conv3d_wgrad_batch_workspace_bytes takes the call's flags (changed: one more argument).
- * 106: sfh_conv3d_pack_master_weights added. 107: sfh_convT3d_fwd_padded, sfh_convT3d_wgrad_bias_padded added. */
+ * 106: sfh_conv3d_pack_master_weights added. 107: sfh_convT3d_fwd_padded, sfh_convT3d_wgrad_bias_padded,
+ * sfh_groupnorm_fwd_pool added. */
 int sfh_version(void);
 const char* sfh_last_error(void);
 /* Fills name (<= name_len bytes), compute-unit count, LDS bytes per workgroup. */
@@ -391,6 +392,15 @@ int sfh_groupnorm_fwd_from_partials(const sfh_groupnorm_desc* p, int x_dtype, in
                                     const void* x, const void* gamma, const void* beta, void* y_slab,
                                     int64_t halo_rows, float* mean, float* rstd, const float* partials,
                                     size_t partials_bytes, int32_t records, void* stream);
+/* The same, and the 2x2x2 maximum of the result (sfh_maxpool2_fwd's values and indices) from the same pass: what an encoder block of
+ * the U-Net ends with and the pooling behind it (ScaFFold/unet/unet_parts.py:165). extents: D, H, W of x. pooled_slab: faces of
+ * pooled_halo_elems elements, zeroed here, around the pooled tensor (0: no faces; sfh_maxpool2_fwd_slab's layout, per sample).
+ * idx: null where no gradient is wanted. 16-bit types on the vector path, extents of at least 2; SFH_ERR_UNSUPPORTED otherwise,
+ * before any launch. */
+int sfh_groupnorm_fwd_pool(const sfh_groupnorm_desc* p, const int32_t extents[3], int dtype, int param_dtype, const void* x,
+                           const void* gamma, const void* beta, void* y_slab, int64_t halo_rows, float* mean, float* rstd,
+                           const float* partials, size_t partials_bytes, int32_t records, void* pooled_slab,
+                           int64_t pooled_halo_elems, uint8_t* idx, void* stream);
 
 /* The forward for callers that cannot allocate: code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc. It has no counterpart in the reference. Same kernels and results as sfh_groupnorm_fwd, but the

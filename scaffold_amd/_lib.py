@@ -159,6 +159,8 @@ _SIGNATURES = {
                                               c_size_t, c_uint32, c_void_p]),
     "sfh_convT3d_fwd_slab": (c_int, [POINTER(ConvTDesc), c_int, c_void_p, c_void_p, POINTER(c_int64), c_void_p, c_void_p, c_int64,
                                      c_void_p, c_size_t, c_uint32, c_void_p]),
+    "sfh_groupnorm_fwd_pool": (c_int, [POINTER(GroupNormDesc), POINTER(c_int32), c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
+                                       c_void_p, c_void_p, c_void_p, c_size_t, c_int32, c_void_p, c_int64, c_void_p, c_void_p]),
     "sfh_groupnorm_fwd_workspace_bytes": (c_size_t, [POINTER(GroupNormDesc), c_int]),
     "sfh_groupnorm_fwd": (c_int, [POINTER(GroupNormDesc), c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),

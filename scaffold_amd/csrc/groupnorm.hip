@@ -506,37 +506,27 @@ __device__ __forceinline__ void fold_welford_records(const float* __restrict__ r
   }
 }
 
-// ---- forward: normalise + affine (+ReLU) (vector path) ------------------------------------
-// When the sample's split partials are few (fold_in_consumer), every workgroup derives mean and rstd from them itself
-// (mean = K + S1/m, var = S2/m - (S1/m)^2, rstd = 1/sqrt(var + eps)): 32 KiB from L2 cost less than a launch of their
-// own, and the first workgroup of a sample writes them out for the backward pass. Otherwise gn_stats_finalize has run.
-template <typename T, typename TO, bool STREAM>
-__global__ void __launch_bounds__(kBlock) gn_normalize(const T* __restrict__ x, TO* __restrict__ y, const float* __restrict__ shift,
-                                                       const float* __restrict__ part, float* __restrict__ mean,
-                                                       float* __restrict__ rstd, const void* __restrict__ gamma,
-                                                       const void* __restrict__ beta, int param_dtype, int64_t S, int C, int G,
-                                                       int tpr, int rpp, int nsplit, int64_t rows_per_split, float m, float eps,
-                                                       int relu, int64_t y_halo, int npart, int welford) {
-  constexpr int V = VecOf<T>::N;
-  extern __shared__ float gstat[];  // sums[2 G] | mean[G] | rstd[G] | fold scratch (4 * kBlock)
+// `slab` is faces of `face` elements around `inner` of them (16-byte multiples): the sample's workgroups zero the two between them.
+template <typename T>
+__device__ __forceinline__ void zero_slab_faces(T* slab, int64_t face, int64_t inner) {
+  const int64_t pieces = face * (int64_t)sizeof(T) / 16;
+  uint4* lo = reinterpret_cast<uint4*>(slab);
+  uint4* hi = reinterpret_cast<uint4*>(slab + face + inner);
+  for (int64_t u = (int64_t)blockIdx.x * kBlock + threadIdx.x; u < pieces; u += (int64_t)gridDim.x * kBlock) {
+    lo[u] = make_uint4(0, 0, 0, 0);
+    hi[u] = make_uint4(0, 0, 0, 0);
+  }
+}
+
+// Mean and rstd of the sample's groups into g_mean / g_rstd (LDS, behind the sums that gstat starts with), from `npart` partial
+// records per sample: the statistics pass's own (one per workgroup of this grid, sums about the common shift), or (`welford`)
+// the records the producer of x left. The caller synchronises.
+__device__ __forceinline__ void group_statistics(const float* __restrict__ part, const float* __restrict__ shift, float* __restrict__ mean,
+                                                 float* __restrict__ rstd, float* gstat, int n, int G, int npart, int welford, float m,
+                                                 float eps) {
   const int tid = threadIdx.x;
-  const int n = blockIdx.y;
-  const int cg = C / G;
-  const int r = tid / tpr, cv = tid - r * tpr;
   float* g_mean = gstat + 2 * G;
   float* g_rstd = gstat + 3 * G;
-  // the workgroup's first rows are requested before anything else: the fold of the statistics below reads other memory
-  constexpr int U = 4;  // rows per batch: the next batch's loads are in flight while the current one is normalised
-  const T* xs = x + (int64_t)n * S * C + cv * V;
-  const int64_t begin = (int64_t)blockIdx.x * rows_per_split;
-  int64_t end = begin + rows_per_split;
-  if (end > S) end = S;
-  const int64_t step = rpp;
-  int64_t row = begin + r;
-  Piece<T, V> cur[U];
-  fetch_rows<STREAM>(cur, xs, row, step, end, begin, C, r < rpp);
-  // `npart` partial records per sample: the statistics pass's own (one per workgroup of this grid, sums about the
-  // common shift), or (`welford`) the records the producer of x left
   if (welford && fold_in_consumer(G, npart, kGnRecordFloats)) {
     fold_welford_records(part + (int64_t)n * npart * G * kGnRecordFloats, G, npart, gstat + 4 * G, [&](int g, float c, float a, float q) {
       const float d = a / m;
@@ -571,18 +561,41 @@ __global__ void __launch_bounds__(kBlock) gn_normalize(const T* __restrict__ x, 
       g_rstd[g] = rstd[n * G + g];
     }
   }
+}
+
+// ---- forward: normalise + affine (+ReLU) (vector path) ------------------------------------
+// When the sample's split partials are few (fold_in_consumer), every workgroup derives mean and rstd from them itself
+// (mean = K + S1/m, var = S2/m - (S1/m)^2, rstd = 1/sqrt(var + eps)): 32 KiB from L2 cost less than a launch of their
+// own, and the first workgroup of a sample writes them out for the backward pass. Otherwise gn_stats_finalize has run.
+template <typename T, typename TO, bool STREAM>
+__global__ void __launch_bounds__(kBlock) gn_normalize(const T* __restrict__ x, TO* __restrict__ y, const float* __restrict__ shift,
+                                                       const float* __restrict__ part, float* __restrict__ mean,
+                                                       float* __restrict__ rstd, const void* __restrict__ gamma,
+                                                       const void* __restrict__ beta, int param_dtype, int64_t S, int C, int G,
+                                                       int tpr, int rpp, int nsplit, int64_t rows_per_split, float m, float eps,
+                                                       int relu, int64_t y_halo, int npart, int welford) {
+  constexpr int V = VecOf<T>::N;
+  extern __shared__ float gstat[];  // sums[2 G] | mean[G] | rstd[G] | fold scratch (4 * kBlock)
+  const int tid = threadIdx.x;
+  const int n = blockIdx.y;
+  const int cg = C / G;
+  const int r = tid / tpr, cv = tid - r * tpr;
+  float* g_mean = gstat + 2 * G;
+  float* g_rstd = gstat + 3 * G;
+  // the workgroup's first rows are requested before anything else: the fold of the statistics below reads other memory
+  constexpr int U = 4;  // rows per batch: the next batch's loads are in flight while the current one is normalised
+  const T* xs = x + (int64_t)n * S * C + cv * V;
+  const int64_t begin = (int64_t)blockIdx.x * rows_per_split;
+  int64_t end = begin + rows_per_split;
+  if (end > S) end = S;
+  const int64_t step = rpp;
+  int64_t row = begin + r;
+  Piece<T, V> cur[U];
+  fetch_rows<STREAM>(cur, xs, row, step, end, begin, C, r < rpp);
+  group_statistics(part, shift, mean, rstd, gstat, n, G, npart, welford, m, eps);
   __syncthreads();
-  // y is a slab of y_halo + S + y_halo rows per sample: the sample's workgroups zero the two faces between them
   const int64_t y_sample = (int64_t)n * (S + 2 * y_halo) * C;
-  if (y_halo > 0) {
-    const int64_t face_pieces = y_halo * C * (int64_t)sizeof(TO) / 16;
-    uint4* lo = reinterpret_cast<uint4*>(y + y_sample);
-    uint4* hi = reinterpret_cast<uint4*>(y + y_sample + (y_halo + S) * C);
-    for (int64_t u = (int64_t)blockIdx.x * kBlock + tid; u < face_pieces; u += (int64_t)gridDim.x * kBlock) {
-      lo[u] = make_uint4(0, 0, 0, 0);
-      hi[u] = make_uint4(0, 0, 0, 0);
-    }
-  }
+  zero_slab_faces(y + y_sample, y_halo * C, S * C);
   if (r >= rpp) return;
   float mu[V], rs[V], ga[V], be[V];
   load_params<V>(gamma, param_dtype, cv * V, 1.f, ga);
@@ -617,6 +630,119 @@ __global__ void __launch_bounds__(kBlock) gn_normalize(const T* __restrict__ x, 
       for (int u = 0; u < U; ++u) cur[u] = nxt[u];
     }
     row = next;
+  }
+}
+
+// The same with the 2x2x2 maximum of what is stored, and which voxel of its cell it is, from one pass (an encoder block's last
+// normalisation and the pooling behind it; the pooling by itself reads the tensor again). A thread takes a 16-byte piece of the channels
+// of a whole cell: eight loads in flight. Cells cover odd extents too, whose last planes are normalised but not pooled. Bound by memory.
+// bf16, the two launches -> this one, us: 64 channels of 128^3 141 -> 106, of 96x80x112 64 -> 48, 128 of 64^3 37.7 -> 31.1, 64 of 32x64x64 16.0 -> 13.4,
+// 32 of 32^3 9.9 -> 7.6 (a launch less); the next cell is requested before the one at hand is worked on (96x80x112 50.7 -> 48, 64^3 33.1 -> 31.1).
+struct PooledOut {
+  void* y;          // slab of faces of `face` elements, or none
+  uint8_t* idx;     // null: not wanted
+  int64_t face;
+};
+template <typename T, bool STREAM>
+__global__ void __launch_bounds__(kBlock) gn_normalize_pool(const T* __restrict__ x, T* __restrict__ y, PooledOut pooled,
+                                                            const float* __restrict__ part, float* __restrict__ mean,
+                                                            float* __restrict__ rstd, const void* __restrict__ gamma,
+                                                            const void* __restrict__ beta, int param_dtype, int D, int H, int W, int C, int G,
+                                                            int tpr, int rpp, int cells, int cells_per, float m, float eps, int relu,
+                                                            int64_t y_halo, int npart) {
+  constexpr int V = 8;
+  extern __shared__ float gstat[];  // sums[2 G] | mean[G] | rstd[G] | fold scratch (4 * kBlock)
+  const int tid = threadIdx.x, n = blockIdx.y, cg = C / G;
+  const int r = tid / tpr, cv = tid - r * tpr;
+  const int64_t S = (int64_t)D * H * W;
+  const int pd = D / 2, ph = H / 2, pw = W / 2, ch = (H + 1) / 2, cw = (W + 1) / 2;
+  const int begin = (int)blockIdx.x * cells_per, end = begin + cells_per < cells ? begin + cells_per : cells;
+  const T* xs = x + (int64_t)n * S * C + cv * V;
+  struct Cell {
+    int od, oh, ow;
+    int64_t at;  // its first voxel
+  };
+  auto place = [&](int cell) {
+    Cell c;
+    c.ow = (int)((uint32_t)cell % (uint32_t)cw);
+    const uint32_t t = (uint32_t)cell / (uint32_t)cw;
+    c.oh = (int)(t % (uint32_t)ch);
+    c.od = (int)(t / (uint32_t)ch);
+    c.at = ((int64_t)2 * c.od * H + 2 * c.oh) * W + 2 * c.ow;
+    return c;
+  };
+  auto inside = [&](const Cell& c, int k) { return (2 * c.od + (k >> 2) < D) & (2 * c.oh + ((k >> 1) & 1) < H) & (2 * c.ow + (k & 1) < W); };
+  auto offset = [&](int k) { return ((int64_t)(k >> 2) * H + ((k >> 1) & 1)) * W + (k & 1); };
+  Piece<T, V> in[8];
+  auto fetch = [&](Piece<T, V> (&b)[8], const Cell& c) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) b[k].template load<STREAM>(xs + (c.at + (inside(c, k) ? offset(k) : 0)) * C);
+  };
+  int cell = begin + (r < rpp ? r : 0);
+  Cell c = place(cell < end ? cell : begin);
+  fetch(in, c);  // before anything else: the fold of the statistics below reads other memory
+  group_statistics(part, nullptr, mean, rstd, gstat, n, G, npart, 1, m, eps);
+  __syncthreads();
+  T* ys = y + (int64_t)n * (S + 2 * y_halo) * C;
+  zero_slab_faces(ys, y_halo * C, S * C);
+  const int64_t p_cells = (int64_t)pd * ph * pw;
+  T* ps = (T*)pooled.y + (int64_t)n * (p_cells * C + 2 * pooled.face);
+  zero_slab_faces(ps, pooled.face, p_cells * C);
+  if (r >= rpp) return;
+  ys += y_halo * C + cv * V;
+  ps += pooled.face + cv * V;
+  uint8_t* is = pooled.idx != nullptr ? pooled.idx + (int64_t)n * p_cells * C + cv * V : nullptr;
+  float mu[V], rs[V], ga[V], be[V];
+  load_params<V>(gamma, param_dtype, cv * V, 1.f, ga);
+  load_params<V>(beta, param_dtype, cv * V, 0.f, be);
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+    const int g = (cv * V + e) / cg;
+    mu[e] = gstat[2 * G + g];
+    rs[e] = gstat[3 * G + g];
+  }
+  while (cell < end) {
+    const Cell now = c;
+    cell += rpp;
+    Piece<T, V> next[8];
+    if (cell < end) {
+      c = place(cell);
+      fetch(next, c);
+    }
+    float best[V];
+    int which[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) { best[e] = -INFINITY; which[e] = 0; }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      float f[V], o[V];
+      in[k].unpack(f);
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const float xh = (f[e] - mu[e]) * rs[e];
+        const float v = fmaf(xh, ga[e], be[e]);
+        o[e] = relu ? relu_keep_nan(v) : v;
+      }
+      Piece<T, V> out;  // what is stored, and compared: the rounded values
+      out.q = pack_piece<T>(o);
+      if (inside(now, k)) *reinterpret_cast<uint4*>(ys + (now.at + offset(k)) * C) = out.q;
+      out.unpack(o);
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const bool take = (best[e] < o[e]) | (o[e] != o[e]);
+        best[e] = take ? o[e] : best[e];
+        which[e] = take ? k : which[e];
+      }
+    }
+    if (now.od < pd && now.oh < ph && now.ow < pw) {
+      const int64_t o = (((int64_t)now.od * ph + now.oh) * pw + now.ow) * C;
+      St<T, V>::run(ps + o, best);
+      if (is != nullptr)
+        *reinterpret_cast<uint2*>(is + o) = make_uint2(which[0] | which[1] << 8 | which[2] << 16 | (uint32_t)which[3] << 24,
+                                                       which[4] | which[5] << 8 | which[6] << 16 | (uint32_t)which[7] << 24);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) in[k] = next[k];
   }
 }
 
@@ -1569,6 +1695,55 @@ extern "C" int sfh_groupnorm_fwd_from_partials(const sfh_groupnorm_desc* p, int 
     return fail(SFH_ERR_WORKSPACE, "groupnorm from partials: %d records per sample are %zu bytes, got %zu", records, need, partials_bytes);
   return groupnorm_fwd_any(p, x_dtype, y_dtype, param_dtype, x, gamma, beta, y_slab, halo_rows, mean, rstd, nullptr, 0, stream, partials,
                            records);
+}
+
+namespace {
+template <typename T>
+int normalize_pool(const sfh_groupnorm_desc& p, const GnPlan& pl, const int32_t extents[3], int param_dtype, const void* x, const void* gamma,
+                   const void* beta, void* y, int64_t y_halo, float* mean, float* rstd, const float* records, int nrec, const PooledOut& out,
+                   hipStream_t st) {
+  const int G = p.groups, C = p.c;
+  const float m = (float)p.spatial * (float)(C / G);
+  if (!fold_in_consumer_host(G, nrec, kGnRecordFloats)) {
+    hipLaunchKernelGGL(gn_welford_finalize, dim3(G, p.n), dim3(kBlock), 0, st, records, mean, rstd, G, nrec, m, p.eps);
+    if (int rc = check_launch("gn_welford_finalize")) return rc;
+  }
+  // as many workgroups as the plain normalisation's, in whole passes over cells
+  const int cells = (int)(cdiv(extents[0], 2) * cdiv(extents[1], 2) * cdiv(extents[2], 2));
+  const int cells_per = (int)cdiv(cdiv(cells, pl.nsplit), pl.rpp) * pl.rpp;
+  const dim3 grid((unsigned)cdiv(cells, cells_per), p.n);
+  hipLaunchKernelGGL((pl.stream ? gn_normalize_pool<T, true> : gn_normalize_pool<T, false>), grid, dim3(kBlock),
+                     (size_t)(4 * G + 4 * kBlock) * sizeof(float), st, (const T*)x, (T*)y, out, records, mean, rstd, gamma, beta, param_dtype,
+                     extents[0], extents[1], extents[2], C, G, pl.tpr, pl.rpp, cells, cells_per, m, p.eps, p.relu, y_halo, nrec);
+  return check_launch("gn_normalize_pool");
+}
+}  // namespace
+
+extern "C" int sfh_groupnorm_fwd_pool(const sfh_groupnorm_desc* p, const int32_t extents[3], int dtype, int param_dtype, const void* x,
+                                      const void* gamma, const void* beta, void* y_slab, int64_t halo_rows, float* mean, float* rstd,
+                                      const float* partials, size_t partials_bytes, int32_t records, void* pooled_slab, int64_t pooled_halo_elems,
+                                      uint8_t* idx, void* stream) {
+  if (int rc = check_desc(p, dtype)) return rc;
+  if (!dtype_ok(param_dtype)) return fail(SFH_ERR_INVALID, "groupnorm: bad param dtype");
+  if (x == nullptr || y_slab == nullptr || mean == nullptr || rstd == nullptr || pooled_slab == nullptr || extents == nullptr)
+    return fail(SFH_ERR_INVALID, "groupnorm with pooling: null tensor");
+  if (halo_rows < 0 || pooled_halo_elems < 0) return fail(SFH_ERR_INVALID, "groupnorm with pooling: negative halo");
+  for (int i = 0; i < 3; ++i)
+    if (extents[i] < 1) return fail(SFH_ERR_INVALID, "groupnorm with pooling: bad extents");
+  if ((int64_t)extents[0] * extents[1] * extents[2] != p->spatial) return fail(SFH_ERR_INVALID, "groupnorm with pooling: the extents are not the descriptor's");
+  if (partials == nullptr || records < 1 || !aligned16(partials)) return fail(SFH_ERR_INVALID, "groupnorm with pooling: no records, or not on 16 bytes");
+  const size_t need = (size_t)p->n * records * p->groups * kGnRecordFloats * sizeof(float);
+  if (partials_bytes < need)
+    return fail(SFH_ERR_WORKSPACE, "groupnorm with pooling: %d records per sample are %zu bytes, got %zu", records, need, partials_bytes);
+  const GnPlan pl = make_plan(*p, dtype, aligned16(x) && aligned16(y_slab) && aligned16(pooled_slab));
+  if (dtype == SFH_FP32 || !pl.vector || (reinterpret_cast<uintptr_t>(idx) & 7u) != 0 || (halo_rows * p->c * 2) % 16 != 0 ||
+      (pooled_halo_elems * 2) % 16 != 0 || extents[0] < 2 || extents[1] < 2 || extents[2] < 2 || p->spatial > 0x7fffffffLL)
+    return fail(SFH_ERR_UNSUPPORTED, "groupnorm with pooling: 16-bit types on the vector path, cells on every axis, faces of 16-byte multiples");
+  const PooledOut out{pooled_slab, idx, pooled_halo_elems};
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == SFH_BF16)
+    return normalize_pool<bf16_t>(*p, pl, extents, param_dtype, x, gamma, beta, y_slab, halo_rows, mean, rstd, partials, records, out, st);
+  return normalize_pool<fp16_t>(*p, pl, extents, param_dtype, x, gamma, beta, y_slab, halo_rows, mean, rstd, partials, records, out, st);
 }
 
 // ---- the forward for callers that may not allocate ------------------------------------------------------------------

@@ -1080,6 +1080,49 @@ NormResult launch_norm(const Tensor& input, int64_t groups, const Tensor& weight
   return r;
 }
 
+// The normalisation with the pooling that follows it, from the records the producer of `input` left, in one launch.
+struct PooledResult {
+  Tensor pooled, slab, idx;  // idx: undefined where no gradient is wanted
+};
+bool launch_norm_pool(const Tensor& input, int64_t groups, const Tensor& weight, const Tensor& bias, double eps, bool relu, int64_t halo,
+                      const Tensor& partials, int32_t records, int64_t pool_halo, bool want_idx, NormResult& r, PooledResult& out) {
+  const int64_t n = input.size(0), c = input.size(1), d2 = input.size(2) / 2, h2 = input.size(3) / 2, w2 = input.size(4) / 2;
+  if (d2 < 1 || h2 < 1 || w2 < 1 || n < 1 || c % 8 != 0 || input.scalar_type() == at::kFloat || (pool_halo > 0 && n != 1)) return false;
+  c10::OptionalDeviceGuard guard(input.device());
+  Tensor w = weight.contiguous(), b = bias.contiguous();
+  if (w.scalar_type() != b.scalar_type()) b = b.to(w.scalar_type());
+  NormResult made;
+  PooledResult pool;
+  made.stats = plain({2, n, groups}, input, at::kFloat);
+  float* mean = (float*)out_ptr(made.stats);
+  int64_t halo_rows = 0;
+  if (halo > 0 && n == 1) {
+    made.slab = volume({1, c, input.size(2) + 2 * halo, input.size(3), input.size(4)}, input, input.scalar_type());
+    made.y = made.slab.narrow(2, halo, input.size(2));
+    halo_rows = halo * input.size(3) * input.size(4);
+  } else {
+    made.y = volume(input.sizes(), input, input.scalar_type());
+  }
+  if (pool_halo > 0) {
+    pool.slab = volume({1, c, d2 + 2 * pool_halo, h2, w2}, input, input.scalar_type());
+    pool.pooled = pool.slab.narrow(2, pool_halo, d2);
+  } else {
+    pool.pooled = volume({n, c, d2, h2, w2}, input, input.scalar_type());
+  }
+  if (want_idx) pool.idx = plain({n, d2, h2, w2, c}, input, at::kByte);
+  const int32_t extents[3] = {(int32_t)input.size(2), (int32_t)input.size(3), (int32_t)input.size(4)};
+  const sfh_groupnorm_desc d{(int32_t)n, (int32_t)c, (int32_t)groups, relu ? 1 : 0, input.numel() / (n * c), (float)eps};
+  const int rc = sfh_groupnorm_fwd_pool(&d, extents, code_of(input.scalar_type()), code_of(w.scalar_type()), ptr(input), ptr(w), ptr(b),
+                                        out_ptr(made.slab.defined() ? made.slab : made.y), halo_rows, mean, mean + n * groups, (const float*)ptr(partials),
+                                        (size_t)partials.numel() * 4, records, out_ptr(pool.slab.defined() ? pool.slab : pool.pooled),
+                                        pool_halo > 0 ? pool_halo * h2 * w2 * c : 0, (uint8_t*)out_ptr(pool.idx), stream_of(input));
+  if (rc == SFH_ERR_UNSUPPORTED) return false;
+  check(rc, "group_norm with pooling");
+  r = std::move(made);
+  out = std::move(pool);
+  return true;
+}
+
 void save_norm(NormSaved& s, const Tensor& input, const Tensor& weight, const Tensor& bias, const Tensor& stats, int64_t groups, bool relu) {
   s.input.keep(input);
   s.weight.keep(weight);
@@ -1147,11 +1190,12 @@ struct ConvNormNode : public LaunchNode {  // edges: x, convolution weight, norm
   }
 };
 
-// modules.conv_then_norm: (y, slab or None), or None (nothing launched) for a call that is not served as it stands.
-// x / x_read, weight / w, packed forms, halo, master, family and early as in record_conv.
+// modules.conv_then_norm: (y, slab or None, pooled), or None (nothing launched) for a call that is not served as it stands.
+// x / x_read, weight / w, packed forms, halo, master, family and early as in record_conv.  `pool_halo` >= 0: a MaxPool3d(2) with that
+// halo follows; pooled is what it will ask for (tensor, slab or None, indices or None), or None where this launch does not make it.
 py::object conv_norm(const Tensor& x, const Tensor& x_read, const Tensor& weight, const Tensor& w, const MaybeTensor& packed_fwd, const MaybeTensor& packed_dgrad,
                      int64_t halo, py::handle stride, py::handle padding, py::handle dilation, bool master, int family, bool early, int64_t groups,
-                     const Tensor& norm_weight, const Tensor& norm_bias, double eps, bool relu, int64_t out_halo) {
+                     const Tensor& norm_weight, const Tensor& norm_bias, double eps, bool relu, int64_t out_halo, int64_t pool_halo) {
   int32_t s[3], p[3], d[3];
   if (!three(stride, s) || !three(padding, p) || !three(dilation, d) || !x_read.is_contiguous(kCL3D)) return py::none();
   const bool graph = wants_grad({&x, &weight, &norm_weight, &norm_bias});
@@ -1162,10 +1206,13 @@ py::object conv_norm(const Tensor& x, const Tensor& x_read, const Tensor& weight
   if (!norm_gate(x_read, prob.key.d.n, prob.key.d.cout, (int64_t)prob.out[0] * prob.out[1] * prob.out[2], groups, norm_weight, norm_bias)) return py::none();
   ConvResult c;
   NormResult r;
+  PooledResult pool;
   {
     at::AutoGradMode no_grad(false);
     c = launch_conv(prob, x_read, Tensor(), w, Tensor(), or_none(packed_fwd), (int)groups);
-    r = launch_norm(c.y, groups, norm_weight, norm_bias, eps, relu, c.y.scalar_type(), out_halo, c.records > 0 ? c.partials : Tensor(), c.records);
+    if (pool_halo < 0 || c.records < 1 ||
+        !launch_norm_pool(c.y, groups, norm_weight, norm_bias, eps, relu, out_halo, c.partials, c.records, pool_halo, graph, r, pool))
+      r = launch_norm(c.y, groups, norm_weight, norm_bias, eps, relu, c.y.scalar_type(), out_halo, c.records > 0 ? c.partials : Tensor(), c.records);
     if (graph && r.slab.defined()) r.y = r.y.detach();
   }
   if (graph) {
@@ -1178,7 +1225,8 @@ py::object conv_norm(const Tensor& x, const Tensor& x_read, const Tensor& weight
     save_norm(node->norm, c.y, norm_weight, norm_bias, r.stats, groups, relu);
     torch::autograd::set_history(r.y, node);
   }
-  return py::make_tuple(r.y, tensor_or_none(r.slab));
+  const py::object pooled = pool.pooled.defined() ? py::object(py::make_tuple(pool.pooled, tensor_or_none(pool.slab), tensor_or_none(pool.idx))) : py::none();
+  return py::make_tuple(r.y, tensor_or_none(r.slab), pooled);
 }
 
 // ---- MaxPool3d(2) --------------------------------------------------------------------------------------------------------
@@ -1211,8 +1259,9 @@ struct MaxPoolNode : public LaunchNode {  // edge: x; the second output, where t
   }
 };
 
-// pooling.max_pool3d_2x: (y, slab or None[, alias of x]), or None for a call that is not served.
-py::object max_pool(const Tensor& x_in, int64_t halo, bool with_skip) {
+// pooling.max_pool3d_2x: (y, slab or None[, alias of x]), or None for a call that is not served.  `given`: what the producer of x_in
+// has pooled from these very bits, for this halo (a call that needs indices it did not keep launches).
+py::object max_pool(const Tensor& x_in, int64_t halo, bool with_skip, const MaybeTensor& given, const MaybeTensor& given_slab, const MaybeTensor& given_idx) {
   if (x_in.dim() != 5 || !on_gpu(x_in) || code_of(x_in.scalar_type()) < 0 || x_in.size(1) < 1) return py::none();
   for (int i = 2; i < 5; ++i)
     if (x_in.size(i) < 1) return py::none();
@@ -1224,11 +1273,16 @@ py::object max_pool(const Tensor& x_in, int64_t halo, bool with_skip) {
     const Tensor x = dense(x_in);
     c10::OptionalDeviceGuard guard(x.device());
     const int64_t n = z[0], c = z[1], d2 = z[2] / 2, h2 = z[3] / 2, w2 = z[4] / 2;
-    idx = plain({n, d2, h2, w2, c}, x, at::kByte);
+    const bool made = given.has_value() && (!graph || given_idx.has_value());
+    idx = made ? or_none(given_idx) : plain({n, d2, h2, w2, c}, x, at::kByte);
     const sfh_pool_desc d{(int32_t)n, (int32_t)c, (int32_t)z[2], (int32_t)z[3], (int32_t)z[4]};
     const int code = code_of(x.scalar_type());
     int rc = SFH_ERR_UNSUPPORTED;
-    if (halo > 0 && n == 1 && d2 > 0 && h2 > 0 && w2 > 0) {
+    if (made) {
+      y = *given;
+      slab = or_none(given_slab);
+      rc = SFH_OK;
+    } else if (halo > 0 && n == 1 && d2 > 0 && h2 > 0 && w2 > 0) {
       slab = volume({1, c, d2 + 2 * halo, h2, w2}, x, x.scalar_type());
       rc = sfh_maxpool2_fwd_slab(&d, code, ptr(x), out_ptr(slab), halo * h2 * w2 * c, (uint8_t*)out_ptr(idx), stream_of(x));
       if (rc != SFH_ERR_UNSUPPORTED) y = slab.narrow(2, halo, d2);

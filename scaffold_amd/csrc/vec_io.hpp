@@ -77,6 +77,15 @@ template <int V> struct St<float, V> {
   }
 };
 
+// Eight values rounded to T, as St stores them.
+template <typename T> __device__ __forceinline__ uint4 pack_piece(const float (&f)[8]);
+template <> __device__ __forceinline__ uint4 pack_piece<bf16_t>(const float (&f)[8]) {
+  return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7]));
+}
+template <> __device__ __forceinline__ uint4 pack_piece<fp16_t>(const float (&f)[8]) {
+  return make_uint4(pack_fp16x2(f[0], f[1]), pack_fp16x2(f[2], f[3]), pack_fp16x2(f[4], f[5]), pack_fp16x2(f[6], f[7]));
+}
+
 template <typename T> struct VecOf { static constexpr int N = 8; };
 template <> struct VecOf<float> { static constexpr int N = 4; };
 

@@ -458,13 +458,17 @@ def conv_then_norm(conv, norm, x):
         family = _deferrable(weight, in_shape, weight.shape, stride, padding, dilation, x_read.dtype)
         _set_early_callbacks()
     pf, pd = (None, None) if packs is None else packs
+    # (a tensor made in inference mode has no version to tell a later write by)
+    pool_halo = -1 if norm.pool_next is None or torch.is_inference_mode_enabled() else norm.pool_next
     done = _lib.native().conv_norm(x, x_read, receives, w, pf, pd, halo, stride, padding, dilation, master, family, defer == 2, norm.num_groups,
-                                   gamma, beta, norm.eps, norm.activation == "relu", norm.out_halo)
+                                   gamma, beta, norm.eps, norm.activation == "relu", norm.out_halo, pool_halo)
     if done is None:
         return None
-    y, slab = done
+    y, slab, pooled = done
     if slab is not None:
         y._sfh_slab = (slab, norm.out_halo)
+    if pooled is not None:
+        y._sfh_pooled = (*pooled, pool_halo, y._version)
     return y
 
 
@@ -547,6 +551,9 @@ class FastGroupNorm(nn.GroupNorm):
     """``nn.GroupNorm`` (+ optional fused ReLU) served by the HIP kernels; output dtype = input dtype."""
 
     activation = None  # class-level default: not a parameter, buffer or state-dict key
+    #: the halo of a ``FastMaxPool3d`` that reads this module's output next (None: none does): where the convolution in front runs
+    #: with this module in one call, that call also leaves what the pooling will ask for on its result
+    pool_next = None
     #: depth planes of zero halo to leave around the output for a following ``FastConv3d.shard_halo`` (0: none)
     out_halo = 0
 

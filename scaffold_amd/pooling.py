@@ -33,7 +33,13 @@ def _refuse(x):
 
 def _pool(x, out_halo, with_skip):
     """The launch and its autograd node: ``(pooled, ...)``; the pooled tensor carries the slab it lies in, if any."""
-    done = _lib.native().max_pool(x, int(out_halo), with_skip) if isinstance(x, torch.Tensor) else None
+    done = None
+    if isinstance(x, torch.Tensor):
+        # the producer of `x` may have pooled these very bits for this halo; a second pooling makes a tensor of its own
+        y, slab, idx, halo, version = x.__dict__.pop("_sfh_pooled", None) or (None, None, None, -1, -1)
+        if halo != int(out_halo) or version != x._version:
+            y = slab = idx = None
+        done = _lib.native().max_pool(x, int(out_halo), with_skip, y, slab, idx)
     if done is None:
         _refuse(x)
     if done[1] is not None:

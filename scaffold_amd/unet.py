@@ -180,9 +180,20 @@ class UNet(nn.Module):
             self.up_list.append(Up(width, width // 2, g, stock=stock))
             width //= 2
         self.up_list.append(OutConv(width, n_classes, stock=stock))
+        self._announce_pooling()
+
+    def _announce_pooling(self):
+        """Tells an encoder block's last GroupNorm of the pooling that reads its output (not under checkpointing, where the two
+        run apart: a recomputed block would pool for nobody)."""
+        for i in range(self.layers):
+            enc, pool = self.down_list[i], self.down_list[i + 1].maxpool_conv[0]
+            norm = (enc if isinstance(enc, DoubleConv) else enc.maxpool_conv[1]).double_conv[4]
+            if isinstance(norm, FastGroupNorm) and isinstance(pool, FastMaxPool3d):
+                norm.pool_next = None if self.checkpointing else pool.out_halo
 
     def use_checkpointing(self):
         self.checkpointing = True
+        self._announce_pooling()
 
     def set_shard_halo(self, enabled: bool = True):
         """Run every 3x3x3 convolution in the depth-shard form (zero halo + depth padding 0)."""
@@ -212,6 +223,7 @@ class UNet(nn.Module):
             block = enc if isinstance(enc, DoubleConv) else enc.maxpool_conv[1]
             if isinstance(block.double_conv[4], FastGroupNorm):
                 block.double_conv[4].out_halo = halo
+        self._announce_pooling()
         return self
 
     def defer_weight_gradients(self, enabled: bool = True, early: bool = False):

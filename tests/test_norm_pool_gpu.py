@@ -1,0 +1,136 @@
+"""The normalisation that pools its result in the same pass, against the two launches: the same bits, values and gradients."""
+
+import pytest
+import torch
+
+import scaffold_amd as sa
+from scaffold_amd.modules import FastConv3d, FastGroupNorm, conv_then_norm
+from scaffold_amd.pooling import FastMaxPool3d
+from scaffold_amd.unet import UNet
+
+pytestmark = pytest.mark.gpu
+CL = torch.channels_last_3d
+
+
+def _pair(c, device, dtype, relu=True):
+    torch.manual_seed(1)
+    conv = FastConv3d(c, c, 3, padding=1, bias=False).to(device, dtype).to(memory_format=CL)
+    norm = FastGroupNorm(8, c, activation="relu" if relu else None).to(device, dtype)
+    with torch.no_grad():
+        norm.weight.add_(0.3 * torch.randn(c, device=device))
+        norm.bias.add_(0.3 * torch.randn(c, device=device))
+    conv.gn_groups = 8
+    return conv, norm
+
+
+@pytest.mark.parametrize("relu", [True, False])
+@pytest.mark.parametrize("halo", [0, 1])
+@pytest.mark.parametrize("n,c,spatial,dtype", [
+    (1, 32, (8, 16, 33), torch.bfloat16),      # four threads to a cell; a column of cells that are not pooled
+    (2, 64, (5, 7, 9), torch.bfloat16),        # odd on every axis, two samples
+    (1, 64, (16, 32, 64), torch.float16),      # several passes a workgroup
+    (1, 128, (2, 2, 2), torch.bfloat16),       # one cell
+    (1, 256, (4, 9, 20), torch.bfloat16),
+    (1, 512, (3, 8, 8), torch.bfloat16),       # 64 threads to a cell
+])
+def test_same_bits_as_two_launches(device, n, c, spatial, dtype, halo, relu):
+    conv, norm = _pair(c, device, dtype, relu)
+    norm.out_halo = halo
+    pool = FastMaxPool3d(2)
+    pool.out_halo = halo
+    x0 = torch.randn(n, c, *spatial, device=device).to(dtype).contiguous(memory_format=CL)
+    gp = torch.randn(n, c, *(s // 2 for s in spatial), device=device).to(dtype).contiguous(memory_format=CL)
+    gs = torch.randn(n, c, *spatial, device=device).to(dtype).contiguous(memory_format=CL)
+    results = []
+    for fused in (False, True):
+        norm.pool_next = halo if fused else None
+        x = x0.clone().requires_grad_(True)
+        torch.full((4 * x0.numel(),), float("nan"), device=device, dtype=dtype)
+        y = conv_then_norm(conv, norm, x)
+        # (a halo asks for one sample, and records come only from the kernels that offer them)
+        assert hasattr(y, "_sfh_pooled") == (fused and not (halo and n > 1) and bool(y is not None and _records(conv, x0)))
+        pooled, skip = pool.with_skip(y)
+        assert not hasattr(y, "_sfh_pooled")
+        slabs = [t._sfh_slab[0].clone() for t in (pooled, skip) if halo and n == 1]
+        grads = torch.autograd.grad((pooled, skip), (x, conv.weight, norm.weight, norm.bias), (gp, gs))
+        with torch.no_grad():
+            again = pool(conv_then_norm(conv, norm, x0))
+        assert torch.equal(again, pooled)
+        results.append([pooled.detach(), skip.detach(), *slabs, *grads])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+def _records(conv, x):
+    return getattr(conv(x), "_sfh_gn_partials", None) is not None
+
+
+def test_what_is_not_reused(device):
+    conv, norm = _pair(64, device, torch.bfloat16)
+    pool, wide = FastMaxPool3d(2), FastMaxPool3d(2)
+    wide.out_halo = 1
+    x = torch.randn(1, 64, 8, 16, 16, device=device).to(torch.bfloat16).contiguous(memory_format=CL)
+    norm.pool_next = 0
+    with torch.no_grad():
+        want = torch.nn.functional.max_pool3d(conv_then_norm(conv, norm, x).float(), 2)
+        y = conv_then_norm(conv, norm, x)
+        assert torch.equal(wide(y).float(), want) and hasattr(wide(y), "_sfh_slab")  # another halo
+        y = conv_then_norm(conv, norm, x)
+        a, b = pool(y), pool(y)                                                      # a second pooling has its own tensor
+        assert a.data_ptr() != b.data_ptr() and torch.equal(a.float(), want) and torch.equal(b.float(), want)
+        y = conv_then_norm(conv, norm, x).add_(1.0)                                  # written since
+        assert torch.equal(pool(y), torch.nn.functional.max_pool3d(y.float(), 2).to(y.dtype))
+    y = conv_then_norm(conv, norm, x.requires_grad_(True)).detach().requires_grad_(True)
+    (g,) = torch.autograd.grad(pool(y).float().sum(), y)
+    assert int((g != 0).sum()) == want.numel()
+    with torch.no_grad():
+        y = conv_then_norm(conv, norm, x)
+    y.requires_grad_(True)  # pooled without indices, and a gradient wanted after all
+    (h,) = torch.autograd.grad(pool(y).float().sum(), y)
+    assert torch.equal(g, h)
+    with torch.inference_mode():
+        y = conv_then_norm(conv, norm, x.detach())
+        assert not hasattr(y, "_sfh_pooled") and torch.equal(pool(y).float(), want)
+
+
+def test_nan_and_infinity(device):
+    conv, norm = _pair(32, device, torch.bfloat16)
+    x = torch.randn(1, 32, 4, 8, 34, device=device).to(torch.bfloat16)
+    x[0, 3, 1, 2, 3] = float("nan")
+    x[0, 3, 1, 5, 20] = float("inf")
+    x = x.contiguous(memory_format=CL)
+    outs = []
+    for pool_next in (None, 0):
+        norm.pool_next = pool_next
+        with torch.no_grad():
+            y = conv_then_norm(conv, norm, x)
+            outs.append((y.clone(), FastMaxPool3d(2)(y)))
+    for a, b in zip(*outs):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num())
+
+
+@pytest.mark.parametrize("shard,size", [(False, (14, 25, 31)), (True, (16, 32, 64))])
+def test_a_step_keeps_its_bits(device, shard, size):
+    torch.manual_seed(5)
+    net = UNet(3, 5, layers=2, base_width=32).to(device).to(memory_format=CL).set_shard_halo(shard)
+    x = torch.randn(1, 3, *size, device=device).contiguous(memory_format=CL)
+    target = torch.randint(0, 5, (1, *size), device=device)
+
+    def step():
+        net.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            logits = net(x)
+            with torch.no_grad():
+                quiet = net(x)
+        loss = sa.ce_dice_loss(logits, target)
+        loss.backward()
+        assert torch.equal(logits, quiet)
+        return [loss.detach(), logits.detach()] + [p.grad.clone() for p in net.parameters()]
+
+    norms = [m for m in net.modules() if isinstance(m, FastGroupNorm) and m.pool_next is not None]
+    assert len(norms) == 2 and all(m.pool_next == int(shard) for m in norms)
+    got = step()
+    for m in norms:
+        m.pool_next = None
+    assert all(torch.equal(a, b) for a, b in zip(step(), got))
+    net.use_checkpointing()
+    assert all(m.pool_next is None for m in net.modules() if isinstance(m, FastGroupNorm))
