@@ -134,9 +134,12 @@ class Up(nn.Module):
 
     def forward(self, x1, x2):
         # an odd level: the upsampled tensor is written with its padding where the module does that by itself
-        padded = self.up.padded_to(x1, x2.shape[2:]) if isinstance(self.up, FastConvTranspose3d) else None
+        _, _, d, h, w = x1.shape
+        wanted = x2.shape[2:]
+        odd = wanted != (2 * d, 2 * h, 2 * w)
+        padded = self.up.padded_to(x1, wanted) if odd and isinstance(self.up, FastConvTranspose3d) else None
         x1 = self.up(x1) if padded is None else padded
-        dz, dy, dx = (x2.size(i) - x1.size(i) for i in (2, 3, 4))
+        dz, dy, dx = (a - b for a, b in zip(wanted, x1.shape[2:]))
         if dx or dy or dz:
             x1 = F.pad(x1, [dx // 2, dx - dx // 2, dy // 2, dy - dy // 2, dz // 2, dz - dz // 2])
         first = self.conv.double_conv[0]
