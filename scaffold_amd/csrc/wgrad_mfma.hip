@@ -165,7 +165,9 @@ __device__ __forceinline__ void wave_compute(const char* lds, int lane, int wave
 }
 
 // The same for one kd: wavefronts 0 .. 2 take the three kw taps of brick row offset kh = wavefront, the fourth only meets the
-// barriers.  Three MFMAs a k-step do not cover a trip to LDS, so fragments are requested two k-steps ahead.
+// barriers.  Three MFMAs a k-step do not cover a trip to LDS, so fragments are requested two k-steps ahead.  Eight k-steps are
+// summed from zero and then added: in one chain through the matrix unit a block's error against 64 bits was 1.5 to 2 times that of
+// the columns (32 -> 32 at 48x64x64 3.2e-7, so 1.3e-7, columns 1.5e-7).
 template <typename T, typename C>
 __device__ __forceinline__ void wave_compute_plane(const char* lds, int lane, int kh, f32x16_t (&acc)[3]) {
   const int i = lane & 31, kg = lane >> 5;
@@ -182,16 +184,28 @@ __device__ __forceinline__ void wave_compute_plane(const char* lds, int lane, in
   };
 #pragma unroll
   for (int ks = 0; ks < LEAD; ++ks) load(ks);
+  constexpr int CHAIN = 8;
+  static_assert(C::NKS % CHAIN == 0, "whole chains");
+  f32x16_t sum[3], none;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) none[r] = 0.f;
 #pragma unroll
   for (int ks = 0; ks < C::NKS; ++ks) {
     const int b = ks % (LEAD + 1);
+    const bool first = ks % CHAIN == 0;
     __builtin_amdgcn_sched_barrier(0);
-    acc[0] = Mma32<T>::run(af[b], lo[b], acc[0]);
+    sum[0] = Mma32<T>::run(af[b], lo[b], first ? none : sum[0]);
     __builtin_amdgcn_sched_barrier(0);
     if (ks + LEAD < C::NKS) load(ks + LEAD);
     __builtin_amdgcn_sched_barrier(0);
-    acc[1] = Mma32<T>::run(af[b], shift_one(lo[b], nx[b]), acc[1]);
-    acc[2] = Mma32<T>::run(af[b], make_uint4(lo[b].y, lo[b].z, lo[b].w, nx[b]), acc[2]);
+    sum[1] = Mma32<T>::run(af[b], shift_one(lo[b], nx[b]), first ? none : sum[1]);
+    sum[2] = Mma32<T>::run(af[b], make_uint4(lo[b].y, lo[b].z, lo[b].w, nx[b]), first ? none : sum[2]);
+    if (ks % CHAIN == CHAIN - 1) {
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[t][r] += sum[t][r];
+    }
   }
   __builtin_amdgcn_sched_barrier(0);
 }
@@ -608,21 +622,39 @@ struct Plan {
   int nblk_ci, nblk;
   int splits, tiles_per_split;
   bool planes;  // three workgroups to a block, one per kd
+  bool ring;    // columns instead of tiles
 };
 
-// Rows of more than 16 voxels take the column-walking kernel.
+// Rows of more than 16 voxels: the column-walking kernel where it serves them.
 bool ring_serves(const WgradArgs& a) { return mfma_wgrad_ring_applies(a); }
+
+// Whether a launch of its own walks columns (rows in pieces of 32 voxels, 20 us before and behind its steps, 25 where rows are cut) or
+// 4x8x8 tiles in planes (less work on padding, a sooner start, a lower rate; where the blocks leave room for three workgroups each).
+// Times with the sum, of padded operations: 20 or 25 us + 0.7 a GFLOP and 12.5 us + 1.25, fitted to 35 problems of 32 to 512 channels
+// on 16x16x32 to 128^3. Columns -> tiles, us: 32 -> 32 channels at 32^3 21.7 -> 14.5, 64 -> 64 at 32^3 30.4 -> 24.1, at 16x32x32 28.1 -> 17.0, at 41x80x34
+// 61 -> 52, at 24x40x28 29.1 -> 21.1, 32 -> 32 at 36x63x66 33.1 -> 24.9, at 32x69x20 24.7 -> 16.2, two samples of 64 -> 128 at 20x33x19 41.8 -> 34.1, of
+// 32 -> 32 at 44x60x75 49.1 -> 42.3; level where the line lies (32 -> 32 at 64^3 30.5 / 31.6), columns past it: 96x80x112 65 / 72, 64^3 of 64
+// channels 62 / 80. Relative error against 64 bits, e-7: 32 -> 32 at 32^3 1.16 -> 1.13, at 48x64x64 1.54 -> 1.37, 128 -> 128 at 9x20x20 0.96 -> 0.94.
+bool walks_columns(const WgradArgs& a) {
+  if (!ring_serves(a)) return false;
+  if (3 * (int64_t)(a.cin / 32) * (a.cout / 32) > kTargetWorkgroups) return true;
+  const double per_voxel = 54e-9 * a.cin * a.cout * a.n;
+  const double columns = per_voxel * (double)cdiv(a.od, 2) * 2 * (double)cdiv(a.oh, 4) * 4 * (double)cdiv(a.ow, 32) * 32;
+  const double tiles = per_voxel * (double)cdiv(a.od, 4) * 4 * (double)cdiv(a.oh, 8) * 8 * (double)cdiv(a.ow, 8) * 8;
+  return (a.ow % 32 == 0 ? 20. : 25.) + 0.7 * columns <= 12.5 + 1.25 * tiles;
+}
 
 Plan make_plan(const WgradArgs& a) {
   Plan p{};
-  if (ring_serves(a)) {
+  p.ring = walks_columns(a);
+  if (p.ring) {
     p.tw = 32;
     p.splits = mfma_wgrad_ring_splits(a);
     return p;
   }
   int td, th;
-  if (a.ow > 16) { p.tw = 32; td = 2; th = 4; }
-  else if (a.ow > 8) { p.tw = 16; td = 2; th = 8; }
+  if (a.ow > 16 && !ring_serves(a)) { p.tw = 32; td = 2; th = 4; }
+  else if (a.ow > 8 && a.ow <= 16) { p.tw = 16; td = 2; th = 8; }
   else { p.tw = 8; td = 4; th = 8; }
   p.tiles_d = (int)cdiv(a.od, td);
   p.tiles_h = (int)cdiv(a.oh, th);
@@ -640,7 +672,7 @@ Plan make_plan(const WgradArgs& a) {
   // bits, one workgroup to a block and a sum pass / three, stored in place where one slice is left): 256 -> 256 channels on
   // 8 x 16 x 16 32.9 / 19.6, on 8 x 8 x 8 18.3 / 9.0, 128 -> 128 on 16 x 16 x 16 21.8 / 17.7 (four slices).
   int64_t best = -1;
-  for (int units = 1; units <= 3; units += 2) {
+  for (int units = ring_serves(a) ? 3 : 1; units <= 3; units += 2) {  // (tiles in the place of columns: in planes, walks_columns)
     if (units == 3 && (p.tw == 32 || units * p.nblk > kTargetWorkgroups)) break;
     const int64_t tile = units == 3 ? 130 : 240;
     int want = kTargetWorkgroups / (p.nblk * units);
@@ -678,7 +710,7 @@ int launch_typed(const WgradArgs& a, const void* x, const void* gy, void* gw, in
                  const ChannelPair& x2) {
   constexpr int kOwn = std::is_same<T, bf16_t>::value ? SFH_BF16 : SFH_FP16;
   const Plan p = make_plan(a);
-  const bool ring = ring_serves(a);
+  const bool ring = p.ring;
   // One slice: what the kernel stores IS the gradient (rounded on the way if it is a 16-bit one), so it is written in place
   // and no sum pass follows.
   const bool direct = p.splits == 1 && (gw_dtype == SFH_FP32 || (gw_dtype == kOwn && !ring));

@@ -70,3 +70,22 @@ def test_blocks_cut_into_parts(n, cin, cout, spatial, padding, grad_dtype):
         orc.assert_close(g.to(torch.bfloat16), orc.conv_reference(prob, ops, "bwd-weight"), prob, "bwd-weight")
     alone = sa.conv3d_backward_weight_batch(items[:1], grad_dtype=grad_dtype)
     assert torch.equal(alone[0], got[0])
+
+
+@pytest.mark.parametrize("case", [
+    (1, 32, 32, (16, 16, 32), 1, torch.bfloat16),            # full rows of a small volume
+    (1, 64, 32, (5, 7, 17), 1, torch.float16),               # rows a voxel past the small-volume kernel's
+    (2, 32, 64, (9, 13, 37), (0, 1, 2), torch.bfloat16),     # cut rows over two samples
+    (1, 96, 64, (3, 33, 20), 1, torch.bfloat16),
+    (1, 288, 320, (2, 4, 18), 1, torch.bfloat16),            # 90 blocks: no room for three workgroups each
+])
+def test_wide_rows_in_tiles(case):
+    """Problems with rows of more than 16 voxels that a launch of their own takes in tiles; a list still walks their columns."""
+    test_alone(case)
+    prob, ops = _problem(*case, seed=3)
+    padding = (case[4],) * 3 if isinstance(case[4], int) else case[4]
+    x, gy = ops["input"].cuda(), ops["grad_output"].cuda()
+    alone = sa.conv3d_backward_weight(x, prob.weight_shape, gy, 1, padding, grad_dtype=torch.float32)
+    (listed,) = sa.conv3d_backward_weight_batch([(x, prob.weight_shape, gy, padding)], grad_dtype=torch.float32)
+    # two orders of the same fp32 sums: each within 2e-7 of 64 bits (relative, in the norm)
+    assert (alone - listed).norm() <= 4e-7 * listed.norm()
