@@ -23,21 +23,19 @@ __device__ __forceinline__ float wave_sum_all(float v) {
   return v;  // lane 0 holds the sum
 }
 
-// The same total, pair by pair, in lane 63 and on the vector pipe alone: halves and rows of 16 lanes traded, then shifts of 8, 4, 2 and 1
-// within the rows. The 3 C + 2 totals of a workgroup made 228 trips through the LDS pipe as shuffles.
-template <int CTRL>
+// The same total in lane 63, on the vector pipe alone: rows of 16 lanes by shifts of 1, 2, 4 and 8, then rows 0 and 2 into
+// rows 1 and 3 and row 1 into rows 2 and 3. The 3 C + 2 totals of a workgroup made 228 trips through the LDS pipe as shuffles.
+template <int CTRL, int ROWS>
 __device__ __forceinline__ float dpp_add(float v) {
-  return v + __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
+  return v + __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, ROWS, 0xf, true));
 }
 __device__ __forceinline__ float wave_sum_last(float v) {
-  const auto half = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = __uint_as_float(half[0]) + __uint_as_float(half[1]);
-  const auto row = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = __uint_as_float(row[0]) + __uint_as_float(row[1]);
-  v = dpp_add<0x118>(v);
-  v = dpp_add<0x114>(v);
-  v = dpp_add<0x112>(v);
-  return dpp_add<0x111>(v);
+  v = dpp_add<0x111, 0xf>(v);
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);
+  return dpp_add<0x143, 0xc>(v);
 }
 
 // Voxels a thread works on between two barriers: as many as keep a tile's logits within 32 KiB of LDS, so that four
@@ -273,8 +271,8 @@ __global__ void __launch_bounds__(64) ce_dice_scalar(const float* __restrict__ s
 }
 
 // Both of the above as one workgroup, for up to kTotalSamples samples and kTotalSlotsMax slots. A wavefront reads a slot's
-// quantities side by side and takes every sixteenth slot, sixteen of them in flight; a sample's sums are those of ce_dice_sum, bit for
-// bit. What bounds it is a launch and the trips of one CU: 128 slots of 35 quantities 5.3 us (the two launches
+// quantities side by side and takes every sixteenth slot, sixteen of them in flight; sums of sixteen by a tree, the
+// wavefronts' by a tree. What bounds it is a launch and the trips of one CU: 128 slots of 35 quantities 5.3 us (the two launches
 // 9.3), 512 slots of 53 10.5 (level), 1024 of 35 17.8.
 constexpr int kTotal = 1024, kTotalWaves = kTotal / 64, kTotalSamples = 4, kTotalQ = 3 * 32 + 2, kTotalSlots = 16, kTotalSlotsMax = 256;
 __global__ void __launch_bounds__(kTotal) ce_dice_total(const float* __restrict__ part, float* __restrict__ stats, float* __restrict__ loss,
@@ -297,11 +295,11 @@ __global__ void __launch_bounds__(kTotal) ce_dice_total(const float* __restrict_
         }
 #pragma unroll
         for (int k = 0; k < kTotalSlots; ++k) v[k] = sp + k * kTotalWaves < nsplit ? v[k] : 0.f;
-        // slots 64 apart one after the other, then those 32 and 16 apart: the order of ce_dice_sum's lanes and of its tree
-        float lane_sum[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) lane_sum[j] = ((v[j] + v[4 + j]) + v[8 + j]) + v[12 + j];
-        s += (lane_sum[0] + lane_sum[2]) + (lane_sum[1] + lane_sum[3]);
+        for (int h = kTotalSlots / 2; h > 0; h >>= 1)
+#pragma unroll
+          for (int k = 0; k < h; ++k) v[k] += v[k + h];
+        s += v[0];
       }
       wave_tot[wave][q] = s;
     }
