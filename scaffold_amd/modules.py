@@ -425,9 +425,12 @@ def _plain_call(module) -> bool:
                 or "forward" in module.__dict__ or module._compiled_call_impl is not None)
 
 
-def conv_then_norm(conv, norm, x):
+def conv_then_norm(conv, norm, x, pools=True):
     """``norm(conv(x))`` as one call into the host path and one autograd node, or ``None`` where the two modules have to run
-    by themselves (a bias, hooks on either or a ``forward`` of its own, a subclass, an input that is not channels-last, ...)."""
+    by themselves (a bias, hooks on either or a ``forward`` of its own, a subclass, an input that is not channels-last, ...).
+
+    ``pools``: where ``norm.pool_next`` announces a pooling, the result also carries what that pooling would compute, as
+    ``result._sfh_pooled``, for a caller that hands it to ``FastMaxPool3d.with_skip`` before anything else sees the result."""
     if type(conv) is not FastConv3d or type(norm) is not FastGroupNorm or conv.groups != 1 or torch.compiler.is_compiling() \
             or conv.padding_mode != "zeros" or isinstance(conv.padding, str) or not _plain_call(conv) or not _plain_call(norm) \
             or torch.nn.modules.module._has_any_global_hook() or _lib.under_transform() or not isinstance(x, torch.Tensor) or x.dim() != 5:
@@ -458,8 +461,7 @@ def conv_then_norm(conv, norm, x):
         family = _deferrable(weight, in_shape, weight.shape, stride, padding, dilation, x_read.dtype)
         _set_early_callbacks()
     pf, pd = (None, None) if packs is None else packs
-    # (a tensor made in inference mode has no version to tell a later write by)
-    pool_halo = -1 if norm.pool_next is None or torch.is_inference_mode_enabled() else norm.pool_next
+    pool_halo = norm.pool_next if pools and norm.pool_next is not None and not torch.is_inference_mode_enabled() else -1
     done = _lib.native().conv_norm(x, x_read, receives, w, pf, pd, halo, stride, padding, dilation, master, family, defer == 2, norm.num_groups,
                                    gamma, beta, norm.eps, norm.activation == "relu", norm.out_halo, pool_halo)
     if done is None:
@@ -468,7 +470,7 @@ def conv_then_norm(conv, norm, x):
     if slab is not None:
         y._sfh_slab = (slab, norm.out_halo)
     if pooled is not None:
-        y._sfh_pooled = (*pooled, pool_halo, y._version)
+        y._sfh_pooled = (*pooled, pool_halo)
     return y
 
 
@@ -552,7 +554,7 @@ class FastGroupNorm(nn.GroupNorm):
 
     activation = None  # class-level default: not a parameter, buffer or state-dict key
     #: the halo of a ``FastMaxPool3d`` that reads this module's output next (None: none does): where the convolution in front runs
-    #: with this module in one call, that call also leaves what the pooling will ask for on its result
+    #: with this module in one call, that call can make the pooled tensor too (:func:`conv_then_norm`)
     pool_next = None
     #: depth planes of zero halo to leave around the output for a following ``FastConv3d.shard_halo`` (0: none)
     out_halo = 0

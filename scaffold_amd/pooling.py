@@ -31,13 +31,16 @@ def _refuse(x):
     raise NotImplementedError(f"unsupported: x={tuple(getattr(x, 'shape', ()))}/{getattr(x, 'dtype', None)}")
 
 
-def _pool(x, out_halo, with_skip):
-    """The launch and its autograd node: ``(pooled, ...)``; the pooled tensor carries the slab it lies in, if any."""
+def _pool(x, out_halo, with_skip, given=None):
+    """The launch and its autograd node: ``(pooled, ...)``; the pooled tensor carries the slab it lies in, if any.  ``given``:
+    what the launch that made ``x`` has pooled already, ``(pooled, slab, indices, halo)``, which is then taken in the launch's place."""
     done = None
     if isinstance(x, torch.Tensor):
-        # the producer of `x` may have pooled these very bits for this halo; a second pooling makes a tensor of its own
-        y, slab, idx, halo, version = x.__dict__.pop("_sfh_pooled", None) or (None, None, None, -1, -1)
-        if halo != int(out_halo) or version != x._version:
+        # What a producer left on its result is never taken from there: by now the result may have been written past its version
+        # counter, and the pooled tensor belongs to the stream and the capture it was made in.
+        x.__dict__.pop("_sfh_pooled", None)
+        y, slab, idx, halo = given or (None, None, None, -1)
+        if halo != int(out_halo):
             y = slab = idx = None
         done = _lib.native().max_pool(x, int(out_halo), with_skip, y, slab, idx)
     if done is None:
@@ -47,14 +50,14 @@ def _pool(x, out_halo, with_skip):
     return done
 
 
-def max_pool3d_2x_with_skip(x: torch.Tensor, out_halo: int = 0):
+def max_pool3d_2x_with_skip(x: torch.Tensor, out_halo: int = 0, _given=None):
     """``(F.max_pool3d(x, 2), x)``: use the returned ``x`` for the skip connection and the gradients of both uses are
     combined in one kernel (same values as autograd's own addition: one fp32 sum, one rounding)."""
     if not is_supported_pool(x):
         _refuse(x)
     if not x.is_contiguous(memory_format=_CL3D) or _lib.under_transform():
         return max_pool3d_2x(x, out_halo), x
-    pooled, _, skip = _pool(x, out_halo, True)
+    pooled, _, skip = _pool(x, out_halo, True, _given)
     slab = getattr(x, "_sfh_slab", None)
     if slab is not None:  # the alias is the same memory: still the interior of the slab its producer wrote it into
         skip._sfh_slab = slab
@@ -92,12 +95,13 @@ class FastMaxPool3d(nn.MaxPool3d):
         """Whether :meth:`with_skip` applies to this module and tensor."""
         return self._is_pool2() and is_supported_pool(input) and input.is_contiguous(memory_format=_CL3D)
 
-    def with_skip(self, input):
+    def with_skip(self, input, given=None):
         """``(self(input), input)`` for an input that is also used elsewhere (the U-Net's skip connection): use the
-        returned pair and the two gradients of ``input`` are summed inside the pooling-gradient kernel."""
+        returned pair and the two gradients of ``input`` are summed inside the pooling-gradient kernel.  ``given``: the
+        ``_sfh_pooled`` of an input that nothing but the caller has seen since ``modules.conv_then_norm`` made it on this stream."""
         if not self._is_pool2():
             raise NotImplementedError("FastMaxPool3d.with_skip supports MaxPool3d(2) only")
-        return max_pool3d_2x_with_skip(input, self.out_halo)
+        return max_pool3d_2x_with_skip(input, self.out_halo, given)
 
     def forward(self, input):
         if not self._is_pool2():

@@ -21,7 +21,7 @@ import torch.nn.functional as F
 import torch.utils.checkpoint
 
 from . import concat as _cat
-from .modules import FastConv3d, FastConvTranspose3d, FastGroupNorm, autocast_dtype, conv_then_norm
+from .modules import FastConv3d, FastConvTranspose3d, FastGroupNorm, _plain_call, autocast_dtype, conv_then_norm
 from .pooling import FastMaxPool3d
 
 __all__ = ["UNet", "DoubleConv", "Down", "Up", "OutConv", "skip_concat"]
@@ -101,14 +101,14 @@ class DoubleConv(nn.Module):
         for c, g in self._pairs:
             self.double_conv[c].gn_groups = self.double_conv[g].num_groups
 
-    def forward(self, x, second=None):
+    def forward(self, x, second=None, pools=False):
         """``second``: the input is ``torch.cat([x, second], 1)``, handed over as the two tensors (the first convolution
-        must have said ``takes_pair``)."""
+        must have said ``takes_pair``).  ``pools``: see ``modules.conv_then_norm``."""
         if not self._pairs:
             return self.double_conv(x if second is None else torch.cat([x, second], dim=1))
         for c, g in self._pairs:  # the Identity modules between the pairs only keep the reference's state-dict indices
             conv, norm = self.double_conv[c], self.double_conv[g]
-            y = conv_then_norm(conv, norm, x) if second is None else None
+            y = conv_then_norm(conv, norm, x, pools) if second is None else None
             x = y if y is not None else norm(conv(x) if second is None else conv(x, second))
             second = None
         return x
@@ -247,15 +247,31 @@ class UNet(nn.Module):
             return torch.utils.checkpoint.checkpoint(block, *inputs, use_reentrant=False)
         return block(*inputs)
 
+    def _encode(self, block, x):
+        """``block(x)``, and what its last normalisation has pooled for the level below: only where the block's call is this
+        class's code alone, so that nobody else has seen the tensor when the pooling takes it (no hook that may write to it or
+        change the stream)."""
+        if torch.compiler.is_compiling() or type(block) is not DoubleConv or not _plain_call(block) or torch.nn.modules.module._has_any_global_hook():
+            return block(x), None
+        y = block(x, pools=True)
+        return y, y.__dict__.pop("_sfh_pooled", None) if isinstance(y, torch.Tensor) else None
+
     def forward(self, x):
-        feats = [self._run(self.down_list[0], x)]
+        given = None
+        if self.checkpointing:
+            feats = [self._run(self.down_list[0], x)]
+        else:
+            x, given = self._encode(self.down_list[0], x)
+            feats = [x]
         for i in range(1, self.layers + 1):
             pool, block = self.down_list[i].maxpool_conv
             if isinstance(pool, FastMaxPool3d) and not self.checkpointing and pool.serves(feats[-1]):
                 # the tensor that is pooled is also the skip connection: both gradients meet in the pooling kernel
-                pooled, feats[-1] = pool.with_skip(feats[-1])
-                feats.append(block(pooled))
+                pooled, feats[-1] = pool.with_skip(feats[-1], given) if type(pool) is FastMaxPool3d else pool.with_skip(feats[-1])
+                x, given = self._encode(block, pooled)
+                feats.append(x)
             else:
+                given = None
                 feats.append(self._run(self.down_list[i], feats[-1]))
         feats.reverse()
         out = feats[0]

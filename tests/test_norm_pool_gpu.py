@@ -134,3 +134,128 @@ def test_a_step_keeps_its_bits(device, shard, size):
     assert all(torch.equal(a, b) for a, b in zip(step(), got))
     net.use_checkpointing()
     assert all(m.pool_next is None for m in net.modules() if isinstance(m, FastGroupNorm))
+
+
+def _captured(fn):
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side), torch.no_grad():
+        fn()  # what a first call packs is not part of a capture
+    torch.cuda.current_stream().wait_stream(side)
+    with torch.cuda.graph(graph), torch.no_grad():
+        out = fn()
+    return graph, out
+
+
+def _pooled(y):
+    return torch.nn.functional.max_pool3d(y.float(), 2).to(y.dtype)
+
+
+@pytest.mark.parametrize("halo", [0, 1])
+@pytest.mark.parametrize("n,c,spatial", [(1, 32, (8, 16, 33)), (1, 64, (5, 7, 9)), (1, 128, (2, 2, 2)), (1, 512, (3, 8, 8))])
+def test_handed_over_is_the_launched_one(device, n, c, spatial, halo):
+    """What the normalisation pooled, taken by the pooling: values, slab and (through the gradients) indices of its own launch."""
+    conv, norm = _pair(c, device, torch.bfloat16)
+    norm.out_halo = norm.pool_next = halo
+    pool = FastMaxPool3d(2)
+    pool.out_halo = halo
+    x0 = torch.randn(n, c, *spatial, device=device).to(torch.bfloat16).contiguous(memory_format=CL)
+    gp, gs = (torch.randn(n, c, *s, device=device).to(torch.bfloat16).contiguous(memory_format=CL) for s in ([v // 2 for v in spatial], spatial))
+    results = []
+    for take in (True, False):
+        x = x0.clone().requires_grad_(True)
+        y = conv_then_norm(conv, norm, x)
+        given = y.__dict__.pop("_sfh_pooled")
+        pooled, skip = pool.with_skip(y, given if take else None)
+        assert (pooled.data_ptr() == given[0].data_ptr()) == take
+        slabs = [t._sfh_slab[0].clone() for t in (pooled, skip) if halo]
+        results.append([pooled.detach(), skip.detach(), *slabs, *torch.autograd.grad((pooled, skip), (x, conv.weight, norm.weight, norm.bias), (gp, gs))])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+def test_a_captured_pooling_reads_its_input(device):
+    conv, norm = _pair(64, device, torch.bfloat16)
+    norm.pool_next = 0
+    pool = FastMaxPool3d(2)
+    x = torch.randn(1, 64, 8, 16, 16, device=device).to(torch.bfloat16).contiguous(memory_format=CL)
+    with torch.no_grad():
+        y = conv_then_norm(conv, norm, x)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph), torch.no_grad():
+        p = pool(y)
+    for seed in range(3):
+        torch.manual_seed(seed)
+        with torch.no_grad():
+            y.copy_(torch.randn_like(y))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(p, _pooled(y))
+
+
+def test_what_was_pooled_from_a_static_output_is_kept(device):
+    conv, norm = _pair(64, device, torch.bfloat16)
+    norm.pool_next = 0
+    x = torch.randn(1, 64, 8, 16, 16, device=device).to(torch.bfloat16).contiguous(memory_format=CL)
+    graph, y = _captured(lambda: conv_then_norm(conv, norm, x))
+    graph.replay()
+    with torch.no_grad():
+        p = FastMaxPool3d(2)(y)
+    want = _pooled(y)
+    for _ in range(2):
+        x.copy_(torch.randn_like(x))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(p, want) and not torch.equal(_pooled(y), want)
+
+
+def test_on_a_stream_of_its_own_and_after_a_write_nobody_counts(device):
+    conv, norm = _pair(64, device, torch.bfloat16)
+    norm.pool_next = 0
+    pool = FastMaxPool3d(2)
+    x = torch.randn(1, 64, 8, 16, 16, device=device).to(torch.bfloat16).contiguous(memory_format=CL)
+    side = torch.cuda.Stream()
+    with torch.no_grad():
+        y = conv_then_norm(conv, norm, x)
+        left = y._sfh_pooled[0]
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            y.record_stream(side)
+            p = pool(y)
+        torch.cuda.current_stream().wait_stream(side)
+        assert p.data_ptr() != left.data_ptr() and torch.equal(p, left)  # memory of the stream it was asked for on
+        y = conv_then_norm(conv, norm, x)
+        y.data.neg_()
+        assert torch.equal(pool(y), _pooled(y))
+
+
+def test_a_network_takes_it_and_its_hooks_are_seen(device, monkeypatch):
+    torch.manual_seed(5)
+    net = UNet(3, 5, layers=2, base_width=32).to(device).to(memory_format=CL)
+    x = torch.randn(1, 3, 16, 32, 32, device=device).contiguous(memory_format=CL)
+    taken = []
+    with_skip = FastMaxPool3d.with_skip
+    monkeypatch.setattr(FastMaxPool3d, "with_skip", lambda self, y, given=None: taken.append(given is not None) or with_skip(self, y, given))
+
+    def forward():
+        taken.clear()
+        with torch.autocast("cuda", dtype=torch.bfloat16), torch.no_grad():
+            return net(x), list(taken)
+
+    assert forward()[1] == [True, True]
+    enc = net.down_list[0]
+
+    def negate(module, args, out):
+        out.data.neg_()
+
+    handle = enc.register_forward_hook(negate)
+    hooked, taken_then = forward()
+    assert taken_then == [False, True]
+    for m in net.modules():
+        if isinstance(m, FastGroupNorm):
+            m.pool_next = None
+    assert torch.equal(hooked, forward()[0])
+    handle.remove()
+    assert not torch.equal(hooked, forward()[0])
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not hasattr(enc(x), "_sfh_pooled")  # a block by itself pools for nobody
