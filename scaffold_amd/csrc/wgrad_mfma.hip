@@ -167,7 +167,8 @@ __device__ __forceinline__ void wave_compute(const char* lds, int lane, int wave
 // The same for one kd: wavefronts 0 .. 2 take the three kw taps of brick row offset kh = wavefront, the fourth only meets the
 // barriers.  Three MFMAs a k-step do not cover a trip to LDS, so fragments are requested two k-steps ahead.  Eight k-steps are
 // summed from zero and then added: in one chain through the matrix unit a block's error against 64 bits was 1.5 to 2 times that of
-// the columns (32 -> 32 at 48x64x64 3.2e-7, so 1.3e-7, columns 1.5e-7).
+// the columns (32 -> 32 at 48x64x64 3.2e-7, so 1.3e-7, columns 1.5e-7).  (The form of all 27 taps above keeps one chain: its seven sums
+// from zero do not fit beside seven accumulators, and two passes over a tile's rows took lists of it from 62 to 82 us, 314 to 400.)
 template <typename T, typename C>
 __device__ __forceinline__ void wave_compute_plane(const char* lds, int lane, int kh, f32x16_t (&acc)[3]) {
   const int i = lane & 31, kg = lane >> 5;
@@ -760,7 +761,8 @@ int64_t busiest(const WTileBatch& b, int units) {
 // it is in a U-Net has 18 blocks: 54 units of 30 tiles' cost each kept 202 workgroups waiting. Where a gradient has up to 64 output
 // channels and more than eight tiles under a block, parts of about six tiles: slices (108 KB a block and part) and a sum pass (5 us) in
 // exchange. Levels of 128 channels and more have blocks enough: cut as well, the lists of 48^3 (width 64) and 125x34x37 (width 32) went
-// from 75 and 45 us to 89 and 53. A function of the problem alone: its bits do not depend on what else is in a list. Lists of the deep
+// from 75 and 45 us to 89 and 53. A function of the problem alone: what else is in a list decides only
+// whether three workgroups share a block (tile_batch_plan), and with that in which chains a tile's k-steps are summed. Lists of the deep
 // levels of a step, us: 56x27x27 47.7 -> 30.4, 32^3 30.2 -> 22.1; 43x124x47, all of 128 channels and more, 54.
 int unit_parts(int ntiles, int cout) { return ntiles <= 8 || cout > 64 ? 1 : (int)cdiv(ntiles, 6); }
 

@@ -36,12 +36,14 @@ def test_alone(case):
 
 
 @pytest.mark.parametrize("grad_dtype", [None, torch.float32])
-@pytest.mark.parametrize("extra", [0, 1])
+@pytest.mark.parametrize("extra", [0, 1, 2])
 def test_in_a_list(grad_dtype, extra):
-    # extra: a problem of 64 blocks more, which takes the list past one round of shared blocks; the bits do not change
+    # extra: a problem of 64 blocks more, with which three workgroups still share a block: the bits do not change. Or one of 272, with
+    # which a workgroup takes whole blocks and sums a tile in one chain: another order of the same fp32 sums
     cases = [(1, 32, 32, (12, 10, 8), (0, 1, 2), torch.bfloat16), (1, 64, 64, (4, 8, 8), 1, torch.bfloat16), (1, 64, 32, (5, 7, 9), 1, torch.bfloat16),
              (1, 64, 64, (16, 16, 16), 1, torch.bfloat16)]
-    problems = [_problem(*c, seed=5 + i) for i, c in enumerate(cases + [(1, 256, 256, (4, 8, 8), 1, torch.bfloat16)] * extra)]
+    more = [(1, 256, 256, (4, 8, 8), 1, torch.bfloat16)] if extra == 1 else [(1, 512, 544, (2, 4, 8), 1, torch.bfloat16)] if extra else []
+    problems = [_problem(*c, seed=5 + i) for i, c in enumerate(cases + more)]
     items = [(o["input"].cuda(), p.weight_shape, o["grad_output"].cuda(), c) for (p, o), c in
              zip(problems, [(0, 1, 2), (1, 1, 1), (1, 1, 1), (1, 1, 1), (1, 1, 1)])]
     got = sa.conv3d_backward_weight_batch(items, grad_dtype=grad_dtype)
@@ -49,7 +51,14 @@ def test_in_a_list(grad_dtype, extra):
         orc.assert_close(g.to(torch.bfloat16), orc.conv_reference(prob, ops, "bwd-weight"), prob, "bwd-weight")
     if extra:
         short = sa.conv3d_backward_weight_batch(items[:4], grad_dtype=grad_dtype)
-        assert all(torch.equal(a, b) for a, b in zip(short, got))
+        assert all(torch.equal(a, b) for a, b in zip(short, got)) == (extra == 1)
+        assert grad_dtype is None or all(_close_in_fp32(a, b) for a, b in zip(short, got))
+
+
+def _close_in_fp32(a, b):
+    # two orders of the same sums of up to 4096 products, each within 4e-7 of 64 bits (relative, in the norm; one chain measured at
+    # 3.2e-7 over 200000)
+    return bool((a - b).norm() <= 8e-7 * b.norm())
 
 
 @pytest.mark.parametrize("grad_dtype", [None, torch.float32])
@@ -61,7 +70,8 @@ def test_in_a_list(grad_dtype, extra):
     (1, 64, 128, (28, 13, 13), 1),     # too many output channels: whole
 ])
 def test_blocks_cut_into_parts(n, cin, cout, spatial, padding, grad_dtype):
-    """The slices of a list's problems lie beside those of its large rows; alone or not, the bits of a problem are the same."""
+    """The slices of a list's problems lie beside those of its large rows; alone or in a list of few blocks, the bits of a problem are the
+    same."""
     cases = [(n, cin, cout, spatial, padding, torch.bfloat16), (1, 32, 32, (4, 5, 33), 1, torch.bfloat16), (1, 32, 64, (11, 16, 16), 1, torch.bfloat16)]
     problems = [_problem(*c, seed=9 + i) for i, c in enumerate(cases)]
     items = [(o["input"].cuda(), p.weight_shape, o["grad_output"].cuda(), p.padding) for p, o in problems]
@@ -70,6 +80,14 @@ def test_blocks_cut_into_parts(n, cin, cout, spatial, padding, grad_dtype):
         orc.assert_close(g.to(torch.bfloat16), orc.conv_reference(prob, ops, "bwd-weight"), prob, "bwd-weight")
     alone = sa.conv3d_backward_weight_batch(items[:1], grad_dtype=grad_dtype)
     assert torch.equal(alone[0], got[0])
+    # beside 272 blocks of another problem a workgroup takes whole blocks: the parts' slices of all 27 taps
+    wide, ops = _problem(1, 512, 544, (2, 4, 8), 1, torch.bfloat16, seed=12)
+    beside = sa.conv3d_backward_weight_batch(items + [(ops["input"].cuda(), wide.weight_shape, ops["grad_output"].cuda(), wide.padding)],
+                                             grad_dtype=grad_dtype)
+    for (prob, o), g, b in zip(problems, got, beside):
+        orc.assert_close(b.to(torch.bfloat16), orc.conv_reference(prob, o, "bwd-weight"), prob, "bwd-weight")
+        assert grad_dtype is None or _close_in_fp32(b, g)
+    orc.assert_close(beside[-1].to(torch.bfloat16), orc.conv_reference(wide, ops, "bwd-weight"), wide, "bwd-weight")
 
 
 @pytest.mark.parametrize("case", [
