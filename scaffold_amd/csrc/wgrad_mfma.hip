@@ -629,30 +629,34 @@ struct Plan {
 // Rows of more than 16 voxels: the column-walking kernel where it serves them.
 bool ring_serves(const WgradArgs& a) { return mfma_wgrad_ring_applies(a); }
 
-// Whether a launch of its own walks columns (rows in pieces of 32 voxels, 20 us before and behind its steps, 25 where rows are cut) or
-// 4x8x8 tiles in planes (less work on padding, a sooner start, a lower rate; where the blocks leave room for three workgroups each).
-// Times with the sum, of padded operations: 20 or 25 us + 0.7 a GFLOP and 12.5 us + 1.25, fitted to 35 problems of 32 to 512 channels
-// on 16x16x32 to 128^3. Columns -> tiles, us: 32 -> 32 channels at 32^3 21.7 -> 14.5, 64 -> 64 at 32^3 30.4 -> 24.1, at 16x32x32 28.1 -> 17.0, at 41x80x34
-// 61 -> 52, at 24x40x28 29.1 -> 21.1, 32 -> 32 at 36x63x66 33.1 -> 25.8, at 32x69x20 24.7 -> 16.3, two samples of 64 -> 128 at 20x33x19 41.8 -> 34.1, of
-// 32 -> 32 at 44x60x75 49.2 -> 43.7; level where the line lies (32 -> 32 at 64^3 30.5 / 31.6), columns past it: 96x80x112 65 / 72, 64^3 of 64
-// channels 62 / 80. Relative error against 64 bits, e-7: 32 -> 32 at 32^3 1.16 -> 1.13, at 48x64x64 1.54 -> 1.37, 128 -> 128 at 9x20x20 0.96 -> 0.94.
-bool walks_columns(const WgradArgs& a) {
-  if (!ring_serves(a)) return false;
-  if (3 * (int64_t)(a.cin / 32) * (a.cout / 32) > kTargetWorkgroups) return true;
+// Rows of more than 16 voxels in a launch of their own: columns (rows in pieces of 32 voxels, 20 us before and behind its steps, 25 where
+// rows are cut) or 4x8x8 tiles in planes (less work on padding, a sooner start, a lower rate; where the blocks leave room for three
+// workgroups each). Times with the sum, of padded operations: 20 or 25 us + 0.7 a GFLOP and 12.5 us + 1.25, fitted to 35 problems of 32 to
+// 512 channels on 16x16x32 to 128^3. Tiles where both that estimate and the plan's own cost are below the columns': the plan knows what the
+// workgroup with the most tiles has to do (128 -> 256 at 19x29x23: 30 tiles in two slices of 32 blocks, 57 us, columns 46; two samples of 256 -> 256 at
+// 22x7x36 98 and 71), the estimate the rate of long slices (64 -> 256 at 32x62x33 205 and 171). Of 98 odd shapes, half of them where the two disagree,
+// 90 take the faster form or one 3 % slower; the worst, two samples of 128 -> 64 at 16x4x64, takes columns, 27.6 and 22.5. Columns -> tiles, us: 32 -> 32 channels at 32^3 21.6 -> 14.4, 64 -> 64 at 32^3 30.4 -> 24.1, at 16x32x32
+// 28.1 -> 17.0, at 41x80x34 63 -> 54, at 24x40x28 29.1 -> 21.1, 32 -> 32 at 36x63x66 33.6 -> 25.7, at 32x69x20 24.7 -> 16.4, at 38x25x55 25.8 -> 18.0, two samples
+// at 22x43x53 30.5 -> 23.7, at 44x60x75 49.9 -> 45.3, of 64 -> 128 at 20x33x19 42.3 -> 34.8; level where the line lies (32 -> 32 at 64^3 30.5 / 31.6), columns
+// past it: 96x80x112 65 / 72, 64^3 of 64 channels 62 / 80. Relative error against 64 bits, e-7: 32 -> 32 at 32^3 1.16 -> 1.13, at 48x64x64 1.54 -> 1.37,
+// 128 -> 128 at 9x20x20 0.96 -> 0.94.
+bool walks_columns(const WgradArgs& a, int64_t tile_plan_cost) {
   const double per_voxel = 54e-9 * a.cin * a.cout * a.n;
-  const double columns = per_voxel * (double)cdiv(a.od, 2) * 2 * (double)cdiv(a.oh, 4) * 4 * (double)cdiv(a.ow, 32) * 32;
-  const double tiles = per_voxel * (double)cdiv(a.od, 4) * 4 * (double)cdiv(a.oh, 8) * 8 * (double)cdiv(a.ow, 8) * 8;
-  return (a.ow % 32 == 0 ? 20. : 25.) + 0.7 * columns <= 12.5 + 1.25 * tiles;
+  const double columns = (a.ow % 32 == 0 ? 20. : 25.) + 0.7 * per_voxel * (double)cdiv(a.od, 2) * 2 * (double)cdiv(a.oh, 4) * 4 * (double)cdiv(a.ow, 32) * 32;
+  const double tiles = 12.5 + 1.25 * per_voxel * (double)cdiv(a.od, 4) * 4 * (double)cdiv(a.oh, 8) * 8 * (double)cdiv(a.ow, 8) * 8;
+  return columns <= tiles || 100 * columns <= (double)tile_plan_cost;
 }
 
 Plan make_plan(const WgradArgs& a) {
   Plan p{};
-  p.ring = walks_columns(a);
-  if (p.ring) {
+  auto columns = [&] {
+    p.ring = true;
+    p.planes = false;
     p.tw = 32;
     p.splits = mfma_wgrad_ring_splits(a);
     return p;
-  }
+  };
+  if (ring_serves(a) && 3 * (int64_t)(a.cin / 32) * (a.cout / 32) > kTargetWorkgroups) return columns();
   int td, th;
   if (a.ow > 16 && !ring_serves(a)) { p.tw = 32; td = 2; th = 4; }
   else if (a.ow > 8 && a.ow <= 16) { p.tw = 16; td = 2; th = 8; }
@@ -672,9 +676,6 @@ Plan make_plan(const WgradArgs& a) {
   // the price of staging the gradient three times: worth it while the chip has room for them.  Measured (us, gradient in 16
   // bits, one workgroup to a block and a sum pass / three, stored in place where one slice is left): 256 -> 256 channels on
   // 8 x 16 x 16 32.9 / 19.6, on 8 x 8 x 8 18.3 / 9.0, 128 -> 128 on 16 x 16 x 16 21.8 / 17.7 (four slices).
-  // The number of slices a caller is told divides a wide volume's bricks of 2 x 4 x 32 whether columns or tiles serve it: the same
-  // share of them to every slice, none left without one.
-  const int64_t rows = ring_serves(a) ? a.n * (int64_t)cdiv(a.od, 2) * cdiv(a.oh, 4) * cdiv(a.ow, 32) : 0;
   int64_t best = -1;
   for (int units = ring_serves(a) ? 3 : 1; units <= 3; units += 2) {  // (tiles in the place of columns: in planes, walks_columns)
     if (units == 3 && (p.tw == 32 || units * p.nblk > kTargetWorkgroups)) break;
@@ -683,11 +684,7 @@ Plan make_plan(const WgradArgs& a) {
     if (want < 1) want = 1;
     if (want > p.ntiles) want = p.ntiles;
     for (int s = want; s >= 1; s /= 2) {
-      int tps, eff;
-      for (int e = s;; e = eff - 1) {  // ends at one slice, which always divides
-        tps = (int)cdiv(p.ntiles, e), eff = (int)cdiv(p.ntiles, tps);
-        if (rows == 0 || cdiv(rows, cdiv(rows, eff)) == eff) break;
-      }
+      const int tps = (int)cdiv(p.ntiles, s), eff = (int)cdiv(p.ntiles, tps);
       const int64_t cost = eff > 1 ? tile * tps + 1000 + 64LL * eff * p.nblk / 10 : tile * tps + 600 + 32LL * p.nblk / 10;
       if (best < 0 || cost < best) {
         best = cost;
@@ -697,6 +694,7 @@ Plan make_plan(const WgradArgs& a) {
       }
     }
   }
+  if (ring_serves(a) && walks_columns(a, best)) return columns();
   return p;
 }
 

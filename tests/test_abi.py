@@ -154,16 +154,21 @@ def test_which_problems_take_a_skip_connection_as_two_tensors():
 
 
 def test_wgrad_split_plan_partitions_the_bricks():
-    """Every brick belongs to exactly one split: splits * ceil(bricks / splits) covers, (splits-1) * that does not."""
+    """Every brick belongs to exactly one split: splits * ceil(bricks / splits) covers, (splits-1) * that does not. Rows of more than 16
+    voxels are walked in bricks of 2x4x32 or, alone, in tiles of 4x8x8."""
     L = _lib.lib()
-    for sp in [(128, 128, 128), (64, 64, 64), (9, 10, 16), (5, 7, 33), (8, 8, 8), (2, 2, 2)]:
+    for sp in [(128, 128, 128), (64, 64, 64), (9, 10, 16), (5, 7, 33), (8, 8, 8), (2, 2, 2), (38, 25, 55), (19, 29, 23)]:
         for cin, cout in [(32, 32), (64, 128), (512, 512)]:
             d = conv_desc(cin=cin, cout=cout, sp=sp)
             splits = L.sfh_conv3d_wgrad_splits(ctypes.byref(d), 0)
-            tw, td, th = (32, 2, 4) if sp[2] > 16 else ((16, 2, 8) if sp[2] > 8 else (8, 4, 8))
-            bricks = -(-sp[0] // td) * -(-sp[1] // th) * -(-sp[2] // tw)
-            per = -(-bricks // splits)
-            assert 1 <= splits <= bricks and splits * per >= bricks and (splits - 1) * per < bricks
+            whole = []
+            for tw, td, th in [(32, 2, 4), (8, 4, 8)] if sp[2] > 16 else [(16, 2, 8)] if sp[2] > 8 else [(8, 4, 8)]:
+                bricks = -(-sp[0] // td) * -(-sp[1] // th) * -(-sp[2] // tw)
+                per = -(-bricks // splits)
+                whole.append(1 <= splits <= bricks and splits * per >= bricks and (splits - 1) * per < bricks)
+            assert any(whole)
+    # 280 tiles under one block, four to each of 70 slices: what the launch has room for, whatever another kernel's bricks divide into
+    assert L.sfh_conv3d_wgrad_splits(ctypes.byref(conv_desc(cin=32, cout=32, sp=(38, 25, 55))), 0) == 70
 
 
 def test_weight_gradient_batch_plan_and_refusals():
