@@ -148,7 +148,7 @@ def _deferrable(param, in_shape, wshape, stride, padding, dilation, dtype) -> in
 
 _EARLY_LOCK = threading.Lock()
 _EARLY_STREAMS: dict = {}  # (device, a pass's stream) -> the side stream beside it
-_EARLY_DONE: dict = {}  # batch sent and not joined yet -> the pass's stream
+_EARLY_DONE: set = set()  # batches sent and not joined yet: what keeps their operands alive
 
 
 def _early_stream(main):
@@ -174,11 +174,11 @@ def _send_early(batch) -> None:
     main = torch.cuda.current_stream(_lib.native().batch_device(batch))
     side = _early_stream(main)
     _lib.native().launch_beside(batch, side.stream_id, side.device_index)
-    _EARLY_DONE[batch] = main
+    _EARLY_DONE.add(batch)
 
 
 def _join_early(batch) -> None:
-    del _EARLY_DONE[batch]
+    _EARLY_DONE.remove(batch)
     _lib.native().join_beside(batch)
 
 
