@@ -879,44 +879,37 @@ __device__ __forceinline__ void block_sum256_pair(float& a, float& b, float* red
   b = (red8[4] + red8[5]) + (red8[6] + red8[7]);
 }
 
-// Two sums at once over a workgroup of kFinalize threads, in a fixed order; thread 0 gets them.
-constexpr int kFinalize = 1024;
-__device__ __forceinline__ void finalize_sum_pair(float& a, float& b, float (*red)[2]) {
-  a = wave_sum(a);
-  b = wave_sum(b);
-  if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6][0] = a; red[threadIdx.x >> 6][1] = b; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    a = b = 0.f;
-#pragma unroll
-    for (int w = 0; w < kFinalize / 64; ++w) { a += red[w][0]; b += red[w][1]; }
-  }
-}
-
 // Workgroups [0, N*G): coef[n][g] = (A, B) with A = mean(dy'*gamma), B = mean(dy'*gamma*xhat) over the group. The others:
 // dgamma[c], dbeta[c] of kFinalizeChannels channels each, summed over samples and splits.
-// A few megabytes out of the caches by a few dozen workgroups: what bounds it is the chain of trips a thread makes. With 256
-// threads, and a workgroup per channel that used 4 bytes of every line it met, 2048 splits of 64 channels took 16 us, now 8.9.
-constexpr int kFinalizeChannels = 16;
+// A few megabytes out of the caches by a few dozen workgroups: what bounds it is the chain of trips a thread makes. As workgroups of
+// 256 threads, one to a channel and using 4 bytes of every line they met, 1680 and 2048 splits of 64 channels took 15.5 us, now 9.4. The additions
+// are those of such workgroups still: 256 sums of every 256th element, wavefront trees over them, the four trees pair by pair.
+// (1024 sums met one after the other, as the layout would have it, had 1.1 to 1.5 times the error against 64 bits: dbeta of 64
+// channels of 96x80x112 7.2e-8 and 10.7e-8.)
+constexpr int kFinalize = 1024, kFinalizeChannels = 16;
 __global__ void __launch_bounds__(kFinalize) gn_bwd_finalize(const float* __restrict__ part, const void* __restrict__ gamma,
                                                              int param_dtype, float* __restrict__ coef, float* __restrict__ dgamma,
                                                              float* __restrict__ dbeta, int N, int C, int G, int nsplit, float m) {
-  __shared__ float red[kFinalize / 64][2 * kFinalizeChannels];
-  const int b = blockIdx.x;
+  constexpr int kRows = kFinalize / kFinalizeChannels;
+  static_assert(kFinalize == 4 * kBlock && kRows == 64, "four elements of every sum in flight; a row is a lane of the trees");
+  __shared__ float sums[2][4][kRows][kFinalizeChannels + 1];  // (a wavefront reads a column of it)
+  const int b = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int cg = C / G;
-  constexpr int U = 8;  // loads of either quantity in flight per thread
   if (b < N * G) {
     const int n = b / G, g = b - n * G;
-    // One flat index over (split, channel of the group): neighbouring threads read neighbouring channels and every
-    // thread's loads are independent of one another.
-    float s1 = 0.f, s2 = 0.f;
+    // One flat index over (split, channel of the group): neighbouring threads read neighbouring channels. Sum t takes elements
+    // t, t + 256, ...: a quarter of the workgroup has 16 of them in flight each, and the four quarters add theirs in turn.
+    constexpr int U = 16;
+    float (*carry)[kBlock] = reinterpret_cast<float(*)[kBlock]>(sums);
+    const int t = threadIdx.x % kBlock, quarter = threadIdx.x / kBlock;
     const float* base = part + (int64_t)n * nsplit * 2 * C + g * cg;
     const int total = nsplit * cg;
-    for (int i0 = threadIdx.x; i0 < total; i0 += U * kFinalize) {
+    float s1 = 0.f, s2 = 0.f;
+    for (int i0 = 0; i0 < total; i0 += 4 * U * kBlock) {
       float a1[U], a2[U], w[U];
 #pragma unroll
       for (int k = 0; k < U; ++k) {
-        const int i = i0 + k * kFinalize;
+        const int i = i0 + (quarter * U + k) * kBlock + t;
         const int ic = i < total ? i : total - 1;
         const int sp = ic / cg, cc = ic - sp * cg;
         const float* p = base + (int64_t)sp * 2 * C + cc;
@@ -924,54 +917,69 @@ __global__ void __launch_bounds__(kFinalize) gn_bwd_finalize(const float* __rest
         a2[k] = p[C];
         w[k] = i < total ? load_param(gamma, param_dtype, g * cg + cc, 1.f) : 0.f;
       }
+      for (int q = 0; q < 4; ++q) {
+        if (quarter == q) {
+          if (q > 0 || i0 > 0) { s1 = carry[0][t]; s2 = carry[1][t]; }
 #pragma unroll
-      for (int k = 0; k < U; ++k) {
-        s1 = fmaf(w[k], i0 + k * kFinalize < total ? a1[k] : 0.f, s1);
-        s2 = fmaf(w[k], i0 + k * kFinalize < total ? a2[k] : 0.f, s2);
+          for (int k = 0; k < U; ++k) {
+            const bool in = i0 + (quarter * U + k) * kBlock + t < total;
+            s1 = fmaf(w[k], in ? a1[k] : 0.f, s1);
+            s2 = fmaf(w[k], in ? a2[k] : 0.f, s2);
+          }
+          carry[0][t] = s1;
+          carry[1][t] = s2;
+        }
+        __syncthreads();
       }
     }
-    finalize_sum_pair(s1, s2, reinterpret_cast<float(*)[2]>(red));
+    float* tot = &sums[1][0][0][0];  // (behind the carried sums)
+    if (wave < 4) {
+      s1 = wave_sum(carry[0][t]);
+      s2 = wave_sum(carry[1][t]);
+      if (lane == 0) { tot[wave] = s1; tot[4 + wave] = s2; }
+    }
+    __syncthreads();
     if (threadIdx.x == 0) {
-      coef[(n * G + g) * 2] = s2 / m;
-      coef[(n * G + g) * 2 + 1] = s1 / m;
+      coef[(n * G + g) * 2] = ((tot[4] + tot[5]) + (tot[6] + tot[7])) / m;
+      coef[(n * G + g) * 2 + 1] = ((tot[0] + tot[1]) + (tot[2] + tot[3])) / m;
     }
   } else {
-    constexpr int ROWS = kFinalize / kFinalizeChannels;
-    const int own = threadIdx.x % kFinalizeChannels, c = (b - N * G) * kFinalizeChannels + own;
-    float s1 = 0.f, s2 = 0.f;
+    // Row r takes elements r, r + 64, ..., which belong to sums r, r + 64, r + 128 and r + 192 in turn.
+    constexpr int U = 8;
+    const int own = threadIdx.x % kFinalizeChannels, row = threadIdx.x / kFinalizeChannels;
+    const int first = (b - N * G) * kFinalizeChannels, c = first + own;
+    float s1[4] = {0.f, 0.f, 0.f, 0.f}, s2[4] = {0.f, 0.f, 0.f, 0.f};
     const int total = c < C ? N * nsplit : 0;
-    for (int i0 = threadIdx.x / kFinalizeChannels; i0 < total; i0 += U * ROWS) {
+    for (int i0 = row; i0 < total; i0 += U * kRows) {
       float a1[U], a2[U];
 #pragma unroll
       for (int k = 0; k < U; ++k) {
-        const int i = i0 + k * ROWS;
+        const int i = i0 + k * kRows;
         const float* p = part + (int64_t)(i < total ? i : total - 1) * 2 * C + c;
         a1[k] = p[0];
         a2[k] = p[C];
       }
 #pragma unroll
       for (int k = 0; k < U; ++k) {
-        s1 += i0 + k * ROWS < total ? a1[k] : 0.f;
-        s2 += i0 + k * ROWS < total ? a2[k] : 0.f;
+        s1[k % 4] += i0 + k * kRows < total ? a1[k] : 0.f;
+        s2[k % 4] += i0 + k * kRows < total ? a2[k] : 0.f;
       }
     }
-    // the rows of a wavefront meet in a butterfly, the wavefronts in order through LDS
 #pragma unroll
-    for (int off = kFinalizeChannels; off < 64; off <<= 1) {
-      s1 += __shfl_xor(s1, off, 64);
-      s2 += __shfl_xor(s2, off, 64);
-    }
-    if ((threadIdx.x & 63) < kFinalizeChannels) {
-      red[threadIdx.x >> 6][own] = s1;
-      red[threadIdx.x >> 6][kFinalizeChannels + own] = s2;
+    for (int w = 0; w < 4; ++w) {
+      sums[0][w][row][own] = s1[w];
+      sums[1][w][row][own] = s2[w];
     }
     __syncthreads();
-    if (threadIdx.x < 2 * kFinalizeChannels && c < C) {
-      float t = 0.f;
+    // wavefront w: channel first + w
+    float tot[2][4];
 #pragma unroll
-      for (int w = 0; w < kFinalize / 64; ++w) t += red[w][threadIdx.x];
-      float* dst = threadIdx.x < kFinalizeChannels ? dgamma : dbeta;
-      if (dst != nullptr) dst[c] = t;
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) tot[q][w] = wave_sum(sums[q][w][lane][wave]);
+    if (lane == 0 && first + wave < C) {
+      if (dgamma != nullptr) dgamma[first + wave] = (tot[0][0] + tot[0][1]) + (tot[0][2] + tot[0][3]);
+      if (dbeta != nullptr) dbeta[first + wave] = (tot[1][0] + tot[1][1]) + (tot[1][2] + tot[1][3]);
     }
   }
 }
