@@ -23,19 +23,21 @@ __device__ __forceinline__ float wave_sum_all(float v) {
   return v;  // lane 0 holds the sum
 }
 
-// The same total in lane 63, on the vector pipe alone: rows of 16 lanes by shifts of 1, 2, 4 and 8, then rows 0 and 2 into
-// rows 1 and 3 and row 1 into rows 2 and 3. The 3 C + 2 totals of a workgroup made 228 trips through the LDS pipe as shuffles.
-template <int CTRL, int ROWS>
+// The same total, pair by pair, in lane 63 and on the vector pipe alone: halves and rows of 16 lanes traded, then shifts of 8, 4, 2 and 1
+// within the rows. The 3 C + 2 totals of a workgroup made 228 trips through the LDS pipe as shuffles.
+template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {
-  return v + __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, ROWS, 0xf, true));
+  return v + __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
 }
 __device__ __forceinline__ float wave_sum_last(float v) {
-  v = dpp_add<0x111, 0xf>(v);
-  v = dpp_add<0x112, 0xf>(v);
-  v = dpp_add<0x114, 0xf>(v);
-  v = dpp_add<0x118, 0xf>(v);
-  v = dpp_add<0x142, 0xa>(v);
-  return dpp_add<0x143, 0xc>(v);
+  const auto half = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(half[0]) + __uint_as_float(half[1]);
+  const auto row = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(row[0]) + __uint_as_float(row[1]);
+  v = dpp_add<0x118>(v);
+  v = dpp_add<0x114>(v);
+  v = dpp_add<0x112>(v);
+  return dpp_add<0x111>(v);
 }
 
 // Voxels a thread works on between two barriers: as many as keep a tile's logits within 32 KiB of LDS, so that four
@@ -271,40 +273,39 @@ __global__ void __launch_bounds__(64) ce_dice_scalar(const float* __restrict__ s
 }
 
 // Both of the above as one workgroup, for up to kTotalSamples samples and kTotalSlotsMax slots. A wavefront reads a slot's
-// quantities side by side and takes every sixteenth slot, sixteen of them in flight; sums of sixteen by a tree, the
-// wavefronts' by a tree. What bounds it is a launch and the trips of one CU: 128 slots of 35 quantities 5.3 us (the two launches
-// 9.3), 512 slots of 53 10.5 (level), 1024 of 35 17.8.
+// quantities side by side and takes every sixteenth slot, all of them in flight; the sums are those of ce_dice_sum, bit for
+// bit. What bounds it is a launch and the trip of one CU: 128 slots of 35 quantities 2.9 us (the two launches 3.9 and 1.6 and the gap
+// between them). With more slots, in rounds, 512 of 53 were level with the two and 1024 of 35 twice as slow.
 constexpr int kTotal = 1024, kTotalWaves = kTotal / 64, kTotalSamples = 4, kTotalQ = 3 * 32 + 2, kTotalSlots = 16, kTotalSlotsMax = 256;
+static_assert(kTotalSlots * kTotalWaves >= kTotalSlotsMax, "a wavefront's slots are read at once");
 __global__ void __launch_bounds__(kTotal) ce_dice_total(const float* __restrict__ part, float* __restrict__ stats, float* __restrict__ loss,
                                                         int N, int C, int nsplit, int unweighted, float count, float eps) {
   __shared__ float wave_tot[kTotalWaves][kTotalQ];
   __shared__ float tot[kTotalSamples * 3 * 32 + 2];
   const int Q = 3 * C + 2;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  float launch_wide = 0.f;  // the last two quantities run over all samples
   for (int n = 0; n < N; ++n) {
-    const float* src = part + (int64_t)n * nsplit * Q;
-    for (int q = lane; q < Q; q += 64) {
-      float s = 0.f;
-      for (int sp = wave; sp < nsplit; sp += kTotalSlots * kTotalWaves) {
-        float v[kTotalSlots];
+    // the last two quantities run over the slots of all samples, beside the first sample's own
+    for (int q = lane; q < (n == 0 ? Q : 3 * C); q += 64) {
+      const bool wide = q >= 3 * C;
+      const int slots = wide ? N * nsplit : nsplit;
+      const float* src = part + (wide ? 0 : (int64_t)n * nsplit * Q) + q;
+      float v[kTotalSlots];
 #pragma unroll
-        for (int k = 0; k < kTotalSlots; ++k) {
-          const int at = sp + k * kTotalWaves;
-          v[k] = src[(int64_t)(at < nsplit ? at : sp) * Q + q];
-        }
-#pragma unroll
-        for (int k = 0; k < kTotalSlots; ++k) v[k] = sp + k * kTotalWaves < nsplit ? v[k] : 0.f;
-#pragma unroll
-        for (int h = kTotalSlots / 2; h > 0; h >>= 1)
-#pragma unroll
-          for (int k = 0; k < h; ++k) v[k] += v[k + h];
-        s += v[0];
+      for (int k = 0; k < kTotalSlots; ++k) {
+        const int at = wave + k * kTotalWaves;
+        v[k] = src[(int64_t)(at < slots ? at : 0) * Q];
       }
-      wave_tot[wave][q] = s;
+#pragma unroll
+      for (int k = 0; k < kTotalSlots; ++k) v[k] = wave + k * kTotalWaves < slots ? v[k] : 0.f;
+      // slots 64 apart one after the other, then those 32 and 16 apart: the order of ce_dice_sum's lanes and of its tree
+      float lane_sum[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) lane_sum[j] = ((v[j] + v[4 + j]) + v[8 + j]) + v[12 + j];
+      wave_tot[wave][q] = (lane_sum[0] + lane_sum[2]) + (lane_sum[1] + lane_sum[3]);
     }
     __syncthreads();
-    if (tid < Q) {
+    if (tid < (n == 0 ? Q : 3 * C)) {
       float v[kTotalWaves];
 #pragma unroll
       for (int w = 0; w < kTotalWaves; ++w) v[w] = wave_tot[w][tid];
@@ -312,19 +313,10 @@ __global__ void __launch_bounds__(kTotal) ce_dice_total(const float* __restrict_
       for (int h = kTotalWaves / 2; h > 0; h >>= 1)
 #pragma unroll
         for (int w = 0; w < h; ++w) v[w] += v[w + h];
-      if (tid < 3 * C) {
-        const int dst = (tid / C) * N * C + n * C + tid % C;
-        tot[dst] = v[0];
-        stats[dst] = v[0];
-      } else {
-        launch_wide += v[0];
-        if (n == N - 1) {
-          // the normaliser of the unweighted mean is the voxel count
-          const float t = tid == 3 * C + 1 && unweighted ? count : launch_wide;
-          tot[N * 3 * C + tid - 3 * C] = t;
-          stats[N * 3 * C + tid - 3 * C] = t;
-        }
-      }
+      const int dst = tid < 3 * C ? (tid / C) * N * C + n * C + tid % C : N * 3 * C + tid - 3 * C;
+      if (tid == 3 * C + 1 && unweighted) v[0] = count;  // the normaliser of the unweighted mean is the voxel count
+      tot[dst] = v[0];
+      stats[dst] = v[0];
     }
     __syncthreads();
   }

@@ -1,10 +1,13 @@
 """GPU parity of the fused cross-entropy + soft-Dice loss head against the oracle (fp64 torch restatement of
 ``ScaFFold/utils/trainer.py:634-663``), through the C ABI."""
 
+import ctypes
+
 import pytest
 import torch
 
 import scaffold_amd as sa
+from scaffold_amd import _lib
 from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -108,9 +111,52 @@ def test_gate_and_determinism(device):
 @pytest.mark.parametrize("shape", [(1, 4, 5, 7, 9), (1, 5, 5, 7, 9), (1, 8, 3, 8, 11), (2, 10, 3, 8, 11), (1, 12, 4, 4, 17), (1, 13, 4, 4, 17),
                                    (1, 16, 4, 4, 17),       # either end of the kernels' class ranges
                                    (5, 3, 2, 3, 4),         # more samples than one workgroup totals
-                                   (2, 6, 16, 32, 33),      # more slots than one workgroup totals
+                                   (2, 6, 16, 32, 33),      # 132 slots, totalled by one workgroup
+                                   (2, 6, 32, 32, 33),      # 264: more than one workgroup totals
                                    (1, 2, 65, 128, 130)])   # several tiles per workgroup, the last of each cut
 def test_loss_class_ranges_and_totals(device, dtype, shape):
     """The class ranges, the two ways the totals are taken and the several tiles of a large volume. Tolerances as above: the loss is a
     quotient of fp32 sums, the gradient is rounded once."""
     test_loss_and_gradient_match_oracle(device, dtype, shape, False)
+
+
+def _tree(v):
+    """A wavefront's sum: halves of 32, 16, ... 1 lanes added to one another (v: (64, ...) float32)."""
+    while v.shape[0] > 1:
+        v = v[:v.shape[0] // 2] + v[v.shape[0] // 2:]
+    return v[0]
+
+
+def _slots_sum(v):
+    """Slots l, l + 64, ... one after the other in lane l, then the tree (v: (slots, ...) float32)."""
+    lanes = torch.zeros((64, *v.shape[1:]), dtype=torch.float32)
+    for at in range(0, v.shape[0], 64):
+        k = min(64, v.shape[0] - at)
+        lanes[:k] += v[at:at + k]
+    return _tree(lanes)
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("n,c,tiles", [(1, 3, 1), (1, 11, 70), (1, 4, 256), (1, 4, 257), (2, 6, 77), (2, 32, 128), (2, 2, 129), (3, 17, 40), (4, 5, 64), (5, 5, 7)])
+def test_totals_are_the_same_sums_whichever_launch_takes_them(device, n, c, tiles, weighted):
+    """Either side of 256 slots and of four samples: the totals are those of the slots the first launch left, added in one order, bit for bit."""
+    spatial = tiles * 256 - 3
+    d = _lib.LossDesc(n, c, spatial, 1e-6)
+    L = _lib.lib()
+    g = torch.Generator(device=device).manual_seed(n * c)
+    logits = torch.randn((n, spatial, c), generator=g, device=device) * 3
+    labels = torch.randint(0, c, (n, spatial), generator=g, device=device)
+    cw = torch.rand(c, generator=g, device=device) + 0.5 if weighted else None
+    need = L.sfh_ce_dice_workspace_bytes(ctypes.byref(d))
+    ws = torch.full((need // 4,), float("nan"), device=device)
+    loss, stats = torch.empty(1, device=device), torch.empty(3 * n * c + 2, device=device)
+    rc = L.sfh_ce_dice_fwd(ctypes.byref(d), 2, logits.data_ptr(), labels.data_ptr(), cw.data_ptr() if weighted else None, loss.data_ptr(),
+                           stats.data_ptr(), ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    slots = ws.cpu().view(n, -1, 3 * c + 2)
+    assert slots.shape[1] == tiles and torch.isfinite(slots).all()
+    want = torch.stack([_slots_sum(s[:, :3 * c]) for s in slots]).view(n, 3, c).transpose(0, 1).reshape(-1)
+    wide = _slots_sum(slots.reshape(-1, 3 * c + 2)[:, 3 * c:])
+    if not weighted:
+        wide[1] = n * spatial
+    assert torch.equal(stats.cpu(), torch.cat((want, wide)))
