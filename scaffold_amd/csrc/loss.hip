@@ -399,6 +399,7 @@ __global__ void __launch_bounds__(kBlock) ce_dice_backward(const T* __restrict__
 #pragma unroll
       for (int c = 0; c < CMAX; ++c) {
         if (has_class<CMAX>(c, C)) {
+#pragma clang fp contract(off)  // p_j - [j == y] of the rounded p_j, for a class that needs no question as for one that does
           const bool hit = c == y;
           const float d = fmaf(p[c], g[c] - dot, cs * (p[c] - (hit ? 1.f : 0.f)));
           row[c] = elem<T>::from_float(d);
