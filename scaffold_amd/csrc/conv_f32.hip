@@ -48,7 +48,8 @@ struct FTile {
   static constexpr int MS = TD * TH * TW / (32 * WM);  // 32-voxel sub-tiles per wavefront
   // One sub-tile to a wavefront is what a volume gets that does not fill the chip: nothing else on the SIMD hides a trip to
   // memory or LDS, and there are registers for requesting the next chunk's brick and the next tap's activations ahead.
-  // 32 -> 32 channels on 32^3: 27.4 -> 20.5 us a launch (its MFMAs alone 11.5; now 19).
+  // 32 -> 32 channels on 32^3: 27.4 -> 20.5 us a launch (its MFMAs alone 11.5; in bricks of
+  // 8-voxel rows 21.3 in a trace with idle time between passes).
   static constexpr bool AHEAD = MS == 1;
   static_assert(TD * TH * TW % (32 * WM) == 0, "tile must split into WM wavefronts of 32-voxel sub-tiles");
   static_assert(KS == 1 || MS == 1, "the parts of a reduction meet in one sub-tile a wavefront");

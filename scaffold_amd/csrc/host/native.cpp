@@ -655,8 +655,8 @@ struct ConvSaved {
     if (need_x || need_2) {
       // The faces of a slab are zeros that the module put there: nobody receives their gradients.  The planes between them
       // are the data gradient of the padded problem, whose launch has no planes to drop (on 8 planes a fifth of the work) and
-      // no workgroups past a round for them; a voxel's sum is the same.  Where the padded problem is not one the gradient
-      // serves (a halo wider than the kernel reaches) the slab's is cut.
+      // no workgroups past a round for them; a voxel's products are the same, added in the order of the kernel that serves
+      // the padded problem.  Where that is not one the gradient serves (a halo wider than the kernel reaches) the slab's is cut.
       Problem inner = prob;
       int64_t cut = halo;
       if (halo > 0 && p[0] + halo <= (int64_t)d[0] * (w_sizes[2] - 1)) {

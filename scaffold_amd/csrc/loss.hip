@@ -41,9 +41,9 @@ __device__ __forceinline__ float wave_sum_last(float v) {
 }
 
 // Voxels a thread works on between two barriers: as many as keep a tile's logits within 32 KiB of LDS, so that four
-// workgroups fit a CU and a workgroup's trips to memory are one or two, not one per 256 voxels. bf16, before and now: partial
-// sums of 11 classes of 64x128x128 27.3 -> 15.8 us (54 MB; the totals' trips through the LDS pipe were 6 us of it), of
-// 6 classes of 128-cube 35.6 -> 15.8, of 11 classes of 32-cube 12.9 -> 5.3; backward 23.4 -> 17.3, 36.7 -> 19.0, 6.9 -> 4.6.
+// workgroups fit a CU and a workgroup's trips to memory are one or two, not one per 256 voxels. bf16 in a trace, before and now: partial
+// sums of 11 classes of 64x128x128 25 -> 18.9 us (54 MB; the totals' trips through the LDS pipe were 6 us of it), of 6 classes of
+// 128-cube 36 -> 18.9, of 11 classes of 32-cube 11.7 -> 6.3, of 17 of 32x64x64 27.7 -> 14.1; backward 23 -> 18.4, 38 -> 21.2, 5.2 -> 4.9, 11.0 -> 10.2.
 template <typename T, int CMAX> constexpr int kVoxels = 32768 / (kBlock * CMAX * (int)sizeof(T)) >= 4   ? 4
                                                         : 32768 / (kBlock * CMAX * (int)sizeof(T)) >= 2 ? 2
                                                                                                         : 1;

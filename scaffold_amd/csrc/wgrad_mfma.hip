@@ -759,9 +759,10 @@ int64_t busiest(const WTileBatch& b, int units) {
 // it is in a U-Net has 18 blocks: 54 units of 30 tiles' cost each kept 202 workgroups waiting. Where a gradient has up to 64 output
 // channels and more than eight tiles under a block, parts of about six tiles: slices (108 KB a block and part) and a sum pass (5 us) in
 // exchange. Levels of 128 channels and more have blocks enough: cut as well, the lists of 48^3 (width 64) and 125x34x37 (width 32) went
-// from 75 and 45 us to 89 and 53. A function of the problem alone: what else is in a list decides only
-// whether three workgroups share a block (tile_batch_plan), and with that in which chains a tile's k-steps are summed. Lists of the deep
-// levels of a step, us: 56x27x27 47.7 -> 30.4, 32^3 30.2 -> 22.1; 43x124x47, all of 128 channels and more, 54.
+// from 75 and 45 us to 89 and 53. Output channels stand in for blocks in that, a problem at a time, so 512 -> 64 (32 blocks) is cut and 32 -> 128
+// (four) is not. A function of the problem alone: what else is in a list decides only whether three workgroups share a block
+// (tile_batch_plan), and with that in which chains a tile's k-steps are summed. Lists of the deep levels of a step, us: 56x27x27 47.7 -> 30.4,
+// 32^3 30.2 -> 22.1; 43x124x47, all of 128 channels and more, 54.
 int unit_parts(int ntiles, int cout) { return ntiles <= 8 || cout > 64 ? 1 : (int)cdiv(ntiles, 6); }
 
 // Lays the units out on the line of cost, `units` to a part of a block.
