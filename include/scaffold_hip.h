@@ -171,7 +171,7 @@ int sfh_conv3d_fwd(const sfh_conv3d_desc* p, int dtype, const void* x, const voi
  * spread, nothing is carried from call to call and nothing comes from the caller.
  * sfh_conv3d_fwd_gn_records gives `records` for a problem and group count, a pure function of both; 0 means
  * the kernel that serves the problem does not offer it (direct / fp32 / 2x2x2 kernels, thin-channel ones other than
- * the one-channel 3x3x3 stem, several samples on the persistent kernel, groups of fewer than 4 or a non-multiple-of-4
+ * the one-channel 3x3x3 stem, several samples whose runs of bricks or columns cross on the persistent kernel, groups of fewer than 4 or a non-multiple-of-4
  * channels) and the caller uses sfh_conv3d_fwd and
  * the ordinary GroupNorm. 16-bit dtypes only. gn_partials must be 16-byte aligned. */
 int32_t sfh_conv3d_fwd_gn_records(const sfh_conv3d_desc* p, int dtype, int groups);

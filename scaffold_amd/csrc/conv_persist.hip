@@ -500,12 +500,13 @@ MfmaConvGeometry mfma_conv_geometry(const MfmaConvArgs& a) {
   return MfmaConvGeometry{kKernelPersist, 512, 1, 1};
 }
 
-// One record per workgroup, so one sample only (a workgroup's run of bricks may cross samples).
+// One record per workgroup, so only where a workgroup stays in one sample (a run of bricks may cross them).
 int mfma_conv_gn_records(const MfmaConvArgs& a, int groups) {
   if (!mfma_conv_persist_applies(a)) return mfma_conv_gather_gn_records(a, groups);
-  if (a.n != 1 || !gn_partials_fit(a.cout, groups, 32)) return 0;
+  if (!gn_partials_fit(a.cout, groups, 32)) return 0;
   const int cg = a.cout / groups;
-  if (ring_serves(a)) return mfma_conv_ring_workgroups_per_block(a) * (cg > 32 ? cg / 32 : 1);
+  if (ring_serves(a)) return mfma_conv_ring_records(a) * (cg > 32 ? cg / 32 : 1);
+  if (a.n != 1) return 0;
   const PersistGeom gm = persist_geom(a);
   if (gm.ntiles <= 0) return 0;
   return gm.wgs_per_block * (cg > 32 ? cg / 32 : 1);

@@ -148,7 +148,8 @@ struct RingGeom {
   int steps;                  // steps of a whole column: ceil(od / 2)
   int segs, seg_steps;        // a column is cut into `segs` segments of `seg_steps` steps (the last one shorter)
   int nblocks;                // 32-channel output blocks
-  int items, wgs_per_block, items_per_wg;  // items = columns x segments; each workgroup takes items_per_wg consecutive ones
+  int parts;                  // the batch is walked as one line of columns (1) or every sample by workgroups of its own (n)
+  int items, wgs, items_per_wg;  // of a part: columns x segments; each of its workgroups takes items_per_wg consecutive ones
 };
 
 // What a lane needs to know for the whole launch.
@@ -359,9 +360,10 @@ conv_ring_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ 
   const int j = lane & 31, kg = lane >> 5;
 
   const int wg = (int)xcd_remap(blockIdx.x, gridDim.x);
-  const int nb = wg / gm.wgs_per_block;
-  const int wg_in_block = wg - nb * gm.wgs_per_block;
-  const int item_begin = wg_in_block * gm.items_per_wg;
+  const int wgs_per_block = gm.parts * gm.wgs;
+  const int nb = wg / wgs_per_block;
+  const int part = (wg - nb * wgs_per_block) / gm.wgs, wg_in_part = (wg - nb * wgs_per_block) % gm.wgs;
+  const int item_begin = wg_in_part * gm.items_per_wg;
   int item_end = item_begin + gm.items_per_wg;
   if (item_end > gm.items) item_end = gm.items;
   if (nb >= gm.nblocks || item_begin >= item_end) return;
@@ -426,7 +428,7 @@ conv_ring_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ 
     // item = segment * columns + column: the workgroups of an XCD work on neighbouring columns over the same depth range
     const int ncols = gm.items / gm.segs;
     const int seg = item / ncols;
-    const RingColumn col = ring_column(item - seg * ncols, gm);
+    const RingColumn col = ring_column(part * ncols + item - seg * ncols, gm);
     const int s_begin = seg * gm.seg_steps;
     int s_end = s_begin + gm.seg_steps;
     if (s_end > gm.steps) s_end = gm.steps;
@@ -491,12 +493,36 @@ conv_ring_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ 
   run_item(item_begin, std::true_type{});
   for (int item = item_begin + 1; item < item_end; ++item) run_item(item, std::false_type{});
   if constexpr (GN) {
-    // one record per workgroup (one sample): the last barrier has freed the LDS
+    // one record per workgroup (of one sample: `part`): the last barrier has freed the LDS
     const int per_wg = gn.cg > 32 ? gn.cg / 32 : 1;  // output blocks that share a group
     RunSums one[1] = {gn_sums};
-    write_group_partials<4, 1>(one, reinterpret_cast<float*>(pair0), gn, 0, wg_in_block * per_wg + nb % per_wg, nb * 32, tid);
+    write_group_partials<4, 1>(one, reinterpret_cast<float*>(pair0), gn, part, wg_in_part * per_wg + nb % per_wg, nb * 32, tid);
   }
 #endif
+}
+
+// How `wgs` workgroups at most walk `ncols` columns of `gm.steps` steps: the columns are cut into as many segments as let the
+// busiest workgroup end soonest. Its time is its steps (3.6 us each where the launch is short of the power limit) and one step
+// per item: two plane pairs from memory with nothing beside them, 1.5 to 2 us measured, and what short items lose otherwise.
+// 32 -> 32, us, against cutting until every workgroup has an item, which left up to half of them idle behind two items of the
+// others: 54x105x99 52.7 -> 35.8, 36x101x119 39.1 -> 28.8, two samples of 57x87x77 67.8 -> 48.1; 32 -> 64 at 75x107x122
+// 111 -> 92. Returns the time in steps; -1: too many items.
+int64_t ring_plan(RingGeom& gm, int64_t ncols, int64_t wgs) {
+  int64_t best = -1;
+  const int64_t most = cdiv(4 * wgs, ncols);  // more than four items to a workgroup even nothing out any more
+  for (int64_t want = 1; want <= most && want <= gm.steps; ++want) {
+    const int64_t len = cdiv(gm.steps, want), segs = cdiv(gm.steps, len), items = ncols * segs;
+    if (items > 0x7fffffffLL) break;
+    const int64_t per_wg = cdiv(items, wgs), cost = per_wg * (len + 1);
+    if (best >= 0 && cost >= best) continue;
+    best = cost;
+    gm.segs = (int)segs;
+    gm.seg_steps = (int)len;
+    gm.items = (int)items;
+    gm.items_per_wg = (int)per_wg;
+    gm.wgs = (int)cdiv(items, per_wg);
+  }
+  return best;
 }
 
 RingGeom ring_geom(const MfmaConvArgs& a) {
@@ -505,22 +531,20 @@ RingGeom ring_geom(const MfmaConvArgs& a) {
   gm.tiles_w = (int)cdiv(a.ow, kTW);
   gm.steps = (int)cdiv(a.od, kTD);
   gm.nblocks = a.cout / 32;
-  const int64_t ncols = (int64_t)a.n * gm.tiles_h * gm.tiles_w;
-  int per_block = kComputeUnits / gm.nblocks;
-  if (per_block < 1) per_block = 1;
-  // segments per column: enough for every workgroup of the block to have one, no more than there are steps
-  int64_t segs = ncols >= per_block ? 1 : cdiv(per_block, ncols);
-  if (segs > gm.steps) segs = gm.steps;
-  gm.seg_steps = (int)cdiv(gm.steps, segs);
-  gm.segs = (int)cdiv(gm.steps, gm.seg_steps);
-  const int64_t items = ncols * gm.segs;
-  gm.items = items > 0x7fffffffLL ? -1 : (int)items;
-  if (gm.items > 0) {
-    if (per_block > gm.items) per_block = gm.items;
-    gm.items_per_wg = (int)cdiv(gm.items, per_block);
-    gm.wgs_per_block = (int)cdiv(gm.items, gm.items_per_wg);
-  }
-  return gm;
+  gm.parts = 1;
+  const int64_t cols = (int64_t)gm.tiles_h * gm.tiles_w;
+  const int64_t per_block = kComputeUnits > gm.nblocks ? kComputeUnits / gm.nblocks : 1;
+  if (cols * a.n <= 0 || gm.steps <= 0) return gm;
+  const int64_t cost = ring_plan(gm, cols * a.n, per_block);
+  if (cost < 0) gm.items = -1;
+  if (cost < 0 || a.n == 1 || per_block / a.n < 8) return gm;
+  // Several samples, each by workgroups of its own: a workgroup's sums are then those of one sample, and the normalisation
+  // behind the convolution needs no statistics pass. Where that ends no more than an eighth later, and a sample is more than
+  // a few columns (the statistics pass of a smaller one is the same launch whatever it reads).
+  RingGeom apart = gm;
+  apart.parts = a.n;
+  const int64_t cost_apart = ring_plan(apart, cols, per_block / a.n);
+  return cost_apart > 0 && 8 * cost_apart <= 9 * cost && apart.wgs >= 8 ? apart : gm;
 }
 
 template <typename T>
@@ -529,7 +553,7 @@ int launch_ring(const MfmaConvArgs& a, const void* x, const void* packed, const 
   const RingGeom gm = ring_geom(a);
   if (gm.items < 0) return fail(SFH_ERR_UNSUPPORTED, "conv mfma: too many columns");
   if (gm.items == 0) return SFH_OK;
-  const unsigned grid = (unsigned)(gm.wgs_per_block * gm.nblocks);
+  const unsigned grid = (unsigned)(gm.parts * gm.wgs * gm.nblocks);
 #define SFH_RING(BIAS, GN)                                                                                                  \
   hipLaunchKernelGGL((conv_ring_kernel<T, BIAS, GN>), dim3(grid), dim3(256), 0, st, a, (const T*)x, (const T*)packed, \
                      (const T*)bias, (T*)y, gm, gn, (T*)out2.second, out2.first)
@@ -553,7 +577,10 @@ bool mfma_conv_ring_applies(const MfmaConvArgs& a) {
          ((int64_t)(a.ih + kBH) * a.iw + kBW) * a.cred * 2 + 64 < kRange && ((int64_t)(a.oh + kTH) * a.ow + kTW) * a.cout * 2 + 64 < kRange;
 }
 
-int mfma_conv_ring_workgroups_per_block(const MfmaConvArgs& a) { return ring_geom(a).wgs_per_block; }
+int mfma_conv_ring_records(const MfmaConvArgs& a) {
+  const RingGeom gm = ring_geom(a);
+  return gm.items > 0 && gm.parts == a.n ? gm.wgs : 0;
+}
 
 int mfma_conv_ring(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                    const GnPartialOut& gn, const ChannelPair& out2) {

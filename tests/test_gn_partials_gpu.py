@@ -142,6 +142,20 @@ def test_random_problems(device, n, cin, cout, spatial, padding, groups):
     assert orc.gn_rel_error(fused, ref) < 2e-2
 
 
+@pytest.mark.parametrize("n,cout,spatial,groups", [(2, 32, (6, 44, 60), 8), (3, 64, (9, 21, 75), 2), (2, 64, (7, 41, 33), 1),
+                                                   (2, 32, (3, 320, 130), 4), (5, 96, (5, 64, 64), 12)])
+def test_samples_walked_apart(device, n, cout, spatial, groups):
+    """Batches whose samples are walked by workgroups of their own (one and two columns to a workgroup, groups within and past a
+    workgroup's 32 channels): every sample has the bits it has alone, and records of its own."""
+    prob = orc.ConvProblem(n=n, cin=32, cout=cout, spatial=spatial, padding=(1, 1, 1), dtype=torch.bfloat16)
+    ops = orc.make_inputs(prob, seed=3 + n, exact=True, density=0.05)
+    x, w = ops["input"].to(device), ops["weight"].to(device)
+    y = sa.conv3d_forward(x, w, None, 1, 1, 1, gn_groups=groups)
+    for i in range(n):
+        assert torch.equal(y[i:i + 1], sa.conv3d_forward(x[i:i + 1].contiguous(memory_format=CL), w, None, 1, 1, 1))
+    check_records(y, groups, y._sfh_gn_partials)
+
+
 @pytest.mark.parametrize("relu", [False, True])
 @pytest.mark.parametrize("n,cin,cout,spatial,padding,groups,kernel", CASES)
 def test_group_norm_from_partials_matches_the_statistics_pass(device, n, cin, cout, spatial, padding, groups, kernel, relu):
