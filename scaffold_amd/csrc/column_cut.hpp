@@ -1,0 +1,37 @@
+// How many workgroups walk the columns of a volume: the launch rule of the kernels that step along depth and keep the
+// planes they have fetched (conv_ring.hip, wgrad_ring.hip).
+#pragma once
+#include "common.hpp"
+
+namespace sfh {
+
+// Columns are cut into `segs` segments of `seg_steps` steps (the last one shorter); of the `items` = columns x segments each
+// of `wgs` workgroups takes `items_per_wg` consecutive ones. cost: the busiest workgroup's time in steps.
+struct ColumnCut {
+  int segs, seg_steps, items, items_per_wg, wgs;
+  int64_t cost;
+};
+
+// The cut by which the busiest of at most `wgs` workgroups ends soonest, `ncols` columns of `steps` steps. Its time is its
+// steps (3.6 us each forward where the launch is short of the power limit, 2.1 in the weight gradient) and one step per item: the
+// item's first planes come from memory with nothing beside them (1.5 to 2 us measured), and what short items lose otherwise.
+// items < 0: too many.
+//
+// us, against cutting until every workgroup has an item, which left up to half of them idle behind two items of the others:
+// forward 32 -> 32 at 54x105x99 53.5 -> 37.7, 36x101x119 39.1 -> 28.8, 96x80x112 59.4 -> 44.5, two samples of 57x87x77 67.1 -> 47.7,
+// 32 -> 64 at 75x107x122 111 -> 92; weight gradient with its sum 32 -> 32 at 96x80x112 63.9 -> 54.3, 54x105x99 53.2 -> 47.0, two
+// samples of 57x87x77 72.5 -> 58.5, 64 -> 32 at 110x48x111 91.2 -> 69.9, 128 -> 64 at 60x35x45 76.4 -> 60.8.
+inline ColumnCut cut_columns(int64_t ncols, int64_t steps, int64_t wgs) {
+  ColumnCut best{};
+  best.items = -1;
+  const int64_t most = cdiv(4 * wgs, ncols);  // more than four items to a workgroup even nothing out any more
+  for (int64_t want = 1; want <= most && want <= steps; ++want) {
+    const int64_t len = cdiv(steps, want), segs = cdiv(steps, len), items = ncols * segs;
+    if (items > 0x7fffffffLL) break;
+    const int64_t per_wg = cdiv(items, wgs), cost = per_wg * (len + 1);
+    if (best.items < 0 || cost < best.cost) best = ColumnCut{(int)segs, (int)len, (int)items, (int)per_wg, (int)cdiv(items, per_wg), cost};
+  }
+  return best;
+}
+
+}  // namespace sfh

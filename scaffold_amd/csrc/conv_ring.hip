@@ -21,6 +21,7 @@
 // offset from one of three per-lane bases.
 #include <utility>
 
+#include "column_cut.hpp"
 #include "conv_mfma.hpp"
 #include "mma.hpp"
 
@@ -501,28 +502,14 @@ conv_ring_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ 
 #endif
 }
 
-// How `wgs` workgroups at most walk `ncols` columns of `gm.steps` steps: the columns are cut into as many segments as let the
-// busiest workgroup end soonest. Its time is its steps (3.6 us each where the launch is short of the power limit) and one step
-// per item: two plane pairs from memory with nothing beside them, 1.5 to 2 us measured, and what short items lose otherwise.
-// 32 -> 32, us, against cutting until every workgroup has an item, which left up to half of them idle behind two items of the
-// others: 54x105x99 52.7 -> 35.8, 36x101x119 39.1 -> 28.8, two samples of 57x87x77 67.8 -> 48.1; 32 -> 64 at 75x107x122
-// 111 -> 92. Returns the time in steps; -1: too many items.
-int64_t ring_plan(RingGeom& gm, int64_t ncols, int64_t wgs) {
-  int64_t best = -1;
-  const int64_t most = cdiv(4 * wgs, ncols);  // more than four items to a workgroup even nothing out any more
-  for (int64_t want = 1; want <= most && want <= gm.steps; ++want) {
-    const int64_t len = cdiv(gm.steps, want), segs = cdiv(gm.steps, len), items = ncols * segs;
-    if (items > 0x7fffffffLL) break;
-    const int64_t per_wg = cdiv(items, wgs), cost = per_wg * (len + 1);
-    if (best >= 0 && cost >= best) continue;
-    best = cost;
-    gm.segs = (int)segs;
-    gm.seg_steps = (int)len;
-    gm.items = (int)items;
-    gm.items_per_wg = (int)per_wg;
-    gm.wgs = (int)cdiv(items, per_wg);
-  }
-  return best;
+// Takes a cut over; its cost, -1 where there are too many items.
+int64_t take_cut(RingGeom& gm, const ColumnCut& c) {
+  gm.segs = c.segs;
+  gm.seg_steps = c.seg_steps;
+  gm.items = c.items;
+  gm.items_per_wg = c.items_per_wg;
+  gm.wgs = c.wgs;
+  return c.items < 0 ? -1 : c.cost;
 }
 
 RingGeom ring_geom(const MfmaConvArgs& a) {
@@ -535,15 +522,14 @@ RingGeom ring_geom(const MfmaConvArgs& a) {
   const int64_t cols = (int64_t)gm.tiles_h * gm.tiles_w;
   const int64_t per_block = kComputeUnits > gm.nblocks ? kComputeUnits / gm.nblocks : 1;
   if (cols * a.n <= 0 || gm.steps <= 0) return gm;
-  const int64_t cost = ring_plan(gm, cols * a.n, per_block);
-  if (cost < 0) gm.items = -1;
+  const int64_t cost = take_cut(gm, cut_columns(cols * a.n, gm.steps, per_block));
   if (cost < 0 || a.n == 1 || per_block / a.n < 8) return gm;
   // Several samples, each by workgroups of its own: a workgroup's sums are then those of one sample, and the normalisation
   // behind the convolution needs no statistics pass. Where that ends no more than an eighth later, and a sample is more than
   // a few columns (the statistics pass of a smaller one is the same launch whatever it reads).
   RingGeom apart = gm;
   apart.parts = a.n;
-  const int64_t cost_apart = ring_plan(apart, cols, per_block / a.n);
+  const int64_t cost_apart = take_cut(apart, cut_columns(cols, gm.steps, per_block / a.n));
   return cost_apart > 0 && 8 * cost_apart <= 9 * cost && apart.wgs >= 8 ? apart : gm;
 }
 

@@ -629,23 +629,14 @@ struct Plan {
 // Rows of more than 16 voxels: the column-walking kernel where it serves them.
 bool ring_serves(const WgradArgs& a) { return mfma_wgrad_ring_applies(a); }
 
-// Rows of more than 16 voxels in a launch of their own: columns (rows in pieces of 32 voxels, 20 us before and behind its steps, 25 where
-// rows are cut) or 4x8x8 tiles in planes (less work on padding, a sooner start, a lower rate; where the blocks leave room for three
-// workgroups each). Times with the sum, of padded operations: 20 or 25 us + 0.7 a GFLOP and 12.5 us + 1.25, fitted to 35 problems of 32 to
-// 512 channels on 16x16x32 to 128^3. Tiles where both that estimate and the plan's own cost are below the columns': the plan knows what the
-// workgroup with the most tiles has to do (128 -> 256 at 19x29x23: 30 tiles in two slices of 32 blocks, 57 us, columns 46; two samples of 256 -> 256 at
-// 22x7x36 98 and 71), the estimate the rate of long slices (64 -> 256 at 32x62x33 205 and 171). Of 98 odd shapes, half of them where the two disagree,
-// 90 take the faster form or one 3 % slower; the worst, two samples of 128 -> 64 at 16x4x64, takes columns, 27.6 and 22.5. Columns -> tiles, us: 32 -> 32 channels at 32^3 21.6 -> 14.4, 64 -> 64 at 32^3 30.4 -> 24.1, at 16x32x32
-// 28.1 -> 17.0, at 41x80x34 63 -> 54, at 24x40x28 29.1 -> 21.1, 32 -> 32 at 36x63x66 33.6 -> 25.7, at 32x69x20 24.7 -> 16.4, at 38x25x55 25.8 -> 18.0, two samples
-// at 22x43x53 30.5 -> 23.7, at 44x60x75 49.9 -> 45.3, of 64 -> 128 at 20x33x19 42.3 -> 34.8; level where the line lies (32 -> 32 at 64^3 30.5 / 31.6), columns
-// past it: 96x80x112 65 / 72, 64^3 of 64 channels 62 / 80. Relative error against 64 bits, e-7: 32 -> 32 at 32^3 1.16 -> 1.13, at 48x64x64 1.54 -> 1.37,
-// 128 -> 128 at 9x20x20 0.96 -> 0.94.
-bool walks_columns(const WgradArgs& a, int64_t tile_plan_cost) {
-  const double per_voxel = 54e-9 * a.cin * a.cout * a.n;
-  const double columns = (a.ow % 32 == 0 ? 20. : 25.) + 0.7 * per_voxel * (double)cdiv(a.od, 2) * 2 * (double)cdiv(a.oh, 4) * 4 * (double)cdiv(a.ow, 32) * 32;
-  const double tiles = 12.5 + 1.25 * per_voxel * (double)cdiv(a.od, 4) * 4 * (double)cdiv(a.oh, 8) * 8 * (double)cdiv(a.ow, 8) * 8;
-  return columns <= tiles || 100 * columns <= (double)tile_plan_cost;
-}
+// Rows of more than 16 voxels in a launch of their own: columns (rows in pieces of 32 voxels) or 4x8x8 tiles in planes (less work on
+// padding, a sooner start, a lower rate; where the blocks leave room for three workgroups each). Both by what their busiest workgroup
+// has to do: columns 20 us and 2.1 a step or item, tiles by the tile plan's own cost, fitted to 150 problems of 32 to 512 channels on
+// 4x8x17 to 128^3, both forms timed: a measured time is within 5 % (rms) of either estimate, 144 of them take the faster form or one 3 %
+// slower, the worst is 128 -> 256 at 6x31x21 (columns 31.8, tiles 29.1). Columns / tiles, us: 32 -> 32 at 32^3 21.6 / 14.4, at 114x95x31 33.5 / 36.7, at 64^3
+// 28.4 / 29.7, at 96x80x112 54.3 / 71.0, two samples at 44x60x75 40.3 / 48.0, 64 -> 64 at 16x32x32 28.1 / 17.0, 128 -> 128 at 9x16x59 30.1 / 26.4, 256 -> 256 at
+// two samples of 6x9x40 45.6 / 64.7. Relative error against 64 bits, e-7: 32 -> 32 at 32^3 1.16 / 1.13, at 48x64x64 1.54 / 1.37, 128 -> 128 at 9x20x20 0.96 / 0.94.
+bool walks_columns(const WgradArgs& a, int64_t tile_plan_cost) { return 2000 + 210 * mfma_wgrad_ring_cost(a) <= tile_plan_cost; }
 
 Plan make_plan(const WgradArgs& a) {
   Plan p{};

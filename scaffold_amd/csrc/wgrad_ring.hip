@@ -25,6 +25,7 @@
 //     the workgroup writes one fp32 slice.
 #include <utility>
 
+#include "column_cut.hpp"
 #include "mma.hpp"
 #include "reduce.hpp"
 #include "wgrad_mfma.hpp"
@@ -171,6 +172,7 @@ struct WRingGeom {
   int tiles_h, tiles_w, steps, segs, seg_steps;
   int nblk_ci, nblk;                       // 32 x 32 blocks of (co, ci)
   int items, splits, items_per_split;      // items = columns x segments; a workgroup (split) takes consecutive ones
+  int64_t cost;                            // steps and items of the busiest one
 };
 
 struct WRingLane {
@@ -764,19 +766,15 @@ WRingGeom wring_geom(const WgradArgs& a) {
   gm.nblk_ci = a.cin / 32;
   gm.nblk = gm.nblk_ci * (a.cout / 32);
   const int64_t ncols = (int64_t)a.n * gm.tiles_h * gm.tiles_w;
-  int want = kComputeUnits / gm.nblk;  // workgroups per block: at most one workgroup per CU over all blocks
-  if (want < 1) want = 1;
-  int64_t segs = ncols >= want ? 1 : cdiv(want, ncols);
-  if (segs > gm.steps) segs = gm.steps;
-  gm.seg_steps = (int)cdiv(gm.steps, segs);
-  gm.segs = (int)cdiv(gm.steps, gm.seg_steps);
-  const int64_t items = ncols * gm.segs;
-  gm.items = items > 0x7fffffffLL ? -1 : (int)items;
-  if (gm.items > 0) {
-    if (want > gm.items) want = gm.items;
-    gm.items_per_split = (int)cdiv(gm.items, want);
-    gm.splits = (int)cdiv(gm.items, gm.items_per_split);
-  }
+  if (ncols <= 0 || gm.steps <= 0) return gm;
+  // workgroups per block: at most one workgroup per CU over all blocks
+  const ColumnCut c = cut_columns(ncols, gm.steps, kComputeUnits > gm.nblk ? kComputeUnits / gm.nblk : 1);
+  gm.segs = c.segs;
+  gm.seg_steps = c.seg_steps;
+  gm.items = c.items;
+  gm.items_per_split = c.items_per_wg;
+  gm.splits = c.wgs;
+  gm.cost = c.cost;
   return gm;
 }
 
@@ -857,6 +855,7 @@ bool mfma_wgrad_ring_applies(const WgradArgs& a) {
 }
 
 int mfma_wgrad_ring_splits(const WgradArgs& a) { return wring_geom(a).splits; }
+int64_t mfma_wgrad_ring_cost(const WgradArgs& a) { return wring_geom(a).cost; }
 
 int mfma_wgrad_ring(const WgradArgs& a, int dtype, const void* x, const void* gy, float* ws, hipStream_t st, const ChannelPair& x2) {
   const WRingGeom gm = wring_geom(a);
