@@ -94,7 +94,7 @@ typedef struct sfh_groupnorm_desc {
  * SFH_KERNEL_SPLIT (6) is a value sfh_conv3d_launch_geometry may report. Nothing removed or changed.
  * 105: SFH_FLAG_SHARE_DEVICE; sfh_conv3d_wgrad_batch_workspace_bytes takes the call's flags (changed: one more argument).
  * 106: sfh_conv3d_pack_master_weights added. 107: sfh_convT3d_fwd_padded, sfh_convT3d_wgrad_bias_padded,
- * sfh_groupnorm_fwd_pool added. */
+ * sfh_groupnorm_fwd_pool added. 108: sfh_groupnorm_bwd_pool added. */
 int sfh_version(void);
 const char* sfh_last_error(void);
 /* Fills name (<= name_len bytes), compute-unit count, LDS bytes per workgroup. */
@@ -401,6 +401,15 @@ int sfh_groupnorm_fwd_pool(const sfh_groupnorm_desc* p, const int32_t extents[3]
                            const void* gamma, const void* beta, void* y_slab, int64_t halo_rows, float* mean, float* rstd,
                            const float* partials, size_t partials_bytes, int32_t records, void* pooled_slab,
                            int64_t pooled_halo_elems, uint8_t* idx, void* stream);
+
+/* sfh_groupnorm_bwd for a result that was also pooled: its gradient is dy plus, in the voxel idx names of every 2x2x2 cell, dpooled
+ * (sfh_maxpool2_bwd_add's sum, rounded as it writes it), formed where the two passes read it. Same bits as the two calls. All three
+ * gradients and x in `dtype`; workspace as for sfh_groupnorm_bwd. 16-bit types on the vector path, extents of at least 2, groups past the
+ * size one workgroup takes; SFH_ERR_UNSUPPORTED otherwise, before any launch. */
+int sfh_groupnorm_bwd_pool(const sfh_groupnorm_desc* p, const int32_t extents[3], int dtype, int param_dtype, const void* dy,
+                           const void* dpooled, const uint8_t* idx, const void* x, const void* gamma, const void* beta,
+                           const float* mean, const float* rstd, void* dx, float* dgamma, float* dbeta, void* workspace,
+                           size_t workspace_bytes, void* stream);
 
 /* The forward for callers that cannot allocate: code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc. It has no counterpart in the reference. Same kernels and results as sfh_groupnorm_fwd, but the

@@ -161,6 +161,8 @@ _SIGNATURES = {
                                      c_void_p, c_size_t, c_uint32, c_void_p]),
     "sfh_groupnorm_fwd_pool": (c_int, [POINTER(GroupNormDesc), POINTER(c_int32), c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
                                        c_void_p, c_void_p, c_void_p, c_size_t, c_int32, c_void_p, c_int64, c_void_p, c_void_p]),
+    "sfh_groupnorm_bwd_pool": (c_int, [POINTER(GroupNormDesc), POINTER(c_int32), c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                       c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "sfh_groupnorm_fwd_workspace_bytes": (c_size_t, [POINTER(GroupNormDesc), c_int]),
     "sfh_groupnorm_fwd": (c_int, [POINTER(GroupNormDesc), c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),

@@ -300,7 +300,7 @@ __global__ void __launch_bounds__(256) stream_copy_kernel(const uint4* __restric
 
 using namespace sfh;
 
-extern "C" int sfh_version(void) { return 107; }
+extern "C" int sfh_version(void) { return 108; }
 
 extern "C" const char* sfh_last_error(void) { return g_error; }
 

@@ -23,6 +23,7 @@
 // set of channels) when C is a multiple of the vector width and the channels of a thread fall
 // into whole groups; the scalar path (one workgroup per (sample, group)) otherwise.
 #include <mutex>
+#include <type_traits>
 
 #include "common.hpp"
 #include "gn_stats.hpp"
@@ -746,15 +747,94 @@ __global__ void __launch_bounds__(kBlock) gn_normalize_pool(const T* __restrict_
   }
 }
 
+// ---- backward: what a pooling behind the normalisation adds to its gradient -------------------------------------------------
+// The gradient that reaches an encoder block's last normalisation is that of the skip connection plus, in the voxel of every
+// 2x2x2 cell that was the maximum, that of the pooled tensor: one sum, one rounding, as maxpool2_bwd_add writes it. The two passes
+// below form it where they read it, so it is never written: the pooled gradient and the indices (an eighth and a sixteenth of a tensor
+// each) come from the caches for seven of a cell's eight voxels. Same sums in the same order as over the written tensor, so both passes
+// stay with rows; bound by vector instructions as much as by memory (160 and 190 a row and 16-byte piece, 100 and 117 without), on half of the
+// chip (beside a batch of weight gradients) by them alone: no gain there and none lost. Pooling gradient and both passes -> the two, us, bf16: 32 channels of 64x128x128
+// 94 -> 71, 64 of 32x64x64 41 -> 37, 64 of 96x80x112 156 -> 129, 128 of 64^3 90 -> 72, 64 of 128^3 366 -> 272; the captured shard step 2796 -> 2780, a step
+// of 128^3 13370 -> 13290. The first pass leaving the sum for the second was no better: 80 at 64x128x128, 134 at 96x80x112.
+struct PooledGrad {
+  const void* g;       // N x pd x ph x pw x C
+  const uint8_t* idx;  // the same extents
+  int pd, ph, pw, H, W;
+  int step_w, step_h, step_d;  // the next row of a thread (rpp rows on), in voxels
+};
+
+struct NoPool {};  // of kernels without a pooling: nothing
+template <bool POOLED> using PoolArg = std::conditional_t<POOLED, PooledGrad, NoPool>;
+
+// One row's share. fetch() is for the row `c` stands on and moves `c` to the thread's next one.
+struct PooledCursor {
+  int w = 0, h = 0, d = 0;
+};
+template <typename T, bool POOLED>
+struct PooledRow {
+  __device__ __forceinline__ void fetch(const NoPool&, PooledCursor&, int, int, int, bool) {}
+  template <int V> __device__ __forceinline__ void add_to(float (&)[V]) const {}
+};
+template <typename T>
+struct PooledRow<T, true> {
+  Piece<T, 8> g;
+  uint2 which;
+  int k;  // the voxel's place in its cell; 8: the cell is not pooled, or the row is past the end
+  __device__ __forceinline__ void fetch(const PooledGrad& p, PooledCursor& c, int n, int C, int c0, bool live) {
+    const int pd = c.d >> 1, ph = c.h >> 1, pw = c.w >> 1;
+    const bool inside = live & (pd < p.pd) & (ph < p.ph) & (pw < p.pw);
+    // (24-bit products: a batch of at most 2^24 cells)
+    const uint32_t cell = __umul24(__umul24((uint32_t)(n * p.pd + pd), (uint32_t)p.ph) + (uint32_t)ph, (uint32_t)p.pw) + (uint32_t)pw;
+    const int64_t at = (int64_t)(inside ? cell : 0u) * C + c0;
+    g.load((const T*)p.g + at);
+    which = *reinterpret_cast<const uint2*>(p.idx + at);
+    k = inside ? (c.d & 1) * 4 + (c.h & 1) * 2 + (c.w & 1) : 8;
+    c.w += p.step_w;
+    int carry = c.w >= p.W ? 1 : 0;
+    c.w -= carry ? p.W : 0;
+    c.h += p.step_h + carry;
+    carry = c.h >= p.H ? 1 : 0;
+    c.h -= carry ? p.H : 0;
+    c.d += p.step_d + carry;
+  }
+  __device__ __forceinline__ void add_to(float (&v)[8]) const {
+    float f[8];
+    g.unpack(f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = ((int)(((e < 4 ? which.x : which.y) >> (8 * (e & 3))) & 0xff) == k ? f[e] : 0.f) + v[e];
+    Piece<T, 8> sum;
+    sum.q = pack_piece<T>(v);
+    sum.unpack(v);
+  }
+};
+template <bool POOLED>
+__device__ __forceinline__ PooledCursor pooled_cursor(const PoolArg<POOLED>& p, int64_t row) {
+  PooledCursor c;
+  if constexpr (POOLED) {
+    const uint32_t v = (uint32_t)row, t = v / (uint32_t)p.W;
+    c.w = (int)(v - t * (uint32_t)p.W);
+    c.d = (int)(t / (uint32_t)p.H);
+    c.h = (int)(t - (uint32_t)c.d * (uint32_t)p.H);
+  }
+  return c;
+}
+// The pooled share of the rows fetch_rows takes.
+template <int U, typename T, bool POOLED>
+__device__ __forceinline__ void fetch_pooled(PooledRow<T, POOLED> (&b)[U], const PoolArg<POOLED>& p, PooledCursor& c, int64_t row0, int64_t step,
+                                             int64_t end, int n, int C, int c0, bool active) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) b[u].fetch(p, c, n, C, c0, active && row0 + u * step < end);
+}
+
 // ---- backward: per-channel partial sums (vector path) --------------------------------------
 // part (floats): [N][nsplit][2][C]  with q = 0: sum dy'*xhat, q = 1: sum dy'
-template <typename T, typename TG, bool STREAM>
-__global__ void __launch_bounds__(kBlock) gn_bwd_partial(const T* __restrict__ x, const TG* __restrict__ dy,
+template <typename T, typename TG, bool STREAM, bool POOLED>
+__global__ void __launch_bounds__(kBlock, POOLED ? 4 : 1) gn_bwd_partial(const T* __restrict__ x, const TG* __restrict__ dy,
                                                          const float* __restrict__ mean, const float* __restrict__ rstd,
                                                          const void* __restrict__ gamma, const void* __restrict__ beta,
                                                          int param_dtype, float* __restrict__ part, float* __restrict__ gpart,
                                                          int64_t S, int C, int G, int tpr, int rpp, int nsplit,
-                                                         int64_t rows_per_split, int relu) {
+                                                         int64_t rows_per_split, int relu, PoolArg<POOLED> pool) {
   constexpr int V = VecOf<T>::N;
   extern __shared__ float smem[];  // 2 * V * kBlock | gamma[C]
   float* gam = smem + 2 * V * kBlock;
@@ -764,7 +844,7 @@ __global__ void __launch_bounds__(kBlock) gn_bwd_partial(const T* __restrict__ x
   const int r = tid / tpr, cv = tid - r * tpr;
   const bool active = r < rpp;
   // the workgroup's first rows are requested before the statistics and parameters they will be combined with
-  constexpr int U = 2;  // rows per batch: the next batch's loads are in flight while the current one is summed
+  constexpr int U = POOLED ? 1 : 2;  // rows per batch: the next batch's loads are in flight while the current one is summed
   const int64_t base = (int64_t)n * S * C + cv * V;
   const T* xs = x + base;
   const TG* gs = dy + base;
@@ -773,10 +853,13 @@ __global__ void __launch_bounds__(kBlock) gn_bwd_partial(const T* __restrict__ x
   if (end > S) end = S;
   const int64_t step = rpp;
   int64_t row = begin + r;
-  Piece<T, V> cx[U];
-  Piece<TG, V> cg_[U];
+  Piece<T, V> cx[U], nx[U];
+  Piece<TG, V> cg_[U], ng[U];
+  PooledRow<T, POOLED> cp[U], np[U];
+  PooledCursor at = pooled_cursor<POOLED>(pool, row);
   fetch_rows<STREAM>(cx, xs, row, step, end, begin, C, active);
   fetch_rows<STREAM>(cg_, gs, row, step, end, begin, C, active);
+  fetch_pooled(cp, pool, at, row, step, end, n, C, active ? cv * V : 0, active);
   float mu[V], rs[V], ga[V], be[V];
   load_params<V>(gamma, param_dtype, active ? cv * V : 0, 1.f, ga);
   load_params<V>(beta, param_dtype, active ? cv * V : 0, 0.f, be);
@@ -789,11 +872,55 @@ __global__ void __launch_bounds__(kBlock) gn_bwd_partial(const T* __restrict__ x
   float acc[2 * V];
 #pragma unroll
   for (int e = 0; e < 2 * V; ++e) acc[e] = 0.f;
-  if (active) {
+  if constexpr (POOLED) {
+    // Two rows are summed as below, but one is in flight while the other is worked on: with two more, a row being three pieces and its
+    // indices, a SIMD held three wavefronts instead of four.
+    auto gated = [&](const Piece<T, V>& px, const Piece<TG, V>& pg, const PooledRow<T, POOLED>& pp, float (&xh)[V], float (&d)[V]) {
+      float f[V];
+      px.unpack(f);
+      pg.unpack(d);
+      pp.add_to(d);
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        xh[e] = (f[e] - mu[e]) * rs[e];
+        d[e] = (fmaf(xh[e], ga[e], be[e]) <= 0.f) & (relu != 0) ? 0.f : d[e];  // (no branch per element)
+      }
+    };
+    if (active) {
+      while (row < end) {
+        const int64_t second = row + step, next = row + 2 * step;
+        float xh[V], d0[V];
+        if (second < end) {
+          fetch_rows<STREAM>(nx, xs, second, step, end, begin, C, true);
+          fetch_rows<STREAM>(ng, gs, second, step, end, begin, C, true);
+          fetch_pooled(np, pool, at, second, step, end, n, C, cv * V, true);
+        }
+        gated(cx[0], cg_[0], cp[0], xh, d0);
+#pragma unroll
+        for (int e = 0; e < V; ++e) acc[e] = fmaf(d0[e], xh[e], acc[e]);
+        if (second < end) {
+          if (next < end) {
+            fetch_rows<STREAM>(cx, xs, next, step, end, begin, C, true);
+            fetch_rows<STREAM>(cg_, gs, next, step, end, begin, C, true);
+            fetch_pooled(cp, pool, at, next, step, end, n, C, cv * V, true);
+          }
+          float d1[V];
+          gated(nx[0], ng[0], np[0], xh, d1);
+#pragma unroll
+          for (int e = 0; e < V; ++e) {
+            acc[e] = fmaf(d1[e], xh[e], acc[e]);
+            acc[V + e] += d0[e] + d1[e];
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < V; ++e) acc[V + e] += d0[e];
+        }
+        row = next;
+      }
+    }
+  } else if (active) {
     while (row < end) {
       const int64_t next = row + U * step;
-      Piece<T, V> nx[U];
-      Piece<TG, V> ng[U];
       if (next < end) {
         fetch_rows<STREAM>(nx, xs, next, step, end, begin, C, true);
         fetch_rows<STREAM>(ng, gs, next, step, end, begin, C, true);
@@ -989,14 +1116,14 @@ __global__ void __launch_bounds__(kFinalize) gn_bwd_finalize(const float* __rest
 // A = mean(dy'*gamma), B = mean(dy'*gamma*xhat) from them itself, and workgroups of sample 0 finish by summing the
 // per-channel partials of one channel each into dgamma / dbeta (samples and splits in index order): no finalize
 // launch. Otherwise gn_bwd_finalize has filled `coef` and the parameter gradients.
-template <typename T, typename TG, bool STREAM>
-__global__ void __launch_bounds__(kBlock) gn_dx(const T* __restrict__ x, const TG* __restrict__ dy, T* __restrict__ dx,
+template <typename T, typename TG, bool STREAM, bool POOLED>
+__global__ void __launch_bounds__(kBlock, POOLED ? 4 : 1) gn_dx(const T* __restrict__ x, const TG* __restrict__ dy, T* __restrict__ dx,
                                                 const float* __restrict__ mean, const float* __restrict__ rstd,
                                                 const void* __restrict__ gamma, const void* __restrict__ beta, int param_dtype,
                                                 const float* __restrict__ coef, const float* __restrict__ part,
                                                 const float* __restrict__ gpart, float* __restrict__ dgamma,
                                                 float* __restrict__ dbeta, int N, int64_t S, int C, int G, int tpr, int rpp,
-                                                int nsplit, int64_t rows_per_split, float m, int relu) {
+                                                int nsplit, int64_t rows_per_split, float m, int relu, PoolArg<POOLED> pool) {
   constexpr int V = VecOf<T>::N;
   extern __shared__ float gco[];  // sums[2 G] | fold scratch (4 * kBlock)
   __shared__ float red8[8];
@@ -1005,7 +1132,7 @@ __global__ void __launch_bounds__(kBlock) gn_dx(const T* __restrict__ x, const T
   const int cg = C / G;
   const int r = tid / tpr, cv = tid - r * tpr;
   // the workgroup's first rows are requested before anything else: the fold of the partials below reads other memory
-  constexpr int U = 2;  // rows per batch: the next batch's loads are in flight while the current one is worked on
+  constexpr int U = POOLED ? 1 : 2;  // rows per batch: the next batch's loads are in flight while the current one is worked on
   const int64_t base = (int64_t)n * S * C + cv * V;
   const T* xs = x + base;
   const TG* gs = dy + base;
@@ -1016,8 +1143,11 @@ __global__ void __launch_bounds__(kBlock) gn_dx(const T* __restrict__ x, const T
   int64_t row = begin + r;
   Piece<T, V> cx[U];
   Piece<TG, V> cg_[U];
+  PooledRow<T, POOLED> cp[U];
+  PooledCursor at = pooled_cursor<POOLED>(pool, row);
   fetch_rows<STREAM>(cx, xs, row, step, end, begin, C, r < rpp);
   fetch_rows<STREAM>(cg_, gs, row, step, end, begin, C, r < rpp);
+  fetch_pooled(cp, pool, at, row, step, end, n, C, r < rpp ? cv * V : 0, r < rpp);
   const bool fused = fold_in_consumer(G, nsplit);
   // The workgroup's share of the parameter gradients (the tail of this kernel) reads the per-channel partials of the
   // launch before: its first loads go out now, so that the tail does not start with a trip to memory of its own.
@@ -1063,9 +1193,11 @@ __global__ void __launch_bounds__(kBlock) gn_dx(const T* __restrict__ x, const T
     const int64_t next = row + U * step;
     Piece<T, V> nx[U];
     Piece<TG, V> ng[U];
+    PooledRow<T, POOLED> np[U];
     if (next < end) {
       fetch_rows<STREAM>(nx, xs, next, step, end, begin, C, true);
       fetch_rows<STREAM>(ng, gs, next, step, end, begin, C, true);
+      fetch_pooled(np, pool, at, next, step, end, n, C, cv * V, true);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -1073,6 +1205,7 @@ __global__ void __launch_bounds__(kBlock) gn_dx(const T* __restrict__ x, const T
         float f[V], g[V], o[V];
         cx[u].unpack(f);
         cg_[u].unpack(g);
+        cp[u].add_to(g);
 #pragma unroll
         for (int e = 0; e < V; ++e) {
           const float xh = (f[e] - mu[e]) * rs[e];
@@ -1088,6 +1221,7 @@ __global__ void __launch_bounds__(kBlock) gn_dx(const T* __restrict__ x, const T
       for (int u = 0; u < U; ++u) {
         cx[u] = nx[u];
         cg_[u] = ng[u];
+        cp[u] = np[u];
       }
     }
     row = next;
@@ -1585,6 +1719,31 @@ int fwd_typed(const sfh_groupnorm_desc& p, const GnPlan& pl, int param_dtype, co
   return check_launch("gn_normalize");
 }
 
+// The two passes of the vector path and what lies between them.
+template <typename T, typename TG, bool POOLED>
+int bwd_vector(const sfh_groupnorm_desc& p, const GnPlan& pl, int param_dtype, const void* dy, const void* x, const void* gamma, const void* beta,
+               const float* mean, const float* rstd, void* dx, float* dgamma, float* dbeta, float* coef, float* part, float* gpart,
+               const PoolArg<POOLED>& pool, hipStream_t st) {
+  const int G = p.groups, C = p.c;
+  const int64_t S = p.spatial;
+  constexpr int V = VecOf<T>::N;
+  const dim3 grid(pl.nsplit, p.n);
+  hipLaunchKernelGGL((pl.stream ? gn_bwd_partial<T, TG, true, POOLED> : gn_bwd_partial<T, TG, false, POOLED>), grid, dim3(kBlock), ((size_t)2 * V * kBlock + C) * sizeof(float), st, (const T*)x,
+                     (const TG*)dy, mean, rstd, gamma, beta, param_dtype, part, gpart, S, C, G, pl.tpr, pl.rpp, pl.nsplit,
+                     pl.rows_per_split, p.relu, pool);
+  if (int rc = check_launch("gn_bwd_partial")) return rc;
+  const float m = (float)S * (float)(C / G);
+  if (!fold_in_consumer_host(G, pl.nsplit)) {
+    hipLaunchKernelGGL(gn_bwd_finalize, dim3(p.n * G + (unsigned)cdiv(C, kFinalizeChannels)), dim3(kFinalize), 0, st, part, gamma, param_dtype, coef, dgamma, dbeta, p.n,
+                       C, G, pl.nsplit, m);
+    if (int rc = check_launch("gn_bwd_finalize")) return rc;
+  }
+  hipLaunchKernelGGL((pl.stream ? gn_dx<T, TG, true, POOLED> : gn_dx<T, TG, false, POOLED>), grid, dim3(kBlock), (size_t)(2 * G + 4 * kBlock) * sizeof(float), st, (const T*)x,
+                     (const TG*)dy, (T*)dx, mean, rstd, gamma, beta, param_dtype, coef, part, gpart, dgamma, dbeta, p.n, S, C, G,
+                     pl.tpr, pl.rpp, pl.nsplit, pl.rows_per_split, m, p.relu, pool);
+  return check_launch("gn_dx");
+}
+
 template <typename T, typename TG>
 int bwd_typed(const sfh_groupnorm_desc& p, const GnPlan& pl, int param_dtype, const void* dy, const void* x, const void* gamma,
               const void* beta, const float* mean, const float* rstd, void* dx, float* dgamma, float* dbeta, float* ws,
@@ -1619,22 +1778,7 @@ int bwd_typed(const sfh_groupnorm_desc& p, const GnPlan& pl, int param_dtype, co
 #undef SFH_GN_SMALL
     return check_launch("gn_small_bwd");
   }
-  constexpr int V = VecOf<T>::N;
-  const dim3 grid(pl.nsplit, p.n);
-  hipLaunchKernelGGL((pl.stream ? gn_bwd_partial<T, TG, true> : gn_bwd_partial<T, TG, false>), grid, dim3(kBlock), ((size_t)2 * V * kBlock + C) * sizeof(float), st, (const T*)x,
-                     (const TG*)dy, mean, rstd, gamma, beta, param_dtype, part, gpart, S, C, G, pl.tpr, pl.rpp, pl.nsplit,
-                     pl.rows_per_split, p.relu);
-  if (int rc = check_launch("gn_bwd_partial")) return rc;
-  const float m = (float)S * (float)(C / G);
-  if (!fold_in_consumer_host(G, pl.nsplit)) {
-    hipLaunchKernelGGL(gn_bwd_finalize, dim3(p.n * G + (unsigned)cdiv(C, kFinalizeChannels)), dim3(kFinalize), 0, st, part, gamma, param_dtype, coef, dgamma, dbeta, p.n,
-                       C, G, pl.nsplit, m);
-    if (int rc = check_launch("gn_bwd_finalize")) return rc;
-  }
-  hipLaunchKernelGGL((pl.stream ? gn_dx<T, TG, true> : gn_dx<T, TG, false>), grid, dim3(kBlock), (size_t)(2 * G + 4 * kBlock) * sizeof(float), st, (const T*)x,
-                     (const TG*)dy, (T*)dx, mean, rstd, gamma, beta, param_dtype, coef, part, gpart, dgamma, dbeta, p.n, S, C, G,
-                     pl.tpr, pl.rpp, pl.nsplit, pl.rows_per_split, m, p.relu);
-  return check_launch("gn_dx");
+  return bwd_vector<T, TG, false>(p, pl, param_dtype, dy, x, gamma, beta, mean, rstd, dx, dgamma, dbeta, coef, part, gpart, NoPool{}, st);
 }
 
 }  // namespace
@@ -1818,6 +1962,38 @@ extern "C" size_t sfh_groupnorm_bwd_workspace_bytes(const sfh_groupnorm_desc* p,
   if (check_desc(p, x_dtype) != SFH_OK) return 0;
   const GnPlan pl = make_plan(*p, x_dtype, true);
   return align_up(bwd_ws_floats(*p, pl) * sizeof(float), 256);
+}
+
+extern "C" int sfh_groupnorm_bwd_pool(const sfh_groupnorm_desc* p, const int32_t extents[3], int dtype, int param_dtype, const void* dy,
+                                      const void* dpooled, const uint8_t* idx, const void* x, const void* gamma, const void* beta, const float* mean,
+                                      const float* rstd, void* dx, float* dgamma, float* dbeta, void* workspace, size_t workspace_bytes,
+                                      void* stream) {
+  if (int rc = check_desc(p, dtype)) return rc;
+  if (!dtype_ok(param_dtype)) return fail(SFH_ERR_INVALID, "groupnorm: bad param dtype");
+  if (dy == nullptr || dpooled == nullptr || idx == nullptr || x == nullptr || dx == nullptr || mean == nullptr || rstd == nullptr || extents == nullptr)
+    return fail(SFH_ERR_INVALID, "groupnorm bwd with pooling: null tensor");
+  for (int i = 0; i < 3; ++i)
+    if (extents[i] < 1) return fail(SFH_ERR_INVALID, "groupnorm bwd with pooling: bad extents");
+  if ((int64_t)extents[0] * extents[1] * extents[2] != p->spatial)
+    return fail(SFH_ERR_INVALID, "groupnorm bwd with pooling: the extents are not the descriptor's");
+  const GnPlan pl = make_plan(*p, dtype, aligned16(x) && aligned16(dy) && aligned16(dx) && aligned16(dpooled));
+  // (a group that one workgroup holds has a launch of its own, which reads a gradient that is written)
+  if (dtype == SFH_FP32 || !pl.vector || (reinterpret_cast<uintptr_t>(idx) & 7u) != 0 || extents[0] < 2 || extents[1] < 2 || extents[2] < 2 ||
+      p->spatial > 0x7fffffffLL || (int64_t)p->n * (extents[0] / 2) * (extents[1] / 2) * (extents[2] / 2) > 1 << 24 ||
+      small_groups(*p, pl, true).threads > 0)
+    return fail(SFH_ERR_UNSUPPORTED, "groupnorm bwd with pooling: 16-bit types on the vector path, cells on every axis, at most 2^24, groups past one workgroup");
+  const size_t need = bwd_ws_floats(*p, pl) * sizeof(float);
+  if (workspace == nullptr || workspace_bytes < need)
+    return fail(SFH_ERR_WORKSPACE, "groupnorm bwd: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+  const PooledGrad pool{dpooled, idx, extents[0] / 2, extents[1] / 2, extents[2] / 2, extents[1], extents[2],
+                        pl.rpp % extents[2], pl.rpp / extents[2] % extents[1], pl.rpp / extents[2] / extents[1]};
+  float* coef = (float*)workspace;
+  float* part = coef + align_up((size_t)p->n * p->groups * 2, 4);
+  float* gpart = part + align_up((size_t)p->n * pl.nsplit * 2 * p->c, 4);
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == SFH_BF16)
+    return bwd_vector<bf16_t, bf16_t, true>(*p, pl, param_dtype, dy, x, gamma, beta, mean, rstd, dx, dgamma, dbeta, coef, part, gpart, pool, st);
+  return bwd_vector<fp16_t, fp16_t, true>(*p, pl, param_dtype, dy, x, gamma, beta, mean, rstd, dx, dgamma, dbeta, coef, part, gpart, pool, st);
 }
 
 extern "C" int sfh_groupnorm_bwd(const sfh_groupnorm_desc* p, int x_dtype, int dy_dtype, int param_dtype, const void* dy,

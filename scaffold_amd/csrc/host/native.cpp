@@ -993,15 +993,17 @@ py::object conv_transpose(const Tensor& x_in, const Tensor& weight, const MaybeT
 // ---- GroupNorm -----------------------------------------------------------------------------------------------------------
 // What the backward of GroupNorm (+ ReLU) needs.
 struct NormSaved {
-  Kept input, weight, bias, stats;
+  Kept input, weight, bias, stats, idx;  // idx: where the pooled result's maxima lie (undefined: the result was not pooled)
   int groups = 1;
   bool relu = false;
-  void release() { input.reset(); weight.reset(); bias.reset(); stats.reset(); }
-  void backward(const Tensor& grad, Tensor& dx, Tensor& dw, Tensor& db) {
-    const Tensor x = input.volume(), st = stats.flat();
+  void release() { input.reset(); weight.reset(); bias.reset(); stats.reset(); idx.reset(); }
+  // grad / pooled: of the result and of what the same launch pooled from it (either may be undefined)
+  void backward(const Tensor& grad, const Tensor& pooled, Tensor& dx, Tensor& dw, Tensor& db) {
+    const Tensor x = input.volume(), st = stats.flat(), ix = pooled.defined() ? idx.flat() : Tensor();
     Tensor w = weight.flat(), b = bias.flat();
-    Tensor gy = dense(grad);
-    if (gy.scalar_type() != x.scalar_type() && gy.scalar_type() != at::kFloat) gy = gy.to(x.scalar_type());
+    Tensor gy = grad.defined() ? dense(grad) : Tensor(), gp = pooled.defined() ? dense(pooled) : Tensor();
+    if (gp.defined() && gp.scalar_type() != x.scalar_type()) gp = gp.to(x.scalar_type());
+    if (gy.defined() && gy.scalar_type() != x.scalar_type() && (gp.defined() || gy.scalar_type() != at::kFloat)) gy = gy.to(x.scalar_type());
     const Tensor w_in = w, b_in = b;
     if (w.defined() && b.defined() && w.scalar_type() != b.scalar_type()) b = b.to(w.scalar_type());
     c10::OptionalDeviceGuard guard(x.device());
@@ -1012,10 +1014,27 @@ struct NormSaved {
     if (w.defined()) dw = plain({c}, x, at::kFloat);
     if (b.defined()) db = plain({c}, x, at::kFloat);
     const Tensor ws = bytes(sfh_groupnorm_bwd_workspace_bytes(&d, code), x);
+    const size_t ws_bytes = ws.defined() ? (size_t)ws.numel() : 0;
     const float* mean = (const float*)ptr(st);
-    check(sfh_groupnorm_bwd(&d, code, code_of(gy.scalar_type()), code_of(w.defined() ? w.scalar_type() : b.defined() ? b.scalar_type() : x.scalar_type()),
-                            ptr(gy), ptr(x), ptr(w), ptr(b), mean, mean + n * groups, out_ptr(dx), (float*)out_ptr(dw), (float*)out_ptr(db), out_ptr(ws),
-                            ws.defined() ? (size_t)ws.numel() : 0, stream_of(x)), "group_norm_backward");
+    const int pcode = code_of(w.defined() ? w.scalar_type() : b.defined() ? b.scalar_type() : x.scalar_type());
+    int rc = SFH_ERR_UNSUPPORTED;
+    if (gp.defined() && gy.defined()) {
+      const int32_t extents[3] = {(int32_t)x.size(2), (int32_t)x.size(3), (int32_t)x.size(4)};
+      rc = sfh_groupnorm_bwd_pool(&d, extents, code, pcode, ptr(gy), ptr(gp), (const uint8_t*)ptr(ix), ptr(x), ptr(w), ptr(b), mean, mean + n * groups,
+                                  out_ptr(dx), (float*)out_ptr(dw), (float*)out_ptr(db), out_ptr(ws), ws_bytes, stream_of(x));
+    }
+    if (rc == SFH_ERR_UNSUPPORTED) {
+      if (gp.defined()) {  // the sum of the two gradients in a launch of its own
+        const sfh_pool_desc pd{(int32_t)n, (int32_t)c, (int32_t)x.size(2), (int32_t)x.size(3), (int32_t)x.size(4)};
+        Tensor sum = volume(x.sizes(), x, x.scalar_type());
+        check(gy.defined() ? sfh_maxpool2_bwd_add(&pd, code, ptr(gp), (const uint8_t*)ptr(ix), ptr(gy), out_ptr(sum), stream_of(x))
+                           : sfh_maxpool2_bwd(&pd, code, ptr(gp), (const uint8_t*)ptr(ix), out_ptr(sum), stream_of(x)), "max_pool3d_2x backward");
+        gy = sum;
+      }
+      rc = sfh_groupnorm_bwd(&d, code, code_of(gy.scalar_type()), pcode, ptr(gy), ptr(x), ptr(w), ptr(b), mean, mean + n * groups, out_ptr(dx),
+                             (float*)out_ptr(dw), (float*)out_ptr(db), out_ptr(ws), ws_bytes, stream_of(x));
+    }
+    check(rc, "group_norm_backward");
     if (dw.defined() && dw.scalar_type() != w_in.scalar_type()) dw = dw.to(w_in.scalar_type());
     if (db.defined() && db.scalar_type() != b_in.scalar_type()) db = db.to(b_in.scalar_type());
   }
@@ -1138,7 +1157,7 @@ struct GroupNormNode : public LaunchNode {  // edges: input, weight, bias
   void release_variables() override { saved.release(); }
   variable_list backward(variable_list& grads) override {
     variable_list out(3);
-    if (grads[0].defined()) saved.backward(grads[0], out[0], out[1], out[2]);
+    if (grads[0].defined()) saved.backward(grads[0], Tensor(), out[0], out[1], out[2]);
     return out;
   }
 };
@@ -1173,16 +1192,17 @@ py::object group_norm(const Tensor& input, int64_t groups, const MaybeTensor& we
 // ---- a convolution and the GroupNorm that reads it -----------------------------------------------------------------------
 // One call and one node for the pair every block of the U-Net is made of (bias-free convolution): half of the module calls
 // and of the nodes of a pass.
-struct ConvNormNode : public LaunchNode {  // edges: x, convolution weight, norm weight, norm bias
+struct ConvNormNode : public LaunchNode {  // edges: x, convolution weight, norm weight, norm bias; the second output, if any: what was pooled
   ConvSaved conv;
   NormSaved norm;
   std::string name() const override { return "ScaffoldConvGroupNormBackward"; }
   void release_variables() override { conv.release(); norm.release(); }
   variable_list backward(variable_list& grads) override {
     variable_list out(4);
-    if (!grads[0].defined()) return out;
+    const Tensor pooled = grads.size() > 1 ? grads[1] : Tensor();
+    if (!grads[0].defined() && !pooled.defined()) return out;
     Tensor gy, c[4];
-    norm.backward(grads[0], gy, out[2], out[3]);
+    norm.backward(grads[0], pooled, gy, out[2], out[3]);
     conv.backward(gy, task_should_compute_output(0), task_should_compute_output(1), false, false, c);
     out[0] = c[0];
     out[1] = c[1];
@@ -1192,7 +1212,7 @@ struct ConvNormNode : public LaunchNode {  // edges: x, convolution weight, norm
 
 // modules.conv_then_norm: (y, slab or None, pooled), or None (nothing launched) for a call that is not served as it stands.
 // x / x_read, weight / w, packed forms, halo, master, family and early as in record_conv.  `pool_halo` >= 0: a MaxPool3d(2) with that
-// halo follows; pooled is what it will ask for (tensor, slab or None, indices or None), or None where this launch does not make it.
+// halo follows; pooled is its result (tensor, slab or None), differentiable as y is, or None where this launch does not make it.
 py::object conv_norm(const Tensor& x, const Tensor& x_read, const Tensor& weight, const Tensor& w, const MaybeTensor& packed_fwd, const MaybeTensor& packed_dgrad,
                      int64_t halo, py::handle stride, py::handle padding, py::handle dilation, bool master, int family, bool early, int64_t groups,
                      const Tensor& norm_weight, const Tensor& norm_bias, double eps, bool relu, int64_t out_halo, int64_t pool_halo) {
@@ -1214,6 +1234,7 @@ py::object conv_norm(const Tensor& x, const Tensor& x_read, const Tensor& weight
         !launch_norm_pool(c.y, groups, norm_weight, norm_bias, eps, relu, out_halo, c.partials, c.records, pool_halo, graph, r, pool))
       r = launch_norm(c.y, groups, norm_weight, norm_bias, eps, relu, c.y.scalar_type(), out_halo, c.records > 0 ? c.partials : Tensor(), c.records);
     if (graph && r.slab.defined()) r.y = r.y.detach();
+    if (graph && pool.slab.defined()) pool.pooled = pool.pooled.detach();
   }
   if (graph) {
     auto node = new_node<ConvNormNode>();
@@ -1223,9 +1244,11 @@ py::object conv_norm(const Tensor& x, const Tensor& x_read, const Tensor& weight
     std::memcpy(node->conv.d, d, sizeof(d));
     save_conv(node->conv, x, x_read, w, or_none(packed_dgrad), halo, master, family > 0 ? weight : Tensor(), family, early);
     save_norm(node->norm, c.y, norm_weight, norm_bias, r.stats, groups, relu);
+    node->norm.idx.keep(pool.idx);
     torch::autograd::set_history(r.y, node);
+    if (pool.pooled.defined()) torch::autograd::set_history(pool.pooled, node);
   }
-  const py::object pooled = pool.pooled.defined() ? py::object(py::make_tuple(pool.pooled, tensor_or_none(pool.slab), tensor_or_none(pool.idx))) : py::none();
+  const py::object pooled = pool.pooled.defined() ? py::object(py::make_tuple(pool.pooled, tensor_or_none(pool.slab))) : py::none();
   return py::make_tuple(r.y, tensor_or_none(r.slab), pooled);
 }
 
@@ -1259,9 +1282,8 @@ struct MaxPoolNode : public LaunchNode {  // edge: x; the second output, where t
   }
 };
 
-// pooling.max_pool3d_2x: (y, slab or None[, alias of x]), or None for a call that is not served.  `given`: what the producer of x_in
-// has pooled from these very bits, for this halo (a call that needs indices it did not keep launches).
-py::object max_pool(const Tensor& x_in, int64_t halo, bool with_skip, const MaybeTensor& given, const MaybeTensor& given_slab, const MaybeTensor& given_idx) {
+// pooling.max_pool3d_2x: (y, slab or None[, alias of x]), or None for a call that is not served.
+py::object max_pool(const Tensor& x_in, int64_t halo, bool with_skip) {
   if (x_in.dim() != 5 || !on_gpu(x_in) || code_of(x_in.scalar_type()) < 0 || x_in.size(1) < 1) return py::none();
   for (int i = 2; i < 5; ++i)
     if (x_in.size(i) < 1) return py::none();
@@ -1273,16 +1295,11 @@ py::object max_pool(const Tensor& x_in, int64_t halo, bool with_skip, const Mayb
     const Tensor x = dense(x_in);
     c10::OptionalDeviceGuard guard(x.device());
     const int64_t n = z[0], c = z[1], d2 = z[2] / 2, h2 = z[3] / 2, w2 = z[4] / 2;
-    const bool made = given.has_value() && (!graph || given_idx.has_value());
-    idx = made ? or_none(given_idx) : plain({n, d2, h2, w2, c}, x, at::kByte);
+    idx = plain({n, d2, h2, w2, c}, x, at::kByte);
     const sfh_pool_desc d{(int32_t)n, (int32_t)c, (int32_t)z[2], (int32_t)z[3], (int32_t)z[4]};
     const int code = code_of(x.scalar_type());
     int rc = SFH_ERR_UNSUPPORTED;
-    if (made) {
-      y = *given;
-      slab = or_none(given_slab);
-      rc = SFH_OK;
-    } else if (halo > 0 && n == 1 && d2 > 0 && h2 > 0 && w2 > 0) {
+    if (halo > 0 && n == 1 && d2 > 0 && h2 > 0 && w2 > 0) {
       slab = volume({1, c, d2 + 2 * halo, h2, w2}, x, x.scalar_type());
       rc = sfh_maxpool2_fwd_slab(&d, code, ptr(x), out_ptr(slab), halo * h2 * w2 * c, (uint8_t*)out_ptr(idx), stream_of(x));
       if (rc != SFH_ERR_UNSUPPORTED) y = slab.narrow(2, halo, d2);

@@ -31,18 +31,14 @@ def _refuse(x):
     raise NotImplementedError(f"unsupported: x={tuple(getattr(x, 'shape', ()))}/{getattr(x, 'dtype', None)}")
 
 
-def _pool(x, out_halo, with_skip, given=None):
-    """The launch and its autograd node: ``(pooled, ...)``; the pooled tensor carries the slab it lies in, if any.  ``given``:
-    what the launch that made ``x`` has pooled already, ``(pooled, slab, indices, halo)``, which is then taken in the launch's place."""
+def _pool(x, out_halo, with_skip):
+    """The launch and its autograd node: ``(pooled, ...)``; the pooled tensor carries the slab it lies in, if any."""
     done = None
     if isinstance(x, torch.Tensor):
         # What a producer left on its result is never taken from there: by now the result may have been written past its version
         # counter, and the pooled tensor belongs to the stream and the capture it was made in.
         x.__dict__.pop("_sfh_pooled", None)
-        y, slab, idx, halo = given or (None, None, None, -1)
-        if halo != int(out_halo):
-            y = slab = idx = None
-        done = _lib.native().max_pool(x, int(out_halo), with_skip, y, slab, idx)
+        done = _lib.native().max_pool(x, int(out_halo), with_skip)
     if done is None:
         _refuse(x)
     if done[1] is not None:
@@ -52,12 +48,18 @@ def _pool(x, out_halo, with_skip, given=None):
 
 def max_pool3d_2x_with_skip(x: torch.Tensor, out_halo: int = 0, _given=None):
     """``(F.max_pool3d(x, 2), x)``: use the returned ``x`` for the skip connection and the gradients of both uses are
-    combined in one kernel (same values as autograd's own addition: one fp32 sum, one rounding)."""
+    combined in one kernel (same values as autograd's own addition: one fp32 sum, one rounding).  ``_given``: what the launch that
+    made ``x`` has pooled, ``(pooled, slab, halo)``, a result of the same node: both gradients meet there."""
     if not is_supported_pool(x):
         _refuse(x)
     if not x.is_contiguous(memory_format=_CL3D) or _lib.under_transform():
         return max_pool3d_2x(x, out_halo), x
-    pooled, _, skip = _pool(x, out_halo, True, _given)
+    if _given is not None and _given[2] == int(out_halo):
+        pooled, slab, halo = _given
+        if slab is not None:
+            pooled._sfh_slab = (slab, halo)
+        return pooled, x
+    pooled, _, skip = _pool(x, out_halo, True)
     slab = getattr(x, "_sfh_slab", None)
     if slab is not None:  # the alias is the same memory: still the interior of the slab its producer wrote it into
         skip._sfh_slab = slab

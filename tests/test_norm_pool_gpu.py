@@ -174,6 +174,33 @@ def test_handed_over_is_the_launched_one(device, n, c, spatial, halo):
     assert all(torch.equal(a, b) for a, b in zip(*results))
 
 
+@pytest.mark.parametrize("relu", [True, False])
+@pytest.mark.parametrize("n,c,spatial,dtype", [
+    (1, 32, (9, 35, 70), torch.float16),       # odd planes, several workgroups, two rows a thread at once
+    (2, 64, (5, 7, 9), torch.bfloat16),        # two samples, less than one pass a workgroup
+    (1, 64, (34, 64, 66), torch.bfloat16),     # several passes
+    (1, 256, (2, 40, 3), torch.bfloat16),      # one cell deep and wide
+    (1, 512, (3, 8, 8), torch.bfloat16),       # a group that one workgroup holds: summed before it
+])
+def test_gradients_meet_in_the_normalisation(device, n, c, spatial, dtype, relu):
+    """The skip connection's gradient, the pooled tensor's, and both, through the launch that made the two and through a pooling of
+    its own: the same bits."""
+    conv, norm = _pair(c, device, dtype, relu)
+    norm.pool_next = 0
+    pool = FastMaxPool3d(2)
+    x0 = torch.randn(n, c, *spatial, device=device).to(dtype).contiguous(memory_format=CL)
+    gp, gs = (torch.randn(n, c, *s, device=device).to(dtype).contiguous(memory_format=CL) for s in ([v // 2 for v in spatial], spatial))
+    for used in ("both", "skip", "pooled"):
+        results = []
+        for take in (True, False):
+            x = x0.clone().requires_grad_(True)
+            y = conv_then_norm(conv, norm, x)
+            given = y.__dict__.pop("_sfh_pooled")
+            outs, grads = zip(*[p for k, p in zip(("pooled", "skip"), zip(pool.with_skip(y, given if take else None), (gp, gs))) if used in ("both", k)])
+            results.append(torch.autograd.grad(outs, (x, conv.weight, norm.weight, norm.bias), grads))
+        assert all(torch.equal(a, b) for a, b in zip(*results)), used
+
+
 def test_a_captured_pooling_reads_its_input(device):
     conv, norm = _pair(64, device, torch.bfloat16)
     norm.pool_next = 0
