@@ -444,6 +444,24 @@ int64_t tiles_of(const MfmaConvArgs& a, int cls, int size) {
   return (int64_t)a.n * cdiv(a.od, t[0]) * cdiv(a.oh, t[1]) * cdiv(a.ow, t[2]);
 }
 
+// What a launch of one brick shape takes, in hundredths of a us: {start of the launch, of a 32-channel chunk; 512 voxels of one block by rounds
+// of workgroups, by rounds counted with fractions; a round}. Fitted to 470 forward problems of 64 to 1024 channels on the levels of
+// networks of 16x24x24 to 128^3, one and two samples, every shape timed unsliced: 2.4 to 4.6 % (rms). Slices add the launch that sums them and its bytes.
+constexpr int kBrickTime[3][2][2][5] = {  // [row class][size][blocks - 1]
+    {{{463, 59, 330, 167, 139}, {257, 216, 332, 107, 332}}, {{301, 131, 381, 142, 120}, {236, 143, 388, 103, 174}}},
+    {{{358, 59, 330, 114, 225}, {157, 191, 334, 70, 437}}, {{289, 136, 366, 110, 163}, {136, 174, 365, 69, 266}}},
+    {{{398, 76, 436, 82, 176}, {241, 109, 360, 75, 345}}, {{294, 120, 413, 90, 144}, {172, 141, 381, 76, 215}}},
+};
+int64_t brick_time(const MfmaConvArgs& a, const GatherPlan& p) {
+  const int* t = kTileDims[p.shape / 3][p.shape % 3];
+  const int* c = kBrickTime[p.shape / 3][p.shape % 3][p.nsub - 1];
+  const int64_t wgs = p.tiles * (a.cout / (32 * p.nsub)) * p.ksplit, chunks = cdiv(a.cred / kChunk, p.ksplit);
+  const int64_t rounds = cdiv(wgs, kComputeUnits), blocks = (int64_t)t[0] * t[1] * t[2] * p.nsub;  // voxels x blocks
+  int64_t time = c[0] + c[4] * rounds + chunks * (c[1] + blocks * (c[2] * rounds * kComputeUnits + c[3] * wgs) / (512 * kComputeUnits));
+  if (p.ksplit > 1) time += 500 + (int64_t)a.n * a.od * a.oh * a.ow * a.cout * p.ksplit * 4 * 40 / 1000000;
+  return time;
+}
+
 // Launch geometry, a pure function of the problem. The row length picks the brick's row class; then, among 512- and
 // 256-voxel tiles with one or two 32-channel output blocks per workgroup, the choice that loads the busiest CU least:
 // workgroups are dealt round-robin, so that CU gets ceil(workgroups / CUs) of them, each worth tile voxels x blocks.
@@ -453,7 +471,7 @@ int64_t tiles_of(const MfmaConvArgs& a, int cls, int size) {
 // 512-voxel tiles from costing a whole round. When even the small tiles leave CUs idle (the deep, small-volume levels)
 // the reduction channels are cut into at most 8 slices that are summed afterwards: a power of two, no more than would
 // give every CU a workgroup (more slices cost more in fp32 partials than they gain).
-GatherPlan gather_plan(const MfmaConvArgs& a) {
+GatherPlan cut_plan(const MfmaConvArgs& a) {
   GatherPlan p{};
   const int cls = a.ow > 16 ? 0 : (a.ow > 8 ? 1 : 2);
   const int ncc = a.cred / kChunk;
@@ -498,6 +516,25 @@ GatherPlan gather_plan(const MfmaConvArgs& a) {
     const int64_t room = kComputeUnits / best_wgs;
     while (p.ksplit * 2 <= room && p.ksplit * 2 <= ncc && p.ksplit < 8) p.ksplit *= 2;
   }
+  return p;
+}
+
+// The rule above knows rounds of workgroups and not what they hold: a launch of one round and a bit, or of bricks cut on several axes,
+// may be sooner done in another shape. Where the times say so by a twentieth (unsliced launches: a sum's order does not depend on the
+// brick). us: 64 -> 64 at 55x28x41 29.2 -> 23.2, at 51x60x31 28.1 -> 25.0, 128 -> 128 at 29x61x35 76 -> 68, 64 -> 128 at two samples of 100x43x72 242 -> 235.
+GatherPlan gather_plan(const MfmaConvArgs& a) {
+  GatherPlan p = cut_plan(a);
+  if (p.ksplit > 1 || p.tiles == 0) return p;
+  int64_t best = brick_time(a, p) * 95 / 100;
+  for (int cls = a.ow > 16 ? 0 : (a.ow > 8 ? 1 : 2); cls < 3; ++cls)
+    for (int size = 0; size < 2; ++size)
+      for (int nsub = 1; nsub <= (a.cout % 64 == 0 ? 2 : 1); ++nsub) {
+        const GatherPlan q{cls * 3 + size, nsub, 1, tiles_of(a, cls, size), p.cost};
+        const int64_t time = brick_time(a, q);
+        if (time >= best) continue;
+        best = time;
+        p = q;
+      }
   return p;
 }
 
@@ -715,7 +752,8 @@ size_t mfma_conv_partial_bytes(const MfmaConvArgs& a) {
   return align_up((size_t)p.ksplit * a.n * a.od * a.oh * a.ow * a.cout * sizeof(float), 256);
 }
 
-int64_t mfma_conv_brick_cost(const MfmaConvArgs& a) { return gather_plan(a).cost; }
+int64_t mfma_conv_brick_cost(const MfmaConvArgs& a) { return cut_plan(a).cost; }
+int64_t mfma_conv_brick_time(const MfmaConvArgs& a) { return brick_time(a, gather_plan(a)); }
 
 MfmaConvGeometry mfma_conv_gather_geometry(const MfmaConvArgs& a) {
   if (mfma_conv_wide_applies(a)) return mfma_conv_wide_geometry(a);
