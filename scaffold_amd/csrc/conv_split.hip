@@ -6,7 +6,7 @@
 // reduction is cut into slices, and slices that meet in memory cost fp32 partial tiles written and read plus a launch
 // of their own. Here the reduction is cut INSIDE the workgroup:
 //
-//   * A workgroup owns a brick of only 2 x 4 x 8 = 64 output voxels and 64 produced channels -- four 32-voxel x
+//   * A workgroup owns a brick of only 64 output voxels (2 x 4 x 8, 4 x 4 x 4 or 2 x 2 x 16) and 64 produced channels -- four 32-voxel x
 //     32-channel accumulator blocks -- so even a level of 2048 voxels has 32 x Cout/64 of them; where those would leave
 //     half of the CUs idle, 32 produced channels.
 //   * Its four wavefronts split the REDUCTION, not the voxels: a round stages the halo bricks of R 32-channel chunks
@@ -31,33 +31,39 @@ namespace sfh {
 namespace {
 
 constexpr int kChunk = 32;
-constexpr int TD = 2, TH = 4, TW = 8;  // output brick: two planes of 4 x 8 voxels, each one MFMA column block
-constexpr int BD = TD + 2, BH = TH + 2, BW = TW + 2;
-constexpr int BV = BD * BH * BW;  // 240 brick voxels with the halo
+constexpr int kBrickVoxels = 64;
 constexpr int MS = 2, kBlocks = 2;                              // accumulator blocks: voxel halves x at most two channel blocks
 constexpr int TAPS = 27, NIT = TAPS * 2, FRAG = 512;
-// LDS of a chunk's brick, NSUB channel blocks to a workgroup: row pitch, channel plane (64 modulo 256), chunk slot. A fragment
-// read covers two rows at a time; 128 modulo 256 apart they share no bank. Two workgroups to a CU (NSUB = 2) have no room
-// for that pitch, and do not miss it; alone on its CU one reads 5 % faster (13.8 -> 13.1 us at 256 -> 256, 8x16x16).
-template <int NSUB>
+// An output brick of 64 voxels: half ms is its voxels 32 ms .. 32 ms + 31 in memory order. PITCH: of its rows in LDS where a workgroup has one
+// channel block. LDS of a chunk's brick, NSUB channel blocks to a workgroup: row pitch, channel plane (64 modulo 256), chunk slot. A fragment
+// read covers sixteen voxels at a time: two rows of 8, 128 modulo 256 apart, four of 4, 64 apart, or one of 16 share no bank. Two workgroups to a
+// CU (NSUB = 2) have no room for that pitch, and do not miss it; alone on its CU one reads 5 % faster (13.8 -> 13.1 us at 256 -> 256, 8x16x16).
+template <int TD_, int TH_, int TW_, int PITCH_>
+struct Shape {
+  static constexpr int TD = TD_, TH = TH_, TW = TW_, PITCH = PITCH_;
+  static constexpr int BD = TD + 2, BH = TH + 2, BW = TW + 2, BV = BD * BH * BW;  // with the halo
+  static_assert(TD * TH * TW == kBrickVoxels && PITCH >= BW * 16, "two blocks of 32 voxels");
+};
+template <typename S, int NSUB>
 struct Brick {
-  static constexpr int ROW = NSUB == 1 ? 384 : BW * 16;
-  static constexpr int PLANE = ((BD * BH * ROW - 64 + 255) / 256) * 256 + 64;
+  static constexpr int ROW = NSUB == 1 ? S::PITCH : S::BW * 16;
+  static constexpr int PLANE = ((S::BD * S::BH * ROW - 64 + 255) / 256) * 256 + 64;
   static constexpr int SLOT = 4 * PLANE + 16;
   // byte offset of a brick voxel in its plane (dense rows: not by row and column, which is 130 instructions a round of four chunks and 1 % of the time)
-  static __device__ __forceinline__ int at(int vox) { return ROW == BW * 16 ? vox * 16 : vox / BW * ROW + vox % BW * 16; }
+  static __device__ __forceinline__ int at(int vox) { return ROW == S::BW * 16 ? vox * 16 : vox / S::BW * ROW + vox % S::BW * 16; }
   // byte offset of (tap, k-step) relative to a lane's voxel at tap (0, 0, 0)
-  static constexpr int tap_off(int tap) { return ((tap / 9) * BH + (tap / 3) % 3) * ROW + tap % 3 * 16; }
+  static constexpr int tap_off(int tap) { return ((tap / 9) * S::BH + (tap / 3) % 3) * ROW + tap % 3 * 16; }
 };
 
 // R: chunks per round. PAIR: the input is two tensors whose channels follow each other (the first `c_first` in x, the
 // rest in x1). Independently, a non-null y1 splits the OUTPUT the same way.
-template <typename T, int R, int NSUB, bool PAIR>
+template <typename T, typename S, int R, int NSUB, bool PAIR>
 __global__ void __launch_bounds__(256, 2)
 conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ wp, const T* __restrict__ bias, T* __restrict__ y,
                   int tiles_d, int tiles_h, int tiles_w, int nblocks, uint32_t total, GnPartialOut gn, const T* __restrict__ x1,
                   T* __restrict__ y1, int c_first) {
-  using B = Brick<NSUB>;
+  using B = Brick<S, NSUB>;
+  constexpr int TD = S::TD, TH = S::TH, TW = S::TW, BH = S::BH, BW = S::BW;
   constexpr int PLANE = B::PLANE, SLOT = B::SLOT;
   constexpr int RED_BYTES = MS * NSUB * 3 * 4096;  // every block from the three wavefronts that do not own it
   constexpr int LDS = R * SLOT > RED_BYTES ? R * SLOT : RED_BYTES;
@@ -82,8 +88,8 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   int abase[MS];  // LDS byte address of the lane's voxel of block row ms at tap (0, 0, 0), in its k-half plane
 #pragma unroll
   for (int ms = 0; ms < MS; ++ms) {
-    const int tw = j % TW, th = j / TW;
-    abase[ms] = slot * SLOT + (kg + 2 * khalf) * PLANE + (ms * BH + th) * B::ROW + tw * 16;
+    const int v = ms * 32 + j, tw = v % TW, th = v / TW % TH, td = v / (TW * TH);
+    abase[ms] = slot * SLOT + (kg + 2 * khalf) * PLANE + (td * BH + th) * B::ROW + tw * 16;
   }
   auto a_off = [](int k) constexpr { return R == 4 ? B::tap_off(k / 2) + (k % 2) * 2 * PLANE : B::tap_off(k); };
 
@@ -97,7 +103,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
 
   const int ncc = a.cred / kChunk;
   const int id0 = od0 - a.pd, ih0 = oh0 - a.ph, iw0 = ow0 - a.pw;
-  constexpr int PIECES = BV * 4 * R;
+  constexpr int PIECES = S::BV * 4 * R;
   constexpr int ITERS = (PIECES + 255) / 256;
   constexpr int WDEPTH = 16 / NSUB;  // weight fragments (per output block) in flight per wavefront
   const int64_t wns = (int64_t)ncc * (NIT * FRAG);  // next 32-channel output block
@@ -213,8 +219,8 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   // two 16-byte pieces.
   const int ms_o = wave / NSUB, ns_o = wave % NSUB;
   const bool owns = MS * NSUB == 4 || wave < MS * NSUB;
-  const int tw = j % TW, th = j / TW;
-  const int od = od0 + ms_o, oh = oh0 + th, ow = ow0 + tw;
+  const int own_v = ms_o * 32 + j;
+  const int od = od0 + own_v / (TW * TH), oh = oh0 + own_v / TW % TH, ow = ow0 + own_v % TW;
   const bool inside = owns && od < a.od && oh < a.oh && ow < a.ow;
   const int64_t vox = (((int64_t)n * a.od + od) * a.oh + oh) * a.ow + ow;
   const int ch = (nb * NSUB + ns_o) * 32;
@@ -262,7 +268,42 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   }
 }
 
-int64_t split_tiles(const MfmaConvArgs& a) { return (int64_t)a.n * cdiv(a.od, TD) * cdiv(a.oh, TH) * cdiv(a.ow, TW); }
+typedef Shape<2, 4, 8, 384> Flat;    // 240 voxels with the halo
+typedef Shape<4, 4, 4, 192> Cube;    // 216
+typedef Shape<2, 2, 16, 288> Rows;   // 288
+
+int64_t tiles_of(const MfmaConvArgs& a, int shape) {
+  static const int t[3][3] = {{2, 4, 8}, {4, 4, 4}, {2, 2, 16}};
+  return (int64_t)a.n * cdiv(a.od, t[shape][0]) * cdiv(a.oh, t[shape][1]) * cdiv(a.ow, t[shape][2]);
+}
+
+// What a launch of `pairs` pairs of channel blocks takes, in hundredths of a us, fitted as the brick kernel's (conv_mfma.hip, brick_time) to 453
+// problems on odd levels: 7 % (rms). Up to half a round is dealt as single blocks.
+int64_t split_time(int64_t pairs, int chunks) {
+  const int64_t rounds = cdiv(pairs, kComputeUnits);
+  return pairs <= kComputeUnits / 2 ? 420 + 100 * chunks
+                                    : 400 + 60 * rounds + chunks * (99 * rounds * kComputeUnits + 54 * pairs) / kComputeUnits;
+}
+
+// The brick that is done soonest: a volume of odd extents takes fewer of one shape than of another, and a round of workgroups less is what
+// that mostly saves. At equal counts 4x4x4 takes 0.99 of the time of 2x4x8 (its halo is smaller) and 2x2x16 1.06. A voxel's sums do not depend on
+// the brick. us, 2x4x8 / 4x4x4 / 2x2x16: 512 -> 512 at 12x10x14 50.0 / 49.0 / 38.9 (288, 288 and 240 pairs), 256 -> 512 28.0 / 27.2 / 22.9, 128 -> 128 at 19x17x58
+// 29.6 / 24.4 / 26.8, 512 -> 512 at 7x9x4 22.1 / 19.5 / 32.2, 256 -> 256 at 8x16x16 13.4 / 12.8 / 13.5; over 136 odd levels the choice is 4.4 % ahead of 2x4x8.
+int split_shape(const MfmaConvArgs& a) {
+  static const int weight[3] = {100, 99, 106};
+  const int pair = a.cout / (32 * kBlocks), chunks = a.cred / kChunk;
+  int best = 0;
+  int64_t least = 0;
+  for (int s = 0; s < 3; ++s) {
+    const int64_t time = split_time(tiles_of(a, s) * pair, chunks) * weight[s];
+    if (s > 0 && time >= least) continue;
+    least = time;
+    best = s;
+  }
+  return best;
+}
+
+int64_t split_tiles(const MfmaConvArgs& a) { return tiles_of(a, split_shape(a)); }
 
 // One channel block per workgroup where pairs would leave half of the CUs idle: each workgroup then has half the weights to fetch and
 // half the MFMAs (the bits of the output do not depend on it). us, caches warm / cold: 256 -> 256 at 8x16x16 16.0 / 18.9 -> 13.1 / 16.2,
@@ -270,17 +311,27 @@ int64_t split_tiles(const MfmaConvArgs& a) { return (int64_t)a.n * cdiv(a.od, TD
 // 256 -> 256 at 10x16x16 16.5 / 22.0 -> 19.2 / 22.2, at 16^3 17.6 -> 19.6 (each CU fetches the same weights and stages twice the bricks).
 int split_blocks(const MfmaConvArgs& a) { return split_tiles(a) * (a.cout / (32 * kBlocks)) <= kComputeUnits / 2 ? 1 : kBlocks; }
 
+template <typename T, typename S, int R, int NSUB, bool PAIR>
+int launch_brick(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
+                 const GnPartialOut& gn, const void* x1, void* y1, int first) {
+  const int tiles_d = (int)cdiv(a.od, S::TD), tiles_h = (int)cdiv(a.oh, S::TH), tiles_w = (int)cdiv(a.ow, S::TW);
+  const int nblocks = a.cout / (32 * NSUB);
+  const int64_t total = (int64_t)a.n * tiles_d * tiles_h * tiles_w * nblocks;
+  if (total == 0) return SFH_OK;
+  if (total > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv split: %lld workgroups exceed the grid limit", (long long)total);
+  hipLaunchKernelGGL((conv_split_kernel<T, S, R, NSUB, PAIR>), dim3((unsigned)total), dim3(256), 0, st, a, (const T*)x, (const T*)packed,
+                     (const T*)bias, (T*)y, tiles_d, tiles_h, tiles_w, nblocks, (uint32_t)total, gn, (const T*)x1, (T*)y1, first);
+  return check_launch("conv_split_kernel");
+}
+
 template <typename T, int R, int NSUB, bool PAIR>
 int launch_split(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                  const GnPartialOut& gn, const void* x1, void* y1, int first) {
-  const int tiles_d = (int)cdiv(a.od, TD), tiles_h = (int)cdiv(a.oh, TH), tiles_w = (int)cdiv(a.ow, TW);
-  const int nblocks = a.cout / (32 * NSUB);
-  const int64_t total = split_tiles(a) * nblocks;
-  if (total == 0) return SFH_OK;
-  if (total > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv split: %lld workgroups exceed the grid limit", (long long)total);
-  hipLaunchKernelGGL((conv_split_kernel<T, R, NSUB, PAIR>), dim3((unsigned)total), dim3(256), 0, st, a, (const T*)x, (const T*)packed,
-                     (const T*)bias, (T*)y, tiles_d, tiles_h, tiles_w, nblocks, (uint32_t)total, gn, (const T*)x1, (T*)y1, first);
-  return check_launch("conv_split_kernel");
+  switch (split_shape(a)) {
+    case 1: return launch_brick<T, Cube, R, NSUB, PAIR>(a, x, packed, bias, y, st, gn, x1, y1, first);
+    case 2: return launch_brick<T, Rows, R, NSUB, PAIR>(a, x, packed, bias, y, st, gn, x1, y1, first);
+    default: return launch_brick<T, Flat, R, NSUB, PAIR>(a, x, packed, bias, y, st, gn, x1, y1, first);
+  }
 }
 
 template <typename T>
@@ -334,14 +385,12 @@ int64_t split_line(int chunks, int cout) {
 bool mfma_conv_split_applies(const MfmaConvArgs& a) {
   if (a.kd != 3 || a.kh != 3 || a.kw != 3) return false;
   if (a.cred < 2 * kChunk || a.cred % (2 * kChunk) != 0 || a.cout % (32 * kBlocks) != 0) return false;
-  const int64_t per_depth = (int64_t)a.n * cdiv(a.oh, TH) * cdiv(a.ow, TW) * (a.cout / (32 * kBlocks));
-  const int chunks = a.cred / kChunk;
+  const int chunks = a.cred / kChunk, pair = a.cout / (32 * kBlocks);
   MfmaConvArgs core = a;
   core.od = a.id < a.od ? a.id : a.od;
-  const int64_t pairs = per_depth * cdiv(core.od, TD), rounds = cdiv(pairs, kComputeUnits);
-  // what the launch takes, in hundredths of a us, fitted as the brick kernel's (conv_mfma.hip, brick_time), 7 % (rms)
-  const int64_t time = pairs <= kComputeUnits / 2 ? 420 + 100 * chunks
-                                                  : 400 + 60 * rounds + chunks * (99 * rounds * kComputeUnits + 54 * pairs) / kComputeUnits;
+  const int64_t per_depth = (int64_t)a.n * cdiv(a.oh, Flat::TH) * cdiv(a.ow, Flat::TW) * pair;
+  const int64_t pairs = per_depth * cdiv(core.od, Flat::TD), rounds = cdiv(pairs, kComputeUnits);
+  const int64_t time = split_time(split_tiles(core) * pair, chunks);
   if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return pairs > kSplitBigPlanePairs && 100 * time < 88 * mfma_conv_brick_time(core);
   const bool few = per_depth <= kSplitFewPerDepth && chunks >= kSplitFewMaxChunks;
   if (pairs < split_line(chunks, a.cout) && (few || per_depth < kSplitMinPerDepth))
@@ -349,7 +398,7 @@ bool mfma_conv_split_applies(const MfmaConvArgs& a) {
   return rounds <= 3 || 100 * time < 110 * mfma_conv_brick_time(core);
 }
 
-MfmaConvGeometry mfma_conv_split_geometry(const MfmaConvArgs&) { return MfmaConvGeometry{kKernelSplit, TD * TH * TW, kBlocks, 1}; }
+MfmaConvGeometry mfma_conv_split_geometry(const MfmaConvArgs&) { return MfmaConvGeometry{kKernelSplit, kBrickVoxels, kBlocks, 1}; }
 
 int mfma_conv_split_gn_records(const MfmaConvArgs& a, int groups) {
   const int span = 32 * split_blocks(a);

@@ -23,6 +23,12 @@ CASES = [
     (1, 512, 512, (9, 9, 6), "split", 64),      # 120 pairs of a long reduction on cut bricks
     (2, 128, 64, (19, 30, 35), "brick", None),  # a round and a bit of the wide kernel's workgroups would be two
     (1, 256, 256, (32, 32, 8), "split", 64),
+    (2, 128, 128, (10, 5, 30), "split", 64),    # bricks of 2 x 2 x 16, a workgroup of one channel block each
+    (2, 128, 512, (6, 9, 29), "split", 64),     # ... two
+    (2, 192, 128, (10, 5, 30), "split", 64),    # ... two chunks a round
+    (2, 192, 256, (10, 5, 30), "split", 64),    # ... two blocks
+    (1, 128, 256, (7, 11, 12), "split", 64),    # bricks of 4 x 4 x 4, cut on two axes, one block
+    (1, 192, 512, (7, 11, 12), "split", 64),    # ... two blocks, two chunks a round
     (1, 64, 64, (55, 28, 41), "brick", 256),    # 4 x 8 x 8 with one block in the place of 4 x 4 x 32
 ]
 
