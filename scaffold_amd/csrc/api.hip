@@ -90,7 +90,7 @@ MfmaConvArgs dgrad_mfma_args(const sfh_conv3d_desc& p, const int32_t out[3]) {
 bool fwd_uses_mfma(const sfh_conv3d_desc& p, int dtype, const int32_t out[3]) {
   return is_unit(p) && mfma_conv_supported(fwd_mfma_args(p, out), dtype);
 }
-// fp32 problems of the tiled shape run on the fp32 matrix pipe (the weight is packed per call into the workspace)
+// fp32 problems of the tiled shape run on the fp32 matrix pipe (a weight that is not channels-last is packed per call into the workspace)
 bool on_16_bytes(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }  // null counts as aligned
 
 bool fwd_uses_f32_tiles(const sfh_conv3d_desc& p, int dtype, const int32_t out[3]) {
@@ -404,8 +404,10 @@ static int conv3d_fwd_any(const sfh_conv3d_desc* p, int dtype, const void* x, co
     const size_t need = f32_conv_packed_weight_bytes(a);
     if (workspace == nullptr || workspace_bytes < need)
       return fail(SFH_ERR_WORKSPACE, "conv3d fwd: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+    const F32Weight form = f32_weight_form(a, w, w_stride, false);
+    if (form != F32Weight::kPacked) return f32_conv(a, x, w, form, bias, y, st);
     if (int rc = f32_pack_weight(a, w, w_stride[0], w_stride[1], w_stride[2], w_stride[3], w_stride[4], 0, workspace, st)) return rc;
-    return f32_conv(a, x, workspace, bias, y, st);
+    return f32_conv(a, x, workspace, form, bias, y, st);
   }
   if (!(flags & SFH_FLAG_FORCE_GENERIC) && (flags & SFH_FLAG_WEIGHT_PACKED) && fwd_uses_patch(*p, dtype, out))
     return patch_gather(patch_args(*p, out), dtype, x, w, false, bias, y, st);
@@ -589,9 +591,11 @@ static int conv3d_dgrad_any(const sfh_conv3d_desc* p, int dtype, const void* gy,
     const size_t need = f32_conv_packed_weight_bytes(a);
     if (workspace == nullptr || workspace_bytes < need)
       return fail(SFH_ERR_WORKSPACE, "conv3d dgrad: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+    const F32Weight form = f32_weight_form(a, w, w_stride, true);
+    if (form != F32Weight::kPacked) return f32_conv(a, gy, w, form, nullptr, gx, st);
     // produced channel = Cin (stride w_stride[1]), reduction channel = Cout (w_stride[0]), taps flipped
     if (int rc = f32_pack_weight(a, w, w_stride[1], w_stride[0], w_stride[2], w_stride[3], w_stride[4], 1, workspace, st)) return rc;
-    return f32_conv(a, gy, workspace, nullptr, gx, st);
+    return f32_conv(a, gy, workspace, form, nullptr, gx, st);
   }
   if (flags & SFH_FLAG_WEIGHT_PACKED) return fail(SFH_ERR_INVALID, "conv3d dgrad: this problem does not read a packed weight");
   if (!(flags & SFH_FLAG_FORCE_GENERIC)) {

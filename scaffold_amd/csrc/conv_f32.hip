@@ -11,12 +11,14 @@
 //     channels 4p .. 4p+3 of every brick voxel; planes 64 bytes apart modulo 256, so a wavefront's ds_read_b128 of rows
 //     of 8 or more voxels is conflict free and every tap is an immediate offset).
 //   * One MFMA contracts 2 reduction channels: k-slot kg (= lane / 32) at step kk of a chunk is channel 8 kg + kk, so a
-//     lane's operands of the 8 steps of a tap are 8 consecutive channels: two 16-byte LDS reads of activations and two
-//     16-byte global loads of the weight, which is repacked once per call into that order
+//     lane's operands of the 8 steps of a tap are 8 consecutive channels: two 16-byte LDS reads of activations and 32 bytes
+//     of the weight. A channels-last weight is read where it lies: forward two 16-byte loads of a row, data gradient eight of one
+//     element, 32 produced channels side by side. An fp32 MFMA takes 64 cycles, so a tap's 8 per sub-tile hide either (a packing
+//     launch in front, which other layouts still take, was 3 to 4 us of the call):
 //       packed[cout/32][cred/16][tap][q(2)][lane(64)][4],  lane = cout % 32 + 32 kg,  channel = 16 cc + 8 kg + 4 q + e.
 //   * The weight is the ROW operand, so a lane ends up with four runs of four consecutive output channels of one voxel
 //     and stores 16-byte pieces.
-// The data gradient runs this kernel with the weight packed transposed and tap-flipped and padding k-1-p
+// The data gradient runs this kernel with the weight transposed and tap-flipped and padding k-1-p
 // (triton_conv3d/bwd_data.py:344-363).
 #include "conv_f32.hpp"
 #include "reduce.hpp"
@@ -69,10 +71,12 @@ __device__ __forceinline__ constexpr int tap_off(int tap) {
   return ((kd * C::BH + kh) * C::BW + kw) * 16;
 }
 
-template <typename C>
+// wt: the weight in the form W (conv_f32.hpp)
+template <typename C, F32Weight W>
 __global__ void __launch_bounds__(C::THREADS, 2)
-conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __restrict__ wp, const float* __restrict__ bias,
+conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __restrict__ wt, const float* __restrict__ bias,
                 float* __restrict__ y, int tiles_d, int tiles_h, int tiles_w, int nblocks, uint32_t total) {
+#if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = (tid >> 6) % C::WM;
@@ -132,17 +136,51 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
       }
     }
   };
-  // weight fragments of tap t: packed + (((nb * ncc + cc) * 27 + t) * 2 + q) * 256 floats + lane * 4; the taps of a chunk
-  // are followed by the next chunk's, so the requests ahead run on over the end of a chunk
+  // A fragment's place is a chunk's, which the wavefront shares, a tap's and the lane's. The taps of a chunk are followed by the next
+  // chunk's, so the requests ahead run on over the end of a chunk. A weight where it lies is read through a buffer: one scalar addition
+  // a tap (64-bit addresses of eight rows were half of the instructions of a tap, and 27 taps of them spilled scalar registers).
   const int last = part < ncc ? part + (ncc - 1 - part) / C::KS * C::KS : -1;  // the wavefront's last chunk
-  const float* wcc = wp + ((int64_t)(nb * ncc + (part < ncc ? part : 0)) * kTaps * 2) * 256 + lane * 4;
+  const int first_chunk = part < ncc ? part : 0;
+  const float* wcc = wt + ((int64_t)nb * ncc + first_chunk) * (kTaps * 2 * 256) + lane * 4;  // kPacked
+  __amdgpu_buffer_rsrc_t wbuf;
+  int wbase = 0, wchunk = 0, wtap = 0, wlane[8];  // bytes
+  if constexpr (W == F32Weight::kRows) {
+    wbase = (nb * 32 * kTaps * a.cred + first_chunk * kChunk) * 4;
+    wchunk = C::KS * kChunk * 4;
+    wtap = a.cred * 4;
+    wlane[0] = (j * (kTaps * a.cred) + 8 * kg) * 4;
+  } else if constexpr (W == F32Weight::kColumns) {
+    wbase = ((first_chunk * kChunk * kTaps + kTaps - 1) * a.cout + nb * 32) * 4;
+    wchunk = C::KS * kChunk * kTaps * a.cout * 4;
+    wtap = -a.cout * 4;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) wlane[e] = ((8 * kg + e) * (kTaps * a.cout) + j) * 4;
+  }
+  if constexpr (W != F32Weight::kPacked)
+    wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(wt), 0, kTaps * a.cred * a.cout * 4, 0x00020000);
+  auto weights = [&](bool next, int tap, float4 (&out)[2]) {
+    if constexpr (W == F32Weight::kPacked) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) out[q] = *reinterpret_cast<const float4*>(wcc + ((tap + (next ? C::KS * kTaps : 0)) * 2 + q) * 256);
+    } else {
+      const int at = wbase + (next ? wchunk : 0) + tap * wtap;
+      if constexpr (W == F32Weight::kRows) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) out[q] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(wbuf, wlane[0] + 16 * q, at, 0));
+      } else {
+        float got[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) got[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wbuf, wlane[e], at, 0));
+        out[0] = make_float4(got[0], got[1], got[2], got[3]);
+        out[1] = make_float4(got[4], got[5], got[6], got[7]);
+      }
+    }
+  };
   constexpr int WDEPTH = 3;  // taps requested ahead
   static_assert(kTaps % WDEPTH == 0, "a chunk ends where the ring of requests began");
   float4 wq[WDEPTH][2];
 #pragma unroll
-  for (int d = 0; d < WDEPTH; ++d)
-#pragma unroll
-    for (int q = 0; q < 2; ++q) wq[d][q] = *reinterpret_cast<const float4*>(wcc + (d * 2 + q) * 256);
+  for (int d = 0; d < WDEPTH; ++d) weights(false, d, wq[d]);
   float4 v[BATCH];
   if (C::AHEAD) request(0, 0, v);
   for (int cc = 0; cc < ncc; cc += C::KS) {
@@ -176,9 +214,8 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
     for (int tap = 0; tap < kTaps; ++tap) {
       float4 wf[2] = {wq[tap % WDEPTH][0], wq[tap % WDEPTH][1]};
       if (tap + WDEPTH < kTaps || ahead) {
-        const int at = tap + WDEPTH < kTaps ? tap + WDEPTH : tap + WDEPTH + (C::KS - 1) * kTaps;
-#pragma unroll
-        for (int q = 0; q < 2; ++q) wq[tap % WDEPTH][q] = *reinterpret_cast<const float4*>(wcc + (at * 2 + q) * 256);
+        const bool next = tap + WDEPTH >= kTaps;
+        weights(next, next ? tap + WDEPTH - kTaps : tap + WDEPTH, wq[tap % WDEPTH]);
       }
       if constexpr (C::AHEAD) {
         if (tap + 1 < kTaps) activations(tap + 1);
@@ -203,6 +240,7 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
       if constexpr (C::AHEAD) __builtin_amdgcn_sched_barrier(0);
     }
     wcc += C::KS * kTaps * 2 * 256;
+    wbase += wchunk;
   }
 
   if constexpr (C::KS > 1) {
@@ -241,6 +279,7 @@ conv_f32_kernel(MfmaConvArgs a, const float* __restrict__ x, const float* __rest
           make_float4(acc[ms][4 * g] + b.x, acc[ms][4 * g + 1] + b.y, acc[ms][4 * g + 2] + b.z, acc[ms][4 * g + 3] + b.w);
     }
   }
+#endif
 }
 
 // One thread per packed 16-byte piece: the 4 consecutive reduction channels of one (output channel, tap, k-slot, q).
@@ -272,14 +311,19 @@ pack_f32_kernel(const float* __restrict__ w, float* __restrict__ packed, int cre
 }
 
 template <typename C>
-int launch(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st) {
+int launch(const MfmaConvArgs& a, const void* x, const void* w, F32Weight form, const void* bias, void* y, hipStream_t st) {
   const int tiles_d = (int)cdiv(a.od, C::TD), tiles_h = (int)cdiv(a.oh, C::TH), tiles_w = (int)cdiv(a.ow, C::TW);
   const int nblocks = a.cout / 32;
   const int64_t total = (int64_t)a.n * tiles_d * tiles_h * tiles_w * nblocks;
   if (total == 0) return SFH_OK;
   if (total > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv fp32: %lld workgroups exceed the grid limit", (long long)total);
-  hipLaunchKernelGGL((conv_f32_kernel<C>), dim3((unsigned)total), dim3(C::THREADS), 0, st, a, (const float*)x, (const float*)packed,
-                     (const float*)bias, (float*)y, tiles_d, tiles_h, tiles_w, nblocks, (uint32_t)total);
+#define SFH_LAUNCH_F32(W)                                                                                                         \
+  hipLaunchKernelGGL((conv_f32_kernel<C, W>), dim3((unsigned)total), dim3(C::THREADS), 0, st, a, (const float*)x, (const float*)w, \
+                     (const float*)bias, (float*)y, tiles_d, tiles_h, tiles_w, nblocks, (uint32_t)total)
+  if (form == F32Weight::kRows) SFH_LAUNCH_F32(F32Weight::kRows);
+  else if (form == F32Weight::kColumns) SFH_LAUNCH_F32(F32Weight::kColumns);
+  else SFH_LAUNCH_F32(F32Weight::kPacked);
+#undef SFH_LAUNCH_F32
   return check_launch("conv_f32_kernel");
 }
 
@@ -486,17 +530,40 @@ int f32_pack_weight(const MfmaConvArgs& a, const void* w, int64_t s_out, int64_t
   return check_launch("pack_f32_kernel");
 }
 
-int f32_conv(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st) {
+// The brick of the least time.
+static int choose_brick(const MfmaConvArgs& a) {
   int best = 0;
   for (int c = 1; c < 6; ++c)
     if (tile_us(a, c) < tile_us(a, best)) best = c;
-  switch (best) {
-    case 0: return launch<WholeTile>(a, x, packed, bias, y, st);
-    case 1: return launch<FlatTile<8>>(a, x, packed, bias, y, st);
-    case 2: return launch<FlatTile<16>>(a, x, packed, bias, y, st);
-    case 3: return launch<HalvedTile<8>>(a, x, packed, bias, y, st);
-    case 4: return launch<HalvedTile<16>>(a, x, packed, bias, y, st);
-    default: return launch<QuarteredTile>(a, x, packed, bias, y, st);
+  return best;
+}
+
+// A channels-last weight is read where it lies: no packing launch, and where the weights are much of what a launch reads the packed
+// ones were written and read once more. Of 70 drawn problems of 32 to 512 channels, us, packed -> as it lies: 32 -> 32 at 32^3 22.7 -> 18.5 and
+// 21.6 -> 18.7 (data gradient), at 8^3 13.9 -> 10.8 and 14.1 -> 11.5, 128 -> 128 at 16^3 39.9 -> 32.5 and 38.3 -> 33.2, 512 -> 512 at
+// 4x8x8 100.7 -> 62.6 and 100.2 -> 63.4, at 16^3 486 -> 415 and 484 -> 429, 64 -> 64 at 64^3 451 -> 417 and 451 -> 425. The line: where many
+// workgroups of few wavefronts a sub-tile share a CU, the data gradient's eight loads a tap are what it waits for (packed / as it lies: 64
+// channels at 63x9x30 45.4 / 52.2, at 33x25x16 61.8 / 68.7, of 128 channels level, of 256 276 / 263), and a forward with fewer
+// produced channels than it reads shares its lines with few (two samples of 64 -> 32 at 20x33x41 65.8 / 71.7, 256 -> 128 at 20x32x9 158.5 / 163.2).
+F32Weight f32_weight_form(const MfmaConvArgs& a, const void* w, const int64_t w_stride[5], bool dgrad) {
+  const int64_t inner = dgrad ? a.cout : a.cred;  // Cin
+  const bool dense = w_stride[1] == 1 && w_stride[4] == inner && w_stride[3] == 3 * inner && w_stride[2] == 9 * inner && w_stride[0] == 27 * inner;
+  if (!dense || (int64_t)a.cout * a.cred * kTaps > 0x1fffffffLL) return F32Weight::kPacked;
+  const int brick = choose_brick(a);
+  const int64_t bricks = (int64_t)a.n * cdiv(a.od, 2) * cdiv(a.oh, 2) * cdiv(a.ow, brick == 4 ? 16 : 8);
+  const bool crowded = brick >= 4 && bricks * (a.cout / 32) > 3 * kComputeUnits;
+  if (dgrad) return crowded && a.cred <= 128 ? F32Weight::kPacked : F32Weight::kColumns;
+  return (crowded && a.cout < a.cred) || (reinterpret_cast<uintptr_t>(w) & 15u) != 0 ? F32Weight::kPacked : F32Weight::kRows;
+}
+
+int f32_conv(const MfmaConvArgs& a, const void* x, const void* w, F32Weight form, const void* bias, void* y, hipStream_t st) {
+  switch (choose_brick(a)) {
+    case 0: return launch<WholeTile>(a, x, w, form, bias, y, st);
+    case 1: return launch<FlatTile<8>>(a, x, w, form, bias, y, st);
+    case 2: return launch<FlatTile<16>>(a, x, w, form, bias, y, st);
+    case 3: return launch<HalvedTile<8>>(a, x, w, form, bias, y, st);
+    case 4: return launch<HalvedTile<16>>(a, x, w, form, bias, y, st);
+    default: return launch<QuarteredTile>(a, x, w, form, bias, y, st);
   }
 }
 
