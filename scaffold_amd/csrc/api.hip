@@ -384,6 +384,8 @@ static int conv3d_fwd_any(const sfh_conv3d_desc* p, int dtype, const void* x, co
     const size_t need = packed_bytes + partial_bytes;
     if (workspace == nullptr || workspace_bytes < need)
       return fail(SFH_ERR_WORKSPACE, "conv3d fwd: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+    const MfmaWeight form = mfma_conv_weight_form(a, w, w_stride, false);
+    if (form != MfmaWeight::kPacked) return mfma_conv_persist(a, dtype, x, w, bias, y, nullptr, st, gn, in2, nullptr, form);
     if (int rc = mfma_pack_weight(a, dtype, w, w_stride[0], w_stride[1], w_stride[2], w_stride[3], w_stride[4], 0, workspace, st))
       return rc;
     void* partial = partial_bytes ? (char*)workspace + packed_bytes : nullptr;
@@ -578,6 +580,8 @@ static int conv3d_dgrad_any(const sfh_conv3d_desc* p, int dtype, const void* gy,
     const size_t need = packed_bytes + partial_bytes;
     if (workspace == nullptr || workspace_bytes < need)
       return fail(SFH_ERR_WORKSPACE, "conv3d dgrad: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+    const MfmaWeight form = mfma_conv_weight_form(a, w, w_stride, true);
+    if (form != MfmaWeight::kPacked) return mfma_conv_persist(a, dtype, gy, w, nullptr, gx, nullptr, st, nullptr, nullptr, out2, form);
     // produced channel = Cin (stride w_stride[1]), reduction channel = Cout (w_stride[0]), taps flipped
     if (int rc = mfma_pack_weight(a, dtype, w, w_stride[1], w_stride[0], w_stride[2], w_stride[3], w_stride[4], 1, workspace, st))
       return rc;

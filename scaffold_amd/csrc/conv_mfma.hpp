@@ -59,16 +59,21 @@ int mfma_conv_split(const MfmaConvArgs& a, int dtype, const void* x, const void*
                     const GnPartialOut* gn = nullptr, const ChannelPair* in2 = nullptr, const ChannelPair* out2 = nullptr);
 int mfma_conv_split_gn_records(const MfmaConvArgs& a, int groups);
 bool mfma_conv_split_pair_ok(const MfmaConvArgs& a, int first, bool as_output);
-// Same contract, persistent one-workgroup-per-CU kernel with register-resident weights.
+// How the column-walking kernel reads the weight: packed, or a channels-last one where it lies, [produced][tap][reduction] or
+// [reduction][tap][produced] with the taps back to front.
+enum class MfmaWeight { kPacked, kRows, kColumns };
+// The form of a weight of these strides (elements; Cout, Cin, kd, kh, kw); kPacked: it has to be packed first.
+MfmaWeight mfma_conv_weight_form(const MfmaConvArgs& a, const void* w, const int64_t w_stride[5], bool dgrad);
+// Same contract, persistent one-workgroup-per-CU kernel with register-resident weights. `form`: what `packed` is.
 int mfma_conv_persist(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y,
                       void* partial, hipStream_t st, const GnPartialOut* gn = nullptr, const ChannelPair* in2 = nullptr,
-                      const ChannelPair* out2 = nullptr);
+                      const ChannelPair* out2 = nullptr, MfmaWeight form = MfmaWeight::kPacked);
 // The persistent kernel's form for rows of more than 16 voxels: columns walked along depth with a ring of input planes in
 // LDS (conv_ring.hip). `applies` is a pure function of the shape; mfma_conv_persist routes to it. gn.cg must be set.
 bool mfma_conv_ring_applies(const MfmaConvArgs& a);
 int mfma_conv_ring_records(const MfmaConvArgs& a);  // workgroups of a sample and output block; 0: they walk across samples
-int mfma_conv_ring(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
-                   const GnPartialOut& gn, const ChannelPair& out2);
+int mfma_conv_ring(const MfmaConvArgs& a, int dtype, const void* x, const void* w, MfmaWeight form, const void* bias, void* y,
+                   hipStream_t st, const GnPartialOut& gn, const ChannelPair& out2);
 // Records of GroupNorm partials per sample that mfma_conv_persist leaves for `groups` groups: a pure function of the
 // shape; 0 when the kernel that serves the problem does not offer them (the caller then runs the statistics pass).
 int mfma_conv_gn_records(const MfmaConvArgs& a, int groups);

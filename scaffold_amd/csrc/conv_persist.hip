@@ -520,8 +520,18 @@ bool mfma_conv_pair_ok(const MfmaConvArgs& a, int first, bool as_output) {
   return as_output && first > 0 && first < a.cout && first % 32 == 0;
 }
 
+MfmaWeight mfma_conv_weight_form(const MfmaConvArgs& a, const void* w, const int64_t w_stride[5], bool dgrad) {
+  if (!mfma_conv_persist_applies(a) || !ring_serves(a) || a.cout > 65536) return MfmaWeight::kPacked;
+  const int64_t cin = dgrad ? a.cout : a.cred;
+  const bool dense = w_stride[1] == 1 && w_stride[4] == cin && w_stride[3] == 3 * cin && w_stride[2] == 9 * cin && w_stride[0] == 27 * cin;
+  if (!dense || (reinterpret_cast<uintptr_t>(w) & 15u) != 0) return MfmaWeight::kPacked;
+  return dgrad ? MfmaWeight::kColumns : MfmaWeight::kRows;
+}
+
 int mfma_conv_persist(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y,
-                      void* partial, hipStream_t st, const GnPartialOut* gn, const ChannelPair* in2, const ChannelPair* out2) {
+                      void* partial, hipStream_t st, const GnPartialOut* gn, const ChannelPair* in2, const ChannelPair* out2, MfmaWeight form) {
+  if (form != MfmaWeight::kPacked && !(mfma_conv_persist_applies(a) && ring_serves(a)))
+    return fail(SFH_ERR_INVALID, "conv mfma: this problem reads a packed weight");
   if (!mfma_conv_persist_applies(a)) return mfma_conv_gather(a, dtype, x, packed, bias, y, partial, st, gn, in2, out2);
   if (in2 != nullptr) return fail(SFH_ERR_UNSUPPORTED, "conv persist: 32 reduction channels cannot be a pair of tensors");
   if (out2 != nullptr && (out2->second == nullptr || !mfma_conv_pair_ok(a, out2->first, true)))
@@ -535,7 +545,7 @@ int mfma_conv_persist(const MfmaConvArgs& a, int dtype, const void* x, const voi
     out = *gn;
     out.cg = a.cout / gn->groups;
   }
-  if (ring_serves(a)) return mfma_conv_ring(a, dtype, x, packed, bias, y, st, out, pair);
+  if (ring_serves(a)) return mfma_conv_ring(a, dtype, x, packed, form, bias, y, st, out, pair);
   if (dtype == SFH_BF16) return launch_typed<bf16_t>(a, x, packed, bias, y, st, out, pair);
   return launch_typed<fp16_t>(a, x, packed, bias, y, st, out, pair);
 }

@@ -346,10 +346,11 @@ __device__ __forceinline__ void ring_round(const f32x16_t (&acc)[4], const float
   }
 }
 
-template <typename T, bool BIAS, bool GN>
+// wp: the packed weight, with `rows` a channels-last weight [out][tap][32], with COLUMNS one [32][tap][out] whose taps run back to front.
+template <typename T, bool BIAS, bool GN, bool COLUMNS>
 __global__ void __launch_bounds__(256, 1)
-conv_ring_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ wp, const T* __restrict__ bias_ptr, T* __restrict__ y,
-                 RingGeom gm, GnPartialOut gn, T* __restrict__ y1, int c_first) {
+conv_ring_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ wp, int rows, const T* __restrict__ bias_ptr,
+                 T* __restrict__ y, RingGeom gm, GnPartialOut gn, T* __restrict__ y1, int c_first) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(16))) char pair0[kPair];
   __shared__ __attribute__((aligned(16))) char pair1[kPair];
@@ -401,15 +402,23 @@ conv_ring_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ 
   // weight is in fragment order, a fragment is 1 KiB as it lies) and every wavefront takes its copy from there: four
   // copies straight from memory cost the CU's address path 216 KiB beside the first plane pairs' 86. They land in the
   // third pair's array, which nothing reads before the first step fills it, and in `wrest`.
+  // A channels-last weight needs no packing launch (2.4 us and its gap) for that: a forward's lane fetches its 16 bytes of a row from
+  // where they lie, a data gradient's k-step is 16 rows of 64 bytes, which the transposing read turns. us, packed -> as it lies,
+  // forward and data gradient: 32 -> 32 at 32^3 11.8 -> 9.7 and 11.9 -> 9.5, at 64^3 20.1 -> 18.0 and 20.2 -> 17.9, at 8x16x20 10.7 -> 8.7, two samples of
+  // 44x60x75 32.4 -> 29.7 and 31.9 -> 29.1.
   {
-    const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(wp + (int64_t)nb * kWeightFrags * FRAG), 0,
-                                                                            kWeightFrags * 1024, 0x00020000);
+    const int piece = rows ? j * (27 * 32 * 2) + kg * 16 : lane * 16, frag = rows ? 32 : 1024;
+    __amdgpu_buffer_rsrc_t wrsrc;
+    if constexpr (COLUMNS) wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(wp), 0, 32 * 27 * a.cout * 2, 0x00020000);
+    else wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(wp + (int64_t)nb * kWeightFrags * FRAG), 0, kWeightFrags * 1024, 0x00020000);
 #pragma unroll
     for (int k = 0; k < (kWeightFrags + 3) / 4; ++k) {
       const int f = wave + 4 * k;  // wave-uniform
       if (f < kWeightFrags) {
         char* dst = f < kWeightInPair ? pair2 + f * 1024 : wrest + (f - kWeightInPair) * 1024;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(wrsrc, (__attribute__((address_space(3))) void*)dst, 16, f * 1024 + lane * 16, 0, 0, 0);
+        int at = f * frag + piece;
+        if constexpr (COLUMNS) at = (((f & 1) * 16 + (lane >> 2)) * 27 + 26 - (f >> 1)) * a.cout * 2 + nb * 64 + (lane & 3) * 16;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wrsrc, (__attribute__((address_space(3))) void*)dst, 16, at, 0, 0, 0);
       }
     }
   }
@@ -457,8 +466,15 @@ conv_ring_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ 
 #pragma unroll
       for (int tap = 0; tap < 27; ++tap) {
         const int f0 = 2 * tap, f1 = 2 * tap + 1;
-        wq[tap] = *reinterpret_cast<const uint4*>((f0 < kWeightInPair ? pair2 + f0 * 1024 : wrest + (f0 - kWeightInPair) * 1024) + lane * 16);
-        wa[tap] = *reinterpret_cast<const ring_i32x4_t*>((f1 < kWeightInPair ? pair2 + f1 * 1024 : wrest + (f1 - kWeightInPair) * 1024) + lane * 16);
+        const char* from0 = f0 < kWeightInPair ? pair2 + f0 * 1024 : wrest + (f0 - kWeightInPair) * 1024;
+        const char* from1 = f1 < kWeightInPair ? pair2 + f1 * 1024 : wrest + (f1 - kWeightInPair) * 1024;
+        if constexpr (COLUMNS) {
+          wq[tap] = tr_fragment<T>(reinterpret_cast<const T*>(from0), 32, lane);
+          wa[tap] = __builtin_bit_cast(ring_i32x4_t, tr_fragment<T>(reinterpret_cast<const T*>(from1), 32, lane));
+        } else {
+          wq[tap] = *reinterpret_cast<const uint4*>(from0 + lane * 16);
+          wa[tap] = *reinterpret_cast<const ring_i32x4_t*>(from1 + lane * 16);
+        }
       }
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the copies are in registers ...
       __syncthreads();                     // ... in every wavefront, before the first step's loads may overwrite them
@@ -534,21 +550,25 @@ RingGeom ring_geom(const MfmaConvArgs& a) {
 }
 
 template <typename T>
-int launch_ring(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
+int launch_ring(const MfmaConvArgs& a, const void* x, const void* w, MfmaWeight form, const void* bias, void* y, hipStream_t st,
                 const GnPartialOut& gn, const ChannelPair& out2) {
   const RingGeom gm = ring_geom(a);
   if (gm.items < 0) return fail(SFH_ERR_UNSUPPORTED, "conv mfma: too many columns");
   if (gm.items == 0) return SFH_OK;
   const unsigned grid = (unsigned)(gm.parts * gm.wgs * gm.nblocks);
-#define SFH_RING(BIAS, GN)                                                                                                  \
-  hipLaunchKernelGGL((conv_ring_kernel<T, BIAS, GN>), dim3(grid), dim3(256), 0, st, a, (const T*)x, (const T*)packed, \
+  const int rows = form == MfmaWeight::kRows;
+#define SFH_RING(BIAS, GN, COLUMNS)                                                                                              \
+  hipLaunchKernelGGL((conv_ring_kernel<T, BIAS, GN, COLUMNS>), dim3(grid), dim3(256), 0, st, a, (const T*)x, (const T*)w, rows, \
                      (const T*)bias, (T*)y, gm, gn, (T*)out2.second, out2.first)
-  if (bias != nullptr) {
-    if (gn.part != nullptr) SFH_RING(true, true);
-    else SFH_RING(true, false);
+  if (form == MfmaWeight::kColumns) {  // a data gradient's: it has neither bias nor records
+    if (bias != nullptr || gn.part != nullptr) return fail(SFH_ERR_UNSUPPORTED, "conv ring: a transposed weight with bias or GroupNorm partials");
+    SFH_RING(false, false, true);
+  } else if (bias != nullptr) {
+    if (gn.part != nullptr) SFH_RING(true, true, false);
+    else SFH_RING(true, false, false);
   } else {
-    if (gn.part != nullptr) SFH_RING(false, true);
-    else SFH_RING(false, false);
+    if (gn.part != nullptr) SFH_RING(false, true, false);
+    else SFH_RING(false, false, false);
   }
 #undef SFH_RING
   return check_launch("conv_ring_kernel");
@@ -568,10 +588,10 @@ int mfma_conv_ring_records(const MfmaConvArgs& a) {
   return gm.items > 0 && gm.parts == a.n ? gm.wgs : 0;
 }
 
-int mfma_conv_ring(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
-                   const GnPartialOut& gn, const ChannelPair& out2) {
-  if (dtype == SFH_BF16) return launch_ring<bf16_t>(a, x, packed, bias, y, st, gn, out2);
-  return launch_ring<fp16_t>(a, x, packed, bias, y, st, gn, out2);
+int mfma_conv_ring(const MfmaConvArgs& a, int dtype, const void* x, const void* w, MfmaWeight form, const void* bias, void* y,
+                   hipStream_t st, const GnPartialOut& gn, const ChannelPair& out2) {
+  if (dtype == SFH_BF16) return launch_ring<bf16_t>(a, x, w, form, bias, y, st, gn, out2);
+  return launch_ring<fp16_t>(a, x, w, form, bias, y, st, gn, out2);
 }
 
 }  // namespace sfh
