@@ -154,7 +154,8 @@ int sfh_mfma_ceiling_probe(int32_t mix, int32_t workgroups, int32_t tiles, const
  * kernel _conv3d_fwd_kernel (gather_gemm.py:112).
  * y[n,co,od,oh,ow] = bias[co] + sum_{ci,kd,kh,kw} x[n,ci,od*sd+kd*dd-pd,...] * w[co,ci,kd,kh,kw]
  * bias may be NULL; when given it has Cout elements of the activation dtype.
- * The workspace holds the weight repacked into MFMA fragment order (16-bit and fp32 tiled problems). */
+ * The workspace holds the weight repacked into MFMA fragment order (16-bit and fp32 tiled problems); most channels-last weights of
+ * fp32 and of 32 reduction channels are read where they lie, and it stays unused. */
 size_t sfh_conv3d_fwd_workspace_bytes(const sfh_conv3d_desc* p, int dtype);
 int sfh_conv3d_fwd(const sfh_conv3d_desc* p, int dtype, const void* x, const void* w,
                    const int64_t w_stride[5], const void* bias, void* y, void* workspace,

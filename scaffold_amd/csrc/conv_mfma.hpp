@@ -59,7 +59,7 @@ int mfma_conv_split(const MfmaConvArgs& a, int dtype, const void* x, const void*
                     const GnPartialOut* gn = nullptr, const ChannelPair* in2 = nullptr, const ChannelPair* out2 = nullptr);
 int mfma_conv_split_gn_records(const MfmaConvArgs& a, int groups);
 bool mfma_conv_split_pair_ok(const MfmaConvArgs& a, int first, bool as_output);
-// How the column-walking kernel reads the weight: packed, or a channels-last one where it lies, [produced][tap][reduction] or
+// How the two kernels of 32 reduction channels read the weight: packed, or a channels-last one where it lies, [produced][tap][reduction] or
 // [reduction][tap][produced] with the taps back to front.
 enum class MfmaWeight { kPacked, kRows, kColumns };
 // The form of a weight of these strides (elements; Cout, Cin, kd, kh, kw); kPacked: it has to be packed first.

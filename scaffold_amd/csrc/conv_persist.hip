@@ -306,9 +306,10 @@ __device__ __forceinline__ void persist_step(const MfmaConvArgs& a, const char* 
   }
 }
 
-template <typename T, typename C, bool BIAS, bool GN>
+// wp: the packed weight, with `rows` a channels-last weight [out][tap][32], with COLUMNS one [32][tap][out] whose taps run back to front.
+template <typename T, typename C, bool BIAS, bool GN, bool COLUMNS>
 __global__ void __launch_bounds__(256, 1)
-conv_persist_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ wp, const T* __restrict__ bias_ptr,
+conv_persist_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ wp, int rows, const T* __restrict__ bias_ptr,
                     T* __restrict__ y, PersistGeom gm, GnPartialOut gn, T* __restrict__ y1, int c_first) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses LDS address-space builtins the host pass cannot type-check
   __shared__ __attribute__((aligned(16))) char buf0[C::BRICK];
@@ -356,16 +357,26 @@ conv_persist_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict
     lg.grel[k] = (((bd * a.ih + bh) * a.iw + bw) * a.cred) * 2;
   }
 
-  constexpr int FRAG = 512;
-  const T* wblock = wp + (int64_t)nb * C::NIT * FRAG + lane * 8;
-  // The first NVEC fragments live in vector registers, the rest in accumulation registers (there are not 216 + the
-  // activation fragments' worth of vector registers; the MFMA reads its row operand from either file).
-  uint4 wq[C::NVEC];
-  sfh_i32x4_t wa[C::NIT - C::NVEC];
+  // The block's fragments come into LDS once per workgroup, into the buffer that the first step fills, beside the first brick; every
+  // wavefront takes its copy from there. A channels-last weight comes from where it lies, without a packing launch, as in conv_ring.hip.
+  // us, packed -> as it lies, forward and data gradient: 32 -> 32 at 16^3 11.7 -> 8.9 and 11.8 -> 9.1, at 64x64x16 12.9 -> 10.1 and 13.0 -> 10.2, 64
+  // channels at 70x40x9 12.6 -> 9.7 and 12.3 -> 9.9, 32 -> 32 at 128x128x16 21.0 -> 18.1 and 20.9 -> 18.3.
+  static_assert(C::NIT * 1024 <= C::BRICK, "the weights in a brick's LDS");
+  {
+    const int piece = rows ? j * (27 * 32 * 2) + kg * 16 : lane * 16, frag = rows ? 32 : 1024;
+    __amdgpu_buffer_rsrc_t wrsrc;
+    if constexpr (COLUMNS) wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(wp), 0, 32 * 27 * a.cout * 2, 0x00020000);
+    else wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(wp + (int64_t)nb * C::NIT * 512), 0, C::NIT * 1024, 0x00020000);
 #pragma unroll
-  for (int it = 0; it < C::NVEC; ++it) wq[it] = *reinterpret_cast<const uint4*>(wblock + it * FRAG);
-#pragma unroll
-  for (int it = C::NVEC; it < C::NIT; ++it) wa[it - C::NVEC] = *reinterpret_cast<const sfh_i32x4_t*>(wblock + it * FRAG);
+    for (int k = 0; k < (C::NIT + 3) / 4; ++k) {
+      const int f = wave + 4 * k;  // wave-uniform
+      if (f < C::NIT) {
+        int at = f * frag + piece;
+        if constexpr (COLUMNS) at = (((f & 1) * 16 + (lane >> 2)) * 27 + 26 - (f >> 1)) * a.cout * 2 + nb * 64 + (lane & 3) * 16;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wrsrc, (__attribute__((address_space(3))) void*)(buf1 + f * 1024), 16, at, 0, 0, 0);
+      }
+    }
+  }
   float bias[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) bias[r] = BIAS ? to_float(bias_ptr[nb * 32 + 8 * (r / 4) + 4 * kg + (r % 4)]) : 0.f;
@@ -379,8 +390,22 @@ conv_persist_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict
   TileCoord tc1 = next_tile(tc, gm);
 #pragma unroll
   for (int k = 0; k < C::GPW; ++k) voff[k] = brick_group_offset<C>(a, tc1, nsteps > 1, lg.gcoord[k], lg.grel[k]);
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // this wave's part of the first brick has landed
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // this wave's part of the first brick and of the weights has landed
   __syncthreads();
+  // The first NVEC fragments live in vector registers, the rest in accumulation registers (there are not 216 + the
+  // activation fragments' worth of vector registers; the MFMA reads its row operand from either file).
+  uint4 wq[C::NVEC];
+  sfh_i32x4_t wa[C::NIT - C::NVEC];
+  auto fragment = [&](int it) -> uint4 {
+    if constexpr (COLUMNS) return tr_fragment<T>(reinterpret_cast<const T*>(buf1 + it * 1024), 32, lane);
+    return *reinterpret_cast<const uint4*>(buf1 + it * 1024 + lane * 16);
+  };
+#pragma unroll
+  for (int it = 0; it < C::NVEC; ++it) wq[it] = fragment(it);
+#pragma unroll
+  for (int it = C::NVEC; it < C::NIT; ++it) wa[it - C::NVEC] = __builtin_bit_cast(sfh_i32x4_t, fragment(it));
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the copies are in registers ...
+  __syncthreads();                     // ... in every wavefront, before the first step's loads may overwrite them
 
   f32x16_t acc[C::MS];
   PendingStore<C> ps;
@@ -451,32 +476,36 @@ PersistGeom persist_geom(const MfmaConvArgs& a) {
 }
 
 template <typename T, typename C>
-int launch_tile(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
+int launch_tile(const MfmaConvArgs& a, const void* x, const void* w, MfmaWeight form, const void* bias, void* y, hipStream_t st,
                 const GnPartialOut& gn, const ChannelPair& out2) {
   const PersistGeom gm = persist_geom(a, C::TD, C::TH, C::TW);
   if (gm.ntiles < 0) return fail(SFH_ERR_UNSUPPORTED, "conv mfma: too many bricks");
   if (gm.ntiles == 0) return SFH_OK;
   const unsigned grid = (unsigned)(gm.wgs_per_block * gm.nblocks);
-#define SFH_PERSIST(BIAS, GN)                                                                                                    \
-  hipLaunchKernelGGL((conv_persist_kernel<T, C, BIAS, GN>), dim3(grid), dim3(256), 0, st, a, (const T*)x, (const T*)packed, \
+  const int rows = form == MfmaWeight::kRows;
+#define SFH_PERSIST(BIAS, GN, COLUMNS)                                                                                                 \
+  hipLaunchKernelGGL((conv_persist_kernel<T, C, BIAS, GN, COLUMNS>), dim3(grid), dim3(256), 0, st, a, (const T*)x, (const T*)w, rows, \
                      (const T*)bias, (T*)y, gm, gn, (T*)out2.second, out2.first)
-  if (bias != nullptr) {
-    if (gn.part != nullptr) SFH_PERSIST(true, true);
-    else SFH_PERSIST(true, false);
+  if (form == MfmaWeight::kColumns) {  // a data gradient's: it has neither bias nor records
+    if (bias != nullptr || gn.part != nullptr) return fail(SFH_ERR_UNSUPPORTED, "conv persist: a transposed weight with bias or GroupNorm partials");
+    SFH_PERSIST(false, false, true);
+  } else if (bias != nullptr) {
+    if (gn.part != nullptr) SFH_PERSIST(true, true, false);
+    else SFH_PERSIST(true, false, false);
   } else {
-    if (gn.part != nullptr) SFH_PERSIST(false, true);
-    else SFH_PERSIST(false, false);
+    if (gn.part != nullptr) SFH_PERSIST(false, true, false);
+    else SFH_PERSIST(false, false, false);
   }
 #undef SFH_PERSIST
   return check_launch("conv_persist_kernel");
 }
 
 template <typename T>
-int launch_typed(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
+int launch_typed(const MfmaConvArgs& a, const void* x, const void* w, MfmaWeight form, const void* bias, void* y, hipStream_t st,
                  const GnPartialOut& gn, const ChannelPair& out2) {
-  if (a.ow > 16) return launch_tile<T, PTile<4, 4, 32>>(a, x, packed, bias, y, st, gn, out2);
-  if (a.ow > 8) return launch_tile<T, PTile<4, 8, 16>>(a, x, packed, bias, y, st, gn, out2);
-  return launch_tile<T, PTile<8, 8, 8>>(a, x, packed, bias, y, st, gn, out2);
+  if (a.ow > 16) return launch_tile<T, PTile<4, 4, 32>>(a, x, w, form, bias, y, st, gn, out2);
+  if (a.ow > 8) return launch_tile<T, PTile<4, 8, 16>>(a, x, w, form, bias, y, st, gn, out2);
+  return launch_tile<T, PTile<8, 8, 8>>(a, x, w, form, bias, y, st, gn, out2);
 }
 
 }  // namespace
@@ -521,7 +550,7 @@ bool mfma_conv_pair_ok(const MfmaConvArgs& a, int first, bool as_output) {
 }
 
 MfmaWeight mfma_conv_weight_form(const MfmaConvArgs& a, const void* w, const int64_t w_stride[5], bool dgrad) {
-  if (!mfma_conv_persist_applies(a) || !ring_serves(a) || a.cout > 65536) return MfmaWeight::kPacked;
+  if (!mfma_conv_persist_applies(a) || a.cout > 65536) return MfmaWeight::kPacked;
   const int64_t cin = dgrad ? a.cout : a.cred;
   const bool dense = w_stride[1] == 1 && w_stride[4] == cin && w_stride[3] == 3 * cin && w_stride[2] == 9 * cin && w_stride[0] == 27 * cin;
   if (!dense || (reinterpret_cast<uintptr_t>(w) & 15u) != 0) return MfmaWeight::kPacked;
@@ -530,8 +559,7 @@ MfmaWeight mfma_conv_weight_form(const MfmaConvArgs& a, const void* w, const int
 
 int mfma_conv_persist(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y,
                       void* partial, hipStream_t st, const GnPartialOut* gn, const ChannelPair* in2, const ChannelPair* out2, MfmaWeight form) {
-  if (form != MfmaWeight::kPacked && !(mfma_conv_persist_applies(a) && ring_serves(a)))
-    return fail(SFH_ERR_INVALID, "conv mfma: this problem reads a packed weight");
+  if (form != MfmaWeight::kPacked && !mfma_conv_persist_applies(a)) return fail(SFH_ERR_INVALID, "conv mfma: this problem reads a packed weight");
   if (!mfma_conv_persist_applies(a)) return mfma_conv_gather(a, dtype, x, packed, bias, y, partial, st, gn, in2, out2);
   if (in2 != nullptr) return fail(SFH_ERR_UNSUPPORTED, "conv persist: 32 reduction channels cannot be a pair of tensors");
   if (out2 != nullptr && (out2->second == nullptr || !mfma_conv_pair_ok(a, out2->first, true)))
@@ -546,8 +574,8 @@ int mfma_conv_persist(const MfmaConvArgs& a, int dtype, const void* x, const voi
     out.cg = a.cout / gn->groups;
   }
   if (ring_serves(a)) return mfma_conv_ring(a, dtype, x, packed, form, bias, y, st, out, pair);
-  if (dtype == SFH_BF16) return launch_typed<bf16_t>(a, x, packed, bias, y, st, out, pair);
-  return launch_typed<fp16_t>(a, x, packed, bias, y, st, out, pair);
+  if (dtype == SFH_BF16) return launch_typed<bf16_t>(a, x, packed, form, bias, y, st, out, pair);
+  return launch_typed<fp16_t>(a, x, packed, form, bias, y, st, out, pair);
 }
 
 }  // namespace sfh

@@ -1,5 +1,5 @@
-"""Convolutions of 32 reduction channels over rows of more than 16 voxels read a channels-last weight where it lies and pack any
-other: the same bits either way."""
+"""Convolutions of 32 reduction channels read a channels-last weight where it lies and pack any other: the same bits either way.
+Rows of more than 16 voxels and shorter ones have kernels of their own."""
 
 import pytest
 import torch
@@ -23,7 +23,8 @@ def _weight(g, cout, cin, dtype):
 
 @pytest.mark.parametrize("layout", ["first", "shifted"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("n,wide,spatial", [(1, 32, (4, 8, 32)), (1, 96, (5, 9, 33)), (2, 64, (3, 7, 17)), (1, 32, (40, 24, 65))])
+@pytest.mark.parametrize("n,wide,spatial", [(1, 32, (4, 8, 32)), (1, 96, (5, 9, 33)), (2, 64, (3, 7, 17)), (1, 32, (40, 24, 65)), (1, 32, (4, 8, 16)),
+                                            (1, 96, (33, 9, 13)), (2, 64, (3, 5, 7)), (1, 32, (40, 41, 8))])
 def test_forms_of_a_weight(n, wide, spatial, dtype, layout):
     g = torch.Generator(device="cuda").manual_seed(5)
     cl = torch.channels_last_3d
