@@ -403,19 +403,22 @@ WidePlan wide_plan(const MfmaConvArgs& a) {
   // Measured against the brick-per-workgroup kernel on every shape of the U-Net and of the cube configurations, this
   // kernel wins where a 64-channel output meets 128 or more reduction channels (one workgroup then produces all of a
   // voxel's channels from one staged brick): 8 x 2 accumulator blocks per wavefront when such workgroups fill the
-  // chip, else 4 x 2. Everything else stays with the other kernels.
+  // chip, else 4 x 2. Everything else stays with the other kernels. The depth counted is that of a shard's planes in both forms of
+  // its gradients, here and below: where the slab's own decided, the padded volume's gradient could be the small-volume kernel's,
+  // which adds in another order (of 64 -> 128 channels at 27x61x33: 256 workgroups of 4x4x32 for the slab, 224 for the volume). An odd
+  // number of chunks never goes there: this kernel and the bricks add alike.
+  MfmaConvArgs core = a;
+  if (a.cred % 64 == 0 && a.id < a.od) core.od = a.id;
   if (a.cout == 64 && a.cred >= 128) {
-    if (wide_workgroups(a, 1) >= kComputeUnits) shape = 1;
-    else if (wide_workgroups(a, 3) >= kComputeUnits) shape = 3;
+    if (wide_workgroups(core, 1) >= kComputeUnits) shape = 1;
+    else if (wide_workgroups(core, 3) >= kComputeUnits) shape = 3;
   }
   if (shape < 0) return p;
   p.fits = true;
   // Past two rounds of workgroups the brick kernel takes its place where 8 x 4 x 32 leaves more over than that kernel's choice of
   // brick, by the busiest CU's share (at equal shares it is the faster one by some 3 % for 128 channels, the slower by 5 for 256).
   // us, here -> there: 128 -> 64 at 96x80x112 353 -> 315, at 100^3 485 -> 387, at 90^3 331 -> 309, at 128^3 761 -> 739; 256 -> 64 at
-  // 64^3 171 -> 180. As for the small volumes the depth counted is that of a shard's planes in both forms of its gradients.
-  MfmaConvArgs core = a;
-  core.od = a.id < a.od ? a.id : a.od;
+  // 64^3 171 -> 180.
   const int64_t wgs = wide_workgroups(core, 1);
   if (a.cred % 64 == 0 && wgs > 2 * kComputeUnits &&  // (half of the channels in whole chunks: both kernels take the same pairs)
       mfma_conv_brick_cost(core) * 100 < cdiv(wgs, kComputeUnits) * 1024 * 2 * 100 * (a.cred < 256 ? 97 : 92)) return p;

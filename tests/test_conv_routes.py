@@ -1,5 +1,7 @@
 """Which kernel a convolution's volume goes to, where two rules meet: the launch query is a pure function of the problem."""
 
+import random
+
 import pytest
 import torch
 
@@ -39,6 +41,20 @@ def test_deep_thin_volumes(cin, cout, spatial, kernel):
     padded = _kernel(1, cout, cin, spatial, "bwd-data")
     d, h, w = spatial
     assert padded == kernel and _kernel(1, cout, cin, (d + 2, h, w), "bwd-data", (0, 1, 1)) == padded
+
+
+@pytest.mark.parametrize("cin,cout", [(64, 128), (64, 192), (64, 256), (64, 512), (64, 64), (128, 128), (256, 128), (512, 256)])
+def test_slab_and_padded_volume_add_in_one_order(cin, cout):
+    """Both forms of a depth shard's convolution, and of its data gradient, are the small-volume kernel's (four partial sums to a
+    voxel) or neither is: bits must not depend on the form.  The other kernels add in one chain."""
+    rng = random.Random(cin + cout)
+    shapes = [(27, 61, 33), (47, 37, 36), (39, 45, 35), (9, 27, 50), (17, 36, 35), (33, 57, 50)]
+    shapes += [tuple(round(4 * 16 ** rng.random()) for _ in range(3)) for _ in range(400)]
+    for d, h, w in shapes:
+        for direction in ("fwd", "bwd-data"):
+            padded = _kernel(1, cin, cout, (d, h, w), direction)
+            slab = _kernel(1, cin, cout, (d + 2, h, w), direction, (0, 1, 1))
+            assert (padded == "split") == (slab == "split"), (direction, (d, h, w), padded, slab)
 
 
 def test_fp32_weight_gradient_of_long_rows():

@@ -51,3 +51,46 @@ def test_slab_and_padded_volume_agree(cin, cout, spatial):
     slab[:, :, 1:-1] = x
     assert torch.equal(sa.conv3d_forward(slab, w, None, 1, (0, 1, 1)), sa.conv3d_forward(x, w, None, 1, 1))
     assert torch.equal(sa.conv3d_backward_data(gy, w, slab.shape, 1, (0, 1, 1))[:, :, 1:-1], sa.conv3d_backward_data(gy, w, x.shape, 1, 1))
+
+
+def _conv64(x, w):
+    """The 3x3x3 convolution of padding 1 in float64: a matrix product a tap."""
+    n, c, d, h, wd = x.shape
+    xp = torch.nn.functional.pad(x.double().permute(0, 2, 3, 4, 1), (0, 0, 1, 1, 1, 1, 1, 1))
+    w64 = w.double()
+    y = torch.zeros((n * d * h * wd, w.shape[0]), dtype=torch.float64, device=x.device)
+    for kd in range(3):
+        for kh in range(3):
+            for kw in range(3):
+                rows = xp[:, kd:kd + d, kh:kh + h, kw:kw + wd].reshape(-1, c).contiguous()
+                y += rows @ w64[:, :, kd, kh, kw].t().contiguous()
+    return y.view(n, d, h, wd, -1).permute(0, 4, 1, 2, 3)
+
+
+@pytest.mark.parametrize("cin,cout,spatial,fwd,dgrad", [
+    (64, 128, (27, 61, 33), "brick", "split"),   # planes past 32 x 32; the slab's data gradient was the wide kernel's
+    (64, 64, (9, 27, 50), "split", "split"),     # ... from 240 pairs on
+    (64, 64, (8, 27, 50), "brick", "brick"),     # 196
+    (64, 128, (14, 13, 6), "split", "brick"),    # few pairs of 128 and more produced channels
+    (128, 128, (4, 6, 12), "brick", "brick"),    # 16 pairs: too few
+    (512, 512, (9, 9, 6), "split", "split"),     # a long reduction by the times
+    (128, 64, (33, 57, 50), "brick", "brick"),   # bricks in the wide kernel's place by the times
+    (128, 64, (31, 61, 65), "wide", "brick"),
+])
+def test_lines_that_the_times_draw(cin, cout, spatial, fwd, dgrad):
+    x, gy, w = _operands(1, cin, cout, spatial, torch.bfloat16)
+    d, h, wd = spatial
+    shapes = (((1, cin, d, h, wd), 1), ((1, cin, d + 2, h, wd), (0, 1, 1)))
+    geom = {k: [c3.launch_geometry(s, w.shape, 1, p, 1, torch.bfloat16, k) for s, p in shapes] for k in ("fwd", "bwd-data")}
+    assert [g["kernel"] for g in geom["fwd"]] == [fwd] * 2 and [g["kernel"] for g in geom["bwd-data"]] == [dgrad] * 2
+    slab = torch.zeros(shapes[1][0], dtype=x.dtype, device="cuda").contiguous(memory_format=CL)
+    slab[:, :, 1:-1] = x
+    for direction, got, from_slab, want in (
+            ("fwd", sa.conv3d_forward(x, w, None, 1, 1), sa.conv3d_forward(slab, w, None, 1, (0, 1, 1)), _conv64(x, w)),
+            ("bwd-data", sa.conv3d_backward_data(gy, w, x.shape, 1, 1), sa.conv3d_backward_data(gy, w, slab.shape, 1, (0, 1, 1))[:, :, 1:-1],
+             _conv64(gy, w.flip(2, 3, 4).transpose(0, 1)))):
+        # one rounding of the result on top of an fp32 sum of up to 27 * 512 terms
+        for result in (got, from_slab):
+            assert torch.all((result.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * want.abs().max())
+        if len({g["slices"] for g in geom[direction]}) == 1:  # (slices are cut by a launch's own planes)
+            assert torch.equal(got, from_slab)
