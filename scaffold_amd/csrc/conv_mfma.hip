@@ -753,6 +753,7 @@ size_t mfma_conv_partial_bytes(const MfmaConvArgs& a) {
 }
 
 int64_t mfma_conv_brick_cost(const MfmaConvArgs& a) { return cut_plan(a).cost; }
+int mfma_conv_brick_slices(const MfmaConvArgs& a) { return cut_plan(a).ksplit; }
 int64_t mfma_conv_brick_time(const MfmaConvArgs& a) { return brick_time(a, gather_plan(a)); }
 
 MfmaConvGeometry mfma_conv_gather_geometry(const MfmaConvArgs& a) {

@@ -92,6 +92,7 @@ bool mfma_conv_persist_applies(const MfmaConvArgs& a);
 MfmaConvGeometry mfma_conv_gather_geometry(const MfmaConvArgs& a);
 // What the brick kernel's launch rule reckons for a problem: output voxels x 32-channel blocks of the busiest CU, in hundredths.
 int64_t mfma_conv_brick_cost(const MfmaConvArgs& a);
+int mfma_conv_brick_slices(const MfmaConvArgs& a);  // the slices it cuts the reduction into
 int64_t mfma_conv_brick_time(const MfmaConvArgs& a);  // what its launch takes, in hundredths of a us
 MfmaConvGeometry mfma_conv_wide_geometry(const MfmaConvArgs& a);
 MfmaConvGeometry mfma_conv_split_geometry(const MfmaConvArgs& a);

@@ -364,23 +364,24 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
 // long reduction lose (512 -> 512 at 8^3, 64 pairs: 17.4 -> 23.2; 256 -> 256 at 4x8x8, 16 pairs: 10.1 -> 10.6), so the line is higher for
 // those. Some below it would gain as well (128 -> 128 at 8^3, 16 pairs: 9.7 -> 7.7; 256 -> 128 at 8x16x16, 64: 14.9 -> 11.4; 512 -> 256 at
 // 8x16x16, 128: 27.8 -> 22.9): their sliced geometry is what the tests of the launch query hold the last two to.
-// Past three rounds of pairs the brick kernel's launches have no slices either and stage less: such a volume comes here only where what
-// either launch takes says so, within a tenth. us, bricks -> here: 64 -> 64 at 256x16x16 (1024 pairs) 19.2 -> 21.2, 128 -> 128 at 128x16x16 31.0 -> 33.9,
-// 256 -> 256 at 32^3 102 -> 109; 128 -> 64 at 200x20x20 (1500 pairs) 56 -> 46, 64 -> 64 at 64x24x24 (576 pairs) 17.9 -> 16.0. So do planes past the line,
-// from about a round of pairs on, by more than a tenth: 64 -> 64 at 17x36x35 15.9 -> 9.7, at 9x27x50 12.1 -> 7.9, 128 -> 128 at 10x28x56 25.8 -> 17.0, 128 -> 256 at
+// Past three rounds of pairs the brick kernel's launches have no slices either and stage less: a volume below the plane's line comes here only
+// where the bricks leave more over, by the busiest CU's share, than the 10 % that 64-voxel bricks lose at equal shares, or where what either launch
+// takes says so within a tenth. us, bricks -> here: 64 -> 64 at 256x16x16 (1024 pairs, equal shares) 19.2 -> 21.2, 128 -> 128 at 128x16x16 31.0 -> 33.9; 128 -> 64
+// at 200x20x20 (1500 pairs, 768 against 993 voxel blocks) 56 -> 46, 64 -> 64 at 64x24x24 (576 pairs) 17.9 -> 16.0. Planes past 32 x 32 come here by the times,
+// from about a round of pairs on and by more than a tenth: 64 -> 64 at 17x36x35 15.9 -> 9.7, at 9x27x50 12.1 -> 7.9, 128 -> 128 at 10x28x56 25.8 -> 17.0, 128 -> 256 at
 // 11x27x45 42.8 -> 30.6.
+// The times take nothing away from this kernel: its four partial sums to a voxel are nearer the 64-bit result than the bricks' one chain (fp16
+// results of 64 to 512 channels that are not the rounded 64-bit ones: 1.5e-3 here, 1.9e-3 in bricks, 28 problems of both directions), so 256 -> 256 at 32^3 stays at
+// 109 us though bricks take 102. Nor do they bring it what the bricks sum in eight slices (1.35e-3 there, 1.75e-3 here; four: level).
 // The data gradient of a depth shard's slab (D + 2 planes from D) and of the padded volume (D from D) must come from the same
 // kernel, or a shard and the whole volume would disagree in the last bit: the depth counted is the smaller of the two.
 constexpr int kSplitMaxPlane = 32 * 32, kSplitMinPerDepth = 24, kSplitFewPerDepth = 32, kSplitFewMaxChunks = 16;
 constexpr int kSplitBigPlanePairs = 240;
-// Pairs from which a volume below the plane line comes here. Levels of 128 and more produced channels need fewer: us, slices and their sum ->
-// here, 64 -> 128 at 14x13x6 (56 pairs) 9.9 -> 5.6, at 5x10x11 (36) 10.0 -> 5.5, 128 -> 128 at 9x12x8 (30) 13.2 -> 7.7, at 4x6x20 (24) 11.5 -> 7.7, 256 -> 256 at
-// 9x10x7 (60) 14.0 -> 11.5. Long reductions on fewer where the slices are far behind: 512 -> 512 at 9x9x6 (120) 35.1 -> 22.1.
-int64_t split_line(int chunks, int cout) {
-  if (chunks <= 4) return cout >= 128 ? 24 : kComputeUnits / 4;
-  if (chunks <= 8) return cout >= 256 ? 48 : kComputeUnits / 4 + 1;
-  return kComputeUnits / 2 + 1;
-}
+// Pairs from which a volume below the plane's line comes here, and the fewer from which it does where the bricks need at most four slices. us, slices
+// and their sum -> here: 64 -> 128 at 14x13x6 (56 pairs) 9.9 -> 5.6, at 5x10x11 (36) 10.0 -> 5.5, 128 -> 128 at 9x12x8 (30) 13.2 -> 7.7, at 4x6x20 (24) 11.5 -> 7.7.
+// Long reductions on fewer where the slices are far behind: 512 -> 512 at 9x9x6 (120) 35.1 -> 22.1.
+int64_t split_line(int chunks) { return chunks <= 4 ? kComputeUnits / 4 : chunks <= 8 ? kComputeUnits / 4 + 1 : kComputeUnits / 2 + 1; }
+int64_t split_line_few_slices(int chunks, int cout) { return chunks <= 4 && cout >= 128 ? 24 : chunks <= 8 && cout >= 256 ? 48 : split_line(chunks); }
 
 bool mfma_conv_split_applies(const MfmaConvArgs& a) {
   if (a.kd != 3 || a.kh != 3 || a.kw != 3) return false;
@@ -390,12 +391,14 @@ bool mfma_conv_split_applies(const MfmaConvArgs& a) {
   core.od = a.id < a.od ? a.id : a.od;
   const int64_t per_depth = (int64_t)a.n * cdiv(a.oh, Flat::TH) * cdiv(a.ow, Flat::TW) * pair;
   const int64_t pairs = per_depth * cdiv(core.od, Flat::TD), rounds = cdiv(pairs, kComputeUnits);
-  const int64_t time = split_time(split_tiles(core) * pair, chunks);
-  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return pairs > kSplitBigPlanePairs && 100 * time < 88 * mfma_conv_brick_time(core);
+  auto sooner = [&](int percent) { return 100 * split_time(split_tiles(core) * pair, chunks) < percent * mfma_conv_brick_time(core); };
+  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return pairs > kSplitBigPlanePairs && sooner(88);
   const bool few = per_depth <= kSplitFewPerDepth && chunks >= kSplitFewMaxChunks;
-  if (pairs < split_line(chunks, a.cout) && (few || per_depth < kSplitMinPerDepth))
-    return chunks >= kSplitFewMaxChunks && 100 * time < 70 * mfma_conv_brick_time(core);
-  return rounds <= 3 || 100 * time < 110 * mfma_conv_brick_time(core);
+  if (!few && per_depth >= kSplitMinPerDepth) return true;
+  if (pairs >= split_line(chunks))
+    return rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || sooner(110);
+  if (mfma_conv_brick_slices(core) > 4) return false;
+  return pairs >= split_line_few_slices(chunks, a.cout) || (chunks >= kSplitFewMaxChunks && sooner(70));
 }
 
 MfmaConvGeometry mfma_conv_split_geometry(const MfmaConvArgs&) { return MfmaConvGeometry{kKernelSplit, kBrickVoxels, kBlocks, 1}; }

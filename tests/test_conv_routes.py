@@ -57,6 +57,21 @@ def test_slab_and_padded_volume_add_in_one_order(cin, cout):
             assert (padded == "split") == (slab == "split"), (direction, (d, h, w), padded, slab)
 
 
+@pytest.mark.parametrize("cin,cout,spatial,kernel", [
+    (256, 256, (32, 32, 32), "split"),
+    (128, 128, (60, 30, 31), "split"),
+    (64, 64, (64, 32, 32), "split"),
+    (256, 256, (29, 28, 14), "split"),
+    (256, 256, (5, 8, 14), "brick"),     # eight slices
+    (256, 256, (11, 4, 9), "split"),     # four
+])
+def test_launch_times_take_no_partial_sums_away(cin, cout, spatial, kernel):
+    """Four partial sums to a voxel are nearer the exact one than the bricks' single chain, eight slices nearer still: where the
+    small-volume kernel served a volume, or the bricks in eight slices, no estimate of times moves it."""
+    for direction in ("fwd", "bwd-data"):
+        assert _kernel(1, cin, cout, spatial, direction) == kernel
+
+
 def test_fp32_weight_gradient_of_long_rows():
     """A row of 2 GiB and more: its offsets are 64-bit, the tiled kernel takes it (the untiled one makes no slices)."""
     assert c3.split_count((1, 32, 1, 1, 16_800_000), (32, 32, 3, 3, 3), 1, 1, 1, torch.float32) > 1
