@@ -632,11 +632,18 @@ bool ring_serves(const WgradArgs& a) { return mfma_wgrad_ring_applies(a); }
 // Rows of more than 16 voxels in a launch of their own: columns (rows in pieces of 32 voxels) or 4x8x8 tiles in planes (less work on
 // padding, a sooner start, a lower rate; where the blocks leave room for three workgroups each). Both by what their busiest workgroup
 // has to do: columns 20 us and 2.1 a step or item, tiles by the tile plan's own cost, fitted to 150 problems of 32 to 512 channels on
-// 4x8x17 to 128^3, both forms timed: a measured time is within 5 % (rms) of either estimate, 144 of them take the faster form or one 3 %
-// slower, the worst is 128 -> 256 at 6x31x21 (columns 31.8, tiles 29.1). Columns / tiles, us: 32 -> 32 at 32^3 21.6 / 14.4, at 114x95x31 33.5 / 36.7, at 64^3
+// 4x8x17 to 128^3, both forms timed: a measured time is within 5 % (rms) of either estimate. Columns / tiles, us: 32 -> 32 at 32^3 21.6 / 14.4, at 114x95x31 33.5 / 36.7, at 64^3
 // 28.4 / 29.7, at 96x80x112 54.3 / 71.0, two samples at 44x60x75 40.3 / 48.0, 64 -> 64 at 16x32x32 28.1 / 17.0, 128 -> 128 at 9x16x59 30.1 / 26.4, 256 -> 256 at
 // two samples of 6x9x40 45.6 / 64.7. Relative error against 64 bits, e-7: 32 -> 32 at 32^3 1.16 / 1.13, at 48x64x64 1.54 / 1.37, 128 -> 128 at 9x20x20 0.96 / 0.94.
-bool walks_columns(const WgradArgs& a, int64_t tile_plan_cost) { return 2000 + 210 * mfma_wgrad_ring_cost(a) <= tile_plan_cost; }
+// Columns sum the longer chains, so that estimate alone does not decide: of 40 problems that only it gives to columns their error is 1.17 times that of
+// tiles (geometric mean; 128 -> 128 at 43x29x34 1.9 -> 3.1e-7, 64 -> 32 at 54x40x76 1.5 -> 1.9) for 0.92 of the time. They are walked where an estimate from padded operations
+// (20 us, 25 where rows are cut, and 0.7 a GFLOP against 12.5 and 1.25, fitted to 35 problems) finds them quicker as well, or quicker than the tile plan's cost.
+bool walks_columns(const WgradArgs& a, int64_t tile_plan_cost) {
+  const double per_voxel = 54e-9 * a.cin * a.cout * a.n;
+  const double columns = (a.ow % 32 == 0 ? 20. : 25.) + 0.7 * per_voxel * (double)cdiv(a.od, 2) * 2 * (double)cdiv(a.oh, 4) * 4 * (double)cdiv(a.ow, 32) * 32;
+  const double tiles = 12.5 + 1.25 * per_voxel * (double)cdiv(a.od, 4) * 4 * (double)cdiv(a.oh, 8) * 8 * (double)cdiv(a.ow, 8) * 8;
+  return (columns <= tiles || 100 * columns <= (double)tile_plan_cost) && 2000 + 210 * mfma_wgrad_ring_cost(a) <= tile_plan_cost;
+}
 
 Plan make_plan(const WgradArgs& a) {
   Plan p{};

@@ -72,6 +72,17 @@ def test_launch_times_take_no_partial_sums_away(cin, cout, spatial, kernel):
         assert _kernel(1, cin, cout, spatial, direction) == kernel
 
 
+@pytest.mark.parametrize("n,cin,cout,spatial,slices", [
+    (1, 128, 128, (43, 29, 34), 5),     # tiles; columns would be 16 slices
+    (1, 64, 32, (54, 40, 76), 42),      # tiles; 120
+    (1, 32, 32, (104, 52, 79), 83),     # tiles; 234
+    (1, 32, 32, (96, 80, 112), 240),    # columns by both estimates
+])
+def test_weight_gradients_of_wide_rows_keep_the_tiles_shorter_sums(n, cin, cout, spatial, slices):
+    """Columns sum longer chains than tiles: they are walked where both estimates find them quicker, not where one does."""
+    assert c3.split_count((n, cin, *spatial), (cout, cin, 3, 3, 3), 1, 1, 1, torch.bfloat16) == slices
+
+
 def test_fp32_weight_gradient_of_long_rows():
     """A row of 2 GiB and more: its offsets are 64-bit, the tiled kernel takes it (the untiled one makes no slices)."""
     assert c3.split_count((1, 32, 1, 1, 16_800_000), (32, 32, 3, 3, 3), 1, 1, 1, torch.float32) > 1
