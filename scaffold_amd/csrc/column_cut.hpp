@@ -1,7 +1,7 @@
 // How many workgroups walk the columns of a volume: the launch rule of the kernels that step along depth and keep the
 // planes they have fetched (conv_ring.hip, wgrad_ring.hip).
 #pragma once
-#include "common.hpp"
+#include <cstdint>
 
 namespace sfh {
 
@@ -22,16 +22,32 @@ struct ColumnCut {
 // 32 -> 64 at 75x107x122 111 -> 92; weight gradient with its sum 32 -> 32 at 96x80x112 63.9 -> 54.3, 54x105x99 53.2 -> 47.0, two
 // samples of 57x87x77 72.5 -> 58.5, 64 -> 32 at 110x48x111 91.2 -> 69.9, 128 -> 64 at 60x35x45 76.4 -> 60.8.
 inline ColumnCut cut_columns(int64_t ncols, int64_t steps, int64_t wgs) {
+  auto parts = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   ColumnCut best{};
   best.items = -1;
-  const int64_t most = cdiv(4 * wgs, ncols);  // more than four items to a workgroup even nothing out any more
+  const int64_t most = parts(4 * wgs, ncols);  // more than four items to a workgroup even nothing out any more
   for (int64_t want = 1; want <= most && want <= steps; ++want) {
-    const int64_t len = cdiv(steps, want), segs = cdiv(steps, len), items = ncols * segs;
+    const int64_t len = parts(steps, want), segs = parts(steps, len), items = ncols * segs;
     if (items > 0x7fffffffLL) break;
-    const int64_t per_wg = cdiv(items, wgs), cost = per_wg * (len + 1);
-    if (best.items < 0 || cost < best.cost) best = ColumnCut{(int)segs, (int)len, (int)items, (int)per_wg, (int)cdiv(items, per_wg), cost};
+    const int64_t per_wg = parts(items, wgs), cost = per_wg * (len + 1);
+    if (best.items < 0 || cost < best.cost) best = ColumnCut{(int)segs, (int)len, (int)items, (int)per_wg, (int)parts(items, per_wg), cost};
   }
   return best;
+}
+
+// The cut of `n` samples of `cols` columns: one line of columns (parts 1), or every sample by workgroups of its own (parts n; the cut is that of
+// one), whose sums are then those of one sample, so that the normalisation behind the convolution needs no statistics pass. That is worth an
+// end up to an eighth later where somebody takes the sums (`records`), and only there: three samples of 51x126x40 end 27 steps against 24 (32 -> 64
+// channels). Samples of a few columns stay in one line (the statistics pass of a smaller one is the same launch whatever it reads).
+struct BatchCut {
+  int parts;
+  ColumnCut cut;
+};
+inline BatchCut cut_batch(int64_t n, int64_t cols, int64_t steps, int64_t wgs, bool records) {
+  const BatchCut line{1, cut_columns(cols * n, steps, wgs)};
+  if (!records || line.cut.items < 0 || n == 1 || wgs / n < 8) return line;
+  const BatchCut apart{(int)n, cut_columns(cols, steps, wgs / n)};
+  return apart.cut.items > 0 && 8 * apart.cut.cost <= 9 * line.cut.cost && apart.cut.wgs >= 8 ? apart : line;
 }
 
 }  // namespace sfh

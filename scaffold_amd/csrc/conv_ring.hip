@@ -518,17 +518,8 @@ conv_ring_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ 
 #endif
 }
 
-// Takes a cut over; its cost, -1 where there are too many items.
-int64_t take_cut(RingGeom& gm, const ColumnCut& c) {
-  gm.segs = c.segs;
-  gm.seg_steps = c.seg_steps;
-  gm.items = c.items;
-  gm.items_per_wg = c.items_per_wg;
-  gm.wgs = c.wgs;
-  return c.items < 0 ? -1 : c.cost;
-}
-
-RingGeom ring_geom(const MfmaConvArgs& a) {
+// records: whether the launch leaves GroupNorm partials
+RingGeom ring_geom(const MfmaConvArgs& a, bool records) {
   RingGeom gm{};
   gm.tiles_h = (int)cdiv(a.oh, kTH);
   gm.tiles_w = (int)cdiv(a.ow, kTW);
@@ -536,23 +527,21 @@ RingGeom ring_geom(const MfmaConvArgs& a) {
   gm.nblocks = a.cout / 32;
   gm.parts = 1;
   const int64_t cols = (int64_t)gm.tiles_h * gm.tiles_w;
-  const int64_t per_block = kComputeUnits > gm.nblocks ? kComputeUnits / gm.nblocks : 1;
   if (cols * a.n <= 0 || gm.steps <= 0) return gm;
-  const int64_t cost = take_cut(gm, cut_columns(cols * a.n, gm.steps, per_block));
-  if (cost < 0 || a.n == 1 || per_block / a.n < 8) return gm;
-  // Several samples, each by workgroups of its own: a workgroup's sums are then those of one sample, and the normalisation
-  // behind the convolution needs no statistics pass. Where that ends no more than an eighth later, and a sample is more than
-  // a few columns (the statistics pass of a smaller one is the same launch whatever it reads).
-  RingGeom apart = gm;
-  apart.parts = a.n;
-  const int64_t cost_apart = take_cut(apart, cut_columns(cols, gm.steps, per_block / a.n));
-  return cost_apart > 0 && 8 * cost_apart <= 9 * cost && apart.wgs >= 8 ? apart : gm;
+  const BatchCut c = cut_batch(a.n, cols, gm.steps, kComputeUnits > gm.nblocks ? kComputeUnits / gm.nblocks : 1, records);
+  gm.parts = c.parts;
+  gm.segs = c.cut.segs;
+  gm.seg_steps = c.cut.seg_steps;
+  gm.items = c.cut.items;
+  gm.items_per_wg = c.cut.items_per_wg;
+  gm.wgs = c.cut.wgs;
+  return gm;
 }
 
 template <typename T>
 int launch_ring(const MfmaConvArgs& a, const void* x, const void* w, MfmaWeight form, const void* bias, void* y, hipStream_t st,
                 const GnPartialOut& gn, const ChannelPair& out2) {
-  const RingGeom gm = ring_geom(a);
+  const RingGeom gm = ring_geom(a, gn.part != nullptr);
   if (gm.items < 0) return fail(SFH_ERR_UNSUPPORTED, "conv mfma: too many columns");
   if (gm.items == 0) return SFH_OK;
   const unsigned grid = (unsigned)(gm.parts * gm.wgs * gm.nblocks);
@@ -584,7 +573,7 @@ bool mfma_conv_ring_applies(const MfmaConvArgs& a) {
 }
 
 int mfma_conv_ring_records(const MfmaConvArgs& a) {
-  const RingGeom gm = ring_geom(a);
+  const RingGeom gm = ring_geom(a, true);
   return gm.items > 0 && gm.parts == a.n ? gm.wgs : 0;
 }
 
