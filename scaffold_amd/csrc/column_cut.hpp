@@ -21,18 +21,29 @@ struct ColumnCut {
 // forward 32 -> 32 at 54x105x99 53.5 -> 37.7, 36x101x119 39.1 -> 28.8, 96x80x112 59.4 -> 44.5, two samples of 57x87x77 67.1 -> 47.7,
 // 32 -> 64 at 75x107x122 111 -> 92; weight gradient with its sum 32 -> 32 at 96x80x112 63.9 -> 54.3, 54x105x99 53.2 -> 47.0, two
 // samples of 57x87x77 72.5 -> 58.5, 64 -> 32 at 110x48x111 91.2 -> 69.9, 128 -> 64 at 60x35x45 76.4 -> 60.8.
-inline ColumnCut cut_columns(int64_t ncols, int64_t steps, int64_t wgs) {
-  auto parts = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+template <typename I>
+inline ColumnCut cut_columns_in(I ncols, I steps, I wgs) {
+  auto parts = [](I a, I b) { return (a + b - 1) / b; };
   ColumnCut best{};
   best.items = -1;
-  const int64_t most = parts(4 * wgs, ncols);  // more than four items to a workgroup even nothing out any more
-  for (int64_t want = 1; want <= most && want <= steps; ++want) {
-    const int64_t len = parts(steps, want), segs = parts(steps, len), items = ncols * segs;
-    if (items > 0x7fffffffLL) break;
-    const int64_t per_wg = parts(items, wgs), cost = per_wg * (len + 1);
-    if (best.items < 0 || cost < best.cost) best = ColumnCut{(int)segs, (int)len, (int)items, (int)per_wg, (int)parts(items, per_wg), cost};
+  const I most = parts(4 * wgs, ncols);  // more than four items to a workgroup even nothing out any more
+  // one count of segments for each length there is, the smallest: `segs` segments are `len` steps long and no fewer are
+  I len = 0;
+  for (I segs = 1; segs <= most && segs <= steps; segs = len > 1 ? parts(steps, len - 1) : steps + 1) {
+    len = parts(steps, segs);
+    const I items = ncols * segs;
+    if (items > 0x7fffffff) break;
+    const I per_wg = parts(items, wgs);
+    const int64_t cost = (int64_t)per_wg * (int64_t)(len + 1);
+    if (best.items < 0 || cost < best.cost) best = ColumnCut{(int)segs, (int)len, (int)items, (int)per_wg, 0, cost};
   }
+  if (best.items > 0) best.wgs = (int)parts((I)best.items, (I)best.items_per_wg);
   return best;
+}
+// (32-bit divisions wherever they do: launches and their queries ask for the cut on the host)
+inline ColumnCut cut_columns(int64_t ncols, int64_t steps, int64_t wgs) {
+  if (ncols < 1 << 20 && steps < 1 << 10 && wgs < 1 << 20) return cut_columns_in<uint32_t>((uint32_t)ncols, (uint32_t)steps, (uint32_t)wgs);
+  return cut_columns_in<int64_t>(ncols, steps, wgs);
 }
 
 // The cut of `n` samples of `cols` columns: one line of columns (parts 1), or every sample by workgroups of its own (parts n; the cut is that of

@@ -432,17 +432,22 @@ __global__ void __launch_bounds__(256) pack_tiles_kernel(TileBatch<N> b) {
 
 struct GatherPlan { int shape; int nsub; int ksplit; int64_t tiles; int64_t cost; };  // cost: the busiest CU's voxels x blocks, in hundredths
 
-// Brick shapes: the row-length class (32-, 16- or 8-voxel rows) times the tile size (512, 256 or 128 output voxels).
-constexpr int kTileDims[3][3][3] = {
-    {{4, 4, 32}, {2, 4, 32}, {1, 4, 32}},
-    {{4, 8, 16}, {2, 8, 16}, {1, 8, 16}},
-    {{8, 8, 8}, {4, 8, 8}, {2, 8, 8}},
+// Brick shapes: the row-length class (32-, 16- or 8-voxel rows) times the tile size (512, 256 or 128 output voxels), as powers of two: a
+// plan is asked for by every query and launch, and counting tiles by 64-bit divisions was most of what it cost the host.
+constexpr int kTileLog2[3][3][3] = {
+    {{2, 2, 5}, {1, 2, 5}, {0, 2, 5}},
+    {{2, 3, 4}, {1, 3, 4}, {0, 3, 4}},
+    {{3, 3, 3}, {2, 3, 3}, {1, 3, 3}},
 };
+constexpr int64_t tile_voxels(int size) { return 512 >> size; }
 
 int64_t tiles_of(const MfmaConvArgs& a, int cls, int size) {
-  const int* t = kTileDims[cls][size];
-  return (int64_t)a.n * cdiv(a.od, t[0]) * cdiv(a.oh, t[1]) * cdiv(a.ow, t[2]);
+  const int* t = kTileLog2[cls][size];
+  auto parts = [](int64_t extent, int log2) { return (extent + (1 << log2) - 1) >> log2; };
+  return a.n * parts(a.od, t[0]) * parts(a.oh, t[1]) * parts(a.ow, t[2]);
 }
+// workgroups of `nsub` blocks (1 or 2), before slices
+int64_t workgroups_of(const MfmaConvArgs& a, int64_t tiles, int nsub) { return tiles * (a.cout >> (4 + nsub)); }
 
 // What a launch of one brick shape takes, in hundredths of a us: {start of the launch, of a 32-channel chunk; 512 voxels of one block by rounds
 // of workgroups, by rounds counted with fractions; a round}. Fitted to 470 forward problems of 64 to 1024 channels on the levels of
@@ -452,14 +457,15 @@ constexpr int kBrickTime[3][2][2][5] = {  // [row class][size][blocks - 1]
     {{{358, 59, 330, 114, 225}, {157, 191, 334, 70, 437}}, {{289, 136, 366, 110, 163}, {136, 174, 365, 69, 266}}},
     {{{398, 76, 436, 82, 176}, {241, 109, 360, 75, 345}}, {{294, 120, 413, 90, 144}, {172, 141, 381, 76, 215}}},
 };
+int64_t brick_time(int shape, int nsub, int64_t wgs, int64_t chunks) {  // unsliced
+  const int* c = kBrickTime[shape / 3][shape % 3][nsub - 1];
+  const uint64_t rounds = (uint64_t)cdiv(wgs, kComputeUnits), blocks = (uint64_t)tile_voxels(shape % 3) * nsub;  // voxels x blocks
+  return c[0] + c[4] * (int64_t)rounds + chunks * (c[1] + (int64_t)(blocks * (c[2] * rounds * kComputeUnits + c[3] * (uint64_t)wgs) / (512 * kComputeUnits)));
+}
 int64_t brick_time(const MfmaConvArgs& a, const GatherPlan& p) {
-  const int* t = kTileDims[p.shape / 3][p.shape % 3];
-  const int* c = kBrickTime[p.shape / 3][p.shape % 3][p.nsub - 1];
-  const int64_t wgs = p.tiles * (a.cout / (32 * p.nsub)) * p.ksplit, chunks = cdiv(a.cred / kChunk, p.ksplit);
-  const int64_t rounds = cdiv(wgs, kComputeUnits), blocks = (int64_t)t[0] * t[1] * t[2] * p.nsub;  // voxels x blocks
-  int64_t time = c[0] + c[4] * rounds + chunks * (c[1] + blocks * (c[2] * rounds * kComputeUnits + c[3] * wgs) / (512 * kComputeUnits));
-  if (p.ksplit > 1) time += 500 + (int64_t)a.n * a.od * a.oh * a.ow * a.cout * p.ksplit * 4 * 40 / 1000000;
-  return time;
+  const int64_t wgs = workgroups_of(a, p.tiles, p.nsub), chunks = a.cred / kChunk;
+  if (p.ksplit == 1) return brick_time(p.shape, p.nsub, wgs, chunks);
+  return brick_time(p.shape, p.nsub, wgs * p.ksplit, cdiv(chunks, p.ksplit)) + 500 + (int64_t)a.n * a.od * a.oh * a.ow * a.cout * p.ksplit * 4 * 40 / 1000000;
 }
 
 // Launch geometry, a pure function of the problem. The row length picks the brick's row class; then, among 512- and
@@ -477,10 +483,9 @@ GatherPlan cut_plan(const MfmaConvArgs& a) {
   const int ncc = a.cred / kChunk;
   int64_t best = -1, best_wgs = 0;
   for (int size = 0; size < 2; ++size) {
-    const int* t = kTileDims[cls][size];
-    const int64_t tiles = tiles_of(a, cls, size), voxels = (int64_t)t[0] * t[1] * t[2];
+    const int64_t tiles = tiles_of(a, cls, size), voxels = tile_voxels(size);
     for (int nsub = 1; nsub <= (a.cout % 64 == 0 ? 2 : 1); ++nsub) {
-      const int64_t wgs = tiles * (a.cout / (32 * nsub));
+      const int64_t wgs = workgroups_of(a, tiles, nsub);
       const int64_t cost = cdiv(wgs, kComputeUnits) * voxels * nsub * (size == 1 ? 115 : 100) * (nsub == 2 ? 97 : 100);
       if (best < 0 || cost < best) {
         best = cost; best_wgs = wgs;
@@ -498,16 +503,17 @@ GatherPlan cut_plan(const MfmaConvArgs& a) {
   if (best_wgs >= kComputeUnits) {
     best *= 100;  // (the native costs count two factors of a hundred, these one)
     for (int c = cls + 1; c < 3; ++c)
-      for (int size = 0; size < 2; ++size)
+      for (int size = 0; size < 2; ++size) {
+        const int64_t tiles = tiles_of(a, c, size);
         for (int nsub = 1; nsub <= (a.cout % 64 == 0 ? 2 : 1); ++nsub) {
-          const int* t = kTileDims[c][size];
-          const int64_t tiles = tiles_of(a, c, size), wgs = tiles * (a.cout / (32 * nsub));
-          const int64_t cost = cdiv(wgs, kComputeUnits) * (t[0] * t[1] * t[2]) * nsub * kStubby[c - 1][size][nsub - 1] * 10000;
+          const int64_t wgs = workgroups_of(a, tiles, nsub);
+          const int64_t cost = cdiv(wgs, kComputeUnits) * tile_voxels(size) * nsub * kStubby[c - 1][size][nsub - 1] * 10000;
           if (cost < best && wgs > kComputeUnits / 2) {
             best = cost; best_wgs = wgs;
             p.shape = c * 3 + size; p.tiles = tiles; p.nsub = nsub;
           }
         }
+      }
     return GatherPlan{p.shape, p.nsub, 1, p.tiles, best / 10000};
   }
   p.ksplit = 1;
@@ -525,16 +531,19 @@ GatherPlan cut_plan(const MfmaConvArgs& a) {
 GatherPlan gather_plan(const MfmaConvArgs& a) {
   GatherPlan p = cut_plan(a);
   if (p.ksplit > 1 || p.tiles == 0) return p;
+  const int64_t chunks = a.cred / kChunk;
+  const int nsubs = a.cout % 64 == 0 ? 2 : 1;
   int64_t best = brick_time(a, p) * 95 / 100;
   for (int cls = a.ow > 16 ? 0 : (a.ow > 8 ? 1 : 2); cls < 3; ++cls)
-    for (int size = 0; size < 2; ++size)
-      for (int nsub = 1; nsub <= (a.cout % 64 == 0 ? 2 : 1); ++nsub) {
-        const GatherPlan q{cls * 3 + size, nsub, 1, tiles_of(a, cls, size), p.cost};
-        const int64_t time = brick_time(a, q);
+    for (int size = 0; size < 2; ++size) {
+      const int64_t tiles = tiles_of(a, cls, size);
+      for (int nsub = 1; nsub <= nsubs; ++nsub) {
+        const int64_t time = brick_time(cls * 3 + size, nsub, workgroups_of(a, tiles, nsub), chunks);
         if (time >= best) continue;
         best = time;
-        p = q;
+        p.shape = cls * 3 + size; p.nsub = nsub; p.tiles = tiles;
       }
+    }
   return p;
 }
 
@@ -746,9 +755,9 @@ int mfma_pack_weight_batch(const MfmaPackItem* items, int n, int dtype, hipStrea
 static bool served_by_split(const MfmaConvArgs& a) { return !mfma_conv_wide_fits(a) && mfma_conv_split_applies(a); }
 
 size_t mfma_conv_partial_bytes(const MfmaConvArgs& a) {
-  if (mfma_conv_wide_applies(a) || served_by_split(a)) return 0;
-  const GatherPlan p = gather_plan(a);
-  if (a.cred == kChunk || p.ksplit == 1) return 0;
+  if (a.cred == kChunk || mfma_conv_wide_applies(a) || served_by_split(a)) return 0;
+  const GatherPlan p = cut_plan(a);
+  if (p.ksplit == 1) return 0;
   return align_up((size_t)p.ksplit * a.n * a.od * a.oh * a.ow * a.cout * sizeof(float), 256);
 }
 
@@ -760,8 +769,7 @@ MfmaConvGeometry mfma_conv_gather_geometry(const MfmaConvArgs& a) {
   if (mfma_conv_wide_applies(a)) return mfma_conv_wide_geometry(a);
   if (served_by_split(a)) return mfma_conv_split_geometry(a);
   const GatherPlan p = gather_plan(a);
-  const int* t = kTileDims[p.shape / 3][p.shape % 3];
-  return MfmaConvGeometry{kKernelBrick, t[0] * t[1] * t[2], p.nsub, p.ksplit};
+  return MfmaConvGeometry{kKernelBrick, (int)tile_voxels(p.shape % 3), p.nsub, p.ksplit};
 }
 
 int mfma_conv_gather_gn_records(const MfmaConvArgs& a, int groups) {

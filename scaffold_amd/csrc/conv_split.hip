@@ -273,8 +273,9 @@ typedef Shape<4, 4, 4, 192> Cube;    // 216
 typedef Shape<2, 2, 16, 288> Rows;   // 288
 
 int64_t tiles_of(const MfmaConvArgs& a, int shape) {
-  static const int t[3][3] = {{2, 4, 8}, {4, 4, 4}, {2, 2, 16}};
-  return (int64_t)a.n * cdiv(a.od, t[shape][0]) * cdiv(a.oh, t[shape][1]) * cdiv(a.ow, t[shape][2]);
+  static const int log2[3][3] = {{1, 2, 3}, {2, 2, 2}, {1, 1, 4}};
+  auto parts = [](int64_t extent, int log2) { return (extent + (1 << log2) - 1) >> log2; };
+  return a.n * parts(a.od, log2[shape][0]) * parts(a.oh, log2[shape][1]) * parts(a.ow, log2[shape][2]);
 }
 
 // What a launch of `pairs` pairs of channel blocks takes, in hundredths of a us, fitted as the brick kernel's (conv_mfma.hip, brick_time) to 453

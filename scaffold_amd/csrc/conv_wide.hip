@@ -381,7 +381,6 @@ conv_wide_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ 
 
 struct WidePlan {
   bool use;
-  bool fits;   // the problem is this kernel's, also where the brick kernel takes its place
   int shape;   // 0: 4x4x32 tile with 4 channel blocks, 1: 8x4x32 with 2, 2: 8x4x32 with 1, 3: 4x4x32 with 2, 4: 4x4x32 with 1
 };
 
@@ -393,28 +392,37 @@ int64_t wide_workgroups(const MfmaConvArgs& a, int shape) {
   return wide_tiles(a, td[shape]) * (a.cout / (32 * nsub[shape]));
 }
 
-// Launch geometry, a pure function of the problem. Rows of more than 16 voxels only (32-voxel sub-tiles are one row).
-WidePlan wide_plan(const MfmaConvArgs& a) {
-  WidePlan p{false, false, 0};
-  if (a.kd != 3 || a.kh != 3 || a.kw != 3 || a.cred < 64 || a.cred % 32 != 0 || a.cout % 32 != 0 || a.ow <= 16) return p;
+// The depth that launch rules count: that of a shard's planes in both forms of its gradients, the slab's (D + 2 planes from D) and the padded
+// volume's. Where the slab's own decided, the padded volume's gradient could be the small-volume kernel's, which adds in another order (of
+// 64 -> 128 channels at 27x61x33: 256 workgroups of 4x4x32 for the slab, 224 for the volume). An odd number of chunks never goes there: this
+// kernel and the bricks add alike.
+MfmaConvArgs wide_core(const MfmaConvArgs& a) {
+  MfmaConvArgs core = a;
+  if (a.cred % 64 == 0 && a.id < a.od) core.od = a.id;
+  return core;
+}
+
+// The accumulator grid for a problem (of this depth), -1: it is not this kernel's. Where it is, the brick kernel may still take its place
+// (wide_plan). Rows of more than 16 voxels only (32-voxel sub-tiles are one row).
+int wide_shape(const MfmaConvArgs& core) {
+  const MfmaConvArgs& a = core;
+  if (a.kd != 3 || a.kh != 3 || a.kw != 3 || a.cred < 64 || a.cred % 32 != 0 || a.cout % 32 != 0 || a.ow <= 16) return -1;
   // a brick (at most 10 input planes and 6 rows) must span less than kRange bytes of the input
-  if (((int64_t)10 * a.ih + 6) * a.iw * a.cred * 2 + 64 >= kRange) return p;
-  int shape = -1;
+  if (((int64_t)10 * a.ih + 6) * a.iw * a.cred * 2 + 64 >= kRange) return -1;
   // Measured against the brick-per-workgroup kernel on every shape of the U-Net and of the cube configurations, this
   // kernel wins where a 64-channel output meets 128 or more reduction channels (one workgroup then produces all of a
   // voxel's channels from one staged brick): 8 x 2 accumulator blocks per wavefront when such workgroups fill the
-  // chip, else 4 x 2. Everything else stays with the other kernels. The depth counted is that of a shard's planes in both forms of
-  // its gradients, here and below: where the slab's own decided, the padded volume's gradient could be the small-volume kernel's,
-  // which adds in another order (of 64 -> 128 channels at 27x61x33: 256 workgroups of 4x4x32 for the slab, 224 for the volume). An odd
-  // number of chunks never goes there: this kernel and the bricks add alike.
-  MfmaConvArgs core = a;
-  if (a.cred % 64 == 0 && a.id < a.od) core.od = a.id;
-  if (a.cout == 64 && a.cred >= 128) {
-    if (wide_workgroups(core, 1) >= kComputeUnits) shape = 1;
-    else if (wide_workgroups(core, 3) >= kComputeUnits) shape = 3;
-  }
+  // chip, else 4 x 2. Everything else stays with the other kernels.
+  if (a.cout != 64 || a.cred < 128) return -1;
+  return wide_workgroups(a, 1) >= kComputeUnits ? 1 : wide_workgroups(a, 3) >= kComputeUnits ? 3 : -1;
+}
+
+// Launch geometry, a pure function of the problem.
+WidePlan wide_plan(const MfmaConvArgs& a) {
+  WidePlan p{false, 0};
+  const MfmaConvArgs core = wide_core(a);
+  const int shape = wide_shape(core);
   if (shape < 0) return p;
-  p.fits = true;
   // Past two rounds of workgroups the brick kernel takes its place where 8 x 4 x 32 leaves more over than that kernel's choice of
   // brick, by the busiest CU's share (at equal shares it is the faster one by some 3 % for 128 channels, the slower by 5 for 256).
   // us, here -> there: 128 -> 64 at 96x80x112 353 -> 315, at 100^3 485 -> 387, at 90^3 331 -> 309, at 128^3 761 -> 739; 256 -> 64 at
@@ -487,8 +495,8 @@ int mfma_conv_wide_gn_records(const MfmaConvArgs& a, int groups) {
 }
 
 // The staging offsets of a lane are those of one tensor: a pair must be two tensors of the same channel count.
-bool mfma_conv_wide_fits(const MfmaConvArgs& a) { return wide_plan(a).fits; }
-bool mfma_conv_wide_pair_ok(const MfmaConvArgs& a, int first) { return wide_plan(a).fits && first * 2 == a.cred && first % 16 == 0; }
+bool mfma_conv_wide_fits(const MfmaConvArgs& a) { return wide_shape(wide_core(a)) >= 0; }
+bool mfma_conv_wide_pair_ok(const MfmaConvArgs& a, int first) { return mfma_conv_wide_fits(a) && first * 2 == a.cred && first % 16 == 0; }
 
 int mfma_conv_wide(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                    const GnPartialOut* gn, const ChannelPair* in2) {

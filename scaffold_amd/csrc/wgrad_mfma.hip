@@ -638,25 +638,28 @@ bool ring_serves(const WgradArgs& a) { return mfma_wgrad_ring_applies(a); }
 // Columns sum the longer chains, so that estimate alone does not decide: of 40 problems that only it gives to columns their error is 1.17 times that of
 // tiles (geometric mean; 128 -> 128 at 43x29x34 1.9 -> 3.1e-7, 64 -> 32 at 54x40x76 1.5 -> 1.9) for 0.92 of the time. They are walked where an estimate from padded operations
 // (20 us, 25 where rows are cut, and 0.7 a GFLOP against 12.5 and 1.25, fitted to 35 problems) finds them quicker as well, or quicker than the tile plan's cost.
-bool walks_columns(const WgradArgs& a, int64_t tile_plan_cost) {
+bool walks_columns(const WgradArgs& a, int64_t columns_cost, int64_t tile_plan_cost) {
   const double per_voxel = 54e-9 * a.cin * a.cout * a.n;
   const double columns = (a.ow % 32 == 0 ? 20. : 25.) + 0.7 * per_voxel * (double)cdiv(a.od, 2) * 2 * (double)cdiv(a.oh, 4) * 4 * (double)cdiv(a.ow, 32) * 32;
   const double tiles = 12.5 + 1.25 * per_voxel * (double)cdiv(a.od, 4) * 4 * (double)cdiv(a.oh, 8) * 8 * (double)cdiv(a.ow, 8) * 8;
-  return (columns <= tiles || 100 * columns <= (double)tile_plan_cost) && 2000 + 210 * mfma_wgrad_ring_cost(a) <= tile_plan_cost;
+  return (columns <= tiles || 100 * columns <= (double)tile_plan_cost) && 2000 + 210 * columns_cost <= tile_plan_cost;
 }
 
 Plan make_plan(const WgradArgs& a) {
   Plan p{};
+  const bool wide_rows = ring_serves(a);
+  int64_t columns_cost = 0;
+  const int columns_splits = wide_rows ? mfma_wgrad_ring_splits(a, columns_cost) : 0;
   auto columns = [&] {
     p.ring = true;
     p.planes = false;
     p.tw = 32;
-    p.splits = mfma_wgrad_ring_splits(a);
+    p.splits = columns_splits;
     return p;
   };
-  if (ring_serves(a) && 3 * (int64_t)(a.cin / 32) * (a.cout / 32) > kTargetWorkgroups) return columns();
+  if (wide_rows && 3 * (int64_t)(a.cin / 32) * (a.cout / 32) > kTargetWorkgroups) return columns();
   int td, th;
-  if (a.ow > 16 && !ring_serves(a)) { p.tw = 32; td = 2; th = 4; }
+  if (a.ow > 16 && !wide_rows) { p.tw = 32; td = 2; th = 4; }
   else if (a.ow > 8 && a.ow <= 16) { p.tw = 16; td = 2; th = 8; }
   else { p.tw = 8; td = 4; th = 8; }
   p.tiles_d = (int)cdiv(a.od, td);
@@ -675,14 +678,14 @@ Plan make_plan(const WgradArgs& a) {
   // bits, one workgroup to a block and a sum pass / three, stored in place where one slice is left): 256 -> 256 channels on
   // 8 x 16 x 16 32.9 / 19.6, on 8 x 8 x 8 18.3 / 9.0, 128 -> 128 on 16 x 16 x 16 21.8 / 17.7 (four slices).
   int64_t best = -1;
-  for (int units = ring_serves(a) ? 3 : 1; units <= 3; units += 2) {  // (tiles in the place of columns: in planes, walks_columns)
+  for (int units = wide_rows ? 3 : 1; units <= 3; units += 2) {  // (tiles in the place of columns: in planes, walks_columns)
     if (units == 3 && (p.tw == 32 || units * p.nblk > kTargetWorkgroups)) break;
     const int64_t tile = units == 3 ? 130 : 240;
     int want = kTargetWorkgroups / (p.nblk * units);
     if (want < 1) want = 1;
     if (want > p.ntiles) want = p.ntiles;
     for (int s = want; s >= 1; s /= 2) {
-      const int tps = (int)cdiv(p.ntiles, s), eff = (int)cdiv(p.ntiles, tps);
+      const int tps = (p.ntiles - 1) / s + 1, eff = (p.ntiles - 1) / tps + 1;
       const int64_t cost = eff > 1 ? tile * tps + 1000 + 64LL * eff * p.nblk / 10 : tile * tps + 600 + 32LL * p.nblk / 10;
       if (best < 0 || cost < best) {
         best = cost;
@@ -692,7 +695,7 @@ Plan make_plan(const WgradArgs& a) {
       }
     }
   }
-  if (ring_serves(a) && walks_columns(a, best)) return columns();
+  if (wide_rows && walks_columns(a, columns_cost, best)) return columns();
   return p;
 }
 

@@ -25,8 +25,7 @@ int mfma_wgrad(const WgradArgs& a, int dtype, const void* x, const void* gy, voi
 // they lie in memory and transposed by the LDS reads. `applies` and the slice count are pure functions of the shape;
 // the kernel writes `splits` fp32 slices [Cout][27][Cin] into ws. mfma_wgrad routes to it.
 bool mfma_wgrad_ring_applies(const WgradArgs& a);
-int mfma_wgrad_ring_splits(const WgradArgs& a);
-int64_t mfma_wgrad_ring_cost(const WgradArgs& a);  // steps and items of its busiest workgroup
+int mfma_wgrad_ring_splits(const WgradArgs& a, int64_t& cost);  // cost: steps and items of its busiest workgroup
 int mfma_wgrad_ring(const WgradArgs& a, int dtype, const void* x, const void* gy, float* ws, hipStream_t st, const ChannelPair& x2);
 
 // Several weight gradients from as few launches as possible: the ring-served problems of a list (rows of more than 16

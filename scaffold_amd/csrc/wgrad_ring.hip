@@ -851,11 +851,14 @@ bool mfma_wgrad_ring_applies(const WgradArgs& a) {
   if (a.ow <= 16 || a.od < 1 || a.oh < 1 || a.n < 1) return false;
   if (((int64_t)(a.ih + kBH) * a.iw + kBW) * a.cin * 2 + 64 >= kRange || ((int64_t)(a.oh + kTH) * a.ow + kTW) * a.cout * 2 + 64 >= kRange)
     return false;
-  return wring_geom(a).items > 0;
+  return a.n * cdiv(a.oh, kTH) * cdiv(a.ow, kTW) <= 0x7fffffffLL;  // columns: positions are 32 bits wide
 }
 
-int mfma_wgrad_ring_splits(const WgradArgs& a) { return wring_geom(a).splits; }
-int64_t mfma_wgrad_ring_cost(const WgradArgs& a) { return wring_geom(a).cost; }
+int mfma_wgrad_ring_splits(const WgradArgs& a, int64_t& cost) {
+  const WRingGeom gm = wring_geom(a);
+  cost = gm.cost;
+  return gm.splits;
+}
 
 int mfma_wgrad_ring(const WgradArgs& a, int dtype, const void* x, const void* gy, float* ws, hipStream_t st, const ChannelPair& x2) {
   const WRingGeom gm = wring_geom(a);

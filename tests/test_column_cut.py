@@ -52,7 +52,8 @@ def _reference(cols, steps, wgs):
 def _problems():
     rng = random.Random(5)
     log = lambda hi: round(hi ** rng.random())
-    return [(rng.choice((1, 2, 3, 5, 6, 7, 8)), log(4000), log(200), rng.choice((256, 128, 64, 32, 4, 1))) for _ in range(1500)]
+    drawn = [(rng.choice((1, 2, 3, 5, 6, 7, 8)), log(4000), log(200), rng.choice((256, 128, 85, 64, 32, 4, 1))) for _ in range(1500)]
+    return drawn + [(2, 900_000, 40, 256), (1, 50, 5000, 256), (1, 1, 1 << 20, 256), (1, 1, 1023, 256), (3, 1 << 20, 1, 7)]  # past 32-bit arithmetic, and the last within it
 
 
 def test_batch_without_records_ends_soonest(cut):
