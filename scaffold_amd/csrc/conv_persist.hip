@@ -470,7 +470,6 @@ PersistGeom persist_geom(const MfmaConvArgs& a, int td, int th, int tw) {
   return gm;
 }
 PersistGeom persist_geom(const MfmaConvArgs& a) {
-  if (a.ow > 16) return persist_geom(a, 4, 4, 32);
   if (a.ow > 8) return persist_geom(a, 4, 8, 16);
   return persist_geom(a, 8, 8, 8);
 }
@@ -503,7 +502,8 @@ int launch_tile(const MfmaConvArgs& a, const void* x, const void* w, MfmaWeight 
 template <typename T>
 int launch_typed(const MfmaConvArgs& a, const void* x, const void* w, MfmaWeight form, const void* bias, void* y, hipStream_t st,
                  const GnPartialOut& gn, const ChannelPair& out2) {
-  if (a.ow > 16) return launch_tile<T, PTile<4, 4, 32>>(a, x, w, form, bias, y, st, gn, out2);
+  // (what mfma_conv_persist_applies admits of such rows is within the ring's bounds too: 9 ih iw and 7 oh ow are more than its 34 and 32)
+  if (a.ow > 16) return fail(SFH_ERR_UNSUPPORTED, "conv persist: rows of more than 16 voxels are the column-walking kernel's");
   if (a.ow > 8) return launch_tile<T, PTile<4, 8, 16>>(a, x, w, form, bias, y, st, gn, out2);
   return launch_tile<T, PTile<8, 8, 8>>(a, x, w, form, bias, y, st, gn, out2);
 }
