@@ -1,9 +1,12 @@
 """The normalisation that pools its result in the same pass, against the two launches: the same bits, values and gradients."""
 
+import ctypes
+
 import pytest
 import torch
 
 import scaffold_amd as sa
+from scaffold_amd import _lib
 from scaffold_amd.modules import FastConv3d, FastGroupNorm, conv_then_norm
 from scaffold_amd.pooling import FastMaxPool3d
 from scaffold_amd.unet import UNet
@@ -49,8 +52,9 @@ def test_same_bits_as_two_launches(device, n, c, spatial, dtype, halo, relu):
         y = conv_then_norm(conv, norm, x)
         # (a halo asks for one sample, and records come only from the kernels that offer them)
         assert hasattr(y, "_sfh_pooled") == (fused and not (halo and n > 1) and bool(y is not None and _records(conv, x0)))
-        pooled, skip = pool.with_skip(y)
-        assert not hasattr(y, "_sfh_pooled")
+        given = y.__dict__.pop("_sfh_pooled", None)
+        pooled, skip = pool.with_skip(y, given)
+        assert given is None or pooled.data_ptr() == given[0].data_ptr()
         slabs = [t._sfh_slab[0].clone() for t in (pooled, skip) if halo and n == 1]
         grads = torch.autograd.grad((pooled, skip), (x, conv.weight, norm.weight, norm.bias), (gp, gs))
         with torch.no_grad():
@@ -73,7 +77,9 @@ def test_what_is_not_reused(device):
     with torch.no_grad():
         want = torch.nn.functional.max_pool3d(conv_then_norm(conv, norm, x).float(), 2)
         y = conv_then_norm(conv, norm, x)
-        assert torch.equal(wide(y).float(), want) and hasattr(wide(y), "_sfh_slab")  # another halo
+        given = y._sfh_pooled
+        pooled = wide.with_skip(y, given)[0]                                         # another halo
+        assert pooled.data_ptr() != given[0].data_ptr() and torch.equal(pooled.float(), want) and hasattr(pooled, "_sfh_slab")
         y = conv_then_norm(conv, norm, x)
         a, b = pool(y), pool(y)                                                      # a second pooling has its own tensor
         assert a.data_ptr() != b.data_ptr() and torch.equal(a.float(), want) and torch.equal(b.float(), want)
@@ -103,7 +109,9 @@ def test_nan_and_infinity(device):
         norm.pool_next = pool_next
         with torch.no_grad():
             y = conv_then_norm(conv, norm, x)
-            outs.append((y.clone(), FastMaxPool3d(2)(y)))
+            given = y.__dict__.pop("_sfh_pooled", None)
+            assert (given is None) == (pool_next is None)
+            outs.append((y.clone(), FastMaxPool3d(2).with_skip(y, given)[0]))
     for a, b in zip(*outs):
         assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num())
 
@@ -199,6 +207,45 @@ def test_gradients_meet_in_the_normalisation(device, n, c, spatial, dtype, relu)
             outs, grads = zip(*[p for k, p in zip(("pooled", "skip"), zip(pool.with_skip(y, given if take else None), (gp, gs))) if used in ("both", k)])
             results.append(torch.autograd.grad(outs, (x, conv.weight, norm.weight, norm.bias), grads))
         assert all(torch.equal(a, b) for a, b in zip(*results)), used
+
+
+@pytest.mark.parametrize("relu", [0, 1])
+@pytest.mark.parametrize("n,c,spatial,dtype", [
+    (2, 32, (1700, 5, 6), torch.bfloat16),    # a thread's next row is 64 voxels on: two planes, a row with a carry, and four voxels
+    (2, 64, (1300, 3, 7), torch.float16),     # 32 on: a plane, a row and four voxels, a carry into either
+    (2, 64, (33, 5, 6), torch.bfloat16),      # one pass
+    (1, 32, (3400, 2, 17), torch.bfloat16),   # seven: the last one is not half of a pair
+    (1, 64, (129, 128, 67), torch.bfloat16),  # 141.6 MB: operands read past the caches
+    (2, 32, (65, 129, 130), torch.float16),   # 139.5 MB, two samples of odd planes
+])
+def test_pooled_gradient_in_both_passes(device, n, c, spatial, dtype, relu):
+    """The two passes that take the pooling's gradient in, against the launch that sums and the two passes behind it: the same bits."""
+    lib, code, groups = _lib.lib(), _lib.dtype_code(dtype), 8
+    def volume(*extents):
+        return torch.randn((n, *extents, c), device=device).to(dtype)
+    torch.manual_seed(3)
+    half = [v // 2 for v in spatial]
+    x, gy, gp = volume(*spatial), volume(*spatial), volume(*half)
+    gamma, beta, mean = (torch.randn(k, device=device) for k in (c, c, n * groups))
+    rstd = torch.rand(n * groups, device=device) + 0.5
+    pooled, idx = volume(*half), torch.empty((n, *half, c), dtype=torch.uint8, device=device)
+    total = torch.empty_like(x)
+    pd = _lib.PoolDesc(n, c, *spatial)
+    gd = _lib.GroupNormDesc(n, c, groups, relu, spatial[0] * spatial[1] * spatial[2], 1e-5)
+    stream = torch.cuda.current_stream().cuda_stream
+    size = lib.sfh_groupnorm_bwd_workspace_bytes(ctypes.byref(gd), code)
+    def run(call):
+        out = torch.full_like(x, float("nan")), torch.empty(c, device=device), torch.empty(c, device=device)
+        ws = torch.empty(size, dtype=torch.uint8, device=device)
+        _lib.check(call(*(t.data_ptr() for t in out), ws.data_ptr(), size, stream), "groupnorm backward")
+        return out
+    _lib.check(lib.sfh_maxpool2_fwd(ctypes.byref(pd), code, volume(*spatial).data_ptr(), pooled.data_ptr(), idx.data_ptr(), stream), "pool")
+    _lib.check(lib.sfh_maxpool2_bwd_add(ctypes.byref(pd), code, gp.data_ptr(), idx.data_ptr(), gy.data_ptr(), total.data_ptr(), stream), "pool")
+    rest = [t.data_ptr() for t in (x, gamma, beta, mean, rstd)]
+    extents, fp32 = (ctypes.c_int32 * 3)(*spatial), _lib.dtype_code(torch.float32)
+    got = run(lambda *out: lib.sfh_groupnorm_bwd_pool(ctypes.byref(gd), extents, code, fp32, gy.data_ptr(), gp.data_ptr(), idx.data_ptr(), *rest, *out))
+    want = run(lambda *out: lib.sfh_groupnorm_bwd(ctypes.byref(gd), code, code, fp32, total.data_ptr(), *rest, *out))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
 def test_a_captured_pooling_reads_its_input(device):
