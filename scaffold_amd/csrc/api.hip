@@ -361,7 +361,7 @@ extern "C" size_t sfh_conv3d_fwd_workspace_bytes(const sfh_conv3d_desc* p, int d
   if (fwd_uses_patch(*p, dtype, out)) return mfma_conv_packed_weight_bytes(patch_pack_args(p->cout, p->cin));
   if (fwd_uses_f32_tiles(*p, dtype, out)) return f32_conv_packed_weight_bytes(fwd_mfma_args(*p, out));
   if (!fwd_uses_mfma(*p, dtype, out)) return 0;
-  return mfma_conv_packed_weight_bytes(fwd_mfma_args(*p, out)) + mfma_conv_partial_bytes(fwd_mfma_args(*p, out));
+  return mfma_conv_packed_weight_bytes(fwd_mfma_args(*p, out)) + mfma_conv_partial_bytes(fwd_mfma_args(*p, out), true);
 }
 
 static int conv3d_fwd_any(const sfh_conv3d_desc* p, int dtype, const void* x, const void* w, const int64_t w_stride[5],
@@ -375,7 +375,7 @@ static int conv3d_fwd_any(const sfh_conv3d_desc* p, int dtype, const void* x, co
   hipStream_t st = (hipStream_t)stream;
   if (!(flags & SFH_FLAG_FORCE_GENERIC) && fwd_uses_mfma(*p, dtype, out)) {
     const MfmaConvArgs a = fwd_mfma_args(*p, out);
-    const size_t packed_bytes = mfma_conv_packed_weight_bytes(a), partial_bytes = mfma_conv_partial_bytes(a);
+    const size_t packed_bytes = mfma_conv_packed_weight_bytes(a), partial_bytes = mfma_conv_partial_bytes(a, true);
     if (flags & SFH_FLAG_WEIGHT_PACKED) {  // w is the packed weight; the workspace only holds the partial slices
       if (partial_bytes && (workspace == nullptr || workspace_bytes < partial_bytes))
         return fail(SFH_ERR_WORKSPACE, "conv3d fwd: workspace of %zu bytes needed, got %zu", partial_bytes, workspace_bytes);
@@ -558,7 +558,7 @@ extern "C" size_t sfh_conv3d_dgrad_workspace_bytes(const sfh_conv3d_desc* p, int
   if (check_dgrad(*p) != SFH_OK) return 0;
   if (dgrad_uses_f32_tiles(*p, dtype, out)) return f32_conv_packed_weight_bytes(dgrad_mfma_args(*p, out));
   if (!dgrad_uses_mfma(*p, dtype, out)) return 0;
-  return mfma_conv_packed_weight_bytes(dgrad_mfma_args(*p, out)) + mfma_conv_partial_bytes(dgrad_mfma_args(*p, out));
+  return mfma_conv_packed_weight_bytes(dgrad_mfma_args(*p, out)) + mfma_conv_partial_bytes(dgrad_mfma_args(*p, out), false);
 }
 
 static int conv3d_dgrad_any(const sfh_conv3d_desc* p, int dtype, const void* gy, const void* w, const int64_t w_stride[5],
@@ -571,7 +571,7 @@ static int conv3d_dgrad_any(const sfh_conv3d_desc* p, int dtype, const void* gy,
   hipStream_t st = (hipStream_t)stream;
   if (!(flags & SFH_FLAG_FORCE_GENERIC) && dgrad_uses_mfma(*p, dtype, out)) {
     const MfmaConvArgs a = dgrad_mfma_args(*p, out);
-    const size_t packed_bytes = mfma_conv_packed_weight_bytes(a), partial_bytes = mfma_conv_partial_bytes(a);
+    const size_t packed_bytes = mfma_conv_packed_weight_bytes(a), partial_bytes = mfma_conv_partial_bytes(a, false);
     if (flags & SFH_FLAG_WEIGHT_PACKED) {
       if (partial_bytes && (workspace == nullptr || workspace_bytes < partial_bytes))
         return fail(SFH_ERR_WORKSPACE, "conv3d dgrad: workspace of %zu bytes needed, got %zu", partial_bytes, workspace_bytes);

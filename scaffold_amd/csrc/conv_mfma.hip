@@ -752,10 +752,11 @@ int mfma_pack_weight_batch(const MfmaPackItem* items, int n, int dtype, hipStrea
 // Where the wide kernel steps aside it does so for the brick kernel, whose share it reckoned: not for the small-volume one, which
 // otherwise goes in front of the bricks (us, small-volume / brick / wide: 128 -> 64 on 32 samples of 32^3 455 / 377 / 371, on 8 of
 // 128x32x32 449 / 367 / 370, on 10 of 64x28x28 234 / 218 / 241; 256 -> 64 on 16 of 48x28x20 404 / 387 / 450).
-static bool served_by_split(const MfmaConvArgs& a) { return !mfma_conv_wide_fits(a) && mfma_conv_split_applies(a); }
+// records: of a launch that leaves GroupNorm records (some of those stay with the bricks' slices, whose bits the small-volume kernel has there).
+static bool served_by_split(const MfmaConvArgs& a, bool records) { return !mfma_conv_wide_fits(a) && mfma_conv_split_applies(a, records); }
 
-size_t mfma_conv_partial_bytes(const MfmaConvArgs& a) {
-  if (a.cred == kChunk || mfma_conv_wide_applies(a) || served_by_split(a)) return 0;
+size_t mfma_conv_partial_bytes(const MfmaConvArgs& a, bool records) {
+  if (a.cred == kChunk || mfma_conv_wide_applies(a) || served_by_split(a, records)) return 0;
   const GatherPlan p = cut_plan(a);
   if (p.ksplit == 1) return 0;
   return align_up((size_t)p.ksplit * a.n * a.od * a.oh * a.ow * a.cout * sizeof(float), 256);
@@ -767,14 +768,14 @@ int64_t mfma_conv_brick_time(const MfmaConvArgs& a) { return brick_time(a, gathe
 
 MfmaConvGeometry mfma_conv_gather_geometry(const MfmaConvArgs& a) {
   if (mfma_conv_wide_applies(a)) return mfma_conv_wide_geometry(a);
-  if (served_by_split(a)) return mfma_conv_split_geometry(a);
+  if (served_by_split(a, false)) return mfma_conv_split_geometry(a);
   const GatherPlan p = gather_plan(a);
   return MfmaConvGeometry{kKernelBrick, (int)tile_voxels(p.shape % 3), p.nsub, p.ksplit};
 }
 
 int mfma_conv_gather_gn_records(const MfmaConvArgs& a, int groups) {
   if (mfma_conv_wide_applies(a)) return mfma_conv_wide_gn_records(a, groups);
-  if (served_by_split(a)) return mfma_conv_split_gn_records(a, groups);
+  if (served_by_split(a, true)) return mfma_conv_split_gn_records(a, groups);
   return gather_gn_records(a, gather_plan(a), groups);
 }
 
@@ -784,14 +785,14 @@ int mfma_conv_gather(const MfmaConvArgs& a, int dtype, const void* x, const void
     if (out2 != nullptr) return fail(SFH_ERR_UNSUPPORTED, "conv wide: the output cannot be a pair of tensors");
     return mfma_conv_wide(a, dtype, x, packed, bias, y, st, gn, in2);
   }
-  if (served_by_split(a)) return mfma_conv_split(a, dtype, x, packed, bias, y, st, gn, in2, out2);
+  if (served_by_split(a, gn != nullptr && gn->part != nullptr)) return mfma_conv_split(a, dtype, x, packed, bias, y, st, gn, in2, out2);
   if (dtype == SFH_BF16) return launch_typed<bf16_t>(a, dtype, x, packed, bias, y, partial, st, gn, in2, out2);
   return launch_typed<fp16_t>(a, dtype, x, packed, bias, y, partial, st, gn, in2, out2);
 }
 
 bool mfma_conv_gather_pair_ok(const MfmaConvArgs& a, int first, bool as_output) {
   if (mfma_conv_wide_fits(a)) return !as_output && mfma_conv_wide_pair_ok(a, first);
-  if (served_by_split(a)) return mfma_conv_split_pair_ok(a, first, as_output);
+  if (served_by_split(a, false)) return mfma_conv_split_pair_ok(a, first, as_output);
   return gather_pair_ok(a, first, as_output);
 }
 

@@ -38,7 +38,7 @@ struct MfmaPackItem {
 constexpr int kPackTable = 72;  // dense weights, both forms each, that one launch takes (the table stays under 4 KB of kernel arguments)
 int mfma_pack_weight_batch(const MfmaPackItem* items, int n, int dtype, hipStream_t st);
 // Bytes of fp32 slices the kernel needs when it cuts the reduction channels to fill the chip (0 when it does not).
-size_t mfma_conv_partial_bytes(const MfmaConvArgs& a);
+size_t mfma_conv_partial_bytes(const MfmaConvArgs& a, bool records);  // records: room for a launch that leaves GroupNorm records as well
 // `gn` (optional): also leave GroupNorm partials of the rounded output (gn_stats.hpp), gn->records per sample as
 // mfma_conv_gn_records says for gn->groups groups.
 // `in2` / `out2` (optional, where mfma_conv_pair_ok says so): x / y given as a ChannelPair.
@@ -54,7 +54,7 @@ int mfma_conv_wide(const MfmaConvArgs& a, int dtype, const void* x, const void* 
 // Same contract, the kernel for the small volumes of the deep levels: 64-voxel bricks, the reduction cut over the four
 // wavefronts of a workgroup and summed in LDS (conv_split.hip). `applies` is a pure function of the shape; mfma_conv_gather
 // routes to it (it needs no partial workspace). Input or output may be a ChannelPair cut at a multiple of 32.
-bool mfma_conv_split_applies(const MfmaConvArgs& a);
+bool mfma_conv_split_applies(const MfmaConvArgs& a, bool records);
 int mfma_conv_split(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                     const GnPartialOut* gn = nullptr, const ChannelPair* in2 = nullptr, const ChannelPair* out2 = nullptr);
 int mfma_conv_split_gn_records(const MfmaConvArgs& a, int groups);

@@ -56,16 +56,19 @@ struct Brick {
 };
 
 // R: chunks per round. PAIR: the input is two tensors whose channels follow each other (the first `c_first` in x, the
-// rest in x1). Independently, a non-null y1 splits the OUTPUT the same way.
-template <typename T, typename S, int R, int NSUB, bool PAIR>
-__global__ void __launch_bounds__(256, 2)
+// rest in x1). Independently, a non-null y1 splits the OUTPUT the same way. APART: the reduction is two rounds, and the first one's sums are
+// set aside (split_rule). They want 32 registers more: one workgroup to a CU, which the brick's LDS leaves room for anyway (with two 11 to 17 registers were
+// spilled and every other launch of one block took 0.5 us longer).
+template <typename T, typename S, int R, int NSUB, bool PAIR, bool APART = false>
+__global__ void __launch_bounds__(256, APART ? 1 : 2)
 conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ wp, const T* __restrict__ bias, T* __restrict__ y,
                   int tiles_d, int tiles_h, int tiles_w, int nblocks, uint32_t total, GnPartialOut gn, const T* __restrict__ x1,
                   T* __restrict__ y1, int c_first) {
   using B = Brick<S, NSUB>;
   constexpr int TD = S::TD, TH = S::TH, TW = S::TW, BH = S::BH, BW = S::BW;
   constexpr int PLANE = B::PLANE, SLOT = B::SLOT;
-  constexpr int RED_BYTES = MS * NSUB * 3 * 4096;  // every block from the three wavefronts that do not own it
+  constexpr int ROUNDS = APART ? 2 : 1;
+  constexpr int RED_BYTES = ROUNDS * MS * NSUB * 3 * 4096;  // every block from the three wavefronts that do not own it
   constexpr int LDS = R * SLOT > RED_BYTES ? R * SLOT : RED_BYTES;
   __shared__ __attribute__((aligned(16))) char lds[LDS];
   const int tid = threadIdx.x;
@@ -93,13 +96,16 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   }
   auto a_off = [](int k) constexpr { return R == 4 ? B::tap_off(k / 2) + (k % 2) * 2 * PLANE : B::tap_off(k); };
 
-  f32x16_t acc[MS][NSUB];
+  static_assert(!APART || NSUB == 1, "one block's sums set aside");
+  f32x16_t acc[MS][NSUB], first[MS];  // first: the first round's sums, where they are chains apart
 #pragma unroll
   for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
-    for (int ns = 0; ns < NSUB; ++ns)
+    for (int r = 0; r < 16; ++r) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[ms][ns][r] = 0.f;
+      for (int ns = 0; ns < NSUB; ++ns) acc[ms][ns][r] = 0.f;
+      first[ms][r] = 0.f;
+    }
 
   const int ncc = a.cred / kChunk;
   const int id0 = od0 - a.pd, ih0 = oh0 - a.ph, iw0 = ow0 - a.pw;
@@ -169,22 +175,36 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-  }
-
-  // The four partial results of every block meet in LDS: wavefront u collects block u = ms * NSUB + ns.
-  __syncthreads();  // the bricks are not read any more
-  float4* red = reinterpret_cast<float4*>(lds);
+    if constexpr (APART) {
+      if (c0 == 0) {
 #pragma unroll
-  for (int u = 0; u < MS * NSUB; ++u) {
-    if (u != wave) {
-      const int from = wave < u ? wave : wave - 1;  // this wavefront's place among block u's three senders
+        for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4)
-        red[((u * 3 + from) * 4 + r4) * 64 + lane] =
-            make_float4(acc[u / NSUB][u % NSUB][4 * r4], acc[u / NSUB][u % NSUB][4 * r4 + 1], acc[u / NSUB][u % NSUB][4 * r4 + 2],
-                        acc[u / NSUB][u % NSUB][4 * r4 + 3]);
+          for (int r = 0; r < 16; ++r) {
+            first[ms][r] = acc[ms][0][r];
+            acc[ms][0][r] = 0.f;
+          }
+      }
     }
   }
+
+  // The four partial results of every block meet in LDS, those of the first round before those of the second where they are apart: wavefront
+  // u collects block u = ms * NSUB + ns.
+  __syncthreads();  // the bricks are not read any more
+  float4* red = reinterpret_cast<float4*>(lds);
+  auto mine_of = [&](int round, int u) -> const f32x16_t& { return APART && round == 0 ? first[u / NSUB] : acc[u / NSUB][u % NSUB]; };
+#pragma unroll
+  for (int round = 0; round < ROUNDS; ++round)
+#pragma unroll
+    for (int u = 0; u < MS * NSUB; ++u) {
+      if (u != wave) {
+        const int from = wave < u ? wave : wave - 1;  // this wavefront's place among block u's three senders
+        const f32x16_t& v = mine_of(round, u);
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+          red[(((round * MS * NSUB + u) * 3 + from) * 4 + r4) * 64 + lane] = make_float4(v[4 * r4], v[4 * r4 + 1], v[4 * r4 + 2], v[4 * r4 + 3]);
+      }
+    }
   __syncthreads();
   f32x16_t tot;
 #pragma unroll
@@ -194,23 +214,25 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
     if (u == wave) {
       // wavefronts 0, 1, 2, 3 in that order, this one's own share from its registers
 #pragma unroll
-      for (int src = 0; src < 4; ++src) {
-        f32x16_t part;
-        if (src == u) {
-          part = acc[u / NSUB][u % NSUB];
-        } else {
-          const int from = src < u ? src : src - 1;
+      for (int round = 0; round < ROUNDS; ++round)
 #pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4) {
-            const float4 e = red[((u * 3 + from) * 4 + r4) * 64 + lane];
-            part[4 * r4] = e.x; part[4 * r4 + 1] = e.y; part[4 * r4 + 2] = e.z; part[4 * r4 + 3] = e.w;
+        for (int src = 0; src < 4; ++src) {
+          f32x16_t part;
+          if (src == u) {
+            part = mine_of(round, u);
+          } else {
+            const int from = src < u ? src : src - 1;
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+              const float4 e = red[(((round * MS * NSUB + u) * 3 + from) * 4 + r4) * 64 + lane];
+              part[4 * r4] = e.x; part[4 * r4 + 1] = e.y; part[4 * r4 + 2] = e.z; part[4 * r4 + 3] = e.w;
+            }
           }
-        }
-        if (src == 0) tot = part;
-        else
+          if (round == 0 && src == 0) tot = part;
+          else
 #pragma unroll
-          for (int r = 0; r < 16; ++r) tot[r] += part[r];
-      }
+            for (int r = 0; r < 16; ++r) tot[r] += part[r];
+        }
     }
   }
 
@@ -310,9 +332,24 @@ int64_t split_tiles(const MfmaConvArgs& a) { return tiles_of(a, split_shape(a));
 // half the MFMAs (the bits of the output do not depend on it). us, caches warm / cold: 256 -> 256 at 8x16x16 16.0 / 18.9 -> 13.1 / 16.2,
 // 128 -> 256 10.2 / 13.8 -> 8.7 / 11.4, 256 -> 256 at 5x7x9 (two samples) 15.0 / 20.5 -> 11.8 / 15.1. With 129 to 256 pairs it loses:
 // 256 -> 256 at 10x16x16 16.5 / 22.0 -> 19.2 / 22.2, at 16^3 17.6 -> 19.6 (each CU fetches the same weights and stages twice the bricks).
-int split_blocks(const MfmaConvArgs& a) { return split_tiles(a) * (a.cout / (32 * kBlocks)) <= kComputeUnits / 2 ? 1 : kBlocks; }
+int split_blocks(int64_t tiles, int cout) { return tiles * (cout / (32 * kBlocks)) <= kComputeUnits / 2 ? 1 : kBlocks; }
 
-template <typename T, typename S, int R, int NSUB, bool PAIR>
+// Whether a problem is this kernel's, and whether its two rounds' sums stay apart: see mfma_conv_split_applies.
+struct SplitRule { bool use, apart; };
+SplitRule split_rule(const MfmaConvArgs& a, bool records);
+constexpr int kApartChunks = 8;
+
+// A launch: its brick (0: 2x4x8, 1: 4x4x4, 2: 2x2x16), their number and the channel blocks of a workgroup. Rounds apart are few pairs: one block
+// and the smallest halo.
+struct SplitPlan { bool apart; int shape, blocks; int64_t tiles; };
+SplitPlan split_plan(const MfmaConvArgs& a, bool records) {
+  const bool apart = a.cred == kApartChunks * kChunk && split_rule(a, records).apart;
+  const int shape = apart ? 1 : split_shape(a);
+  const int64_t tiles = tiles_of(a, shape);
+  return SplitPlan{apart, shape, apart ? 1 : split_blocks(tiles, a.cout), tiles};
+}
+
+template <typename T, typename S, int R, int NSUB, bool PAIR, bool APART = false>
 int launch_brick(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                  const GnPartialOut& gn, const void* x1, void* y1, int first) {
   const int tiles_d = (int)cdiv(a.od, S::TD), tiles_h = (int)cdiv(a.oh, S::TH), tiles_w = (int)cdiv(a.ow, S::TW);
@@ -320,15 +357,15 @@ int launch_brick(const MfmaConvArgs& a, const void* x, const void* packed, const
   const int64_t total = (int64_t)a.n * tiles_d * tiles_h * tiles_w * nblocks;
   if (total == 0) return SFH_OK;
   if (total > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv split: %lld workgroups exceed the grid limit", (long long)total);
-  hipLaunchKernelGGL((conv_split_kernel<T, S, R, NSUB, PAIR>), dim3((unsigned)total), dim3(256), 0, st, a, (const T*)x, (const T*)packed,
+  hipLaunchKernelGGL((conv_split_kernel<T, S, R, NSUB, PAIR, APART>), dim3((unsigned)total), dim3(256), 0, st, a, (const T*)x, (const T*)packed,
                      (const T*)bias, (T*)y, tiles_d, tiles_h, tiles_w, nblocks, (uint32_t)total, gn, (const T*)x1, (T*)y1, first);
   return check_launch("conv_split_kernel");
 }
 
 template <typename T, int R, int NSUB, bool PAIR>
-int launch_split(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
+int launch_split(int shape, const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                  const GnPartialOut& gn, const void* x1, void* y1, int first) {
-  switch (split_shape(a)) {
+  switch (shape) {
     case 1: return launch_brick<T, Cube, R, NSUB, PAIR>(a, x, packed, bias, y, st, gn, x1, y1, first);
     case 2: return launch_brick<T, Rows, R, NSUB, PAIR>(a, x, packed, bias, y, st, gn, x1, y1, first);
     default: return launch_brick<T, Flat, R, NSUB, PAIR>(a, x, packed, bias, y, st, gn, x1, y1, first);
@@ -338,13 +375,16 @@ int launch_split(const MfmaConvArgs& a, const void* x, const void* packed, const
 template <typename T>
 int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                        const GnPartialOut& gn, const void* x1, void* y1, int first) {
+  const SplitPlan p = split_plan(a, gn.part != nullptr);
   const bool four = (a.cred / kChunk) % 4 == 0;
-#define SFH_SPLIT(NSUB)                                                                                \
-  x1 != nullptr ? (four ? launch_split<T, 4, NSUB, true>(a, x, packed, bias, y, st, gn, x1, y1, first)   \
-                        : launch_split<T, 2, NSUB, true>(a, x, packed, bias, y, st, gn, x1, y1, first))  \
-                : (four ? launch_split<T, 4, NSUB, false>(a, x, packed, bias, y, st, gn, x1, y1, first)  \
-                        : launch_split<T, 2, NSUB, false>(a, x, packed, bias, y, st, gn, x1, y1, first))
-  return split_blocks(a) == 1 ? SFH_SPLIT(1) : SFH_SPLIT(2);
+  if (p.apart) return x1 != nullptr ? launch_brick<T, Cube, 4, 1, true, true>(a, x, packed, bias, y, st, gn, x1, y1, first)
+                                    : launch_brick<T, Cube, 4, 1, false, true>(a, x, packed, bias, y, st, gn, x1, y1, first);
+#define SFH_SPLIT(NSUB)                                                                                         \
+  x1 != nullptr ? (four ? launch_split<T, 4, NSUB, true>(p.shape, a, x, packed, bias, y, st, gn, x1, y1, first)   \
+                        : launch_split<T, 2, NSUB, true>(p.shape, a, x, packed, bias, y, st, gn, x1, y1, first))  \
+                : (four ? launch_split<T, 4, NSUB, false>(p.shape, a, x, packed, bias, y, st, gn, x1, y1, first)  \
+                        : launch_split<T, 2, NSUB, false>(p.shape, a, x, packed, bias, y, st, gn, x1, y1, first))
+  return p.blocks == 1 ? SFH_SPLIT(1) : SFH_SPLIT(2);
 #undef SFH_SPLIT
 }
 
@@ -373,42 +413,53 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
 // 11x27x45 42.8 -> 30.6.
 // The times take nothing away from this kernel: its four partial sums to a voxel are nearer the 64-bit result than the bricks' one chain (fp16
 // results of 64 to 512 channels that are not the rounded 64-bit ones: 1.5e-3 here, 1.9e-3 in bricks, 28 problems of both directions), so 256 -> 256 at 32^3 stays at
-// 109 us though bricks take 102. Nor do they bring it what the bricks sum in eight slices (1.35e-3 there, 1.75e-3 here; four: level).
+// 109 us though bricks take 102. Eight slices are nearer still (1.35e-3, 1.75e-3 here with four sums; four: level). So what the bricks would sum in
+// eight comes here only where a slice is one chunk (256 reduction channels): the two rounds' sums stay apart and meet in the slices' order.
+// Those have the slices' bits, and so have four chunks in the place of four slices; a launch that leaves GroupNorm records stays with the
+// slices there, whose records are sums of other voxels. us, slices and their sum / four sums / eight sums: 256 -> 256 at 14x6x4 10.2 / 10.8 / 11.9, at 5x8x14
+// 11.6 / 11.4 / 12.5, at 8x4x20 12.3 / 11.1 / 12.2: no gain there, but no launch and no workspace beside it.
 // The data gradient of a depth shard's slab (D + 2 planes from D) and of the padded volume (D from D) must come from the same
 // kernel, or a shard and the whole volume would disagree in the last bit: the depth counted is the smaller of the two.
 constexpr int kSplitMaxPlane = 32 * 32, kSplitMinPerDepth = 24, kSplitFewPerDepth = 32, kSplitFewMaxChunks = 16;
 constexpr int kSplitBigPlanePairs = 240;
-// Pairs from which a volume below the plane's line comes here, and the fewer from which it does where the bricks need at most four slices. us, slices
+// Pairs from which a volume below the plane's line comes here, and the fewer from which it does where its sums are no longer than the slices'. us, slices
 // and their sum -> here: 64 -> 128 at 14x13x6 (56 pairs) 9.9 -> 5.6, at 5x10x11 (36) 10.0 -> 5.5, 128 -> 128 at 9x12x8 (30) 13.2 -> 7.7, at 4x6x20 (24) 11.5 -> 7.7.
 // Long reductions on fewer where the slices are far behind: 512 -> 512 at 9x9x6 (120) 35.1 -> 22.1.
 int64_t split_line(int chunks) { return chunks <= 4 ? kComputeUnits / 4 : chunks <= 8 ? kComputeUnits / 4 + 1 : kComputeUnits / 2 + 1; }
-int64_t split_line_few_slices(int chunks, int cout) { return chunks <= 4 && cout >= 128 ? 24 : chunks <= 8 && cout >= 256 ? 48 : split_line(chunks); }
+int64_t split_line_few(int chunks, int cout) { return chunks <= 4 && cout >= 128 ? 24 : chunks <= 8 && cout >= 256 ? 48 : split_line(chunks); }
 
-bool mfma_conv_split_applies(const MfmaConvArgs& a) {
-  if (a.kd != 3 || a.kh != 3 || a.kw != 3) return false;
-  if (a.cred < 2 * kChunk || a.cred % (2 * kChunk) != 0 || a.cout % (32 * kBlocks) != 0) return false;
+namespace {
+SplitRule split_rule(const MfmaConvArgs& a, bool records) {
+  if (a.kd != 3 || a.kh != 3 || a.kw != 3) return {false, false};
+  if (a.cred < 2 * kChunk || a.cred % (2 * kChunk) != 0 || a.cout % (32 * kBlocks) != 0) return {false, false};
   const int chunks = a.cred / kChunk, pair = a.cout / (32 * kBlocks);
   MfmaConvArgs core = a;
   core.od = a.id < a.od ? a.id : a.od;
   const int64_t per_depth = (int64_t)a.n * cdiv(a.oh, Flat::TH) * cdiv(a.ow, Flat::TW) * pair;
   const int64_t pairs = per_depth * cdiv(core.od, Flat::TD), rounds = cdiv(pairs, kComputeUnits);
   auto sooner = [&](int percent) { return 100 * split_time(split_tiles(core) * pair, chunks) < percent * mfma_conv_brick_time(core); };
-  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return pairs > kSplitBigPlanePairs && sooner(88);
+  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return {pairs > kSplitBigPlanePairs && sooner(88), false};
   const bool few = per_depth <= kSplitFewPerDepth && chunks >= kSplitFewMaxChunks;
-  if (!few && per_depth >= kSplitMinPerDepth) return true;
+  if (!few && per_depth >= kSplitMinPerDepth) return {true, false};
   if (pairs >= split_line(chunks))
-    return rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || sooner(110);
-  if (mfma_conv_brick_slices(core) > 4) return false;
-  return pairs >= split_line_few_slices(chunks, a.cout) || (chunks >= kSplitFewMaxChunks && sooner(70));
+    return {rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || sooner(110), false};
+  const int slices = mfma_conv_brick_slices(core);
+  const bool apart = slices > 4;
+  if ((apart && chunks != kApartChunks) || (records && slices == chunks)) return {false, false};
+  return {pairs >= split_line_few(chunks, a.cout) || (chunks >= kSplitFewMaxChunks && sooner(70)), apart};
 }
+}  // namespace
+
+bool mfma_conv_split_applies(const MfmaConvArgs& a, bool records) { return split_rule(a, records).use; }
 
 MfmaConvGeometry mfma_conv_split_geometry(const MfmaConvArgs&) { return MfmaConvGeometry{kKernelSplit, kBrickVoxels, kBlocks, 1}; }
 
 int mfma_conv_split_gn_records(const MfmaConvArgs& a, int groups) {
-  const int span = 32 * split_blocks(a);
+  const SplitPlan p = split_plan(a, true);
+  const int span = 32 * p.blocks;
   if (!gn_partials_fit(a.cout, groups, span)) return 0;
   const int cg = a.cout / groups;
-  const int64_t records = split_tiles(a) / a.n * (cg > span ? cg / span : 1);
+  const int64_t records = p.tiles / a.n * (cg > span ? cg / span : 1);
   return records <= 0x7fffffff ? (int)records : 0;
 }
 

@@ -62,7 +62,8 @@ def test_slab_and_padded_volume_add_in_one_order(cin, cout):
     (128, 128, (60, 30, 31), "split"),
     (64, 64, (64, 32, 32), "split"),
     (256, 256, (29, 28, 14), "split"),
-    (256, 256, (5, 8, 14), "brick"),     # eight slices
+    (512, 512, (5, 8, 8), "brick"),      # eight slices of two chunks each
+    (256, 256, (5, 8, 14), "split"),     # eight of one: as many partial sums there
     (256, 256, (11, 4, 9), "split"),     # four
 ])
 def test_launch_times_take_no_partial_sums_away(cin, cout, spatial, kernel):

@@ -19,8 +19,7 @@ CASES = [
     (1, 128, 128, (4, 6, 20), "split", 64),     # 24: the fewest
     (1, 128, 128, (4, 6, 12), "brick", 256),    # 16
     (1, 256, 256, (3, 8, 14), "brick", 256),    # 32
-    (1, 256, 256, (5, 8, 14), "brick", 256),    # 48, but the bricks' eight slices are the nearer sums
-    (1, 256, 256, (11, 4, 9), "split", 64),     # 48 against four slices
+    (1, 256, 256, (5, 8, 14), "split", 64),     # 48
     (1, 512, 512, (9, 9, 6), "split", 64),      # 120 pairs of a long reduction on cut bricks
     (2, 128, 64, (19, 30, 35), "brick", None),  # a round and a bit of the wide kernel's workgroups would be two
     (1, 256, 256, (32, 32, 8), "split", 64),

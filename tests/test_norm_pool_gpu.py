@@ -52,9 +52,8 @@ def test_same_bits_as_two_launches(device, n, c, spatial, dtype, halo, relu):
         y = conv_then_norm(conv, norm, x)
         # (a halo asks for one sample, and records come only from the kernels that offer them)
         assert hasattr(y, "_sfh_pooled") == (fused and not (halo and n > 1) and bool(y is not None and _records(conv, x0)))
-        given = y.__dict__.pop("_sfh_pooled", None)
-        pooled, skip = pool.with_skip(y, given)
-        assert given is None or pooled.data_ptr() == given[0].data_ptr()
+        pooled, skip = pool.with_skip(y)
+        assert not hasattr(y, "_sfh_pooled")
         slabs = [t._sfh_slab[0].clone() for t in (pooled, skip) if halo and n == 1]
         grads = torch.autograd.grad((pooled, skip), (x, conv.weight, norm.weight, norm.bias), (gp, gs))
         with torch.no_grad():
@@ -77,9 +76,7 @@ def test_what_is_not_reused(device):
     with torch.no_grad():
         want = torch.nn.functional.max_pool3d(conv_then_norm(conv, norm, x).float(), 2)
         y = conv_then_norm(conv, norm, x)
-        given = y._sfh_pooled
-        pooled = wide.with_skip(y, given)[0]                                         # another halo
-        assert pooled.data_ptr() != given[0].data_ptr() and torch.equal(pooled.float(), want) and hasattr(pooled, "_sfh_slab")
+        assert torch.equal(wide(y).float(), want) and hasattr(wide(y), "_sfh_slab")  # another halo
         y = conv_then_norm(conv, norm, x)
         a, b = pool(y), pool(y)                                                      # a second pooling has its own tensor
         assert a.data_ptr() != b.data_ptr() and torch.equal(a.float(), want) and torch.equal(b.float(), want)
@@ -109,9 +106,7 @@ def test_nan_and_infinity(device):
         norm.pool_next = pool_next
         with torch.no_grad():
             y = conv_then_norm(conv, norm, x)
-            given = y.__dict__.pop("_sfh_pooled", None)
-            assert (given is None) == (pool_next is None)
-            outs.append((y.clone(), FastMaxPool3d(2).with_skip(y, given)[0]))
+            outs.append((y.clone(), FastMaxPool3d(2)(y)))
     for a, b in zip(*outs):
         assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num())
 
@@ -180,6 +175,24 @@ def test_handed_over_is_the_launched_one(device, n, c, spatial, halo):
         slabs = [t._sfh_slab[0].clone() for t in (pooled, skip) if halo]
         results.append([pooled.detach(), skip.detach(), *slabs, *torch.autograd.grad((pooled, skip), (x, conv.weight, norm.weight, norm.bias), (gp, gs))])
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+def test_handed_over_nan_infinity_and_another_halo(device):
+    conv, norm = _pair(32, device, torch.bfloat16)
+    norm.pool_next = 0
+    pool, wide = FastMaxPool3d(2), FastMaxPool3d(2)
+    wide.out_halo = 1
+    x = torch.randn(1, 32, 4, 8, 34, device=device).to(torch.bfloat16)
+    x[0, 3, 1, 2, 3] = float("nan")
+    x[0, 3, 1, 5, 20] = float("inf")
+    x = x.contiguous(memory_format=CL)
+    with torch.no_grad():
+        y = conv_then_norm(conv, norm, x)
+        given = y.__dict__.pop("_sfh_pooled")
+        want, taken, other = pool(y), pool.with_skip(y, given)[0], wide.with_skip(y, given)[0]
+    assert taken.data_ptr() == given[0].data_ptr() and other.data_ptr() != given[0].data_ptr() and hasattr(other, "_sfh_slab")
+    for got in (taken, other):
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
 
 
 @pytest.mark.parametrize("relu", [True, False])

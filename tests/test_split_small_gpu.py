@@ -74,6 +74,9 @@ def _conv64(x, w):
     (64, 128, (14, 13, 6), "split", "brick"),    # few pairs of 128 and more produced channels
     (128, 128, (4, 6, 12), "brick", "brick"),    # 16 pairs: too few
     (512, 512, (9, 9, 6), "split", "split"),     # a long reduction by the times
+    (256, 256, (5, 8, 14), "split", "split"),    # in the place of eight slices: two rounds, their sums apart
+    (256, 256, (3, 16, 12), "split", "split"),   # ... a row over
+    (256, 256, (11, 4, 9), "split", "split"),    # in the place of four: one chain a wavefront
     (128, 64, (33, 57, 50), "brick", "brick"),   # bricks in the wide kernel's place by the times
     (128, 64, (31, 61, 65), "wide", "brick"),
 ])
@@ -94,3 +97,20 @@ def test_lines_that_the_times_draw(cin, cout, spatial, fwd, dgrad):
             assert torch.all((result.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * want.abs().max())
         if len({g["slices"] for g in geom[direction]}) == 1:  # (slices are cut by a launch's own planes)
             assert torch.equal(got, from_slab)
+
+
+@pytest.mark.parametrize("n,cin,cout,spatial", [(1, 128, 256, (8, 8, 8)), (1, 128, 128, (4, 6, 20)), (2, 128, 128, (5, 7, 9)),
+                                                (1, 256, 256, (5, 8, 14)), (1, 256, 256, (8, 4, 20)), (2, 256, 256, (7, 6, 4))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_slices_and_their_bits(n, cin, cout, spatial, dtype):
+    """A chunk to a slice: the launch that leaves GroupNorm records is the bricks' in slices, the one without the small-volume kernel's,
+    whose wavefronts (and rounds) add in the slices' order.  Against float64 as well."""
+    x, _, w = _operands(n, cin, cout, spatial, dtype)
+    assert c3.launch_geometry(x.shape, w.shape, 1, 1, 1, dtype, "fwd")["kernel"] == "split"
+    b = torch.randn(cout, device="cuda").to(dtype)
+    alone, recorded = sa.conv3d_forward(x, w, b, 1, 1), sa.conv3d_forward(x, w, b, 1, 1, gn_groups=8)
+    assert recorded._sfh_gn_partials[1] == -(-cout * spatial[0] * spatial[1] * spatial[2] // 1024)  # of the launch that sums the slices
+    assert torch.equal(alone, recorded)
+    want = _conv64(x, w) + b.double().view(1, -1, 1, 1, 1)
+    half_ulp = 2.0 ** -8 if dtype is torch.bfloat16 else 2.0 ** -11
+    assert torch.all((alone.double() - want).abs() <= half_ulp * want.abs() + 1e-5 * want.abs().max())
