@@ -46,15 +46,35 @@ inline ColumnCut cut_columns(int64_t ncols, int64_t steps, int64_t wgs) {
   return cut_columns_in<int64_t>(ncols, steps, wgs);
 }
 
+// The cut until every workgroup has an item, and no further: the order of sums that were taken before the busiest workgroup's time decided. For
+// launches whose sums are read: statistics move with their order, and with them all that a network computes behind them (its
+// logits by 4e-3, as by any other rounding).
+inline ColumnCut cut_until_busy(int64_t ncols, int64_t steps, int64_t wgs) {
+  auto parts = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  int64_t segs = ncols >= wgs ? 1 : parts(wgs, ncols);
+  if (segs > steps) segs = steps;
+  const int64_t len = parts(steps, segs);
+  segs = parts(steps, len);
+  ColumnCut c{(int)segs, (int)len, -1, 0, 0, 0};
+  if (ncols * segs > 0x7fffffff) return c;
+  c.items = (int)(ncols * segs);
+  c.items_per_wg = (int)parts(c.items, wgs);
+  c.wgs = (int)parts(c.items, c.items_per_wg);
+  c.cost = c.items_per_wg * (len + 1);
+  return c;
+}
+
 // The cut of `n` samples of `cols` columns: one line of columns (parts 1), or every sample by workgroups of its own (parts n; the cut is that of
 // one), whose sums are then those of one sample, so that the normalisation behind the convolution needs no statistics pass. That is worth an
 // end up to an eighth later where somebody takes the sums (`records`), and only there: three samples of 51x126x40 end 27 steps against 24 (32 -> 64
-// channels). Samples of a few columns stay in one line (the statistics pass of a smaller one is the same launch whatever it reads).
+// channels). Samples of a few columns stay in one line (the statistics pass of a smaller one is the same launch whatever it reads). One sample
+// whose sums are taken keeps their order.
 struct BatchCut {
   int parts;
   ColumnCut cut;
 };
 inline BatchCut cut_batch(int64_t n, int64_t cols, int64_t steps, int64_t wgs, bool records) {
+  if (records && n == 1) return BatchCut{1, cut_until_busy(cols, steps, wgs)};
   const BatchCut line{1, cut_columns(cols * n, steps, wgs)};
   if (!records || line.cut.items < 0 || n == 1 || wgs / n < 8) return line;
   const BatchCut apart{(int)n, cut_columns(cols, steps, wgs / n)};

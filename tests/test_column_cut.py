@@ -64,13 +64,24 @@ def test_batch_without_records_ends_soonest(cut):
         assert got == (1, *rest, cost), (n, cols, steps, wgs)
 
 
+def test_one_sample_with_records_keeps_the_order_of_its_sums(cut):
+    """Until every workgroup has an item, and no further."""
+    problems = [(1, *p[1:]) for p in _problems()] + [(1, 54 // 4 * 27, 53, 256), (1, 64, 32, 256), (1, 700, 3, 256)]
+    for (n, cols, steps, wgs), got in zip(problems, cut([(*p, 1) for p in problems])):
+        want = 1 if cols >= wgs else min(-(-wgs // cols), steps)
+        length = -(-steps // want)
+        segs = -(-steps // length)
+        per_wg = -(-cols * segs // wgs)
+        assert got == (1, segs, length, cols * segs, per_wg, -(-cols * segs // per_wg), per_wg * (length + 1)), (n, cols, steps, wgs)
+
+
 def test_batch_with_records_is_walked_apart_where_that_costs_an_eighth_at_most(cut):
-    problems = _problems()
+    problems = [p for p in _problems() if p[0] > 1]
     apart = 0
     for (n, cols, steps, wgs), got in zip(problems, cut([(*p, 1) for p in problems])):
         line = _reference(n * cols, steps, wgs)
         want = (1, *line[1:], line[0])
-        if n > 1 and wgs // n >= 8:
+        if wgs // n >= 8:
             one = _reference(cols, steps, wgs // n)
             if 8 * one[0] <= 9 * line[0] and one[5] >= 8:
                 want = (n, *one[1:], one[0])

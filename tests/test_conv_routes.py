@@ -73,6 +73,18 @@ def test_launch_times_take_no_partial_sums_away(cin, cout, spatial, kernel):
         assert _kernel(1, cin, cout, spatial, direction) == kernel
 
 
+@pytest.mark.parametrize("cin,cout,spatial,records", [
+    (32, 32, (54, 105, 99), 140),      # columns for every workgroup once; by their times 224
+    (256, 256, (24, 20, 28), 240),     # bricks of 2 x 4 x 8; 210 of 4 x 4 x 4
+    (512, 512, (12, 10, 14), 36),      # 30 of 2 x 2 x 16
+    (64, 64, (55, 28, 41), 196),       # 336 of another brick
+    (128, 64, (33, 57, 50), 270),      # the wide kernel's; 504 bricks
+])
+def test_groupnorm_records_do_not_go_by_times(cin, cout, spatial, records):
+    """Records are sums of a launch's bricks: what a network computes behind them has the bits it had before launch times chose bricks."""
+    assert c3._Problem((1, cin, *spatial), (cout, cin, 3, 3, 3), 1, 1, 1, torch.bfloat16).gn_records(8) == records
+
+
 @pytest.mark.parametrize("n,cin,cout,spatial,slices", [
     (1, 128, 128, (43, 29, 34), 5),     # tiles; columns would be 16 slices
     (1, 64, 32, (54, 40, 76), 42),      # tiles; 120
