@@ -84,6 +84,7 @@ MfmaConvArgs dgrad_mfma_args(const sfh_conv3d_desc& p, const int32_t out[3]) {
   a.cout = p.cin; a.od = p.in_d; a.oh = p.in_h; a.ow = p.in_w;
   a.kd = p.kd; a.kh = p.kh; a.kw = p.kw;
   a.pd = (p.kd - 1) - p.pd; a.ph = (p.kh - 1) - p.ph; a.pw = (p.kw - 1) - p.pw;
+  a.gradient = 1;
   return a;
 }
 

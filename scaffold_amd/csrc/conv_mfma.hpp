@@ -13,6 +13,7 @@ struct MfmaConvArgs {
   int n, cred, id, ih, iw;
   int cout, od, oh, ow;
   int kd, kh, kw, pd, ph, pw;
+  int gradient;  // 1: a data gradient, whose order of sums estimated times do not choose
 };
 
 bool mfma_conv_supported(const MfmaConvArgs& a, int dtype);

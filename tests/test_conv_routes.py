@@ -57,20 +57,24 @@ def test_slab_and_padded_volume_add_in_one_order(cin, cout):
             assert (padded == "split") == (slab == "split"), (direction, (d, h, w), padded, slab)
 
 
-@pytest.mark.parametrize("cin,cout,spatial,kernel", [
-    (256, 256, (32, 32, 32), "split"),
-    (128, 128, (60, 30, 31), "split"),
-    (64, 64, (64, 32, 32), "split"),
-    (256, 256, (29, 28, 14), "split"),
-    (512, 512, (5, 8, 8), "brick"),      # eight slices of two chunks each
-    (256, 256, (5, 8, 14), "split"),     # eight of one: as many partial sums there
-    (256, 256, (11, 4, 9), "split"),     # four
+@pytest.mark.parametrize("cin,cout,spatial,forward,gradient", [
+    (256, 256, (32, 32, 32), "split", "split"),
+    (128, 128, (60, 30, 31), "split", "split"),
+    (64, 64, (64, 32, 32), "split", "split"),
+    (256, 256, (29, 28, 14), "split", "split"),
+    (512, 512, (5, 8, 8), "brick", "brick"),     # eight slices of two chunks each
+    (256, 256, (5, 8, 14), "split", "split"),    # eight of one: as many partial sums there
+    (128, 128, (9, 12, 8), "split", "split"),    # four of one
+    (256, 256, (11, 4, 9), "split", "brick"),    # four of two
+    (64, 128, (14, 13, 6), "split", "brick"),
+    (128, 64, (14, 13, 6), "brick", "brick"),    # the gradient's two slices are one chunk each, which the small-volume kernel cuts in two
+    (64, 64, (9, 27, 50), "split", "brick"),     # a plane past 32 x 32
 ])
-def test_launch_times_take_no_partial_sums_away(cin, cout, spatial, kernel):
+def test_launch_times_take_no_partial_sums_away(cin, cout, spatial, forward, gradient):
     """Four partial sums to a voxel are nearer the exact one than the bricks' single chain, eight slices nearer still: where the
-    small-volume kernel served a volume, or the bricks in eight slices, no estimate of times moves it."""
-    for direction in ("fwd", "bwd-data"):
-        assert _kernel(1, cin, cout, spatial, direction) == kernel
+    small-volume kernel served a volume, or the bricks in eight slices, no estimate of times moves it; nor a data gradient to another order."""
+    assert _kernel(1, cin, cout, spatial) == forward
+    assert _kernel(1, cin, cout, spatial, "bwd-data") == gradient
 
 
 @pytest.mark.parametrize("cin,cout,spatial,records", [

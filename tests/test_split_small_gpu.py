@@ -68,15 +68,16 @@ def _conv64(x, w):
 
 
 @pytest.mark.parametrize("cin,cout,spatial,fwd,dgrad", [
-    (64, 128, (27, 61, 33), "brick", "split"),   # planes past 32 x 32; the slab's data gradient was the wide kernel's
-    (64, 64, (9, 27, 50), "split", "split"),     # ... from 240 pairs on
+    (64, 128, (27, 61, 33), "brick", "brick"),   # planes past 32 x 32
+    (64, 64, (9, 27, 50), "split", "brick"),     # ... from 240 pairs on
     (64, 64, (8, 27, 50), "brick", "brick"),     # 196
     (64, 128, (14, 13, 6), "split", "brick"),    # few pairs of 128 and more produced channels
+    (128, 128, (9, 12, 8), "split", "split"),    # ... whose four sums are the slices', so that the data gradient comes too
     (128, 128, (4, 6, 12), "brick", "brick"),    # 16 pairs: too few
-    (512, 512, (9, 9, 6), "split", "split"),     # a long reduction by the times
+    (512, 512, (9, 9, 6), "split", "brick"),     # a long reduction by the times
     (256, 256, (5, 8, 14), "split", "split"),    # in the place of eight slices: two rounds, their sums apart
-    (256, 256, (3, 16, 12), "split", "split"),   # ... a row over
-    (256, 256, (11, 4, 9), "split", "split"),    # in the place of four: one chain a wavefront
+    (256, 256, (3, 16, 12), "split", "split"),   # 72 pairs
+    (256, 256, (11, 4, 9), "split", "brick"),    # in the place of four: one chain a wavefront
     (128, 64, (33, 57, 50), "brick", "brick"),   # bricks in the wide kernel's place by the times
     (128, 64, (31, 61, 65), "wide", "brick"),
 ])
