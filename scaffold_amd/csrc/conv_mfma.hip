@@ -757,7 +757,7 @@ int mfma_pack_weight_batch(const MfmaPackItem* items, int n, int dtype, hipStrea
 static bool served_by_split(const MfmaConvArgs& a, bool records) { return !mfma_conv_wide_fits(a) && mfma_conv_split_applies(a, records); }
 
 size_t mfma_conv_partial_bytes(const MfmaConvArgs& a, bool records) {
-  if (a.cred == kChunk || mfma_conv_wide_applies(a, records) || served_by_split(a, records)) return 0;
+  if (a.cred == kChunk || mfma_conv_wide_applies(a) || served_by_split(a, records)) return 0;
   const GatherPlan p = cut_plan(a);
   if (p.ksplit == 1) return 0;
   return align_up((size_t)p.ksplit * a.n * a.od * a.oh * a.ow * a.cout * sizeof(float), 256);
@@ -768,26 +768,25 @@ int mfma_conv_brick_slices(const MfmaConvArgs& a) { return cut_plan(a).ksplit; }
 int64_t mfma_conv_brick_time(const MfmaConvArgs& a) { return brick_time(a, gather_plan(a, false)); }
 
 MfmaConvGeometry mfma_conv_gather_geometry(const MfmaConvArgs& a) {
-  if (mfma_conv_wide_applies(a, false)) return mfma_conv_wide_geometry(a);
+  if (mfma_conv_wide_applies(a)) return mfma_conv_wide_geometry(a);
   if (served_by_split(a, false)) return mfma_conv_split_geometry(a);
   const GatherPlan p = gather_plan(a, false);
   return MfmaConvGeometry{kKernelBrick, (int)tile_voxels(p.shape % 3), p.nsub, p.ksplit};
 }
 
 int mfma_conv_gather_gn_records(const MfmaConvArgs& a, int groups) {
-  if (mfma_conv_wide_applies(a, true)) return mfma_conv_wide_gn_records(a, groups);
+  if (mfma_conv_wide_applies(a)) return mfma_conv_wide_gn_records(a, groups);
   if (served_by_split(a, true)) return mfma_conv_split_gn_records(a, groups);
   return gather_gn_records(a, gather_plan(a, true), groups);
 }
 
 int mfma_conv_gather(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y,
                      void* partial, hipStream_t st, const GnPartialOut* gn, const ChannelPair* in2, const ChannelPair* out2) {
-  const bool records = gn != nullptr && gn->part != nullptr;
-  if (mfma_conv_wide_applies(a, records)) {
+  if (mfma_conv_wide_applies(a)) {
     if (out2 != nullptr) return fail(SFH_ERR_UNSUPPORTED, "conv wide: the output cannot be a pair of tensors");
     return mfma_conv_wide(a, dtype, x, packed, bias, y, st, gn, in2);
   }
-  if (served_by_split(a, records)) return mfma_conv_split(a, dtype, x, packed, bias, y, st, gn, in2, out2);
+  if (served_by_split(a, gn != nullptr && gn->part != nullptr)) return mfma_conv_split(a, dtype, x, packed, bias, y, st, gn, in2, out2);
   if (dtype == SFH_BF16) return launch_typed<bf16_t>(a, dtype, x, packed, bias, y, partial, st, gn, in2, out2);
   return launch_typed<fp16_t>(a, dtype, x, packed, bias, y, partial, st, gn, in2, out2);
 }

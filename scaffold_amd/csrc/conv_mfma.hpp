@@ -47,16 +47,15 @@ int mfma_conv_gather(const MfmaConvArgs& a, int dtype, const void* x, const void
                      void* partial, hipStream_t st, const GnPartialOut* gn = nullptr, const ChannelPair* in2 = nullptr,
                      const ChannelPair* out2 = nullptr);
 // Same contract, wide-tile kernel (64 or more reduction channels, rows of more than 16 voxels): `applies` is a pure
-// function of the shape; mfma_conv_gather routes to it (it needs no partial workspace). records: for a launch that leaves GroupNorm records,
-// which are sums of bricks: those do not go by estimated times, here and below.
-bool mfma_conv_wide_applies(const MfmaConvArgs& a, bool records);
+// function of the shape; mfma_conv_gather routes to it (it needs no partial workspace).
+bool mfma_conv_wide_applies(const MfmaConvArgs& a);
 bool mfma_conv_wide_fits(const MfmaConvArgs& a);  // also where the brick kernel serves it: what pairs of tensors it takes follows this
 int mfma_conv_wide(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                    const GnPartialOut* gn = nullptr, const ChannelPair* in2 = nullptr);
 // Same contract, the kernel for the small volumes of the deep levels: 64-voxel bricks, the reduction cut over the four
 // wavefronts of a workgroup and summed in LDS (conv_split.hip). `applies` is a pure function of the shape; mfma_conv_gather
 // routes to it (it needs no partial workspace). Input or output may be a ChannelPair cut at a multiple of 32.
-bool mfma_conv_split_applies(const MfmaConvArgs& a, bool records);
+bool mfma_conv_split_applies(const MfmaConvArgs& a, bool records);  // records: for a launch that leaves GroupNorm records
 int mfma_conv_split(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                     const GnPartialOut* gn = nullptr, const ChannelPair* in2 = nullptr, const ChannelPair* out2 = nullptr);
 int mfma_conv_split_gn_records(const MfmaConvArgs& a, int groups);

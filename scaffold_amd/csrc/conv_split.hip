@@ -411,11 +411,11 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
 // where the bricks leave more over, by the busiest CU's share, than the 10 % that 64-voxel bricks lose at equal shares, or where what either launch
 // takes says so within a tenth. us, bricks -> here: 64 -> 64 at 256x16x16 (1024 pairs, equal shares) 19.2 -> 21.2, 128 -> 128 at 128x16x16 31.0 -> 33.9; 128 -> 64
 // at 200x20x20 (1500 pairs, 768 against 993 voxel blocks) 56 -> 46, 64 -> 64 at 64x24x24 (576 pairs) 17.9 -> 16.0. Planes past 32 x 32 come here by the times,
-// from about a round of pairs on and by more than a tenth: 64 -> 64 at 17x36x35 15.9 -> 9.7, at 9x27x50 12.1 -> 7.9, 128 -> 128 at 10x28x56 25.8 -> 17.0, 128 -> 256 at
-// 11x27x45 42.8 -> 30.6.
-// All that is for a forward by itself. A launch that leaves GroupNorm records and a data gradient come here by the rules before the times: a change in
-// the order of their sums would go through every layer behind them (4 to 7e-3 of a step's logits and gradients, each as exact). Where the
-// slices' bits are kept (below), a data gradient comes here by the fewer pairs too.
+// from about a round of pairs on and where a quarter and more is gained (another order of sums is worth no less): 64 -> 64 at 17x36x35
+// 15.9 -> 9.7, at 9x27x50 12.1 -> 7.9, 128 -> 128 at 10x28x56 25.8 -> 17.0.
+// All that is for the forward, with GroupNorm records or without (the result is the same bits either way). A data gradient comes here by the rules
+// before the times: nothing is gained by another order of its sums that is worth a step's gradients in other bits. Where the slices' bits
+// are kept (below), it comes here by the fewer pairs too.
 // The times take nothing away from this kernel: its four partial sums to a voxel are nearer the 64-bit result than the bricks' one chain (fp16
 // results of 64 to 512 channels that are not the rounded 64-bit ones: 1.5e-3 here, 1.9e-3 in bricks, 28 problems of both directions), so 256 -> 256 at 32^3 stays at
 // 109 us though bricks take 102. Eight slices are nearer still (1.35e-3, 1.75e-3 here with four sums; four: level). So what the bricks would sum in
@@ -442,17 +442,18 @@ SplitRule split_rule(const MfmaConvArgs& a, bool records) {
   core.od = a.id < a.od ? a.id : a.od;
   const int64_t per_depth = (int64_t)a.n * cdiv(a.oh, Flat::TH) * cdiv(a.ow, Flat::TW) * pair;
   const int64_t pairs = per_depth * cdiv(core.od, Flat::TD), rounds = cdiv(pairs, kComputeUnits);
-  const bool kept = records || a.gradient != 0;  // the order of sums does not go by the times
+  const bool kept = a.gradient != 0;  // the order of sums does not go by the times
   auto sooner = [&](int percent) { return 100 * split_time(split_tiles(core) * pair, chunks) < percent * mfma_conv_brick_time(core); };
-  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return {!kept && pairs > kSplitBigPlanePairs && sooner(88), false};
+  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return {!kept && pairs > kSplitBigPlanePairs && sooner(72), false};
   const bool few = per_depth <= kSplitFewPerDepth && chunks >= kSplitFewMaxChunks;
   if (!few && per_depth >= kSplitMinPerDepth) return {true, false};
   if (pairs >= split_line(chunks))
     return {rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || (!kept && sooner(110)), false};
   const int slices = mfma_conv_brick_slices(core);
   const bool apart = slices > 4, same_bits = slices == chunks && chunks % 4 == 0;  // (two chunks are cut in halves of 16 channels here)
-  if ((apart && !same_bits) || records || (a.gradient && !same_bits)) return {false, false};
-  return {pairs >= split_line_few(chunks, a.cout) || (chunks >= kSplitFewMaxChunks && sooner(70)), apart};
+  if (same_bits ? records : apart || kept) return {false, false};
+  const bool enough = pairs >= split_line_few(chunks, a.cout) && (same_bits || sooner(72));
+  return {enough || (chunks >= kSplitFewMaxChunks && sooner(70)), apart};
 }
 }  // namespace
 

@@ -393,12 +393,11 @@ int64_t wide_workgroups(const MfmaConvArgs& a, int shape) {
 }
 
 // The depth that launch rules count: that of a shard's planes in both forms of its gradients, the slab's (D + 2 planes from D) and the padded
-// volume's. Where the slab's own decided, the padded volume's gradient could be the small-volume kernel's, which adds in another order (of
-// 64 -> 128 channels at 27x61x33: 256 workgroups of 4x4x32 for the slab, 224 for the volume). An odd number of chunks never goes there: this
-// kernel and the bricks add alike.
+// volume's. Where the slab's own decided, the padded volume's gradient could be another kernel's, and each adds in an order of its own: this
+// one 16 channels of all taps after 16, the bricks 32 (of 64 -> 128 channels at 27x61x33: 256 workgroups of 4x4x32 for the slab, 224 for the volume).
 MfmaConvArgs wide_core(const MfmaConvArgs& a) {
   MfmaConvArgs core = a;
-  if (a.cred % 64 == 0 && a.id < a.od) core.od = a.id;
+  if (a.id < a.od) core.od = a.id;
   return core;
 }
 
@@ -417,8 +416,8 @@ int wide_shape(const MfmaConvArgs& core) {
   return wide_workgroups(a, 1) >= kComputeUnits ? 1 : wide_workgroups(a, 3) >= kComputeUnits ? 3 : -1;
 }
 
-// Launch geometry, a pure function of the problem and of whether the launch leaves GroupNorm records.
-WidePlan wide_plan(const MfmaConvArgs& a, bool records) {
+// Launch geometry, a pure function of the problem.
+WidePlan wide_plan(const MfmaConvArgs& a) {
   WidePlan p{false, 0};
   const MfmaConvArgs core = wide_core(a);
   const int shape = wide_shape(core);
@@ -432,11 +431,11 @@ WidePlan wide_plan(const MfmaConvArgs& a, bool records) {
       mfma_conv_brick_cost(core) * 100 < cdiv(wgs, kComputeUnits) * 1024 * 2 * 100 * (a.cred < 256 ? 97 : 92)) return p;
   // Up to there it does where the times say that the bricks take two thirds of this kernel's (10 us a chunk and round of 1024-voxel
   // workgroups, 5.6 of 512, a last round counted at four fifths of a whole one; 4 % rms): a round and a bit of workgroups of a whole CU each. us, here ->
-  // there: 128 -> 64 at two samples of 45x30x35 79.6 -> 45.6, of 17x100x52 153 -> 91, at 33x57x50 84.8 -> 53; 31x61x65, 76 % by the times, stays. (Both add a
-  // voxel's products in one order; records are sums of tiles, so a launch that leaves them does not go by the times.)
+  // there: 128 -> 64 at two samples of 45x30x35 79.6 -> 45.6, of 17x100x52 153 -> 91, at 33x57x50 84.8 -> 53; 31x61x65, 76 % by the times, stays. A data
+  // gradient stays as well: its bits do not go by the times.
   const int64_t own = wide_workgroups(core, shape), rounds = cdiv(own, kComputeUnits);
   const int64_t time = a.cred / 32 * (shape == 1 ? 2002 : 1111) * (4 * rounds * kComputeUnits + own) / (5 * kComputeUnits);
-  if (!records && a.cred % 64 == 0 && 3 * mfma_conv_brick_time(core) < 2 * time) return p;
+  if (!a.gradient && a.cred % 64 == 0 && 3 * mfma_conv_brick_time(core) < 2 * time) return p;
   p.use = true;
   p.shape = shape;
   return p;
@@ -475,19 +474,18 @@ int launch_typed(const MfmaConvArgs& a, const WidePlan& p, const void* x, const 
 
 }  // namespace
 
-bool mfma_conv_wide_applies(const MfmaConvArgs& a, bool records) { return wide_plan(a, records).use; }
+bool mfma_conv_wide_applies(const MfmaConvArgs& a) { return wide_plan(a).use; }
 
-static MfmaConvGeometry geometry_of(const WidePlan& p) {
+MfmaConvGeometry mfma_conv_wide_geometry(const MfmaConvArgs& a) {
   static const int td[5] = {4, 8, 8, 4, 4}, nsub[5] = {4, 2, 1, 2, 1};
+  const WidePlan p = wide_plan(a);
   return MfmaConvGeometry{kKernelWide, td[p.shape] * 4 * 32, nsub[p.shape], 1};
 }
 
-MfmaConvGeometry mfma_conv_wide_geometry(const MfmaConvArgs& a) { return geometry_of(wide_plan(a, false)); }
-
 int mfma_conv_wide_gn_records(const MfmaConvArgs& a, int groups) {
-  const WidePlan p = wide_plan(a, true);
+  const WidePlan p = wide_plan(a);
   if (!p.use) return 0;
-  const MfmaConvGeometry g = geometry_of(p);
+  const MfmaConvGeometry g = mfma_conv_wide_geometry(a);
   const int span = 32 * g.blocks;
   if (!gn_partials_fit(a.cout, groups, span)) return 0;
   const int cg = a.cout / groups;
@@ -502,7 +500,7 @@ bool mfma_conv_wide_pair_ok(const MfmaConvArgs& a, int first) { return mfma_conv
 
 int mfma_conv_wide(const MfmaConvArgs& a, int dtype, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                    const GnPartialOut* gn, const ChannelPair* in2) {
-  const WidePlan p = wide_plan(a, gn != nullptr && gn->part != nullptr);
+  const WidePlan p = wide_plan(a);
   if (!p.use) return fail(SFH_ERR_UNSUPPORTED, "conv wide: not applicable to this problem");
   if (in2 != nullptr && (in2->second == nullptr || !mfma_conv_wide_pair_ok(a, in2->first)))
     return fail(SFH_ERR_UNSUPPORTED, "conv wide: the input cannot be cut at channel %d of %d", in2->first, a.cred);

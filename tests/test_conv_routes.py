@@ -43,10 +43,10 @@ def test_deep_thin_volumes(cin, cout, spatial, kernel):
     assert padded == kernel and _kernel(1, cout, cin, (d + 2, h, w), "bwd-data", (0, 1, 1)) == padded
 
 
-@pytest.mark.parametrize("cin,cout", [(64, 128), (64, 192), (64, 256), (64, 512), (64, 64), (128, 128), (256, 128), (512, 256)])
+@pytest.mark.parametrize("cin,cout", [(64, 128), (64, 160), (64, 192), (64, 256), (64, 512), (64, 64), (128, 64), (128, 128), (256, 128), (512, 256)])
 def test_slab_and_padded_volume_add_in_one_order(cin, cout):
-    """Both forms of a depth shard's convolution, and of its data gradient, are the small-volume kernel's (four partial sums to a
-    voxel) or neither is: bits must not depend on the form.  The other kernels add in one chain."""
+    """Both forms of a depth shard's convolution, and of its data gradient, are one kernel's: bits must not depend on the form, and each
+    kernel adds in an order of its own."""
     rng = random.Random(cin + cout)
     shapes = [(27, 61, 33), (47, 37, 36), (39, 45, 35), (9, 27, 50), (17, 36, 35), (33, 57, 50)]
     shapes += [tuple(round(4 * 16 ** rng.random()) for _ in range(3)) for _ in range(400)]
@@ -54,7 +54,7 @@ def test_slab_and_padded_volume_add_in_one_order(cin, cout):
         for direction in ("fwd", "bwd-data"):
             padded = _kernel(1, cin, cout, (d, h, w), direction)
             slab = _kernel(1, cin, cout, (d + 2, h, w), direction, (0, 1, 1))
-            assert (padded == "split") == (slab == "split"), (direction, (d, h, w), padded, slab)
+            assert padded == slab, (direction, (d, h, w), padded, slab)
 
 
 @pytest.mark.parametrize("cin,cout,spatial,forward,gradient", [
@@ -82,7 +82,6 @@ def test_launch_times_take_no_partial_sums_away(cin, cout, spatial, forward, gra
     (256, 256, (24, 20, 28), 240),     # bricks of 2 x 4 x 8; 210 of 4 x 4 x 4
     (512, 512, (12, 10, 14), 36),      # 30 of 2 x 2 x 16
     (64, 64, (55, 28, 41), 196),       # 336 of another brick
-    (128, 64, (33, 57, 50), 270),      # the wide kernel's; 504 bricks
 ])
 def test_groupnorm_records_do_not_go_by_times(cin, cout, spatial, records):
     """Records are sums of a launch's bricks: what a network computes behind them has the bits it had before launch times chose bricks."""

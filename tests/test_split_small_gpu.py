@@ -100,6 +100,16 @@ def test_lines_that_the_times_draw(cin, cout, spatial, fwd, dgrad):
             assert torch.equal(got, from_slab)
 
 
+@pytest.mark.parametrize("n,cin,cout,spatial", [(1, 64, 64, (9, 27, 50)), (1, 64, 128, (14, 13, 6)), (1, 512, 512, (9, 9, 6)), (1, 256, 256, (11, 4, 9)),
+                                                (1, 128, 64, (33, 57, 50)), (1, 64, 64, (55, 28, 41)), (1, 512, 512, (12, 10, 14)), (2, 128, 64, (19, 30, 35)),
+                                                (1, 32, 32, (11, 75, 97)), (2, 32, 64, (9, 21, 75))])
+def test_statistics_change_no_bit(n, cin, cout, spatial):
+    """The result is the same bits with GroupNorm records and without, whichever launches estimated times choose for either."""
+    x, _, w = _operands(n, cin, cout, spatial, torch.bfloat16)
+    y = sa.conv3d_forward(x, w, None, 1, 1, gn_groups=8)
+    assert hasattr(y, "_sfh_gn_partials") and torch.equal(y, sa.conv3d_forward(x, w, None, 1, 1))
+
+
 @pytest.mark.parametrize("n,cin,cout,spatial", [(1, 128, 256, (8, 8, 8)), (1, 128, 128, (4, 6, 20)), (2, 128, 128, (5, 7, 9)),
                                                 (1, 256, 256, (5, 8, 14)), (1, 256, 256, (8, 4, 20)), (2, 256, 256, (7, 6, 4))])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
