@@ -244,6 +244,8 @@ def _run_conv_here(x, second, x_read, second_read, weight, bias, w, b, packs, ha
         # host time is free (under graph capture) or when asked for (PACK_WEIGHTS_ONCE).
         pf, pd = _c3.pack_weights(w, in_shape, stride, padding, dilation)
     # gn_groups: a GroupNorm of that many groups follows; the launch leaves its statistics on y where it can
+    if x_read.shape[0] > 1 and in_shape[1] == 32:
+        gn_groups = 0  # (module_groups in native.cpp: a batch's statistics stay with the pass that reads it)
     if second is None:
         y = _c3.conv3d_forward(x_read, w, b, stride, padding, dilation, 1, packed_weight=pf, gn_groups=gn_groups, _checked=True)
     else:

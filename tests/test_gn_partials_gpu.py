@@ -19,6 +19,7 @@ import torch.nn.functional as F
 import scaffold_amd as sa
 from oracle import oracle as orc
 from scaffold_amd import conv3d as c3
+from scaffold_amd.modules import conv_then_norm
 from scaffold_amd.unet import DoubleConv
 
 pytestmark = pytest.mark.gpu
@@ -154,6 +155,22 @@ def test_samples_walked_apart(device, n, cout, spatial, groups):
     for i in range(n):
         assert torch.equal(y[i:i + 1], sa.conv3d_forward(x[i:i + 1].contiguous(memory_format=CL), w, None, 1, 1, 1))
     check_records(y, groups, y._sfh_gn_partials)
+
+
+@pytest.mark.parametrize("n,cin,cout,spatial", [(2, 32, 32, (6, 44, 60)), (3, 32, 64, (9, 21, 75)), (1, 32, 32, (6, 44, 60)), (2, 64, 64, (6, 20, 24))])
+def test_modules_take_a_batch_of_32_channels_from_the_statistics_pass(device, n, cin, cout, spatial):
+    """The operator leaves records of its own for every sample there; a network's normalisation keeps the pass's bits."""
+    conv = sa.FastConv3d(cin, cout, 3, padding=1, bias=False).to(device, torch.bfloat16).to(memory_format=CL)
+    norm = sa.FastGroupNorm(8, cout, activation="relu").to(device, torch.bfloat16)
+    conv.gn_groups = 8
+    x = torch.randn(n, cin, *spatial, device=device).to(torch.bfloat16).contiguous(memory_format=CL)
+    with torch.no_grad():
+        left = sa.conv3d_forward(x, conv.weight, None, 1, 1, 1, gn_groups=8)
+        assert hasattr(left, "_sfh_gn_partials")
+        y = conv(x)
+        assert hasattr(y, "_sfh_gn_partials") == (n == 1 or cin != 32) and torch.equal(y, left)
+        want = norm(y.clone(memory_format=torch.preserve_format) if n > 1 and cin == 32 else y)
+        assert torch.equal(conv_then_norm(conv, norm, x), want)
 
 
 @pytest.mark.parametrize("relu", [False, True])
