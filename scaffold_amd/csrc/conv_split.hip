@@ -57,13 +57,13 @@ struct Brick {
 
 // R: chunks per round. PAIR: the input is two tensors whose channels follow each other (the first `c_first` in x, the
 // rest in x1). Independently, a non-null y1 splits the OUTPUT the same way. APART: the reduction is two rounds, and the first one's sums are
-// set aside (split_rule). They want 32 registers more: one workgroup to a CU, which the brick's LDS leaves room for anyway (with two 11 to 17 registers were
+// set aside (split_rule). chunk_stride: 1, a round's slots are R chunks that follow each other; more, a slot's rounds are that many that do. They want 32 registers more: one workgroup to a CU, which the brick's LDS leaves room for anyway (with two 11 to 17 registers were
 // spilled and every other launch of one block took 0.5 us longer).
 template <typename T, typename S, int R, int NSUB, bool PAIR, bool APART = false>
 __global__ void __launch_bounds__(256, APART ? 1 : 2)
 conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ wp, const T* __restrict__ bias, T* __restrict__ y,
                   int tiles_d, int tiles_h, int tiles_w, int nblocks, uint32_t total, GnPartialOut gn, const T* __restrict__ x1,
-                  T* __restrict__ y1, int c_first) {
+                  T* __restrict__ y1, int c_first, int chunk_stride) {
   using B = Brick<S, NSUB>;
   constexpr int TD = S::TD, TH = S::TH, TW = S::TW, BH = S::BH, BW = S::BW;
   constexpr int PLANE = B::PLANE, SLOT = B::SLOT;
@@ -116,7 +116,8 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
 
   for (int c0 = 0; c0 < ncc; c0 += R) {
     // The wavefront's first weight fragments are requested before the bricks are staged: they depend on nothing in LDS.
-    const T* wcc = wp + ((int64_t)(nb * NSUB) * ncc + c0 + slot) * (NIT * FRAG) + khalf * FRAG + lane * 8;
+    const int first_chunk = chunk_stride == 1 ? c0 : c0 / R;  // slot 0's
+    const T* wcc = wp + ((int64_t)(nb * NSUB) * ncc + first_chunk + slot * chunk_stride) * (NIT * FRAG) + khalf * FRAG + lane * 8;
     uint4 wq[NITS][NSUB];  // fully unrolled: every slot is its own register set, live for WDEPTH iterations
 #pragma unroll
     for (int k = 0; k < WDEPTH; ++k)
@@ -130,7 +131,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
       for (int u = 0; u < ITERS; ++u) {
         const int p = u * 256 + tid;
         const int q = p % (4 * R), vox = p / (4 * R);
-        const int cc = c0 + (q >> 2), piece = q & 3;
+        const int cc = first_chunk + (q >> 2) * chunk_stride, piece = q & 3;
         const int bw = vox % BW, bh = (vox / BW) % BH, bd = vox / (BW * BH);
         const int id = id0 + bd, ih = ih0 + bh, iw = iw0 + bw;
         const bool in = p < PIECES && (unsigned)id < (unsigned)a.id && (unsigned)ih < (unsigned)a.ih && (unsigned)iw < (unsigned)a.iw;
@@ -334,25 +335,28 @@ int64_t split_tiles(const MfmaConvArgs& a) { return tiles_of(a, split_shape(a));
 // 256 -> 256 at 10x16x16 16.5 / 22.0 -> 19.2 / 22.2, at 16^3 17.6 -> 19.6 (each CU fetches the same weights and stages twice the bricks).
 int split_blocks(int64_t tiles, int cout) { return tiles * (cout / (32 * kBlocks)) <= kComputeUnits / 2 ? 1 : kBlocks; }
 
-// Whether a problem is this kernel's, and whether its two rounds' sums stay apart: see mfma_conv_split_applies.
-struct SplitRule { bool use, apart; };
+// Whether a problem is this kernel's, whether its two rounds' sums stay apart, and whether a wavefront takes chunks that follow each other, as a
+// slice does: see mfma_conv_split_applies.
+struct SplitRule { bool use, apart, quarters; };
 SplitRule split_rule(const MfmaConvArgs& a, bool records);
-constexpr int kApartChunks = 8;
+constexpr int kApartChunks = 8, kQuartersChunks = 8;  // (exactly, at least)
 
 // A launch: its brick (0: 2x4x8, 1: 4x4x4, 2: 2x2x16), their number and the channel blocks of a workgroup. GroupNorm records are sums of bricks: a
 // launch that leaves them keeps 2x4x8, so that the statistics behind it, and with them all that a network computes from there on, do not hang on
 // an estimate of times (us it costs: where a brick less saves a round, 512 -> 512 at 12x10x14, 39 -> 50; elsewhere 1 to 5 %). Rounds apart are
 // few pairs: one block and the smallest halo.
-struct SplitPlan { bool apart; int shape, blocks; int64_t tiles; };
+struct SplitPlan { bool apart; int chunk_stride, shape, blocks; int64_t tiles; };
 SplitPlan split_plan(const MfmaConvArgs& a, bool records) {
-  const bool apart = a.cred == kApartChunks * kChunk && split_rule(a, records).apart;
+  const int chunks = a.cred / kChunk;
+  const SplitRule rule = chunks >= kQuartersChunks && chunks % 4 == 0 ? split_rule(a, records) : SplitRule{true, false, false};
+  const bool apart = rule.apart;
   const int shape = records ? 0 : apart ? 1 : split_shape(a);
   const int64_t tiles = tiles_of(a, shape);
-  return SplitPlan{apart, shape, apart ? 1 : split_blocks(tiles, a.cout), tiles};
+  return SplitPlan{apart, rule.quarters ? chunks / 4 : 1, shape, apart ? 1 : split_blocks(tiles, a.cout), tiles};
 }
 
 template <typename T, typename S, int R, int NSUB, bool PAIR, bool APART = false>
-int launch_brick(const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
+int launch_brick(int chunk_stride, const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                  const GnPartialOut& gn, const void* x1, void* y1, int first) {
   const int tiles_d = (int)cdiv(a.od, S::TD), tiles_h = (int)cdiv(a.oh, S::TH), tiles_w = (int)cdiv(a.ow, S::TW);
   const int nblocks = a.cout / (32 * NSUB);
@@ -360,17 +364,17 @@ int launch_brick(const MfmaConvArgs& a, const void* x, const void* packed, const
   if (total == 0) return SFH_OK;
   if (total > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv split: %lld workgroups exceed the grid limit", (long long)total);
   hipLaunchKernelGGL((conv_split_kernel<T, S, R, NSUB, PAIR, APART>), dim3((unsigned)total), dim3(256), 0, st, a, (const T*)x, (const T*)packed,
-                     (const T*)bias, (T*)y, tiles_d, tiles_h, tiles_w, nblocks, (uint32_t)total, gn, (const T*)x1, (T*)y1, first);
+                     (const T*)bias, (T*)y, tiles_d, tiles_h, tiles_w, nblocks, (uint32_t)total, gn, (const T*)x1, (T*)y1, first, chunk_stride);
   return check_launch("conv_split_kernel");
 }
 
 template <typename T, int R, int NSUB, bool PAIR>
-int launch_split(int shape, const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
+int launch_split(const SplitPlan& p, const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                  const GnPartialOut& gn, const void* x1, void* y1, int first) {
-  switch (shape) {
-    case 1: return launch_brick<T, Cube, R, NSUB, PAIR>(a, x, packed, bias, y, st, gn, x1, y1, first);
-    case 2: return launch_brick<T, Rows, R, NSUB, PAIR>(a, x, packed, bias, y, st, gn, x1, y1, first);
-    default: return launch_brick<T, Flat, R, NSUB, PAIR>(a, x, packed, bias, y, st, gn, x1, y1, first);
+  switch (p.shape) {
+    case 1: return launch_brick<T, Cube, R, NSUB, PAIR>(p.chunk_stride, a, x, packed, bias, y, st, gn, x1, y1, first);
+    case 2: return launch_brick<T, Rows, R, NSUB, PAIR>(p.chunk_stride, a, x, packed, bias, y, st, gn, x1, y1, first);
+    default: return launch_brick<T, Flat, R, NSUB, PAIR>(p.chunk_stride, a, x, packed, bias, y, st, gn, x1, y1, first);
   }
 }
 
@@ -379,13 +383,13 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
                        const GnPartialOut& gn, const void* x1, void* y1, int first) {
   const SplitPlan p = split_plan(a, gn.part != nullptr);
   const bool four = (a.cred / kChunk) % 4 == 0;
-  if (p.apart) return x1 != nullptr ? launch_brick<T, Cube, 4, 1, true, true>(a, x, packed, bias, y, st, gn, x1, y1, first)
-                                    : launch_brick<T, Cube, 4, 1, false, true>(a, x, packed, bias, y, st, gn, x1, y1, first);
+  if (p.apart) return x1 != nullptr ? launch_brick<T, Cube, 4, 1, true, true>(1, a, x, packed, bias, y, st, gn, x1, y1, first)
+                                    : launch_brick<T, Cube, 4, 1, false, true>(1, a, x, packed, bias, y, st, gn, x1, y1, first);
 #define SFH_SPLIT(NSUB)                                                                                         \
-  x1 != nullptr ? (four ? launch_split<T, 4, NSUB, true>(p.shape, a, x, packed, bias, y, st, gn, x1, y1, first)   \
-                        : launch_split<T, 2, NSUB, true>(p.shape, a, x, packed, bias, y, st, gn, x1, y1, first))  \
-                : (four ? launch_split<T, 4, NSUB, false>(p.shape, a, x, packed, bias, y, st, gn, x1, y1, first)  \
-                        : launch_split<T, 2, NSUB, false>(p.shape, a, x, packed, bias, y, st, gn, x1, y1, first))
+  x1 != nullptr ? (four ? launch_split<T, 4, NSUB, true>(p, a, x, packed, bias, y, st, gn, x1, y1, first)   \
+                        : launch_split<T, 2, NSUB, true>(p, a, x, packed, bias, y, st, gn, x1, y1, first))  \
+                : (four ? launch_split<T, 4, NSUB, false>(p, a, x, packed, bias, y, st, gn, x1, y1, first)  \
+                        : launch_split<T, 2, NSUB, false>(p, a, x, packed, bias, y, st, gn, x1, y1, first))
   return p.blocks == 1 ? SFH_SPLIT(1) : SFH_SPLIT(2);
 #undef SFH_SPLIT
 }
@@ -418,11 +422,11 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
 // are kept (below), it comes here by the fewer pairs too.
 // The times take nothing away from this kernel: its four partial sums to a voxel are nearer the 64-bit result than the bricks' one chain (fp16
 // results of 64 to 512 channels that are not the rounded 64-bit ones: 1.5e-3 here, 1.9e-3 in bricks, 28 problems of both directions), so 256 -> 256 at 32^3 stays at
-// 109 us though bricks take 102. Eight slices are nearer still (1.35e-3, 1.75e-3 here with four sums; four: level). So what the bricks would sum in
-// eight comes here only where a slice is one chunk (256 reduction channels): the two rounds' sums stay apart and meet in the slices' order.
-// Those have the slices' bits, and so have four chunks in the place of four slices (a launch that leaves GroupNorm records stays with the
-// slices, whose records are sums of other voxels). us, slices and their sum / four sums / eight sums: 256 -> 256 at 14x6x4 10.2 / 10.8 / 11.9, at 5x8x14
-// 11.6 / 11.4 / 12.5, at 8x4x20 12.3 / 11.1 / 12.2: no gain there, but no launch and no workspace beside it.
+// 109 us though bricks take 102. Eight slices are nearer still (1.35e-3, 1.75e-3 here with four sums; four: level).
+// What the bricks would sum in four slices comes here with the slices' bits: a wavefront takes a quarter of the chunks in their order. Eight slices of one
+// chunk (256 reduction channels) do so as well, the two rounds' sums kept apart until the end, and no other eight. A launch that leaves
+// GroupNorm records stays with the slices, whose records are sums of other voxels. us, slices and their sum / four sums / eight sums, 256 -> 256 at
+// 14x6x4 10.2 / 10.8 / 11.9, at 5x8x14 11.6 / 11.4 / 12.5, at 8x4x20 12.3 / 11.1 / 12.2: no gain there, but no launch and no workspace beside it.
 // The data gradient of a depth shard's slab (D + 2 planes from D) and of the padded volume (D from D) must come from the same
 // kernel, or a shard and the whole volume would disagree in the last bit: the depth counted is the smaller of the two.
 constexpr int kSplitMaxPlane = 32 * 32, kSplitMinPerDepth = 24, kSplitFewPerDepth = 32, kSplitFewMaxChunks = 16;
@@ -435,8 +439,8 @@ int64_t split_line_few(int chunks, int cout) { return chunks <= 4 && cout >= 128
 
 namespace {
 SplitRule split_rule(const MfmaConvArgs& a, bool records) {
-  if (a.kd != 3 || a.kh != 3 || a.kw != 3) return {false, false};
-  if (a.cred < 2 * kChunk || a.cred % (2 * kChunk) != 0 || a.cout % (32 * kBlocks) != 0) return {false, false};
+  if (a.kd != 3 || a.kh != 3 || a.kw != 3) return {};
+  if (a.cred < 2 * kChunk || a.cred % (2 * kChunk) != 0 || a.cout % (32 * kBlocks) != 0) return {};
   const int chunks = a.cred / kChunk, pair = a.cout / (32 * kBlocks);
   MfmaConvArgs core = a;
   core.od = a.id < a.od ? a.id : a.od;
@@ -444,16 +448,17 @@ SplitRule split_rule(const MfmaConvArgs& a, bool records) {
   const int64_t pairs = per_depth * cdiv(core.od, Flat::TD), rounds = cdiv(pairs, kComputeUnits);
   const bool kept = a.gradient != 0;  // the order of sums does not go by the times
   auto sooner = [&](int percent) { return 100 * split_time(split_tiles(core) * pair, chunks) < percent * mfma_conv_brick_time(core); };
-  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return {!kept && pairs > kSplitBigPlanePairs && sooner(72), false};
+  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return {!kept && pairs > kSplitBigPlanePairs && sooner(72), false, false};
   const bool few = per_depth <= kSplitFewPerDepth && chunks >= kSplitFewMaxChunks;
-  if (!few && per_depth >= kSplitMinPerDepth) return {true, false};
+  if (!few && per_depth >= kSplitMinPerDepth) return {true, false, false};
   if (pairs >= split_line(chunks))
-    return {rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || (!kept && sooner(110)), false};
+    return {rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || (!kept && sooner(110)), false, false};
   const int slices = mfma_conv_brick_slices(core);
-  const bool apart = slices > 4, same_bits = slices == chunks && chunks % 4 == 0;  // (two chunks are cut in halves of 16 channels here)
-  if (same_bits ? records : apart || kept) return {false, false};
+  const bool eight = slices == 8 && chunks == kApartChunks, four = slices == 4 && chunks % 4 == 0;  // (two chunks are cut in halves of 16 channels here)
+  const bool same_bits = (eight || four) && (a.gradient || core.od == a.od || mfma_conv_brick_slices(a) == slices);
+  if (same_bits ? records : slices > 4 || kept) return {};
   const bool enough = pairs >= split_line_few(chunks, a.cout) && (same_bits || sooner(72));
-  return {enough || (chunks >= kSplitFewMaxChunks && sooner(70)), apart};
+  return {enough || (chunks >= kSplitFewMaxChunks && sooner(70)), same_bits && eight, same_bits && four && chunks >= kQuartersChunks};
 }
 }  // namespace
 

@@ -65,7 +65,8 @@ def test_slab_and_padded_volume_add_in_one_order(cin, cout):
     (512, 512, (5, 8, 8), "brick", "brick"),     # eight slices of two chunks each
     (256, 256, (5, 8, 14), "split", "split"),    # eight of one: as many partial sums there
     (128, 128, (9, 12, 8), "split", "split"),    # four of one
-    (256, 256, (11, 4, 9), "split", "brick"),    # four of two
+    (256, 256, (11, 4, 9), "split", "split"),    # four of two
+    (192, 256, (6, 15, 7), "split", "brick"),    # four of one and of two: the small-volume kernel cannot
     (64, 128, (14, 13, 6), "split", "brick"),
     (128, 64, (14, 13, 6), "brick", "brick"),    # the gradient's two slices are one chunk each, which the small-volume kernel cuts in two
     (64, 64, (9, 27, 50), "split", "brick"),     # a plane past 32 x 32

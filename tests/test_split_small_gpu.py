@@ -77,7 +77,7 @@ def _conv64(x, w):
     (512, 512, (9, 9, 6), "split", "brick"),     # a long reduction by the times
     (256, 256, (5, 8, 14), "split", "split"),    # in the place of eight slices: two rounds, their sums apart
     (256, 256, (3, 16, 12), "split", "split"),   # 72 pairs
-    (256, 256, (11, 4, 9), "split", "brick"),    # in the place of four: one chain a wavefront
+    (256, 256, (11, 4, 9), "split", "split"),    # in the place of four: one chain a wavefront
     (128, 64, (33, 57, 50), "brick", "brick"),   # bricks in the wide kernel's place by the times
     (128, 64, (31, 61, 65), "wide", "brick"),
 ])
@@ -102,19 +102,22 @@ def test_lines_that_the_times_draw(cin, cout, spatial, fwd, dgrad):
 
 @pytest.mark.parametrize("n,cin,cout,spatial", [(1, 64, 64, (9, 27, 50)), (1, 64, 128, (14, 13, 6)), (1, 512, 512, (9, 9, 6)), (1, 256, 256, (11, 4, 9)),
                                                 (1, 128, 64, (33, 57, 50)), (1, 64, 64, (55, 28, 41)), (1, 512, 512, (12, 10, 14)), (2, 128, 64, (19, 30, 35)),
-                                                (1, 32, 32, (11, 75, 97)), (2, 32, 64, (9, 21, 75))])
-def test_statistics_change_no_bit(n, cin, cout, spatial):
+                                                (1, 32, 32, (11, 75, 97)), (2, 32, 64, (9, 21, 75)), (2, 128, 128, (11, 2, 6))])
+@pytest.mark.parametrize("depth_padding", [1, 2])
+def test_statistics_change_no_bit(n, cin, cout, spatial, depth_padding):
     """The result is the same bits with GroupNorm records and without, whichever launches estimated times choose for either."""
     x, _, w = _operands(n, cin, cout, spatial, torch.bfloat16)
-    y = sa.conv3d_forward(x, w, None, 1, 1, gn_groups=8)
-    assert hasattr(y, "_sfh_gn_partials") and torch.equal(y, sa.conv3d_forward(x, w, None, 1, 1))
+    padding = (depth_padding, 1, 1)
+    y = sa.conv3d_forward(x, w, None, 1, padding, gn_groups=8)
+    assert hasattr(y, "_sfh_gn_partials") and torch.equal(y, sa.conv3d_forward(x, w, None, 1, padding))
 
 
 @pytest.mark.parametrize("n,cin,cout,spatial", [(1, 128, 256, (8, 8, 8)), (1, 128, 128, (4, 6, 20)), (2, 128, 128, (5, 7, 9)),
-                                                (1, 256, 256, (5, 8, 14)), (1, 256, 256, (8, 4, 20)), (2, 256, 256, (7, 6, 4))])
+                                                (1, 256, 256, (5, 8, 14)), (1, 256, 256, (8, 4, 20)), (2, 256, 256, (7, 6, 4)),
+                                                (1, 256, 256, (11, 4, 9)), (1, 256, 512, (6, 7, 5))])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_slices_and_their_bits(n, cin, cout, spatial, dtype):
-    """A chunk to a slice: the launch that leaves GroupNorm records is the bricks' in slices, the one without the small-volume kernel's,
+    """A slice to a wavefront, or to a wavefront and round: the launch that leaves GroupNorm records is the bricks' in slices, the one without the small-volume kernel's,
     whose wavefronts (and rounds) add in the slices' order.  Against float64 as well."""
     x, _, w = _operands(n, cin, cout, spatial, dtype)
     assert c3.launch_geometry(x.shape, w.shape, 1, 1, 1, dtype, "fwd")["kernel"] == "split"
