@@ -56,17 +56,23 @@ struct Brick {
 };
 
 // R: chunks per round. PAIR: the input is two tensors whose channels follow each other (the first `c_first` in x, the
-// rest in x1). Independently, a non-null y1 splits the OUTPUT the same way. APART: the reduction is two rounds, and the first one's sums are
-// set aside (split_rule). chunk_stride: 1, a round's slots are R chunks that follow each other; more, a slot's rounds are that many that do. They want 32 registers more: one workgroup to a CU, which the brick's LDS leaves room for anyway (with two 11 to 17 registers were
-// spilled and every other launch of one block took 0.5 us longer).
-template <typename T, typename S, int R, int NSUB, bool PAIR, bool APART = false>
-__global__ void __launch_bounds__(256, APART ? 1 : 2)
+// rest in x1). Independently, a non-null y1 splits the OUTPUT the same way. chunk_stride: 1, a round's slots are R chunks that follow each other;
+// more, a slot's rounds are that many that do. FORM, of launches that add as the bricks' slices do (split_rule):
+//   kApart   the reduction is two rounds, and the first one's sums are set aside. They want 32 registers more: one workgroup to a CU, which the
+//            brick's LDS leaves room for anyway (with two 11 to 17 registers were spilled and every other launch of one block took 0.5 us longer).
+//   kHalves  (R = 2) a wavefront has one of the two voxel halves and all 32 channels of its chunks, in place of both halves and 16.
+enum SplitForm { kOrdinary, kApart, kHalves };
+template <typename T, typename S, int R, int NSUB, bool PAIR, SplitForm FORM = kOrdinary>
+__global__ void __launch_bounds__(256, FORM == kApart ? 1 : 2)
 conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ wp, const T* __restrict__ bias, T* __restrict__ y,
                   int tiles_d, int tiles_h, int tiles_w, int nblocks, uint32_t total, GnPartialOut gn, const T* __restrict__ x1,
                   T* __restrict__ y1, int c_first, int chunk_stride) {
   using B = Brick<S, NSUB>;
   constexpr int TD = S::TD, TH = S::TH, TW = S::TW, BH = S::BH, BW = S::BW;
   constexpr int PLANE = B::PLANE, SLOT = B::SLOT;
+  constexpr bool APART = FORM == kApart, HALVES = FORM == kHalves, WHOLE = R == 4 || HALVES;  // WHOLE: both k-steps of a tap
+  static_assert(FORM == kOrdinary || (NSUB == 1 && R == (APART ? 4 : 2)), "one block");
+  constexpr int MSW = HALVES ? 1 : MS;  // voxel halves of a wavefront
   constexpr int ROUNDS = APART ? 2 : 1;
   constexpr int RED_BYTES = ROUNDS * MS * NSUB * 3 * 4096;  // every block from the three wavefronts that do not own it
   constexpr int LDS = R * SLOT > RED_BYTES ? R * SLOT : RED_BYTES;
@@ -83,23 +89,22 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   const int n = t / tiles_d;
   const int od0 = td_i * TD, oh0 = th_i * TH, ow0 = tw_i * TW;
 
-  // This wavefront's share of a round: chunk slot `slot`; with R = 2 also one of the two k-steps of every tap.
+  // This wavefront's share of a round: chunk slot `slot`; with R = 2 also one of the two k-steps of every tap, or one of the voxel halves.
   const int slot = R == 4 ? wave : wave >> 1;
-  const int khalf = R == 4 ? 0 : wave & 1;
-  constexpr int NITS = R == 4 ? NIT : TAPS;  // iterations of a wavefront per round
-  constexpr int WSTEP = R == 4 ? FRAG : 2 * FRAG;
-  int abase[MS];  // LDS byte address of the lane's voxel of block row ms at tap (0, 0, 0), in its k-half plane
+  const int khalf = WHOLE ? 0 : wave & 1, half = HALVES ? wave & 1 : 0;
+  constexpr int NITS = WHOLE ? NIT : TAPS;  // iterations of a wavefront per round
+  constexpr int WSTEP = WHOLE ? FRAG : 2 * FRAG;
+  int abase[MSW];  // LDS byte address of the lane's voxel of block row ms at tap (0, 0, 0), in its k-half plane
 #pragma unroll
-  for (int ms = 0; ms < MS; ++ms) {
-    const int v = ms * 32 + j, tw = v % TW, th = v / TW % TH, td = v / (TW * TH);
+  for (int ms = 0; ms < MSW; ++ms) {
+    const int v = (half + ms) * 32 + j, tw = v % TW, th = v / TW % TH, td = v / (TW * TH);
     abase[ms] = slot * SLOT + (kg + 2 * khalf) * PLANE + (td * BH + th) * B::ROW + tw * 16;
   }
-  auto a_off = [](int k) constexpr { return R == 4 ? B::tap_off(k / 2) + (k % 2) * 2 * PLANE : B::tap_off(k); };
+  auto a_off = [](int k) constexpr { return WHOLE ? B::tap_off(k / 2) + (k % 2) * 2 * PLANE : B::tap_off(k); };
 
-  static_assert(!APART || NSUB == 1, "one block's sums set aside");
-  f32x16_t acc[MS][NSUB], first[MS];  // first: the first round's sums, where they are chains apart
+  f32x16_t acc[MSW][NSUB], first[MSW];  // first: the first round's sums, where they are chains apart
 #pragma unroll
-  for (int ms = 0; ms < MS; ++ms)
+  for (int ms = 0; ms < MSW; ++ms)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
 #pragma unroll
@@ -116,8 +121,9 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
 
   for (int c0 = 0; c0 < ncc; c0 += R) {
     // The wavefront's first weight fragments are requested before the bricks are staged: they depend on nothing in LDS.
-    const int first_chunk = chunk_stride == 1 ? c0 : c0 / R;  // slot 0's
-    const T* wcc = wp + ((int64_t)(nb * NSUB) * ncc + first_chunk + slot * chunk_stride) * (NIT * FRAG) + khalf * FRAG + lane * 8;
+    const int stride = NSUB == 1 ? chunk_stride : 1;  // (two blocks have no registers for it)
+    const int first_chunk = stride == 1 ? c0 : c0 / R;  // slot 0's
+    const T* wcc = wp + ((int64_t)(nb * NSUB) * ncc + first_chunk + slot * stride) * (NIT * FRAG) + khalf * FRAG + lane * 8;
     uint4 wq[NITS][NSUB];  // fully unrolled: every slot is its own register set, live for WDEPTH iterations
 #pragma unroll
     for (int k = 0; k < WDEPTH; ++k)
@@ -131,7 +137,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
       for (int u = 0; u < ITERS; ++u) {
         const int p = u * 256 + tid;
         const int q = p % (4 * R), vox = p / (4 * R);
-        const int cc = first_chunk + (q >> 2) * chunk_stride, piece = q & 3;
+        const int cc = first_chunk + (q >> 2) * stride, piece = q & 3;
         const int bw = vox % BW, bh = (vox / BW) % BH, bd = vox / (BW * BH);
         const int id = id0 + bd, ih = ih0 + bh, iw = iw0 + bw;
         const bool in = p < PIECES && (unsigned)id < (unsigned)a.id && (unsigned)ih < (unsigned)a.ih && (unsigned)iw < (unsigned)a.iw;
@@ -157,14 +163,14 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
 
     // Software pipeline over the wavefront's iterations: the weight fragments of iteration k + WDEPTH and the
     // activation fragments of iteration k + 1 are requested between the MFMAs of iteration k, one behind each.
-    uint4 aq[2][MS];
+    uint4 aq[2][MSW];
 #pragma unroll
-    for (int ms = 0; ms < MS; ++ms) aq[0][ms] = *reinterpret_cast<const uint4*>(lds + abase[ms] + a_off(0));
+    for (int ms = 0; ms < MSW; ++ms) aq[0][ms] = *reinterpret_cast<const uint4*>(lds + abase[ms] + a_off(0));
 #pragma unroll
     for (int k = 0; k < NITS; ++k) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int m = 0; m < MS * NSUB; ++m) {
+      for (int m = 0; m < MSW * NSUB; ++m) {
         const int ms = m / NSUB, ns = m % NSUB;
         acc[ms][ns] = Mma32<T>::run(wq[k][ns], aq[k & 1][ms], acc[ms][ns]);
         __builtin_amdgcn_sched_barrier(0);
@@ -179,7 +185,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
     if constexpr (APART) {
       if (c0 == 0) {
 #pragma unroll
-        for (int ms = 0; ms < MS; ++ms)
+        for (int ms = 0; ms < MSW; ++ms)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             first[ms][r] = acc[ms][0][r];
@@ -194,22 +200,44 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   __syncthreads();  // the bricks are not read any more
   float4* red = reinterpret_cast<float4*>(lds);
   auto mine_of = [&](int round, int u) -> const f32x16_t& { return APART && round == 0 ? first[u / NSUB] : acc[u / NSUB][u % NSUB]; };
+  auto send = [&](int place, const f32x16_t& v) {
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) red[(place * 4 + r4) * 64 + lane] = make_float4(v[4 * r4], v[4 * r4 + 1], v[4 * r4 + 2], v[4 * r4 + 3]);
+  };
+  auto receive = [&](int place) {
+    f32x16_t v;
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+      const float4 e = red[(place * 4 + r4) * 64 + lane];
+      v[4 * r4] = e.x; v[4 * r4 + 1] = e.y; v[4 * r4 + 2] = e.z; v[4 * r4 + 3] = e.w;
+    }
+    return v;
+  };
+  if constexpr (HALVES) {
+    send(half * 2 + slot, acc[0][0]);
+  } else {
 #pragma unroll
   for (int round = 0; round < ROUNDS; ++round)
 #pragma unroll
     for (int u = 0; u < MS * NSUB; ++u) {
       if (u != wave) {
         const int from = wave < u ? wave : wave - 1;  // this wavefront's place among block u's three senders
-        const f32x16_t& v = mine_of(round, u);
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4)
-          red[(((round * MS * NSUB + u) * 3 + from) * 4 + r4) * 64 + lane] = make_float4(v[4 * r4], v[4 * r4 + 1], v[4 * r4 + 2], v[4 * r4 + 3]);
+        send((round * MS * NSUB + u) * 3 + from, mine_of(round, u));
       }
     }
+  }
   __syncthreads();
   f32x16_t tot;
 #pragma unroll
   for (int r = 0; r < 16; ++r) tot[r] = 0.f;
+  if constexpr (HALVES) {
+    if (wave < MS) {
+      tot = receive(wave * 2);
+      const f32x16_t second = receive(wave * 2 + 1);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) tot[r] += second[r];
+    }
+  } else
 #pragma unroll
   for (int u = 0; u < MS * NSUB; ++u) {
     if (u == wave) {
@@ -222,12 +250,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
           if (src == u) {
             part = mine_of(round, u);
           } else {
-            const int from = src < u ? src : src - 1;
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-              const float4 e = red[(((round * MS * NSUB + u) * 3 + from) * 4 + r4) * 64 + lane];
-              part[4 * r4] = e.x; part[4 * r4 + 1] = e.y; part[4 * r4 + 2] = e.z; part[4 * r4 + 3] = e.w;
-            }
+            part = receive((round * MS * NSUB + u) * 3 + (src < u ? src : src - 1));
           }
           if (round == 0 && src == 0) tot = part;
           else
@@ -335,27 +358,24 @@ int64_t split_tiles(const MfmaConvArgs& a) { return tiles_of(a, split_shape(a));
 // 256 -> 256 at 10x16x16 16.5 / 22.0 -> 19.2 / 22.2, at 16^3 17.6 -> 19.6 (each CU fetches the same weights and stages twice the bricks).
 int split_blocks(int64_t tiles, int cout) { return tiles * (cout / (32 * kBlocks)) <= kComputeUnits / 2 ? 1 : kBlocks; }
 
-// Whether a problem is this kernel's, whether its two rounds' sums stay apart, and whether a wavefront takes chunks that follow each other, as a
-// slice does: see mfma_conv_split_applies.
-struct SplitRule { bool use, apart, quarters; };
+// Whether a problem is this kernel's, and how many of the bricks' slices it adds like (0: in its own order): see mfma_conv_split_applies.
+struct SplitRule { bool use; int slices; };
 SplitRule split_rule(const MfmaConvArgs& a, bool records);
-constexpr int kApartChunks = 8, kQuartersChunks = 8;  // (exactly, at least)
 
 // A launch: its brick (0: 2x4x8, 1: 4x4x4, 2: 2x2x16), their number and the channel blocks of a workgroup. GroupNorm records are sums of bricks: a
 // launch that leaves them keeps 2x4x8, so that the statistics behind it, and with them all that a network computes from there on, do not hang on
-// an estimate of times (us it costs: where a brick less saves a round, 512 -> 512 at 12x10x14, 39 -> 50; elsewhere 1 to 5 %). Rounds apart are
-// few pairs: one block and the smallest halo.
-struct SplitPlan { bool apart; int chunk_stride, shape, blocks; int64_t tiles; };
+// an estimate of times (us it costs: where a brick less saves a round, 512 -> 512 at 12x10x14, 39 -> 50; elsewhere 1 to 5 %). Launches that add
+// as slices do are few pairs: one block, and where two or eight are followed the smallest halo.
+struct SplitPlan { SplitForm form; int chunk_stride, shape, blocks; int64_t tiles; };
 SplitPlan split_plan(const MfmaConvArgs& a, bool records) {
-  const int chunks = a.cred / kChunk;
-  const SplitRule rule = chunks >= kQuartersChunks && chunks % 4 == 0 ? split_rule(a, records) : SplitRule{true, false, false};
-  const bool apart = rule.apart;
-  const int shape = records ? 0 : apart ? 1 : split_shape(a);
+  const int slices = split_rule(a, records).slices;
+  const SplitForm form = slices == 8 ? kApart : slices == 2 ? kHalves : kOrdinary;
+  const int shape = records ? 0 : form != kOrdinary ? 1 : split_shape(a);
   const int64_t tiles = tiles_of(a, shape);
-  return SplitPlan{apart, rule.quarters ? chunks / 4 : 1, shape, apart ? 1 : split_blocks(tiles, a.cout), tiles};
+  return SplitPlan{form, slices == 2 || slices == 4 ? a.cred / kChunk / slices : 1, shape, slices > 0 ? 1 : split_blocks(tiles, a.cout), tiles};
 }
 
-template <typename T, typename S, int R, int NSUB, bool PAIR, bool APART = false>
+template <typename T, typename S, int R, int NSUB, bool PAIR, SplitForm FORM = kOrdinary>
 int launch_brick(int chunk_stride, const MfmaConvArgs& a, const void* x, const void* packed, const void* bias, void* y, hipStream_t st,
                  const GnPartialOut& gn, const void* x1, void* y1, int first) {
   const int tiles_d = (int)cdiv(a.od, S::TD), tiles_h = (int)cdiv(a.oh, S::TH), tiles_w = (int)cdiv(a.ow, S::TW);
@@ -363,7 +383,7 @@ int launch_brick(int chunk_stride, const MfmaConvArgs& a, const void* x, const v
   const int64_t total = (int64_t)a.n * tiles_d * tiles_h * tiles_w * nblocks;
   if (total == 0) return SFH_OK;
   if (total > 0x7fffffffLL) return fail(SFH_ERR_UNSUPPORTED, "conv split: %lld workgroups exceed the grid limit", (long long)total);
-  hipLaunchKernelGGL((conv_split_kernel<T, S, R, NSUB, PAIR, APART>), dim3((unsigned)total), dim3(256), 0, st, a, (const T*)x, (const T*)packed,
+  hipLaunchKernelGGL((conv_split_kernel<T, S, R, NSUB, PAIR, FORM>), dim3((unsigned)total), dim3(256), 0, st, a, (const T*)x, (const T*)packed,
                      (const T*)bias, (T*)y, tiles_d, tiles_h, tiles_w, nblocks, (uint32_t)total, gn, (const T*)x1, (T*)y1, first, chunk_stride);
   return check_launch("conv_split_kernel");
 }
@@ -383,8 +403,12 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
                        const GnPartialOut& gn, const void* x1, void* y1, int first) {
   const SplitPlan p = split_plan(a, gn.part != nullptr);
   const bool four = (a.cred / kChunk) % 4 == 0;
-  if (p.apart) return x1 != nullptr ? launch_brick<T, Cube, 4, 1, true, true>(1, a, x, packed, bias, y, st, gn, x1, y1, first)
-                                    : launch_brick<T, Cube, 4, 1, false, true>(1, a, x, packed, bias, y, st, gn, x1, y1, first);
+  if (p.form == kApart)
+    return x1 != nullptr ? launch_brick<T, Cube, 4, 1, true, kApart>(1, a, x, packed, bias, y, st, gn, x1, y1, first)
+                         : launch_brick<T, Cube, 4, 1, false, kApart>(1, a, x, packed, bias, y, st, gn, x1, y1, first);
+  if (p.form == kHalves)
+    return x1 != nullptr ? launch_brick<T, Cube, 2, 1, true, kHalves>(p.chunk_stride, a, x, packed, bias, y, st, gn, x1, y1, first)
+                         : launch_brick<T, Cube, 2, 1, false, kHalves>(p.chunk_stride, a, x, packed, bias, y, st, gn, x1, y1, first);
 #define SFH_SPLIT(NSUB)                                                                                         \
   x1 != nullptr ? (four ? launch_split<T, 4, NSUB, true>(p, a, x, packed, bias, y, st, gn, x1, y1, first)   \
                         : launch_split<T, 2, NSUB, true>(p, a, x, packed, bias, y, st, gn, x1, y1, first))  \
@@ -423,10 +447,14 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
 // The times take nothing away from this kernel: its four partial sums to a voxel are nearer the 64-bit result than the bricks' one chain (fp16
 // results of 64 to 512 channels that are not the rounded 64-bit ones: 1.5e-3 here, 1.9e-3 in bricks, 28 problems of both directions), so 256 -> 256 at 32^3 stays at
 // 109 us though bricks take 102. Eight slices are nearer still (1.35e-3, 1.75e-3 here with four sums; four: level).
-// What the bricks would sum in four slices comes here with the slices' bits: a wavefront takes a quarter of the chunks in their order. Eight slices of one
-// chunk (256 reduction channels) do so as well, the two rounds' sums kept apart until the end, and no other eight. A launch that leaves
-// GroupNorm records stays with the slices, whose records are sums of other voxels. us, slices and their sum / four sums / eight sums, 256 -> 256 at
-// 14x6x4 10.2 / 10.8 / 11.9, at 5x8x14 11.6 / 11.4 / 12.5, at 8x4x20 12.3 / 11.1 / 12.2: no gain there, but no launch and no workspace beside it.
+// What the bricks would sum in slices comes here with the slices' bits, so that it may in both directions: of four a wavefront takes one's chunks in
+// their order; of two, up to 128 channels, a voxel half of one's; eight of one chunk (256 channels) are two rounds whose sums meet at the end. Where none
+// of these is, eight slices stay (nearer the exact value still, 1.35e-3, 1.75e-3 here with four sums), and two or four become this kernel's sums where
+// a quarter of the time is gained. A launch that leaves GroupNorm records stays with the slices, whose records are sums of other voxels.
+// us, slices and their sum -> here, with their bits: 64 -> 128 at 14x13x6 9.3 -> 6.0, 64 -> 512 at 7x3x6 8.8 -> 6.0, 128 -> 64 (data gradient) at 14x13x6 9.4 -> 6.0,
+// three samples of 128 -> 256 at 10x3x6 12.8 -> 8.9, 128 -> 512 at 3x4x9 9.0 -> 7.0, 256 -> 256 at 11x4x9 12.6 -> 10.3, at 8x4x20 (eight) 12.0 -> 11.4, at 5x8x14 11.2 -> 11.7.
+// Two slices of eight chunks each would lose (512 -> 512 at 9x9x6 37.8 -> 39.8; four sums 22.6), and so would eight where rows are short or 512 channels
+// are produced (256 -> 256 at 14x6x4 10.2 -> 11.5, 256 -> 512 at 6x7x5 10.2 -> 14.6).
 // The data gradient of a depth shard's slab (D + 2 planes from D) and of the padded volume (D from D) must come from the same
 // kernel, or a shard and the whole volume would disagree in the last bit: the depth counted is the smaller of the two.
 constexpr int kSplitMaxPlane = 32 * 32, kSplitMinPerDepth = 24, kSplitFewPerDepth = 32, kSplitFewMaxChunks = 16;
@@ -448,17 +476,17 @@ SplitRule split_rule(const MfmaConvArgs& a, bool records) {
   const int64_t pairs = per_depth * cdiv(core.od, Flat::TD), rounds = cdiv(pairs, kComputeUnits);
   const bool kept = a.gradient != 0;  // the order of sums does not go by the times
   auto sooner = [&](int percent) { return 100 * split_time(split_tiles(core) * pair, chunks) < percent * mfma_conv_brick_time(core); };
-  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return {!kept && pairs > kSplitBigPlanePairs && sooner(72), false, false};
+  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return {!kept && pairs > kSplitBigPlanePairs && sooner(72), 0};
   const bool few = per_depth <= kSplitFewPerDepth && chunks >= kSplitFewMaxChunks;
-  if (!few && per_depth >= kSplitMinPerDepth) return {true, false, false};
+  if (!few && per_depth >= kSplitMinPerDepth) return {true, 0};
   if (pairs >= split_line(chunks))
-    return {rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || (!kept && sooner(110)), false, false};
+    return {rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || (!kept && sooner(110)), 0};
   const int slices = mfma_conv_brick_slices(core);
-  const bool eight = slices == 8 && chunks == kApartChunks, four = slices == 4 && chunks % 4 == 0;  // (two chunks are cut in halves of 16 channels here)
-  const bool same_bits = (eight || four) && (a.gradient || core.od == a.od || mfma_conv_brick_slices(a) == slices);
+  const bool like_slices = slices == 8 ? chunks == 8 && a.cout <= 256 && a.ow > 8 : slices == 4 ? chunks % 4 == 0 : slices == 2 && chunks <= 4;
+  const bool same_bits = like_slices && (a.gradient || core.od == a.od || mfma_conv_brick_slices(a) == slices);
   if (same_bits ? records : slices > 4 || kept) return {};
   const bool enough = pairs >= split_line_few(chunks, a.cout) && (same_bits || sooner(72));
-  return {enough || (chunks >= kSplitFewMaxChunks && sooner(70)), same_bits && eight, same_bits && four && chunks >= kQuartersChunks};
+  return {enough || (chunks >= kSplitFewMaxChunks && sooner(70)), same_bits ? slices : 0};
 }
 }  // namespace
 

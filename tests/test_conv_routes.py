@@ -68,7 +68,9 @@ def test_slab_and_padded_volume_add_in_one_order(cin, cout):
     (256, 256, (11, 4, 9), "split", "split"),    # four of two
     (192, 256, (6, 15, 7), "split", "brick"),    # four of one and of two: the small-volume kernel cannot
     (64, 128, (14, 13, 6), "split", "brick"),
-    (128, 64, (14, 13, 6), "brick", "brick"),    # the gradient's two slices are one chunk each, which the small-volume kernel cuts in two
+    (128, 64, (14, 13, 6), "brick", "split"),    # the gradient's two slices are one chunk each
+    (512, 512, (9, 9, 6), "split", "brick"),     # two of eight
+    (256, 512, (6, 7, 5), "brick", "brick"),     # eight of one, but 512 channels produced
     (64, 64, (9, 27, 50), "split", "brick"),     # a plane past 32 x 32
 ])
 def test_launch_times_take_no_partial_sums_away(cin, cout, spatial, forward, gradient):
