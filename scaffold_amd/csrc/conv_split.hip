@@ -436,8 +436,8 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
 // those. Some below it would gain as well (128 -> 128 at 8^3, 16 pairs: 9.7 -> 7.7; 256 -> 128 at 8x16x16, 64: 14.9 -> 11.4; 512 -> 256 at
 // 8x16x16, 128: 27.8 -> 22.9): their sliced geometry is what the tests of the launch query hold the last two to.
 // Past three rounds of pairs the brick kernel's launches have no slices either and stage less: a volume below the plane's line comes here only
-// where the bricks leave more over, by the busiest CU's share, than the 10 % that 64-voxel bricks lose at equal shares, or where what either launch
-// takes says so within a tenth. us, bricks -> here: 64 -> 64 at 256x16x16 (1024 pairs, equal shares) 19.2 -> 21.2, 128 -> 128 at 128x16x16 31.0 -> 33.9; 128 -> 64
+// where the bricks leave more over, by the busiest CU's share, than the 10 % that 64-voxel bricks lose at equal shares, or where
+// the times say that a quarter is gained. us, bricks -> here: 64 -> 64 at 256x16x16 (1024 pairs, equal shares) 19.2 -> 21.2, 128 -> 128 at 128x16x16 31.0 -> 33.9; 128 -> 64
 // at 200x20x20 (1500 pairs, 768 against 993 voxel blocks) 56 -> 46, 64 -> 64 at 64x24x24 (576 pairs) 17.9 -> 16.0. Planes past 32 x 32 come here by the times,
 // from about a round of pairs on and where a quarter and more is gained (another order of sums is worth no less): 64 -> 64 at 17x36x35
 // 15.9 -> 9.7, at 9x27x50 12.1 -> 7.9, 128 -> 128 at 10x28x56 25.8 -> 17.0.
@@ -480,7 +480,7 @@ SplitRule split_rule(const MfmaConvArgs& a, bool records) {
   const bool few = per_depth <= kSplitFewPerDepth && chunks >= kSplitFewMaxChunks;
   if (!few && per_depth >= kSplitMinPerDepth) return {true, 0};
   if (pairs >= split_line(chunks))
-    return {rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || (!kept && sooner(110)), 0};
+    return {rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || (!kept && sooner(72)), 0};
   const int slices = mfma_conv_brick_slices(core);
   const bool like_slices = slices == 8 ? chunks == 8 && a.cout <= 256 && a.ow > 8 : slices == 4 ? chunks % 4 == 0 : slices == 2 && chunks <= 4;
   const bool same_bits = like_slices && (a.gradient || core.od == a.od || mfma_conv_brick_slices(a) == slices);
