@@ -429,13 +429,8 @@ WidePlan wide_plan(const MfmaConvArgs& a) {
   const int64_t wgs = wide_workgroups(core, 1);
   if (a.cred % 64 == 0 && wgs > 2 * kComputeUnits &&  // (half of the channels in whole chunks: both kernels take the same pairs)
       mfma_conv_brick_cost(core) * 100 < cdiv(wgs, kComputeUnits) * 1024 * 2 * 100 * (a.cred < 256 ? 97 : 92)) return p;
-  // Up to there it does where the times say that the bricks take three fifths of this kernel's (10 us a chunk and round of 1024-voxel
-  // workgroups, 5.6 of 512, a last round counted at four fifths of a whole one; 4 % rms): a round and a bit of workgroups of a whole CU each. us, here ->
-  // there: 128 -> 64 at two samples of 45x30x35 79.6 -> 45.6, of 17x100x52 153 -> 91, at 33x57x50 84.8 -> 53 (the sums' order changes by it, which is worth no less). A data
-  // gradient stays as well: its bits do not go by the times.
-  const int64_t own = wide_workgroups(core, shape), rounds = cdiv(own, kComputeUnits);
-  const int64_t time = a.cred / 32 * (shape == 1 ? 2002 : 1111) * (4 * rounds * kComputeUnits + own) / (5 * kComputeUnits);
-  if (!a.gradient && a.cred % 64 == 0 && 5 * mfma_conv_brick_time(core) < 3 * time) return p;
+  // Up to there it stays: bricks would be sooner where a round and a bit of workgroups is two (128 -> 64 at 33x57x50 84.8 against 53 us), but they add in
+  // another order, and a network's bits do not go by the times.
   p.use = true;
   p.shape = shape;
   return p;

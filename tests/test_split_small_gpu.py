@@ -79,7 +79,7 @@ def _conv64(x, w):
     (256, 256, (5, 8, 14), "split", "split"),    # in the place of eight slices: two rounds, their sums apart
     (256, 256, (3, 16, 12), "split", "split"),   # 72 pairs
     (256, 256, (11, 4, 9), "split", "split"),    # in the place of four: one chain a wavefront
-    (128, 64, (33, 57, 50), "brick", "brick"),   # bricks in the wide kernel's place by the times
+    (128, 64, (33, 57, 50), "wide", "brick"),    # bricks would be sooner, in another order
     (128, 64, (31, 61, 65), "wide", "brick"),
 ])
 def test_lines_that_the_times_draw(cin, cout, spatial, fwd, dgrad):
