@@ -121,7 +121,7 @@ int sfh_conv3d_uses_mfma(const sfh_conv3d_desc* p, int dtype, int direction);
  * voxels for the weight gradient) whose fp32 partials are summed in fixed order. A pure function of the problem and
  * the compute-unit count the library is written for -- the property the reference's plan machinery exists to
  * guarantee (triton_conv3d/_rungs.py, reduce_gemm.py:71-96: the split count must not depend on the device or the
- * run). [1] and [2] are 0 for SFH_KERNEL_DIRECT (the direct and the thin-channel kernels: whatever
+ * run). Direction 0 is sfh_conv3d_fwd; sfh_conv3d_fwd_gn gives the same bits, where its records are offered from bricks or slices of its own. [1] and [2] are 0 for SFH_KERNEL_DIRECT (the direct and the thin-channel kernels: whatever
  * sfh_conv3d_uses_mfma answers 0 for) and SFH_KERNEL_OTHER_MATRIX (2x2x2 family, fp32 tiles). */
 #define SFH_KERNEL_DIRECT 0
 #define SFH_KERNEL_PERSIST 1

@@ -475,8 +475,8 @@ def pack_weights(w: torch.Tensor, in_shape, stride=1, padding=0, dilation=1, *, 
     ``in_shape``: returns ``(packed_fwd, packed_dgrad)`` to pass as ``packed_weight=``; an entry is ``None`` when it
     was not asked for or when that direction of the problem does not read a packed weight (it then takes ``w``).
     ``out=(packed_fwd, packed_dgrad)`` reuses the buffers of an earlier call for the same problem.
-    The default entry points repack on every call (but for channels-last weights of 32 reduction channels); a train step that packs once
-    here saves a launch per convolution."""
+    The default entry points repack on every call (but for channels-last weights of 32 reduction channels and most of fp32, which are read
+    as they lie); a train step that packs once here saves a launch per convolution."""
     if not w.is_cuda:
         raise NotImplementedError(f"pack_weights: a weight on {w.device}; the packing kernel reads GPU memory")
     nbf, nbd, desc, code = _pack_plan(w, in_shape, stride, padding, dilation)

@@ -17,8 +17,8 @@ struct ColumnCut {
 // item's first planes come from memory with nothing beside them (1.5 to 2 us measured), and what short items lose otherwise.
 // items < 0: too many.
 //
-// us, against cutting until every workgroup has an item, which left up to half of them idle behind two items of the others:
-// forward 32 -> 32 at 54x105x99 53.5 -> 37.7, 36x101x119 39.1 -> 28.8, 96x80x112 59.4 -> 44.5, two samples of 57x87x77 67.1 -> 47.7,
+// us, against cutting until every workgroup has an item, which leaves up to half of them idle behind two items of the others:
+// forward (and data gradient; of a forward only where nobody takes its sums, cut_batch) 32 -> 32 at 54x105x99 53.5 -> 37.7, 36x101x119 39.1 -> 28.8, 96x80x112 59.4 -> 44.5, two samples of 57x87x77 67.1 -> 47.7,
 // 32 -> 64 at 75x107x122 111 -> 92; weight gradient with its sum 32 -> 32 at 96x80x112 63.9 -> 54.3, 54x105x99 53.2 -> 47.0, two
 // samples of 57x87x77 72.5 -> 58.5, 64 -> 32 at 110x48x111 91.2 -> 69.9, 128 -> 64 at 60x35x45 76.4 -> 60.8.
 template <typename I>

@@ -754,8 +754,8 @@ __global__ void __launch_bounds__(kBlock) gn_normalize_pool(const T* __restrict_
 // each) come from the caches for seven of a cell's eight voxels. Same sums in the same order as over the written tensor, so both passes
 // stay with rows; bound by vector instructions as much as by memory (160 and 190 a row and 16-byte piece, 100 and 117 without), on half of the
 // chip (beside a batch of weight gradients) by them alone: no gain there and none lost. Pooling gradient and both passes -> the two, us, bf16: 32 channels of 64x128x128
-// 94 -> 71, 64 of 32x64x64 41 -> 37, 64 of 96x80x112 156 -> 129, 128 of 64^3 90 -> 72, 64 of 128^3 366 -> 272; the captured shard step 2796 -> 2780, a step
-// of 128^3 13370 -> 13290. The first pass leaving the sum for the second was no better: 80 at 64x128x128, 134 at 96x80x112.
+// 94 -> 71, 64 of 32x64x64 41 -> 37, 64 of 96x80x112 156 -> 129, 128 of 64^3 90 -> 72, 64 of 128^3 366 -> 272; a step
+// of 128^3 13370 -> 13290 (that of a 64x128x128 shard, 0.6 %, is within what runs differ by). The first pass leaving the sum for the second was no better: 80 at 64x128x128, 134 at 96x80x112.
 struct PooledGrad {
   const void* g;       // N x pd x ph x pw x C
   const uint8_t* idx;  // the same extents
