@@ -376,7 +376,7 @@ static int conv3d_fwd_any(const sfh_conv3d_desc* p, int dtype, const void* x, co
   hipStream_t st = (hipStream_t)stream;
   if (!(flags & SFH_FLAG_FORCE_GENERIC) && fwd_uses_mfma(*p, dtype, out)) {
     const MfmaConvArgs a = fwd_mfma_args(*p, out);
-    const size_t packed_bytes = mfma_conv_packed_weight_bytes(a), partial_bytes = mfma_conv_partial_bytes(a, true);
+    const size_t packed_bytes = mfma_conv_packed_weight_bytes(a), partial_bytes = mfma_conv_partial_bytes(a, gn != nullptr && gn->part != nullptr);
     if (flags & SFH_FLAG_WEIGHT_PACKED) {  // w is the packed weight; the workspace only holds the partial slices
       if (partial_bytes && (workspace == nullptr || workspace_bytes < partial_bytes))
         return fail(SFH_ERR_WORKSPACE, "conv3d fwd: workspace of %zu bytes needed, got %zu", partial_bytes, workspace_bytes);

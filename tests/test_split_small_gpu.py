@@ -1,10 +1,13 @@
 """The small-volume convolution kernel on the launches of few workgroups (one channel block each) and below its plane line: against
 float64, on both sides of the line, and the same bits from a depth shard's slab as from the padded volume."""
 
+import ctypes
+
 import pytest
 import torch
 
 import scaffold_amd as sa
+from scaffold_amd import _lib
 from scaffold_amd import conv3d as c3
 
 CL = torch.channels_last_3d
@@ -130,3 +133,16 @@ def test_slices_and_their_bits(n, cin, cout, spatial, dtype):
     want = _conv64(x, w) + b.double().view(1, -1, 1, 1, 1)
     half_ulp = 2.0 ** -8 if dtype is torch.bfloat16 else 2.0 ** -11
     assert torch.all((alone.double() - want).abs() <= half_ulp * want.abs() + 1e-5 * want.abs().max())
+
+
+def test_packed_launch_without_slices_takes_no_workspace():
+    """The query has room for the slices behind GroupNorm records; the launch that makes none asks for none."""
+    n, cin, cout, spatial = 1, 64, 128, (14, 13, 6)
+    x, _, w = _operands(n, cin, cout, spatial, torch.bfloat16)
+    packed, _ = c3.pack_weights(w, x.shape, 1, 1, 1)
+    prob, lib = c3._Problem(x.shape, w.shape, 1, 1, 1, torch.bfloat16), _lib.lib()
+    assert lib.sfh_conv3d_fwd_workspace_bytes(ctypes.byref(prob.desc), prob.code) > packed.numel()
+    y = torch.empty_like(sa.conv3d_forward(x, w, None, 1, 1))
+    _lib.check(lib.sfh_conv3d_fwd(ctypes.byref(prob.desc), prob.code, x.data_ptr(), packed.data_ptr(), None, None, y.data_ptr(), None, 0,
+                                  _lib.SFH_FLAG_WEIGHT_PACKED, torch.cuda.current_stream().cuda_stream), "conv3d forward")
+    assert torch.equal(y, sa.conv3d_forward(x, w, None, 1, 1))
