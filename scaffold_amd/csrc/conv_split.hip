@@ -60,8 +60,10 @@ struct Brick {
 // more, a slot's rounds are that many that do. FORM, of launches that add as the bricks' slices do (split_rule):
 //   kApart   the reduction is two rounds, and the first one's sums are set aside. They want 32 registers more: one workgroup to a CU, which the
 //            brick's LDS leaves room for anyway (with two 11 to 17 registers were spilled and every other launch of one block took 0.5 us longer).
-//   kHalves  (R = 2) a wavefront has one of the two voxel halves and all 32 channels of its chunks, in place of both halves and 16.
-enum SplitForm { kOrdinary, kApart, kHalves };
+//   kHalves  (R = 2, one block) a wavefront has one of the two voxel halves and all 32 channels of its chunks, in place of both halves and 16.
+//   kPairs   (R = 4, two blocks) a wavefront has one of the two blocks and two chunks a round: every weight still goes to one wavefront
+//            only, which the halves' do not.
+enum SplitForm { kOrdinary, kApart, kHalves, kPairs };
 template <typename T, typename S, int R, int NSUB, bool PAIR, SplitForm FORM = kOrdinary>
 __global__ void __launch_bounds__(256, FORM == kApart ? 1 : 2)
 conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__ wp, const T* __restrict__ bias, T* __restrict__ y,
@@ -70,9 +72,9 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   using B = Brick<S, NSUB>;
   constexpr int TD = S::TD, TH = S::TH, TW = S::TW, BH = S::BH, BW = S::BW;
   constexpr int PLANE = B::PLANE, SLOT = B::SLOT;
-  constexpr bool APART = FORM == kApart, HALVES = FORM == kHalves, WHOLE = R == 4 || HALVES;  // WHOLE: both k-steps of a tap
-  static_assert(FORM == kOrdinary || (NSUB == 1 && R == (APART ? 4 : 2)), "one block");
-  constexpr int MSW = HALVES ? 1 : MS;  // voxel halves of a wavefront
+  constexpr bool APART = FORM == kApart, HALVES = FORM == kHalves, PAIRS = FORM == kPairs, WHOLE = R == 4 || HALVES;  // WHOLE: both k-steps of a tap
+  static_assert(FORM == kOrdinary || (NSUB == (PAIRS ? 2 : 1) && R == (HALVES ? 2 : 4)), "forms");
+  constexpr int MSW = HALVES ? 1 : MS, NSW = PAIRS ? 1 : NSUB, CHW = PAIRS ? 2 : 1;  // voxel halves, blocks and chunks of a wavefront
   constexpr int ROUNDS = APART ? 2 : 1;
   constexpr int RED_BYTES = ROUNDS * MS * NSUB * 3 * 4096;  // every block from the three wavefronts that do not own it
   constexpr int LDS = R * SLOT > RED_BYTES ? R * SLOT : RED_BYTES;
@@ -90,9 +92,9 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   const int od0 = td_i * TD, oh0 = th_i * TH, ow0 = tw_i * TW;
 
   // This wavefront's share of a round: chunk slot `slot`; with R = 2 also one of the two k-steps of every tap, or one of the voxel halves.
-  const int slot = R == 4 ? wave : wave >> 1;
-  const int khalf = WHOLE ? 0 : wave & 1, half = HALVES ? wave & 1 : 0;
-  constexpr int NITS = WHOLE ? NIT : TAPS;  // iterations of a wavefront per round
+  const int slot = PAIRS ? wave & ~1 : R == 4 ? wave : wave >> 1;
+  const int khalf = WHOLE ? 0 : wave & 1, half = HALVES ? wave & 1 : 0, block = PAIRS ? wave & 1 : 0;
+  constexpr int NITC = WHOLE ? NIT : TAPS, NITS = CHW * NITC;  // iterations of a wavefront per chunk, per round
   constexpr int WSTEP = WHOLE ? FRAG : 2 * FRAG;
   int abase[MSW];  // LDS byte address of the lane's voxel of block row ms at tap (0, 0, 0), in its k-half plane
 #pragma unroll
@@ -100,15 +102,15 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
     const int v = (half + ms) * 32 + j, tw = v % TW, th = v / TW % TH, td = v / (TW * TH);
     abase[ms] = slot * SLOT + (kg + 2 * khalf) * PLANE + (td * BH + th) * B::ROW + tw * 16;
   }
-  auto a_off = [](int k) constexpr { return WHOLE ? B::tap_off(k / 2) + (k % 2) * 2 * PLANE : B::tap_off(k); };
+  auto a_off = [](int k) constexpr { return k / NITC * SLOT + (WHOLE ? B::tap_off(k % NITC / 2) + (k % 2) * 2 * PLANE : B::tap_off(k)); };
 
-  f32x16_t acc[MSW][NSUB], first[MSW];  // first: the first round's sums, where they are chains apart
+  f32x16_t acc[MSW][NSW], first[MSW];  // first: the first round's sums, where they are chains apart
 #pragma unroll
   for (int ms = 0; ms < MSW; ++ms)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
 #pragma unroll
-      for (int ns = 0; ns < NSUB; ++ns) acc[ms][ns][r] = 0.f;
+      for (int ns = 0; ns < NSW; ++ns) acc[ms][ns][r] = 0.f;
       first[ms][r] = 0.f;
     }
 
@@ -116,19 +118,20 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   const int id0 = od0 - a.pd, ih0 = oh0 - a.ph, iw0 = ow0 - a.pw;
   constexpr int PIECES = S::BV * 4 * R;
   constexpr int ITERS = (PIECES + 255) / 256;
-  constexpr int WDEPTH = 16 / NSUB;  // weight fragments (per output block) in flight per wavefront
+  constexpr int WDEPTH = 16 / NSW;  // weight fragments (per output block) in flight per wavefront
   const int64_t wns = (int64_t)ncc * (NIT * FRAG);  // next 32-channel output block
 
   for (int c0 = 0; c0 < ncc; c0 += R) {
     // The wavefront's first weight fragments are requested before the bricks are staged: they depend on nothing in LDS.
     const int stride = NSUB == 1 ? chunk_stride : 1;  // (two blocks have no registers for it)
-    const int first_chunk = stride == 1 ? c0 : c0 / R;  // slot 0's
-    const T* wcc = wp + ((int64_t)(nb * NSUB) * ncc + first_chunk + slot * stride) * (NIT * FRAG) + khalf * FRAG + lane * 8;
-    uint4 wq[NITS][NSUB];  // fully unrolled: every slot is its own register set, live for WDEPTH iterations
+    const int first_chunk = PAIRS ? c0 / 2 : stride == 1 ? c0 : c0 / R;  // slot 0's
+    auto chunk_of = [&](int q) { return PAIRS ? first_chunk + (q >> 1) * (ncc >> 1) + (q & 1) : first_chunk + q * stride; };
+    const T* wcc = wp + ((int64_t)(nb * NSUB + block) * ncc + chunk_of(slot)) * (NIT * FRAG) + khalf * FRAG + lane * 8;
+    uint4 wq[NITS][NSW];  // fully unrolled: every slot is its own register set, live for WDEPTH iterations
 #pragma unroll
     for (int k = 0; k < WDEPTH; ++k)
 #pragma unroll
-      for (int ns = 0; ns < NSUB; ++ns) wq[k][ns] = *reinterpret_cast<const uint4*>(wcc + ns * wns + k * WSTEP);
+      for (int ns = 0; ns < NSW; ++ns) wq[k][ns] = *reinterpret_cast<const uint4*>(wcc + ns * wns + k * WSTEP);
     __syncthreads();  // every wavefront is done reading the previous round
     {
       // A voxel's 4 R pieces (R chunks of 4) are consecutive threads: 64 R contiguous bytes when the chunks lie in one tensor.
@@ -137,7 +140,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
       for (int u = 0; u < ITERS; ++u) {
         const int p = u * 256 + tid;
         const int q = p % (4 * R), vox = p / (4 * R);
-        const int cc = first_chunk + (q >> 2) * stride, piece = q & 3;
+        const int cc = chunk_of(q >> 2), piece = q & 3;
         const int bw = vox % BW, bh = (vox / BW) % BH, bd = vox / (BW * BH);
         const int id = id0 + bd, ih = ih0 + bh, iw = iw0 + bw;
         const bool in = p < PIECES && (unsigned)id < (unsigned)a.id && (unsigned)ih < (unsigned)a.ih && (unsigned)iw < (unsigned)a.iw;
@@ -170,13 +173,13 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
     for (int k = 0; k < NITS; ++k) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int m = 0; m < MSW * NSUB; ++m) {
-        const int ms = m / NSUB, ns = m % NSUB;
+      for (int m = 0; m < MSW * NSW; ++m) {
+        const int ms = m / NSW, ns = m % NSW;
         acc[ms][ns] = Mma32<T>::run(wq[k][ns], aq[k & 1][ms], acc[ms][ns]);
         __builtin_amdgcn_sched_barrier(0);
-        if (m < NSUB && k + WDEPTH < NITS) wq[k + WDEPTH][m] = *reinterpret_cast<const uint4*>(wcc + m * wns + (k + WDEPTH) * WSTEP);
-        if (NSUB == 1 ? true : m >= NSUB) {
-          constexpr int first = NSUB == 1 ? 0 : NSUB;
+        if (m < NSW && k + WDEPTH < NITS) wq[k + WDEPTH][m] = *reinterpret_cast<const uint4*>(wcc + m * wns + (k + WDEPTH) * WSTEP);
+        if (NSW == 1 ? true : m >= NSW) {
+          constexpr int first = NSW == 1 ? 0 : NSW;
           if (k + 1 < NITS) aq[(k + 1) & 1][m - first] = *reinterpret_cast<const uint4*>(lds + abase[m - first] + a_off(k + 1));
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -199,7 +202,7 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   // u collects block u = ms * NSUB + ns.
   __syncthreads();  // the bricks are not read any more
   float4* red = reinterpret_cast<float4*>(lds);
-  auto mine_of = [&](int round, int u) -> const f32x16_t& { return APART && round == 0 ? first[u / NSUB] : acc[u / NSUB][u % NSUB]; };
+  auto mine_of = [&](int round, int u) -> const f32x16_t& { return APART && round == 0 ? first[u / NSUB] : acc[u / NSUB % MSW][u % NSUB % NSW]; };
   auto send = [&](int place, const f32x16_t& v) {
 #pragma unroll
     for (int r4 = 0; r4 < 4; ++r4) red[(place * 4 + r4) * 64 + lane] = make_float4(v[4 * r4], v[4 * r4 + 1], v[4 * r4 + 2], v[4 * r4 + 3]);
@@ -215,6 +218,9 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   };
   if constexpr (HALVES) {
     send(half * 2 + slot, acc[0][0]);
+  } else if constexpr (PAIRS) {
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms) send((ms * NSUB + block) * 2 + (slot >> 1), acc[ms][0]);
   } else {
 #pragma unroll
   for (int round = 0; round < ROUNDS; ++round)
@@ -230,8 +236,8 @@ conv_split_kernel(MfmaConvArgs a, const T* __restrict__ x, const T* __restrict__
   f32x16_t tot;
 #pragma unroll
   for (int r = 0; r < 16; ++r) tot[r] = 0.f;
-  if constexpr (HALVES) {
-    if (wave < MS) {
+  if constexpr (HALVES || PAIRS) {
+    if (wave < MS * NSUB) {
       tot = receive(wave * 2);
       const f32x16_t second = receive(wave * 2 + 1);
 #pragma unroll
@@ -369,10 +375,11 @@ SplitRule split_rule(const MfmaConvArgs& a, bool records);
 struct SplitPlan { SplitForm form; int chunk_stride, shape, blocks; int64_t tiles; };
 SplitPlan split_plan(const MfmaConvArgs& a, bool records) {
   const int slices = split_rule(a, records).slices;
-  const SplitForm form = slices == 8 ? kApart : slices == 2 ? kHalves : kOrdinary;
+  const SplitForm form = slices == 8 ? kApart : slices != 2 ? kOrdinary : a.cred <= 4 * kChunk ? kHalves : kPairs;
   const int shape = records ? 0 : form != kOrdinary ? 1 : split_shape(a);
   const int64_t tiles = tiles_of(a, shape);
-  return SplitPlan{form, slices == 2 || slices == 4 ? a.cred / kChunk / slices : 1, shape, slices > 0 ? 1 : split_blocks(tiles, a.cout), tiles};
+  return SplitPlan{form, slices == 2 || slices == 4 ? a.cred / kChunk / slices : 1, shape,
+                   form == kPairs ? 2 : slices > 0 ? 1 : split_blocks(tiles, a.cout), tiles};
 }
 
 template <typename T, typename S, int R, int NSUB, bool PAIR, SplitForm FORM = kOrdinary>
@@ -409,6 +416,9 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
   if (p.form == kHalves)
     return x1 != nullptr ? launch_brick<T, Cube, 2, 1, true, kHalves>(p.chunk_stride, a, x, packed, bias, y, st, gn, x1, y1, first)
                          : launch_brick<T, Cube, 2, 1, false, kHalves>(p.chunk_stride, a, x, packed, bias, y, st, gn, x1, y1, first);
+  if (p.form == kPairs)
+    return x1 != nullptr ? launch_brick<T, Cube, 4, 2, true, kPairs>(1, a, x, packed, bias, y, st, gn, x1, y1, first)
+                         : launch_brick<T, Cube, 4, 2, false, kPairs>(1, a, x, packed, bias, y, st, gn, x1, y1, first);
 #define SFH_SPLIT(NSUB)                                                                                         \
   x1 != nullptr ? (four ? launch_split<T, 4, NSUB, true>(p, a, x, packed, bias, y, st, gn, x1, y1, first)   \
                         : launch_split<T, 2, NSUB, true>(p, a, x, packed, bias, y, st, gn, x1, y1, first))  \
@@ -437,9 +447,9 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
 // 8x16x16, 128: 27.8 -> 22.9): their sliced geometry is what the tests of the launch query hold the last two to.
 // Past three rounds of pairs the brick kernel's launches have no slices either and stage less: a volume below the plane's line comes here only
 // where the bricks leave more over, by the busiest CU's share, than the 10 % that 64-voxel bricks lose at equal shares, or where
-// the times say that a quarter is gained. us, bricks -> here: 64 -> 64 at 256x16x16 (1024 pairs, equal shares) 19.2 -> 21.2, 128 -> 128 at 128x16x16 31.0 -> 33.9; 128 -> 64
+// the times say that a third is gained. us, bricks -> here: 64 -> 64 at 256x16x16 (1024 pairs, equal shares) 19.2 -> 21.2, 128 -> 128 at 128x16x16 31.0 -> 33.9; 128 -> 64
 // at 200x20x20 (1500 pairs, 768 against 993 voxel blocks) 56 -> 46, 64 -> 64 at 64x24x24 (576 pairs) 17.9 -> 16.0. Planes past 32 x 32 come here by the times,
-// from about a round of pairs on and where a quarter and more is gained (another order of sums is worth no less): 64 -> 64 at 17x36x35
+// from about a round of pairs on and where a third is gained (another order of sums is worth no less): 64 -> 64 at 17x36x35
 // 15.9 -> 9.7, at 9x27x50 12.1 -> 7.9, 128 -> 128 at 10x28x56 25.8 -> 17.0.
 // All that is for the forward, with GroupNorm records or without (the result is the same bits either way). A data gradient comes here by the rules
 // before the times: nothing is gained by another order of its sums that is worth a step's gradients in other bits. Where the slices' bits
@@ -448,20 +458,20 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
 // results of 64 to 512 channels that are not the rounded 64-bit ones: 1.5e-3 here, 1.9e-3 in bricks, 28 problems of both directions), so 256 -> 256 at 32^3 stays at
 // 109 us though bricks take 102. Eight slices are nearer still (1.35e-3, 1.75e-3 here with four sums; four: level).
 // What the bricks would sum in slices comes here with the slices' bits, so that it may in both directions: of four a wavefront takes one's chunks in
-// their order; of two, up to 128 channels, a voxel half of one's; eight of one chunk (256 channels) are two rounds whose sums meet at the end. Where none
-// of these is, eight slices stay (nearer the exact value still, 1.35e-3, 1.75e-3 here with four sums), and two or four become this kernel's sums where
-// a quarter of the time is gained. A launch that leaves GroupNorm records stays with the slices, whose records are sums of other voxels.
+// their order; of two, up to 128 channels, a voxel half of one's, past that one of two blocks of one's; eight of one chunk (256 channels) are two
+// rounds whose sums meet at the end. Where none of these is, eight slices stay (nearer the exact value still, 1.35e-3, 1.75e-3 here with four sums), and four become this
+// kernel's sums where a third of the time is gained. A launch that leaves GroupNorm records stays with the slices, whose records are sums of other voxels.
 // us, slices and their sum -> here, with their bits: 64 -> 128 at 14x13x6 9.3 -> 6.0, 64 -> 512 at 7x3x6 8.8 -> 6.0, 128 -> 64 (data gradient) at 14x13x6 9.4 -> 6.0,
-// three samples of 128 -> 256 at 10x3x6 12.8 -> 8.9, 128 -> 512 at 3x4x9 9.0 -> 7.0, 256 -> 256 at 11x4x9 12.6 -> 10.3, at 8x4x20 (eight) 12.0 -> 11.4, at 5x8x14 11.2 -> 11.7.
-// Two slices of eight chunks each would lose (512 -> 512 at 9x9x6 37.8 -> 39.8; four sums 22.6), and so would eight where rows are short or 512 channels
-// are produced (256 -> 256 at 14x6x4 10.2 -> 11.5, 256 -> 512 at 6x7x5 10.2 -> 14.6).
+// three samples of 128 -> 256 at 10x3x6 12.8 -> 8.9, 128 -> 512 at 3x4x9 9.0 -> 7.0, 256 -> 256 at 11x4x9 12.6 -> 10.3, at 8x4x20 (eight) 12.0 -> 11.4, at 5x8x14 11.2 -> 11.7,
+// 512 -> 512 at 9x9x6 38.4 -> 31.2 (four sums 24.2; by voxel halves, whose every weight goes to two wavefronts, 39.8), 512 -> 256 at 10x8x22 39.1 -> 31.3. Eight would
+// lose where rows are short or 512 channels are produced (256 -> 256 at 14x6x4 10.2 -> 11.5, 256 -> 512 at 6x7x5 10.2 -> 14.6).
 // The data gradient of a depth shard's slab (D + 2 planes from D) and of the padded volume (D from D) must come from the same
 // kernel, or a shard and the whole volume would disagree in the last bit: the depth counted is the smaller of the two.
 constexpr int kSplitMaxPlane = 32 * 32, kSplitMinPerDepth = 24, kSplitFewPerDepth = 32, kSplitFewMaxChunks = 16;
 constexpr int kSplitBigPlanePairs = 240;
 // Pairs from which a volume below the plane's line comes here, and the fewer from which it does where its sums are no longer than the slices'. us, slices
 // and their sum -> here: 64 -> 128 at 14x13x6 (56 pairs) 9.9 -> 5.6, at 5x10x11 (36) 10.0 -> 5.5, 128 -> 128 at 9x12x8 (30) 13.2 -> 7.7, at 4x6x20 (24) 11.5 -> 7.7.
-// Long reductions on fewer where the slices are far behind: 512 -> 512 at 9x9x6 (120) 35.1 -> 22.1.
+// Long reductions on fewer where the slices are far behind (512 -> 512 at 9x9x6, 120 pairs).
 int64_t split_line(int chunks) { return chunks <= 4 ? kComputeUnits / 4 : chunks <= 8 ? kComputeUnits / 4 + 1 : kComputeUnits / 2 + 1; }
 int64_t split_line_few(int chunks, int cout) { return chunks <= 4 && cout >= 128 ? 24 : chunks <= 8 && cout >= 256 ? 48 : split_line(chunks); }
 
@@ -476,16 +486,16 @@ SplitRule split_rule(const MfmaConvArgs& a, bool records) {
   const int64_t pairs = per_depth * cdiv(core.od, Flat::TD), rounds = cdiv(pairs, kComputeUnits);
   const bool kept = a.gradient != 0;  // the order of sums does not go by the times
   auto sooner = [&](int percent) { return 100 * split_time(split_tiles(core) * pair, chunks) < percent * mfma_conv_brick_time(core); };
-  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return {!kept && pairs > kSplitBigPlanePairs && sooner(72), 0};
+  if ((int64_t)a.oh * a.ow > kSplitMaxPlane) return {!kept && pairs > kSplitBigPlanePairs && sooner(68), 0};
   const bool few = per_depth <= kSplitFewPerDepth && chunks >= kSplitFewMaxChunks;
   if (!few && per_depth >= kSplitMinPerDepth) return {true, 0};
   if (pairs >= split_line(chunks))
-    return {rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || (!kept && sooner(72)), 0};
+    return {rounds <= 3 || rounds * (kBrickVoxels * kBlocks) * 110 < mfma_conv_brick_cost(core) || (!kept && sooner(68)), 0};
   const int slices = mfma_conv_brick_slices(core);
-  const bool like_slices = slices == 8 ? chunks == 8 && a.cout <= 256 && a.ow > 8 : slices == 4 ? chunks % 4 == 0 : slices == 2 && chunks <= 4;
+  const bool like_slices = slices == 8 ? chunks == 8 && a.cout <= 256 && a.ow > 8 : slices == 4 || (slices == 2 && chunks > 4) ? chunks % 4 == 0 : slices == 2;
   const bool same_bits = like_slices && (a.gradient || core.od == a.od || mfma_conv_brick_slices(a) == slices);
   if (same_bits ? records : slices > 4 || kept) return {};
-  const bool enough = pairs >= split_line_few(chunks, a.cout) && (same_bits || sooner(72));
+  const bool enough = pairs >= split_line_few(chunks, a.cout) && (same_bits || sooner(68));
   return {enough || (chunks >= kSplitFewMaxChunks && sooner(70)), same_bits ? slices : 0};
 }
 }  // namespace

@@ -69,7 +69,8 @@ def test_slab_and_padded_volume_add_in_one_order(cin, cout):
     (192, 256, (6, 15, 7), "split", "brick"),    # four of one and of two: the small-volume kernel cannot
     (64, 128, (14, 13, 6), "split", "brick"),
     (128, 64, (14, 13, 6), "brick", "split"),    # the gradient's two slices are one chunk each
-    (512, 512, (9, 9, 6), "split", "brick"),     # two of eight
+    (512, 512, (9, 9, 6), "split", "split"),     # two of eight
+    (128, 64, (20, 34, 42), "brick", "brick"),   # a plane past 32 x 32 that would gain a quarter
     (256, 512, (6, 7, 5), "brick", "brick"),     # eight of one, but 512 channels produced
     (64, 64, (9, 27, 50), "split", "brick"),     # a plane past 32 x 32
 ])

@@ -78,7 +78,7 @@ def _conv64(x, w):
     (128, 64, (14, 13, 6), "brick", "split"),    # ... in the gradient
     (128, 128, (9, 12, 8), "split", "split"),    # ... whose four sums are the slices', so that the data gradient comes too
     (128, 128, (4, 6, 12), "brick", "brick"),    # 16 pairs: too few
-    (512, 512, (9, 9, 6), "split", "brick"),     # a long reduction by the times
+    (512, 512, (9, 9, 6), "split", "split"),     # a long reduction by the times, two slices
     (256, 256, (5, 8, 14), "split", "split"),    # in the place of eight slices: two rounds, their sums apart
     (256, 256, (3, 16, 12), "split", "split"),   # 72 pairs
     (256, 256, (11, 4, 9), "split", "split"),    # in the place of four: one chain a wavefront
@@ -119,7 +119,8 @@ def test_statistics_change_no_bit(n, cin, cout, spatial, depth_padding):
 @pytest.mark.parametrize("n,cin,cout,spatial", [(1, 128, 256, (8, 8, 8)), (1, 128, 128, (4, 6, 20)), (2, 128, 128, (5, 7, 9)),
                                                 (1, 256, 256, (5, 8, 14)), (1, 256, 256, (8, 4, 20)), (2, 256, 256, (5, 4, 14)),
                                                 (1, 256, 256, (11, 4, 9)), (2, 256, 512, (8, 3, 3)), (1, 64, 128, (14, 13, 6)), (2, 64, 128, (5, 7, 9)),
-                                                (1, 64, 512, (7, 3, 6)), (3, 128, 256, (10, 3, 6))])
+                                                (1, 64, 512, (7, 3, 6)), (3, 128, 256, (10, 3, 6)),
+                                                (1, 512, 512, (9, 9, 6)), (1, 512, 256, (10, 8, 22)), (2, 512, 1024, (5, 4, 4))])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_slices_and_their_bits(n, cin, cout, spatial, dtype):
     """A slice to a wavefront, or to a wavefront and round: the launch that leaves GroupNorm records is the bricks' in slices, the one without the small-volume kernel's,
