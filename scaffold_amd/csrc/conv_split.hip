@@ -15,6 +15,7 @@
 //     four MFMAs (two in the brick kernel at this size), every fragment of the workgroup is fetched by exactly one
 //     wavefront (the brick kernel's four wavefronts fetch the same ones), and the chunks of a round are staged with
 //     one trip to memory instead of one per chunk.
+//     (In the place of the bricks' slices the shares are those of the slices, so that the sums are too: SplitForm.)
 //   * At the end the wavefronts' partial accumulators meet in LDS: wavefront u collects block u from the other three
 //     in wavefront order (a fixed order: the same bits on every run), adds the bias, rounds once, leaves the GroupNorm
 //     records of what it stores (gn_stats.hpp) and writes 16-byte pieces.
@@ -469,9 +470,8 @@ int launch_split_typed(const MfmaConvArgs& a, const void* x, const void* packed,
 // kernel, or a shard and the whole volume would disagree in the last bit: the depth counted is the smaller of the two.
 constexpr int kSplitMaxPlane = 32 * 32, kSplitMinPerDepth = 24, kSplitFewPerDepth = 32, kSplitFewMaxChunks = 16;
 constexpr int kSplitBigPlanePairs = 240;
-// Pairs from which a volume below the plane's line comes here, and the fewer from which it does where its sums are no longer than the slices'. us, slices
-// and their sum -> here: 64 -> 128 at 14x13x6 (56 pairs) 9.9 -> 5.6, at 5x10x11 (36) 10.0 -> 5.5, 128 -> 128 at 9x12x8 (30) 13.2 -> 7.7, at 4x6x20 (24) 11.5 -> 7.7.
-// Long reductions on fewer where the slices are far behind (512 -> 512 at 9x9x6, 120 pairs).
+// Pairs from which a volume below the plane's line comes here, and the fewer from which it does in the place of slices (figures above; longer reductions where
+// the times say that three tenths are gained).
 int64_t split_line(int chunks) { return chunks <= 4 ? kComputeUnits / 4 : chunks <= 8 ? kComputeUnits / 4 + 1 : kComputeUnits / 2 + 1; }
 int64_t split_line_few(int chunks, int cout) { return chunks <= 4 && cout >= 128 ? 24 : chunks <= 8 && cout >= 256 ? 48 : split_line(chunks); }
 
